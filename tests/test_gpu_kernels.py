@@ -941,3 +941,32 @@ def test_the_measurement_tool_runs(capsys):
     assert main(["product", "--rows", "40", "--out", "96", "--in", "64", "--kind", "residual", "--copies", "3", "--reps", "2"]) == 0
     out = capsys.readouterr().out
     assert out.count(" us; ") == 3 and "attention 100:1x3,0:40" in out and "product residual rows 40" in out
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 16, 255), (15, 17, 256), (16, 33, 257), (17, 16, 16), (40, 130, 300), (16, 700, 513),
+                                   (130, 15, 1028), (33, 31, 7)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_plain_product_of_few_rows_or_columns(ops_for, M, N, K, dtype):
+    """Tiles of 16 x 16 with chunks of 256: edges of rows, columns and chunks, rows that start on 16 bytes and rows that do not,
+    against 64 bits; and a row gives the same bits alone, in a tile with others, and from a product large enough for tiles of 64 x 64."""
+    from tiny_inference_server_amd.ops.hip_ops import _ptr
+    ops = ops_for(torch.float32)
+    w, r = rnd((N, K), dtype, 601).cuda(), rnd((M, N), torch.float32, 602).cuda()
+
+    def product(x, residual, rows, n=N, weights=w):
+        out = torch.full((rows, n), float("nan"), device="cuda")
+        ops.gemm_plain.tis_gemm_plain(0 if dtype == torch.float32 else 1, 0, _ptr(x), x.stride(0), _ptr(weights), K, _ptr(residual),
+                                      residual.stride(0) if residual is not None else 0, _ptr(out), n, rows, n, K, ops._stream())
+        return out
+
+    for pad in (0, 1, 4):          # the rows' stride: as wide as a row, odd, a multiple of four beyond
+        x = rnd((M, K + pad), dtype, 603 + pad).cuda()[:, :K]
+        got = product(x, r, M)
+        want = x.double() @ w.double().T + r.double()
+        # K products and as many additions, each rounded once: (K + 1) half units of the sum of magnitudes
+        bound = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + r.double().abs())
+        assert ((got.double() - want).abs() <= bound).all()
+        assert torch.equal(product(x[M - 1:], None, 1)[0], product(x, None, M)[M - 1])
+    many = torch.cat([rnd((64 * 16, K), dtype, 610).cuda(), x.contiguous()])
+    wide = torch.cat([w, rnd((64 * 40, K), dtype, 611).cuda()])
+    assert torch.equal(product(many, None, len(many), len(wide), wide)[-M:, :N], product(x, None, M))

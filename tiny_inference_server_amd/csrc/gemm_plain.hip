@@ -65,22 +65,122 @@ __global__ __launch_bounds__(GP_THREADS) void gemm_plain_kernel(const TI* __rest
   }
 }
 
+// The same product for few rows or few columns, where tiles of 64 x 64 leave most compute units idle and their chunks of 16
+// are one trip to memory each: a workgroup owns 16 rows and 16 columns, a thread one output, and K comes through LDS in
+// chunks of 256, the next chunk's loads in flight in registers while one is summed. Same order of sums as above, so the
+// results are the same bits. What bounds it is the chain of K multiply-adds and two LDS reads for every four of them.
+// A row of LDS is four floats longer than a chunk: the 16 columns a read takes 16 bytes of lie in 16 different bank groups.
+// VEC: rows of A and W start on 16 bytes and K is a multiple of 4. MI355X, float, us, tiles of 64 x 64 / these:
+// 3 rows 64 x 64 8.9 / 3.2, 64 x 176 17.7 / 3.8; 1 row 1536 x 1536 136 / 15; 8 rows 1536 x 4096 365 / 35, 48000 x 1536 253 / 97;
+// 100 rows 1536 x 4096 436 / 74.
+static constexpr int GS_BM = 16, GS_BN = 16, GS_BK = 256, GS_LD = GS_BK + 4;
+
+template <bool VEC, typename TI, typename TO>
+__global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI* __restrict__ A, long lda, const TI* __restrict__ W,
+                                                                   long ldw, const TO* __restrict__ R, long ldr,
+                                                                   TO* __restrict__ C, long ldc, int M, int N, int K) {
+  constexpr int THREADS = GS_BM * GS_BN, ROWS = GS_BN + GS_BM, PER = ROWS * (GS_BK / 4) / THREADS;   // groups of four a thread copies
+  __shared__ __attribute__((aligned(16))) float lds[2][ROWS][GS_LD];                           // W's rows, then A's
+  const int t = threadIdx.x, tx = t % GS_BN, ty = t / GS_BN;
+  const long m0 = (long)blockIdx.y * GS_BM, n0 = (long)blockIdx.x * GS_BN;
+  float4 held[PER];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int row = (i * THREADS + t) / (GS_BK / 4), at = (i * THREADS + t) % (GS_BK / 4);
+      const bool is_w = row < GS_BN;
+      const long r = is_w ? n0 + row : m0 + row - GS_BN;
+      const bool ok = r < (is_w ? N : M);
+      const TI* src = is_w ? W + (ok ? r : 0) * ldw : A + (ok ? r : 0) * lda;
+      held[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (VEC && sizeof(TI) == 4) {
+        if (ok && k0 + at * 4 < K) held[i] = *reinterpret_cast<const float4*>(src + k0 + at * 4);
+      } else {               // elements at, at + 64, ...: neighbouring threads read neighbours
+        float* h = reinterpret_cast<float*>(&held[i]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = k0 + at + e * (GS_BK / 4);
+          if (ok && k < K) h[e] = to_f(src[k]);
+        }
+      }
+    }
+  };
+  auto commit = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int row = (i * THREADS + t) / (GS_BK / 4), at = (i * THREADS + t) % (GS_BK / 4);
+      if constexpr (VEC && sizeof(TI) == 4) {
+        *reinterpret_cast<float4*>(&lds[buf][row][at * 4]) = held[i];
+      } else {
+        const float* h = reinterpret_cast<const float*>(&held[i]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lds[buf][row][at + e * (GS_BK / 4)] = h[e];
+      }
+    }
+  };
+  const long m = m0 + ty, n = n0 + tx;
+  const bool live = m < M && n < N;
+  float res = 0.f;
+  if (R && live) res = to_f(R[m * ldr + n]);
+  float acc = 0.f;
+  fetch(0);
+  commit(0);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += GS_BK, buf ^= 1) {
+    const bool more = k0 + GS_BK < K;
+    if (more) fetch(k0 + GS_BK);
+    const float* wr = lds[buf][tx];
+    const float* ar = lds[buf][GS_BN + ty];
+    const int kc = min(GS_BK, (K - k0 + 15) / 16 * 16);
+    for (int k = 0; k < kc; k += 16) {
+#pragma unroll
+      for (int j = 0; j < 16; j += 4) {
+        const float4 a = *reinterpret_cast<const float4*>(ar + k + j), b = *reinterpret_cast<const float4*>(wr + k + j);
+        acc = fmaf(a.x, b.x, acc);
+        acc = fmaf(a.y, b.y, acc);
+        acc = fmaf(a.z, b.z, acc);
+        acc = fmaf(a.w, b.w, acc);
+      }
+    }
+    if (more) commit(buf ^ 1);
+    __syncthreads();
+  }
+  if (live) C[m * ldc + n] = from_f<TO>(R ? acc + res : acc);
+}
+
+template <typename TI, typename TO>
+static void launch_plain(const void* A, long lda, const void* W, long ldw, const void* R, long ldr, void* C, long ldc, int M,
+                         int N, int K, hipStream_t stream) {
+  const long tiles = (long)((N + GP_BN - 1) / GP_BN) * ((M + GP_BM - 1) / GP_BM);
+  // Up to 16 rows, and wherever 64 x 64 tiles would be fewer than two for every compute unit (a chain of K / 16 trips to
+  // memory on a chip that is mostly idle); below 512 columns of K that chain is short, and half a tile a unit is the line.
+  // us, tiles of 64 x 64 / of 16 x 16: 384 tiles of K = 1536 248 / 187, 512 tiles 243 / 252, 768 tiles 297 / 371; K = 64:
+  // 256 tiles 11.7 / 19.9; K = 176: 32 tiles 20.2 / 4.9.
+  if (M <= 16 || tiles < (K >= 512 ? 512 : 128)) {
+    const bool vec = sizeof(TI) == 4 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+    const dim3 grid((N + GS_BN - 1) / GS_BN, (M + GS_BM - 1) / GS_BM);
+    const auto kernel = vec ? gemm_plain_few_kernel<true, TI, TO> : gemm_plain_few_kernel<false, TI, TO>;
+    kernel<<<grid, GS_BM * GS_BN, 0, stream>>>((const TI*)A, lda, (const TI*)W, ldw, (const TO*)R, ldr, (TO*)C, ldc, M, N, K);
+    return;
+  }
+  const dim3 grid((N + GP_BN - 1) / GP_BN, (M + GP_BM - 1) / GP_BM);
+  gemm_plain_kernel<TI, TO><<<grid, GP_THREADS, 0, stream>>>((const TI*)A, lda, (const TI*)W, ldw, (const TO*)R, ldr, (TO*)C,
+                                                             ldc, M, N, K);
+}
+
 // in_dtype / out_dtype: 0 float, 1 bfloat16. Supported: (0,0), (1,1), (1,0).
 TIS_EXPORT int tis_gemm_plain(int in_dtype, int out_dtype, const void* A, long lda, const void* W, long ldw,
                               const void* R, long ldr, void* C, long ldc, int M, int N, int K, hipStream_t stream) {
   if (M == 0 || N == 0) return 0;
   if (M < 0 || N < 0 || K < 1) return tis_fail("gemm: bad size M=%d N=%d K=%d", M, N, K);
-  dim3 grid((N + GP_BN - 1) / GP_BN, (M + GP_BM - 1) / GP_BM);
-  if (grid.y > 65535) return tis_fail("gemm: %d rows exceed the grid", M);
+  if ((M + GP_BM - 1) / GP_BM > 65535) return tis_fail("gemm: %d rows exceed the grid", M);
   if (in_dtype == TIS_F32 && out_dtype == TIS_F32)
-    gemm_plain_kernel<float, float><<<grid, GP_THREADS, 0, stream>>>((const float*)A, lda, (const float*)W, ldw,
-                                                                     (const float*)R, ldr, (float*)C, ldc, M, N, K);
+    launch_plain<float, float>(A, lda, W, ldw, R, ldr, C, ldc, M, N, K, stream);
   else if (in_dtype == TIS_BF16 && out_dtype == TIS_BF16)
-    gemm_plain_kernel<bf16, bf16><<<grid, GP_THREADS, 0, stream>>>((const bf16*)A, lda, (const bf16*)W, ldw,
-                                                                   (const bf16*)R, ldr, (bf16*)C, ldc, M, N, K);
+    launch_plain<bf16, bf16>(A, lda, W, ldw, R, ldr, C, ldc, M, N, K, stream);
   else if (in_dtype == TIS_BF16 && out_dtype == TIS_F32)
-    gemm_plain_kernel<bf16, float><<<grid, GP_THREADS, 0, stream>>>((const bf16*)A, lda, (const bf16*)W, ldw,
-                                                                    (const float*)R, ldr, (float*)C, ldc, M, N, K);
+    launch_plain<bf16, float>(A, lda, W, ldw, R, ldr, C, ldc, M, N, K, stream);
   else
     return tis_fail("gemm: unsupported dtype pair in=%d out=%d", in_dtype, out_dtype);
   return tis_launch_status("gemm_plain");
