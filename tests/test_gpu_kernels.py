@@ -970,3 +970,21 @@ def test_plain_product_of_few_rows_or_columns(ops_for, M, N, K, dtype):
     many = torch.cat([rnd((64 * 16, K), dtype, 610).cuda(), x.contiguous()])
     wide = torch.cat([w, rnd((64 * 40, K), dtype, 611).cuda()])
     assert torch.equal(product(many, None, len(many), len(wide), wide)[-M:, :N], product(x, None, M))
+
+
+@pytest.mark.parametrize("K", [8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 520])
+@pytest.mark.parametrize("M,N", [(129, 60), (1900, 2044), (1301, 3508), (2047, 8188)])
+def test_tiled_product_of_few_steps_of_each_tile(ops_for, M, N, K):
+    """Tiles of 64, 128, 192 and 256 columns: a K of one step and of as many as are copied ahead, one more and one less, whole and
+    ragged last steps, rows and columns that end inside a tile; plain, gated and 32-bit results against 64 bits."""
+    ops = ops_for(torch.bfloat16)
+    x, w = rnd((M, K), torch.bfloat16, 701).cuda(), rnd((N, K), torch.bfloat16, 702, K ** -0.5).cuda()
+    want = x.double() @ w.double().T
+    # 32-bit sums of exact products: K additions, each within half a unit of the sum of magnitudes so far
+    bound = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    got = ops.linear(x, w, out_dtype=torch.float32)
+    assert ((got.double() - want).abs() <= bound).all()
+    # a bfloat16 result is the 32-bit sum rounded once
+    assert torch.equal(ops.linear(x, w), got.to(torch.bfloat16))
+    gate, up = got[:, 0::2].clamp(max=7.0), got[:, 1::2].clamp(-7.0, 7.0)
+    torch.testing.assert_close(ops.linear_gated(x, w, 7.0).float(), gate * torch.sigmoid(1.702 * gate) * (up + 1.0), rtol=5e-3, atol=1e-3)

@@ -4,17 +4,24 @@
 // PFLOP/s at 2,048 rows. This kernel reaches 0.45 to 0.95 on the same shapes; the library's kernels, where they may be
 // used, 0.5 to 1.3.) The reference's engine uses a library product here (x @ W, main_models_new.py:19-20).
 //
-// A workgroup of four waves (2 x 2) owns a tile of 128 rows x 192, 128 or 64 columns, or one of eight waves (2 x 4) a tile
-// of 256 x 256 where that still gives every compute unit a workgroup, and walks K in steps of 64. A step's
+// A workgroup owns a tile of BM rows x BN columns and walks K in steps of 64. A step's
 // operand rows, 128 bytes each, are copied into LDS by global_load_lds_dwordx4 (no registers; eight lanes read one
-// row's 128 bytes), one step ahead of the products, into one of two buffers; two workgroups share a compute unit and
-// fill each other's waits. A row's eight 16-byte pieces lie in LDS with their index XORed by half the row's number:
+// row's 128 bytes) into a ring of NSTAGE buffers, one to three steps ahead of the products. A row's eight 16-byte pieces lie in LDS with their index XORed by half the row's number:
 // an operand fetch reads one piece index of 32 rows, LDS serves sixteen lanes at a time, and sixteen rows of 128
 // bytes are eight such indices at each of two offsets in the 256 bytes that the banks span, so no two of them meet
 // (XORed by the row's number itself, rows r and r + 8 did: half of the LDS's busy cycles were bank conflicts). The
 // copying lane picks the piece that belongs in its slot. The result tile is computed transposed (W's rows are the first operand), so that a
 // lane ends up with four consecutive columns of one row: 8-byte stores, and the residual read the same way.
 // A row's sums run over K in the same order whatever M is: its result does not depend on the other rows.
+//
+// What bounds it: the clock under load (8,192 cubed runs at 1.42 PFLOP/s here: 1.5 us for a step of a 256 x 256 tile on every
+// compute unit), for tiles of 64 x 64 and 128 x 128 the LDS, whose reads and writes take 1.5 to 2 times the products' cycles, and for
+// products of one tile a unit the beginning and end (4 us, and 16 or 32 MB of results at 5 TB/s). Operands are fetched from LDS one
+// or two 16-wide slices ahead of their products (a wave alone on its SIMD waits 230 cycles for four fetches that all waves issue at
+// once, and its products take 128), and a slice's instructions keep a pinned order. Before that (operands fetched where they are
+// used, one step ahead into two buffers) and now, us: 2,048 rows x 2,048 x 2,048 28.0 / 22.7; inner 5,632 62.9 / 48.0; 2,048 x 5,632
+// x 2,048 54.0 / 49.6; 1,800 x 32,000 x 2,048 271 / 247; 1,531 x 2,048 x 2,048 24.1 / 18.2; 300 x 1,024 x 1,024 12.1 / 6.8; 8
+// columns 14.9 / 7.9.
 #include "common.h"
 
 TIS_DEFINE_LAST_ERROR(tis_gemm_tiles)
@@ -56,20 +63,39 @@ template <int ACT> __device__ __forceinline__ float gt_activated(float z) {
   return z;
 }
 
-template <int BM, int BN, int WM, int WN, bool RESIDUAL, typename TO, int ACT = 0>
+template <int V> struct IntC { constexpr operator int() const { return V; } };
+
+// Which tile a workgroup takes. Workgroups go to the eight XCDs in turn, each with an L2 of its own: an XCD gets a run of
+// neighbouring tiles, in an order that walks four rows of tiles side by side, so that what its workgroups read at a time
+// is few rows of X and of W.
+struct GtTile { int m, n; };
+__device__ __forceinline__ GtTile gt_tile(unsigned id, int tiles_m, int tiles_n) {
+  const unsigned total = (unsigned)tiles_m * (unsigned)tiles_n, xcd = id % 8, per = total / 8, more = total % 8;
+  const unsigned t = xcd * per + min(xcd, more) + id / 8;
+  const unsigned band = 4u * (unsigned)tiles_n, g = t / band, in = t - g * band;
+  const unsigned rows = min(4u, (unsigned)tiles_m - g * 4);
+  return {(int)(g * 4 + in % rows), (int)(in / rows)};
+}
+
+// NSTAGE: buffers of LDS; AHEAD: slices of 16 of K that operands are fetched from LDS before their products
+template <int BM, int BN, int WM, int WN, int NSTAGE, int AHEAD, bool RESIDUAL, typename TO, int ACT = 0>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
     const bf16* __restrict__ X, long x_ld, const bf16* __restrict__ W, const bf16* R, long r_ld, TO* C, long c_ld,
     int M, int N, int K, float limit) {
-  constexpr int BK = GT_BK, PCS = GT_PIECES, ROWS = BM + BN, GT_WAVES = WM * WN;
+  constexpr int BK = GT_BK, PCS = GT_PIECES, ROWS = BM + BN, GT_WAVES = WM * WN, KS = BK / 16;
   constexpr int STAGE = ROWS * BK * 2;                  // bytes of a buffer: X's rows, then W's
   constexpr int LPW = ROWS * PCS / 64 / GT_WAVES;       // loads of a step that each wave issues, 8 rows each
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32;   // 32 x 32 result tiles of a wave
-  static_assert(ROWS * PCS % (64 * GT_WAVES) == 0 && TM >= 1 && TN >= 1 && 2 * STAGE <= 160 * 1024, "tile sizes");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * STAGE];
+  static_assert(ROWS * PCS % (64 * GT_WAVES) == 0 && TM >= 1 && TN >= 1 && NSTAGE * STAGE <= 160 * 1024, "tile sizes");
+  constexpr int FLIGHT = AHEAD == 1 ? NSTAGE : NSTAGE - 1;   // steps that are copied ahead
+  constexpr int SETS = AHEAD == 1 ? 2 : KS;             // operand registers: a set a slice, in turn
+  static_assert((AHEAD == 1 || AHEAD == 2) && FLIGHT >= 2 && FLIGHT <= 3 && KS == 4, "what the loop below is written for");
+  static_assert((FLIGHT - 1) * LPW <= 63, "more loads in flight than the counter counts");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[NSTAGE * STAGE];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r32 = lane & 31, h = lane >> 5;
   const int wm = wave / WN, wn = wave % WN;
-  const int tiles_m = (M + BM - 1) / BM;
-  const long m0 = (long)(blockIdx.x % tiles_m) * BM, n0 = (long)(blockIdx.x / tiles_m) * BN;
+  const GtTile tile = gt_tile(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN);
+  const long m0 = (long)tile.m * BM, n0 = (long)tile.n * BN;
   const unsigned lds0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds;
 
   // The wave's loads of a step: load j brings rows 8 (wave * LPW + j) .. +7 of the buffer, lane (row, slot) the piece
@@ -77,32 +103,26 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
   // stored).
   const unsigned char* first_row[LPW];       // of the load's first row, at K offset 0 (the same on all lanes)
   unsigned lane_off[LPW];                    // the lane's piece from there, in bytes
-  int lane_piece[LPW];                       // which 8 elements of a step's 64 the lane brings
 #pragma unroll
   for (int j = 0; j < LPW; ++j) {
     const int row0 = (wave * LPW + j) * 8, row = row0 + (lane >> 3);
-    lane_piece[j] = (lane & 7) ^ ((row >> 1) & 7);
     const bool of_x = row0 < BM;
     const long ld = of_x ? x_ld : (long)K;
     const long last = of_x ? (long)M - 1 : (long)N - 1;
     const long g_first = min(last, of_x ? m0 + row0 : n0 + (row0 - BM));
     const long g_row = min(last, of_x ? m0 + row : n0 + (row - BM));
     first_row[j] = (const unsigned char*)(of_x ? X : W) + g_first * ld * 2;
-    lane_off[j] = (unsigned)((g_row - g_first) * ld * 2 + lane_piece[j] * 16);
+    lane_off[j] = (unsigned)((g_row - g_first) * ld * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16);
   }
-  auto stage = [&](int k0, int buf) {
-#pragma unroll
-    for (int j = 0; j < LPW; ++j)
-      gt_copy16(first_row[j] + (long)k0 * 2, lane_off[j], lds0 + buf * STAGE + (wave * LPW + j) * 1024);
+  const int nk = (K + BK - 1) / BK;
+  const bool ragged = K % BK != 0;                      // the last step's pieces past the end of K come from a block of zeros
+  auto load = [&](int kt, unsigned at, int j) {         // at: where the buffer begins
+    gt_copy16(first_row[j] + (long)kt * (BK * 2), lane_off[j], at + (wave * LPW + j) * 1024);
   };
-  // the last step of a K that is no multiple of 64: pieces past the end come from a block of zeros
-  auto stage_tail = [&](int k0, int buf) {
-#pragma unroll
-    for (int j = 0; j < LPW; ++j) {
-      const bool inside = k0 + lane_piece[j] * 8 < K;
-      const unsigned char* src = inside ? first_row[j] + (long)k0 * 2 + lane_off[j] : gt_zeros;
-      gt_copy16(src, lds0 + buf * STAGE + (wave * LPW + j) * 1024);
-    }
+  auto load_ragged = [&](int kt, unsigned at, int j) {
+    const int row = (wave * LPW + j) * 8 + (lane >> 3);
+    const bool inside = kt * BK + ((lane & 7) ^ ((row >> 1) & 7)) * 8 < K;
+    gt_copy16(inside ? first_row[j] + (long)kt * (BK * 2) + lane_off[j] : gt_zeros, at + (wave * LPW + j) * 1024);
   };
 
   f32x16 acc[TM][TN];
@@ -113,41 +133,85 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  // operand pieces: row r of the buffer, elements 16 ks + 8 h .. of the step, at piece r * 8 + ((2 ks + h) ^ ((r >> 1) & 7))
-  unsigned a_row[TM], b_row[TN];
+  // operand pieces: row r of the buffer, elements 16 ks + 8 h .. of the step, lie at r * 128 + ((2 ks + h) ^ ((r >> 1) & 7)) * 16:
+  // 32 rows on, the same piece; two pieces on (the next ks), the address with bits 5 and 6 changed
+  const unsigned a_row = wm * (BM / WM) + r32, b_row = BM + wn * (BN / WN) + r32;
+  const unsigned a_at = a_row * 128 + ((h ^ ((a_row >> 1) & 7)) * 16), b_at = b_row * 128 + ((h ^ ((b_row >> 1) & 7)) * 16);
+  bf16x8 a[SETS][TM], b[SETS][TN];
+  auto fetch = [&](int ks, unsigned at) {               // at: where the buffer begins, from the first
 #pragma unroll
-  for (int i = 0; i < TM; ++i) a_row[i] = wm * (BM / WM) + i * 32 + r32;
+    for (int i = 0; i < TM; ++i) a[ks % SETS][i] = *(const bf16x8*)(lds + (at + (a_at ^ (ks * 32)) + i * 4096));
 #pragma unroll
-  for (int j = 0; j < TN; ++j) b_row[j] = BM + wn * (BN / WN) + j * 32 + r32;
+    for (int j = 0; j < TN; ++j) b[ks % SETS][j] = *(const bf16x8*)(lds + (at + (b_at ^ (ks * 32)) + j * 4096));
+  };
 
-  const int nk = (K + BK - 1) / BK;
-  const bool tail = K % BK != 0;
-  if (tail && nk == 1) stage_tail(0, 0); else stage(0, 0);
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");      // this wave's pieces of step kt are in LDS
-    __builtin_amdgcn_s_barrier();                             // ... and everyone's; everyone has read step kt - 1
-    if (kt + 1 < nk) {
-      if (tail && kt + 2 == nk) stage_tail((kt + 1) * BK, buf ^ 1);
-      else stage((kt + 1) * BK, buf ^ 1);
+  // The loop. While a slice's products run, the operands of the slice AHEAD of it are on their way out of LDS, also across
+  // steps: AHEAD slices before its end, step kt waits until step kt + 1 is in LDS for every wave (the barrier) and fetches from there.
+  // After that barrier a buffer is free for copies: with AHEAD 2 step kt - 1's, whose last operands every wave has used; with
+  // AHEAD 1 step kt's own, whose last operands every wave has in registers, because it waited for them too. Each gives FLIGHT
+  // steps that are under way. The order of a slice's instructions is pinned: the first product, the LDS reads, the other products with
+  // the copies between them, so that a wave that has its SIMD to itself keeps the matrix core busy while it issues them.
+  // MODE 0: copies a whole step; 1: the ragged last one; 2: none. LEFT: the steps beyond the next that are under way meanwhile.
+  unsigned at = 0, prev = (NSTAGE - 1) * STAGE;
+  auto step = [&](int kt, auto mode, auto left, auto last) {
+    constexpr int MODE = mode, LEFT = left;
+    constexpr bool LAST = last;
+    const unsigned next = at + STAGE == NSTAGE * STAGE ? 0 : at + STAGE;
+    const unsigned into = lds0 + (AHEAD == 1 ? at : prev);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      if (ks == KS - AHEAD && !LAST) {
+        if (AHEAD == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LEFT * LPW) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(LEFT * LPW) : "memory");
+      }
+#pragma unroll
+      for (int m = 0; m < TM * TN; ++m) {
+        acc[m / TN][m % TN] =
+            __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[ks % SETS][m % TN], a[ks % SETS][m / TN], acc[m / TN][m % TN], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (m == 0) {
+          if (ks + AHEAD < KS) fetch(ks + AHEAD, at);
+          else if (!LAST) fetch(ks + AHEAD - KS, next);
+        }
+        if (MODE < 2 && ks >= KS - AHEAD) {
+          constexpr int SLOTS = AHEAD * TM * TN;
+          const int slot = (ks - (KS - AHEAD)) * TM * TN + m;
+#pragma unroll
+          for (int j = slot * LPW / SLOTS; j < (slot + 1) * LPW / SLOTS; ++j) {
+            if (MODE == 0) load(kt + FLIGHT, into, j);
+            else load_ragged(kt + FLIGHT, into, j);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
-    const unsigned char* st = lds + buf * STAGE;
+    prev = at;
+    at = next;
+  };
+  const int whole = ragged ? nk - 1 : nk;
 #pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      bf16x8 a[TM], b[TN];
+  for (int s = 0; s < FLIGHT; ++s) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-        a[i] = *(const bf16x8*)(st + (a_row[i] * PCS + ((2 * ks + h) ^ ((a_row[i] >> 1) & 7))) * 16);
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        b[j] = *(const bf16x8*)(st + (b_row[j] * PCS + ((2 * ks + h) ^ ((b_row[j] >> 1) & 7))) * 16);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+    for (int j = 0; j < LPW; ++j) {
+      if (s < whole) load(s, lds0 + s * STAGE, j);
+      else if (s < nk) load_ragged(s, lds0 + s * STAGE, j);
     }
   }
+  if (nk >= FLIGHT) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((FLIGHT - 1) * LPW) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" : : : "memory");
+#pragma unroll
+  for (int ks = 0; ks < AHEAD; ++ks) fetch(ks, 0);
+  int kt = 0;
+  for (; kt + FLIGHT < whole; ++kt) step(kt, IntC<0>{}, IntC<FLIGHT - 2>{}, IntC<0>{});
+  if (kt + FLIGHT < nk) {
+    step(kt, IntC<1>{}, IntC<FLIGHT - 2>{}, IntC<0>{});
+    ++kt;
+  }
+  // the last steps, whose copies are all under way
+  if constexpr (FLIGHT == 3)
+    if (nk >= 3) step(kt++, IntC<2>{}, IntC<1>{}, IntC<0>{});
+  if (nk >= 2) step(kt++, IntC<2>{}, IntC<0>{}, IntC<0>{});
+  step(kt, IntC<2>{}, IntC<0>{}, IntC<1>{});
 
   // accumulator 4 q + e of block (i, j): row m0 + wm * (BM / WM) + i * 32 + r32, column n0 + wn * (BN / WN) + j * 32 + 8 q + 4 h + e
 #pragma unroll
@@ -208,34 +272,45 @@ TIS_EXPORT int tis_gemm_tiles(const void* X, long x_ld, const void* W, const voi
   if (act < 0 || act > 3 || (act && (out_f32 || R))) return tis_fail("gemm_tiles: an activation (%d) goes with a plain bfloat16 result", act);
   if (out_f32 && R) return tis_fail("gemm_tiles: a 32-bit result takes no residual");
   if ((long)x_ld * 16 >= (1L << 31) || (long)K * 16 >= (1L << 31)) return tis_fail("gemm_tiles: rows of %ld elements are too long for 32-bit offsets", x_ld);
-  // The tile: 256 x 256 on eight waves where that gives every compute unit a workgroup (it moves half the bytes into
-  // LDS per product that 128 x 128 does: 2,048 x 8,192 x 1,536 at 0.92 instead of 0.84 PFLOP/s); else 128 x 128 on
-  // four; 128 x 64 where 128 x 128 would leave compute units without a workgroup or with one alone. Two workgroups share a
-  // unit (three of 128 x 64): where tiles of 128 columns would take a further, mostly empty round, tiles of 192 may end in one round less
-  // (2,048 rows and 2,048 inner columns, us: 5,120 columns 128: 77, 192: 59, 256: 66; 5,632: 76, 60, 63; but 2,816: 43, 43, 58).
-  const long big = (long)((M + 255) / 256) * ((N + 255) / 256), mid = (long)((M + 127) / 128) * ((N + 127) / 128);
-  const long rounds128 = (mid + 2 * g_units - 1) / (2 * g_units);
-  const long rounds192 = ((long)((M + 127) / 128) * ((N + 191) / 192) + 2 * g_units - 1) / (2 * g_units);
-  const int bm = big >= g_units ? 256 : 128;
-  const int bn = big >= g_units ? 256 : mid <= g_units ? 64 : 3 * rounds192 < 2 * rounds128 ? 192 : 128;
-  const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-  if (tiles >= (1L << 31)) return tis_fail("gemm_tiles: %ld tiles are more than a grid holds", tiles);
-#define LAUNCH(BMV, BNV, WMV, WNV, RV, TOV, ACTV)                                                          \
-  gemm_tiles_kernel<BMV, BNV, WMV, WNV, RV, TOV, ACTV><<<dim3((unsigned)tiles), WMV * WNV * 64, 0, stream>>>(    \
-      (const bf16*)X, x_ld, (const bf16*)W, (const bf16*)R, r_ld, (TOV*)C, c_ld, M, N, K, limit)
-#define PICK(BMV, BNV, WMV, WNV)                                \
-  {                                                             \
-    if (out_f32) LAUNCH(BMV, BNV, WMV, WNV, false, float, 0);   \
-    else if (R) LAUNCH(BMV, BNV, WMV, WNV, true, bf16, 0);      \
-    else if (act == 1) LAUNCH(BMV, BNV, WMV, WNV, false, bf16, 1); \
-    else if (act == 2) LAUNCH(BMV, BNV, WMV, WNV, false, bf16, 2); \
-    else if (act == 3) LAUNCH(BMV, BNV, WMV, WNV, false, bf16, 3); \
-    else LAUNCH(BMV, BNV, WMV, WNV, false, bf16, 0);            \
+  // The tile: the one that is estimated to end first, by the microseconds a step of 64 takes with one or more workgroups a
+  // compute unit (measured at K of 1,408 to 5,632; the clock falls as more of the chip works, hence 1.36 to 1.85 for the largest):
+  //   256 x 256, eight waves, two buffers    1.36 up to 0.7 workgroups a unit, then to 1.72 at one; 1.85 a full round
+  //   128 x 192, four waves, two buffers     0.79 up to one a unit, two share one: 0.79 for each on average
+  //   128 x 128, eight waves, four buffers   0.47, and 0.6 a further round
+  //   64 x 64, four waves, four buffers      0.21 up to one a unit, two share one: 0.21 for each on average
+  // (us, 256 / 192 / 128 / 64, 2,048 inner columns: 2,048 x 2,048 48.4, 31.4, 22.7, 30.5; 2,048 x 2,816 47.0, 31.3, 33.0, 39.2;
+  // 2,048 x 5,120 49.0, 48.6, 51.9, 66.5; 1,800 x 8,192 62.8, 71.3, 70.8, 98.2; 1,536 x 11,264 102.9, 75.1, 84.9, 110.0;
+  // 1,800 x 32,000 247, 280, 333, 420; 700 x 1,024 x 2,816 59.4, 37.4, 20.6, 13.8.)
+  struct { int bm, bn; } const shapes[4] = {{256, 256}, {128, 192}, {128, 128}, {64, 64}};
+  int pick = 0;
+  float best = 0.f;
+  long tiles = 0;
+  for (int i = 0; i < 4; ++i) {
+    const long n = (long)((M + shapes[i].bm - 1) / shapes[i].bm) * ((N + shapes[i].bn - 1) / shapes[i].bn);
+    const float r = (float)n / g_units, full = floorf(r), part = r - full;
+    float t;
+    if (i == 0) t = 1.85f * full + (part > 0.f ? fmaxf(1.36f, 1.36f + 1.2f * (part - 0.7f)) : 0.f);
+    else if (i == 2) t = 0.47f + 0.6f * (ceilf(r) - 1.f);
+    else t = (i == 1 ? 0.79f : 0.21f) * fmaxf(r, 1.f);
+    if (i == 0 || t < best) best = t, pick = i, tiles = n;
   }
-  if (bm == 256) PICK(256, 256, 2, 4)
-  else if (bn == 192) PICK(128, 192, 2, 2)
-  else if (bn == 128) PICK(128, 128, 2, 2)
-  else PICK(128, 64, 2, 2)
+  if (tiles >= (1L << 31)) return tis_fail("gemm_tiles: %ld tiles are more than a grid holds", tiles);
+#define LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, RV, TOV, ACTV)                                                     \
+  gemm_tiles_kernel<BMV, BNV, WMV, WNV, NSV, AHV, RV, TOV, ACTV><<<dim3((unsigned)tiles), WMV * WNV * 64, 0, stream>>>(    \
+      (const bf16*)X, x_ld, (const bf16*)W, (const bf16*)R, r_ld, (TOV*)C, c_ld, M, N, K, limit)
+#define PICK(BMV, BNV, WMV, WNV, NSV, AHV)                                     \
+  {                                                                             \
+    if (out_f32) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, float, 0);   \
+    else if (R) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, true, bf16, 0);      \
+    else if (act == 1) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 1); \
+    else if (act == 2) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 2); \
+    else if (act == 3) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 3); \
+    else LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 0);            \
+  }
+  if (pick == 0) PICK(256, 256, 2, 4, 2, 1)
+  else if (pick == 1) PICK(128, 192, 2, 2, 2, 1)
+  else if (pick == 2) PICK(128, 128, 2, 4, 4, 2)
+  else PICK(64, 64, 2, 2, 4, 2)
 #undef PICK
 #undef LAUNCH
   return tis_launch_status("gemm_tiles");
