@@ -988,3 +988,63 @@ def test_tiled_product_of_few_steps_of_each_tile(ops_for, M, N, K):
     assert torch.equal(ops.linear(x, w), got.to(torch.bfloat16))
     gate, up = got[:, 0::2].clamp(max=7.0), got[:, 1::2].clamp(-7.0, 7.0)
     torch.testing.assert_close(ops.linear_gated(x, w, 7.0).float(), gate * torch.sigmoid(1.702 * gate) * (up + 1.0), rtol=5e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("groups,line,N,K,counts", [
+    (8, 2048, 2048, 72, "even"),            # 4,096 entries: tiles of 192 columns
+    (8, 1000, 5632, 264, "even"),           # 256 x 256
+    (8, 500, 2044, 520, "uneven"),          # 128 x 128, a workgroup a unit
+    (8, 129, 5636, 256, "uneven"),          # 128 x 128, two a unit
+    (8, 30, 1024, 320, "uneven"), (3, 24, 60, 64, "one"), (130, 40, 132, 200, "uneven"),   # 64 x 64; more groups than lanes
+])
+@pytest.mark.parametrize("out32,act", [(True, 0), (False, 2)])
+def test_grouped_product_in_tiles_numbered_through(ops_for, groups, line, N, K, counts, out32, act):
+    """Every tile of the grouped product of many entries: groups that are empty, hold one entry, end inside a tile or hold every
+    row; entries that no list names stay as they were. 32-bit sums against 64 bits, the gate against the sums."""
+    from tiny_inference_server_amd.ops.hip_ops import _ptr
+    ops = ops_for(torch.bfloat16)
+    g = torch.Generator().manual_seed(groups * N + K)
+    share = {"even": [line // 4] * groups, "one": [0] * (groups - 1) + [line],
+             "uneven": [0, 1, line] + [int(v) for v in torch.randint(0, line // 2 + 1, (max(0, groups - 3),), generator=g)]}[counts][:groups]
+    entries = line * 2                       # as a router that takes two gives them
+    lists, cnt = torch.zeros(groups, line, dtype=torch.int32), torch.tensor(share, dtype=torch.int32)
+    for e, n in enumerate(share):
+        lists[e, :n] = torch.randperm(entries, generator=g)[:n].sort().values.to(torch.int32)
+    lists, cnt = lists.cuda(), cnt.cuda()
+    x, w = rnd((line, K + 8), torch.bfloat16, 801).cuda()[:, :K], rnd((groups, N, K), torch.bfloat16, 802, K ** -0.5).cuda()
+    for e in range(groups):                  # an entry is one group's: the groups are run one by one against what they write
+        one = torch.zeros_like(cnt)
+        one[e] = cnt[e]
+        if share[e] == 0 and e:
+            continue
+        out = torch.full((entries, N // 2 if act else N), 7.5, device="cuda", dtype=torch.float32 if out32 else torch.bfloat16)
+        ops._lazy("experts").tis_grouped_linear(1, 0 if out32 else 1, _ptr(x), x.stride(0), 0, 2, _ptr(w), _ptr(out), out.shape[1], 0,
+                                                _ptr(lists), _ptr(one), line, groups, line, entries, N, K, act, None, 0, 7.0, ops._stream())
+        at = lists[e, :share[e]].long()
+        rows = x[at // 2].double()
+        want = rows @ w[e].double().T
+        if act:
+            gate, up = want[:, 0::2].clamp(max=7.0), want[:, 1::2].clamp(-7.0, 7.0)
+            torch.testing.assert_close(out[at].double(), gate * torch.sigmoid(1.702 * gate) * (up + 1.0), rtol=8e-3, atol=2e-3)
+        else:
+            bound = (K + 2) * 2.0 ** -24 * (rows.abs() @ w[e].double().abs().T)
+            assert ((out[at].double() - want).abs() <= bound).all()
+        rest = torch.ones(entries, dtype=torch.bool, device="cuda")
+        rest[at] = False
+        assert (out[rest] == 7.5).all()
+        if groups > 8 and e > 4:
+            break
+    # all groups together give what they gave alone where no later group writes
+    if counts == "even" and groups * share[0] <= entries:
+        perm = torch.randperm(entries, generator=g)[:groups * share[0]].view(groups, -1).sort(-1).values.to(torch.int32).cuda()
+        lists[:, :share[0]] = perm
+        out = torch.full((entries, N // 2 if act else N), 7.5, device="cuda", dtype=torch.float32 if out32 else torch.bfloat16)
+        ops._lazy("experts").tis_grouped_linear(1, 0 if out32 else 1, _ptr(x), x.stride(0), 0, 2, _ptr(w), _ptr(out), out.shape[1], 0,
+                                                _ptr(lists), _ptr(cnt), line, groups, line, entries, N, K, act, None, 0, 7.0, ops._stream())
+        for e in range(groups):
+            want = x[perm[e].long() // 2].double() @ w[e].double().T
+            if not act:
+                assert (out[perm[e].long()].double() - want).abs().max() < 1e-4
+            else:
+                gate, up = want[:, 0::2].clamp(max=7.0), want[:, 1::2].clamp(-7.0, 7.0)
+                torch.testing.assert_close(out[perm[e].long()].double(), gate * torch.sigmoid(1.702 * gate) * (up + 1.0), rtol=8e-3, atol=2e-3)

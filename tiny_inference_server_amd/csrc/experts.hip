@@ -16,12 +16,9 @@
 // product), with a_div = 1 both lie by assignment (its second); without lists every group takes all rows, and a_group /
 // c_group move from one group's columns to the next (a product per head on a head's own columns). Sums are 32-bit in
 // an order that depends on K alone, so a row's result does not depend on what else is in the step.
-#include "common.h"
+#include "tile_loop.h"
 
 TIS_DEFINE_LAST_ERROR(tis_experts)
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 static constexpr int EX_MAX_PER_LANE = 16;      // router outputs a lane keeps: up to 1,024 outputs a row
 
@@ -228,7 +225,7 @@ __global__ __launch_bounds__(256) void grouped_plain_kernel(const TA* __restrict
 // straight from memory, 16 bytes a lane (rows 16-byte aligned, K a multiple of 8); a wave's RM + RN loads of a step feed
 // RM RN products, and what the waves of a workgroup share meets in the caches. Each result is one wave's sum over K in
 // steps of 32. Two shapes are built: 16 entries x 64 columns for groups of a few rows (decoded tokens: the job is to
-// stream the matrices once), 64 x 128 for groups of many.
+// stream the matrices once), 64 x 128 for groups of many that the tiles below do not take.
 template <typename TO, int WM, int WN, int RM, int RN>
 __global__ __launch_bounds__(256) void grouped_mfma_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                            TO* __restrict__ C, GroupedArgs p) {
@@ -308,59 +305,85 @@ __global__ __launch_bounds__(256) void grouped_mfma_kernel(const bf16* __restric
   }
 }
 
-// Groups of many rows: the same product tiled in both directions on v_mfma_f32_32x32x16_bf16 with both operands
-// through LDS, as the tiled product for many rows does it (gemm_tiles.hip: direct loads into LDS one step of 64 ahead,
-// two buffers, a row's eight 16-byte pieces XORed by half the row's number against bank conflicts, the tile computed
-// transposed so that a lane ends up with four consecutive columns). What differs: a tile's rows are list entries, each
-// with an address of its own for reading and for writing, the matrix is the group's, a tile past the group's count
-// leaves at once, and the epilogue may apply the activation. 128 entries x BN columns, four waves.
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-static __device__ __attribute__((aligned(16))) unsigned char ex_zeros[16];
-
-#pragma clang diagnostic ignored "-Winline-asm"   // M0 in a clobber list: meant
-__device__ __forceinline__ void ex_copy16(const void* lane_src, unsigned lds_addr) {
-  const unsigned base = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_addr);
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(lane_src), "s"(base) : "memory", "m0");
-}
-
-template <typename TO, int BN>
-__global__ __launch_bounds__(256) void grouped_tiles_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
-                                                            TO* __restrict__ C, GroupedArgs p) {
-  constexpr int BM = 128, WN = 2, BK = 64, PCS = 8, ROWS = BM + BN, WAVES = 4;
-  constexpr int STAGE = ROWS * BK * 2;                  // bytes of a buffer: the entries' rows, then the matrix's
-  constexpr int LPW = ROWS * PCS / 64 / WAVES;          // loads of a step that each wave issues, 8 rows each
-  constexpr int TM = 2, TN = BN / 64;                   // 32 x 32 result tiles of a wave
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * STAGE];
-  const int g = blockIdx.z;
-  const int count = p.lists ? p.counts[g] : p.rows;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  if (m0 >= count) return;
+// Groups of many rows: the same product tiled in both directions with both operands through LDS, by the loop of the tiled product
+// (tile_loop.h). What differs: a tile's rows are list entries, each with an address of its own for reading and for writing,
+// the matrix is the group's, and the epilogue may apply the activation. A grid row of tiles per group would be as tall as the
+// largest group could be, and most of its workgroups would leave at once; here the row tiles of all groups are numbered through,
+// and a workgroup finds its group from the groups' counts (a lane a group, 64 at a time). us, 8 groups, before (4,096 entries: tiles
+// of 128 x 128 or 64 in a grid as tall as a group; fewer: 64 x 128 straight from memory) / now: 5,632 columns of 2,048, 4,096 entries
+// 162 / 133, 2,000 301 / 101, 1,000 322 / 73, 260 115 / 53; 2,048 of 2,816 93 / 74, 185 / 47, 176 / 28, 73 / 20.
+template <typename TO, int BM, int BN, int WM, int WN, int NSTAGE, int AHEAD>
+__global__ __launch_bounds__(WM * WN * 64) void grouped_tiles_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
+                                                                     TO* __restrict__ C, GroupedArgs p, int groups) {
+  typedef TileLoop<BM, BN, WM, WN, NSTAGE, AHEAD> Loop;
+  constexpr int LPW = Loop::LPW, TM = Loop::TM, TN = Loop::TN;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[NSTAGE * Loop::STAGE];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r32 = lane & 31, h = lane >> 5;
   const int wm = wave / WN, wn = wave % WN;
-  const unsigned lds0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds;
+  // row tiles of all groups, and then this workgroup's tile and group
+  int tiles_m = 0;
+  if (p.lists) {
+    for (int g0 = 0; g0 < groups; g0 += 64) {
+      int n = g0 + lane < groups ? (p.counts[g0 + lane] + BM - 1) / BM : 0;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) n += __shfl_xor(n, o, 64);
+      tiles_m += n;
+    }
+  } else {
+    tiles_m = groups * ((p.rows + BM - 1) / BM);
+  }
+  tiles_m = __builtin_amdgcn_readfirstlane(tiles_m);
+  const int tiles_n = (p.N + BN - 1) / BN;
+  if (blockIdx.x >= (unsigned)tiles_m * (unsigned)tiles_n) return;
+  const GtTile tile = gt_tile(blockIdx.x, tiles_m, tiles_n);
+  int g = 0, before = 0;                                // the group, and the row tiles before it
+  if (p.lists) {
+    for (int g0 = 0; g0 < groups; g0 += 64) {
+      int upto = g0 + lane < groups ? (p.counts[g0 + lane] + BM - 1) / BM : 0;
+      const int own = upto;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(upto, o, 64);
+        if (lane >= o) upto += v;
+      }
+      const unsigned long long holds = __ballot(before + upto > tile.m);
+      if (holds) {
+        const int at = __ffsll(holds) - 1;
+        g = g0 + at;
+        before += __shfl(upto - own, at, 64);
+        break;
+      }
+      before += __shfl(upto, 63, 64);
+    }
+  } else {
+    const int per = (p.rows + BM - 1) / BM;
+    g = tile.m / per;
+    before = g * per;
+  }
+  g = __builtin_amdgcn_readfirstlane(g);
+  const int m0 = (tile.m - __builtin_amdgcn_readfirstlane(before)) * BM, n0 = tile.n * BN;
+  const int count = p.lists ? p.counts[g] : p.rows;
   const bf16* Wg = W + (long)g * p.N * p.K;
+  const bf16* Ag = A + (long)g * p.a_group;
   auto entry = [&](int m) {                             // the list entry of the tile's row m (the last one again past the count)
     const int e = min(m0 + m, count - 1);
     return p.lists ? p.lists[(long)g * p.line + e] : e;
   };
-  const unsigned char* lane_src[LPW];                   // the lane's piece of its row at K offset 0
-  int lane_piece[LPW];
+  const unsigned char* first[LPW];
+  unsigned lane_off[LPW];                               // (the host has seen that they fit)
 #pragma unroll
   for (int j = 0; j < LPW; ++j) {
-    const int row = (wave * LPW + j) * 8 + (lane >> 3);
-    lane_piece[j] = (lane & 7) ^ ((row >> 1) & 7);
-    const bf16* src = row < BM ? A + (long)(entry(row) / p.a_div) * p.lda + (long)g * p.a_group
-                               : Wg + (long)min(p.N - 1, n0 + row - BM) * p.K;
-    lane_src[j] = (const unsigned char*)src + lane_piece[j] * 16;
-  }
-  auto stage = [&](int k0, int buf) {
-#pragma unroll
-    for (int j = 0; j < LPW; ++j) {
-      const bool inside = k0 + lane_piece[j] * 8 < p.K;
-      ex_copy16(inside ? lane_src[j] + (long)k0 * 2 : ex_zeros, lds0 + buf * STAGE + (wave * LPW + j) * 1024);
+    const int row0 = Loop::row_of(wave, 0, j), row = Loop::row_of(wave, lane, j);
+    if (row0 < BM) {
+      first[j] = (const unsigned char*)Ag;
+      lane_off[j] = (unsigned)(entry(row) / p.a_div) * (unsigned)(p.lda * 2);
+    } else {
+      const int r0 = min(p.N - 1, n0 + row0 - BM), r = min(p.N - 1, n0 + row - BM);
+      first[j] = (const unsigned char*)(Wg + (long)r0 * p.K);
+      lane_off[j] = (unsigned)((r - r0) * p.K * 2);
     }
-  };
+    lane_off[j] += Loop::piece_of(lane, row) * 16;
+  }
   f32x16 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -368,46 +391,19 @@ __global__ __launch_bounds__(256) void grouped_tiles_kernel(const bf16* __restri
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  unsigned a_row[TM], b_row[TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i) a_row[i] = wm * 64 + i * 32 + r32;
-#pragma unroll
-  for (int j = 0; j < TN; ++j) b_row[j] = BM + wn * (BN / 2) + j * 32 + r32;
-  const int nk = (p.K + BK - 1) / BK;
-  stage(0, 0);
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");      // this wave's pieces of step kt are in LDS
-    __builtin_amdgcn_s_barrier();                             // ... and everyone's; everyone has read step kt - 1
-    if (kt + 1 < nk) stage((kt + 1) * BK, buf ^ 1);
-    const unsigned char* st = lds + buf * STAGE;
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      bf16x8 a[TM], b[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        a[i] = *(const bf16x8*)(st + (a_row[i] * PCS + ((2 * ks + h) ^ ((a_row[i] >> 1) & 7))) * 16);
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        b[j] = *(const bf16x8*)(st + (b_row[j] * PCS + ((2 * ks + h) ^ ((b_row[j] >> 1) & 7))) * 16);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
-    }
-  }
-  // accumulator 4 q + e of block (i, j): entry wm * 64 + i * 32 + r32 of the tile, column n0 + wn * (BN / 2) + j * 32 + 8 q + 4 h + e
+  Loop::run(lds, first, lane_off, p.K, acc);
+
+  // accumulator 4 q + e of block (i, j): entry wm * (BM / WM) + i * 32 + r32 of the tile, column n0 + wn * (BN / WN) + j * 32 + 8 q + 4 h + e
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int m = wm * 64 + i * 32 + r32;
+    const int m = wm * (BM / WM) + i * 32 + r32;
     if (m0 + m >= count) continue;
     TO* dst = C + (long)entry(m) * p.ldc + (long)g * p.c_group;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int n = n0 + wn * (BN / 2) + j * 32 + q * 8 + h * 4;
+        const int n = n0 + wn * (BN / WN) + j * 32 + q * 8 + h * 4;
         if (n >= p.N) continue;               // (N is a multiple of 4: the four columns are inside or outside together)
         if (p.act == 2) {
           const float a0 = clamped_swish(acc[i][j][q * 4], acc[i][j][q * 4 + 1], p.limit);
@@ -498,17 +494,47 @@ TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, lo
     // what a lane stores four columns at a time must be aligned for it
     const int oa = out_dtype == TIS_BF16 ? 8 : 16;
     const bool wide_ok = aligned && N % 4 == 0 && ldc % 4 == 0 && c_group % 4 == 0 && ((uintptr_t)C % oa) == 0 && K >= 64;
-    if (wide_ok && most_rows >= 128 * (lists ? groups : 1)) {
-      // groups of many rows (with lists: if the rows were spread evenly): 128 entries x 128 columns through LDS
-      // (64 columns where tiles of 128 would end in a second round of workgroups that leaves most of the chip idle; with lists
-      // a group is taken to have begun half a tile more than its even share of the entries)
-      const long tiles = (long)((N + 127) / 128) * (lists ? most_entries / 128 + groups / 2 : (long)groups * ((most_rows + 127) / 128));
-      const int bn = tiles < 4 * 256 ? 64 : 128;
-      dim3 big((N + bn - 1) / bn, (most_rows + 127) / 128, groups);
-      if (big.y > 65535) return tis_fail("grouped_linear: %d rows are too many for one call", most_rows);
-#define TILES(TO, BN) grouped_tiles_kernel<TO, BN><<<big, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (TO*)C, p)
-      if (out_dtype == TIS_BF16) { if (bn == 64) TILES(bf16, 64); else TILES(bf16, 128); }
-      else { if (bn == 64) TILES(float, 64); else TILES(float, 128); }
+    // an entry's row lies within 32 bits of the group's first, and so does a tile's last matrix row of its first
+    const bool near = ((lists ? most_entries : most_rows) / a_div + 1) * (lda * 2) < (1L << 32) && (long)K * 512 < (1L << 31);
+    if (wide_ok && near && (lists ? most_entries >= 48 : most_rows >= 64)) {
+      // From 48 list entries, or 64 rows of every group, on (8 groups of 5,632 columns and 2,048 inner ones, us, 16 x 64 straight from
+      // memory / tiles: 32 entries 43.7 / 50.8, 48 53.7 / 50.7, 64 55.5 / 50.7, 128 88 / 55; 2,048 of 2,816: 19.6 / 19.3, 32.4 / 19.5,
+      // 35.4 / 19.5, 79.5 / 19.7; without lists, 16 groups of 512 of 128: 48 rows 4.4 / 4.7, 64 8.7 / 4.8). The tile that is estimated to end first, by the microseconds a step of 64 takes with r workgroups
+      // a compute unit. With lists, entries / bm row tiles and half a tile more in every group.
+      //   128 x 192, four waves, two buffers, two a unit     1.05 r, at least 1.15
+      //   64 x 64, four waves, four buffers, two a unit      0.3 r, at least 0.33
+      //   128 x 128, eight waves, four buffers               0.58 a round
+      //   256 x 256, eight waves, two buffers                1.85 a round
+      //   128 x 128, four waves, two buffers, two a unit     0.78 r, at least 0.8
+      struct Shape { int bm, bn; float step, least; bool rounds; };
+      static const Shape shapes[5] = {{128, 192, 1.05f, 1.15f, false}, {64, 64, 0.3f, 0.33f, false}, {128, 128, 0.58f, 0.58f, true},
+                                      {256, 256, 1.85f, 1.85f, true}, {128, 128, 0.78f, 0.8f, false}};
+      int pick = 0;
+      float best = INFINITY;
+      for (int i = 0; i < 5; ++i) {
+        if (K < 256 && i != 1 && i != 4) continue;     // few steps: what counts is a tile's beginning and end (2,048 rows, 16 groups
+        const Shape& q = shapes[i];                    // of 512 of 128: 24 us in tiles of 128 x 128, 33 in 256 x 256)
+        const long tn = (N + q.bn - 1) / q.bn;
+        const float r = (lists ? (float)most_entries / q.bm + 0.5f * groups : (float)((long)groups * ((most_rows + q.bm - 1) / q.bm))) * tn / 256.f;
+        const float t = fmaxf(q.least, q.step * (q.rounds ? ceilf(r) : r));
+        if (t < best) best = t, pick = i;
+      }
+      // the most row tiles there can be: the entries' own, and one that is begun in every group
+      const int bm = shapes[pick].bm, bn = shapes[pick].bn;
+      const long tiles = (lists ? most_entries / bm + groups : (long)groups * ((most_rows + bm - 1) / bm)) * ((N + bn - 1) / bn);
+      if (tiles >= (1L << 31)) return tis_fail("grouped_linear: %ld tiles are more than a grid holds", tiles);
+#define TILES(BM, BN, WM, WN, NS, AH)                                                                                     \
+  {                                                                                                                       \
+    if (out_dtype == TIS_BF16) grouped_tiles_kernel<bf16, BM, BN, WM, WN, NS, AH><<<dim3((unsigned)tiles), WM * WN * 64, 0, stream>>>(  \
+        (const bf16*)A, (const bf16*)W, (bf16*)C, p, groups);                                                             \
+    else grouped_tiles_kernel<float, BM, BN, WM, WN, NS, AH><<<dim3((unsigned)tiles), WM * WN * 64, 0, stream>>>(                       \
+        (const bf16*)A, (const bf16*)W, (float*)C, p, groups);                                                            \
+  }
+      if (pick == 0) TILES(128, 192, 2, 2, 2, 1)
+      else if (pick == 1) TILES(64, 64, 2, 2, 4, 2)
+      else if (pick == 2) TILES(128, 128, 2, 4, 4, 2)
+      else if (pick == 3) TILES(256, 256, 2, 4, 2, 1)
+      else TILES(128, 128, 2, 2, 2, 1)
 #undef TILES
     } else if (aligned && most_rows >= 64 * (lists ? groups : 1)) {
       // 64 entries x 128 columns a workgroup, operands straight from memory

@@ -4,55 +4,13 @@
 // PFLOP/s at 2,048 rows. This kernel reaches 0.45 to 0.95 on the same shapes; the library's kernels, where they may be
 // used, 0.5 to 1.3.) The reference's engine uses a library product here (x @ W, main_models_new.py:19-20).
 //
-// A workgroup owns a tile of BM rows x BN columns and walks K in steps of 64. A step's
-// operand rows, 128 bytes each, are copied into LDS by global_load_lds_dwordx4 (no registers; eight lanes read one
-// row's 128 bytes) into a ring of NSTAGE buffers, one to three steps ahead of the products. A row's eight 16-byte pieces lie in LDS with their index XORed by half the row's number:
-// an operand fetch reads one piece index of 32 rows, LDS serves sixteen lanes at a time, and sixteen rows of 128
-// bytes are eight such indices at each of two offsets in the 256 bytes that the banks span, so no two of them meet
-// (XORed by the row's number itself, rows r and r + 8 did: half of the LDS's busy cycles were bank conflicts). The
-// copying lane picks the piece that belongs in its slot. The result tile is computed transposed (W's rows are the first operand), so that a
-// lane ends up with four consecutive columns of one row: 8-byte stores, and the residual read the same way.
-// A row's sums run over K in the same order whatever M is: its result does not depend on the other rows.
-//
-// What bounds it: the clock under load (8,192 cubed runs at 1.42 PFLOP/s here: 1.5 us for a step of a 256 x 256 tile on every
-// compute unit), for tiles of 64 x 64 and 128 x 128 the LDS, whose reads and writes take 1.5 to 2 times the products' cycles, and for
-// products of one tile a unit the beginning and end (4 us, and 16 or 32 MB of results at 5 TB/s). Operands are fetched from LDS one
-// or two 16-wide slices ahead of their products (a wave alone on its SIMD waits 230 cycles for four fetches that all waves issue at
-// once, and its products take 128), and a slice's instructions keep a pinned order. Before that (operands fetched where they are
-// used, one step ahead into two buffers) and now, us: 2,048 rows x 2,048 x 2,048 28.0 / 22.7; inner 5,632 62.9 / 48.0; 2,048 x 5,632
-// x 2,048 54.0 / 49.6; 1,800 x 32,000 x 2,048 271 / 247; 1,531 x 2,048 x 2,048 24.1 / 18.2; 300 x 1,024 x 1,024 12.1 / 6.8; 8
-// columns 14.9 / 7.9.
-#include "common.h"
+// tile_loop.h holds the loop. A row's sums run over K in the same order whatever M is: its result does not depend on the other rows.
+// With operands fetched where they are used and copies one step ahead (before) and as the loop is now, us: 2,048 rows x 2,048 x 2,048
+// 28.0 / 22.7; inner 5,632 62.9 / 48.0; 2,048 x 5,632 x 2,048 54.0 / 49.6; 1,800 x 32,000 x 2,048 271 / 247; 1,531 x 2,048 x 2,048
+// 24.1 / 18.2; 300 x 1,024 x 1,024 12.1 / 6.8; 8 columns 14.9 / 7.9.
+#include "tile_loop.h"
 
 TIS_DEFINE_LAST_ERROR(tis_gemm_tiles)
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
-static constexpr int GT_BK = 64, GT_PIECES = GT_BK / 8;
-
-// what lanes past the end of K read in the last step: zeros
-static __device__ __attribute__((aligned(16))) unsigned char gt_zeros[16];
-
-#pragma clang diagnostic ignored "-Winline-asm"   // M0 in a clobber list: meant
-// One 16-byte piece per lane from global memory straight into LDS: lane i's piece lands at lds_addr + 16 * i. In
-// assembly, because the compiler would order every later LDS read behind such a load, whichever buffer it reads; so
-// the compiler does not count these loads either, and whoever reads the pieces waits for them (vmcnt) and for the
-// other waves (barrier).
-__device__ __forceinline__ void gt_copy16(const void* scalar_src, unsigned lane_bytes, unsigned lds_addr) {
-  const uint64_t a = (uint64_t)scalar_src;
-  const uint64_t sc = ((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) |
-                      (unsigned)__builtin_amdgcn_readfirstlane((int)a);
-  const unsigned base = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_addr);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_bytes), "s"(sc), "s"(base) : "memory", "m0");
-}
-// the same with every lane's own address
-__device__ __forceinline__ void gt_copy16(const void* lane_src, unsigned lds_addr) {
-  const unsigned base = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_addr);
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(lane_src), "s"(base) : "memory", "m0");
-}
 
 // BM x BN: the workgroup's tile; WM x WN: its waves, each with (BM / WM) x (BN / WN) of it
 // ACT: what becomes of a sum before it is rounded (0 nothing; 1 the tanh form of gelu, 0.5 z (1 + tanh(u)) written as
@@ -63,68 +21,32 @@ template <int ACT> __device__ __forceinline__ float gt_activated(float z) {
   return z;
 }
 
-template <int V> struct IntC { constexpr operator int() const { return V; } };
-
-// Which tile a workgroup takes. Workgroups go to the eight XCDs in turn, each with an L2 of its own: an XCD gets a run of
-// neighbouring tiles, in an order that walks four rows of tiles side by side, so that what its workgroups read at a time
-// is few rows of X and of W.
-struct GtTile { int m, n; };
-__device__ __forceinline__ GtTile gt_tile(unsigned id, int tiles_m, int tiles_n) {
-  const unsigned total = (unsigned)tiles_m * (unsigned)tiles_n, xcd = id % 8, per = total / 8, more = total % 8;
-  const unsigned t = xcd * per + min(xcd, more) + id / 8;
-  const unsigned band = 4u * (unsigned)tiles_n, g = t / band, in = t - g * band;
-  const unsigned rows = min(4u, (unsigned)tiles_m - g * 4);
-  return {(int)(g * 4 + in % rows), (int)(in / rows)};
-}
-
-// NSTAGE: buffers of LDS; AHEAD: slices of 16 of K that operands are fetched from LDS before their products
 template <int BM, int BN, int WM, int WN, int NSTAGE, int AHEAD, bool RESIDUAL, typename TO, int ACT = 0>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
     const bf16* __restrict__ X, long x_ld, const bf16* __restrict__ W, const bf16* R, long r_ld, TO* C, long c_ld,
     int M, int N, int K, float limit) {
-  constexpr int BK = GT_BK, PCS = GT_PIECES, ROWS = BM + BN, GT_WAVES = WM * WN, KS = BK / 16;
-  constexpr int STAGE = ROWS * BK * 2;                  // bytes of a buffer: X's rows, then W's
-  constexpr int LPW = ROWS * PCS / 64 / GT_WAVES;       // loads of a step that each wave issues, 8 rows each
-  constexpr int TM = BM / WM / 32, TN = BN / WN / 32;   // 32 x 32 result tiles of a wave
-  static_assert(ROWS * PCS % (64 * GT_WAVES) == 0 && TM >= 1 && TN >= 1 && NSTAGE * STAGE <= 160 * 1024, "tile sizes");
-  constexpr int FLIGHT = AHEAD == 1 ? NSTAGE : NSTAGE - 1;   // steps that are copied ahead
-  constexpr int SETS = AHEAD == 1 ? 2 : KS;             // operand registers: a set a slice, in turn
-  static_assert((AHEAD == 1 || AHEAD == 2) && FLIGHT >= 2 && FLIGHT <= 3 && KS == 4, "what the loop below is written for");
-  static_assert((FLIGHT - 1) * LPW <= 63, "more loads in flight than the counter counts");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[NSTAGE * STAGE];
+  typedef TileLoop<BM, BN, WM, WN, NSTAGE, AHEAD> Loop;
+  constexpr int LPW = Loop::LPW, TM = Loop::TM, TN = Loop::TN;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[NSTAGE * Loop::STAGE];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r32 = lane & 31, h = lane >> 5;
   const int wm = wave / WN, wn = wave % WN;
   const GtTile tile = gt_tile(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN);
   const long m0 = (long)tile.m * BM, n0 = (long)tile.n * BN;
-  const unsigned lds0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds;
 
-  // The wave's loads of a step: load j brings rows 8 (wave * LPW + j) .. +7 of the buffer, lane (row, slot) the piece
-  // slot ^ ((row >> 1) & 7) of its row. Rows past the matrix's last are the last row again (their results are not
-  // stored).
-  const unsigned char* first_row[LPW];       // of the load's first row, at K offset 0 (the same on all lanes)
-  unsigned lane_off[LPW];                    // the lane's piece from there, in bytes
+  // Rows past the matrix's last are the last row again (their results are not stored).
+  const unsigned char* first[LPW];
+  unsigned lane_off[LPW];
 #pragma unroll
   for (int j = 0; j < LPW; ++j) {
-    const int row0 = (wave * LPW + j) * 8, row = row0 + (lane >> 3);
+    const int row0 = Loop::row_of(wave, 0, j), row = Loop::row_of(wave, lane, j);
     const bool of_x = row0 < BM;
     const long ld = of_x ? x_ld : (long)K;
     const long last = of_x ? (long)M - 1 : (long)N - 1;
     const long g_first = min(last, of_x ? m0 + row0 : n0 + (row0 - BM));
     const long g_row = min(last, of_x ? m0 + row : n0 + (row - BM));
-    first_row[j] = (const unsigned char*)(of_x ? X : W) + g_first * ld * 2;
-    lane_off[j] = (unsigned)((g_row - g_first) * ld * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16);
+    first[j] = (const unsigned char*)(of_x ? X : W) + g_first * ld * 2;
+    lane_off[j] = (unsigned)((g_row - g_first) * ld * 2 + Loop::piece_of(lane, row) * 16);
   }
-  const int nk = (K + BK - 1) / BK;
-  const bool ragged = K % BK != 0;                      // the last step's pieces past the end of K come from a block of zeros
-  auto load = [&](int kt, unsigned at, int j) {         // at: where the buffer begins
-    gt_copy16(first_row[j] + (long)kt * (BK * 2), lane_off[j], at + (wave * LPW + j) * 1024);
-  };
-  auto load_ragged = [&](int kt, unsigned at, int j) {
-    const int row = (wave * LPW + j) * 8 + (lane >> 3);
-    const bool inside = kt * BK + ((lane & 7) ^ ((row >> 1) & 7)) * 8 < K;
-    gt_copy16(inside ? first_row[j] + (long)kt * (BK * 2) + lane_off[j] : gt_zeros, at + (wave * LPW + j) * 1024);
-  };
-
   f32x16 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -132,86 +54,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  // operand pieces: row r of the buffer, elements 16 ks + 8 h .. of the step, lie at r * 128 + ((2 ks + h) ^ ((r >> 1) & 7)) * 16:
-  // 32 rows on, the same piece; two pieces on (the next ks), the address with bits 5 and 6 changed
-  const unsigned a_row = wm * (BM / WM) + r32, b_row = BM + wn * (BN / WN) + r32;
-  const unsigned a_at = a_row * 128 + ((h ^ ((a_row >> 1) & 7)) * 16), b_at = b_row * 128 + ((h ^ ((b_row >> 1) & 7)) * 16);
-  bf16x8 a[SETS][TM], b[SETS][TN];
-  auto fetch = [&](int ks, unsigned at) {               // at: where the buffer begins, from the first
-#pragma unroll
-    for (int i = 0; i < TM; ++i) a[ks % SETS][i] = *(const bf16x8*)(lds + (at + (a_at ^ (ks * 32)) + i * 4096));
-#pragma unroll
-    for (int j = 0; j < TN; ++j) b[ks % SETS][j] = *(const bf16x8*)(lds + (at + (b_at ^ (ks * 32)) + j * 4096));
-  };
-
-  // The loop. While a slice's products run, the operands of the slice AHEAD of it are on their way out of LDS, also across
-  // steps: AHEAD slices before its end, step kt waits until step kt + 1 is in LDS for every wave (the barrier) and fetches from there.
-  // After that barrier a buffer is free for copies: with AHEAD 2 step kt - 1's, whose last operands every wave has used; with
-  // AHEAD 1 step kt's own, whose last operands every wave has in registers, because it waited for them too. Each gives FLIGHT
-  // steps that are under way. The order of a slice's instructions is pinned: the first product, the LDS reads, the other products with
-  // the copies between them, so that a wave that has its SIMD to itself keeps the matrix core busy while it issues them.
-  // MODE 0: copies a whole step; 1: the ragged last one; 2: none. LEFT: the steps beyond the next that are under way meanwhile.
-  unsigned at = 0, prev = (NSTAGE - 1) * STAGE;
-  auto step = [&](int kt, auto mode, auto left, auto last) {
-    constexpr int MODE = mode, LEFT = left;
-    constexpr bool LAST = last;
-    const unsigned next = at + STAGE == NSTAGE * STAGE ? 0 : at + STAGE;
-    const unsigned into = lds0 + (AHEAD == 1 ? at : prev);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      if (ks == KS - AHEAD && !LAST) {
-        if (AHEAD == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LEFT * LPW) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(LEFT * LPW) : "memory");
-      }
-#pragma unroll
-      for (int m = 0; m < TM * TN; ++m) {
-        acc[m / TN][m % TN] =
-            __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[ks % SETS][m % TN], a[ks % SETS][m / TN], acc[m / TN][m % TN], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (m == 0) {
-          if (ks + AHEAD < KS) fetch(ks + AHEAD, at);
-          else if (!LAST) fetch(ks + AHEAD - KS, next);
-        }
-        if (MODE < 2 && ks >= KS - AHEAD) {
-          constexpr int SLOTS = AHEAD * TM * TN;
-          const int slot = (ks - (KS - AHEAD)) * TM * TN + m;
-#pragma unroll
-          for (int j = slot * LPW / SLOTS; j < (slot + 1) * LPW / SLOTS; ++j) {
-            if (MODE == 0) load(kt + FLIGHT, into, j);
-            else load_ragged(kt + FLIGHT, into, j);
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    prev = at;
-    at = next;
-  };
-  const int whole = ragged ? nk - 1 : nk;
-#pragma unroll
-  for (int s = 0; s < FLIGHT; ++s) {
-#pragma unroll
-    for (int j = 0; j < LPW; ++j) {
-      if (s < whole) load(s, lds0 + s * STAGE, j);
-      else if (s < nk) load_ragged(s, lds0 + s * STAGE, j);
-    }
-  }
-  if (nk >= FLIGHT) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((FLIGHT - 1) * LPW) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" : : : "memory");
-#pragma unroll
-  for (int ks = 0; ks < AHEAD; ++ks) fetch(ks, 0);
-  int kt = 0;
-  for (; kt + FLIGHT < whole; ++kt) step(kt, IntC<0>{}, IntC<FLIGHT - 2>{}, IntC<0>{});
-  if (kt + FLIGHT < nk) {
-    step(kt, IntC<1>{}, IntC<FLIGHT - 2>{}, IntC<0>{});
-    ++kt;
-  }
-  // the last steps, whose copies are all under way
-  if constexpr (FLIGHT == 3)
-    if (nk >= 3) step(kt++, IntC<2>{}, IntC<1>{}, IntC<0>{});
-  if (nk >= 2) step(kt++, IntC<2>{}, IntC<0>{}, IntC<0>{});
-  step(kt, IntC<2>{}, IntC<0>{}, IntC<1>{});
+  Loop::run(lds, first, lane_off, K, acc);
 
   // accumulator 4 q + e of block (i, j): row m0 + wm * (BM / WM) + i * 32 + r32, column n0 + wn * (BN / WN) + j * 32 + 8 q + 4 h + e
 #pragma unroll

@@ -51,7 +51,7 @@ SOURCES: Dict[str, str] = {
     "hyper_streams": "hyper_streams.hip",
     "convolved_attention": "convolved_attention.hip",
 }
-HEADERS = ["common.h", "attention_mfma.h"]
+HEADERS = ["common.h", "attention_mfma.h", "tile_loop.h"]
 # what a library links beyond the HIP runtime
 LINK: Dict[str, List[str]] = {"gemm_library": ["-lhipblaslt"]}
 
