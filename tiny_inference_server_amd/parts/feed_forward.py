@@ -288,6 +288,8 @@ class GroupedChoiceExperts:
             if self.shared_gated:
                 # one product for the shared expert's gate, its other factor, and the number that gates its result
                 w_in = torch.cat([tensors.of(spec, k) for k in ("shared_gate", "shared_up", "shared_sg")], dim=0)
+                # (rows of zeros up to a multiple of four: what the tiled product of many rows takes)
+                w_in = torch.cat([w_in, w_in.new_zeros(-w_in.shape[0] % 4, w_in.shape[1])])
             else:
                 w_in = _paired_rows(tensors.of(spec, "shared_gate"), tensors.of(spec, "shared_up"))
             self.w_shared_in = to_compute(ops, w_in)
