@@ -383,3 +383,66 @@ def test_generation_command_line_and_replay_program(tmp_path):
         else:
             errs = FM.errors("A8", cfg, w64, reqs, got)        # (the router chooses here: most rows are not close calls)
             assert errs[len(errs) // 2][0] <= TOL["bfloat16"] / 2
+
+
+@pytest.mark.parametrize("Hh,G,D,V,seqs", [
+    (2, 1, 64, 16, [48]), (4, 2, 128, 40, [63, 47, 1, 64]), (2, 2, 17, 5, [49, 200]), (3, 1, 200, 33, [65]), (1, 1, 256, 16, [96, 50]),
+    (2, 1, 130, 16, [48] * 3 + [2] * 70 + [81])])
+def test_the_delta_rules_walk_in_chunks(Hh, G, D, V, seqs):
+    """Requests of many rows beside requests of few: whole and ragged chunks, channels that fill no tile, strong and no decays, used state
+    lines; against 64 bits, and never further off than a few times what the walk row by row is. A row that is not finite reaches
+    no row before it."""
+    ops = hip_ops("float32")
+    g = torch.Generator().manual_seed(sum(seqs) + D)
+    n, C = sum(seqs), 2 * G * D + Hh * V
+    firsts = [sum(seqs[:i]) for i in range(len(seqs))]
+    b = fake_batch([(f, 0, r) for f, r in zip(firsts, seqs)], list(range(len(seqs)))[::-1], None, 8, "cuda")
+    k, q = (torch.nn.functional.normalize(torch.randn(n, G, D, generator=g), dim=-1) for _ in range(2))
+    v, beta = torch.randn(n, Hh * V, generator=g), torch.rand(n, Hh, generator=g)
+    decay = torch.exp(-torch.rand(n, Hh * D, generator=g) * torch.rand(1, Hh * D, generator=g) * 3.0)
+    decay[n // 2, :D // 2] = 0.0
+    decay[:, D // 2:D] = 1.0
+    blocks = -(-V // 16)
+    line = torch.zeros(len(seqs), Hh, blocks, D, 16)
+    line.permute(0, 1, 3, 2, 4).reshape(len(seqs), Hh, D, blocks * 16)[..., :V]
+    start = torch.randn(len(seqs), Hh, D, V, generator=g)
+    for c in range(V):
+        line[:, :, c // 16, :, c % 16] = start[..., c]
+
+    def engine(v):
+        state = line.reshape(len(seqs), -1).clone().cuda()
+        u = torch.cat([(q * D ** -0.5).reshape(n, -1), k.reshape(n, -1), v, beta], 1).cuda()
+        out = ops.delta_scan(u, 0, G * D, 2 * G * D, C, decay.cuda(), state, b, Hh, G, D, V)
+        return out.cpu(), state.cpu().view(len(seqs), Hh, blocks, D, 16)
+
+    def plain(dt):
+        out, end = torch.empty(n, Hh, V, dtype=dt), start.to(dt).flip(0).clone()
+        kk, qq = (t.to(dt).repeat_interleave(Hh // G, 1) for t in (k, q * D ** -0.5))
+        for i, (f, r) in enumerate(zip(firsts, seqs)):
+            S = end[i]
+            for t in range(f, f + r):
+                S = S * decay[t].to(dt).view(Hh, D, 1)
+                w = beta[t].to(dt)[:, None, None] * (v[t].to(dt).view(Hh, 1, V) - kk[t][:, None] @ S)
+                S = S + kk[t][:, :, None] * w
+                out[t] = (qq[t][:, None] @ S)[:, 0]
+            end[i] = S
+        return out.reshape(n, -1), end.flip(0)
+
+    out, state = engine(v)
+    want, end = plain(torch.float64)
+    near, near_end = plain(torch.float32)
+    kept = torch.stack([state[:, :, c // 16, :, c % 16] for c in range(V)], -1)
+    for got, exact, row in ((out, want, near), (kept, end, near_end)):
+        off = lambda t: float((t.double() - exact).norm() / exact.norm())
+        assert off(got) <= 3 * off(row) + 1e-7, (off(got), off(row))
+    for c in range(V, blocks * 16):
+        assert (state[:, :, c // 16, :, c % 16] == 0).all()
+    longest = max(range(len(seqs)), key=lambda i: seqs[i])
+    at = firsts[longest] + 37
+    bad = v.clone()
+    bad[at] = float("inf")
+    broken, _ = engine(bad)
+    before = torch.ones(n, dtype=torch.bool)
+    before[at:firsts[longest] + seqs[longest]] = False
+    torch.testing.assert_close(broken[before], out[before], rtol=1e-4, atol=1e-5)
+    assert not torch.isfinite(broken[at]).any()

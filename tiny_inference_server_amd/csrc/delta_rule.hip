@@ -4,9 +4,10 @@
 //
 // per head and row, S being 32-bit floats in the request's state line, laid out [head][block of 16 value channels]
 // [key channel][16] (value channels rounded up to a multiple of 16; the channels beyond stay zero), so that the part
-// of a line that one workgroup of the walk owns is one run of memory. Two kernels: the
+// of a line that one workgroup of the walk owns is one run of memory. The kernels: the
 // step before the walk (a short causal convolution with silu over the q, k and v columns of a 32-bit input product,
-// unit q and k per head, beta) and the walk itself. Everything is 32-bit.
+// unit q and k per head, beta); the walk, row by row; and for a request's many rows the walk in chunks of 16, with
+// the step before it. Everything is 32-bit.
 //
 // A request's state line holds S and, from float `conv_at` on, the convolution's last taps - 1
 // inputs [taps - 1][channels], oldest first. Rows of the step are grouped by request: request s owns the rows
@@ -96,17 +97,17 @@ __device__ __forceinline__ float dr_row_sum(float v) {
 // S' = diag(a) S, a token needs S'^T k for its write and (S' + k w^T)^T q = S'^T q + (k . q) w for its read: the three
 // sums over the key channels (S'^T k, S'^T q, k . q) are R terms a lane each and then one pass over the 16 lanes of a
 // column for all three together. Every state element sees its rows strictly in order and every sum has one fixed
-// order, so a row's result does not depend on how its prompt was cut or on what else is in the step, bit for bit.
+// order: a row's result does not depend on what else is in the step. Requests of `from` rows and more are left to the chunks below.
 // Rows come through LDS 16 at a time (8 where a lane holds 16 key channels): [rows][k: Dp | decay: Dp | q: Dp | v: 16 | beta | 3 unused].
 template <int R>
 __global__ __launch_bounds__(256) void delta_scan_kernel(
     const float* __restrict__ u, long ldu, int q_off, int k_off, int v_off, int beta_off, const float* __restrict__ decay,
     long ldd, float* __restrict__ state, long lds, const int* __restrict__ cu_rows, const int* __restrict__ seq_slots,
-    float* __restrict__ out, long ldo, int H, int G, int D, int V, int tokens) {
+    float* __restrict__ out, long ldo, int H, int G, int D, int V, int from) {
   extern __shared__ __attribute__((aligned(16))) float dr_lds[];
   const int s = blockIdx.z, h = blockIdx.y, vb = blockIdx.x, t = threadIdx.x;
   const int first = cu_rows[s], n_rows = cu_rows[s + 1] - first;
-  if (n_rows <= 0) return;
+  if (n_rows <= 0 || n_rows >= from) return;
   const int cl = t / 16, l = t % 16;
   const int c = vb * 16 + cl;
   const bool live = c < V;
@@ -126,7 +127,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(
   }
   // Rows go through two LDS buffers: while one chunk of rows is walked, the next one's loads are in flight in registers
   // and are put into the other buffer afterwards, so one barrier a chunk and no wait for memory between chunks.
-  constexpr int TOK = R <= 8 ? 16 : 8;       // rows a chunk (`tokens`)
+  constexpr int TOK = R <= 8 ? 16 : 8;       // rows a chunk
   constexpr int NI = TOK * Dp / 256;         // k, decay and q elements a thread fetches for a chunk
   float pk[NI], pa[NI], pq[NI], pv[2];
   auto fetch = [&](int r0) {
@@ -224,6 +225,296 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(
     reinterpret_cast<float4*>(S_line)[e] = reinterpret_cast<const float4*>(dr_lds)[e];
 }
 
+// ---- a request's many rows: the walk in chunks of 16 ------------------------------------------------------------------
+//
+// The walk above is one serial chain: every row waits for three sums over the key channels of the state that the row before left
+// (270 ns a row, on one wave a SIMD of half the chip). Sixteen rows at a time the sums of all of them against the state at the
+// chunk's beginning, S0, are matrix products, and what the rows of a chunk do to one another needs no state at all. With
+// A(i, j) = the decays of rows i + 1 .. j multiplied up per channel (products of numbers up to 1: nothing is ever divided by),
+//   G(i, j) = sum_d k_i k_j A(i, j),  Q(j, i) = sum_d k_i q_j A(i, j)  (i <= j)
+//   w_j = beta_j (v_j - S0^T (k_j A(-1, j)) - sum_{i<j} G(i, j) w_i)            that is  W = T (V - K~ S0)
+//   o_j = S0^T (q_j A(-1, j)) + sum_{i<=j} Q(j, i) w_i                                   O = Q~ S0 + Q W
+//   S <- A(-1, 15) S0 + sum_i (k_i A(i, 15)) w_i^T                                       S = A S0 + K^ W
+// with T = (I + beta G)^-1 beta, solved column by column. delta_chunks_kernel makes K~, Q~, K^, A, T and Q of every chunk and head,
+// all chunks at once; delta_chunk_walk_kernel walks them with S in registers, all products on v_mfma_f32_16x16x4_f32 (32-bit
+// multiply-adds). Rows past a request's last have k = q = 0, decay 1 and beta 0 and change nothing. MI355X, 8 heads of 128 x 256,
+// us row by row / in chunks with the step before them: 2,048 rows 545 / 196, 1,531 410 / 153, 512 140 / 58, 128 39 / 24; off from 64
+// bits by 1.7e-7 and 1.8e-7.
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+static constexpr int DC = 16;                    // rows of a chunk
+static constexpr int DR_CHUNK_FROM = 48;         // rows of a request from which on its rows are walked in chunks (us, row by row / in
+                                                 // chunks: 32 rows 13.3 / 14.5, 48 17.9 / 16.1, 128 39 / 24)
+
+__host__ __device__ constexpr int dc_floats(int Dp) { return 3 * DC * Dp + Dp + 2 * DC * DC; }   // of a chunk and head: K~, Q~, K^ [d][row], A, T, Q
+
+__device__ __forceinline__ int dc_chunks(int n) { return n >= DR_CHUNK_FROM ? (n + DC - 1) / DC : 0; }
+
+// grid (chunks, heads), 256 threads: thread (i, l) = (t / 16, t % 16) takes row i and the key channels l, l + 16, ...
+template <int Dp>
+__global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restrict__ u, long ldu, int q_off, int k_off, int beta_off,
+                                                           const float* __restrict__ decay, long ldd,
+                                                           const int* __restrict__ cu_rows, int n_seqs, float* __restrict__ work,
+                                                           int H, int G, int D) {
+  __shared__ __attribute__((aligned(16))) float k[DC][Dp], q[DC][Dp], a[DC][Dp], L[DC][DC], beta[DC];
+  const int h = blockIdx.y, hq = h / (H / G), t = threadIdx.x, lane = t % 64;
+  // which request's, and which of its chunks: the requests' chunks numbered through (a lane a request, 64 at a time)
+  int first = -1, n = 0, before = 0;
+  for (int s0 = 0; s0 < n_seqs && first < 0; s0 += 64) {
+    const int s = s0 + lane;
+    const int rows = s < n_seqs ? cu_rows[s + 1] - cu_rows[s] : 0;
+    const int own = dc_chunks(rows);
+    int upto = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, 64);
+      if (lane >= o) upto += v;
+    }
+    const unsigned long long holds = __ballot(before + upto > (int)blockIdx.x);
+    if (holds) {
+      const int at = __ffsll(holds) - 1;
+      const int c = (int)blockIdx.x - before - __shfl(upto - own, at, 64);
+      first = cu_rows[s0 + at] + c * DC;
+      n = min(DC, __shfl(rows, at, 64) - c * DC);
+    } else {
+      before += __shfl(upto, 63, 64);
+    }
+  }
+  if (first < 0) return;                         // the grid is as wide as there could be chunks
+  for (int e = t; e < DC * Dp; e += 256) {
+    const int r = e / Dp, d = e % Dp;
+    const long row = first + r;
+    const bool ok = r < n && d < D;
+    k[r][d] = ok ? u[row * ldu + k_off + hq * D + d] : 0.f;
+    q[r][d] = ok ? u[row * ldu + q_off + hq * D + d] : 0.f;
+    a[r][d] = ok ? decay[row * ldd + h * D + d] : 1.f;
+  }
+  if (t < DC) beta[t] = t < n ? u[(long)(first + t) * ldu + beta_off + h] : 0.f;
+  __syncthreads();
+  float* mine = work + ((long)blockIdx.x * H + h) * dc_floats(Dp);
+  float *Kt = mine, *Qt = mine + DC * Dp, *Kh = mine + 2 * DC * Dp, *A = mine + 3 * DC * Dp, *T = A + Dp, *Q = T + DC * DC;
+  const int i = t / 16, l = t % 16;
+  float g[DC], p[DC];                            // (of rows that do not follow i: numbers that nobody reads)
+#pragma unroll
+  for (int j = 0; j < DC; ++j) g[j] = p[j] = 0.f;
+#pragma unroll 1
+  for (int d = l * 4; d < Dp; d += 64) {
+    const f32x4 ki = *reinterpret_cast<const f32x4*>(&k[i][d]), qi = *reinterpret_cast<const f32x4*>(&q[i][d]);
+    f32x4 upto = {1.f, 1.f, 1.f, 1.f}, ka = ki;  // the decays of rows 0 .. i; k_i times those of rows i + 1 .. j
+#pragma unroll
+    for (int j = 0; j < DC; ++j) {
+      const f32x4 aj = *reinterpret_cast<const f32x4*>(&a[j][d]), kj = *reinterpret_cast<const f32x4*>(&k[j][d]);
+      const f32x4 qj = *reinterpret_cast<const f32x4*>(&q[j][d]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        upto[e] *= j <= i ? aj[e] : 1.f;
+        ka[e] *= j > i ? aj[e] : 1.f;
+        g[j] = fmaf(ka[e], kj[e], g[j]);
+        p[j] = fmaf(ka[e], qj[e], p[j]);
+      }
+    }
+    *reinterpret_cast<f32x4*>(Kt + i * Dp + d) = ki * upto;
+    *reinterpret_cast<f32x4*>(Qt + i * Dp + d) = qi * upto;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) Kh[(d + e) * DC + i] = ka[e];
+    if (i == DC - 1) *reinterpret_cast<f32x4*>(A + d) = upto;
+  }
+#pragma unroll
+  for (int j = 0; j < DC; ++j) {
+    const float gs = dr_row_sum(g[j]), ps = dr_row_sum(p[j]);
+    if (l == j) {
+      L[j][i] = gs;
+      Q[j * DC + i] = i <= j ? ps : 0.f;
+    }
+  }
+  __syncthreads();
+  if (t < DC) {                                  // column t of T: x_j = beta_j ((j == t) - sum of G(m, j) x_m over t <= m < j)
+    float x[DC];
+#pragma unroll
+    for (int j = 0; j < DC; ++j) {
+      float v = j == t ? 1.f : 0.f;
+#pragma unroll
+      for (int m = 0; m < j; ++m) v = m >= t ? fmaf(-L[j][m], x[m], v) : v;
+      x[j] = j >= t ? beta[j] * v : 0.f;
+      T[j * DC + t] = x[j];
+    }
+  }
+}
+
+// grid (heads, blocks of 16 value channels, requests), five waves. Wave w < 4 keeps key channels [16 NT w, 16 NT (w + 1)) of S as NT
+// result tiles of 16 channels x 16 value channels: lane (g, n) = (lane / 16, lane % 16) holds channels 16 t + 4 g + r of value
+// channel n in register r of tile t. As the second operand of a product over channels, register r of tile t is what the four channels
+// 16 t + 4 g + r (g = 0 .. 3) make up, so S goes into the products as it lies; the same holds for V - K~ S0 and W, whose rows are
+// 4 g + r. The waves' parts of K~ S0 meet in LDS, one barrier a chunk; each then makes W for itself. Q~ S0 is worked out while the parts
+// are on their way, and the fifth wave, which makes W too, adds up the rows' results a chunk later. Three chunks' operands are
+// under way (one ahead, a chunk took what memory takes), or one where a head's channels leave no more registers. Workgroups of one head follow one another by `heads`, so that with 8 heads
+// (or 16, ...) an XCD's L2 serves a head to all of its value channels. What bounds it is a chunk's chain: the products with S, LDS, W, and
+// the products that change S.
+template <int NT>
+__global__ __launch_bounds__(320) void delta_chunk_walk_kernel(const float* __restrict__ u, long ldu, int v_off,
+                                                               const float* __restrict__ work, float* __restrict__ state, long lds,
+                                                               const int* __restrict__ cu_rows, const int* __restrict__ seq_slots,
+                                                               float* __restrict__ out, long ldo, int H, int D, int V) {
+  constexpr int SETS = NT <= 2 ? 4 : 2;          // chunks whose operands are held or under way
+  constexpr int Dp = 64 * NT, OFF_A = 3 * DC * Dp, OFF_T = OFF_A + Dp, OFF_Q = OFF_T + DC * DC;
+  __shared__ f32x4 ks_parts[2][4][64], qs_parts[2][4][64];       // turn, wave, lane
+  const int h = blockIdx.x, vb = blockIdx.y, s = blockIdx.z, t = threadIdx.x;
+  const int first = cu_rows[s], n_rows = cu_rows[s + 1] - first;
+  if (n_rows < DR_CHUNK_FROM) return;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, g = lane >> 4, n = lane & 15;
+  int chunk0 = 0;                                // the chunks of the requests before
+  for (int s0 = 0; s0 < s; s0 += 64) {
+    int c = s0 + lane < s ? dc_chunks(cu_rows[s0 + lane + 1] - cu_rows[s0 + lane]) : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) c += __shfl_xor(c, o, 64);
+    chunk0 += c;
+  }
+  const int c_v = vb * 16 + n;
+  const bool live = c_v < V;
+  const float* base = work + ((long)chunk0 * H + h) * dc_floats(Dp);
+  const long stride = (long)H * dc_floats(Dp);
+  const float* v_column = u + (long)first * ldu + v_off + h * V + min(c_v, V - 1);
+  const int chunks = (n_rows + DC - 1) / DC;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+
+  // W of chunk c from the four parts of K~ S0 in LDS. T and Q are triangular, but a product takes their zeros times every row: a row that
+  // is not finite must not reach the rows before it, so such a chunk goes without the matrix product.
+  auto triangle = [&](const float* M, f32x4 m, f32x4 x, f32x4 sum) {      // sum + M x, M lower triangular [16][16], m: the lane's four
+    const float none = fmaf(x[3], 0.f, fmaf(x[2], 0.f, fmaf(x[1], 0.f, x[0] * 0.f)));
+    if (__all(none == 0.f)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], x[r], sum, 0, 0, 0);
+      return sum;
+    }
+#pragma unroll 1
+    for (int i = 0; i < DC; ++i) {
+      const float xi = __shfl(i % 4 == 0 ? x[0] : i % 4 == 1 ? x[1] : i % 4 == 2 ? x[2] : x[3], (i / 4) * 16 + n, 64);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (i <= g * 4 + r) sum[r] += M[(g * 4 + r) * DC + i] * xi;
+    }
+    return sum;
+  };
+  auto make_w = [&](int c, f32x4 m, f32x4 v) {
+    f32x4 x = v - (ks_parts[c & 1][0][lane] + ks_parts[c & 1][1][lane] + ks_parts[c & 1][2][lane] + ks_parts[c & 1][3][lane]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = live ? x[r] : 0.f;
+    return triangle(base + c * stride + OFF_T, m, x, zero);
+  };
+  // (rows past the last: the last one's values, which T's zeros keep out)
+  auto fetch_v = [&](int c) {
+    f32x4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = v_column[(long)min(c * DC + g * 4 + r, n_rows - 1) * ldu];
+    return v;
+  };
+  // (not __syncthreads, which also waits for what is under way from memory)
+  auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
+
+  if (wave == 4) {                               // the rows' results
+    struct Operands { f32x4 t, q, v; } sets[SETS];
+    auto fetch = [&](Operands& o, int c) {
+      o.t = *reinterpret_cast<const f32x4*>(base + c * stride + OFF_T + n * DC + g * 4);
+      o.q = *reinterpret_cast<const f32x4*>(base + c * stride + OFF_Q + n * DC + g * 4);
+      o.v = fetch_v(c);
+    };
+    f32x4 W = zero, q = zero;                    // of the chunk before
+    auto results = [&](int c) {
+      const f32x4 o = triangle(base + c * stride + OFF_Q, q, W,
+                               qs_parts[c & 1][0][lane] + qs_parts[c & 1][1][lane] + qs_parts[c & 1][2][lane] + qs_parts[c & 1][3][lane]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = c * DC + g * 4 + r;
+        if (row < n_rows && live) out[(long)(first + row) * ldo + h * V + c_v] = o[r];
+      }
+    };
+#pragma unroll
+    for (int c = 0; c < SETS - 1; ++c)
+      if (c < chunks) fetch(sets[c], c);
+    for (int c0 = 0; c0 < chunks; c0 += SETS) {
+#pragma unroll
+      for (int e = 0; e < SETS; ++e) {
+        const int c = c0 + e;
+        if (c >= chunks) break;
+        if (c + SETS - 1 < chunks) fetch(sets[(e + SETS - 1) % SETS], c + SETS - 1);
+        meet();
+        const f32x4 now = make_w(c, sets[e].t, sets[e].v);
+        if (c) results(c - 1);
+        W = now;
+        q = sets[e].q;
+      }
+    }
+    meet();
+    results(chunks - 1);
+    return;
+  }
+
+  const int d0 = wave * NT * 16;                 // the wave's first key channel
+  float* S_line = state + (long)seq_slots[s] * lds + ((long)h * gridDim.y + vb) * D * 16;
+  f32x4 S[NT];
+#pragma unroll
+  for (int k = 0; k < NT; ++k)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d = d0 + k * 16 + g * 4 + r;
+      S[k][r] = d < D ? S_line[d * 16 + n] : 0.f;
+    }
+  struct Operands { f32x4 kt[NT], qt[NT], kh[NT], a[NT], t, v; } sets[SETS];
+  auto fetch = [&](Operands& o, int c) {
+    const float* p = base + c * stride;
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+      o.kt[k] = *reinterpret_cast<const f32x4*>(p + n * Dp + d0 + k * 16 + g * 4);
+      o.qt[k] = *reinterpret_cast<const f32x4*>(p + DC * Dp + n * Dp + d0 + k * 16 + g * 4);
+      o.kh[k] = *reinterpret_cast<const f32x4*>(p + 2 * DC * Dp + (d0 + k * 16 + n) * DC + g * 4);
+      o.a[k] = *reinterpret_cast<const f32x4*>(p + OFF_A + d0 + k * 16 + g * 4);
+    }
+    o.t = *reinterpret_cast<const f32x4*>(p + OFF_T + n * DC + g * 4);
+    o.v = fetch_v(c);
+  };
+  auto chunk = [&](int c, const Operands& now) {
+    f32x4 ks = zero, qs = zero;
+#pragma unroll
+    for (int k = 0; k < NT; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ks = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kt[k][r], S[k][r], ks, 0, 0, 0);
+    ks_parts[c & 1][wave][lane] = ks;
+    meet();
+#pragma unroll
+    for (int k = 0; k < NT; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) qs = __builtin_amdgcn_mfma_f32_16x16x4f32(now.qt[k][r], S[k][r], qs, 0, 0, 0);
+    const f32x4 W = make_w(c, now.t, now.v);
+    qs_parts[c & 1][wave][lane] = qs;
+#pragma unroll
+    for (int k = 0; k < NT; ++k) S[k] *= now.a[k];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int k = 0; k < NT; ++k) S[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kh[k][r], W[r], S[k], 0, 0, 0);
+  };
+#pragma unroll
+  for (int c = 0; c < SETS - 1; ++c)
+    if (c < chunks) fetch(sets[c], c);
+  for (int c0 = 0; c0 < chunks; c0 += SETS) {
+#pragma unroll
+    for (int e = 0; e < SETS; ++e) {
+      const int c = c0 + e;
+      if (c >= chunks) break;
+      if (c + SETS - 1 < chunks) fetch(sets[(e + SETS - 1) % SETS], c + SETS - 1);
+      chunk(c, sets[e]);
+    }
+  }
+  meet();                                        // the fifth wave's last results
+  // (channels beyond vdim have seen values of zero only and are still zero)
+#pragma unroll
+  for (int k = 0; k < NT; ++k)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d = d0 + k * 16 + g * 4 + r;
+      if (d < D) S_line[d * 16 + n] = S[k][r];
+    }
+}
+
 TIS_EXPORT int tis_delta_prepare(const float* proj, long ldp, int conv_off, int beta_off, const float* taps, int K,
                                  const float* state, long lds, int conv_at, const int* row_seq, const int* cu_rows,
                                  const int* seq_slots, float* out, long ldo, int rows, int H, int G, int D, int V,
@@ -239,29 +530,57 @@ TIS_EXPORT int tis_delta_prepare(const float* proj, long ldp, int conv_off, int 
   return tis_launch_status("delta_prepare");
 }
 
+// The most chunks that `rows` rows can have, over all requests of DR_CHUNK_FROM rows and more (each begins one that it may not fill).
+static long dc_most(long rows) { return rows / DC + rows / DR_CHUNK_FROM + 1; }
+
+// Floats of work space that tis_delta_scan wants for the walk in chunks; 0: rows too few for it.
+TIS_EXPORT long tis_delta_scan_work(int rows, int H, int D) {
+  return rows < DR_CHUNK_FROM ? 0 : dc_most(rows) * H * dc_floats((D + 63) / 64 * 64);
+}
+
+// work: null, or tis_delta_scan_work floats, 16-byte aligned: requests of DR_CHUNK_FROM rows and more are then walked in chunks.
 TIS_EXPORT int tis_delta_scan(const float* u, long ldu, int q_off, int k_off, int v_off, int beta_off, const float* decay,
-                              long ldd, float* state, long lds, const int* cu_rows, const int* seq_slots, int n_seqs,
-                              float* out, long ldo, int H, int G, int D, int V, hipStream_t stream) {
+                              long ldd, float* state, long lds, const int* cu_rows, const int* seq_slots, int n_seqs, int rows,
+                              float* work, float* out, long ldo, int H, int G, int D, int V, hipStream_t stream) {
   if (n_seqs == 0) return 0;
-  if (n_seqs < 0 || n_seqs > 65535 || H < 1 || H > 65535 || G < 1 || H % G || D < 1 || D > 256 || V < 1 || lds % 4 ||
-      ((uintptr_t)state % 16))
+  if (n_seqs < 0 || n_seqs > 65535 || rows < 0 || H < 1 || H > 65535 || G < 1 || H % G || D < 1 || D > 256 || V < 1 || lds % 4 ||
+      ((uintptr_t)state % 16) || ((uintptr_t)work % 16))
     return tis_fail("delta_scan: bad size requests=%d heads=%d qk_heads=%d dim=%d (at most 256) vdim=%d, or state lines that are "
                     "not 16 bytes aligned", n_seqs, H, G, D, V);
-  const int R = D <= 16 ? 1 : D <= 32 ? 2 : D <= 64 ? 4 : D <= 128 ? 8 : 16;
-  const int tokens = R <= 8 ? 16 : 8;
-  size_t lds_bytes = 2 * (size_t)tokens * (3 * 16 * R + 20) * sizeof(float);      // two buffers of rows
-  if (lds_bytes < (size_t)D * 16 * sizeof(float)) lds_bytes = (size_t)D * 16 * sizeof(float);      // the line's way in and out
-  dim3 grid((V + 15) / 16, H, n_seqs);
+  const bool chunks = work && rows >= DR_CHUNK_FROM && (V + 15) / 16 <= 65535 && dc_most(rows) < (1L << 31);
+  const int from = chunks ? DR_CHUNK_FROM : 0x7fffffff;
+  if (!(chunks && n_seqs == 1)) {           // (a single request of that many rows has none left for the walk row by row)
+    const int R = D <= 16 ? 1 : D <= 32 ? 2 : D <= 64 ? 4 : D <= 128 ? 8 : 16;
+    const int tokens = R <= 8 ? 16 : 8;
+    size_t lds_bytes = 2 * (size_t)tokens * (3 * 16 * R + 20) * sizeof(float);      // two buffers of rows
+    if (lds_bytes < (size_t)D * 16 * sizeof(float)) lds_bytes = (size_t)D * 16 * sizeof(float);      // the line's way in and out
+    dim3 grid((V + 15) / 16, H, n_seqs);
 #define DR_SCAN(RR)                                                                                                        \
   delta_scan_kernel<RR><<<grid, 256, lds_bytes, stream>>>(u, ldu, q_off, k_off, v_off, beta_off, decay, ldd, state, lds,   \
-                                                          cu_rows, seq_slots, out, ldo, H, G, D, V, tokens)
-  switch (R) {
-    case 1: DR_SCAN(1); break;
-    case 2: DR_SCAN(2); break;
-    case 4: DR_SCAN(4); break;
-    case 8: DR_SCAN(8); break;
-    default: DR_SCAN(16); break;
-  }
+                                                          cu_rows, seq_slots, out, ldo, H, G, D, V, from)
+    switch (R) {
+      case 1: DR_SCAN(1); break;
+      case 2: DR_SCAN(2); break;
+      case 4: DR_SCAN(4); break;
+      case 8: DR_SCAN(8); break;
+      default: DR_SCAN(16); break;
+    }
 #undef DR_SCAN
+  }
+  if (chunks) {
+    const dim3 each((unsigned)dc_most(rows), H), walk(H, (V + 15) / 16, n_seqs);
+#define DR_CHUNKS(NT)                                                                                                        \
+  {                                                                                                                         \
+    delta_chunks_kernel<64 * NT><<<each, 256, 0, stream>>>(u, ldu, q_off, k_off, beta_off, decay, ldd, cu_rows, n_seqs, work, H, G, D);  \
+    delta_chunk_walk_kernel<NT><<<walk, 320, 0, stream>>>(u, ldu, v_off, work, state, lds, cu_rows, seq_slots, out, ldo, H, D, V);      \
+  }
+    switch ((D + 63) / 64) {
+      case 1: DR_CHUNKS(1); break;
+      case 2: DR_CHUNKS(2); break;
+      case 3: DR_CHUNKS(3); break;
+      default: DR_CHUNKS(4); break;
+    }
+#undef DR_CHUNKS
+  }
   return tis_launch_status("delta_scan");
 }

@@ -156,7 +156,7 @@ _SIGNATURES["ssm_parts"] = ("tis_ssm", {
 
 _SIGNATURES["delta_rule"] = ("tis_delta_rule", {
     "tis_delta_prepare": [_P, _L, _I, _I, _P, _I, _P, _L, _I, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _P],
-    "tis_delta_scan": [_P, _L, _I, _I, _I, _I, _P, _L, _P, _L, _P, _P, _I, _P, _L, _I, _I, _I, _I, _P],
+    "tis_delta_scan": [_P, _L, _I, _I, _I, _I, _P, _L, _P, _L, _P, _P, _I, _I, _P, _P, _L, _I, _I, _I, _I, _P],
 })
 
 _SIGNATURES["attention_mixed"] = ("tis_attention_mixed", {
@@ -260,6 +260,7 @@ _ATTN_TILE_MIN_WORK_MIXED = 1500   # tile steps times key/value heads below whic
                                    # beside decoded tokens deep in their requests (few tiles with long chains: the
                                    # one-wave kernel spreads them over more waves, and its splits are merged anyway)
 _ATTN_WORKSPACE_FLOATS = 16 << 20
+_DELTA_WORK_FLOATS = 128 << 20   # most work space of a delta rule's walk in chunks (8 heads of 128: steps of 26,000 rows)
 
 
 def tile_columns(head_dim: int) -> int:
@@ -2188,10 +2189,15 @@ class HipOps:
         if state.stride(0) % 4 or state.data_ptr() % 16:
             raise KernelError("delta_scan: state lines must be 16 bytes aligned")
         out = torch.empty(n, n_heads * vdim, dtype=torch.float32, device=self.device)
-        self._lazy("delta_rule").tis_delta_scan(
+        lib = self._lazy("delta_rule")
+        # (work space for requests of many rows, which are walked in chunks; without it row by row)
+        lib.cdll.tis_delta_scan_work.restype = c_long
+        floats = lib.cdll.tis_delta_scan_work(n, n_heads, dim)
+        work = torch.empty(floats, dtype=torch.float32, device=self.device) if 0 < floats <= _DELTA_WORK_FLOATS else None
+        lib.tis_delta_scan(
             _ptr(u), u.stride(0), int(q_off), int(k_off), int(v_off), int(beta_off), _ptr(decay), decay.stride(0), _ptr(state),
-            state.stride(0), _ptr(batch.cu_rows), _ptr(batch.seq_slots), batch.n_seqs, _ptr(out), out.stride(0), n_heads,
-            qk_heads, dim, vdim, self._stream())
+            state.stride(0), _ptr(batch.cu_rows), _ptr(batch.seq_slots), batch.n_seqs, n, _ptr(work), _ptr(out), out.stride(0),
+            n_heads, qk_heads, dim, vdim, self._stream())
         return out
 
     # ---- recurrent mixers with a matrix state per head ---------------------------------------------------
