@@ -117,25 +117,6 @@ __global__ __launch_bounds__(TIS_WAVE) void head_norm_gate_kernel(const float* _
   }
 }
 
-// decay[r][c] = sigmoid(z)^(1/tau) with z = sum_k low[r][k] * w2[c][k] + bias[c], as exp(log_sigmoid(z) / tau)
-__global__ __launch_bounds__(S32_THREADS) void lowrank_decay_kernel(const float* __restrict__ low, long ldl, int rank,
-                                                                     const float* __restrict__ w2,
-                                                                     const float* __restrict__ bias, float tau,
-                                                                     float* __restrict__ out, int C) {
-  extern __shared__ float a[];
-  const long r = blockIdx.x;
-  for (int k = threadIdx.x; k < rank; k += S32_THREADS) a[k] = low[r * ldl + k];
-  __syncthreads();
-  for (int c = threadIdx.x; c < C; c += S32_THREADS) {
-    float z = 0.f;
-    const float* w = w2 + (long)c * rank;
-    for (int k = 0; k < rank; ++k) z += a[k] * w[k];
-    z += bias[c];
-    out[r * C + c] = expf(log_sigmoid_f(z) / tau);
-  }
-}
-
-
 // Layer norm of a 32-bit row into the compute type: (x - mean) / sqrt(var + eps) * gain + bias, the variance being the
 // mean of the squared deviations (two passes over the row; bias may be null).
 template <typename T>
@@ -379,12 +360,16 @@ TIS_EXPORT int tis_head_norm_gate(int dtype, const float* o, long ldo, const flo
   return tis_launch_status("head_norm_gate");
 }
 
+static void launch_lowrank(const float* low, long ldl, int rank, const float* w2, const float* bias, int kind, float tau,
+                           const float* rate, int group, float* out, int rows, int C, hipStream_t stream);
+
+// sigmoid(z)^(1/tau), as exp(log_sigmoid(z) / tau), of z = low . w2^T + bias
 TIS_EXPORT int tis_lowrank_decay(const float* low, long ldl, int rank, const float* w2, const float* bias, float tau,
                                  float* out, int rows, int C, hipStream_t stream) {
   if (rows == 0) return 0;
   if (rows < 0 || rank < 1 || rank > 8192 || C < 1 || !(tau > 0.f))
     return tis_fail("lowrank_decay: bad size rows=%d rank=%d channels=%d tau=%g", rows, rank, C, (double)tau);
-  lowrank_decay_kernel<<<rows, S32_THREADS, rank * sizeof(float), stream>>>(low, ldl, rank, w2, bias, tau, out, C);
+  launch_lowrank(low, ldl, rank, w2, bias, 0, tau, nullptr, 1, out, rows, C, stream);
   return tis_launch_status("lowrank_decay");
 }
 
@@ -604,40 +589,71 @@ TIS_EXPORT int tis_softcap(float* z, long ldz, float cap, int rows, int W, hipSt
 // out[r][c] = act(z) with z = sum_k low[r][k] * w2[c][k] + bias[c] (bias may be null): the second half of a low-rank
 // projection, in 32-bit. kind 0: sigmoid(z)^(1/tau); 1: exp(-rate[c / group] * softplus(z)), a decay whose rate is one
 // number per run of `group` channels; 2: z itself.
-static constexpr int LR_ROWS = 8;      // rows a workgroup of lowrank_act takes: a channel's line of w2 is read once for them
-
+// A workgroup takes 32 channels and 8 RT rows, a thread one channel of RT of them, and both factors come through LDS in chunks of 64 of
+// the rank, read in whole runs (a thread that walked its channel's line of w2 by itself touched a line of memory per lane and
+// term, and 5 rows of 512 channels were two workgroups). k in rising order for every row, whatever RT. us before / now, rank 64: 5 rows
+// x 1,024 7.0 / 4.3, 64 x 1,024 8.5 / 4.4, 1,531 x 1,024 15.4 / 12.4, 1,531 x 2,048 25.0 / 22.4.
+static constexpr int LR_COLS = 32, LR_BY = S32_THREADS / LR_COLS, LR_K = 64;
+template <int RT>
 __global__ __launch_bounds__(S32_THREADS) void lowrank_act_kernel(const float* __restrict__ low, long ldl, int rank,
                                                                    const float* __restrict__ w2,
                                                                    const float* __restrict__ bias, int kind, float tau,
                                                                    const float* __restrict__ rate, int group,
                                                                    float* __restrict__ out, int rows, int C, int col_blocks) {
-  extern __shared__ float a[];                   // [LR_ROWS][rank]
-  // grid (blocks of rows * blocks of channels, a row block's side by side): a few rows still fill the chip
-  const long r0 = (long)(blockIdx.x / col_blocks) * LR_ROWS;
-  const int n = (int)min((long)LR_ROWS, rows - r0);
-  for (int i = threadIdx.x; i < n * rank; i += S32_THREADS) a[i] = low[(r0 + i / rank) * ldl + i % rank];
-  __syncthreads();
-  const int c = (blockIdx.x % col_blocks) * S32_THREADS + threadIdx.x;
-  if (c >= C) return;
-  float z[LR_ROWS];
+  __shared__ __attribute__((aligned(16))) float w[LR_COLS][LR_K + 4], a[LR_BY * RT][LR_K];
+  // grid (blocks of rows * blocks of channels, a row block's side by side)
+  const long r0 = (long)(blockIdx.x / col_blocks) * (LR_BY * RT);
+  const int n = (int)min((long)LR_BY * RT, rows - r0);
+  const int c0 = (blockIdx.x % col_blocks) * LR_COLS, cl = threadIdx.x % LR_COLS, rl = threadIdx.x / LR_COLS, c = c0 + cl;
+  const float b = bias && c < C ? bias[c] : 0.f;
+  const float rt = kind == 1 && c < C ? rate[c / group] : 0.f;
+  float z[RT];
 #pragma unroll
-  for (int r = 0; r < LR_ROWS; ++r) z[r] = 0.f;
-  const float* w = w2 + (long)c * rank;
-  for (int k = 0; k < rank; ++k) {
-    const float wk = w[k];
+  for (int i = 0; i < RT; ++i) z[i] = 0.f;
+  for (int k0 = 0; k0 < rank; k0 += LR_K) {
+    if (k0) __syncthreads();
 #pragma unroll
-    for (int r = 0; r < LR_ROWS; ++r) z[r] += a[(r < n ? r : 0) * rank + k] * wk;      // (k in rising order for every row)
+    for (int i = threadIdx.x; i < LR_COLS * LR_K; i += S32_THREADS) {
+      const int row = i / LR_K, k = i % LR_K;
+      w[row][k] = c0 + row < C && k0 + k < rank ? w2[(long)(c0 + row) * rank + k0 + k] : 0.f;
+    }
+#pragma unroll
+    for (int i = threadIdx.x; i < LR_BY * RT * LR_K; i += S32_THREADS) {
+      const int row = i / LR_K, k = i % LR_K;
+      a[row][k] = row < n && k0 + k < rank ? low[(r0 + row) * ldl + k0 + k] : 0.f;
+    }
+    __syncthreads();
+    const int kc = min(LR_K, rank - k0);
+    for (int k = 0; k < kc; k += 4) {            // (terms past the rank are zeros)
+      const float4 wk = *reinterpret_cast<const float4*>(&w[cl][k]);
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const float4 ak = *reinterpret_cast<const float4*>(&a[rl + i * LR_BY][k]);
+        z[i] = fmaf(ak.w, wk.w, fmaf(ak.z, wk.z, fmaf(ak.y, wk.y, fmaf(ak.x, wk.x, z[i]))));
+      }
+    }
   }
-  const float b = bias ? bias[c] : 0.f;
-  const float rt = kind == 1 ? rate[c / group] : 0.f;
+  if (c >= C) return;
 #pragma unroll
-  for (int r = 0; r < LR_ROWS; ++r) {
-    if (r >= n) break;
-    float v = z[r] + b;
+  for (int i = 0; i < RT; ++i) {
+    if (rl + i * LR_BY >= n) break;
+    float v = z[i] + b;
     if (kind == 0) v = expf(log_sigmoid_f(v) / tau);
     else if (kind == 1) v = expf(-rt * (v > 20.f ? v : log1pf(expf(v))));
-    out[(r0 + r) * C + c] = v;
+    out[(r0 + rl + i * LR_BY) * C + c] = v;
   }
+}
+
+// (eight rows a workgroup up to 256 rows, for the shortest chain: 100 rows x 1,024 4.9 us, 7.6 with 32; 32 beyond, which read w2 a
+// quarter as often)
+static void launch_lowrank(const float* low, long ldl, int rank, const float* w2, const float* bias, int kind, float tau,
+                           const float* rate, int group, float* out, int rows, int C, hipStream_t stream) {
+  const int col_blocks = (C + LR_COLS - 1) / LR_COLS;
+  const bool few = rows <= 256;
+  const int per = few ? LR_BY : 4 * LR_BY;
+  const long blocks = ((long)rows + per - 1) / per * col_blocks;
+  if (few) lowrank_act_kernel<1><<<blocks, S32_THREADS, 0, stream>>>(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, col_blocks);
+  else lowrank_act_kernel<4><<<blocks, S32_THREADS, 0, stream>>>(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, col_blocks);
 }
 
 // out[r] = (1 / n) * sum_i y_i[r] / sqrt(mean(y_i[r]^2) + eps) * gain_i: the mean of one or two RMS-normed rows, 32-bit.
@@ -688,11 +704,8 @@ TIS_EXPORT int tis_lowrank_act(const float* low, long ldl, int rank, const float
   if (rows < 0 || rank < 1 || rank > 8192 || C < 1 || kind < 0 || kind > 2 || (kind == 0 && !(tau > 0.f)) ||
       (kind == 1 && (!rate || group < 1)))
     return tis_fail("lowrank_act: bad arguments rows=%d rank=%d channels=%d kind=%d", rows, rank, C, kind);
-  const int col_blocks = (C + S32_THREADS - 1) / S32_THREADS;
-  const long row_blocks = ((long)rows + LR_ROWS - 1) / LR_ROWS;
   if (rank > 1024) return tis_fail("lowrank_act: rank %d (at most 1024)", rank);
-  lowrank_act_kernel<<<row_blocks * col_blocks, S32_THREADS, LR_ROWS * rank * sizeof(float), stream>>>(
-      low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, col_blocks);
+  launch_lowrank(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, stream);
   return tis_launch_status("lowrank_act");
 }
 
