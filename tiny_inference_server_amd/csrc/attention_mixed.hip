@@ -43,17 +43,28 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 __device__ __forceinline__ bf16x8 amx_load8(const bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
 __device__ __forceinline__ bf16x4 amx_load4(const bf16* p) { return *reinterpret_cast<const bf16x4*>(p); }
 
-// items: (first row, rows) pairs, or null: item i is row i alone. LDS (floats): talk [H * H, rounded up to 4] | weights [H][64][8].
+__device__ __forceinline__ float amx_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+__device__ __forceinline__ float amx_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+
+// items: (first row, rows) pairs, or null: item i is row i alone. LDS (floats): talk [4 HPW][4 HPW], heads that are mixed from outside,
+// wave's heads inside | weights [H][64][8].
+//
+// What bounds it: a wave's instructions (a step of 32 keys: 64 products, two exponentials and two reciprocals for each of 8 weights
+// of 4 heads, 512 multiply-adds of the mixture), as 16 heads' results and queries leave one wave a SIMD; so nothing may wait
+// for memory either: the next step's pages are looked up a step ahead, its first head's keys are fetched as soon as this
+// step's scores are made and the values before this step's weights meet, once for the heads that share them. us, 16
+// heads of 128 in chunks of 1,024: 1,531 rows 203 before that (and with divisions), 96 now; 5 single rows near 600 keys 10.4, 8.9.
 __global__ __launch_bounds__(256) void attention_mixed_mfma_kernel(
     const bf16* __restrict__ q, long ldq, const bf16* __restrict__ plane, const int* __restrict__ block_tables, int bt_ld,
     const int* __restrict__ row_seq, const int* __restrict__ positions, const int* __restrict__ items,
     bf16* __restrict__ out, long ldo, float* __restrict__ partial, int n_splits, int H, int G, int chunk, float scale,
     float softcap, const float* __restrict__ head_bias, const float* __restrict__ talk) {
-  extern __shared__ float amx_lds[];
-  float* tk = amx_lds;
-  float* wl = amx_lds + ((H * H + 3) & ~3);      // (16-byte reads and writes)
+  constexpr int HM = 4 * HPW;                    // heads there is room for
+  extern __shared__ __attribute__((aligned(16))) float amx_lds[];
+  float* tk = amx_lds;                           // [from head][to head]
+  float* wl = amx_lds + HM * HM;
   const int item = blockIdx.x, split = blockIdx.y;
-  const int wave = threadIdx.x / TIS_WAVE, lane = threadIdx.x % TIS_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TIS_WAVE), lane = threadIdx.x % TIS_WAVE;
   const int c16 = lane % 16, g4 = lane / 16;
   const int first = items ? items[2 * item] : item;
   const int n_rows = items ? items[2 * item + 1] : 1;
@@ -62,19 +73,23 @@ __global__ __launch_bounds__(256) void attention_mixed_mfma_kernel(
   const int* bt = block_tables + (long)row_seq[first] * bt_ld;
   const int k_first = chunk > 0 ? pos0 - pos0 % chunk : 0;
   const int group_size = H / G;
-  for (int i = threadIdx.x; i < H * H; i += 256) tk[i] = talk[i];
+  for (int i = threadIdx.x; i < HM * HM; i += 256) {
+    const int from = i / HM, to = i % HM;
+    tk[i] = from < H && to < H ? talk[to * H + from] : 0.f;
+  }
   // the lane's row: its position, its first visible key, whether it is a row at all
   const bool row_ok = c16 < n_rows;
-  const int p_row = pos0 + (row_ok ? c16 : 0);
-  const int lo_row = chunk > 0 ? p_row - p_row % chunk : 0;
+  const int p_row = row_ok ? pos0 + c16 : -1;    // (no row: no key lies before it)
+  const int lo_row = chunk > 0 && row_ok ? p_row - p_row % chunk : 0;
   const bf16* q_row = q + (long)(first + (row_ok ? c16 : 0)) * ldq;
   // this wave's heads: queries as B operands, biases
+  constexpr float LOG2E = 1.4426950408889634f;
   bf16x8 qb[HPW][DC];
   float hb[HPW];
 #pragma unroll
   for (int u = 0; u < HPW; ++u) {
     const int h = wave * HPW + u;
-    hb[u] = h < H ? head_bias[h] : 0.f;
+    hb[u] = h < H ? -LOG2E * head_bias[h] : 0.f;
 #pragma unroll
     for (int dc = 0; dc < DC; ++dc) {
       const int d = dc * 32 + g4 * 8;
@@ -90,111 +105,141 @@ __global__ __launch_bounds__(256) void attention_mixed_mfma_kernel(
     for (int db = 0; db < DB; ++db) o[u][db] = (f32x4){0.f, 0.f, 0.f, 0.f};
   const long page_stride = (long)G * PAGE * (KD + VD);
   const long v_base = (long)G * PAGE * KD;
-  const float inv_cap = softcap > 0.f ? 1.f / softcap : 0.f;
+  // tanh(y) = 1 - 2 / (1 + exp(2 y)), |y| capped so that exp stays finite; sigmoid(x) = 1 / (1 + exp(-x)); both on base 2
+  const float to_cap = softcap > 0.f ? 2.f * LOG2E * scale / softcap : 0.f, from_cap = -LOG2E * softcap, plain = -LOG2E * scale;
   const int s_first = k_first / 32, s_last = p_hi / 32;
-  for (int s = s_first + split; s <= s_last; s += n_splits) {
-    // the step's two pages; one past the item's last position is not looked up
-    const bf16* base[2];
-    bool page_ok[2];
+  // a step's two pages; one past the item's last position is not looked up
+  auto page_of = [&](int s, int t) { return bt[min(s * 32 + t * 16, p_hi) / PAGE]; };
+  auto load_keys = [&](bf16x8 (&ka)[2][DC], const int (&page)[2], int kv_head) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const int key0 = s * 32 + t * 16;
-      page_ok[t] = key0 <= p_hi;
-      base[t] = plane + (long)bt[(page_ok[t] ? key0 : p_hi) / PAGE] * page_stride;
+      const bf16* kp = plane + (long)page[t] * page_stride + (long)kv_head * PAGE * KD + (long)c16 * KD;
+#pragma unroll
+      for (int dc = 0; dc < DC; ++dc) {
+        const int d = dc * 32 + g4 * 8;
+        const bool ok = d < KD;
+        const bf16x8 kv = amx_load8(kp + (ok ? d : 0));
+        ka[t][dc] = ok ? kv : (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
+      }
+    }
+  };
+  bf16x4 va[DB][2];
+  auto load_values = [&](const int (&page)[2], int kv_head) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const bf16* vp = plane + (long)page[t] * page_stride + v_base + (long)kv_head * VD * PAGE + (long)c16 * PAGE + g4 * 4;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) va[db][t] = amx_load4(vp + (long)db * 16 * PAGE);
+    }
+  };
+  const int kv_first = min(wave * HPW, H - 1) / group_size;      // the key/value head of the wave's first head
+  int page[2], page_next[2];
+  bf16x8 ka[2][DC];
+  int s = s_first + split;
+  if (s <= s_last) {
+    page[0] = page_of(s, 0);
+    page[1] = page_of(s, 1);
+    load_keys(ka, page, kv_first);
+  }
+  for (; s <= s_last; s += n_splits) {
+    const bool more = s + n_splits <= s_last;
+    if (more) {
+      page_next[0] = page_of(s + n_splits, 0);
+      page_next[1] = page_of(s + n_splits, 1);
+    }
+    bool seen[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int j = s * 32 + (e / 4) * 16 + g4 * 4 + e % 4;
+      seen[e] = j <= p_row && j >= lo_row;
     }
     // scores and weights of this wave's heads; the keys of a key/value head are fetched once for the heads that share it
-    bf16x8 ka[2][DC];
-    int kv_have = -1;
+    int kv_have = kv_first;
 #pragma unroll
     for (int u = 0; u < HPW; ++u) {
       const int h = wave * HPW + u;
       if (h < H) {
-        const int kv_head = h / group_size;
-        if (kv_head != kv_have) {
-          kv_have = kv_head;
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            const bf16* kp = base[t] + (long)kv_head * PAGE * KD + (long)c16 * KD;
-#pragma unroll
-            for (int dc = 0; dc < DC; ++dc) {
-              const int d = dc * 32 + g4 * 8;
-              const bool ok = d < KD;
-              const bf16x8 kv = amx_load8(kp + (ok ? d : 0));
-              ka[t][dc] = ok ? kv : (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
-            }
-          }
+        if (h / group_size != kv_have) {
+          kv_have = h / group_size;
+          load_keys(ka, page, kv_have);
         }
-        f32x4 st[2];
+        float* dst = wl + ((long)h * TIS_WAVE + lane) * 8;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-          st[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+          f32x4 st = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int dc = 0; dc < DC; ++dc) st[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[t][dc], qb[u][dc], st[t], 0, 0, 0);
-        }
-        float w[8];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
+          for (int dc = 0; dc < DC; ++dc) st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[t][dc], qb[u][dc], st, 0, 0, 0);
+          f32x4 w;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int j = s * 32 + t * 16 + g4 * 4 + i;
-            float x = st[t][i] * scale;
-            // tanh(y) = 1 - 2 / (1 + exp(2 y)), on the fast exponential (|y| is capped so that exp stays finite)
-            if (softcap > 0.f) x = softcap * (1.f - 2.f / (1.f + __expf(2.f * fminf(fmaxf(x * inv_cap, -15.f), 15.f))));
-            const float sg = 1.f / (1.f + __expf(-(x + hb[u])));
-            w[t * 4 + i] = (row_ok && j <= p_row && j >= lo_row) ? sg : 0.f;
+            float x;               // minus the capped score with its bias, times log2 e
+            if (softcap > 0.f) {
+              const float e2 = amx_exp2(fminf(fmaxf(st[i] * to_cap, -30.f * LOG2E), 30.f * LOG2E));
+              x = fmaf(from_cap, fmaf(-2.f, amx_rcp(1.f + e2), 1.f), hb[u]);
+            } else {
+              x = fmaf(st[i], plain, hb[u]);
+            }
+            w[i] = seen[t * 4 + i] ? amx_rcp(1.f + amx_exp2(x)) : 0.f;
           }
-        float* dst = wl + ((long)h * TIS_WAVE + lane) * 8;
-        *reinterpret_cast<f32x4*>(dst) = (f32x4){w[0], w[1], w[2], w[3]};
-        *reinterpret_cast<f32x4*>(dst + 4) = (f32x4){w[4], w[5], w[6], w[7]};
+          *reinterpret_cast<f32x4*>(dst + t * 4) = w;
+        }
       }
     }
-    __syncthreads();
+    if (more) load_keys(ka, page_next, kv_first);
+    load_values(page, kv_first);
+    // (not __syncthreads, which also waits for what is under way from memory)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
     // the mixture for this wave's heads, from all heads' weights of the lane's own keys and row
     float m[HPW][8];
 #pragma unroll
     for (int u = 0; u < HPW; ++u)
 #pragma unroll
       for (int e = 0; e < 8; ++e) m[u][e] = 0.f;
+#pragma unroll 4
     for (int gg = 0; gg < H; ++gg) {
       const float* src = wl + ((long)gg * TIS_WAVE + lane) * 8;
       const f32x4 a = *reinterpret_cast<const f32x4*>(src), b = *reinterpret_cast<const f32x4*>(src + 4);
+      float tt[HPW];
 #pragma unroll
-      for (int u = 0; u < HPW; ++u) {
-        const int h = wave * HPW + u;
-        const float tt = h < H ? tk[h * H + gg] : 0.f;
+      for (int u = 0; u < HPW; ++u) tt[u] = tk[gg * HM + wave * HPW + u];
+#pragma unroll
+      for (int u = 0; u < HPW; ++u)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          m[u][e] += tt * a[e];
-          m[u][4 + e] += tt * b[e];
+          m[u][e] = fmaf(tt[u], a[e], m[u][e]);
+          m[u][4 + e] = fmaf(tt[u], b[e], m[u][4 + e]);
         }
-      }
     }
     // O^T += V^T . m^T
+    int v_have = -1;
 #pragma unroll
     for (int u = 0; u < HPW; ++u) {
       const int h = wave * HPW + u;
       if (h < H) {
+        if (h / group_size != v_have) {
+          if (v_have >= 0) load_values(page, h / group_size);
+          v_have = h / group_size;
+          if (s * 32 + 31 > p_hi) {              // slots past the item's last position
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                if (s * 32 + (e / 4) * 16 + g4 * 4 + e % 4 > p_hi) va[db][e / 4][e % 4] = static_cast<__bf16>(0.f);
+          }
+        }
         bf16x8 pb;
 #pragma unroll
         for (int e = 0; e < 8; ++e) pb[e] = static_cast<__bf16>(m[u][e]);
-        const long v_head = v_base + (long)(h / group_size) * VD * PAGE;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-          bf16x8 va;
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            const bf16x4 x = amx_load4(base[t] + v_head + (long)(db * 16 + c16) * PAGE + g4 * 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const bool ok = page_ok[t] && s * 32 + t * 16 + g4 * 4 + e <= p_hi;
-              va[t * 4 + e] = ok ? x[e] : static_cast<__bf16>(0.f);
-            }
-          }
-          o[u][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb, o[u][db], 0, 0, 0);
+          const bf16x8 v8 = __builtin_shufflevector(va[db][0], va[db][1], 0, 1, 2, 3, 4, 5, 6, 7);
+          o[u][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, pb, o[u][db], 0, 0, 0);
         }
       }
     }
-    __syncthreads();      // the next step's weights overwrite this step's
+    page[0] = page_next[0];
+    page[1] = page_next[1];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");      // the next step's weights overwrite this step's
   }
   // O^T[channel = db * 16 + g4 * 4 + i][row = c16]
   if (!row_ok) return;
@@ -219,6 +264,7 @@ __global__ __launch_bounds__(256) void attention_mixed_mfma_kernel(
   }
 }
 
+// (eight parts are asked for at a time: with a runtime count one after the other, 33 parts of 5 rows took 9.4 us, now 4.1)
 __global__ __launch_bounds__(256) void attention_mixed_sum_kernel(const float* __restrict__ partial, int n_splits,
                                                                   bf16* __restrict__ out, long ldo, int rows, int n_out) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
@@ -226,7 +272,16 @@ __global__ __launch_bounds__(256) void attention_mixed_sum_kernel(const float* _
   const long r = i / n_out;
   const int c = (int)(i % n_out);
   float a = 0.f;
-  for (int s = 0; s < n_splits; ++s) a += partial[(r * n_splits + s) * n_out + c];
+  const float* mine = partial + r * n_splits * n_out + c;
+  int s = 0;
+  for (; s + 8 <= n_splits; s += 8) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = mine[(long)(s + i) * n_out];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a += v[i];
+  }
+  for (; s < n_splits; ++s) a += mine[(long)s * n_out];
   out[r * ldo + c] = static_cast<bf16>(a);
 }
 
@@ -255,7 +310,7 @@ TIS_EXPORT int tis_attention_mixed_mfma(const void* q, long ldq, const void* pla
   if (ldq % 8 || ldo % 4 || ((uintptr_t)q % 16) || ((uintptr_t)out % 8))
     return tis_fail("attention_mixed_mfma: rows of q and out must be 16 and 8 bytes aligned");
   if (n_splits > 1 && (!partial || ((uintptr_t)partial % 16))) return tis_fail("attention_mixed_mfma: key splits without a workspace");
-  const size_t lds = ((size_t)((H * H + 3) & ~3) + (size_t)H * TIS_WAVE * 8) * sizeof(float);
+  const size_t lds = ((size_t)16 * HPW * HPW + (size_t)H * TIS_WAVE * 8) * sizeof(float);
   if (lds > 64 * 1024) return tis_fail("attention_mixed_mfma: %d heads need %zu bytes of LDS", H, lds);
   attention_mixed_mfma_kernel<<<dim3(n_items, n_splits), 256, lds, stream>>>(
       (const bf16*)q, ldq, (const bf16*)plane, block_tables, bt_ld, row_seq, positions, items, (bf16*)out, ldo, partial, n_splits,
