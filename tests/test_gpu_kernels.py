@@ -1048,3 +1048,16 @@ def test_grouped_product_in_tiles_numbered_through(ops_for, groups, line, N, K, 
             else:
                 gate, up = want[:, 0::2].clamp(max=7.0), want[:, 1::2].clamp(-7.0, 7.0)
                 torch.testing.assert_close(out[perm[e].long()].double(), gate * torch.sigmoid(1.702 * gate) * (up + 1.0), rtol=8e-3, atol=2e-3)
+
+
+@pytest.mark.parametrize("M", [1, 7, 8])
+@pytest.mark.parametrize("N,K", [(1536, 4096), (40, 4096), (2044, 4032), (24, 8192)])
+def test_few_rows_in_batches_of_eight_steps(ops_for, M, N, K):
+    """A K that gives each of eight waves eight steps (4,096 and, short of the last step, 4,032), or sixteen: 32-bit sums against 64
+    bits, and a row's bits do not depend on the others."""
+    ops = ops_for(torch.bfloat16)
+    x, w = rnd((M, K), torch.bfloat16, 901).cuda(), rnd((N, K), torch.bfloat16, 902, K ** -0.5).cuda()
+    got = ops.linear(x, w, out_dtype=torch.float32)
+    bound = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((got.double() - x.double() @ w.double().T).abs() <= bound).all()
+    assert torch.equal(ops.linear(x[M - 1:], w, out_dtype=torch.float32)[0], got[M - 1])

@@ -63,8 +63,8 @@ struct RopeArgs {
 // GS_WAVES: waves per workgroup; U: steps of K whose loads a wave issues together before the first product.
 // Eight waves of three or four steps measured best on MI355X for K of 1536 to 4096 (5.6 us for a 25 MB matrix,
 // 23 us for the 147 MB output table: 80 % of the HBM peak); four waves where K is too short to feed eight. Batches
-// of eight steps, or sixteen waves, so that all of a wave's loads are in flight at once, measured the same within
-// noise (the gated product at 64 rows slower: fewer workgroups fit a compute unit).
+// of eight steps where a wave has eight (K of 4096: all its loads in flight at once) take 0.56 us off; sixteen waves measured the
+// same within noise (the gated product at 64 rows slower: fewer workgroups fit a compute unit).
 //
 // MB: blocks of 16 rows of X that share every weight tile a wave loads, and CT: column tiles of 16 a workgroup
 // owns. One of each is built. With two row blocks a wave fetches its own pieces of twice the activations, 16 bytes a
@@ -653,7 +653,8 @@ static int launch(const void* X, long x_ld, const void* W, const float* gain, fl
   if (steps >= 24) {
     waves = 8;
     const int per_wave = (steps + 7) / 8;
-    u = (per_wave % 3 == 0 && per_wave % 4 != 0) ? 3 : 4;
+    // (eight where a wave has them: 1536 x 4096 from cold memory, us, 1 row 6.80 / 6.24, 8 rows 7.41 / 6.84)
+    u = per_wave % 8 == 0 ? 8 : (per_wave % 3 == 0 && per_wave % 4 != 0) ? 3 : 4;
   } else {
     waves = 4;
     u = (steps % 3 == 0 && steps % 4 != 0) || steps == 12 ? 3 : 4;
@@ -665,7 +666,7 @@ static int launch(const void* X, long x_ld, const void* W, const float* gain, fl
         (const bf16*)X, x_ld, (const bf16*)W, gain, eps, (const bf16*)R, r_ld, (TO*)C, c_ld, M, N, K, rope);     \
     return 0;                                                                                                    \
   }
-  CFG(4, 3) CFG(4, 4) CFG(8, 3) CFG(8, 4)
+  CFG(4, 3) CFG(4, 4) CFG(8, 3) CFG(8, 4) CFG(8, 8)
 #undef CFG
   return tis_fail("gemm_skinny: no kernel for %d waves of %d steps", waves, u);
 }

@@ -118,9 +118,9 @@ TIS_EXPORT int tis_gemm_tiles(const void* X, long x_ld, const void* W, const voi
   // The tile: the one that is estimated to end first, by the microseconds a step of 64 takes with one or more workgroups a
   // compute unit (measured at K of 1,408 to 5,632; the clock falls as more of the chip works, hence 1.36 to 1.85 for the largest):
   //   256 x 256, eight waves, two buffers    1.36 up to 0.7 workgroups a unit, then to 1.72 at one; 1.85 a full round
-  //   128 x 192, four waves, two buffers     0.79 up to one a unit, two share one: 0.79 for each on average
+  //   128 x 192, four waves, two buffers     0.79 up to one a unit; two share one: from 1.25 on, 0.79 for each on average
   //   128 x 128, eight waves, four buffers   0.47, and 0.6 a further round
-  //   64 x 64, four waves, four buffers      0.21 up to one a unit, two share one: 0.21 for each on average
+  //   64 x 64, four waves, four buffers      0.21 up to one a unit; two share one: from 0.42 on, 0.21 for each on average
   // (us, 256 / 192 / 128 / 64, 2,048 inner columns: 2,048 x 2,048 48.4, 31.4, 22.7, 30.5; 2,048 x 2,816 47.0, 31.3, 33.0, 39.2;
   // 2,048 x 5,120 49.0, 48.6, 51.9, 66.5; 1,800 x 8,192 62.8, 71.3, 70.8, 98.2; 1,536 x 11,264 102.9, 75.1, 84.9, 110.0;
   // 1,800 x 32,000 247, 280, 333, 420; 700 x 1,024 x 2,816 59.4, 37.4, 20.6, 13.8.)
@@ -134,7 +134,8 @@ TIS_EXPORT int tis_gemm_tiles(const void* X, long x_ld, const void* W, const voi
     float t;
     if (i == 0) t = 1.85f * full + (part > 0.f ? fmaxf(1.36f, 1.36f + 1.2f * (part - 0.7f)) : 0.f);
     else if (i == 2) t = 0.47f + 0.6f * (ceilf(r) - 1.f);
-    else t = (i == 1 ? 0.79f : 0.21f) * fmaxf(r, 1.f);
+    else if (i == 1) t = r <= 1.f ? 0.79f : fmaxf(1.25f, 0.79f * r);
+    else t = r <= 1.f ? 0.21f : fmaxf(0.42f, 0.21f * r);
     if (i == 0 || t < best) best = t, pick = i, tiles = n;
   }
   if (tiles >= (1L << 31)) return tis_fail("gemm_tiles: %ld tiles are more than a grid holds", tiles);
