@@ -55,6 +55,39 @@ def close(a, b, dtype, what, tol=None):
 
 # ---- kernels ---------------------------------------------------------------------------------------------------
 
+# Rows read four values at a time, at the edges of what a thread keeps (4 x 256, 4 x 512, 4 x 1,024 and 16 x 256 values a workgroup)
+# and of the rule on rows (64); a branch that starts a value off (shift 1) cannot be read so and takes the kernel of single values.
+# The bounds are those of the other tests of these kernels: 32-bit sums in another order, or one rounding to bfloat16.
+@pytest.mark.parametrize("shift", [8, 1])
+@pytest.mark.parametrize("n,D", [(1, 4), (3, 1020), (65, 1024), (64, 1028), (65, 2048), (2, 2052), (64, 4096), (66, 4096), (5, 4100)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_sums_and_norms_in_fours(dtype, n, D, shift):
+    from tiny_inference_server_amd.ops.hip_ops import ChosenExperts
+    ops, ref = hip_ops(dtype), TorchOps("cpu", DT[dtype])
+    g = torch.Generator().manual_seed(D + n)
+    x, lines, extra = torch.randn(n, D, generator=g) * 3 + 0.7, torch.randn(2 * n, D, generator=g), torch.randn(n, D, generator=g)
+    wide = torch.randn(n, D + 8, generator=g)
+    gain, bias, ygain = (1 + 0.2 * torch.randn(D, generator=g) for _ in range(3))
+    ids, wts = torch.randint(0, 5, (n, 2), generator=g, dtype=torch.int32), torch.rand(n, 2, generator=g)
+    rows = torch.randn(n, D, generator=g).to(DT[dtype])
+    cols = slice(shift, shift + D)
+    for norm in (("layer", gain, bias, 1e-5), ("rms", gain, None, 1e-5)):
+        for chosen in (False, True):
+            res = []
+            for o, dev in ((ops, "cuda"), (ref, "cpu")):
+                m = lambda t: None if t is None else t.to(dev)
+                y = (ChosenExperts(m(lines), m(ids), m(wts), 4, m(rows), m(extra), None) if chosen else m(wide)[:, cols])
+                res.append(o.residual_norm(m(x.clone()), y, y_rms=(m(ygain), 1e-6), copy=True,
+                                           norm=(norm[0], m(norm[1]), m(norm[2]), norm[3])))
+            for a, b, kind, what in zip(res[0], res[1], ("float32", dtype, dtype), ("sum", "copy", "norm")):
+                close(a, b, kind, what)
+    got = ops.gated_postnorm(x.cuda(), [(wide.cuda()[:, cols], 1.3), (extra.cuda(), 0.7)], wide.cuda()[:, cols], bias.cuda(), 1.9,
+                             gain.cuda(), 1e-5)
+    want = ref.gated_postnorm(x, [(wide[:, cols], 1.3), (extra, 0.7)], wide[:, cols], bias, 1.9, gain, 1e-5)
+    close(got[0], want[0], "float32", "gated_postnorm 32-bit")
+    close(got[1], want[1], dtype, "gated_postnorm")
+
+
 @pytest.mark.parametrize("D", [44, 300, 1500, 4200])      # (a row in 4 or 16 registers a thread, or in memory)
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_sums_and_norms_of_the_stream(dtype, D):

@@ -79,6 +79,69 @@ __global__ __launch_bounds__(S32_THREADS) void gated_postnorm_kernel(
   }
 }
 
+// Four neighbouring values at a time, 32-bit or in the compute type (16- or 8-byte pieces).
+__device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+__device__ __forceinline__ float4 load4(const bf16* p) {
+  const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
+  return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+}
+__device__ __forceinline__ void store4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
+__device__ __forceinline__ void store4(bf16* p, float4 v) {
+  *reinterpret_cast<bf16x4*>(p) = (bf16x4){static_cast<__bf16>(v.x), static_cast<__bf16>(v.y), static_cast<__bf16>(v.z), static_cast<__bf16>(v.w)};
+}
+__device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+__device__ __forceinline__ float4 mul4(float4 a, float4 b) { return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w); }
+__device__ __forceinline__ float4 scale4(float f, float4 a) { return make_float4(f * a.x, f * a.y, f * a.z, f * a.w); }
+__device__ __forceinline__ float sum4(float4 a) { return (a.x + a.y) + (a.z + a.w); }
+__device__ __forceinline__ float square4(float4 a) { return (a.x * a.x + a.y * a.y) + (a.z * a.z + a.w * a.w); }
+// whether rows of 32-bit numbers at p, `ld` apart, may be read in such pieces (a null pointer may: it is not read)
+static inline bool fours32(const void* p, long ld) { return !p || ((uintptr_t)p % 16 == 0 && ld % 4 == 0); }
+static inline bool foursT(const void* p, long ld, int dtype) { return !p || ((uintptr_t)p % (dtype == TIS_F32 ? 16 : 8) == 0 && ld % 4 == 0); }
+
+// The same for a width that is a multiple of four, PER pieces of four values a thread (width <= 4 PER THREADS): what bounds it
+// is memory, and a lane's 4-byte loads of five arrays kept too little under way. us, 2,048 wide, before / now:
+// 8 rows 7.2 / 3.4, 300 rows of 1,024 4.8 / 3.3, 1,531 rows 17.4 / 13.1, 2,048 rows 18.2 / 15.4.
+template <typename T, int PER>
+__global__ __launch_bounds__(S32_THREADS) void gated_postnorm_fours_kernel(
+    const float* __restrict__ x, const float* __restrict__ y0, long ld0, float s0, const float* __restrict__ y1, long ld1,
+    float s1, const float* __restrict__ gate, long ldg, const float* __restrict__ bias, float alpha,
+    const float* __restrict__ gain, float eps, float* __restrict__ out32, T* __restrict__ outT, int D) {
+  __shared__ float red[16];
+  const long r = blockIdx.x;
+  float4 xv[PER], y0v[PER], y1v[PER], zv[PER], gv[PER];
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = (threadIdx.x + k * S32_THREADS) * 4;
+    const bool in = c < D;
+    xv[k] = in ? load4(x + r * D + c) : zero;
+    y0v[k] = in ? load4(y0 + r * ld0 + c) : zero;
+    y1v[k] = y1 && in ? load4(y1 + r * ld1 + c) : zero;
+    zv[k] = gate && in ? load4(gate + r * ldg + c) : zero;
+    if (gate && bias && in) zv[k] = add4(zv[k], load4(bias + c));
+    gv[k] = in ? load4(gain + c) : zero;
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    float4 y = scale4(s0, y0v[k]);
+    if (y1) y = add4(y, scale4(s1, y1v[k]));
+    if (gate) y = mul4(y, make_float4(sigmoid_f(zv[k].x), sigmoid_f(zv[k].y), sigmoid_f(zv[k].z), sigmoid_f(zv[k].w)));
+    xv[k] = add4(scale4(alpha, xv[k]), y);
+    ss += square4(xv[k]);
+  }
+  const float inv = 1.f / sqrtf(block_sum(ss, red) / (float)D + eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = (threadIdx.x + k * S32_THREADS) * 4;
+    if (c >= D) continue;
+    const float4 v = mul4(scale4(inv, xv[k]), gv[k]);
+    store4(out32 + r * D + c, v);
+    if (outT) store4(outT + r * D + c, v);
+  }
+}
+
 // out = x / sqrt(mean(x^2) + eps) * gain, from the 32-bit stream into the compute type
 template <typename T>
 __global__ __launch_bounds__(S32_THREADS) void rmsnorm32_kernel(const float* __restrict__ x, long ldx, const float* __restrict__ gain,
@@ -266,6 +329,89 @@ __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
   each([&](float v, int c, float g, float b) { normed[r * ldn + c] = from_f<T>((v - mean) * inv * g + b); });
 }
 
+// The same for a width that is a multiple of four, PER pieces of four values a thread (width <= 4 PER THREADS): a lane's
+// 4-byte loads kept too little under way for many rows, and a row alone waits for fewer of the wider ones. us, 2,048 wide,
+// before / now: a branch with a norm of its own, copy and next norm: 1 row 4.6 / 3.1, 1,531 rows 14.5 / 9.2, 2,048 rows
+// 17.9 / 11.6; two chosen experts and a shared term: 8 rows 6.2 / 3.8, 65 rows 11.0 / 4.8, 2,048 rows 36.9 / 15.8.
+template <typename T, int PER, int THREADS>
+__global__ __launch_bounds__(THREADS) void residual_norm_fours_kernel(
+    const float* __restrict__ x, const float* __restrict__ y_in, long ldy, const float* __restrict__ y_gain, float y_eps,
+    float* __restrict__ out32, T* __restrict__ copy, long ldc, int norm_kind, const float* __restrict__ gain,
+    const float* __restrict__ bias, float eps, T* __restrict__ normed, long ldn, int D, ChosenSum cs) {
+  __shared__ float red[16];
+  const long r = blockIdx.x;
+  const bool y = y_in != nullptr || cs.ids != nullptr;        // whether there is a branch at all
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f), one = make_float4(1.f, 1.f, 1.f, 1.f);
+  float4 xv[PER], yv[PER], ygv[PER], gv[PER], bv[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = (threadIdx.x + k * THREADS) * 4;
+    const bool in = c < D;
+    xv[k] = in ? load4(x + r * D + c) : zero;
+    yv[k] = y && !cs.ids && in ? load4(y_in + r * ldy + c) : zero;
+    ygv[k] = y && y_gain && in ? load4(y_gain + c) : one;
+    gv[k] = norm_kind && in ? load4(gain + c) : zero;
+    bv[k] = norm_kind == 1 && bias && in ? load4(bias + c) : zero;
+  }
+  if (cs.ids) {                    // (a row's choices are the same for all its threads: scalar loads)
+    for (int i = 0; i < cs.top; ++i) {
+      const int e = cs.ids[r * cs.top + i];
+      const float w = cs.weights[r * cs.top + i];
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int c = (threadIdx.x + k * THREADS) * 4;
+        if (c < D)
+          yv[k] = add4(yv[k], scale4(w, e < cs.n_experts ? load4(y_in + (r * cs.top + i) * ldy + c)
+                                                         : load4(static_cast<const T*>(cs.rows) + r * cs.ldr + c)));
+      }
+    }
+    if (cs.extra) {
+      const float w = cs.extra_gate ? sigmoid_f(cs.extra_gate[r * cs.ldg]) : 1.f;
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int c = (threadIdx.x + k * THREADS) * 4;
+        if (c < D) yv[k] = add4(yv[k], scale4(w, load4(cs.extra + r * cs.lde + c)));
+      }
+    }
+  }
+  float y_inv = 1.f;
+  if (y && y_gain) {
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) ss += square4(yv[k]);
+    y_inv = 1.f / sqrtf(block_sum(ss, red) / (float)D + y_eps);
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = (threadIdx.x + k * THREADS) * 4;
+    if (c >= D) continue;
+    if (y) xv[k] = add4(xv[k], y_gain ? mul4(scale4(y_inv, yv[k]), ygv[k]) : yv[k]);
+    store4(out32 + r * D + c, xv[k]);
+    if (copy) store4(copy + r * ldc + c, xv[k]);
+    s += norm_kind == 2 ? square4(xv[k]) : sum4(xv[k]);
+  }
+  if (!normed || norm_kind == 0) return;
+  float mean = 0.f;
+  if (norm_kind == 1) {
+    mean = block_sum(s, red) / (float)D;
+    s = 0.f;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int c = (threadIdx.x + k * THREADS) * 4;
+      if (c < D) s += square4(add4(xv[k], make_float4(-mean, -mean, -mean, -mean)));
+    }
+  }
+  const float inv = 1.f / sqrtf(block_sum(s, red) / (float)D + eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = (threadIdx.x + k * THREADS) * 4;
+    if (c >= D) continue;
+    const float4 v = norm_kind == 2 ? xv[k] : add4(xv[k], make_float4(-mean, -mean, -mean, -mean));
+    store4(normed + r * ldn + c, add4(mul4(scale4(inv, v), gv[k]), bv[k]));
+  }
+}
+
 __device__ __forceinline__ float gelu_tanh_f(float z) {
   return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
@@ -329,12 +475,21 @@ TIS_EXPORT int tis_gated_postnorm(int dtype, const float* x, const float* y0, lo
 #define S32_POSTNORM(T, PER)                                                                                           \
   gated_postnorm_kernel<T, PER><<<rows, S32_THREADS, 0, stream>>>(x, y0, ld0, s0, y1, ld1, s1, gate, ldg, bias, alpha, gain, \
                                                                   eps, out32, (T*)outT, D)
+#define S32_POSTNORM4(T, PER)                                                                                          \
+  gated_postnorm_fours_kernel<T, PER><<<rows, S32_THREADS, 0, stream>>>(x, y0, ld0, s0, y1, ld1, s1, gate, ldg, bias, alpha, \
+                                                                        gain, eps, out32, (T*)outT, D)
+  const bool fours = D % 4 == 0 && D <= 16 * S32_THREADS && fours32(x, D) && fours32(y0, ld0) && fours32(y1, ld1) &&
+                     fours32(gate, ldg) && fours32(bias, 0) && fours32(gain, 0) && fours32(out32, D) && foursT(outT, D, dtype);
 #define S32_POSTNORM_BY_WIDTH(T)                         \
-  if (D <= 4 * S32_THREADS) { S32_POSTNORM(T, 4); }      \
+  if (fours && D <= 4 * S32_THREADS) { S32_POSTNORM4(T, 1); }      \
+  else if (fours && D <= 8 * S32_THREADS) { S32_POSTNORM4(T, 2); } \
+  else if (fours) { S32_POSTNORM4(T, 4); }                \
+  else if (D <= 4 * S32_THREADS) { S32_POSTNORM(T, 4); } \
   else if (D <= 16 * S32_THREADS) { S32_POSTNORM(T, 16); } \
   else { S32_POSTNORM(T, 0); }
   S32_DISPATCH(S32_POSTNORM_BY_WIDTH(float), S32_POSTNORM_BY_WIDTH(bf16))
 #undef S32_POSTNORM_BY_WIDTH
+#undef S32_POSTNORM4
 #undef S32_POSTNORM
   return tis_launch_status("gated_postnorm");
 }
@@ -398,14 +553,27 @@ TIS_EXPORT int tis_residual_norm(int dtype, const float* x, const float* y, long
 #define S32_RESIDUAL(T, PER, THREADS)                                                                                      \
   residual_norm_kernel<T, PER, THREADS><<<rows, THREADS, 0, stream>>>(x, y, ldy, y_gain, y_eps, out32, (T*)copy, ldc, norm_kind, \
                                                                       gain, bias, eps, (T*)normed, ldn, D, cs)
-  // (a step of few rows leaves most of the chip idle: the widest workgroups then, for the shortest chains)
+#define S32_RESIDUAL4(T, PER, THREADS)                                                                                     \
+  residual_norm_fours_kernel<T, PER, THREADS><<<rows, THREADS, 0, stream>>>(x, y, ldy, y_gain, y_eps, out32, (T*)copy, ldc, \
+                                                                            norm_kind, gain, bias, eps, (T*)normed, ldn, D, cs)
+  const bool fours = D % 4 == 0 && D <= 4096 && fours32(x, D) && fours32(y, ldy) && fours32(y_gain, 0) && fours32(out32, D) &&
+                     foursT(copy, ldc, dtype) && fours32(gain, 0) && fours32(bias, 0) && foursT(normed, ldn, dtype) &&
+                     foursT(chosen_rows, ldr, dtype) && fours32(extra, lde);
+  // (a step of few rows leaves most of the chip idle: the widest workgroups then, for the shortest chains. What cannot be
+  // read in fours, or is wider than a thread's registers hold, goes through the kernel of single values.)
 #define S32_RESIDUAL_BY_WIDTH(T)                                                        \
-  if (rows <= 64 && D > 1024 && D <= 4096) { S32_RESIDUAL(T, 4, 1024); }                  \
+  if (fours && D <= 1024) { S32_RESIDUAL4(T, 1, 256); }                                 \
+  else if (fours && rows <= 64 && D <= 2048) { S32_RESIDUAL4(T, 1, 512); }              \
+  else if (fours && rows <= 64) { S32_RESIDUAL4(T, 1, 1024); }                          \
+  else if (fours && D <= 2048) { S32_RESIDUAL4(T, 2, 256); }                            \
+  else if (fours) { S32_RESIDUAL4(T, 4, 256); }                                         \
+  else if (rows <= 64 && D > 1024 && D <= 4096) { S32_RESIDUAL(T, 4, 1024); }                  \
   else if (D <= 4 * S32_THREADS) { S32_RESIDUAL(T, 4, S32_THREADS); }                     \
   else if (D <= 16 * S32_THREADS) { S32_RESIDUAL(T, 16, S32_THREADS); }                   \
   else { S32_RESIDUAL(T, 0, S32_THREADS); }
   S32_DISPATCH(S32_RESIDUAL_BY_WIDTH(float), S32_RESIDUAL_BY_WIDTH(bf16))
 #undef S32_RESIDUAL_BY_WIDTH
+#undef S32_RESIDUAL4
 #undef S32_RESIDUAL
   return tis_launch_status("residual_norm");
 }
