@@ -167,6 +167,49 @@ def test_state_scan_against_the_token_by_token_rule(kind, Hh, D, V, segment):
     assert state_gpu[[1, 2]].abs().max() == 0 and state_gpu[:, floats:].abs().max() == 0
 
 
+# Segments by matrix products at the edges of their tiles (16 rows, 16 channels, 64 and 128 channels), of whole segments and of one row
+# more, requests without rows in the middle and from more than 64 requests, a decay per head and keys shared by heads; against the
+# walk row by row. Both ways round 32-bit sums of up to 64 rows and D channels and carry them over segments: 2e-5 of the largest result, as
+# elsewhere here. A row that is not finite leaves the rows before it and the other requests alone.
+@pytest.mark.parametrize("kind,Hh,D,V,per_head", [("decay", 2, 64, 16, False), ("decay", 3, 65, 80, False), ("decay", 4, 128, 256, False),
+                                                  ("decay", 4, 128, 64, True), ("decay", 2, 48, 33, True), ("gated_max", 2, 64, 16, False),
+                                                  ("gated_max", 3, 66, 80, False), ("gated_max", 4, 128, 256, False)])
+@pytest.mark.parametrize("lens", [[128], [129, 0, 64, 63, 1], [17, 145, 16], [1] * 66 + [200, 2]])
+def test_state_scan_in_segments_by_matrix_products(kind, Hh, D, V, per_head, lens):
+    ops, ref = hip_ops("float32"), TorchOps("cpu", torch.float32)
+    g = torch.Generator().manual_seed(D + V)
+    group = 2 if Hh % 2 == 0 and per_head else 1
+    n, qk = sum(lens), Hh // group * D
+    qo, ko, vo, io, fo = 1, 1 + qk, 1 + 2 * qk, 1 + 2 * qk + Hh * V, 1 + 2 * qk + Hh * V + Hh
+    proj = torch.randn(n, 1 + 2 * qk + Hh * V + 2 * Hh, generator=g)
+    decay = torch.rand(n, Hh if per_head else Hh * D, generator=g) ** 0.1
+    bi, bf = torch.randn(Hh, generator=g), 2 + torch.randn(Hh, generator=g)
+    state = torch.randn(len(lens), ops.state_scan_floats(kind, Hh, D, V), generator=g)
+    if kind == "gated_max":      # one n and m for all blocks of value channels, as every call leaves them
+        nm = state[:, Hh * D * V:].view(len(lens), Hh, -1, D + 1)
+        nm[:] = nm[:, :, :1].clone()
+    rows, r = [], 0
+    for k in lens:
+        rows.append((r, 0, k))
+        r += k
+    def run(o, dev, p, st):
+        kw = dict(i_off=io, f_off=fo, bias_i=bi.to(dev), bias_f=bf.to(dev), cap=9.0) if kind == "gated_max" else dict(decay=decay.to(dev))
+        return o.state_scan(kind, p.to(dev), qo, ko, vo, D ** -0.5, st, fake_batch(rows, list(range(len(lens))), None, 1, dev), Hh, D, V,
+                            qk_group=group, decay_per_head=per_head, **kw)
+    want_state, got_state = state.clone(), state.cuda()
+    want, got = run(ref, "cpu", proj, want_state), run(ops, "cuda", proj, got_state)
+    close(got, want, "float32", "results")
+    close(got_state, want_state, "float32", "states")
+    bad, at = proj.clone(), lens.index(max(lens)) and sum(lens[:lens.index(max(lens))])
+    at += 70
+    bad[at, vo:vo + Hh * V] = float("nan")
+    again = run(ops, "cuda", bad, state.cuda())
+    last = sum(lens[:lens.index(max(lens)) + 1])
+    close(again[:at], want[:at], "float32", "rows before")
+    close(again[last:], want[last:], "float32", "other requests") if last < n else None
+    assert torch.isnan(again[at:last]).all()
+
+
 # ---- the engine ------------------------------------------------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

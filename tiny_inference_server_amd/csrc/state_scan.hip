@@ -15,8 +15,8 @@
 // chunk size or on what else is in the batch, bit for bit. State, gates and sums are 32-bit. Kind 1 keeps n and m once
 // per block of value channels (every block needs them, none may read what another has already advanced).
 //
-// Long portions of prompts are cut into segments of `seg_len` tokens that run side by side (`segments` > 0): the same
-// kernel walks every segment from an empty state and leaves the segment's own state, its outputs as if nothing had
+// Long portions of prompts are cut into segments of `seg_len` tokens that run side by side (`segments` > 0): up to 128 key
+// channels and 64 tokens by products of matrices (see there); beyond that the same kernel walks every segment from an empty state and leaves the segment's own state, its outputs as if nothing had
 // come before, and what ties them to the past (kind 0: the product of the decays from the segment's start to each
 // token; kind 1: the running maximum, the sum of log forget gates and n . q from the segment's start). A second kernel
 // then walks the segments of a request in order, element by element, to the state at every segment's start and the
@@ -26,6 +26,7 @@
 //           exp(m'_t - m_t) and the start's part scaled by exp(F_t + m_start - m_t); o_t as above.
 // Everything is still 32-bit; only the order of additions differs from the token-by-token walk.
 #include "common.h"
+#include <type_traits>
 
 TIS_DEFINE_LAST_ERROR(tis_state_scan)
 
@@ -62,18 +63,16 @@ struct SegArgs {
   float* aux;
 };
 
-// VB value channels a workgroup, R = 256 / VB threads a column. A request's state line keeps n and m once per 16 value
-// channels, so the walk in order runs with VB = 16; segments keep n and m once per head and may take 64 channels a
-// workgroup, which loads a head's q, k and decays a quarter as often.
-template <int KIND, int NS, bool SEG, int VB>
+// SC_VB value channels a workgroup, SC_R threads a column. A request's state line keeps n and m once per 16 value
+// channels, a segment's own state once per head.
+template <int KIND, int NS, bool SEG>
 __global__ __launch_bounds__(SC_THREADS) void state_scan_kernel(
     const float* __restrict__ proj, long ldp, int q_off, int k_off, int v_off, float q_scale,
     const float* __restrict__ decay, long ldd, int i_off, int f_off, const float* __restrict__ bias_i,
     const float* __restrict__ bias_f, float cap, float* __restrict__ state, long state_ld,
     const int* __restrict__ cu_rows, const int* __restrict__ seq_slots, float* __restrict__ out, long ldo, int H, int D,
     int V, int n_vb, int chunk, SegArgs sg, ScanLayout lay) {
-  static_assert(SEG || VB == SC_VB, "a state line keeps n and m per 16 value channels");
-  constexpr int R = SC_THREADS / VB;
+  constexpr int VB = SC_VB, R = SC_R;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int DP = R * NS;                         // a token's row in LDS: the head's channels, then zeros
   float* sq = lds;                                   // [chunk][DP]
@@ -347,38 +346,619 @@ __global__ __launch_bounds__(SC_THREADS) void segment_outputs_kernel(const float
   }
 }
 
-static constexpr int SC_WIDE_VB = 64;      // value channels of a workgroup that walks a segment, where the sizes allow
+// ---- segments by matrix products --------------------------------------------------------------------------------------
+//
+// For up to 128 key channels and segments of up to 64 rows. Row by row a segment's walk is bound by LDS: every thread reads its
+// share of a row's q, k and decays for each of its own state elements, and all that is done with them is one multiply-add each.
+// As sums over a segment's rows (S_0 the state at its start, P lower triangular, all in 32 bits, nothing divided by a decay),
+//   kind 0:  o_t = (q_t A(-1, t)) S_0 + sum_{i<=t} P(t, i) v_i,  P(t, i) = sum_d q_t k_i A(i, t);   S <- A(-1, last) S_0 + sum_i (k_i A(i, last)) v_i^T
+//            with A(i, t) the decays of rows i + 1 .. t multiplied up per channel;
+//   kind 1:  P(t, i) = (q_t . k_i) exp(f_(i+1) + .. + f_t + i_i - m'_t), each such sum of forget gates taken from row i on; the own
+//            and the start's part put together as in the segments above
+// they are products on v_mfma_f32_16x16x4_f32 (32-bit multiply-adds). Three kernels: segment_rows makes P, the scaled queries and
+// keys and a segment's decay (or its gates' sums) for every segment and head; segment_walk takes 16 value channels of a head
+// through a request's segments in order with S in registers, and leaves S at every segment's start; segment_results makes the
+// rows' outputs, all segments at once. Operands lie in the workspace as the products read them, 16 bytes a lane. A request's segments
+// are numbered through over the requests of the step, so a step of one long and many short ones needs no more room than its rows.
+// MI355X, 8 heads of 128 x 256, us row by row in segments / by products:
+// 2,048 rows 233 / 81 (kind 1: 250 / 86), two requests of 1,216 and 584 rows 229 / 70 (250 / 71), 512 rows 124 / 39, 128 rows
+// 110 / 30, eight requests of 512 rows 417 / 136. Of the 70 the rows' kernel takes 25 (LDS, pair by pair; kind 1: 15), the walk 24 (a chain of
+// one segment after another, 1 us each) and the results 25 (memory: the states at the starts twice over). Off from 64 bits by
+// 1.4e-7 / 1.2e-7 (kind 0; sums of products run in four accumulators each, which keeps their chains as short as the row by
+// row kernel's), kind 1 by 0.5e-6 to 3e-6 both ways (its division).
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+static constexpr int SP_ROWS = 64;               // rows a segment can have: four tiles of 16
+
+// What the workspace holds of a segment and head, in floats, Dp = 64 or 128 the head's channels as they are multiplied.
+// Tiles of 16 x 16 are kept as lanes hold them, [lane (g, n)][4]: P and q have row n and columns 4 g .. 4 g + 3 there, k and S
+// rows 4 g .. 4 g + 3 of column n.
+struct SegmentBlock {
+  int q, k, a, x, n, s;        // P [row tile][row tile] lies at 0; scaled q [row tile][channel tile]; scaled k [channel tile][row tile];
+                               // decays (kind 0) or the segment's own n [Dp]; m', sums of f, own n . q [64] each and m at the start;
+                               // n at the start [Dp]; S at the start [block of 16 value channels][channel tile]
+  long floats;
+  __host__ __device__ SegmentBlock(int D, int V) {
+    const int Dp = D <= 64 ? 64 : 128;
+    q = SP_ROWS * SP_ROWS;
+    k = q + SP_ROWS * Dp;
+    a = k + SP_ROWS * Dp;
+    x = a + Dp;
+    n = x + 4 * SP_ROWS;      // (every piece begins on a whole line of memory)
+    s = n + Dp;
+    floats = s + (long)((V + 15) / 16) * 16 * Dp;
+  }
+};
+// The most segments that `rows` rows of `n_seqs` requests can have.
+__host__ __device__ constexpr long sp_most(long rows, int seg_len, int n_seqs) { return rows / seg_len + n_seqs; }
+
+struct Segment {
+  int first, n;                // its first row of the step, its rows; n 0: there is none of this number
+};
+// The segment numbered `at` (a lane a request, 64 at a time).
+__device__ __forceinline__ Segment find_segment(const int* __restrict__ cu_rows, int n_seqs, int seg_len, int at) {
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  for (int s0 = 0; s0 < n_seqs; s0 += 64) {
+    const int s = s0 + lane;
+    const int rows = s < n_seqs ? cu_rows[s + 1] - cu_rows[s] : 0;
+    const int own = (rows + seg_len - 1) / seg_len;
+    int upto = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, 64);
+      if (lane >= o) upto += v;
+    }
+    const unsigned long long holds = __ballot(before + upto > at);
+    if (holds) {
+      const int which = __ffsll(holds) - 1;
+      const int c = at - before - __shfl(upto - own, which, 64);
+      return {__builtin_amdgcn_readfirstlane(cu_rows[s0 + which] + c * seg_len),
+              __builtin_amdgcn_readfirstlane(min(seg_len, __shfl(rows, which, 64) - c * seg_len))};
+    }
+    before += __shfl(upto, 63, 64);
+  }
+  return {0, 0};
+}
+
+// Sum over the 16 lanes 16 r .. 16 r + 15, every lane gets it, by moves inside the row of lanes.
+__device__ __forceinline__ float sp_row_sum(float v) {
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true));    // quad_perm [2,3,0,1]
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, true));   // row_half_mirror
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, true));   // row_mirror
+  return v;
+}
+
+// grid (heads, segments), eight waves. Kind 0 has to take the decays between two rows per channel, which no product of matrices
+// can where it may not divide: inside 16 rows that is done pair by pair (as thread (i, l): row i, channels 4 l .. 4 l + 3 and
+// so on by 64), between tiles of 16 rows by a product of q scaled from its tile's start with k scaled to its tile's end, with the tiles
+// between them multiplied into q. LDS rows are 4 floats longer than the channels: 16 lanes read 16 rows at one column.
+template <int KIND, int NT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void segment_rows_kernel(const float* __restrict__ proj, long ldp, int q_off, int k_off,
+                                                           float q_scale, const float* __restrict__ decay, long ldd, int i_off,
+                                                           int f_off, const float* __restrict__ bias_i,
+                                                           const float* __restrict__ bias_f, float cap,
+                                                           const int* __restrict__ cu_rows, int n_seqs, int seg_len,
+                                                           float* __restrict__ work, int H, int D, int V, ScanLayout lay) {
+  constexpr int Dp = 64 * NT, LD = Dp + 4, LP = SP_ROWS + 4;
+  __shared__ __attribute__((aligned(16))) float sq[SP_ROWS][LD], sk[SP_ROWS][LD], sp[SP_ROWS][LP];
+  __shared__ __attribute__((aligned(16))) float sa[KIND == 0 ? SP_ROWS : 1][LD], total[4][Dp];     // decays; their products over a tile's rows
+  __shared__ float sw[KIND == 1 ? SP_ROWS : 1][LP], gate_i[SP_ROWS], gate_f[SP_ROWS], gate_m[SP_ROWS];
+  const Segment seg = find_segment(cu_rows, n_seqs, seg_len, blockIdx.y);
+  if (seg.n <= 0) return;                        // (the grid is as wide as there could be segments)
+  const int h = blockIdx.x, hq = h / lay.qk_group, t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, g = lane >> 4, n = lane & 15;
+  const int nc = (seg.n + 15) / 16;              // tiles of rows
+  const SegmentBlock at(D, V);
+  float* mine = work + ((long)blockIdx.y * H + h) * at.floats;
+  {
+    constexpr int STEP = 512 / Dp, PER = SP_ROWS / STEP;   // a thread's rows, STEP apart, of one channel: all loads under way at once
+    const int d = t % Dp, r0 = t / Dp;
+    // (channels and rows past the last lie behind the buffers' ends: zeros)
+    const int at_p = d < D ? (r0 * (int)ldp + d) * 4 : -4, at_d = d < D ? (r0 * (int)ldd + d * lay.decay_cs) * 4 : -4;
+    const int bytes = ((seg.n - 1) * (int)ldp + D) * 4;
+    const float* row = proj + (long)seg.first * ldp + hq * D;
+    auto q_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(row + q_off), 0, bytes, 0x00020000);
+    auto k_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(row + k_off), 0, bytes, 0x00020000);
+    auto d_rows = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(KIND == 0 ? decay + (long)seg.first * ldd + h * lay.decay_hs : row), 0,
+        KIND == 0 ? ((seg.n - 1) * (int)ldd + (D - 1) * lay.decay_cs + 1) * 4 : 0, 0x00020000);
+    float q[PER], k[PER], a[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const int more = d < D ? e * STEP * (int)ldp * 4 : 0;
+      q[e] = __builtin_bit_cast(float, (int)__builtin_amdgcn_raw_buffer_load_b32(q_rows, at_p + more, 0, 0));
+      k[e] = __builtin_bit_cast(float, (int)__builtin_amdgcn_raw_buffer_load_b32(k_rows, at_p + more, 0, 0));
+      if (KIND == 0)
+        a[e] = __builtin_bit_cast(float, (int)__builtin_amdgcn_raw_buffer_load_b32(
+                                             d_rows, at_d + (d < D ? e * STEP * (int)ldd * 4 : 0), 0, 0));
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const int r = r0 + e * STEP;
+      sq[r][d] = q[e] * q_scale;
+      sk[r][d] = k[e];
+      if (KIND == 0) sa[r][d] = r < seg.n && d < D ? a[e] : 1.f;
+    }
+  }
+  if (KIND == 1 && t < 64) {                     // rows past the last take nothing and keep everything
+    const float* row = proj + (long)(seg.first + min(t, seg.n - 1)) * ldp;
+    const float xi = row[i_off + h] + bias_i[h], xf = row[f_off + h] + bias_f[h];
+    const float gi = t < seg.n ? cap * tanhf(xi / cap) : -INFINITY;
+    const float gf = t < seg.n ? sc_log_sigmoid(cap * tanhf(xf / cap)) : 0.f;
+    float m = gi, f = gf;                        // the running maximum and the sum of f up to this row
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const float mu = __shfl_up(m, o, 64), fu = __shfl_up(f, o, 64);
+      if (lane >= o) {
+        m = fmaxf(f + mu, m);
+        f += fu;
+      }
+    }
+    gate_i[t] = gi;
+    gate_f[t] = gf;
+    gate_m[t] = m;
+    mine[at.x + t] = m;
+    mine[at.x + SP_ROWS + t] = f;
+  }
+  __syncthreads();
+  if (KIND == 1) {                               // lane i, rows 8 w .. 8 w + 7: the weight of row i in row t
+    const float gi = gate_i[lane];
+    float f = 0.f;
+    for (int u = 0; u < wave * 8; ++u) f += u > lane ? gate_f[u] : 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int u = wave * 8 + e;
+      f += u > lane ? gate_f[u] : 0.f;
+      sw[u][lane] = lane <= u ? expf(f + gi - gate_m[u]) : 0.f;
+    }
+    __syncthreads();
+  } else {
+    const int i = (t % 256) / 16, l = t % 16;
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+      const int c = t / 256 * 2 + pass;
+      f32x4 qt[NT], kt[NT], upto[NT];
+      if (c < nc) {
+        float p[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) p[j] = 0.f;
+#pragma unroll
+        for (int v = 0; v < NT; ++v) {
+          const int d = l * 4 + v * 64;
+          f32x4 up = {1.f, 1.f, 1.f, 1.f}, ka = *reinterpret_cast<const f32x4*>(&sk[c * 16 + i][d]);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const f32x4 aj = *reinterpret_cast<const f32x4*>(&sa[c * 16 + j][d]);
+            const f32x4 qj = *reinterpret_cast<const f32x4*>(&sq[c * 16 + j][d]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              up[e] *= j <= i ? aj[e] : 1.f;
+              ka[e] *= j > i ? aj[e] : 1.f;
+              p[j] = fmaf(ka[e], qj[e], p[j]);
+            }
+          }
+          qt[v] = *reinterpret_cast<const f32x4*>(&sq[c * 16 + i][d]) * up;
+          kt[v] = ka;
+          upto[v] = up;
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const float ps = sp_row_sum(p[j]);
+          if (l == j) sp[c * 16 + j][c * 16 + i] = i <= j ? ps : 0.f;
+        }
+      }
+      __syncthreads();                           // the tile's rows have been read
+      if (c < nc) {
+#pragma unroll
+        for (int v = 0; v < NT; ++v) {
+          const int d = l * 4 + v * 64;
+          *reinterpret_cast<f32x4*>(&sq[c * 16 + i][d]) = qt[v];
+          *reinterpret_cast<f32x4*>(&sk[c * 16 + i][d]) = kt[v];
+          if (i == 15) *reinterpret_cast<f32x4*>(&total[c][d]) = upto[v];
+        }
+      }
+    }
+    __syncthreads();
+  }
+  for (int idx = wave; idx < 16; idx += 8) {     // P between tiles of rows (kind 1: and inside them)
+    const int J = idx / 4, I = idx % 4;
+    if (J >= nc || I > J || (KIND == 0 && I == J)) continue;
+    f32x4 part[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[r] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int tt = 0; tt < 4 * NT; ++tt) {
+      f32x4 qf = *reinterpret_cast<const f32x4*>(&sq[J * 16 + n][tt * 16 + g * 4]);
+      const f32x4 kf = *reinterpret_cast<const f32x4*>(&sk[I * 16 + n][tt * 16 + g * 4]);
+      if (KIND == 0)
+        for (int m = I + 1; m < J; ++m) qf *= *reinterpret_cast<const f32x4*>(&total[m][tt * 16 + g * 4]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) part[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[r], kf[r], part[r], 0, 0, 0);
+    }
+    const f32x4 acc = (part[0] + part[1]) + (part[2] + part[3]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = J * 16 + g * 4 + r, col = I * 16 + n;
+      sp[row][col] = KIND == 0 ? acc[r] : col <= row ? acc[r] * sw[row][col] : 0.f;
+    }
+  }
+  __syncthreads();
+  const int last = nc * 16 - 1;
+  if (KIND == 1) {
+    const int row = t / 8;
+    if (row < nc * 16) {
+      float a = 0.f;
+      for (int i = t % 8; i <= row; i += 8) a += sp[row][i];
+      a += __shfl_xor(a, 1, 64);
+      a += __shfl_xor(a, 2, 64);
+      a += __shfl_xor(a, 4, 64);
+      if (t % 8 == 0) mine[at.x + 2 * SP_ROWS + row] = a;
+    }
+    if (t < Dp) {
+      float a[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i <= last; i += 4)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a[r] += sw[last][i + r] * sk[i + r][t];
+      mine[at.a + t] = (a[0] + a[1]) + (a[2] + a[3]);
+    }
+  } else if (t < Dp) {
+    float a = 1.f;
+    for (int c = 0; c < nc; ++c) a *= total[c][t];
+    mine[at.a + t] = a;
+  }
+  for (int e = wave; e < nc * 4; e += 8) {
+    const int J = e / 4, I = e % 4;
+    if (I <= J) *reinterpret_cast<f32x4*>(mine + (e * 64 + lane) * 4) = *reinterpret_cast<const f32x4*>(&sp[J * 16 + n][I * 16 + g * 4]);
+  }
+  for (int e = wave; e < nc * 4 * NT; e += 8) {
+    const int J = e / (4 * NT), d = e % (4 * NT) * 16 + g * 4;
+    f32x4 qf = *reinterpret_cast<const f32x4*>(&sq[J * 16 + n][d]);
+    if (KIND == 0)
+      for (int m = 0; m < J; ++m) qf *= *reinterpret_cast<const f32x4*>(&total[m][d]);
+    *reinterpret_cast<f32x4*>(mine + at.q + (e * 64 + lane) * 4) = qf;
+  }
+  for (int e = wave; e < nc * 4 * NT; e += 8) {
+    const int tt = e / nc, rt = e % nc, d = tt * 16 + n;
+    float scale = 1.f;
+    if (KIND == 0)
+      for (int m = rt + 1; m < nc; ++m) scale *= total[m][d];
+    f32x4 kf;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) kf[r] = sk[rt * 16 + g * 4 + r][d] * (KIND == 0 ? scale : sw[last][rt * 16 + g * 4 + r]);
+    *reinterpret_cast<f32x4*>(mine + at.k + ((tt * 4 + rt) * 64 + lane) * 4) = kf;
+  }
+}
+
+// The rows 4 g .. 4 g + 3 of every tile of 16 of a segment's values, one column of 16 at `block`: through a buffer that ends behind
+// the segment's last value there, so that rows past the last read as zeros and an address is one register that stays (as 64-bit
+// addresses, worked out for each of 16 loads, this was most of what the walk did). Columns past the head's are other numbers of the row.
+struct ValueRows {
+  int offset[4][4];
+  int ldp4;
+  __device__ __forceinline__ ValueRows(long ldp, int g, int n) : ldp4((int)ldp * 4) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) offset[c][r] = (c * 16 + g * 4 + r) * ldp4 + n * 4;
+  }
+  __device__ __forceinline__ void fetch(f32x4 (&v)[4], const float* __restrict__ block, int cols, const Segment& seg) const {
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(block + (long)seg.first * (ldp4 / 4)), 0,
+                                                  (seg.n - 1) * ldp4 + cols * 4, 0x00020000);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        v[c][r] = __builtin_bit_cast(float, (int)__builtin_amdgcn_raw_buffer_load_b32(rsrc, offset[c][r], 0, 0));
+  }
+};
+
+// grid (heads, blocks of 16 value channels, requests), four waves of NT tiles of 16 channels each: register r of lane (g, n) in a
+// tile is channel 4 g + r of value channel n, as results of products lie. The next segment's operands are under way while
+// one is multiplied. Every block of value channels keeps n and m for itself, as a state line does. Workgroups of one head follow one
+// another by `heads`: with 8 heads an XCD's L2 serves a head's keys to all of its value channels.
+template <int KIND, int NT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void segment_walk_kernel(const float* __restrict__ proj, long ldp, int v_off,
+                                                           float* __restrict__ state, long state_ld,
+                                                           const int* __restrict__ cu_rows, const int* __restrict__ seq_slots,
+                                                           int seg_len, float* __restrict__ work, int H, int D, int V) {
+  constexpr int Dp = 64 * NT, SETS = 4;
+  const int h = blockIdx.x, vb = blockIdx.y, s = blockIdx.z, t = threadIdx.x, n_vb = gridDim.y;
+  const int first = cu_rows[s], n_rows = cu_rows[s + 1] - first;
+  if (n_rows <= 0) return;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, g = lane >> 4, n = lane & 15;
+  int before = 0;                                // the segments of the requests before
+  for (int s0 = 0; s0 < s; s0 += 64) {
+    int c = s0 + lane < s ? (cu_rows[s0 + lane + 1] - cu_rows[s0 + lane] + seg_len - 1) / seg_len : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) c += __shfl_xor(c, o, 64);
+    before += c;
+  }
+  const SegmentBlock at(D, V);
+  float* base = work + ((long)before * H + h) * at.floats;
+  const long stride = (long)H * at.floats;
+  const int n_seg = (n_rows + seg_len - 1) / seg_len;
+  const int col = vb * 16 + n;
+  const float* block = proj + v_off + h * V + vb * 16;
+  const int cols = min(16, V - vb * 16);
+  const ValueRows values(ldp, g, n);
+  float* st = state + (long)seq_slots[s] * state_ld;
+  float* S_line = st + (long)h * D * V;
+  float* nm = st + (long)H * D * V + ((long)h * n_vb + vb) * (D + 1);
+  f32x4 S[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d = (wave * NT + u) * 16 + g * 4 + r;
+      S[u][r] = d < D && col < V ? S_line[(long)d * V + col] : 0.f;
+    }
+  float n_mine = KIND == 1 && t < D ? nm[t] : 0.f, m = KIND == 1 ? nm[D] : 0.f;
+
+  if (KIND == 1) __syncthreads();                // m has been read before the first thread is through and writes it
+  struct Operands { f32x4 k[NT][4], v[4], a[NT]; float own, m, f; } sets[SETS];
+  auto rows_of = [&](int c) { return Segment{first + c * seg_len, min(seg_len, n_rows - c * seg_len)}; };
+  auto fetch = [&](Operands& o, int c) {
+    const float* p = base + c * stride;
+    const Segment seg = rows_of(c);
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)             // (of tiles that the segment does not have: memory that nobody uses)
+        o.k[u][rt] = *reinterpret_cast<const f32x4*>(p + at.k + (((wave * NT + u) * 4 + rt) * 64 + lane) * 4);
+    if (KIND == 0) {
+#pragma unroll
+      for (int u = 0; u < NT; ++u) o.a[u] = *reinterpret_cast<const f32x4*>(p + at.a + (wave * NT + u) * 16 + g * 4);
+    } else {
+      const int last = (seg.n + 15) / 16 * 16 - 1;
+      o.own = p[at.a + min(t, Dp - 1)];
+      o.m = p[at.x + last];
+      o.f = p[at.x + SP_ROWS + last];
+    }
+    values.fetch(o.v, block, cols, seg);
+  };
+  auto walk = [&](int c, Operands& o) {
+    float* p = base + c * stride;
+    const Segment seg = rows_of(c);
+    const int nc = (seg.n + 15) / 16;
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+      *reinterpret_cast<f32x4*>(p + at.s + (((long)vb * 4 * NT + wave * NT + u) * 64 + lane) * 4) = S[u];
+    if (KIND == 0) {
+#pragma unroll
+      for (int u = 0; u < NT; ++u) S[u] *= o.a[u];
+    } else {
+      if (vb == 0 && t < Dp) p[at.n + t] = n_mine;
+      if (vb == 0 && t == 0) p[at.x + 3 * SP_ROWS] = m;
+      const float m_next = fmaxf(o.f + m, o.m), keep = expf(o.f + m - m_next), take = expf(o.m - m_next);
+      m = m_next;
+      n_mine = keep * n_mine + take * o.own;
+#pragma unroll
+      for (int u = 0; u < NT; ++u) S[u] *= keep;
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) o.v[rt] *= take;
+    }
+    f32x4 own[NT][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int u = 0; u < NT; ++u)
+        own[u][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.k[u][0][r], o.v[0][r], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int rt = 1; rt < 4; ++rt)
+      if (rt < nc) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int u = 0; u < NT; ++u) own[u][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.k[u][rt][r], o.v[rt][r], own[u][r], 0, 0, 0);
+      }
+#pragma unroll
+    for (int u = 0; u < NT; ++u) S[u] += (own[u][0] + own[u][1]) + (own[u][2] + own[u][3]);
+  };
+#pragma unroll
+  for (int c = 0; c < SETS - 1; ++c) fetch(sets[c], min(c, n_seg - 1));
+  for (int c0 = 0; c0 < n_seg; c0 += SETS) {
+#pragma unroll
+    for (int e = 0; e < SETS; ++e) {
+      const int c = c0 + e;
+      if (c >= n_seg) break;
+      fetch(sets[(e + SETS - 1) % SETS], min(c + SETS - 1, n_seg - 1));
+      walk(c, sets[e]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d = (wave * NT + u) * 16 + g * 4 + r;
+      if (d < D && col < V) S_line[(long)d * V + col] = S[u][r];
+    }
+  if (KIND == 1 && t < D) nm[t] = n_mine;
+  if (KIND == 1 && t == 0) nm[D] = m;
+}
+
+// grid (heads, blocks of 64 value channels, segments), a wave 16 value channels of all the segment's rows: the operands that hang
+// on the value channels (S at the start, v) stay in registers, P and q go through LDS once for the four waves; everything is under
+// way at once.
+template <int KIND, int NT>
+__global__ __launch_bounds__(256) void segment_results_kernel(const float* __restrict__ proj, long ldp, int v_off,
+                                                              const int* __restrict__ cu_rows, int n_seqs, int seg_len,
+                                                              const float* __restrict__ work, float* __restrict__ out, long ldo,
+                                                              int H, int D, int V, int n_vb) {
+  __shared__ f32x4 q_lds[16 * NT][64], p_lds[10][64];
+  __shared__ float w_own[SP_ROWS], w_start[SP_ROWS], below[SP_ROWS];
+  const Segment seg = find_segment(cu_rows, n_seqs, seg_len, blockIdx.z);
+  if (seg.n <= 0) return;
+  const int h = blockIdx.x, t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, g = lane >> 4, n = lane & 15;
+  const int nc = (seg.n + 15) / 16, vb = blockIdx.y * 4 + wave, col = vb * 16 + n;
+  const SegmentBlock at(D, V);
+  const float* mine = work + ((long)blockIdx.z * H + h) * at.floats;
+  f32x4 S[4 * NT], v[4], q_in[4 * NT], p_in[3];   // (of tiles that the segment does not have: its last ones)
+#pragma unroll
+  for (int e = 0; e < 4 * NT; ++e)
+    q_in[e] = *reinterpret_cast<const f32x4*>(mine + at.q + (min(e * 4 + wave, nc * 4 * NT - 1) * 64 + lane) * 4);
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    const int tile = min(e * 4 + wave, nc * (nc + 1) / 2 - 1), J = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3;
+    p_in[e] = *reinterpret_cast<const f32x4*>(mine + ((J * 4 + tile - J * (J + 1) / 2) * 64 + lane) * 4);
+  }
+  const int vb_in = min(vb, n_vb - 1);
+#pragma unroll
+  for (int tt = 0; tt < 4 * NT; ++tt)
+    S[tt] = *reinterpret_cast<const f32x4*>(mine + at.s + (((long)vb_in * 4 * NT + tt) * 64 + lane) * 4);
+  const float* block = proj + v_off + h * V + vb_in * 16;
+  ValueRows(ldp, g, n).fetch(v, block, min(16, V - vb_in * 16), seg);
+#pragma unroll
+  for (int e = 0; e < 4 * NT; ++e) q_lds[e * 4 + wave][lane] = q_in[e];
+#pragma unroll
+  for (int e = 0; e < 3; ++e)
+    if (e * 4 + wave < 10) p_lds[e * 4 + wave][lane] = p_in[e];
+  __syncthreads();
+  if (KIND == 1) {
+    if (wave < nc) {
+      float a = 0.f;                             // q . n at the start, of row n of the wave's tile
+#pragma unroll
+      for (int tt = 0; tt < 4 * NT; ++tt) {
+        const f32x4 x = q_lds[wave * 4 * NT + tt][lane] *
+                        *reinterpret_cast<const f32x4*>(mine + at.n + tt * 16 + g * 4);
+        a += (x[0] + x[1]) + (x[2] + x[3]);
+      }
+      a += __shfl_xor(a, 16, 64);
+      a += __shfl_xor(a, 32, 64);
+      if (g == 0) {
+        const int row = wave * 16 + n;
+        const float m_own = mine[at.x + row], from = mine[at.x + SP_ROWS + row] + mine[at.x + 3 * SP_ROWS];
+        const float m = fmaxf(m_own, from), own = expf(m_own - m), start = expf(from - m);
+        w_own[row] = own;
+        w_start[row] = start;
+        below[row] = fmaxf(fabsf(own * mine[at.x + 2 * SP_ROWS + row] + start * a), expf(-m)) + 1e-6f;
+      }
+    }
+    __syncthreads();
+  }
+  if (vb >= n_vb) return;
+  // P is triangular, but a product takes its zeros times every row: a row that is not finite must not reach the rows before it, so such
+  // a segment goes without the matrix product.
+  float none = 0.f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) none = fmaf(v[c][r], 0.f, none);
+  const bool finite = __all(col >= V || none == 0.f);
+  auto to = __builtin_amdgcn_make_buffer_rsrc(out + (long)seg.first * ldo + h * V + vb * 16, 0,
+                                              ((seg.n - 1) * (int)ldo + min(16, V - vb * 16)) * 4, 0x00020000);
+  auto rows = [&](auto count, int j0) {          // the tiles of rows j0 .. j0 + count - 1
+    constexpr int N = decltype(count)::value;
+    f32x4 part[N][4], acc[N];
+    auto clear = [&] {
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[j][r] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    };
+    clear();
+    if (finite) {
+#pragma unroll
+      for (int I = 0; I < 4; ++I)
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          if (I <= j0 + j) {
+            const f32x4 p = p_lds[(j0 + j) * (j0 + j + 1) / 2 + I][lane];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[j][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[r], v[I][r], part[j][r], 0, 0, 0);
+          }
+    } else {
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+#pragma unroll 1
+        for (int i = 0; i < min((j0 + j) * 16 + 16, seg.n); ++i) {
+          const float vi = col < V ? block[(long)(seg.first + i) * ldp + n] : 0.f;
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (i <= (j0 + j) * 16 + g * 4 + r)
+              part[j][0][r] += mine[(((j0 + j) * 4 + i / 16) * 64 + i % 16 / 4 * 16 + g * 4 + r) * 4 + i % 4] * vi;
+        }
+    }
+    float start[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      acc[j] = (part[j][0] + part[j][1]) + (part[j][2] + part[j][3]);
+      start[j] = 1.f;
+      if (KIND == 1) {
+        start[j] = w_start[(j0 + j) * 16 + n];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[j][r] *= w_own[(j0 + j) * 16 + g * 4 + r];
+      }
+    }
+    clear();
+#pragma unroll
+    for (int tt = 0; tt < 4 * NT; ++tt) {
+      f32x4 q[N];
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        q[j] = q_lds[(j0 + j) * 4 * NT + tt][lane];
+        if (KIND == 1) q[j] *= start[j];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < N; ++j) part[j][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[j][r], S[tt][r], part[j][r], 0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) acc[j] += (part[j][0] + part[j][1]) + (part[j][2] + part[j][3]);
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {              // (rows past the last lie behind the buffer's end)
+        const int row = (j0 + j) * 16 + g * 4 + r;
+        const float o = KIND == 1 ? acc[j][r] / below[row] : acc[j][r];
+        if (col < V) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, o), to, row * (int)ldo * 4 + n * 4, 0, 0);
+      }
+  };
+  if (nc == 4) rows(std::integral_constant<int, 4>{}, 0);
+  else
+    for (int j = 0; j < nc; ++j) rows(std::integral_constant<int, 1>{}, j);
+}
+
+template <int KIND, int NT>
+static int launch_products(const float* proj, long ldp, int q_off, int k_off, int v_off, float q_scale, const float* decay, long ldd,
+                           int i_off, int f_off, const float* bias_i, const float* bias_f, float cap, float* state, long state_ld,
+                           const int* cu_rows, const int* seq_slots, int n_seqs, float* out, long ldo, int H, int D, int V,
+                           int seg_len, int rows, float* work, ScanLayout lay, hipStream_t stream) {
+  const unsigned most = (unsigned)sp_most(rows, seg_len, n_seqs);
+  const int n_vb = (V + 15) / 16;
+  segment_rows_kernel<KIND, NT><<<dim3(H, most), 512, 0, stream>>>(proj, ldp, q_off, k_off, q_scale, decay, ldd, i_off, f_off, bias_i,
+                                                                   bias_f, cap, cu_rows, n_seqs, seg_len, work, H, D, V, lay);
+  if (tis_launch_status("segment_rows")) return -1;
+  segment_walk_kernel<KIND, NT><<<dim3(H, n_vb, n_seqs), 256, 0, stream>>>(proj, ldp, v_off, state, state_ld, cu_rows, seq_slots,
+                                                                          seg_len, work, H, D, V);
+  if (tis_launch_status("segment_walk")) return -1;
+  segment_results_kernel<KIND, NT><<<dim3(H, (n_vb + 3) / 4, most), 256, 0, stream>>>(proj, ldp, v_off, cu_rows, n_seqs, seg_len, work,
+                                                                                      out, ldo, H, D, V, n_vb);
+  return tis_launch_status("segment_results");
+}
 
 template <int KIND>
-static int launch_scan(bool wide, int ns, dim3 grid, size_t lds, hipStream_t stream, const float* proj, long ldp, int q_off, int k_off,
+static int launch_scan(int ns, dim3 grid, size_t lds, hipStream_t stream, const float* proj, long ldp, int q_off, int k_off,
                        int v_off, float q_scale, const float* decay, long ldd, int i_off, int f_off, const float* bias_i,
                        const float* bias_f, float cap, float* state, long state_ld, const int* cu_rows,
                        const int* seq_slots, float* out, long ldo, int H, int D, int V, int n_vb, int chunk, SegArgs sg,
                        ScanLayout lay) {
 #define SC_LAUNCH(NS)                                                                                                   \
   if (sg.segments)                                                                                                      \
-    state_scan_kernel<KIND, NS, true, SC_VB><<<grid, SC_THREADS, lds, stream>>>(                                        \
+    state_scan_kernel<KIND, NS, true><<<grid, SC_THREADS, lds, stream>>>(                                        \
         proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off, bias_i, bias_f, cap, state, state_ld,        \
         cu_rows, seq_slots, out, ldo, H, D, V, n_vb, chunk, sg, lay);                                                   \
   else                                                                                                                  \
-    state_scan_kernel<KIND, NS, false, SC_VB><<<grid, SC_THREADS, lds, stream>>>(                                       \
+    state_scan_kernel<KIND, NS, false><<<grid, SC_THREADS, lds, stream>>>(                                       \
         proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off, bias_i, bias_f, cap, state, state_ld,        \
         cu_rows, seq_slots, out, ldo, H, D, V, n_vb, chunk, sg, lay)
-#define SC_LAUNCH_WIDE(NS)                                                                                              \
-  state_scan_kernel<KIND, NS, true, SC_WIDE_VB><<<grid, SC_THREADS, lds, stream>>>(                                     \
-      proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off, bias_i, bias_f, cap, state, state_ld, cu_rows, \
-      seq_slots, out, ldo, H, D, V, n_vb, chunk, sg, lay)
-  if (wide) {
-    if (ns <= 8) { SC_LAUNCH_WIDE(8); }
-    else if (ns <= 16) { SC_LAUNCH_WIDE(16); }
-    else { SC_LAUNCH_WIDE(32); }
-  } else
   if (ns <= 1) { SC_LAUNCH(1); }
   else if (ns <= 2) { SC_LAUNCH(2); }
   else if (ns <= 4) { SC_LAUNCH(4); }
   else if (ns <= 8) { SC_LAUNCH(8); }
   else { SC_LAUNCH(16); }
-#undef SC_LAUNCH_WIDE
 #undef SC_LAUNCH
   if (tis_launch_status("state_scan")) return -1;
   if (!sg.segments) return 0;
@@ -398,8 +978,15 @@ TIS_EXPORT int tis_state_scan_segmentable(int D) {
   return sizeof(float) * ((size_t)D * SG_COLS + (size_t)SG_ROWS * (D + 1) + SG_ROWS) <= 64 * 1024;
 }
 
-// 32-bit floats of the workspace a segmented call needs: the states, then `rows` lines of decay products or gate sums.
-TIS_EXPORT long tis_state_scan_workspace(int kind, int n_seqs, int segments, int rows, int H, int D, int V) {
+// Whether a segmented call goes through the kernels of matrix products.
+static bool by_products(int n_seqs, int seg_len, int D, long rows) {
+  return D <= 128 && seg_len <= SP_ROWS && n_seqs <= 65535 && sp_most(rows, seg_len, n_seqs) <= 65535;
+}
+
+// 32-bit floats of the workspace a segmented call needs: a block for every segment and head; or, off the matrix products, the
+// states, then `rows` lines of decay products or gate sums.
+TIS_EXPORT long tis_state_scan_workspace(int kind, int n_seqs, int segments, int seg_len, int rows, int H, int D, int V) {
+  if (by_products(n_seqs, seg_len, D, rows)) return sp_most(rows, seg_len, n_seqs) * H * SegmentBlock(D, V).floats;
   return (long)n_seqs * segments * H * ((long)D * V + D + 2) + (kind == 0 ? (long)rows * H * D : (long)rows * H * 3);
 }
 
@@ -428,17 +1015,12 @@ TIS_EXPORT int tis_state_scan(int kind, const float* proj, long ldp, int q_off, 
   if (n_vb > 65535) return tis_fail("state_scan: %d value channels exceed the grid", V);
   if (state_ld < tis_state_scan_floats(kind, H, D, V))
     return tis_fail("state_scan: a state line of %ld floats is too short for %ld", state_ld, tis_state_scan_floats(kind, H, D, V));
-  // segments of heads with up to 128 key channels and whole blocks of 64 value channels: 64 channels a workgroup
-  const bool wide = segments > 0 && V % SC_WIDE_VB == 0 && D <= 32 * (SC_THREADS / SC_WIDE_VB);
-  const int vb_cols = wide ? SC_WIDE_VB : SC_VB, col_threads = SC_THREADS / vb_cols;
   int chunk = 16;
-  const int ns_need = (D + col_threads - 1) / col_threads;
-  const int ns_built = wide ? (ns_need <= 8 ? 8 : ns_need <= 16 ? 16 : 32) : (D + SC_R - 1) / SC_R <= 1 ? 1 : (D + SC_R - 1) / SC_R <= 2 ? 2 : (D + SC_R - 1) / SC_R <= 4 ? 4
-                       : (D + SC_R - 1) / SC_R <= 8 ? 8 : 16;
-  const size_t dp = (size_t)col_threads * ns_built;      // a token's row in LDS (see the kernel)
+  const int ns = (D + SC_R - 1) / SC_R, ns_built = ns <= 1 ? 1 : ns <= 2 ? 2 : ns <= 4 ? 4 : ns <= 8 ? 8 : 16;
+  const size_t dp = (size_t)SC_R * ns_built;      // a token's row in LDS (see the kernel)
   auto bytes = [&](int c) {
-    return sizeof(float) * ((size_t)c * dp * 2 + (kind == 0 ? (size_t)c * dp : (size_t)c * 4) + (size_t)c * vb_cols +
-                            (size_t)c * col_threads * (vb_cols + 1));
+    return sizeof(float) * ((size_t)c * dp * 2 + (kind == 0 ? (size_t)c * dp : (size_t)c * 4) + (size_t)c * SC_VB +
+                            (size_t)c * SC_R * (SC_VB + 1));
   };
   while (chunk > 1 && bytes(chunk) > SC_LDS_BYTES) chunk /= 2;
   if (bytes(chunk) > SC_LDS_BYTES) return tis_fail("state_scan: %d key channels do not fit the chunk buffers", D);
@@ -446,6 +1028,17 @@ TIS_EXPORT int tis_state_scan(int kind, const float* proj, long ldp, int q_off, 
   if (segments > 0) {
     if (seg_len < 1 || rows < 1 || !workspace || (long)n_seqs * segments > 0x7fffffffL)
       return tis_fail("state_scan: %d segments of %d rows need a workspace", segments, seg_len);
+    if (by_products(n_seqs, seg_len, D, rows)) {
+      if ((uintptr_t)workspace % 16) return tis_fail("state_scan: the workspace is not 16 bytes aligned");
+#define SP_LAUNCH(KIND, NT)                                                                                                       \
+  return launch_products<KIND, NT>(proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off, bias_i, bias_f, cap, state, \
+                                   state_ld, cu_rows, seq_slots, n_seqs, out, ldo, H, D, V, seg_len, rows, workspace, lay, stream)
+      if (kind == 0 && D <= 64) SP_LAUNCH(0, 1);
+      if (kind == 0) SP_LAUNCH(0, 2);
+      if (D <= 64) SP_LAUNCH(1, 1);
+      SP_LAUNCH(1, 2);
+#undef SP_LAUNCH
+    }
     sg.segments = segments;
     sg.seg_len = seg_len;
     sg.seg_state = workspace;
@@ -455,11 +1048,10 @@ TIS_EXPORT int tis_state_scan(int kind, const float* proj, long ldp, int q_off, 
     if (sizeof(float) * ((size_t)D * SG_COLS + (size_t)SG_ROWS * (D + 1) + SG_ROWS) > 64 * 1024)
       return tis_fail("state_scan: %d key channels do not fit the segment kernels (see tis_state_scan_segmentable)", D);
   }
-  dim3 grid(segments > 0 ? n_seqs * segments : n_seqs, H, (V + vb_cols - 1) / vb_cols);
-  const int ns = ns_need;
+  dim3 grid(segments > 0 ? n_seqs * segments : n_seqs, H, n_vb);
   if (kind == 0)
-    return launch_scan<0>(wide, ns, grid, bytes(chunk), stream, proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off,
+    return launch_scan<0>(ns, grid, bytes(chunk), stream, proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off,
                           bias_i, bias_f, cap, state, state_ld, cu_rows, seq_slots, out, ldo, H, D, V, n_vb, chunk, sg, lay);
-  return launch_scan<1>(wide, ns, grid, bytes(chunk), stream, proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off,
+  return launch_scan<1>(ns, grid, bytes(chunk), stream, proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off,
                         bias_i, bias_f, cap, state, state_ld, cu_rows, seq_slots, out, ldo, H, D, V, n_vb, chunk, sg, lay);
 }

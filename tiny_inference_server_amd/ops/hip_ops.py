@@ -2220,8 +2220,9 @@ class HipOps:
         of them). decay_per_head: `decay` holds one number per head and row instead of one per key channel.
 
         A step whose longest portion has at least two segments' rows (self.scan_segment, 64) is run in segments side
-        by side, with a second pass for the states at the segments' starts and a third for what they add to the
-        rows' outputs; shorter portions and single tokens are walked in order by one kernel."""
+        by side, with a pass for the states at the segments' starts and one for what they add to the rows' outputs (as
+        products of matrices for up to 128 key channels); shorter portions and single tokens are walked in order by one
+        kernel."""
         n = proj.shape[0]
         if qk_group < 1 or n_heads % qk_group:
             raise KernelError(f"state_scan: {n_heads} heads in groups of {qk_group}")
@@ -2251,8 +2252,8 @@ class HipOps:
         if seg_len > 0 and batch.max_seq_rows >= 2 * seg_len and lib.cdll.tis_state_scan_segmentable(dim):
             segments = -(-batch.max_seq_rows // seg_len)
             lib.cdll.tis_state_scan_workspace.restype = c_long
-            floats = lib.cdll.tis_state_scan_workspace(0 if kind == "decay" else 1, batch.n_seqs, segments, n, n_heads,
-                                                       dim, vdim)
+            floats = lib.cdll.tis_state_scan_workspace(0 if kind == "decay" else 1, batch.n_seqs, segments, seg_len, n,
+                                                       n_heads, dim, vdim)
             workspace = torch.empty(floats, dtype=torch.float32, device=self.device)
         lib.tis_state_scan(
             0 if kind == "decay" else 1, _ptr(proj), proj.stride(0), q_off, k_off, v_off, float(q_scale), _ptr(decay),
