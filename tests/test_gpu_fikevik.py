@@ -210,6 +210,29 @@ def test_state_scan_in_segments_by_matrix_products(kind, Hh, D, V, per_head, len
     assert torch.isnan(again[at:last]).all()
 
 
+# Heads of more than 128 key channels take the row by row kernels for segments. Every workgroup of the pass over the states reads a
+# request's running maximum, so nothing may write the new one before they all have: single-row requests beside a long one, whose
+# pass is the shortest. (The bound is the one above.)
+def test_the_running_maximum_after_segments_row_by_row():
+    ops, ref = hip_ops("float32"), TorchOps("cpu", torch.float32)
+    Hh, D, V = 2, 144, 48
+    g = torch.Generator().manual_seed(9)
+    lens = [130] + [1] * 12
+    n, nc = sum(lens), 2 * Hh * D + Hh * V
+    proj = torch.randn(n, nc + 2 * Hh, generator=g)
+    bi, bf = torch.randn(Hh, generator=g), 2 + torch.randn(Hh, generator=g)
+    rows = [(0, 0, 130)] + [(130 + i, 5, 1) for i in range(12)]
+    states, res = [], []
+    for o, dev in ((ops, "cuda"), (ref, "cpu")):
+        st = torch.zeros(len(lens), ops.state_scan_floats("gated_max", Hh, D, V), device=dev)
+        res.append(o.state_scan("gated_max", proj.to(dev), 0, Hh * D, 2 * Hh * D, D ** -0.5, st,
+                                fake_batch(rows, list(range(len(lens))), None, 1, dev), Hh, D, V, i_off=nc, f_off=nc + Hh,
+                                bias_i=bi.to(dev), bias_f=bf.to(dev), cap=9.0))
+        states.append(st)
+    close(res[0], res[1], "float32", "results")
+    close(states[0], states[1], "float32", "states")
+
+
 # ---- the engine ------------------------------------------------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(SC_THREADS) void state_scan_kernel(
 
 // Kernel 2 of a segmented call: one thread per element of a head's S (and of n), segment after segment in order. What
 // the first kernel left as a segment's own state is replaced by the state at the segment's start; the request's state
-// line receives the state after its last row.
+// line receives the state after its last row, but for kind 1's m, which every workgroup here reads: kernel 3 writes it.
 template <int KIND>
 __global__ __launch_bounds__(SC_THREADS) void segment_states_kernel(float* __restrict__ state, long state_ld,
                                                                     const int* __restrict__ cu_rows,
@@ -274,8 +274,6 @@ __global__ __launch_bounds__(SC_THREADS) void segment_states_kernel(float* __res
   } else {
     st[(long)h * D * V + el] = x;
   }
-  if (KIND == 1 && el == 0)
-    for (int b = 0; b < n_vb; ++b) st[(long)H * D * V + ((long)h * n_vb + b) * (D + 1) + D] = m;
 }
 
 // Kernel 3 of a segmented call: what the state at a segment's start adds to its rows. One workgroup per (request and
@@ -284,9 +282,11 @@ static constexpr int SG_COLS = 64, SG_ROWS = 32;
 
 template <int KIND>
 __global__ __launch_bounds__(SC_THREADS) void segment_outputs_kernel(const float* __restrict__ proj, long ldp, int q_off,
-                                                                     float q_scale, const int* __restrict__ cu_rows,
+                                                                     float q_scale, float* __restrict__ state, long state_ld,
+                                                                     const int* __restrict__ cu_rows,
+                                                                     const int* __restrict__ seq_slots,
                                                                      float* __restrict__ out, long ldo, int H, int D,
-                                                                     int V, SegArgs sg, ScanLayout lay) {
+                                                                     int V, int n_vb, SegArgs sg, ScanLayout lay) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   float* s0 = lds;                       // [D][SG_COLS]
   float* qt = s0 + D * SG_COLS;          // [SG_ROWS][D + 1]
@@ -302,6 +302,11 @@ __global__ __launch_bounds__(SC_THREADS) void segment_outputs_kernel(const float
     s0[idx] = c0 + cc < V ? start[(long)i * V + c0 + cc] : 0.f;
   }
   const float m0 = KIND == 1 ? start[per - 1] : 0.f;
+  if (KIND == 1 && blockIdx.z == 0 && t < n_vb && r1 == cu_rows[seq + 1]) {      // after the request's last row
+    const float m = fmaxf(sg.aux[((long)(r1 - 1) * H + h) * 3 + 1] + m0, start[per - 2]);
+    for (int b = t; b < n_vb; b += SC_THREADS)
+      state[(long)seq_slots[seq] * state_ld + (long)H * D * V + ((long)h * n_vb + b) * (D + 1) + D] = m;
+  }
   for (int t0 = r0; t0 < r1; t0 += SG_ROWS) {
     const int nr = min(SG_ROWS, r1 - t0);
     __syncthreads();
@@ -969,7 +974,7 @@ static int launch_scan(int ns, dim3 grid, size_t lds, hipStream_t stream, const 
   if (tis_launch_status("segment_states")) return -1;
   const size_t lds3 = sizeof(float) * ((size_t)D * SG_COLS + (size_t)SG_ROWS * (D + 1) + SG_ROWS);
   segment_outputs_kernel<KIND><<<dim3(grid.x, H, (V + SG_COLS - 1) / SG_COLS), SC_THREADS, lds3, stream>>>(
-      proj, ldp, q_off, q_scale, cu_rows, out, ldo, H, D, V, sg, lay);
+      proj, ldp, q_off, q_scale, state, state_ld, cu_rows, seq_slots, out, ldo, H, D, V, n_vb, sg, lay);
   return tis_launch_status("segment_outputs");
 }
 
