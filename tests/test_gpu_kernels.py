@@ -254,6 +254,27 @@ def test_decoded_rows_of_uneven_lengths_beside_a_portions_tiles(ops_for, monkeyp
         torch.testing.assert_close(got[r].view(n_heads, hd).double(), want, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("cut", [2, 3, 4, 5, 7])
+def test_many_rows_merged_from_few_and_more_key_splits(ops_for, monkeypatch, cut):
+    """A portion whose tiles are cut into `cut` key splits: rows of up to four are merged with all loads at once, rows of more
+    split after split; rows whose own keys need fewer splits stand beside them. (Bounds as for the test above.)"""
+    from tiny_inference_server_amd.ops import hip_ops
+    n_heads, n_kv, hd, page_size, p0, n = 12, 3, 128, 16, 40, 700          # 8,400 (row, head) pairs: the merge of many rows
+    monkeypatch.setattr(hip_ops, "_tiles_cut_pays", lambda *a: True)
+    monkeypatch.setattr(hip_ops, "_tiles_cut", lambda n, n_tiles, tile_steps, *a: (cut, -(-tile_steps[1] // cut)))
+    ops = ops_for(torch.bfloat16)
+    plane, tables, ks, vs = make_paged([p0 + n], n_kv, hd, page_size, torch.bfloat16, seed=31)
+    positions = torch.arange(p0, p0 + n, dtype=torch.int32)
+    q = rnd((n, n_heads * hd), torch.bfloat16, 32)
+    batch = SimpleNamespace(positions=positions.cuda(), row_seq=torch.zeros(n, dtype=torch.int32).cuda(),
+                            block_tables={"g": tables.cuda()}, max_kv_len=p0 + n, extras={}, n_rows=n, max_seq_rows=n,
+                            seq_rows=[(0, p0, n)])
+    got = ops.paged_attention(q.cuda(), plane.cuda(), batch, "g", n_heads, n_kv, hd).cpu()
+    for r in list(range(0, n, 23)) + [n - 1]:
+        want = dense_reference(q[r].view(n_heads, hd), ks[0], vs[0], n_heads // n_kv, p0 + r)
+        torch.testing.assert_close(got[r].view(n_heads, hd).double(), want, rtol=2e-2, atol=2e-2)
+
+
 @pytest.mark.parametrize("page_size", [16, 32])
 def test_single_rows_walking_a_long_context_without_splits(ops_for, monkeypatch, page_size):
     """With no key splits one wave walks a request's whole context alone: thousands of keys, hundreds of steps,
@@ -563,6 +584,26 @@ def test_rope_and_cache_write_of_pair_ordered_rows(ops_for, n_heads, n_kv, hd, p
         torch.testing.assert_close(pa.cpu().float(), pb.float(), **tol(dtype))
         if not write_cache:
             assert torch.equal(pa.cpu(), plane0)
+
+
+def test_rope_and_cache_write_of_thousands_of_rows(ops_for):
+    """From 4,096 rows on a workgroup takes several heads, queries, keys and values: against the same rows in two calls of fewer,
+    which take a head each. The arithmetic is the same, so are the results, bit for bit."""
+    ops = ops_for(torch.bfloat16)
+    n, n_heads, n_kv, hd, page_size = 4101, 9, 2, 64, 16
+    qkv = rnd((n, (n_heads + 2 * n_kv) * hd), torch.bfloat16, 57).cuda()
+    table = rnd((n, hd // 2, 2), torch.float32, 58).cuda()
+    at = torch.arange(n, dtype=torch.int32).cuda()
+    res = []
+    for parts in ((0, n), (0, 2050, n)):
+        plane = torch.zeros(n // page_size + 1, 2, n_kv, page_size, hd, dtype=torch.bfloat16).cuda()
+        q = torch.zeros(n, n_heads * hd, dtype=torch.bfloat16).cuda()
+        for a, b in zip(parts, parts[1:]):
+            ops.rope_write_kv(qkv[a:b].clone(), at[a:b].contiguous(), at[a:b].contiguous(), table, plane, n_heads, n_kv, hd, page_size,
+                              False, write_cache=True, paired=True, q_out=q[a:b])
+        res.append((q, plane))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+    assert res[0][0].abs().sum() > 0 and res[0][1].abs().sum() > 0
 
 
 def assert_same_draws(ref, got, logits, temperature, top_k, top_p, pen, u, ctx_t, off, note=None):

@@ -896,7 +896,9 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_kernel(const float* _
 // The same merge for many rows (prompt portions): a workgroup takes four heads of a row, one a wave, and a row that
 // was not split costs one load. With a workgroup per (row, head) the thousands of rows of a prompt would mean tens of
 // thousands of workgroups; with a wave taking several heads in turn, each head's two round trips to memory follow
-// the previous head's.
+// the previous head's. Up to four splits are asked for all at once, before their weights are known: split after split, each one's
+// load waited for the one before (2,048 rows of 12 heads of 128, up to three splits: 11.3 us; 6.8 so).
+static constexpr int FEW_SPLITS = 4;
 __global__ __launch_bounds__(MG * 64) void attention_merge_rows_kernel(const float* __restrict__ part_o,
                                                                        const float2* __restrict__ part_ml,
                                                                        bf16* __restrict__ out, long out_ld,
@@ -905,7 +907,7 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_rows_kernel(const flo
   const long row = blockIdx.x;
   const int n_splits = row_splits ? row_splits[row] : max_splits;
   if (n_splits <= 1) return;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int head = blockIdx.y * MG + wave;
   if (head >= n_heads) return;
   const long base = (row * n_heads + head) * max_splits;
@@ -913,31 +915,53 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_rows_kernel(const flo
 #pragma unroll
   for (int j = 0; j < MD; ++j) acc[j] = 0.f;
   float M = -INFINITY, L = 0.f;
-  for (int s0 = 0; s0 < n_splits; s0 += 64)
-    if (s0 + lane < n_splits) M = fmaxf(M, part_ml[base + s0 + lane].x);
+  if (n_splits <= FEW_SPLITS) {                  // everything under way at once (past the last split: the last one's again)
+    float2 ml[FEW_SPLITS];
+    float o[FEW_SPLITS][MD], w[FEW_SPLITS];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-  for (int s0 = 0; s0 < n_splits; s0 += 64) {
-    float w = 0.f;
-    if (s0 + lane < n_splits) {
-      const float2 ml = part_ml[base + s0 + lane];
-      if (ml.x != -INFINITY) {
-        w = exp2f(ml.x - M);
-        L += w * ml.y;
+    for (int i = 0; i < FEW_SPLITS; ++i) {
+      const long at = base + min(i, n_splits - 1);
+      ml[i] = part_ml[at];
+#pragma unroll
+      for (int j = 0; j < MD; ++j) o[i][j] = part_o[at * VD + min(j * 64 + lane, VD - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < FEW_SPLITS; ++i) M = fmaxf(M, ml[i].x);
+#pragma unroll
+    for (int i = 0; i < FEW_SPLITS; ++i) {
+      w[i] = i < n_splits && ml[i].x != -INFINITY ? exp2f(ml[i].x - M) : 0.f;
+#pragma unroll
+      for (int j = 0; j < MD; ++j) acc[j] = w[i] != 0.f ? acc[j] + w[i] * o[i][j] : acc[j];
+      ml[i].y = w[i] != 0.f ? w[i] * ml[i].y : 0.f;
+    }
+    L = (ml[0].y + ml[2].y) + (ml[1].y + ml[3].y);
+  } else {
+    for (int s0 = 0; s0 < n_splits; s0 += 64)
+      if (s0 + lane < n_splits) M = fmaxf(M, part_ml[base + s0 + lane].x);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    for (int s0 = 0; s0 < n_splits; s0 += 64) {
+      float w = 0.f;
+      if (s0 + lane < n_splits) {
+        const float2 ml = part_ml[base + s0 + lane];
+        if (ml.x != -INFINITY) {
+          w = exp2f(ml.x - M);
+          L += w * ml.y;
+        }
+      }
+      const int cnt = min(64, n_splits - s0);
+      for (int i = 0; i < cnt; ++i) {
+        const float wi = __shfl(w, i, 64);
+#pragma unroll
+        for (int j = 0; j < MD; ++j) {
+          const int d = j * 64 + lane;
+          if (d < VD && wi != 0.f) acc[j] += wi * part_o[(base + s0 + i) * VD + d];
+        }
       }
     }
-    const int cnt = min(64, n_splits - s0);
-    for (int i = 0; i < cnt; ++i) {
-      const float wi = __shfl(w, i, 64);
 #pragma unroll
-      for (int j = 0; j < MD; ++j) {
-        const int d = j * 64 + lane;
-        if (d < VD && wi != 0.f) acc[j] += wi * part_o[(base + s0 + i) * VD + d];
-      }
-    }
+    for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off, 64);
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off, 64);
   if (sink) L += sink_share(sinks, head, M);
 #pragma unroll
   for (int j = 0; j < MD; ++j) {

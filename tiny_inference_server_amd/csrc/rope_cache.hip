@@ -99,8 +99,9 @@ __global__ __launch_bounds__(RC_THREADS) void rope_write_kv_rows_kernel(
   const int n_rows = (int)min((long)RB, rows - r0);
   const int half = head_dim / 2, pieces = head_dim / 8;     // a piece: four pairs, 16 bytes
   const int rotated = n_heads + (write_cache ? n_kv_heads : 0);
-  // queries and keys of this workgroup's share of the heads: piece after piece over (head, row, piece)
-  for (int hh = blockIdx.y; hh < rotated; hh += gridDim.y) {
+  // this workgroup's share of the heads, the values' last
+  int hh = blockIdx.y;
+  for (; hh < rotated; hh += gridDim.y) {        // queries and keys: piece after piece over (row, piece)
     for (int i = threadIdx.x; i < n_rows * pieces; i += RC_THREADS) {
       const int row = i / pieces, piece = i % pieces;
       const long r = r0 + row;
@@ -127,15 +128,14 @@ __global__ __launch_bounds__(RC_THREADS) void rope_write_kv_rows_kernel(
       *reinterpret_cast<rc_bf16x4*>(dst + half + piece * 4) = y2;
     }
   }
-  if (!write_cache) return;
-  // values
+  if (!write_cache || hh >= rotated + n_kv_heads) return;
   const int row_t = threadIdx.x % RB, d_t = threadIdx.x / RB;          // on the way out: rows side by side
   long v_dst = 0;
   if (row_t < n_rows) {
     const int slot = write_slots[r0 + row_t];
     v_dst = ((long)(slot / page_size) * 2 + 1) * n_kv_heads * page_size * head_dim + slot % page_size;
   }
-  for (int kvh = blockIdx.y; kvh < n_kv_heads; kvh += gridDim.y) {
+  for (int kvh = hh - rotated; kvh < n_kv_heads; kvh += gridDim.y) {
     __syncthreads();                                                     // the tile's last readers are done
     for (int i = threadIdx.x; i < n_rows * pieces; i += RC_THREADS) {
       const int row = i / pieces, piece = i % pieces;
@@ -162,7 +162,11 @@ TIS_EXPORT int tis_rope_write_kv(int dtype, void* qkv, long ld, const int* posit
   if (dtype == TIS_BF16 && paired && !interleaved && table && rows >= 4 * RB && head_dim % 8 == 0 && head_dim <= 256 &&
       ld % 8 == 0 && q_out_ld % 4 == 0 && ((uintptr_t)qkv % 16) == 0 && ((uintptr_t)q_out % 8) == 0 &&
       (!write_cache || (uintptr_t)plane % 8 == 0)) {
-    dim3 grid((rows + RB - 1) / RB, std::min(total_heads, 4));
+    // a head a workgroup, so that a chain is one position, its factors and one result; thousands of rows fill the chip with eight. us,
+    // four workgroups of several heads (before) / eight / one each, 18 heads of 128: 64 rows 4.2 / 3.3 / 2.5, 512 4.5 / 3.6 / 2.9,
+    // 2,048 5.7 / 4.9 / 4.9, 4,096 8.3 / 7.6 / 7.8, 8,000 13.7 / 13.5 / 13.9
+    const int shares = write_cache ? total_heads : n_heads;
+    dim3 grid((rows + RB - 1) / RB, std::min(shares, rows < 4096 ? 65535 : 8));
     rope_write_kv_rows_kernel<<<grid, RC_THREADS, 0, stream>>>((const bf16*)qkv, ld, positions, write_slots,
                                                               (const float2*)table, (bf16*)plane, rows, n_heads,
                                                               n_kv_heads, head_dim, page_size, write_cache,
