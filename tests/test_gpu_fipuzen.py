@@ -86,6 +86,18 @@ def test_sums_and_norms_in_fours(dtype, n, D, shift):
     want = ref.gated_postnorm(x, [(wide[:, cols], 1.3), (extra, 0.7)], wide[:, cols], bias, 1.9, gain, 1e-5)
     close(got[0], want[0], "float32", "gated_postnorm 32-bit")
     close(got[1], want[1], dtype, "gated_postnorm")
+    for two in (False, True):
+        res = [o.normed_mean([(wide.to(dev)[:, cols], gain.to(dev)), (x.to(dev), ygain.to(dev))][:1 + two], 1e-5)
+               for o, dev in ((ops, "cuda"), (ref, "cpu"))]
+        close(res[0], res[1], "float32", "normed_mean")
+    for heads in (1, 4):
+        if D // heads > 1028:
+            continue
+        V = D // heads
+        res = [o.head_norm_gate(x.to(dev), wide.to(dev)[:, cols], gn.to(dev), heads, V, 1e-5, "silu")
+               for gn in (gain[:V], gain) for o, dev in ((ops, "cuda"), (ref, "cpu"))]
+        close(res[0], res[1], dtype, "head_norm_gate")
+        close(res[2], res[3], dtype, "head_norm_gate, a gain a head")
 
 
 @pytest.mark.parametrize("D", [44, 300, 1500, 4200])      # (a row in 4 or 16 registers a thread, or in memory)

@@ -180,6 +180,40 @@ __global__ __launch_bounds__(TIS_WAVE) void head_norm_gate_kernel(const float* _
   }
 }
 
+// The same for channels that are a multiple of four, PER pieces of four a lane (V <= 256 PER): everything a head needs is asked for
+// at once, where single values went to memory twice, one after the other. us, single values /
+// fours: 8 rows of 8 heads of 256 2.9 / 2.3, 1,531 rows 8.5 / 6.1, 2,048 rows of 16 heads of 128 12.5 / 11.3.
+template <typename T, int PER>
+__global__ __launch_bounds__(TIS_WAVE) void head_norm_gate_fours_kernel(const float* __restrict__ o, long ldo,
+                                                                         const float* __restrict__ g, long ldg,
+                                                                         const float* __restrict__ gain, int gain_per_head,
+                                                                         int act, float eps, T* __restrict__ out, long ldout,
+                                                                         int V) {
+  const long r = blockIdx.x;
+  const int h = blockIdx.y;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 x[PER], z[PER], gn[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = (threadIdx.x + k * TIS_WAVE) * 4;
+    const bool in = c < V;
+    x[k] = in ? load4(o + r * ldo + (long)h * V + c) : zero;
+    z[k] = in ? load4(g + r * ldg + (long)h * V + c) : zero;
+    gn[k] = in ? load4(gain + (gain_per_head ? h * V : 0) + c) : zero;
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) ss += square4(x[k]);
+  const float inv = 1.f / sqrtf(wave_sum(ss) / (float)V + eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = (threadIdx.x + k * TIS_WAVE) * 4;
+    if (c >= V) continue;
+    const float4 q = make_float4(sigmoid_f(z[k].x), sigmoid_f(z[k].y), sigmoid_f(z[k].z), sigmoid_f(z[k].w));
+    store4(out + r * ldout + (long)h * V + c, mul4(mul4(scale4(inv, x[k]), gn[k]), act == 0 ? mul4(z[k], q) : q));
+  }
+}
+
 // Layer norm of a 32-bit row into the compute type: (x - mean) / sqrt(var + eps) * gain + bias, the variance being the
 // mean of the squared deviations (two passes over the row; bias may be null).
 template <typename T>
@@ -510,6 +544,17 @@ TIS_EXPORT int tis_head_norm_gate(int dtype, const float* o, long ldo, const flo
   if (rows < 0 || H < 1 || H > 65535 || V < 1 || (act != 0 && act != 1))
     return tis_fail("head_norm_gate: bad size rows=%d heads=%d vdim=%d act=%d", rows, H, V, act);
   dim3 grid(rows, H);
+  if (V % 4 == 0 && V <= 1024 && fours32(o, ldo) && fours32(g, ldg) && fours32(gain, 0) && foursT(out, ldout, dtype)) {
+#define S32_HEADS(T, PER) \
+  head_norm_gate_fours_kernel<T, PER><<<grid, TIS_WAVE, 0, stream>>>(o, ldo, g, ldg, gain, gain_per_head, act, eps, (T*)out, ldout, V)
+    if (V <= 256) {
+      S32_DISPATCH(S32_HEADS(float, 1), S32_HEADS(bf16, 1))
+    } else {
+      S32_DISPATCH(S32_HEADS(float, 4), S32_HEADS(bf16, 4))
+    }
+#undef S32_HEADS
+    return tis_launch_status("head_norm_gate");
+  }
   S32_DISPATCH((head_norm_gate_kernel<float><<<grid, TIS_WAVE, 0, stream>>>(o, ldo, g, ldg, gain, gain_per_head, act, eps, (float*)out, ldout, V)),
                (head_norm_gate_kernel<bf16><<<grid, TIS_WAVE, 0, stream>>>(o, ldo, g, ldg, gain, gain_per_head, act, eps, (bf16*)out, ldout, V)))
   return tis_launch_status("head_norm_gate");
@@ -852,6 +897,56 @@ __global__ __launch_bounds__(S32_THREADS) void normed_mean_kernel(const float* _
   }
 }
 
+// The same for a width that is a multiple of four, PER pieces of four a thread (width <= 4 PER THREADS): both rows and gains are
+// asked for at once and stay in registers, and both sums meet in one pass through LDS. us, single values /
+// fours, 2,048 wide: 8 rows 5.3 / 2.6, 1,531 rows 10.7 / 6.1, 2,048 rows 13.6 / 8.4.
+template <int PER, int THREADS>
+__global__ __launch_bounds__(THREADS) void normed_mean_fours_kernel(const float* __restrict__ y0, long ld0,
+                                                                     const float* __restrict__ g0,
+                                                                     const float* __restrict__ y1, long ld1,
+                                                                     const float* __restrict__ g1, float eps,
+                                                                     float* __restrict__ out, int D) {
+  __shared__ float2 red[THREADS / TIS_WAVE];
+  const long r = blockIdx.x;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 a[PER], b[PER], ga[PER], gb[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = (threadIdx.x + k * THREADS) * 4;
+    const bool in = c < D;
+    a[k] = in ? load4(y0 + r * ld0 + c) : zero;
+    b[k] = y1 && in ? load4(y1 + r * ld1 + c) : zero;
+    ga[k] = in ? load4(g0 + c) : zero;
+    gb[k] = y1 && in ? load4(g1 + c) : zero;
+  }
+  float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    s0 += square4(a[k]);
+    s1 += square4(b[k]);
+  }
+  s0 = wave_sum(s0);
+  s1 = wave_sum(s1);
+  if (threadIdx.x % TIS_WAVE == 0) red[threadIdx.x / TIS_WAVE] = make_float2(s0, s1);
+  __syncthreads();
+  s0 = s1 = 0.f;
+#pragma unroll
+  for (int i = 0; i < THREADS / TIS_WAVE; ++i) {
+    s0 += red[i].x;
+    s1 += red[i].y;
+  }
+  const float i0 = 1.f / sqrtf(s0 / (float)D + eps), i1 = y1 ? 1.f / sqrtf(s1 / (float)D + eps) : 0.f;
+  const float share = y1 ? 0.5f : 1.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = (threadIdx.x + k * THREADS) * 4;
+    if (c >= D) continue;
+    float4 v = mul4(scale4(i0, a[k]), ga[k]);
+    if (y1) v = add4(v, mul4(scale4(i1, b[k]), gb[k]));
+    store4(out + r * D + c, scale4(share, v));
+  }
+}
+
 // out = act(z) in the compute type, z 32-bit (a strided view is fine). act 0: tanh-form gelu, 1: silu, 2: sigmoid,
 // 3: the square of relu.
 template <typename T>
@@ -881,6 +976,16 @@ TIS_EXPORT int tis_normed_mean(const float* y0, long ld0, const float* g0, const
                                float* out, int rows, int D, hipStream_t stream) {
   if (rows == 0) return 0;
   if (rows < 0 || D < 1 || !y0 || !g0 || (y1 && !g1) || !out) return tis_fail("normed_mean: bad arguments rows=%d width=%d", rows, D);
+  if (D % 4 == 0 && D <= 4096 && fours32(y0, ld0) && fours32(y1, ld1) && fours32(g0, 0) && fours32(g1, 0) && fours32(out, 0)) {
+#define S32_MEAN(PER, THREADS) normed_mean_fours_kernel<PER, THREADS><<<rows, THREADS, 0, stream>>>(y0, ld0, g0, y1, ld1, g1, eps, out, D)
+    if (D <= 1024) S32_MEAN(1, 256);
+    else if (rows <= 64 && D <= 2048) S32_MEAN(1, 512);
+    else if (rows <= 64) S32_MEAN(1, 1024);
+    else if (D <= 2048) S32_MEAN(2, 256);
+    else S32_MEAN(4, 256);
+#undef S32_MEAN
+    return tis_launch_status("normed_mean");
+  }
   normed_mean_kernel<<<rows, S32_THREADS, 0, stream>>>(y0, ld0, g0, y1, ld1, g1, eps, out, D);
   return tis_launch_status("normed_mean");
 }
