@@ -210,6 +210,34 @@ def test_state_scan_in_segments_by_matrix_products(kind, Hh, D, V, per_head, len
     assert torch.isnan(again[at:last]).all()
 
 
+# Rows that lie one over the other (a row distance of 0, as a broadcast row's), whose last segment is not a whole number of tiles, and
+# rows too far apart for 32-bit addresses, which take the row by row kernels. (The bound is the one above.)
+@pytest.mark.parametrize("kind", ["decay", "gated_max"])
+@pytest.mark.parametrize("distance", [0, (1 << 22) + 4])
+def test_segments_of_rows_at_odd_distances(kind, distance):
+    ops, ref = hip_ops("float32"), TorchOps("cpu", torch.float32)
+    Hh, D, V, n = 2, 32, 16, 131
+    g = torch.Generator().manual_seed(3)
+    cols = 2 * Hh * D + Hh * V + 2 * Hh
+    row = torch.randn(1, cols, generator=g) if distance == 0 else torch.randn(n, cols, generator=g)
+    rows = row.expand(n, cols)
+    if distance:
+        far = torch.empty((n - 1) * distance + cols, dtype=torch.float32, device="cuda").as_strided((n, cols), (distance, 1))
+        far.copy_(rows)
+    else:
+        far = row.cuda().expand(n, cols)
+    at = dict(i_off=cols - 2 * Hh, f_off=cols - Hh, cap=9.0)
+    bi, bf, decay = torch.randn(Hh, generator=g), 2 + torch.randn(Hh, generator=g), torch.rand(n, Hh * D, generator=g) * 0.3 + 0.7
+    res = []
+    for o, dev, p in ((ops, "cuda", far), (ref, "cpu", rows)):
+        st = torch.zeros(1, ops.state_scan_floats(kind, Hh, D, V), device=dev)
+        kw = dict(decay=decay.to(dev)) if kind == "decay" else dict(at, bias_i=bi.to(dev), bias_f=bf.to(dev))
+        out = o.state_scan(kind, p, 0, Hh * D, 2 * Hh * D, D ** -0.5, st, fake_batch([(0, 0, n)], [0], None, 1, dev), Hh, D, V, **kw)
+        res.append((out, st))
+    close(res[0][0], res[1][0], "float32", "results")
+    close(res[0][1], res[1][1], "float32", "states")
+
+
 # Heads of more than 128 key channels take the row by row kernels for segments. Every workgroup of the pass over the states reads a
 # request's running maximum, so nothing may write the new one before they all have: single-row requests beside a long one, whose
 # pass is the shortest. (The bound is the one above.)

@@ -26,6 +26,7 @@
 //           exp(m'_t - m_t) and the start's part scaled by exp(F_t + m_start - m_t); o_t as above.
 // Everything is still 32-bit; only the order of additions differs from the token-by-token walk.
 #include "common.h"
+#include <algorithm>
 #include <type_traits>
 
 TIS_DEFINE_LAST_ERROR(tis_state_scan)
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int e = 0; e < PER; ++e) {
       const int r = r0 + e * STEP;
       sq[r][d] = q[e] * q_scale;
-      sk[r][d] = k[e];
+      sk[r][d] = r < seg.n ? k[e] : 0.f;         // (rows may lie one over the other: a step of 0)
       if (KIND == 0) sa[r][d] = r < seg.n && d < D ? a[e] : 1.f;
     }
   }
@@ -983,15 +984,17 @@ TIS_EXPORT int tis_state_scan_segmentable(int D) {
   return sizeof(float) * ((size_t)D * SG_COLS + (size_t)SG_ROWS * (D + 1) + SG_ROWS) <= 64 * 1024;
 }
 
-// Whether a segmented call goes through the kernels of matrix products.
-static bool by_products(int n_seqs, int seg_len, int D, long rows) {
-  return D <= 128 && seg_len <= SP_ROWS && n_seqs <= 65535 && sp_most(rows, seg_len, n_seqs) <= 65535;
+// Whether a segmented call goes through the kernels of matrix products, whose addresses inside a segment are 32-bit (ld: the longest
+// distance between two rows).
+static bool by_products(int n_seqs, int seg_len, int D, long rows, long ld) {
+  return D <= 128 && ld >= 0 && ld < (1L << 22) && seg_len <= SP_ROWS && n_seqs <= 65535 && sp_most(rows, seg_len, n_seqs) <= 65535;
 }
 
-// 32-bit floats of the workspace a segmented call needs: a block for every segment and head; or, off the matrix products, the
+// 32-bit floats of the workspace a segmented call needs (ld: the longest row distance of projections, decays and results): a block for every segment and head; or, off the matrix products, the
 // states, then `rows` lines of decay products or gate sums.
-TIS_EXPORT long tis_state_scan_workspace(int kind, int n_seqs, int segments, int seg_len, int rows, int H, int D, int V) {
-  if (by_products(n_seqs, seg_len, D, rows)) return sp_most(rows, seg_len, n_seqs) * H * SegmentBlock(D, V).floats;
+TIS_EXPORT long tis_state_scan_workspace(int kind, int n_seqs, int segments, int seg_len, int rows, int H, int D, int V,
+                                         long ld) {
+  if (by_products(n_seqs, seg_len, D, rows, ld)) return sp_most(rows, seg_len, n_seqs) * H * SegmentBlock(D, V).floats;
   return (long)n_seqs * segments * H * ((long)D * V + D + 2) + (kind == 0 ? (long)rows * H * D : (long)rows * H * 3);
 }
 
@@ -1033,7 +1036,7 @@ TIS_EXPORT int tis_state_scan(int kind, const float* proj, long ldp, int q_off, 
   if (segments > 0) {
     if (seg_len < 1 || rows < 1 || !workspace || (long)n_seqs * segments > 0x7fffffffL)
       return tis_fail("state_scan: %d segments of %d rows need a workspace", segments, seg_len);
-    if (by_products(n_seqs, seg_len, D, rows)) {
+    if (by_products(n_seqs, seg_len, D, rows, std::max(ldo, std::max(ldp, ldd)))) {
       if ((uintptr_t)workspace % 16) return tis_fail("state_scan: the workspace is not 16 bytes aligned");
 #define SP_LAUNCH(KIND, NT)                                                                                                       \
   return launch_products<KIND, NT>(proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off, bias_i, bias_f, cap, state, \

@@ -2253,7 +2253,8 @@ class HipOps:
             segments = -(-batch.max_seq_rows // seg_len)
             lib.cdll.tis_state_scan_workspace.restype = c_long
             floats = lib.cdll.tis_state_scan_workspace(0 if kind == "decay" else 1, batch.n_seqs, segments, seg_len, n,
-                                                       n_heads, dim, vdim)
+                                                       n_heads, dim, vdim, c_long(max(proj.stride(0), out.stride(0),
+                                                       decay.stride(0) if decay is not None else 0)))
             workspace = torch.empty(floats, dtype=torch.float32, device=self.device)
         lib.tis_state_scan(
             0 if kind == "decay" else 1, _ptr(proj), proj.stride(0), q_off, k_off, v_off, float(q_scale), _ptr(decay),
