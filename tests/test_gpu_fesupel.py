@@ -118,6 +118,42 @@ def test_matrix_core_attention_with_mixed_sigmoid_weights(Hq, G, kd, vd, chunk, 
         close(res[0], res[1], "bfloat16", f"attention of {seq_rows}", tol=2.5e-2)
 
 
+def test_mixed_weights_are_quotients_rounded_as_a_division_rounds_them():
+    """The matrix-core kernel's weights, to the last bit: with scores of zero and biases that are whole numbers on base 2 a weight is
+    1 / (1 + 2^n), the power is exact, and only the reciprocal rounds. Head 0's weight is a half; every other head takes its own weight
+    less the rounded quotient times that half, so that what is left is the weight's error, exact in bfloat16. Half a unit of the last place
+    is a division's error; the bound leaves the hundredth of one for a quotient next to the middle of two numbers."""
+    ops = hip_ops("bfloat16")
+    H, kd, vd, ps = 16, 128, 128, 16
+    log2e = np.float32(1.4426950408889634)
+    exponents = []
+    for n in list(range(-23, 24)) + list(range(30, 60)) + [128, 300]:      # 1 + 2^n is exact, or 2^n to all 24 bits, or infinite: weight 0
+        bias = np.float32(-n / float(log2e))
+        for b in (bias, np.nextafter(bias, np.float32(np.inf)), np.nextafter(bias, np.float32(-np.inf))):
+            if np.float32(-log2e * b) == n:
+                exponents.append((n, float(b)))
+                break
+    assert len(exponents) >= 45
+    plane = torch.zeros(1, ps * (kd + vd), dtype=torch.bfloat16)
+    plane[0, ps * kd:] = 1.0
+    for at in range(0, len(exponents), H - 1):
+        part = exponents[at:at + H - 1]
+        head_bias, talk, want = torch.zeros(H), torch.zeros(H, H), torch.full((H,), 0.5, dtype=torch.float64)
+        talk[0, 0] = 1.0
+        for h, (n, b) in enumerate(part, 1):
+            want[h] = 1.0 / (1.0 + 2.0 ** n) if n < 128 else 0.0
+            head_bias[h] = b
+            talk[h, h], talk[h, 0] = 1.0, -2.0 * want[h].float()
+        batch = fake_batch([(0, 0, 1)], [0], [[0]], ps, "cuda")
+        out = ops.mixed_sigmoid_attention(torch.zeros(1, H * kd, dtype=torch.bfloat16, device="cuda"), plane.cuda(), batch, "g", H, 1, kd, vd, ps,
+                                          0, 0.5, 0.0, head_bias.cuda(), talk.cuda()).double().cpu().view(H, vd)
+        assert (out == out[:, :1]).all() and out[0, 0] == 0.5
+        for h, (n, _) in enumerate(part, 1):
+            weight = out[h, 0].item() + want[h].float().double().item()
+            unit = float(np.spacing(np.float32(want[h].item()))) if want[h] > 0 else 0.0
+            assert abs(weight - want[h].item()) <= 0.51 * unit, (n, weight, want[h].item(), (weight - want[h].item()) / (unit or 1.0))
+
+
 def test_attention_of_many_rows_and_long_chunks():
     """Hundreds of rows (one workgroup a row, no key splits) over chunks longer than a block of keys."""
     ops, ref = hip_ops("float32"), TorchOps("cpu", torch.float32)

@@ -44,7 +44,18 @@ __device__ __forceinline__ bf16x8 amx_load8(const bf16* p) { return *reinterpret
 __device__ __forceinline__ bf16x4 amx_load4(const bf16* p) { return *reinterpret_cast<const bf16x4*>(p); }
 
 __device__ __forceinline__ float amx_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-__device__ __forceinline__ float amx_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+// 1 / x for x >= 1 and infinity: the instruction's quotient is off by up to a unit in the last place; one Newton step rounds it as a
+// division does (but for the rare quotient next to the middle of two numbers) in two multiply-adds instead of a division's ten instructions. The step would
+// make NaN of infinity, which keeps its 0; NaN stays NaN.
+__device__ __forceinline__ float amx_inverse(float x) {
+  const float r = __builtin_amdgcn_rcpf(x), better = fmaf(fmaf(-x, r, 1.f), r, r);
+  return x == INFINITY ? 0.f : better;
+}
+// the same where x is known to be finite
+__device__ __forceinline__ float amx_inverse_finite(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return fmaf(fmaf(-x, r, 1.f), r, r);
+}
 
 // items: (first row, rows) pairs, or null: item i is row i alone. LDS (floats): talk [4 HPW][4 HPW], heads that are mixed from outside,
 // wave's heads inside | weights [H][64][8].
@@ -53,7 +64,7 @@ __device__ __forceinline__ float amx_rcp(float x) { return __builtin_amdgcn_rcpf
 // of 4 heads, 512 multiply-adds of the mixture), as 16 heads' results and queries leave one wave a SIMD; so nothing may wait
 // for memory either: the next step's pages are looked up a step ahead, its first head's keys are fetched as soon as this
 // step's scores are made and the values before this step's weights meet, once for the heads that share them. us, 16
-// heads of 128 in chunks of 1,024: 1,531 rows 203 before that (and with divisions), 96 now; 5 single rows near 600 keys 10.4, 8.9.
+// heads of 128 in chunks of 1,024, with the sum of the cuts: 1,531 rows 203 before that (and with divisions), 98 now (92 with bare reciprocals).
 __global__ __launch_bounds__(256) void attention_mixed_mfma_kernel(
     const bf16* __restrict__ q, long ldq, const bf16* __restrict__ plane, const int* __restrict__ block_tables, int bt_ld,
     const int* __restrict__ row_seq, const int* __restrict__ positions, const int* __restrict__ items,
@@ -175,11 +186,11 @@ __global__ __launch_bounds__(256) void attention_mixed_mfma_kernel(
             float x;               // minus the capped score with its bias, times log2 e
             if (softcap > 0.f) {
               const float e2 = amx_exp2(fminf(fmaxf(st[i] * to_cap, -30.f * LOG2E), 30.f * LOG2E));
-              x = fmaf(from_cap, fmaf(-2.f, amx_rcp(1.f + e2), 1.f), hb[u]);
+              x = fmaf(from_cap, fmaf(-2.f, amx_inverse_finite(1.f + e2), 1.f), hb[u]);
             } else {
               x = fmaf(st[i], plain, hb[u]);
             }
-            w[i] = seen[t * 4 + i] ? amx_rcp(1.f + amx_exp2(x)) : 0.f;
+            w[i] = seen[t * 4 + i] ? amx_inverse(1.f + amx_exp2(x)) : 0.f;
           }
           *reinterpret_cast<f32x4*>(dst + t * 4) = w;
         }
