@@ -100,6 +100,18 @@ def test_sums_and_norms_in_fours(dtype, n, D, shift):
         close(res[2], res[3], dtype, "head_norm_gate, a gain a head")
 
 
+@pytest.mark.parametrize("D", [1024, 1028, 2048, 2052, 4096, 4100, 1030])
+def test_a_row_of_the_mean_of_norms_does_not_depend_on_how_many_there_are(D):
+    """The same bits alone, among 64 rows and among 65, where the workgroups are of other sizes; widths read in fours and not."""
+    ops = hip_ops("float32")
+    g = torch.Generator().manual_seed(D)
+    y0, y1, g0, g1 = (torch.randn(s, generator=g).cuda() for s in ((65, D), (65, D), (D,), (D,)))
+    for two in (False, True):
+        part = lambda a, b: ops.normed_mean([(y0[a:b], g0), (y1[a:b], g1)][:1 + two], 1e-5)
+        whole = part(0, 65)
+        assert torch.equal(part(0, 64), whole[:64]) and torch.equal(part(64, 65), whole[64:])
+
+
 @pytest.mark.parametrize("D", [44, 300, 1500, 4200])      # (a row in 4 or 16 registers a thread, or in memory)
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_sums_and_norms_of_the_stream(dtype, D):

@@ -870,7 +870,7 @@ static void launch_lowrank(const float* low, long ldl, int rank, const float* w2
 }
 
 // out[r] = (1 / n) * sum_i y_i[r] / sqrt(mean(y_i[r]^2) + eps) * gain_i: the mean of one or two RMS-normed rows, 32-bit.
-// One workgroup a row; the sums' order depends on the width alone.
+// One workgroup a row; the sums' order depends on the width (and on whether it can be read in fours, see below) alone.
 __global__ __launch_bounds__(S32_THREADS) void normed_mean_kernel(const float* __restrict__ y0, long ld0,
                                                                    const float* __restrict__ g0,
                                                                    const float* __restrict__ y1, long ld1,
@@ -898,17 +898,23 @@ __global__ __launch_bounds__(S32_THREADS) void normed_mean_kernel(const float* _
 }
 
 // The same for a width that is a multiple of four, PER pieces of four a thread (width <= 4 PER THREADS): both rows and gains are
-// asked for at once and stay in registers, and both sums meet in one pass through LDS. us, single values /
-// fours, 2,048 wide: 8 rows 5.3 / 2.6, 1,531 rows 10.7 / 6.1, 2,048 rows 13.6 / 8.4.
+// asked for at once and stay in registers, and both sums meet in one pass through LDS: every wave sums runs of 256 columns, and the runs'
+// sums are added in the order of the columns, whichever threads they come from, so a row's bits are the same on workgroups of any
+// size. us, 2,048 wide, single values / fours: 8 rows 5.3 / 2.5, 1,531 rows 10.7 / 7.1, 2,048 rows 13.6 / 8.6 (added in the order of the
+// threads, which tells 64 rows from 65: 2.5, 6.4, 8.7; workgroups of 512 for every number of rows: 2.5, 7.4, 9.6).
 template <int PER, int THREADS>
 __global__ __launch_bounds__(THREADS) void normed_mean_fours_kernel(const float* __restrict__ y0, long ld0,
                                                                      const float* __restrict__ g0,
                                                                      const float* __restrict__ y1, long ld1,
                                                                      const float* __restrict__ g1, float eps,
                                                                      float* __restrict__ out, int D) {
-  __shared__ float2 red[THREADS / TIS_WAVE];
+  constexpr int WAVES = THREADS / TIS_WAVE;
+  __shared__ float2 red[PER * WAVES];
   const long r = blockIdx.x;
   const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  // (multiply-adds spelled out: which of two products the compiler takes into one may differ from kernel to kernel)
+  auto squares = [](float4 v) { return fmaf(v.y, v.y, v.x * v.x) + fmaf(v.w, v.w, v.z * v.z); };
+  auto both = [](float p, float g, float q, float h) { return fmaf(p, g, q * h); };
   float4 a[PER], b[PER], ga[PER], gb[PER];
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
@@ -919,19 +925,15 @@ __global__ __launch_bounds__(THREADS) void normed_mean_fours_kernel(const float*
     ga[k] = in ? load4(g0 + c) : zero;
     gb[k] = y1 && in ? load4(g1 + c) : zero;
   }
-  float s0 = 0.f, s1 = 0.f;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    s0 += square4(a[k]);
-    s1 += square4(b[k]);
+    const float2 run = make_float2(wave_sum(squares(a[k])), wave_sum(squares(b[k])));
+    if (threadIdx.x % TIS_WAVE == 0) red[k * WAVES + threadIdx.x / TIS_WAVE] = run;
   }
-  s0 = wave_sum(s0);
-  s1 = wave_sum(s1);
-  if (threadIdx.x % TIS_WAVE == 0) red[threadIdx.x / TIS_WAVE] = make_float2(s0, s1);
   __syncthreads();
-  s0 = s1 = 0.f;
+  float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-  for (int i = 0; i < THREADS / TIS_WAVE; ++i) {
+  for (int i = 0; i < PER * WAVES; ++i) {
     s0 += red[i].x;
     s1 += red[i].y;
   }
@@ -941,8 +943,9 @@ __global__ __launch_bounds__(THREADS) void normed_mean_fours_kernel(const float*
   for (int k = 0; k < PER; ++k) {
     const int c = (threadIdx.x + k * THREADS) * 4;
     if (c >= D) continue;
-    float4 v = mul4(scale4(i0, a[k]), ga[k]);
-    if (y1) v = add4(v, mul4(scale4(i1, b[k]), gb[k]));
+    const float4 p = scale4(i0, a[k]), q = scale4(i1, b[k]);
+    float4 v = mul4(p, ga[k]);
+    if (y1) v = make_float4(both(p.x, ga[k].x, q.x, gb[k].x), both(p.y, ga[k].y, q.y, gb[k].y), both(p.z, ga[k].z, q.z, gb[k].z), both(p.w, ga[k].w, q.w, gb[k].w));
     store4(out + r * D + c, scale4(share, v));
   }
 }
