@@ -482,3 +482,22 @@ def test_the_delta_rules_walk_in_chunks(Hh, G, D, V, seqs):
     before[at:firsts[longest] + seqs[longest]] = False
     torch.testing.assert_close(broken[before], out[before], rtol=1e-4, atol=1e-5)
     assert not torch.isfinite(broken[at]).any()
+
+
+@pytest.mark.parametrize("lens,chunks", [([1] * 64, False), ([47, 47], False), ([48], True), ([1] * 20 + [48], True)])
+def test_the_delta_rule_asks_for_chunks_only_where_a_request_is_long(lens, chunks):
+    """Single tokens of 64 requests are many rows and no long request: the call takes no memory beyond its result (the chunks' operands
+    would be megabytes, and two kernels would be launched for them); one request of 48 rows does."""
+    ops = hip_ops("float32")
+    H, D, V, n = 4, 64, 32, sum(lens)
+    firsts = [sum(lens[:i]) for i in range(len(lens))]
+    b = fake_batch([(f, 0, r) for f, r in zip(firsts, lens)], list(range(len(lens))), None, 8, "cuda")
+    C = 2 * H * D + H * V
+    u, decay = torch.randn(n, C + H, device="cuda"), torch.rand(n, H * D, device="cuda")
+    state = torch.zeros(len(lens), H * V * D, device="cuda")
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = ops.delta_scan(u, 0, H * D, 2 * H * D, C, decay, state, b, H, H, D, V)
+    more = torch.cuda.max_memory_allocated() - before - out.numel() * 4
+    assert (more > 4096) == chunks, more

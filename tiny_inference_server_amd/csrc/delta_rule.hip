@@ -533,23 +533,26 @@ TIS_EXPORT int tis_delta_prepare(const float* proj, long ldp, int conv_off, int 
 // The most chunks that `rows` rows can have, over all requests of DR_CHUNK_FROM rows and more (each begins one that it may not fill).
 static long dc_most(long rows) { return rows / DC + rows / DR_CHUNK_FROM + 1; }
 
-// Floats of work space that tis_delta_scan wants for the walk in chunks; 0: rows too few for it.
-TIS_EXPORT long tis_delta_scan_work(int rows, int H, int D) {
-  return rows < DR_CHUNK_FROM ? 0 : dc_most(rows) * H * dc_floats((D + 63) / 64 * 64);
+// Floats of work space that tis_delta_scan wants for the walk in chunks; 0: no request (the longest has `longest` rows) is long enough for it.
+TIS_EXPORT long tis_delta_scan_work(int rows, int longest, int H, int D) {
+  return longest < DR_CHUNK_FROM ? 0 : dc_most(rows) * H * dc_floats((D + 63) / 64 * 64);
 }
 
-// work: null, or tis_delta_scan_work floats, 16-byte aligned: requests of DR_CHUNK_FROM rows and more are then walked in chunks.
+// longest: the rows of the longest request, as the host knows it. work: null, or tis_delta_scan_work floats, 16-byte aligned: requests of
+// DR_CHUNK_FROM rows and more are then walked in chunks. A step without such a request (decoded tokens, however many) launches the
+// walk row by row alone: the kernels of the chunks would find nothing to do in thousands of workgroups (64 single rows of 128 x 256,
+// us with / without them: 8 heads 59 / 53, 16 heads 108 / 99; two requests of 47 rows 20 / 17).
 TIS_EXPORT int tis_delta_scan(const float* u, long ldu, int q_off, int k_off, int v_off, int beta_off, const float* decay,
                               long ldd, float* state, long lds, const int* cu_rows, const int* seq_slots, int n_seqs, int rows,
-                              float* work, float* out, long ldo, int H, int G, int D, int V, hipStream_t stream) {
+                              int longest, float* work, float* out, long ldo, int H, int G, int D, int V, hipStream_t stream) {
   if (n_seqs == 0) return 0;
   if (n_seqs < 0 || n_seqs > 65535 || rows < 0 || H < 1 || H > 65535 || G < 1 || H % G || D < 1 || D > 256 || V < 1 || lds % 4 ||
       ((uintptr_t)state % 16) || ((uintptr_t)work % 16))
     return tis_fail("delta_scan: bad size requests=%d heads=%d qk_heads=%d dim=%d (at most 256) vdim=%d, or state lines that are "
                     "not 16 bytes aligned", n_seqs, H, G, D, V);
-  const bool chunks = work && rows >= DR_CHUNK_FROM && (V + 15) / 16 <= 65535 && dc_most(rows) < (1L << 31);
+  const bool chunks = work && longest >= DR_CHUNK_FROM && (V + 15) / 16 <= 65535 && dc_most(rows) < (1L << 31);
   const int from = chunks ? DR_CHUNK_FROM : 0x7fffffff;
-  if (!(chunks && n_seqs == 1)) {           // (a single request of that many rows has none left for the walk row by row)
+  if (!(chunks && n_seqs == 1 && longest == rows)) {      // (a single request of that many rows leaves none for the walk row by row)
     const int R = D <= 16 ? 1 : D <= 32 ? 2 : D <= 64 ? 4 : D <= 128 ? 8 : 16;
     const int tokens = R <= 8 ? 16 : 8;
     size_t lds_bytes = 2 * (size_t)tokens * (3 * 16 * R + 20) * sizeof(float);      // two buffers of rows

@@ -156,7 +156,7 @@ _SIGNATURES["ssm_parts"] = ("tis_ssm", {
 
 _SIGNATURES["delta_rule"] = ("tis_delta_rule", {
     "tis_delta_prepare": [_P, _L, _I, _I, _P, _I, _P, _L, _I, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _P],
-    "tis_delta_scan": [_P, _L, _I, _I, _I, _I, _P, _L, _P, _L, _P, _P, _I, _I, _P, _P, _L, _I, _I, _I, _I, _P],
+    "tis_delta_scan": [_P, _L, _I, _I, _I, _I, _P, _L, _P, _L, _P, _P, _I, _I, _I, _P, _P, _L, _I, _I, _I, _I, _P],
 })
 
 _SIGNATURES["attention_mixed"] = ("tis_attention_mixed", {
@@ -2191,14 +2191,15 @@ class HipOps:
             raise KernelError("delta_scan: state lines must be 16 bytes aligned")
         out = torch.empty(n, n_heads * vdim, dtype=torch.float32, device=self.device)
         lib = self._lazy("delta_rule")
-        # (work space for requests of many rows, which are walked in chunks; without it row by row)
+        # (work space if a request has many rows, which are walked in chunks; without it row by row)
+        longest = int(batch.max_seq_rows)
         lib.cdll.tis_delta_scan_work.restype = c_long
-        floats = lib.cdll.tis_delta_scan_work(n, n_heads, dim)
+        floats = lib.cdll.tis_delta_scan_work(n, longest, n_heads, dim)
         work = torch.empty(floats, dtype=torch.float32, device=self.device) if 0 < floats <= _DELTA_WORK_FLOATS else None
         lib.tis_delta_scan(
             _ptr(u), u.stride(0), int(q_off), int(k_off), int(v_off), int(beta_off), _ptr(decay), decay.stride(0), _ptr(state),
-            state.stride(0), _ptr(batch.cu_rows), _ptr(batch.seq_slots), batch.n_seqs, n, _ptr(work), _ptr(out), out.stride(0),
-            n_heads, qk_heads, dim, vdim, self._stream())
+            state.stride(0), _ptr(batch.cu_rows), _ptr(batch.seq_slots), batch.n_seqs, n, longest, _ptr(work), _ptr(out),
+            out.stride(0), n_heads, qk_heads, dim, vdim, self._stream())
         return out
 
     # ---- recurrent mixers with a matrix state per head ---------------------------------------------------
