@@ -1032,16 +1032,16 @@ def test_tiled_product_of_few_steps_of_each_tile(ops_for, M, N, K):
 
 
 @pytest.mark.parametrize("groups,line,N,K,counts", [
-    (8, 2048, 2048, 72, "even"),            # 4,096 entries: tiles of 192 columns
-    (8, 1000, 5632, 264, "even"),           # 256 x 256
-    (8, 500, 2044, 520, "uneven"),          # 128 x 128, a workgroup a unit
-    (8, 129, 5636, 256, "uneven"),          # 128 x 128, two a unit
-    (8, 30, 1024, 320, "uneven"), (3, 24, 60, 64, "one"), (130, 40, 132, 200, "uneven"),   # 64 x 64; more groups than lanes
+    (8, 2048, 2048, 72, "even"), (8, 129, 5636, 256, "uneven"),         # tiles of 128 x 128 on four waves
+    (8, 1000, 5632, 264, "even"), (8, 500, 2044, 520, "uneven"),        # 128 x 128 on eight
+    (3, 24, 60, 64, "one"),                                             # 64 x 64
+    (8, 30, 1024, 320, "uneven"), (130, 40, 132, 200, "uneven"),        # few entries a group: straight from memory
 ])
 @pytest.mark.parametrize("out32,act", [(True, 0), (False, 2)])
 def test_grouped_product_in_tiles_numbered_through(ops_for, groups, line, N, K, counts, out32, act):
-    """Every tile of the grouped product of many entries: groups that are empty, hold one entry, end inside a tile or hold every
-    row; entries that no list names stay as they were. 32-bit sums against 64 bits, the gate against the sums."""
+    """Groups by themselves, as full as a group can be: groups that are empty, hold one entry, end inside a tile or hold every
+    row; entries that no list names stay as they were. 32-bit sums against 64 bits, the gate against the sums. (Uneven groups in one
+    call, and every tile: the next test.)"""
     from tiny_inference_server_amd.ops.hip_ops import _ptr
     ops = ops_for(torch.bfloat16)
     g = torch.Generator().manual_seed(groups * N + K)
@@ -1089,6 +1089,69 @@ def test_grouped_product_in_tiles_numbered_through(ops_for, groups, line, N, K, 
             else:
                 gate, up = want[:, 0::2].clamp(max=7.0), want[:, 1::2].clamp(-7.0, 7.0)
                 torch.testing.assert_close(out[perm[e].long()].double(), gate * torch.sigmoid(1.702 * gate) * (up + 1.0), rtol=8e-3, atol=2e-3)
+
+
+def grouped_tile(ops, lists, groups, most_rows, most_entries, N, K):
+    """The tile a grouped product takes: 0 to 4 for 128 x 192, 64 x 64, 128 x 128 on eight waves, 256 x 256, 128 x 128 on four; -1: none."""
+    from ctypes import c_long
+    return ops._lazy("experts").cdll.tis_grouped_tile(lists, groups, most_rows, c_long(most_entries), N, K)
+
+
+@pytest.mark.parametrize("tile,groups,line,N,K", [(0, 8, 2048, 2044, 328), (0, 8, 2048, 2048, 256), (1, 130, 1040, 132, 200), (1, 12, 90, 1036, 1032),
+                                                  (2, 8, 500, 2044, 520), (2, 70, 600, 640, 264), (3, 8, 2048, 5628, 264), (3, 8, 2040, 5632, 320),
+                                                  (4, 8, 129, 5636, 264), (4, 67, 1600, 1024, 72)])
+@pytest.mark.parametrize("out32,act", [(True, 0), (False, 2)])
+def test_uneven_groups_of_a_product_at_once(ops_for, tile, groups, line, N, K, out32, act):
+    """Every tile of the grouped product, all groups in one call and no two of one size: empty groups, groups of one entry, of a whole tile and
+    of one more, before, at and behind the 64th and the last group; entries that no list names stay as they were."""
+    from tiny_inference_server_amd.ops.hip_ops import _ptr
+    ops = ops_for(torch.bfloat16)
+    entries = 2 * line                       # as a router that takes two gives them
+    assert grouped_tile(ops, 1, groups, line, entries, N, K) == tile
+    g = torch.Generator().manual_seed(groups * N + K)
+    share = torch.zeros(groups, dtype=torch.long)
+    for e, n in ((0, 3), (2, 1), (groups // 2, 65), (63, 64), (64, 129), (65, 2), (groups - 3, 130), (groups - 1, 1)):
+        if e < groups and int(share.sum()) + n <= entries:
+            share[e] = min(n, line)
+    rest = entries - int(share.sum()) - 5    # five entries are in no list
+    for e in torch.randperm(groups, generator=g).tolist():
+        if share[e] == 0 and e % 3 and rest > 0:
+            share[e] = min(rest, line, int(torch.randint(1, 2 * entries // groups + 2, (1,), generator=g)))
+            rest -= int(share[e])
+    perm = torch.randperm(entries, generator=g)
+    lists = torch.zeros(groups, line, dtype=torch.int32)
+    group_of, at = torch.full((entries,), -1), 0
+    for e, n in enumerate(share.tolist()):
+        mine = perm[at:at + n].sort().values
+        lists[e, :n], group_of[mine], at = mine.to(torch.int32), e, at + n
+    lists, cnt = lists.cuda(), share.to(torch.int32).cuda()
+    x, w = rnd((line, K + 8), torch.bfloat16, 811).cuda()[:, :K], rnd((groups, N, K), torch.bfloat16, 812, K ** -0.5).cuda()
+    out = torch.full((entries, N // 2 if act else N), 7.5, device="cuda", dtype=torch.float32 if out32 else torch.bfloat16)
+    ops._lazy("experts").tis_grouped_linear(1, 0 if out32 else 1, _ptr(x), x.stride(0), 0, 2, _ptr(w), _ptr(out), out.shape[1], 0,
+                                            _ptr(lists), _ptr(cnt), line, groups, line, entries, N, K, act, None, 0, 7.0, ops._stream())
+    for e in range(groups):
+        mine = (group_of == e).nonzero()[:, 0].cuda()
+        rows = x[mine // 2].double()
+        want = rows @ w[e].double().T
+        if act:
+            gate, up = want[:, 0::2].clamp(max=7.0), want[:, 1::2].clamp(-7.0, 7.0)
+            torch.testing.assert_close(out[mine].double(), gate * torch.sigmoid(1.702 * gate) * (up + 1.0), rtol=8e-3, atol=2e-3)
+        else:       # 32-bit sums of exact products: K additions, each within half a unit of the sum of magnitudes so far
+            bound = (K + 2) * 2.0 ** -24 * (rows.abs() @ w[e].double().abs().T)
+            assert ((out[mine].double() - want).abs() <= bound).all(), e
+    assert (out[(group_of < 0).cuda()] == 7.5).all()
+
+
+def test_when_a_grouped_product_takes_tiles(ops_for):
+    """With lists by the entries a group and the rows of the step, without by the rows of every group."""
+    ops = ops_for(torch.bfloat16)
+    tiles = lambda *a: grouped_tile(ops, *a) >= 0
+    for groups, top in ((2, 1), (8, 2), (64, 8), (64, 2), (128, 8)):
+        for K, per in ((64, 12), (1016, 12), (1024, 4), (2048, 4)):
+            for n in range(1, 600):
+                want = n > 16 and n * top >= max(48, per * groups)
+                assert tiles(1, groups, n, n * top, 2048, K) == want, (groups, top, K, n)
+    assert [tiles(0, 16, n, 16 * n, 512, 128) for n in (48, 63, 64, 2048)] == [False, False, True, True]
 
 
 @pytest.mark.parametrize("M", [1, 7, 8])

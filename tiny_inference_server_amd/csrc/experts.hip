@@ -15,7 +15,9 @@
 // g * c_group: with a_div = top the input rows are the step's rows and the outputs lie by assignment (an expert's first
 // product), with a_div = 1 both lie by assignment (its second); without lists every group takes all rows, and a_group /
 // c_group move from one group's columns to the next (a product per head on a head's own columns). Sums are 32-bit in
-// an order that depends on K alone, so a row's result does not depend on what else is in the step.
+// an order that depends on K and on the kernel: the products straight from memory add steps of 32, the tiles steps of 16. Within one of them a
+// row's result does not depend on what else is in the step; which of them a step takes hangs on its entries (tis_grouped_tile), and a
+// row's last bits may differ from one to the other.
 #include "tile_loop.h"
 
 TIS_DEFINE_LAST_ERROR(tis_experts)
@@ -473,6 +475,49 @@ TIS_EXPORT int tis_expert_lists(const int* ids, int n_assign, int n_experts, int
   return tis_launch_status("expert_lists");
 }
 
+static int g_units = 256;      // compute units of the device: set by whoever knows (the default is an MI355X)
+TIS_EXPORT void tis_experts_units(int n) { if (n > 0) g_units = n; }
+
+// The tiles of grouped_tiles_kernel, and the microseconds a step of 64 takes with r workgroups a compute unit:
+//   128 x 192, four waves, two buffers, two a unit     1.05 r, at least 1.15
+//   64 x 64, four waves, four buffers, two a unit      0.3 r, at least 0.33
+//   128 x 128, eight waves, four buffers               0.58 a round
+//   256 x 256, eight waves, two buffers                1.85 a round
+//   128 x 128, four waves, two buffers, two a unit     0.78 r, at least 0.8
+struct GroupedShape { int bm, bn; float step, least; bool rounds; };
+static const GroupedShape g_shapes[5] = {{128, 192, 1.05f, 1.15f, false}, {64, 64, 0.3f, 0.33f, false}, {128, 128, 0.58f, 0.58f, true},
+                                         {256, 256, 1.85f, 1.85f, true}, {128, 128, 0.78f, 0.8f, false}};
+
+// The tile that a grouped product of bfloat16 rows that lie as it needs them takes, an index into g_shapes; -1: the products straight from memory.
+// lists: most_rows is the most entries a group can have, most_entries the most that all groups have together.
+// Without lists: from 64 rows of every group on (16 groups of 512 of 128, us, straight from memory / tiles: 48 rows 4.4 / 4.7, 64 8.7 / 4.8).
+// With lists, what counts is the entries a group: while they are few both ways are bound by the matrices' way from memory, where 16 x 64
+// straight from memory waits least. Up to 16 rows in the step no group can need a second tile of 16 there, and it is as fast or faster
+// for any groups (16 groups, 64 entries: 2,816 of 1,024 20.9 / 28.3; 64 groups, 128 entries: 5,632 of 2,048 221 / 246, 2,048 of 704 36 / 47).
+// Beyond, from 48 entries and 4 a group on (12 below 1,024 inner columns, where a tile's few steps do not hide its beginning), us
+// straight from memory / tiles at 1, 2, 4, 6, 8, 12 entries a group, 64 groups of 8 choices a row: 5,632 of 2,048 189 / 193, 221 / 246, 277 / 281, 281 / 267,
+// 322 / 290, 370 / 293; 2,048 of 2,816 106 / 96, 127 / 127, 140 / 135, 152 / 137, 164 / 140, 204 / 140; 2,048 of 704 26 / 35, 36 / 47, 39 / 49, 42 / 49,
+// 44 / 49, 55 / 51. 8 groups of 2, at 4, 6, 8, 12: 5,632 of 2,048 43 / 52, 54 / 52, 54 / 52, 108 / 52; 2,048 of 2,816 25 / 24, 35 / 24, 35 / 24, 31 / 24.
+// (The way straight from memory is not even: its workgroups of tiles that no group fills are spread so that heights of 2, 4, 8 .. tiles leave
+// part of the chip idle. Over 805 sizes of 2 to 128 groups and 1 to 64 entries a group, this rule takes 1.04 times the better way's time, and
+// on 58 of them more than the way straight from memory: most by 1 or 2 us of 8, 64 groups of 2,816 of 1,024 at 4 to 6 entries by an eighth.
+// A line at 48 entries alone takes 1.04 times too, but more than the way straight from memory on 151, up to 1.5 times.)
+TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_entries, int N, int K) {
+  if (lists ? most_rows <= 16 || most_entries < 48 || most_entries < (K < 1024 ? 12L : 4L) * groups : most_rows < 64) return -1;
+  int pick = 0;
+  float best = INFINITY;
+  for (int i = 0; i < 5; ++i) {
+    if (K < 256 && i != 1 && i != 4) continue;     // few steps: what counts is a tile's beginning and end (2,048 rows, 16 groups
+    const GroupedShape& q = g_shapes[i];           // of 512 of 128: 24 us in tiles of 128 x 128, 33 in 256 x 256)
+    const long tn = (N + q.bn - 1) / q.bn;
+    // (with lists, entries / bm row tiles and half a tile more in every group)
+    const float r = (lists ? (float)most_entries / q.bm + 0.5f * groups : (float)((long)groups * ((most_rows + q.bm - 1) / q.bm))) * tn / g_units;
+    const float t = fmaxf(q.least, q.step * (q.rounds ? ceilf(r) : r));
+    if (t < best) best = t, pick = i;
+  }
+  return pick;
+}
+
 // in_dtype / out_dtype: 0 float, 1 bfloat16 (a bfloat16 input may give a 32-bit output). most_rows: the most entries a
 // group can have (the grid's height); most_entries: the most that all groups' lists can have together.
 TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, long lda, long a_group, int a_div, const void* W,
@@ -496,31 +541,10 @@ TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, lo
     const bool wide_ok = aligned && N % 4 == 0 && ldc % 4 == 0 && c_group % 4 == 0 && ((uintptr_t)C % oa) == 0 && K >= 64;
     // an entry's row lies within 32 bits of the group's first, and so does a tile's last matrix row of its first
     const bool near = ((lists ? most_entries : most_rows) / a_div + 1) * (lda * 2) < (1L << 32) && (long)K * 512 < (1L << 31);
-    if (wide_ok && near && (lists ? most_entries >= 48 : most_rows >= 64)) {
-      // From 48 list entries, or 64 rows of every group, on (8 groups of 5,632 columns and 2,048 inner ones, us, 16 x 64 straight from
-      // memory / tiles: 32 entries 43.7 / 50.8, 48 53.7 / 50.7, 64 55.5 / 50.7, 128 88 / 55; 2,048 of 2,816: 19.6 / 19.3, 32.4 / 19.5,
-      // 35.4 / 19.5, 79.5 / 19.7; without lists, 16 groups of 512 of 128: 48 rows 4.4 / 4.7, 64 8.7 / 4.8). The tile that is estimated to end first, by the microseconds a step of 64 takes with r workgroups
-      // a compute unit. With lists, entries / bm row tiles and half a tile more in every group.
-      //   128 x 192, four waves, two buffers, two a unit     1.05 r, at least 1.15
-      //   64 x 64, four waves, four buffers, two a unit      0.3 r, at least 0.33
-      //   128 x 128, eight waves, four buffers               0.58 a round
-      //   256 x 256, eight waves, two buffers                1.85 a round
-      //   128 x 128, four waves, two buffers, two a unit     0.78 r, at least 0.8
-      struct Shape { int bm, bn; float step, least; bool rounds; };
-      static const Shape shapes[5] = {{128, 192, 1.05f, 1.15f, false}, {64, 64, 0.3f, 0.33f, false}, {128, 128, 0.58f, 0.58f, true},
-                                      {256, 256, 1.85f, 1.85f, true}, {128, 128, 0.78f, 0.8f, false}};
-      int pick = 0;
-      float best = INFINITY;
-      for (int i = 0; i < 5; ++i) {
-        if (K < 256 && i != 1 && i != 4) continue;     // few steps: what counts is a tile's beginning and end (2,048 rows, 16 groups
-        const Shape& q = shapes[i];                    // of 512 of 128: 24 us in tiles of 128 x 128, 33 in 256 x 256)
-        const long tn = (N + q.bn - 1) / q.bn;
-        const float r = (lists ? (float)most_entries / q.bm + 0.5f * groups : (float)((long)groups * ((most_rows + q.bm - 1) / q.bm))) * tn / 256.f;
-        const float t = fmaxf(q.least, q.step * (q.rounds ? ceilf(r) : r));
-        if (t < best) best = t, pick = i;
-      }
+    const int pick = wide_ok && near ? tis_grouped_tile(lists ? 1 : 0, groups, most_rows, most_entries, N, K) : -1;
+    if (pick >= 0) {
       // the most row tiles there can be: the entries' own, and one that is begun in every group
-      const int bm = shapes[pick].bm, bn = shapes[pick].bn;
+      const int bm = g_shapes[pick].bm, bn = g_shapes[pick].bn;
       const long tiles = (lists ? most_entries / bm + groups : (long)groups * ((most_rows + bm - 1) / bm)) * ((N + bn - 1) / bn);
       if (tiles >= (1L << 31)) return tis_fail("grouped_linear: %ld tiles are more than a grid holds", tiles);
 #define TILES(BM, BN, WM, WN, NS, AH)                                                                                     \

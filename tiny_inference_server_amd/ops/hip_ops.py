@@ -1219,6 +1219,8 @@ class HipOps:
         lib = self.__dict__.get("_lib_" + name)
         if lib is None:
             lib = self.__dict__["_lib_" + name] = library(name)
+            if name == "experts":
+                lib.cdll.tis_experts_units(self.units)
         return lib
 
     def _f32(self, t, what, n=None):
