@@ -4,7 +4,7 @@ import random
 import numpy as np
 import pytest
 
-from tiny_inference_server_amd.ops.hip_ops import attention_items, tile_columns
+from tiny_inference_server_amd.ops.hip_ops import attention_items, mixed_key_cuts, tile_columns
 
 
 @pytest.mark.parametrize("group", [1, 3, 4, 5, 8, 16, 40, 64])
@@ -104,3 +104,14 @@ def test_decoded_tokens_get_a_whole_multiple_of_the_chips_units_in_waves_where_f
         s = splits(requests, kv_heads, keys)
         assert 1 <= s <= max(1, keys // 64) and s < 2 * 512 // (requests * kv_heads) + 2
     assert splits(64, 3, 4096, single=False) == 11     # 2,048 waves offered to rows of prompts; 12 would be the multiple
+
+
+def test_cuts_of_the_mixed_attentions_keys():
+    for resident, wanted in ((1, 288), (2, 512), (4, 512)):
+        for items in (1, 5, 96, 128, 250, 288, 289, 512, 513, 5000):
+            for longest in (1, 31, 700, 5000):
+                cuts = mixed_key_cuts(items, longest, 256, resident, 40)
+                assert 1 <= cuts <= 40 and (cuts == 1 or cuts * items <= wanted) and cuts <= (longest + 62) // 32
+                # as many as the units take, the keys give steps for and the work space has room for
+                assert cuts == 40 or cuts == (longest + 62) // 32 or (cuts + 1) * items > wanted
+    assert mixed_key_cuts(4, 5000, 256, 1, 0) == 1

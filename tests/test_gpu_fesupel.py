@@ -118,6 +118,34 @@ def test_matrix_core_attention_with_mixed_sigmoid_weights(Hq, G, kd, vd, chunk, 
         close(res[0], res[1], "bfloat16", f"attention of {seq_rows}", tol=2.5e-2)
 
 
+@pytest.mark.parametrize("heads,dim,resident", [(4, 128, 2), (16, 128, 1), (4, 64, 2), (16, 64, 1)])
+def test_cuts_of_the_keys_for_what_a_unit_holds(heads, dim, resident):
+    """The library tells how many workgroups a compute unit holds for its sizes, and the cuts that the kernel is called with fill two a unit
+    where that many fit; whatever the cuts, the same sums."""
+    ops = hip_ops("bfloat16")
+    assert min(2, ops._lazy(f"attention_mixed@{dim * 100000 + dim * 100 + -(-heads // 4)}").cdll.tis_attention_mixed_resident(heads)) == resident
+    n, ps, G = 64, 16, max(1, heads // 4)
+    g = torch.Generator().manual_seed(heads + dim)
+    plane = (0.5 * torch.randn(64, G * ps * 2 * dim, generator=g)).to(torch.bfloat16).cuda()
+    q = torch.randn(n, heads * dim, generator=g).to(torch.bfloat16).cuda()
+    bias, talk = torch.full((heads,), -5.0).cuda(), (torch.eye(heads) + 0.2 * torch.randn(heads, heads, generator=g)).cuda()
+    batch = fake_batch([(i, 600 + i, 1) for i in range(n)], list(range(n)), [torch.randperm(64, generator=g).tolist() for _ in range(n)], ps, "cuda")
+
+    def parts():
+        """The cuts, from how much of the work space a call writes."""
+        ops._workspace.fill_(float("nan"))
+        out = ops.mixed_sigmoid_attention(q, plane, batch, "g", heads, G, dim, dim, ps, 0, dim ** -0.5, 30.0, bias, talk)
+        return int((~ops._workspace.isnan()).sum()) // (n * heads * dim), out
+
+    cuts, out = parts()
+    assert cuts == (8 if resident == 2 else 4) * ops.units // 256
+    units, ops.units = ops.units, 1
+    none, whole = parts()
+    ops.units = units
+    assert none == 0
+    close(out, whole, "bfloat16", "sums of cuts", tol=1e-2)      # (one rounding to bfloat16 each, of sums in another order)
+
+
 def test_mixed_weights_are_quotients_rounded_as_a_division_rounds_them():
     """The matrix-core kernel's weights, to the last bit: with scores of zero and biases that are whole numbers on base 2 a weight is
     1 / (1 + 2^n), the power is exact, and only the reciprocal rounds. Head 0's weight is a half; every other head takes its own weight

@@ -303,6 +303,18 @@ TIS_EXPORT int tis_attention_mixed_sizes(int* kd, int* vd, int* hpw) {
   return 0;
 }
 
+static size_t lds_bytes(int H) { return ((size_t)16 * HPW * HPW + (size_t)H * TIS_WAVE * 8) * sizeof(float); }
+
+// How many workgroups of the kernel a compute unit holds at a time for H heads (1 where the runtime cannot tell).
+TIS_EXPORT int tis_attention_mixed_resident(int H) {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attention_mixed_mfma_kernel, 256, lds_bytes(H)) != hipSuccess) {
+    (void)hipGetLastError();
+    return 1;
+  }
+  return n < 1 ? 1 : n;
+}
+
 // items: n_items (first row, rows <= 16) pairs of consecutive rows of one request each, or null: every row by itself.
 // partial: [rows * n_splits * H * VD] floats where n_splits > 1. q, out: bfloat16 with 16-byte aligned rows.
 TIS_EXPORT int tis_attention_mixed_mfma(const void* q, long ldq, const void* plane, const int* block_tables, int bt_ld,
@@ -321,7 +333,7 @@ TIS_EXPORT int tis_attention_mixed_mfma(const void* q, long ldq, const void* pla
   if (ldq % 8 || ldo % 4 || ((uintptr_t)q % 16) || ((uintptr_t)out % 8))
     return tis_fail("attention_mixed_mfma: rows of q and out must be 16 and 8 bytes aligned");
   if (n_splits > 1 && (!partial || ((uintptr_t)partial % 16))) return tis_fail("attention_mixed_mfma: key splits without a workspace");
-  const size_t lds = ((size_t)16 * HPW * HPW + (size_t)H * TIS_WAVE * 8) * sizeof(float);
+  const size_t lds = lds_bytes(H);
   if (lds > 64 * 1024) return tis_fail("attention_mixed_mfma: %d heads need %zu bytes of LDS", H, lds);
   attention_mixed_mfma_kernel<<<dim3(n_items, n_splits), 256, lds, stream>>>(
       (const bf16*)q, ldq, (const bf16*)plane, block_tables, bt_ld, row_seq, positions, items, (bf16*)out, ldo, partial, n_splits,

@@ -470,6 +470,18 @@ def latent_items(seq_rows, n_heads: int, columns: int = 64):
     return np.stack((np.repeat(first, k) + r, counts), axis=1).astype(np.int32)
 
 
+def mixed_key_cuts(n_items: int, longest: int, units: int, resident: int, most: int) -> int:
+    """Over how many workgroups the keys of each of the matrix-core mixed attention's items are cut (their parts are added up), for
+    items that see up to `longest` keys on `units` compute units that hold `resident` workgroups each; at most `most`. Workgroups for two a
+    unit where a unit holds two, a little over one where it holds one. Measured, us at 1 / 2 / 3 / 4 / 5 / 8 cuts: a unit holds one (16 heads
+    of 128), 96 items 224 / 129 / 98 / 111 / 114 / 114, 128 items 225 / 132 / 141 / 143 / 143 / 143, 250 items 229 / 250 / 250 / 250 / 250 / 249; (8 heads of
+    128) 96 items 125 / 73 / 57 / 65 / 66 / 62; a unit holds two (4 heads of 128) 96 items 83 / 49 / 38 / 34 / 33 / 33, 250 items 84 / 66 / 65 / 64 / 62 / 62,
+    64 single rows 82 / 47 / 34 / 27 / 28 / 19; (8 heads of 64) 96 items 104 / 59 / 45 / 38 / 36 / 35, 250 items 104 / 70 / 69 / 69 / 65 / 66; (16 heads of 32)
+    96 items 171 / 93 / 68 / 58 / 51 / 51; a unit holds four (4 heads of 64) 96 items 64 / 37 / 28 / 24 / 23 / 19."""
+    wanted = 2 * units if resident >= 2 else 9 * units // 8
+    return int(max(1, min(-(-(longest + 31) // 32), wanted // n_items, 64, most)))
+
+
 class ChosenExperts(NamedTuple):
     """A routed feed-forward's result before the sum over a row's choices."""
     results: Optional[torch.Tensor]     # [rows * top, width] 32-bit, a line per (row, choice); None with no real expert
@@ -629,6 +641,7 @@ class HipOps:
             with torch.cuda.device(self.device):
                 self.gemm_library.tis_gemm_library_init()
         self._attn_mfma = {}               # head size -> library
+        self._mixed_resident = {}          # (key size, value size, heads) -> workgroups of the mixed attention a unit holds
         # partial results of split key ranges: one buffer of fixed size that never moves (captured graphs hold its address)
         self._workspace = torch.empty(_ATTN_WORKSPACE_FLOATS, dtype=torch.float32, device=self.device) \
             if dtype == torch.bfloat16 else None
@@ -2113,12 +2126,13 @@ class HipOps:
                 items, n_items = plan[0].reshape(-1), plan[1]
                 if items.numel() < 2 * n_items or items.dtype != torch.int32 or not items.is_contiguous():
                     raise KernelError(f"attention: a list of {items.numel()} integers for {n_items} items")
-            # few items: an item's keys are cut over several workgroups, whose parts are added up. A unit holds one workgroup: a
-            # little over one each (1,531 rows, 96 items, ms of a prefill: 3 cuts 3.34, 4 3.40, 5 3.43, 1 3.83)
-            most = max(1, self._workspace.numel() // (n * n_heads * value_dim))
-            n_splits = int(max(1, min(-(-(longest + 31) // 32), (9 * self.units // 8) // n_items, 64, most)))
             hpw = -(-n_heads // 4)
             lib = self._lazy(f"attention_mixed@{key_dim * 100000 + value_dim * 100 + hpw}")
+            # few items: an item's keys are cut over several workgroups, whose parts are added up
+            resident = self._mixed_resident.get((key_dim, value_dim, n_heads))
+            if resident is None:
+                resident = self._mixed_resident[key_dim, value_dim, n_heads] = int(lib.cdll.tis_attention_mixed_resident(n_heads))
+            n_splits = mixed_key_cuts(n_items, longest, self.units, resident, self._workspace.numel() // (n * n_heads * value_dim))
             lib.tis_attention_mixed_mfma(
                 _ptr(q), q.stride(0), _ptr(plane), _ptr(tables), tables.stride(0), _ptr(batch.row_seq), _ptr(batch.positions),
                 _ptr(items), n_items, _ptr(out), out.stride(0), _ptr(self._workspace if n_splits > 1 else None), n_splits, n,
