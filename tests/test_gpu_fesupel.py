@@ -266,6 +266,30 @@ def test_row_kernels_of_the_block(dtype, n, W):
     close(res[0][2], res[1][2], dtype, "the next norm", tol=1e-4 if dtype == "float32" else 3e-2)
 
 
+@pytest.mark.parametrize("rank", [1, 64, 65, 130, 257])
+@pytest.mark.parametrize("n,C", [(1, 33), (256, 70), (257, 64), (299, 100)])
+def test_low_rank_projections_of_several_chunks_of_the_rank(rank, n, C):
+    """The rank comes in chunks of 64, rows by eight or (from 257 on) by 32 a workgroup: ranks of one chunk, of one more and of several, whole and
+    not; the sums against 64 bits, the decays against the sums."""
+    ops = hip_ops("float32")
+    g = torch.Generator().manual_seed(rank * n + C)
+    low, w2 = torch.randn(n, rank + 3, generator=g)[:, 1:1 + rank], torch.randn(C, rank, generator=g) * rank ** -0.5
+    bias, rate = torch.randn(C, generator=g), torch.rand(C, generator=g) * 4
+    on = lambda t: t.cuda()
+    wide = torch.full((n, rank + 3), float("nan"))
+    wide[:, 1:1 + rank] = low
+    dev = on(wide)[:, 1:1 + rank]           # rows that begin beside a number that is none
+    want = low.double() @ w2.double().T
+    # `rank` products and as many additions, each within half a unit of the sum of magnitudes
+    bound = (rank + 1) * 2.0 ** -24 * (low.double().abs() @ w2.double().abs().T)
+    got = ops.lowrank_act(dev, on(w2), None, "none").cpu()
+    assert ((got.double() - want).abs() <= bound).all()
+    z = want + bias.double()
+    close(ops.lowrank_act(dev, on(w2), on(bias), "exp_softplus", rate=on(rate), group=1),
+          torch.exp(-rate.double() * torch.nn.functional.softplus(z)), "float32", "decays")
+    close(ops.lowrank_decay(dev, on(w2), on(bias), 7.0), torch.exp(torch.nn.functional.logsigmoid(z) / 7.0), "float32", "decays of a sigmoid")
+
+
 @pytest.mark.parametrize("n,N,top,groups", [(37, 8, 2, (4, 2)), (5, 12, 3, (3, 1)), (200, 16, 3, (2, 1)), (9, 6, 6, None), (64, 64, 4, (16, 3)),
                                             (33, 10, 1, (10, 1)), (20, 130, 5, (13, 2))])
 def test_choice_in_groups(n, N, top, groups):
