@@ -1013,6 +1013,30 @@ def test_plain_product_of_few_rows_or_columns(ops_for, M, N, K, dtype):
     assert torch.equal(product(many, None, len(many), len(wide), wide)[-M:, :N], product(x, None, M))
 
 
+def test_when_a_plain_product_takes_small_tiles(ops_for):
+    """By the tiles of 64 x 64 there would be, fewer where rows are read value by value (bfloat16) than 16 bytes at a time; and both
+    tilings give the same bits on either side of the line."""
+    from tiny_inference_server_amd.ops.hip_ops import _ptr
+    few = ops_for(torch.float32).gemm_plain.cdll.tis_gemm_plain_few
+    for wide, lines in ((1, {64: 96, 124: 96, 128: 128, 508: 128, 512: 512, 4096: 512}), (0, {65: 96, 511: 96, 512: 128, 4097: 128})):
+        for K, most in lines.items():
+            for M, N in ((17, 64), (64, 64 * most - 64), (64, 64 * most), (65, 32 * most - 64), (65, 32 * most), (2048, 2 * most), (16, 48000), (1, 64)):
+                tiles = -(-M // 64) * -(-N // 64)
+                assert bool(few(wide, M, N, K)) == (tiles < most or bool(wide and M <= 16 and K >= 128)), (wide, M, N, K)
+    ops = ops_for(torch.float32)
+    for dtype, K, cols in ((torch.bfloat16, 65, 95 * 64), (torch.bfloat16, 513, 127 * 64), (torch.float32, 64, 95 * 64), (torch.float32, 132, 127 * 64)):
+        x, w = rnd((33, K), dtype, 621).cuda(), rnd((cols + 64, K), dtype, 622).cuda()
+
+        def product(n):
+            out = torch.empty(33, n, device="cuda")
+            ops.gemm_plain.tis_gemm_plain(0 if dtype == torch.float32 else 1, 0, _ptr(x), K, _ptr(w), K, None, 0, _ptr(out), n, 33, n, K, ops._stream())
+            return out
+
+        wide = 1 if dtype == torch.float32 else 0
+        assert few(wide, 33, cols, K) and not few(wide, 33, cols + 64, K)
+        assert torch.equal(product(cols), product(cols + 64)[:, :cols])
+
+
 @pytest.mark.parametrize("K", [8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 520])
 @pytest.mark.parametrize("M,N", [(129, 60), (1900, 2044), (1301, 3508), (2047, 8188)])
 def test_tiled_product_of_few_steps_of_each_tile(ops_for, M, N, K):

@@ -149,16 +149,25 @@ __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI*
   if (live) C[m * ldc + n] = from_f<TO>(R ? acc + res : acc);
 }
 
+// Whether a product of M rows takes the tiles of 16 x 16; wide: its rows are read 16 bytes at a time. What counts is how many tiles of 64 x 64
+// there would be: few of them are a chain of K / 16 trips to memory on a chip that is mostly idle, many fill the chip and read each row a
+// quarter as often. us, tiles of 64 x 64 / of 16 x 16, read wide (float): K = 1536, 384 tiles 248 / 187, 512 tiles 243 / 252, 768 tiles
+// 297 / 371; K = 176, 32 tiles 20.2 / 4.9; K = 64, 256 tiles 11.7 / 19.9, 120 tiles 10.8 / 12.3, 64 tiles 10.6 / 7.8. Up to 16 rows most of
+// a 64 x 64 tile's rows are not there: 16 rows of 48,000 columns (750 tiles) K = 1536 260 / 111, K = 176 31 / 23, but K = 64 15.0 / 17.3.
+// Read value by value (bfloat16, rows that do not start on 16 bytes) a small tile costs more: K = 1537, 120 tiles 172 / 149, 128 tiles of 2,048 x 200
+// 178 / 223, 320 tiles 214 / 369, 384 tiles 234 / 550; K = 65, 64 tiles 11.0 / 10.6, 120 tiles 11.1 / 19.3; 16 rows of 48,000 columns
+// K = 1537 272 / 348, K = 4097 845 / 1,266.
+TIS_EXPORT int tis_gemm_plain_few(int wide, int M, int N, int K) {
+  const long tiles = (long)((N + GP_BN - 1) / GP_BN) * ((M + GP_BM - 1) / GP_BM);
+  if (wide) return (M <= 16 && K >= 128) || tiles < (K >= 512 ? 512 : K >= 128 ? 128 : 96);
+  return tiles < (K >= 512 ? 128 : 96);
+}
+
 template <typename TI, typename TO>
 static void launch_plain(const void* A, long lda, const void* W, long ldw, const void* R, long ldr, void* C, long ldc, int M,
                          int N, int K, hipStream_t stream) {
-  const long tiles = (long)((N + GP_BN - 1) / GP_BN) * ((M + GP_BM - 1) / GP_BM);
-  // Up to 16 rows, and wherever 64 x 64 tiles would be fewer than two for every compute unit (a chain of K / 16 trips to
-  // memory on a chip that is mostly idle); below 512 columns of K that chain is short, and half a tile a unit is the line.
-  // us, tiles of 64 x 64 / of 16 x 16: 384 tiles of K = 1536 248 / 187, 512 tiles 243 / 252, 768 tiles 297 / 371; K = 64:
-  // 256 tiles 11.7 / 19.9; K = 176: 32 tiles 20.2 / 4.9.
-  if (M <= 16 || tiles < (K >= 512 ? 512 : 128)) {
-    const bool vec = sizeof(TI) == 4 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+  const bool vec = sizeof(TI) == 4 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+  if (tis_gemm_plain_few(vec, M, N, K)) {
     const dim3 grid((N + GS_BN - 1) / GS_BN, (M + GS_BM - 1) / GS_BM);
     const auto kernel = vec ? gemm_plain_few_kernel<true, TI, TO> : gemm_plain_few_kernel<false, TI, TO>;
     kernel<<<grid, GS_BM * GS_BN, 0, stream>>>((const TI*)A, lda, (const TI*)W, ldw, (const TO*)R, ldr, (TO*)C, ldc, M, N, K);

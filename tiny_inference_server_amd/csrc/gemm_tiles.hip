@@ -1,7 +1,7 @@
 // C[M,N] = X[M,K] . W[N,K]^T (+ R[M,N]) in bfloat16 for many rows at widths where the library's product is not used:
 // a product tiled in both directions on v_mfma_f32_32x32x16_bf16 (gfx950), operands through LDS by direct loads.
 // (The few-row kernel takes such a product in panels of 32 rows, each of which streams all of W again: 0.25 to 0.3
-// PFLOP/s at 2,048 rows. This kernel reaches 0.45 to 0.95 on the same shapes; the library's kernels, where they may be
+// PFLOP/s at 2,048 rows. This kernel reaches 0.75 to 1.0 on the same shapes; the library's kernels, where they may be
 // used, 0.5 to 1.3.) The reference's engine uses a library product here (x @ W, main_models_new.py:19-20).
 //
 // tile_loop.h holds the loop. A row's sums run over K in the same order whatever M is: its result does not depend on the other rows.

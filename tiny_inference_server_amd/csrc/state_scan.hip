@@ -11,9 +11,9 @@
 // zeros beyond the head's channels, so a thread reads its share in 16-byte pieces), from the request's state slot before the first token to
 // the slot after the last. Tokens are taken in chunks: a chunk's q, k, v and gates go into LDS, the 16 threads of a
 // column leave a partial o per token there, and one pass adds them up. Each state element sees its tokens strictly in
-// order with nothing else mixed in, so the result of a token does not depend on how a prompt was cut into steps, on the
-// chunk size or on what else is in the batch, bit for bit. State, gates and sums are 32-bit. Kind 1 keeps n and m once
-// per block of value channels (every block needs them, none may read what another has already advanced).
+// order with nothing else mixed in, so among steps that are walked so (no portion of two segments and more in them) the result of a token
+// does not depend on how a prompt was cut into steps, on the chunk size or on what else is in the batch, bit for bit. State, gates and sums
+// are 32-bit. Kind 1 keeps n and m once per block of value channels (every block needs them, none may read what another has already advanced).
 //
 // Long portions of prompts are cut into segments of `seg_len` tokens that run side by side (`segments` > 0): up to 128 key
 // channels and 64 tokens by products of matrices (see there); beyond that the same kernel walks every segment from an empty state and leaves the segment's own state, its outputs as if nothing had
@@ -24,7 +24,8 @@
 //   kind 0: o_t += (q_t * decay product to t)^T S_start
 //   kind 1: m_t = max(m'_t, F_t + m_start); numerator and n . q are sums of the segment's own part scaled by
 //           exp(m'_t - m_t) and the start's part scaled by exp(F_t + m_start - m_t); o_t as above.
-// Everything is still 32-bit; only the order of additions differs from the token-by-token walk.
+// Everything is still 32-bit; only the order of additions differs from the token-by-token walk, for every request of such a step, the
+// ones of a single token too: a token's last bits depend on whether a long portion was in its step.
 #include "common.h"
 #include <algorithm>
 #include <type_traits>
@@ -368,9 +369,11 @@ __global__ __launch_bounds__(SC_THREADS) void segment_outputs_kernel(const float
 // are numbered through over the requests of the step, so a step of one long and many short ones needs no more room than its rows.
 // MI355X, 8 heads of 128 x 256, us row by row in segments / by products:
 // 2,048 rows 233 / 81 (kind 1: 250 / 86), two requests of 1,216 and 584 rows 229 / 70 (250 / 71), 512 rows 124 / 39, 128 rows
-// 110 / 30, eight requests of 512 rows 417 / 136. Of the 70 the rows' kernel takes 25 (LDS, pair by pair; kind 1: 15), the walk 24 (a chain of
-// one segment after another, 1 us each) and the results 25 (memory: the states at the starts twice over). Off from 64 bits by
-// 1.4e-7 / 1.2e-7 (kind 0; sums of products run in four accumulators each, which keeps their chains as short as the row by
+// 110 / 30, eight requests of 512 rows 417 / 136. Inside a prompt step of 1,200 and 600 rows, traced kernel by kernel, the rows' kernel takes 28.9
+// (LDS, pair by pair; kind 1: 16.6), the walk 26.0 (30.1; a chain of one segment after another, 1.4 us each) and the results 26.9 (32.1; memory:
+// the states at the starts twice over). The workspace is 3,360 bytes a row and head of these sizes (the row by row segments' was 2,570 for
+// one request, and more than this for requests of unequal lengths). Off from 64 bits by 1.4e-7 (row by row) and 1.2e-7 (kind 0; sums
+// of products run in four accumulators each, which keeps their chains as short as the row by
 // row kernel's), kind 1 by 0.5e-6 to 3e-6 both ways (its division).
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 static constexpr int SP_ROWS = 64;               // rows a segment can have: four tiles of 16
