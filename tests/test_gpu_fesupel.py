@@ -266,11 +266,12 @@ def test_row_kernels_of_the_block(dtype, n, W):
     close(res[0][2], res[1][2], dtype, "the next norm", tol=1e-4 if dtype == "float32" else 3e-2)
 
 
-@pytest.mark.parametrize("rank", [1, 64, 65, 130, 257])
-@pytest.mark.parametrize("n,C", [(1, 33), (256, 70), (257, 64), (299, 100)])
+@pytest.mark.parametrize("rank", [1, 15, 16, 17, 32, 33, 64, 65, 130, 257])
+@pytest.mark.parametrize("n,C", [(1, 33), (257, 64), (299, 100), (513, 514), (90, 6000)])
 def test_low_rank_projections_of_several_chunks_of_the_rank(rank, n, C):
-    """The rank comes in chunks of 64, rows by eight or (from 257 on) by 32 a workgroup: ranks of one chunk, of one more and of several, whole and
-    not; the sums against 64 bits, the decays against the sums."""
+    """The rank comes in chunks of 16, 32 or 64, rows by eight or (many rows times channels: the last two sizes) by 32 a workgroup: ranks of
+    one chunk, of one more and of several, whole and not; the sums against 64 bits, the decays against the sums; and a row's bits do not
+    depend on how many rows there are."""
     ops = hip_ops("float32")
     g = torch.Generator().manual_seed(rank * n + C)
     low, w2 = torch.randn(n, rank + 3, generator=g)[:, 1:1 + rank], torch.randn(C, rank, generator=g) * rank ** -0.5
@@ -284,6 +285,7 @@ def test_low_rank_projections_of_several_chunks_of_the_rank(rank, n, C):
     bound = (rank + 1) * 2.0 ** -24 * (low.double().abs() @ w2.double().abs().T)
     got = ops.lowrank_act(dev, on(w2), None, "none").cpu()
     assert ((got.double() - want).abs() <= bound).all()
+    assert torch.equal(ops.lowrank_act(dev[n // 2:n // 2 + 1], on(w2), None, "none").cpu(), got[n // 2:n // 2 + 1])
     z = want + bias.double()
     close(ops.lowrank_act(dev, on(w2), on(bias), "exp_softplus", rate=on(rate), group=1),
           torch.exp(-rate.double() * torch.nn.functional.softplus(z)), "float32", "decays")

@@ -802,12 +802,12 @@ TIS_EXPORT int tis_softcap(float* z, long ldz, float cap, int rows, int W, hipSt
 // out[r][c] = act(z) with z = sum_k low[r][k] * w2[c][k] + bias[c] (bias may be null): the second half of a low-rank
 // projection, in 32-bit. kind 0: sigmoid(z)^(1/tau); 1: exp(-rate[c / group] * softplus(z)), a decay whose rate is one
 // number per run of `group` channels; 2: z itself.
-// A workgroup takes 32 channels and 8 RT rows, a thread one channel of RT of them, and both factors come through LDS in chunks of 64 of
+// A workgroup takes 32 channels and 8 RT rows, a thread one channel of RT of them, and both factors come through LDS in chunks of LR_K of
 // the rank, read in whole runs (a thread that walked its channel's line of w2 by itself touched a line of memory per lane and
 // term, and 5 rows of 512 channels were two workgroups). k in rising order for every row, whatever RT. us before / now, rank 64: 5 rows
 // x 1,024 7.0 / 4.3, 64 x 1,024 8.5 / 4.4, 1,531 x 1,024 15.4 / 12.4, 1,531 x 2,048 25.0 / 22.4.
-static constexpr int LR_COLS = 32, LR_BY = S32_THREADS / LR_COLS, LR_K = 64;
-template <int RT>
+static constexpr int LR_COLS = 32, LR_BY = S32_THREADS / LR_COLS;
+template <int RT, int LR_K>
 __global__ __launch_bounds__(S32_THREADS) void lowrank_act_kernel(const float* __restrict__ low, long ldl, int rank,
                                                                    const float* __restrict__ w2,
                                                                    const float* __restrict__ bias, int kind, float tau,
@@ -857,16 +857,25 @@ __global__ __launch_bounds__(S32_THREADS) void lowrank_act_kernel(const float* _
   }
 }
 
-// (eight rows a workgroup up to 256 rows, for the shortest chain: 100 rows x 1,024 4.9 us, 7.6 with 32; 32 beyond, which read w2 a
-// quarter as often)
+// Eight rows a workgroup while the chip holds all of them at a time, eight a unit of up to 64 terms of the rank (four where a rank of up to
+// 32 leaves little to do but the results): the shortest chain. 32 rows beyond, which read w2 a quarter as often. And a chunk of the rank is no longer than a
+// short rank is, or copying zeros is most of the work. us, eight rows / 32: rank 64, 256 rows x 1,024 6.3 / 8.1, 256 x 2,048 8.5 / 9.0, 257 x 2,048
+// 10.9 / 8.9, 2,048 x 2,048 52 / 31; 2,048 x 32 4.6 / 7.7; rank 16, 256 x 1,024 4.6 / 4.7, 1,000 x 512 7.1 / 5.5, 2,048 x 4,096 71 / 34 (43
+// in chunks of 64; a channel's line of w2 walked by one thread: 31); 1 row x 1,024 3.3 (4.1 in chunks of 64).
 static void launch_lowrank(const float* low, long ldl, int rank, const float* w2, const float* bias, int kind, float tau,
                            const float* rate, int group, float* out, int rows, int C, hipStream_t stream) {
   const int col_blocks = (C + LR_COLS - 1) / LR_COLS;
-  const bool few = rows <= 256;
-  const int per = few ? LR_BY : 4 * LR_BY;
-  const long blocks = ((long)rows + per - 1) / per * col_blocks;
-  if (few) lowrank_act_kernel<1><<<blocks, S32_THREADS, 0, stream>>>(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, col_blocks);
-  else lowrank_act_kernel<4><<<blocks, S32_THREADS, 0, stream>>>(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, col_blocks);
+  const long small = ((long)rows + LR_BY - 1) / LR_BY * col_blocks;
+  const bool few = small <= (rank > 32 ? 2048 : 1024);
+  const long blocks = few ? small : ((long)rows + 4 * LR_BY - 1) / (4 * LR_BY) * col_blocks;
+#define LOWRANK(RT, K) \
+  lowrank_act_kernel<RT, K><<<blocks, S32_THREADS, 0, stream>>>(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, col_blocks)
+#define LOWRANK_BY_ROWS(K) { if (few) LOWRANK(1, K); else LOWRANK(4, K); }
+  if (rank <= 16) LOWRANK_BY_ROWS(16)
+  else if (rank <= 32) LOWRANK_BY_ROWS(32)
+  else LOWRANK_BY_ROWS(64)
+#undef LOWRANK_BY_ROWS
+#undef LOWRANK
 }
 
 // out[r] = (1 / n) * sum_i y_i[r] / sqrt(mean(y_i[r]^2) + eps) * gain_i: the mean of one or two RMS-normed rows, 32-bit.
