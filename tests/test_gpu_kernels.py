@@ -1115,10 +1115,11 @@ def test_grouped_product_in_tiles_numbered_through(ops_for, groups, line, N, K, 
                 torch.testing.assert_close(out[perm[e].long()].double(), gate * torch.sigmoid(1.702 * gate) * (up + 1.0), rtol=8e-3, atol=2e-3)
 
 
-def grouped_tile(ops, lists, groups, most_rows, most_entries, N, K):
-    """The tile a grouped product takes: 0 to 4 for 128 x 192, 64 x 64, 128 x 128 on eight waves, 256 x 256, 128 x 128 on four; -1: none."""
+def grouped_tile(ops, lists, groups, most_rows, most_entries, N, K, gate=0):
+    """The tile a grouped product takes: 0 to 5 for 128 x 192, 64 x 64, 128 x 128 on eight waves, 256 x 256, 128 x 128 on four, 64 x 64 with
+    two buffers; -1: none."""
     from ctypes import c_long
-    return ops._lazy("experts").cdll.tis_grouped_tile(lists, groups, most_rows, c_long(most_entries), N, K)
+    return ops._lazy("experts").cdll.tis_grouped_tile(lists, groups, most_rows, c_long(most_entries), N, K, gate)
 
 
 @pytest.mark.parametrize("tile,groups,line,N,K", [(0, 8, 2048, 2044, 328), (0, 8, 2048, 2048, 256), (1, 130, 1040, 132, 200), (1, 12, 90, 1036, 1032),
@@ -1176,6 +1177,30 @@ def test_when_a_grouped_product_takes_tiles(ops_for):
                 want = n > 16 and n * top >= max(48, per * groups)
                 assert tiles(1, groups, n, n * top, 2048, K) == want, (groups, top, K, n)
     assert [tiles(0, 16, n, 16 * n, 512, 128) for n in (48, 63, 64, 2048)] == [False, False, True, True]
+    # a product per head of few steps: the small tile with two buffers, but thousands of gated ones of narrow heads
+    small = lambda n, N, K, gate: grouped_tile(ops, 0, 64, n, 64 * n, N, K, gate)
+    assert [small(n, 128, 64, g) for n in (64, 1024, 1025) for g in (0, 1)] == [5, 5, 5, 5, 5, 1]
+    assert [small(4096, N, K, 1) for N, K in ((132, 64), (128, 248), (64, 200))] == [5, 1, 1] and small(4096, 128, 256, 0) != 5
+
+
+@pytest.mark.parametrize("heads,N,K,rows", [(64, 128, 64, 1025), (64, 128, 128, 1000), (3, 60, 72, 64), (16, 512, 128, 300), (5, 68, 248, 129), (2, 4, 64, 191)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_products_per_head_of_few_steps(ops_for, heads, N, K, rows, gated):
+    """Few steps of K, whole and ragged; rows and columns that end inside a tile; with a gate per result and without; columns that belong to no head stay."""
+    ops = ops_for(torch.bfloat16)
+    x, w = rnd((rows, heads * K), torch.bfloat16, 821).cuda(), rnd((heads, N, K), torch.bfloat16, 822, K ** -0.5).cuda()
+    gate = rnd((rows, heads * N), torch.float32, 823).cuda() if gated else None
+    out = torch.full((rows, 4 + heads * (N + 4)), 7.5, device="cuda")
+    ops.heads_linear(x, w, out, N + 4, 4, gate=gate)
+    got = out[:, 4:].view(rows, heads, N + 4)
+    assert (got[:, :, N:] == 7.5).all() and (out[:, :4] == 7.5).all()
+    for h in range(heads):
+        a = x[:, h * K:(h + 1) * K].double()
+        want, bound = a @ w[h].double().T, (K + 2) * 2.0 ** -24 * (a.abs() @ w[h].double().abs().T)
+        if gated:       # the gate's sigmoid is off by a few units of the last place
+            z = torch.sigmoid(gate[:, h * N:(h + 1) * N].double())
+            want, bound = want * z, bound * z + 2.0 ** -21 * (want * z).abs()
+        assert ((got[:, h, :N].double() - want).abs() <= bound).all(), h
 
 
 @pytest.mark.parametrize("M", [1, 7, 8])

@@ -484,9 +484,10 @@ TIS_EXPORT void tis_experts_units(int n) { if (n > 0) g_units = n; }
 //   128 x 128, eight waves, four buffers               0.58 a round
 //   256 x 256, eight waves, two buffers                1.85 a round
 //   128 x 128, four waves, two buffers, two a unit     0.78 r, at least 0.8
+//   64 x 64, four waves, two buffers, five a unit      (not by this estimate: for products of few steps)
 struct GroupedShape { int bm, bn; float step, least; bool rounds; };
-static const GroupedShape g_shapes[5] = {{128, 192, 1.05f, 1.15f, false}, {64, 64, 0.3f, 0.33f, false}, {128, 128, 0.58f, 0.58f, true},
-                                         {256, 256, 1.85f, 1.85f, true}, {128, 128, 0.78f, 0.8f, false}};
+static const GroupedShape g_shapes[6] = {{128, 192, 1.05f, 1.15f, false}, {64, 64, 0.3f, 0.33f, false}, {128, 128, 0.58f, 0.58f, true},
+                                         {256, 256, 1.85f, 1.85f, true}, {128, 128, 0.78f, 0.8f, false}, {64, 64, 0.f, 0.f, false}};
 
 // The tile that a grouped product of bfloat16 rows that lie as it needs them takes, an index into g_shapes; -1: the products straight from memory.
 // lists: most_rows is the most entries a group can have, most_entries the most that all groups have together.
@@ -502,13 +503,20 @@ static const GroupedShape g_shapes[5] = {{128, 192, 1.05f, 1.15f, false}, {64, 6
 // part of the chip idle. Over 805 sizes of 2 to 128 groups and 1 to 64 entries a group, this rule takes 1.04 times the better way's time, and
 // on 58 of them more than the way straight from memory: most by 1 or 2 us of 8, 64 groups of 2,816 of 1,024 at 4 to 6 entries by an eighth.
 // A line at 48 entries alone takes 1.04 times too, but more than the way straight from memory on 151, up to 1.5 times.)
-TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_entries, int N, int K) {
+// A product per head of few steps (K below 256) is bound by its results' way to memory and by the beginnings and ends of its tiles: the small tile
+// of which most fit a unit. us, the tiles before the loop / as the estimate picks them / so: 4,096 rows of 64 heads of 128 x 128 46 / 59 / 42,
+// 1,531 rows of 16 of 512 x 128 21 / 20 / 17, 300 of 16 of 512 x 128 7.3 / 8.5 / 6.3, 1,531 of 64 of 64 x 64 9.3 / 13.1 / 10.5. With a gate and heads no
+// wider than 128, thousands of such tiles at a time read and write short pieces of rows that lie far apart, and fewer of them are faster: 4,096 rows of 64
+// heads of 128 x 128 159 / 177 / 229, with four buffers (two a unit) 130; 1,531 rows 45 / 55 / 58, 49.
+TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_entries, int N, int K, int gate) {
   if (lists ? most_rows <= 16 || most_entries < 48 || most_entries < (K < 1024 ? 12L : 4L) * groups : most_rows < 64) return -1;
+  if (!lists && K < 256)
+    return gate && N <= 128 && (long)groups * ((most_rows + 63) / 64) * ((N + 63) / 64) > 2048 ? 1 : 5;
   int pick = 0;
   float best = INFINITY;
   for (int i = 0; i < 5; ++i) {
-    if (K < 256 && i != 1 && i != 4) continue;     // few steps: what counts is a tile's beginning and end (2,048 rows, 16 groups
-    const GroupedShape& q = g_shapes[i];           // of 512 of 128: 24 us in tiles of 128 x 128, 33 in 256 x 256)
+    if (K < 256 && i != 1 && i != 4) continue;     // few steps: what counts is a tile's beginning and end
+    const GroupedShape& q = g_shapes[i];
     const long tn = (N + q.bn - 1) / q.bn;
     // (with lists, entries / bm row tiles and half a tile more in every group)
     const float r = (lists ? (float)most_entries / q.bm + 0.5f * groups : (float)((long)groups * ((most_rows + q.bm - 1) / q.bm))) * tn / g_units;
@@ -541,7 +549,7 @@ TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, lo
     const bool wide_ok = aligned && N % 4 == 0 && ldc % 4 == 0 && c_group % 4 == 0 && ((uintptr_t)C % oa) == 0 && K >= 64;
     // an entry's row lies within 32 bits of the group's first, and so does a tile's last matrix row of its first
     const bool near = ((lists ? most_entries : most_rows) / a_div + 1) * (lda * 2) < (1L << 32) && (long)K * 512 < (1L << 31);
-    const int pick = wide_ok && near ? tis_grouped_tile(lists ? 1 : 0, groups, most_rows, most_entries, N, K) : -1;
+    const int pick = wide_ok && near ? tis_grouped_tile(lists ? 1 : 0, groups, most_rows, most_entries, N, K, gate ? 1 : 0) : -1;
     if (pick >= 0) {
       // the most row tiles there can be: the entries' own, and one that is begun in every group
       const int bm = g_shapes[pick].bm, bn = g_shapes[pick].bn;
@@ -558,7 +566,8 @@ TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, lo
       else if (pick == 1) TILES(64, 64, 2, 2, 4, 2)
       else if (pick == 2) TILES(128, 128, 2, 4, 4, 2)
       else if (pick == 3) TILES(256, 256, 2, 4, 2, 1)
-      else TILES(128, 128, 2, 2, 2, 1)
+      else if (pick == 4) TILES(128, 128, 2, 2, 2, 1)
+      else TILES(64, 64, 2, 2, 2, 1)
 #undef TILES
     } else if (aligned && most_rows >= 64 * (lists ? groups : 1)) {
       // 64 entries x 128 columns a workgroup, operands straight from memory
