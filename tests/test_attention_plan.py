@@ -4,7 +4,7 @@ import random
 import numpy as np
 import pytest
 
-from tiny_inference_server_amd.ops.hip_ops import attention_items, mixed_key_cuts, tile_columns
+from tiny_inference_server_amd.ops.hip_ops import attention_items, even_keys, latent_items, mixed_key_cuts, tile_columns
 
 
 @pytest.mark.parametrize("group", [1, 3, 4, 5, 8, 16, 40, 64])
@@ -107,11 +107,34 @@ def test_decoded_tokens_get_a_whole_multiple_of_the_chips_units_in_waves_where_f
 
 
 def test_cuts_of_the_mixed_attentions_keys():
-    for resident, wanted in ((1, 288), (2, 512), (4, 512)):
-        for items in (1, 5, 96, 128, 250, 288, 289, 512, 513, 5000):
+    for resident, even, wanted in ((1, False, 288), (1, True, 256), (2, False, 512), (2, True, 512), (4, True, 512)):
+        for items in (1, 5, 32, 96, 128, 250, 257, 288, 289, 512, 513, 5000):
             for longest in (1, 31, 700, 5000):
-                cuts = mixed_key_cuts(items, longest, 256, resident, 40)
+                cuts = mixed_key_cuts(items, longest, 256, resident, 40, even)
                 assert 1 <= cuts <= 40 and (cuts == 1 or cuts * items <= wanted) and cuts <= (longest + 62) // 32
                 # as many as the units take, the keys give steps for and the work space has room for
                 assert cuts == 40 or cuts == (longest + 62) // 32 or (cuts + 1) * items > wanted
     assert mixed_key_cuts(4, 5000, 256, 1, 0) == 1
+
+
+@pytest.mark.parametrize("chunk", [0, 1, 16, 100, 1024])
+def test_whether_items_see_as_many_keys(chunk):
+    """Against every item's own rows, where the mean is not right at the line; a request's rows stand for its items."""
+    rng = random.Random(chunk)
+    assert even_keys([(0, 1999, 1)] * 5, 0) and even_keys([(0, 1500, 500)], 0) and not even_keys([(0, 0, 1531)], 0)
+    assert even_keys([], chunk) and not even_keys([(0, 0, 2048)], 1024) and even_keys([(0, 700, 300)], 1024)
+    for _ in range(200):
+        seq_rows, row = [], 0
+        for _ in range(rng.randint(1, 5)):
+            n = rng.choice([0, 1, 16, 160, 320, 640, 2048])
+            seq_rows.append((row, rng.choice([0, 3, 100, 700, 2000]), n))
+            row += n
+        position = {first + i: p0 + i for first, p0, n in seq_rows for i in range(n)}
+        seen = {r: (p % chunk if chunk else p) + 1 for r, p in position.items()}
+        items = latent_items(seq_rows, 1, 16)
+        if not len(items):
+            continue
+        means = [np.mean([seen[r] for r in range(f, f + c)]) for f, c in items.tolist()]
+        share = np.mean(means) / max(chunk if any(chunk and p0 // chunk != (p0 + n - 1) // chunk for _, p0, n in seq_rows if n) else 0, max(seen.values()))
+        if abs(share - 0.7) > 0.01:
+            assert even_keys(seq_rows, chunk) == (share >= 0.7), (seq_rows, share)

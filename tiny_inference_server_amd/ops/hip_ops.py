@@ -470,15 +470,37 @@ def latent_items(seq_rows, n_heads: int, columns: int = 64):
     return np.stack((np.repeat(first, k) + r, counts), axis=1).astype(np.int32)
 
 
-def mixed_key_cuts(n_items: int, longest: int, units: int, resident: int, most: int) -> int:
+def even_keys(seq_rows, chunk: int) -> bool:
+    """Whether the matrix-core mixed attention's items (up to 16 rows of one request) see about as many keys each: their mean at least 0.7
+    of the most. A prompt from its start does not (0.5), a portion far behind it or single rows do. chunk: as for the attention."""
+    items = total = most = 0
+    for _, p0, n in seq_rows:
+        if n <= 0:
+            continue
+        if chunk > 0 and p0 // chunk != (p0 + n - 1) // chunk:      # over a chunk's edge: up to the edge, whole chunks, what is left
+            tail = (p0 + n) % chunk
+            parts = [(p0 % chunk, chunk - p0 % chunk), (0, (p0 + n) // chunk * chunk - (p0 // chunk + 1) * chunk), (0, tail)]
+            keys = sum(m * (a + (min(m, chunk) + 1) / 2) for a, m in parts) / n
+            end = chunk
+        else:
+            a = p0 % chunk if chunk > 0 else p0
+            keys, end = a + (n + 1) / 2, a + n
+        w = -(-n // 16)
+        items, total, most = items + w, total + w * keys, max(most, end)
+    return total >= 0.7 * items * most
+
+
+def mixed_key_cuts(n_items: int, longest: int, units: int, resident: int, most: int, even: bool = False) -> int:
     """Over how many workgroups the keys of each of the matrix-core mixed attention's items are cut (their parts are added up), for
     items that see up to `longest` keys on `units` compute units that hold `resident` workgroups each; at most `most`. Workgroups for two a
-    unit where a unit holds two, a little over one where it holds one. Measured, us at 1 / 2 / 3 / 4 / 5 / 8 cuts: a unit holds one (16 heads
-    of 128), 96 items 224 / 129 / 98 / 111 / 114 / 114, 128 items 225 / 132 / 141 / 143 / 143 / 143, 250 items 229 / 250 / 250 / 250 / 250 / 249; (8 heads of
-    128) 96 items 125 / 73 / 57 / 65 / 66 / 62; a unit holds two (4 heads of 128) 96 items 83 / 49 / 38 / 34 / 33 / 33, 250 items 84 / 66 / 65 / 64 / 62 / 62,
-    64 single rows 82 / 47 / 34 / 27 / 28 / 19; (8 heads of 64) 96 items 104 / 59 / 45 / 38 / 36 / 35, 250 items 104 / 70 / 69 / 69 / 65 / 66; (16 heads of 32)
-    96 items 171 / 93 / 68 / 58 / 51 / 51; a unit holds four (4 heads of 64) 96 items 64 / 37 / 28 / 24 / 23 / 19."""
-    wanted = 2 * units if resident >= 2 else 9 * units // 8
+    unit where a unit holds two. Where it holds one, a little over one for items with chains of all lengths (a prompt from its start), and no more than
+    one where they are `even`, which would all run twice for the few that are left over. Measured, us: a unit holds one, uneven, at 1 / 2 / 3 / 4 / 5 / 8
+    cuts (16 heads of 128) 96 items 224 / 129 / 98 / 111 / 114 / 114, 128 items 225 / 132 / 141 / 143 / 143 / 143, 250 items 229 / 250 / 250 / 250 / 250 / 249;
+    even, at 8 / 9 / 12 / 16 cuts 32 single rows of 2,000 keys 65 / 108 / 82 / 69, 500 rows behind 1,500 others (32 items) 73 / 119 / 97 / 84, (8 heads of
+    128) the rows 39 / 64 / 49 / 41, the portion 46 / 68 / 57 / 50. A unit holds two (4 heads of 128), at 1 / 2 / 3 / 4 / 5 / 8, 96 items 83 / 49 / 38 / 34 / 33 / 33,
+    250 items 84 / 66 / 65 / 64 / 62 / 62, 64 single rows 82 / 47 / 34 / 27 / 28 / 19; (8 heads of 64) 96 items 104 / 59 / 45 / 38 / 36 / 35, 250 items
+    104 / 70 / 69 / 69 / 65 / 66; (16 heads of 32) 96 items 171 / 93 / 68 / 58 / 51 / 51; it holds four (4 heads of 64) 96 items 64 / 37 / 28 / 24 / 23 / 19."""
+    wanted = 2 * units if resident >= 2 else units if even else 9 * units // 8
     return int(max(1, min(-(-(longest + 31) // 32), wanted // n_items, 64, most)))
 
 
@@ -2132,7 +2154,8 @@ class HipOps:
             resident = self._mixed_resident.get((key_dim, value_dim, n_heads))
             if resident is None:
                 resident = self._mixed_resident[key_dim, value_dim, n_heads] = int(lib.cdll.tis_attention_mixed_resident(n_heads))
-            n_splits = mixed_key_cuts(n_items, longest, self.units, resident, self._workspace.numel() // (n * n_heads * value_dim))
+            n_splits = mixed_key_cuts(n_items, longest, self.units, resident, self._workspace.numel() // (n * n_heads * value_dim),
+                                      even=items is None or (resident < 2 and even_keys(batch.seq_rows, int(chunk))))
             lib.tis_attention_mixed_mfma(
                 _ptr(q), q.stride(0), _ptr(plane), _ptr(tables), tables.stride(0), _ptr(batch.row_seq), _ptr(batch.positions),
                 _ptr(items), n_items, _ptr(out), out.stride(0), _ptr(self._workspace if n_splits > 1 else None), n_splits, n,
