@@ -238,6 +238,40 @@ def test_segments_of_rows_at_odd_distances(kind, distance):
     close(res[0][1], res[1][1], "float32", "states")
 
 
+# Segments of more than 64 rows, where the key channels allow products of matrices: cut into theirs of 64, so that the results are the
+# same bits as with 64. Portions shorter than two segments are
+# walked in order as before.
+@pytest.mark.parametrize("kind,D,V", [("decay", 128, 64), ("gated_max", 96, 48)])
+@pytest.mark.parametrize("segment", [65, 100, 128])
+def test_segments_longer_than_the_products_take(kind, D, V, segment):
+    ops, ref = hip_ops("float32"), TorchOps("cpu", torch.float32)
+    Hh, lens = 2, [2 * segment + 3, 1, 2 * segment - 1]
+    n, nc = sum(lens), 2 * Hh * D + Hh * V
+    g = torch.Generator().manual_seed(segment)
+    proj, decay = torch.randn(n, nc + 2 * Hh, generator=g), torch.rand(n, Hh * D, generator=g) ** 0.1
+    bi, bf = torch.randn(Hh, generator=g), 2 + torch.randn(Hh, generator=g)
+    rows = [(sum(lens[:i]), 0, k) for i, k in enumerate(lens)]
+
+    def run(o, dev, rows, upto):
+        st = torch.zeros(len(rows), ops.state_scan_floats(kind, Hh, D, V), device=dev)
+        kw = dict(i_off=nc, f_off=nc + Hh, bias_i=bi.to(dev), bias_f=bf.to(dev), cap=9.0) if kind == "gated_max" else dict(decay=decay.to(dev))
+        out = o.state_scan(kind, proj.to(dev)[:upto], 0, Hh * D, 2 * Hh * D, D ** -0.5, st,
+                           fake_batch(rows, list(range(len(rows))), None, 1, dev), Hh, D, V, **{k: v[:upto] if k == "decay" else v for k, v in kw.items()})
+        return out, st
+    want = run(ref, "cpu", rows, n)
+    ops.scan_segment = 64
+    short = run(ops, "cuda", rows, n)
+    ops.scan_segment = segment
+    got = run(ops, "cuda", rows, n)
+    for a, b, c in zip(got, short, want):
+        assert torch.equal(a, b)
+        close(a, c, "float32", "results and states")
+    one = [(0, 0, 2 * segment - 1)]
+    in_order = run(ops, "cuda", one, 2 * segment - 1)
+    ops.scan_segment = 0
+    assert torch.equal(in_order[0], run(ops, "cuda", one, 2 * segment - 1)[0])
+
+
 # Heads of more than 128 key channels take the row by row kernels for segments. Every workgroup of the pass over the states reads a
 # request's running maximum, so nothing may write the new one before they all have: single-row requests beside a long one, whose
 # pass is the shortest. (The bound is the one above.)

@@ -16,8 +16,8 @@
 // are 32-bit. Kind 1 keeps n and m once per block of value channels (every block needs them, none may read what another has already advanced).
 //
 // Long portions of prompts are cut into segments of `seg_len` tokens that run side by side (`segments` > 0): up to 128 key
-// channels and 64 tokens by products of matrices (see there); beyond that the same kernel walks every segment from an empty state and leaves the segment's own state, its outputs as if nothing had
-// come before, and what ties them to the past (kind 0: the product of the decays from the segment's start to each
+// channels by products of matrices, 64 tokens at most a segment (see there); beyond that the same kernel walks every segment from an
+// empty state and leaves the segment's own state, its outputs as if nothing had come before, and what ties them to the past (kind 0: the product of the decays from the segment's start to each
 // token; kind 1: the running maximum, the sum of log forget gates and n . q from the segment's start). A second kernel
 // then walks the segments of a request in order, element by element, to the state at every segment's start and the
 // request's new state; a third adds to every token's output what the state at its segment's start contributes:
@@ -355,7 +355,7 @@ __global__ __launch_bounds__(SC_THREADS) void segment_outputs_kernel(const float
 
 // ---- segments by matrix products --------------------------------------------------------------------------------------
 //
-// For up to 128 key channels and segments of up to 64 rows. Row by row a segment's walk is bound by LDS: every thread reads its
+// For up to 128 key channels, in segments of up to 64 rows. Row by row a segment's walk is bound by LDS: every thread reads its
 // share of a row's q, k and decays for each of its own state elements, and all that is done with them is one multiply-add each.
 // As sums over a segment's rows (S_0 the state at its start, P lower triangular, all in 32 bits, nothing divided by a decay),
 //   kind 0:  o_t = (q_t A(-1, t)) S_0 + sum_{i<=t} P(t, i) v_i,  P(t, i) = sum_d q_t k_i A(i, t);   S <- A(-1, last) S_0 + sum_i (k_i A(i, last)) v_i^T
@@ -988,16 +988,18 @@ TIS_EXPORT int tis_state_scan_segmentable(int D) {
 }
 
 // Whether a segmented call goes through the kernels of matrix products, whose addresses inside a segment are 32-bit (ld: the longest
-// distance between two rows).
+// distance between two rows). Longer segments are cut into theirs of SP_ROWS rows: what was gained by longer ones, fewer states
+// to carry, was the row by row kernels'. Segments of
+// 128, us, row by row / cut: 2,048 rows of 8 heads of 128 x 256 277 / 83 (kind 1: 269 / 86), 300 rows 124 / 35.
 static bool by_products(int n_seqs, int seg_len, int D, long rows, long ld) {
-  return D <= 128 && ld >= 0 && ld < (1L << 22) && seg_len <= SP_ROWS && n_seqs <= 65535 && sp_most(rows, seg_len, n_seqs) <= 65535;
+  return D <= 128 && ld >= 0 && ld < (1L << 22) && n_seqs <= 65535 && sp_most(rows, std::min(seg_len, SP_ROWS), n_seqs) <= 65535;
 }
 
-// 32-bit floats of the workspace a segmented call needs (ld: the longest row distance of projections, decays and results): a block for every segment and head; or, off the matrix products, the
-// states, then `rows` lines of decay products or gate sums.
+// 32-bit floats of the workspace a segmented call needs (ld: the longest row distance of projections, decays and results): a block
+// for every segment and head; or, off the matrix products, the states, then `rows` lines of decay products or gate sums.
 TIS_EXPORT long tis_state_scan_workspace(int kind, int n_seqs, int segments, int seg_len, int rows, int H, int D, int V,
                                          long ld) {
-  if (by_products(n_seqs, seg_len, D, rows, ld)) return sp_most(rows, seg_len, n_seqs) * H * SegmentBlock(D, V).floats;
+  if (by_products(n_seqs, seg_len, D, rows, ld)) return sp_most(rows, std::min(seg_len, SP_ROWS), n_seqs) * H * SegmentBlock(D, V).floats;
   return (long)n_seqs * segments * H * ((long)D * V + D + 2) + (kind == 0 ? (long)rows * H * D : (long)rows * H * 3);
 }
 
@@ -1043,7 +1045,8 @@ TIS_EXPORT int tis_state_scan(int kind, const float* proj, long ldp, int q_off, 
       if ((uintptr_t)workspace % 16) return tis_fail("state_scan: the workspace is not 16 bytes aligned");
 #define SP_LAUNCH(KIND, NT)                                                                                                       \
   return launch_products<KIND, NT>(proj, ldp, q_off, k_off, v_off, q_scale, decay, ldd, i_off, f_off, bias_i, bias_f, cap, state, \
-                                   state_ld, cu_rows, seq_slots, n_seqs, out, ldo, H, D, V, seg_len, rows, workspace, lay, stream)
+                                   state_ld, cu_rows, seq_slots, n_seqs, out, ldo, H, D, V, std::min(seg_len, SP_ROWS), rows, workspace, lay, \
+                                   stream)
       if (kind == 0 && D <= 64) SP_LAUNCH(0, 1);
       if (kind == 0) SP_LAUNCH(0, 2);
       if (D <= 64) SP_LAUNCH(1, 1);

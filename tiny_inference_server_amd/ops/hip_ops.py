@@ -2261,7 +2261,7 @@ class HipOps:
 
         A step whose longest portion has at least two segments' rows (self.scan_segment, 64) is run in segments side
         by side, with a pass for the states at the segments' starts and one for what they add to the rows' outputs (as
-        products of matrices for up to 128 key channels); shorter portions and single tokens are walked in order by one
+        products of matrices for up to 128 key channels, there in segments of 64 rows at most); shorter portions and single tokens are walked in order by one
         kernel."""
         n = proj.shape[0]
         if qk_group < 1 or n_heads % qk_group:
