@@ -3,7 +3,8 @@
 // of recurrent mixers, and the low-rank decay of gated linear attention.
 //
 // The RMS norm here is x / sqrt(mean(x^2) + eps) * gain, eps under the root. Every sum is taken in 32-bit in an order
-// that depends on the row's width alone. `T` is the compute type (float or bf16): what the next matrix product reads.
+// that depends on the row's width and on whether rows are read in fours (alignment, strides) alone; residual_norm's beyond 1,024
+// columns also on whether the step has more than 64 rows. `T` is the compute type (float or bf16): what the next matrix product reads.
 #include "common.h"
 
 TIS_DEFINE_LAST_ERROR(tis_stream32)
