@@ -538,6 +538,39 @@ def test_the_delta_rules_walk_in_chunks(Hh, G, D, V, seqs):
     assert not torch.isfinite(broken[at]).any()
 
 
+# Rows walked in chunks against the walk row by row, both against 64 bits: the chunks add the same products up in sums of no more terms and
+# in the rows' order, so neither results nor states lie further off. Either error is the norm of some 100,000 independent roundings of
+# which every one weighs the same, so the two would differ by 1 % if their roundings were as many; 8 % leaves room for T, which
+# the walk row by row does not have (chunks whose products took rows out of their order: 12 to 35 %).
+@pytest.mark.parametrize("H,G,D,V", [(8, 4, 128, 256), (4, 2, 64, 64), (2, 2, 200, 48)])
+@pytest.mark.parametrize("least", [0.5, 0.9, 0.995])
+def test_the_delta_rule_in_chunks_is_no_further_off_than_row_by_row(monkeypatch, H, G, D, V, least):
+    from tiny_inference_server_amd.ops import hip_ops as module
+    ops, n, blocks = hip_ops("float32"), 300, V // 16
+    g = torch.Generator().manual_seed(D)
+    qk = torch.nn.functional.normalize(torch.randn(n, 2 * G, D, generator=g), dim=-1)
+    qk[:, :G] *= D ** -0.5
+    u = torch.cat((qk.reshape(n, -1), torch.nn.functional.silu(torch.randn(n, H * V, generator=g)), torch.rand(n, H, generator=g)), 1).cuda()
+    decay = (least + (1 - least) * torch.rand(n, H * D, generator=g)).cuda()
+    line = (0.3 * torch.randn(1, H * blocks * D * 16, generator=g)).cuda()
+    as_state = lambda t: t.view(H, blocks, D, 16).permute(0, 2, 1, 3).reshape(H, D, V)
+    S, C, want = as_state(line).double(), 2 * G * D + H * V, []
+    wide, slow = u.double(), decay.double()
+    for r in range(n):
+        q, k = (wide[r, i * G * D:(i + 1) * G * D].view(G, D).repeat_interleave(H // G, 0) for i in (0, 1))
+        S = S * slow[r].view(H, D, 1)
+        w = wide[r, C:, None] * (wide[r, 2 * G * D:C].view(H, V) - (S * k[:, :, None]).sum(1))
+        S = S + k[:, :, None] * w[:, None]
+        want.append((S * q[:, :, None]).sum(1).reshape(-1))
+    want, off = torch.stack(want), []
+    for most in (0, module._DELTA_WORK_FLOATS):      # without work space: row by row
+        monkeypatch.setattr(module, "_DELTA_WORK_FLOATS", most)
+        st = line.clone()
+        out = ops.delta_scan(u, 0, G * D, 2 * G * D, C, decay, st, fake_batch([(0, 0, n)], [0], None, 1, "cuda"), H, G, D, V)
+        off.append([((a.double() - b).norm() / b.norm()).item() for a, b in ((out, want), (as_state(st), S))])
+    assert all(chunks <= 1.08 * rows for rows, chunks in zip(*off)), off
+
+
 @pytest.mark.parametrize("lens,chunks", [([1] * 64, False), ([47, 47], False), ([48], True), ([1] * 20 + [48], True)])
 def test_the_delta_rule_asks_for_chunks_only_where_a_request_is_long(lens, chunks):
     """Single tokens of 64 requests are many rows and no long request: the call takes no memory beyond its result (the chunks' operands

@@ -238,14 +238,20 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(
 // with T = (I + beta G)^-1 beta, solved column by column. delta_chunks_kernel makes K~, Q~, K^, A, T and Q of every chunk and head,
 // all chunks at once; delta_chunk_walk_kernel walks them with S in registers, all products on v_mfma_f32_16x16x4_f32 (32-bit
 // multiply-adds). Rows past a request's last have k = q = 0, decay 1 and beta 0 and change nothing. MI355X, 8 heads of 128 x 256,
-// us row by row / in chunks with the step before them: 2,048 rows 545 / 196, 1,531 410 / 153, 512 140 / 58, 128 39 / 24; off from 64
-// bits by 1.7e-7 and 1.8e-7.
+// us row by row / in chunks with the step before them: 2,048 rows 546 / 199, 1,531 410 / 155, 512 141 / 59, 128 38 / 24. Off from 64 bits, row
+// by row / in chunks, by decays from 0.5, 0.9 and 0.995 on: results 0.99e-7 / 0.98e-7, 1.39e-7 / 1.40e-7, 3.3e-7 / 3.0e-7, states 0.62e-7 / 0.62e-7,
+// 1.16e-7 / 1.19e-7, 3.6e-7 / 3.2e-7. (With rows four apart in a product, the newest among the first, 1.15e-7 and 0.87e-7 at the strongest
+// decays, where the newest are the largest; with one sum over a wave's channels 5 % more, and 162 us where the four take 155.)
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 static constexpr int DC = 16;                    // rows of a chunk
 static constexpr int DR_CHUNK_FROM = 48;         // rows of a request from which on its rows are walked in chunks (us, row by row / in
                                                  // chunks: 32 rows 13.3 / 14.5, 48 17.9 / 16.1, 128 39 / 24)
 
 __host__ __device__ constexpr int dc_floats(int Dp) { return 3 * DC * Dp + Dp + 2 * DC * DC; }   // of a chunk and head: K~, Q~, K^ [d][row], A, T, Q
+
+// Where row i of a chunk lies in the products: register r of lane (g, n) is place 4 g + r and row 4 r + g, so that a product over rows adds
+// them four at a time in their order, oldest first, as the walk row by row does (its own inverse).
+__host__ __device__ constexpr int dc_place(int i) { return i % 4 * 4 + i / 4; }
 
 __device__ __forceinline__ int dc_chunks(int n) { return n >= DR_CHUNK_FROM ? (n + DC - 1) / DC : 0; }
 
@@ -312,10 +318,10 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
         p[j] = fmaf(ka[e], qj[e], p[j]);
       }
     }
-    *reinterpret_cast<f32x4*>(Kt + i * Dp + d) = ki * upto;
-    *reinterpret_cast<f32x4*>(Qt + i * Dp + d) = qi * upto;
+    *reinterpret_cast<f32x4*>(Kt + dc_place(i) * Dp + d) = ki * upto;
+    *reinterpret_cast<f32x4*>(Qt + dc_place(i) * Dp + d) = qi * upto;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) Kh[(d + e) * DC + i] = ka[e];
+    for (int e = 0; e < 4; ++e) Kh[(d + e) * DC + dc_place(i)] = ka[e];
     if (i == DC - 1) *reinterpret_cast<f32x4*>(A + d) = upto;
   }
 #pragma unroll
@@ -323,7 +329,7 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
     const float gs = dr_row_sum(g[j]), ps = dr_row_sum(p[j]);
     if (l == j) {
       L[j][i] = gs;
-      Q[j * DC + i] = i <= j ? ps : 0.f;
+      Q[dc_place(j) * DC + dc_place(i)] = i <= j ? ps : 0.f;
     }
   }
   __syncthreads();
@@ -335,7 +341,7 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
 #pragma unroll
       for (int m = 0; m < j; ++m) v = m >= t ? fmaf(-L[j][m], x[m], v) : v;
       x[j] = j >= t ? beta[j] * v : 0.f;
-      T[j * DC + t] = x[j];
+      T[dc_place(j) * DC + dc_place(t)] = x[j];
     }
   }
 }
@@ -344,7 +350,7 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
 // result tiles of 16 channels x 16 value channels: lane (g, n) = (lane / 16, lane % 16) holds channels 16 t + 4 g + r of value
 // channel n in register r of tile t. As the second operand of a product over channels, register r of tile t is what the four channels
 // 16 t + 4 g + r (g = 0 .. 3) make up, so S goes into the products as it lies; the same holds for V - K~ S0 and W, whose rows are
-// 4 g + r. The waves' parts of K~ S0 meet in LDS, one barrier a chunk; each then makes W for itself. Q~ S0 is worked out while the parts
+// 4 r + g (see dc_place). The waves' parts of K~ S0 meet in LDS, one barrier a chunk; each then makes W for itself. Q~ S0 is worked out while the parts
 // are on their way, and the fifth wave, which makes W too, adds up the rows' results a chunk later. Three chunks' operands are
 // under way (one ahead, a chunk took what memory takes), or one where a head's channels leave no more registers. Workgroups of one head follow one another by `heads`, so that with 8 heads
 // (or 16, ...) an XCD's L2 serves a head to all of its value channels. What bounds it is a chunk's chain: the products with S, LDS, W, and
@@ -387,15 +393,15 @@ __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(const float* __re
     }
 #pragma unroll 1
     for (int i = 0; i < DC; ++i) {
-      const float xi = __shfl(i % 4 == 0 ? x[0] : i % 4 == 1 ? x[1] : i % 4 == 2 ? x[2] : x[3], (i / 4) * 16 + n, 64);
+      const float xi = __shfl(i / 4 == 0 ? x[0] : i / 4 == 1 ? x[1] : i / 4 == 2 ? x[2] : x[3], i % 4 * 16 + n, 64);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (i <= g * 4 + r) sum[r] += M[(g * 4 + r) * DC + i] * xi;
+        if (i <= r * 4 + g) sum[r] += M[(g * 4 + r) * DC + dc_place(i)] * xi;
     }
     return sum;
   };
   auto make_w = [&](int c, f32x4 m, f32x4 v) {
-    f32x4 x = v - (ks_parts[c & 1][0][lane] + ks_parts[c & 1][1][lane] + ks_parts[c & 1][2][lane] + ks_parts[c & 1][3][lane]);
+    f32x4 x = v - ((ks_parts[c & 1][0][lane] + ks_parts[c & 1][1][lane]) + (ks_parts[c & 1][2][lane] + ks_parts[c & 1][3][lane]));
 #pragma unroll
     for (int r = 0; r < 4; ++r) x[r] = live ? x[r] : 0.f;
     return triangle(base + c * stride + OFF_T, m, x, zero);
@@ -404,7 +410,7 @@ __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(const float* __re
   auto fetch_v = [&](int c) {
     f32x4 v;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = v_column[(long)min(c * DC + g * 4 + r, n_rows - 1) * ldu];
+    for (int r = 0; r < 4; ++r) v[r] = v_column[(long)min(c * DC + r * 4 + g, n_rows - 1) * ldu];
     return v;
   };
   // (not __syncthreads, which also waits for what is under way from memory)
@@ -420,10 +426,10 @@ __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(const float* __re
     f32x4 W = zero, q = zero;                    // of the chunk before
     auto results = [&](int c) {
       const f32x4 o = triangle(base + c * stride + OFF_Q, q, W,
-                               qs_parts[c & 1][0][lane] + qs_parts[c & 1][1][lane] + qs_parts[c & 1][2][lane] + qs_parts[c & 1][3][lane]);
+                               (qs_parts[c & 1][0][lane] + qs_parts[c & 1][1][lane]) + (qs_parts[c & 1][2][lane] + qs_parts[c & 1][3][lane]));
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = c * DC + g * 4 + r;
+        const int row = c * DC + r * 4 + g;
         if (row < n_rows && live) out[(long)(first + row) * ldo + h * V + c_v] = o[r];
       }
     };
@@ -471,18 +477,19 @@ __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(const float* __re
     o.t = *reinterpret_cast<const f32x4*>(p + OFF_T + n * DC + g * 4);
     o.v = fetch_v(c);
   };
+  // the wave's part of a product with S, in four sums, so that none is a longer chain than the walk row by row has
+  auto against = [&](const f32x4 (&rows)[NT]) {
+    f32x4 part[4];
+#pragma unroll
+    for (int k = 0; k < NT; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) part[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(rows[k][r], S[k][r], k ? part[r] : zero, 0, 0, 0);
+    return (part[0] + part[1]) + (part[2] + part[3]);
+  };
   auto chunk = [&](int c, const Operands& now) {
-    f32x4 ks = zero, qs = zero;
-#pragma unroll
-    for (int k = 0; k < NT; ++k)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ks = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kt[k][r], S[k][r], ks, 0, 0, 0);
-    ks_parts[c & 1][wave][lane] = ks;
+    ks_parts[c & 1][wave][lane] = against(now.kt);
     meet();
-#pragma unroll
-    for (int k = 0; k < NT; ++k)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) qs = __builtin_amdgcn_mfma_f32_16x16x4f32(now.qt[k][r], S[k][r], qs, 0, 0, 0);
+    const f32x4 qs = against(now.qt);
     const f32x4 W = make_w(c, now.t, now.v);
     qs_parts[c & 1][wave][lane] = qs;
 #pragma unroll
