@@ -372,9 +372,11 @@ __global__ __launch_bounds__(SC_THREADS) void segment_outputs_kernel(const float
 // 110 / 30, eight requests of 512 rows 417 / 136. Inside a prompt step of 1,200 and 600 rows, traced kernel by kernel, the rows' kernel takes 28.9
 // (LDS, pair by pair; kind 1: 16.6), the walk 26.0 (30.1; a chain of one segment after another, 1.4 us each) and the results 26.9 (32.1; memory:
 // the states at the starts twice over). The workspace is 3,360 bytes a row and head of these sizes (the row by row segments' was 2,570 for
-// one request, and more than this for requests of unequal lengths). Off from 64 bits by 1.4e-7 (row by row) and 1.2e-7 (kind 0; sums
-// of products run in four accumulators each, which keeps their chains as short as the row by
-// row kernel's), kind 1 by 0.5e-6 to 3e-6 both ways (its division).
+// one request, and more than this for requests of unequal lengths). Off from 64 bits, row by row in segments / by products, 130 rows of these
+// heads, decays from 0.5, 0.9 and 0.995 on: results 1.26e-7 / 1.01e-7, 1.51e-7 / 1.35e-7, 2.22e-7 / 1.83e-7, states 0.49e-7 / 0.54e-7, 0.87e-7 /
+// 0.96e-7, 1.76e-7 / 1.67e-7: sums of products run in four accumulators each, which keeps their chains short, but the decays up to a row's
+// segment's end are multiplied up before they meet the row. (One sum in the order of the rows: states 0.49e-7, 1.08e-7, 2.02e-7, results as here;
+// a sum for each 16 rows 0.51e-7, 1.02e-7, 1.68e-7, and 92 us where these take 83.) Kind 1 by 0.2e-6 to 2e-6 both ways (its division).
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 static constexpr int SP_ROWS = 64;               // rows a segment can have: four tiles of 16
 
