@@ -63,7 +63,8 @@ struct RopeArgs {
 // GS_WAVES: waves per workgroup; U: steps of K whose loads a wave issues together before the first product.
 // Eight waves of three or four steps measured best on MI355X for K of 1536 to 4096 (5.6 us for a 25 MB matrix,
 // 23 us for the 147 MB output table: 80 % of the HBM peak); four waves where K is too short to feed eight. Batches
-// of eight steps where a wave has eight (K of 4096: all its loads in flight at once) take 0.56 us off; sixteen waves measured the
+// of eight steps where a wave has eight (K of 4096: all its loads in flight at once) take 0.56 us off alone and as much inside a
+// step (1536 x 4096 in its place, traced: 1 row 7.48 / 6.95, 8 rows 7.83 / 7.19; 1 % of the step); sixteen waves measured the
 // same within noise (the gated product at 64 rows slower: fewer workgroups fit a compute unit).
 //
 // MB: blocks of 16 rows of X that share every weight tile a wave loads, and CT: column tiles of 16 a workgroup
