@@ -4,21 +4,25 @@
 // PFLOP/s at 2,048 rows. This kernel reaches 0.75 to 1.0 on the same shapes; the library's kernels, where they may be
 // used, 0.5 to 1.3.) The reference's engine uses a library product here (x @ W, main_models_new.py:19-20).
 //
-// tile_loop.h holds the loop. A row's sums run over K in the same order whatever M is: its result does not depend on the other rows.
-// With operands fetched where they are used and copies one step ahead (before) and as the loop is now, us: 2,048 rows x 2,048 x 2,048
-// 28.0 / 22.7; inner 5,632 62.9 / 48.0; 2,048 x 5,632 x 2,048 54.0 / 49.6; 1,800 x 32,000 x 2,048 271 / 247; 1,531 x 2,048 x 2,048
-// 24.1 / 18.2; 300 x 1,024 x 1,024 12.1 / 6.8; 8 columns 14.9 / 7.9.
+// tile_loop.h holds the loop. A row's sums run over K in the same order whatever M is and whichever tile is taken: its result does not depend on the other rows.
 #include "tile_loop.h"
 
 TIS_DEFINE_LAST_ERROR(tis_gemm_tiles)
 
 // BM x BN: the workgroup's tile; WM x WN: its waves, each with (BM / WM) x (BN / WN) of it
 // ACT: what becomes of a sum before it is rounded (0 nothing; 1 the tanh form of gelu, 0.5 z (1 + tanh(u)) written as
-// z / (1 + exp(-2u)); 2 the square of relu; 3 clamped_swish of the columns' pairs (2j, 2j + 1): C has N / 2 columns)
+// z / (1 + exp(-2u)); 2 the square of relu; of the columns' pairs (2j, 2j + 1), for a C of N / 2 columns: 3 clamped_swish, 4 silu(g) u)
 template <int ACT> __device__ __forceinline__ float gt_activated(float z) {
   if (ACT == 1) return z / (1.f + __expf(-1.5957691216057308f * (z + 0.044715f * z * z * z)));
   if (ACT == 2) { const float p = fmaxf(z, 0.f); return p * p; }
   return z;
+}
+template <int ACT> __device__ __forceinline__ float gt_gated(float g, float u, float limit) {
+  if (ACT == 3) return clamped_swish(g, u, limit);
+  // the gate of the rounded product, as the kernel that reads a stored one takes it: the same bits whichever way a step went
+  g = static_cast<float>(static_cast<__bf16>(g));
+  u = static_cast<float>(static_cast<__bf16>(u));
+  return g / (1.f + expf(-g)) * u;
 }
 
 template <int BM, int BN, int WM, int WN, int NSTAGE, int AHEAD, bool RESIDUAL, typename TO, int ACT = 0>
@@ -32,7 +36,6 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
   const int wm = wave / WN, wn = wave % WN;
   const GtTile tile = gt_tile(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN);
   const long m0 = (long)tile.m * BM, n0 = (long)tile.n * BN;
-
   // Rows past the matrix's last are the last row again (their results are not stored).
   const unsigned char* first[LPW];
   unsigned lane_off[LPW];
@@ -67,11 +70,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
       for (int q = 0; q < 4; ++q) {
         const long n = n0 + wn * (BN / WN) + j * 32 + q * 8 + h * 4;
         if (n >= N) continue;                 // (N is a multiple of 4: the four columns are inside or outside together)
-        if constexpr (ACT == 3) {
+        if constexpr (ACT >= 3) {
           typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-          *(bf16x2*)(C + m * c_ld + n / 2) =
-              (bf16x2){static_cast<__bf16>(clamped_swish(acc[i][j][q * 4], acc[i][j][q * 4 + 1], limit)),
-                       static_cast<__bf16>(clamped_swish(acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3], limit))};
+          *(bf16x2*)(C + m * c_ld + n / 2) = (bf16x2){static_cast<__bf16>(gt_gated<ACT>(acc[i][j][q * 4], acc[i][j][q * 4 + 1], limit)),
+                                                      static_cast<__bf16>(gt_gated<ACT>(acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3], limit))};
           continue;
         }
         float v[4];
@@ -97,64 +99,94 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
 static int g_units = 256;      // compute units of the device: set by whoever knows (the default is an MI355X)
 TIS_EXPORT void tis_gemm_tiles_units(int n) { if (n > 0) g_units = n; }
 
+// The tiles, and what a product is estimated to take with each, us: a beginning and end, and the time of a step of 64 by r, the tiles a
+// compute unit. Measured with matrices that come from memory (none that a cache still holds), 200 to 3,000 rows, widths of 256 to 32,000. Over
+// 271 such products the one picked here takes 1.009 times the fastest's time on average.
+//
+// What bounds a product of few hundred rows is the way of its matrix from memory: a tile's copies reach three to five steps ahead (what
+// its buffers hold; 5 instead of 4 buffers of 64 x 64, 6 of 64 x 32 and 128 x 64), and there are tiles enough for the chip. us before
+// (tiles of 64 x 64 up to 256 x 256, three steps ahead) / now, and the library's product: 300 rows of 1,536 x 1,536 11.1 / 8.1 (10.6), of
+// 2,304 x 1,536 11.4 / 9.4 (16.6), of 1,536 x 4,096 26 / 15.5 (21.1); 140 rows of 1,536 x 4,096 24.6 / 14.7 (15.6); 700 rows of 2,304 x 1,536
+// 15.2 / 11.3 (16.4); 2,048 rows of 2,304 x 1,536 33 / 22.6 (23.7), of 2,816 x 2,048 41.1 / 31.2 (30.4), of 3,072 x 2,048 41.0 / 32.4 (30.5).
+// (K in two parts by two sets of waves, for products of less than a tile a unit: 1 to 2.5 us less, but other sums than every other tile's,
+// and than the library's, with which all of these agree to the bit.)
+// Beyond one tile a unit a tile's LDS says how many share one: two of 128 x 192, 64 x 64 and 64 x 32, else one.
+struct TileShape { int bm, bn; };
+static const TileShape g_shapes[8] = {{256, 256}, {256, 128}, {192, 128}, {128, 192}, {128, 128}, {128, 64}, {64, 64}, {64, 32}};
+static long tiles_of(int i, int M, int N) {
+  return (long)((M + g_shapes[i].bm - 1) / g_shapes[i].bm) * ((N + g_shapes[i].bn - 1) / g_shapes[i].bn);
+}
+static float tile_estimate(int i, int M, int N, int K) {
+  const float r = (float)tiles_of(i, M, N) / g_units, steps = (float)((K + GT_BK - 1) / GT_BK), part = r - floorf(r);
+  switch (i) {
+    case 0: return 5.0f + steps * (1.85f * floorf(r) + (part > 0.f ? fmaxf(1.5f, 1.5f + 1.2f * (part - 0.6f)) : 0.f));
+    case 1: return 4.5f + steps * (r <= 0.75f ? 0.82f : r <= 1.f ? 1.05f : 0.55f + 0.95f * r);
+    case 2: return 4.2f + steps * (r <= 0.75f ? 0.63f : r <= 1.f ? 0.77f : 0.45f + 0.72f * r);
+    case 3: return 4.5f + steps * (r <= 1.f ? 1.1f : r <= 2.f ? fmaxf(1.42f, 0.79f * r) : fmaxf(2.3f, 0.78f * r));
+    case 4: return 4.0f + steps * (r <= 1.f ? 0.53f : 0.2f + 0.6f * r);
+    case 5: return 4.0f + steps * (r <= 0.75f ? 0.32f : r <= 1.f ? 0.37f : 0.03f + 0.36f * ceilf(r));
+    case 6: return 3.4f + steps * (r <= 1.f ? 0.25f : r <= 1.25f ? 0.36f : 0.22f * ceilf(r));
+    default: return 3.7f + steps * (r <= 1.f ? 0.175f : 0.29f * ceilf(0.5f * r));
+  }
+}
+
+// The tile that a product takes, an index into g_shapes.
+TIS_EXPORT int tis_gemm_tiles_pick(int M, int N, int K) {
+  int pick = 0;
+  float best = tile_estimate(0, M, N, K);
+  for (int i = 1; i < 8; ++i) {
+    const float t = tile_estimate(i, M, N, K);
+    if (t < best) best = t, pick = i;
+  }
+  return pick;
+}
+
 // W: [N, K] contiguous. R: null, or the residual (bfloat16) added to the product; it may be C itself (every element is
 // read and then written by the same lane). out_f32: C holds 32-bit floats, the sums as they are (the output table's
 // logits), and takes no residual. act: 1 the tanh form of gelu, 2 the square of relu, 3 clamped_swish of pairs of columns at
-// `limit` (C has N / 2 columns), applied to the 32-bit sums of a bfloat16 result without a residual. Sizes: K and x_ld multiples of 8, N, c_ld and r_ld multiples of 4; X and W 16-byte
+// `limit`, 4 silu(g) u of pairs of columns of the rounded product
+// (3 and 4: C has N / 2 columns), the others applied to the 32-bit sums; a bfloat16 result without a residual.
+// Sizes: K and x_ld multiples of 8, N, c_ld and r_ld multiples of 4; X and W 16-byte
 // aligned, C and R 8-byte aligned (a 32-bit C 16-byte). Launches only: safe under stream capture.
 TIS_EXPORT int tis_gemm_tiles(const void* X, long x_ld, const void* W, const void* R, long r_ld, void* C, long c_ld,
                               int M, int N, int K, int out_f32, int act, float limit, hipStream_t stream) {
   if (M < 0 || N < 0 || K < 1) return tis_fail("gemm_tiles: bad size M=%d N=%d K=%d", M, N, K);
   if (M == 0 || N == 0) return 0;
   if (K % 8 || x_ld % 8 || x_ld < K) return tis_fail("gemm_tiles: K=%d and the input's row stride %ld must be multiples of 8", K, x_ld);
-  if (N % 4 || c_ld % (act == 3 ? 2 : 4) || c_ld < (act == 3 ? N / 2 : N) || (R && (r_ld % 4 || r_ld < N)))
+  if (N % 4 || c_ld % (act >= 3 ? 2 : 4) || c_ld < (act >= 3 ? N / 2 : N) || (R && (r_ld % 4 || r_ld < N)))
     return tis_fail("gemm_tiles: N=%d and the row strides of the output (%ld) and residual (%ld) must be multiples of 4", N, c_ld, r_ld);
   if (((uintptr_t)X | (uintptr_t)W) % 16 || ((uintptr_t)C | (uintptr_t)R) % 8 || (out_f32 && (uintptr_t)C % 16))
     return tis_fail("gemm_tiles: inputs must be 16-byte aligned, output and residual 8-byte aligned (a 32-bit output 16-byte)");
   if (act == 3 && !(limit > 0.f)) return tis_fail("gemm_tiles: a clamp at %g", (double)limit);
-  if (act < 0 || act > 3 || (act && (out_f32 || R))) return tis_fail("gemm_tiles: an activation (%d) goes with a plain bfloat16 result", act);
+  if (act < 0 || act > 4 || (act && (out_f32 || R))) return tis_fail("gemm_tiles: an activation (%d) goes with a plain bfloat16 result", act);
   if (out_f32 && R) return tis_fail("gemm_tiles: a 32-bit result takes no residual");
   if ((long)x_ld * 16 >= (1L << 31) || (long)K * 16 >= (1L << 31)) return tis_fail("gemm_tiles: rows of %ld elements are too long for 32-bit offsets", x_ld);
-  // The tile: the one that is estimated to end first, by the microseconds a step of 64 takes with one or more workgroups a
-  // compute unit (measured at K of 1,408 to 5,632; the clock falls as more of the chip works, hence 1.36 to 1.85 for the largest):
-  //   256 x 256, eight waves, two buffers    1.36 up to 0.7 workgroups a unit, then to 1.72 at one; 1.85 a full round
-  //   128 x 192, four waves, two buffers     0.79 up to one a unit; two share one: from 1.25 on, 0.79 for each on average
-  //   128 x 128, eight waves, four buffers   0.47, and 0.6 a further round
-  //   64 x 64, four waves, four buffers      0.21 up to one a unit; two share one: from 0.42 on, 0.21 for each on average
-  // (us, 256 / 192 / 128 / 64, 2,048 inner columns: 2,048 x 2,048 48.4, 31.4, 22.7, 30.5; 2,048 x 2,816 47.0, 31.3, 33.0, 39.2;
-  // 2,048 x 5,120 49.0, 48.6, 51.9, 66.5; 1,800 x 8,192 62.8, 71.3, 70.8, 98.2; 1,536 x 11,264 102.9, 75.1, 84.9, 110.0;
-  // 1,800 x 32,000 247, 280, 333, 420; 700 x 1,024 x 2,816 59.4, 37.4, 20.6, 13.8.)
-  struct { int bm, bn; } const shapes[4] = {{256, 256}, {128, 192}, {128, 128}, {64, 64}};
-  int pick = 0;
-  float best = 0.f;
-  long tiles = 0;
-  for (int i = 0; i < 4; ++i) {
-    const long n = (long)((M + shapes[i].bm - 1) / shapes[i].bm) * ((N + shapes[i].bn - 1) / shapes[i].bn);
-    const float r = (float)n / g_units, full = floorf(r), part = r - full;
-    float t;
-    if (i == 0) t = 1.85f * full + (part > 0.f ? fmaxf(1.36f, 1.36f + 1.2f * (part - 0.7f)) : 0.f);
-    else if (i == 2) t = 0.47f + 0.6f * (ceilf(r) - 1.f);
-    else if (i == 1) t = r <= 1.f ? 0.79f : fmaxf(1.25f, 0.79f * r);
-    else t = r <= 1.f ? 0.21f : fmaxf(0.42f, 0.21f * r);
-    if (i == 0 || t < best) best = t, pick = i, tiles = n;
-  }
+  const int pick = tis_gemm_tiles_pick(M, N, K);
+  const long tiles = tiles_of(pick, M, N);
   if (tiles >= (1L << 31)) return tis_fail("gemm_tiles: %ld tiles are more than a grid holds", tiles);
-#define LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, RV, TOV, ACTV)                                                     \
-  gemm_tiles_kernel<BMV, BNV, WMV, WNV, NSV, AHV, RV, TOV, ACTV><<<dim3((unsigned)tiles), WMV * WNV * 64, 0, stream>>>(    \
+#define LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, RV, TOV, ACTV)                                                               \
+  gemm_tiles_kernel<BMV, BNV, WMV, WNV, NSV, AHV, RV, TOV, ACTV><<<dim3((unsigned)tiles), WMV * WNV * 64, 0, stream>>>(   \
       (const bf16*)X, x_ld, (const bf16*)W, (const bf16*)R, r_ld, (TOV*)C, c_ld, M, N, K, limit)
 #define PICK(BMV, BNV, WMV, WNV, NSV, AHV)                                     \
   {                                                                             \
-    if (out_f32) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, float, 0);   \
-    else if (R) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, true, bf16, 0);      \
-    else if (act == 1) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 1); \
-    else if (act == 2) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 2); \
-    else if (act == 3) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 3); \
-    else LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 0);            \
+    if (out_f32) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, float, 0);       \
+    else if (R) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, true, bf16, 0);          \
+    else if (act == 1) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 1);  \
+    else if (act == 2) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 2);  \
+    else if (act == 3) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 3);  \
+    else if (act == 4) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 4);  \
+    else LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 0);                \
   }
-  if (pick == 0) PICK(256, 256, 2, 4, 2, 1)
-  else if (pick == 1) PICK(128, 192, 2, 2, 2, 1)
-  else if (pick == 2) PICK(128, 128, 2, 4, 4, 2)
-  else PICK(64, 64, 2, 2, 4, 2)
+  switch (pick) {
+    case 0: PICK(256, 256, 2, 4, 2, 1) break;
+    case 1: PICK(256, 128, 4, 2, 3, 1) break;
+    case 2: PICK(192, 128, 2, 4, 4, 2) break;
+    case 3: PICK(128, 192, 2, 2, 2, 1) break;
+    case 4: PICK(128, 128, 2, 4, 5, 2) break;
+    case 5: PICK(128, 64, 4, 2, 6, 2) break;
+    case 6: PICK(64, 64, 2, 2, 5, 2) break;
+    default: PICK(64, 32, 2, 1, 6, 2) break;
+  }
 #undef PICK
 #undef LAUNCH
   return tis_launch_status("gemm_tiles");

@@ -3,14 +3,13 @@
 //
 // A workgroup owns a tile of BM rows of X x BN rows of W and walks K in steps of 64. A step's
 // operand rows, 128 bytes each, are copied into LDS by global_load_lds_dwordx4 (no registers; eight lanes read one
-// row's 128 bytes) into a ring of NSTAGE buffers, one to three steps ahead of the products. A row's eight 16-byte pieces lie in LDS with their index XORed by half the row's number:
+// row's 128 bytes) into a ring of NSTAGE buffers, two to five steps ahead of the products. A row's eight 16-byte pieces lie in LDS with their index XORed by half the row's number:
 // an operand fetch reads one piece index of 32 rows, LDS serves sixteen lanes at a time, and sixteen rows of 128
 // bytes are eight such indices at each of two offsets in the 256 bytes that the banks span, so no two of them meet
 // (XORed by the row's number itself, rows r and r + 8 did: half of the LDS's busy cycles were bank conflicts). The
 // copying lane picks the piece that belongs in its slot. The result tile is computed transposed (W's rows are the first operand), so that a
 // lane ends up with four consecutive columns of one row: 8-byte stores, and the residual read the same way.
 // A row's sums run over K in the same order whatever M is: its result does not depend on the other rows.
-//
 //
 // What bounds it: the clock under load (8,192 cubed runs at 1.42 PFLOP/s here: 1.5 us for a step of a 256 x 256 tile on every
 // compute unit), for tiles of 64 x 64 and 128 x 128 the LDS, whose reads and writes take 1.5 to 2 times the products' cycles, and for
@@ -73,7 +72,7 @@ struct TileLoop {
   static constexpr int FLIGHT = AHEAD == 1 ? NSTAGE : NSTAGE - 1;   // steps that are copied ahead
   static constexpr int SETS = AHEAD == 1 ? 2 : KS;             // operand registers: a set a slice, in turn
   static_assert(ROWS * PCS % (64 * WAVES) == 0 && TM >= 1 && TN >= 1 && NSTAGE * STAGE <= 160 * 1024, "tile sizes");
-  static_assert((AHEAD == 1 || AHEAD == 2) && FLIGHT >= 2 && FLIGHT <= 3 && KS == 4, "what the loop below is written for");
+  static_assert((AHEAD == 1 || AHEAD == 2) && FLIGHT >= 2 && KS == 4, "what the loop below is written for");
   static_assert((FLIGHT - 1) * LPW <= 63, "more loads in flight than the counter counts");
 
   // the row of the buffer that a lane's piece of load j belongs to, and which of the row's pieces it is
@@ -171,10 +170,13 @@ struct TileLoop {
       step(kt, IntC<1>{}, IntC<FLIGHT - 2>{}, IntC<0>{});
       ++kt;
     }
-    // the last steps, whose copies are all under way
-    if constexpr (FLIGHT == 3)
-      if (nk >= 3) step(kt++, IntC<2>{}, IntC<1>{}, IntC<0>{});
-    if (nk >= 2) step(kt++, IntC<2>{}, IntC<0>{}, IntC<0>{});
+    // the last steps, whose copies are all under way: while `remain` are left, remain - 2 beyond the next
+    auto last_steps = [&](auto self, auto remain) {
+      constexpr int REMAIN = remain;
+      if (nk >= REMAIN) step(kt++, IntC<2>{}, IntC<REMAIN - 2>{}, IntC<0>{});
+      if constexpr (REMAIN > 2) self(self, IntC<REMAIN - 1>{});
+    };
+    last_steps(last_steps, IntC<FLIGHT>{});
     step(kt, IntC<2>{}, IntC<0>{}, IntC<1>{});
   }
 };

@@ -184,6 +184,14 @@ def library(name: str) -> _Lib:
 
 
 _FEW_ROWS = 128                 # up to this many rows a product goes to the few-row kernels whatever its widths
+_TILES_UP_TO = 1024             # a model's own products of more rows than that, but no more than these, run on this repository's tiles
+                                # also at the library's widths, where the library has a product of few tiles wait for its matrix.
+                                # us, library / tiles, matrices from memory: 2,304 x 1,536 at 140, 320, 640, 1,024 rows 10 / 8, 17 / 9.6,
+                                # 17 / 13, 18 / 18; 1,536 x 4,096 16 / 15, 21 / 16, 24 / 20, 25 / 25; 2,048 x 5,632 21 / 19, 26 / 27, 34 / 37,
+                                # 41 / 37; with the gate (library and gate kernel / tiles) 8,192 x 1,536 23 / 13, 25 / 18, 31 / 26, 38 / 32;
+                                # 11,264 x 2,048 30 / 21, 37 / 27, 48 / 45, 58 / 57. At 1,532 and 2,048 rows the library is the faster:
+                                # 1,536 x 4,096 34 / 35, 35 / 36, 8,192 x 1,536 45 / 48, 53 / 56, 11,264 x 2,048 83 / 78, 96 / 100.
+                                # Both add a row's products up in the same order and give the same bits
 
 _WIDTHS_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "library_widths.json")
 
@@ -872,15 +880,39 @@ class HipOps:
         if route == "tiles":
             if out_dtype == torch.float32 and residual is not None:
                 raise KernelError("linear: a 32-bit result of bfloat16 operands takes no residual")
-            out = self.empty(M, N, dtype=out_dtype)
-            self.gemm_tiles.tis_gemm_tiles(_ptr(x), x.stride(0), _ptr(w), _ptr(residual),
-                                           residual.stride(0) if residual is not None else 0, _ptr(out), out.stride(0),
-                                           M, N, K, 1 if out_dtype == torch.float32 else 0, 0, 0.0, self._stream())
-            return out
+            return self._linear_tiles(x, w, residual, self.empty(M, N, dtype=out_dtype), N, 1 if out_dtype == torch.float32 else 0, 0)
         out = self.empty(M, N, dtype=out_dtype)
         self.gemm_plain.tis_gemm_plain(1, _DT[out_dtype], _ptr(x), x.stride(0), _ptr(w), K, _ptr(residual),
                                        residual.stride(0) if residual is not None else 0, _ptr(out), out.stride(0), M, N,
                                        K, self._stream())
+        return out
+
+    def _tiles_at_any_width(self, x, M, N, K, residual=None):
+        """Whether a bfloat16 product of these rows runs on the tiled product whatever its widths (see _TILES_UP_TO)."""
+        return (self.dtype == torch.bfloat16 and self.few_rows < M <= _TILES_UP_TO and N % 4 == 0
+                and self._route(x, M, N, K, residual=residual) in ("library", "tiles")
+                and (residual is None or (residual.stride(0) % 4 == 0 and residual.data_ptr() % 8 == 0)))
+
+    def linear_by_rows(self, x, w, residual=None, rms=None, reuse_residual=False):
+        """What linear gives in the compute type; between this repository's tiles and the library's product the number of rows
+        decides, not the widths alone: for the products of a model's own layers."""
+        _rows_view(self._check(x, "linear x"), "linear x")
+        self._check(w, "linear w")
+        (M, K), N = x.shape, w.shape[0]
+        if not (w.dim() == 2 and w.shape[1] == K and w.is_contiguous() and self._tiles_at_any_width(x, M, N, K, residual)):
+            return self.linear(x, w, residual=residual, rms=rms, reuse_residual=reuse_residual)
+        if residual is not None:
+            _rows_view(self._check(residual, "linear residual"), "linear residual")
+            if tuple(residual.shape) != (M, N):
+                raise KernelError(f"linear: residual {tuple(residual.shape)} for result {(M, N)}")
+        if rms is not None:
+            x = self.rmsnorm(x, rms[0], rms[1])
+        return self._linear_tiles(x, w, residual, self.empty(M, N), N, 0, 0)
+
+    def _linear_tiles(self, x, w, residual, out, N, out_f32, act):
+        M, K = x.shape
+        self.gemm_tiles.tis_gemm_tiles(_ptr(x), x.stride(0), _ptr(w), _ptr(residual), residual.stride(0) if residual is not None else 0,
+                                       _ptr(out), out.stride(0), M, N, K, out_f32, act, 0.0, self._stream())
         return out
 
     def _route(self, x, M, N, K, out_dtype=None, residual=None):
@@ -919,6 +951,12 @@ class HipOps:
                 _ptr(x), x.stride(0), _ptr(w), _ptr(rms[0] if rms else None), float(rms[1]) if rms else 0.0,
                 _ptr(None), 0, _ptr(out), out.stride(0), M, N, K, 2, 1, self._stream())
             return out
+        if w.dim() == 2 and w.shape[1] == K and w.is_contiguous() and self._tiles_at_any_width(x, M, w.shape[0], K):
+            # the gate on the product's 32-bit sums; N in steps of 4, so that gate and up lie in one lane
+            self._check(w, "linear w")
+            if rms is not None:
+                x = self.rmsnorm(x, rms[0], rms[1])
+            return self._linear_tiles(x, w, None, self.empty(M, w.shape[0] // 2), w.shape[0], 0, 4)
         return self.swiglu(self.linear(x, w, rms=rms))
 
     # activations that a bfloat16 product applies to its 32-bit sums: (few-row kernel's epilogue, tiled kernel's code)
@@ -1070,7 +1108,7 @@ class HipOps:
                 _ptr(plane if write_cache else None), n_heads, n_kv_heads, head_dim, page_size,
                 int(bool(interleaved)), int(bool(write_cache)), self._stream())
             return q
-        qkv = self.linear(x, w, rms=rms)
+        qkv = self.linear_by_rows(x, w, rms=rms)
         q = self.empty(M, n_heads * head_dim)
         self.rope_write_kv(qkv, positions, write_slots, table, plane, n_heads, n_kv_heads, head_dim, page_size,
                            interleaved, write_cache, paired=True, q_out=q)

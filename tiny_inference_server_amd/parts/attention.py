@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from .base import MIXERS, build_part, to_compute
+from .base import MIXERS, build_part, layer_product, to_compute
 from .spec import PagedKvNeed, StateNeed
 
 
@@ -90,7 +90,7 @@ class GqaAttention:
         extra = {"slopes": self.slopes} if self.slopes is not None else {}
         attn = ops.paged_attention(q, ctx.plane, b, ctx.group, self.n_heads, self.n_kv_heads,
                                    self.head_dim, self.window, self.scale, **extra)
-        return ops.linear(attn, self.w_o, residual=residual, reuse_residual=ctx.residual_is_spent)
+        return layer_product(ops)(attn, self.w_o, residual=residual, reuse_residual=ctx.residual_is_spent)
 
 
 @MIXERS.register("windowed_qknorm_attention")

@@ -145,6 +145,12 @@ def expected_tensors(spec):
     return out
 
 
+def layer_product(ops):
+    """The product x . w^T (+ residual) of a layer's own matrices: by rows, where the operations object tells such products
+    apart (it has kernels of its own for them), else its plain product."""
+    return getattr(ops, "linear_by_rows", None) or ops.linear
+
+
 def normed_linear(ops, x, w, norm, **kw):
     """norm(x) . w^T: through the fused kernel if the norm offers its (gain, eps), else in two steps."""
     if norm is None:

@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from .base import FEED_FORWARDS, to_compute
+from .base import FEED_FORWARDS, layer_product, to_compute
 
 
 def _paired_rows(gate, up):
@@ -40,7 +40,7 @@ class SwiGlu:
         if norm is not None and not hasattr(norm, "as_rms"):
             x, norm = norm(x), None
         hidden = ops.linear_swiglu(x, self.w_gate_up, rms=norm.as_rms() if norm is not None else None)
-        return ops.linear(hidden, self.w_down, residual=residual, reuse_residual=residual_is_spent)
+        return layer_product(ops)(hidden, self.w_down, residual=residual, reuse_residual=residual_is_spent)
 
 
 @FEED_FORWARDS.register("routed_experts")

@@ -1,7 +1,7 @@
 """Stage inputs: where the rows of a stage come from."""
 from __future__ import annotations
 
-from .base import STAGE_INPUTS, build_part, to_compute
+from .base import STAGE_INPUTS, build_part, layer_product, to_compute
 from .spec import StateNeed
 
 
@@ -69,7 +69,7 @@ class FusePreviousStage:
             ops.embedding_rmsnorm(shared["embedding"], batch.tokens, gain, eps, out=fused[:, D:])
         else:
             fused[:, D:].copy_(self.embed_norm(ops.embedding(shared["embedding"], batch.tokens)))
-        return ops.linear(fused, self.w_proj)
+        return layer_product(ops)(fused, self.w_proj)
 
     def after_step(self, batch, previous, state):
         """Once every stage has read its state: the previous stage's newest row of each request waits for the next step."""
