@@ -54,3 +54,34 @@ def test_products_by_rows(ops, M):
         assert torch.equal(ops.linear_by_rows(x, w, residual=whole), ops.linear(x, w, residual=whole))
         assert torch.equal(ops.linear_by_rows(x, w, rms=(gain, 1e-5)), ops.linear(x, w, rms=(gain, 1e-5)))
         assert torch.equal(ops.linear_swiglu(x, w, rms=(gain, 1e-5)), ops.swiglu(ops.linear(x, w, rms=(gain, 1e-5))))
+
+
+@pytest.mark.parametrize("tile,rows,N,K", [(6, 600, 1020, 1416), (7, 1531, 2044, 1992), (8, 900, 2044, 712), (1, 129, 2052, 648), (2, 600, 2044, 1416)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_grouped_product_of_many_steps(ops, tile, rows, N, K, gated):
+    """Eight groups of uneven sizes (one empty, one of a single entry) in the tiles that many steps of K bring: every entry the sum that
+    the group's matrix gives, one whole row of a tile behind the other; the gate one rounding to bfloat16 further."""
+    from ctypes import c_long
+    lib = ops._lazy("experts")
+    assert lib.cdll.tis_grouped_tile(1, 8, rows, c_long(2 * rows), N, K, 0) == tile
+    x, w = rnd((rows, K), 41).cuda(), rnd((8, N, K), 42, K ** -0.5).cuda()
+    order = torch.randperm(2 * rows, generator=torch.Generator().manual_seed(6))
+    left = 2 * rows - 1
+    sizes = [1, 0] + [left // 6 + d for d in (-30, 30, -3, 3, -1)]
+    sizes.append(2 * rows - sum(sizes))
+    lists = torch.zeros(8, rows, dtype=torch.int32)
+    at, group_of = 0, torch.empty(2 * rows, dtype=torch.long)
+    for e, n in enumerate(sizes):
+        mine = order[at:at + n].sort().values
+        lists[e, :n], group_of[mine], at = mine.to(torch.int32), e, at + n
+    lists, counts = lists.cuda(), torch.tensor(sizes, dtype=torch.int32, device="cuda")
+    out = torch.empty(2 * rows, N // 2 if gated else N, device="cuda", dtype=torch.bfloat16 if gated else torch.float32)
+    ops._grouped(x, x.stride(0), 0, 2, w, out, out.shape[1], 0, lists, counts, rows, rows, act=2 if gated else 0, limit=7.0)
+    for e in range(8):
+        mine = (group_of == e).nonzero()[:, 0].cuda()
+        want = x[mine // 2].double() @ w[e].double().t()
+        if gated:
+            g, u = want[:, 0::2].clamp(max=7.0), want[:, 1::2].clamp(-7.0, 7.0)
+            torch.testing.assert_close(out[mine].double(), g * torch.sigmoid(1.702 * g) * (u + 1.0), rtol=8e-3, atol=2e-3)
+        else:
+            torch.testing.assert_close(out[mine].double(), want, rtol=1e-4, atol=1e-4)

@@ -480,14 +480,20 @@ TIS_EXPORT void tis_experts_units(int n) { if (n > 0) g_units = n; }
 
 // The tiles of grouped_tiles_kernel, and the microseconds a step of 64 takes with r workgroups a compute unit:
 //   128 x 192, four waves, two buffers, two a unit     1.05 r, at least 1.15
-//   64 x 64, four waves, four buffers, two a unit      0.3 r, at least 0.33
-//   128 x 128, eight waves, four buffers               0.58 a round
+//   64 x 64, four waves, five buffers, two a unit      0.3 r, at least 0.33
+//   128 x 128, eight waves, five buffers               0.58 a round
 //   256 x 256, eight waves, two buffers                1.85 a round
 //   128 x 128, four waves, two buffers, two a unit     0.78 r, at least 0.8
 //   64 x 64, four waves, two buffers, five a unit      (not by this estimate: for products of few steps)
+//   128 x 64, eight waves, six buffers                 0.42 a round        (these three from ten steps on: what they gain is
+//   256 x 128, eight waves, three buffers              1.1 a round          in the steps, and their buffers take longer to fill)
+//   192 x 128, eight waves, four buffers               0.85 a round
+// us before the last three / with them, 8 groups, two choices a row: 1,531 rows, 5,632 of 2,048 126 / 106, 2,048 of 2,816 70 / 56; 1,000 rows
+// 100 / 88, 60 / 44; 2,048 rows 1,024 of 1,408 37 / 29; 600 rows 2,816 of 1,024 27 / 22, 1,024 of 1,408 18 / 15. A result is the same sum in any tile.
 struct GroupedShape { int bm, bn; float step, least; bool rounds; };
-static const GroupedShape g_shapes[6] = {{128, 192, 1.05f, 1.15f, false}, {64, 64, 0.3f, 0.33f, false}, {128, 128, 0.58f, 0.58f, true},
-                                         {256, 256, 1.85f, 1.85f, true}, {128, 128, 0.78f, 0.8f, false}, {64, 64, 0.f, 0.f, false}};
+static const GroupedShape g_shapes[9] = {{128, 192, 1.05f, 1.15f, false}, {64, 64, 0.3f, 0.33f, false}, {128, 128, 0.58f, 0.58f, true},
+                                         {256, 256, 1.85f, 1.85f, true}, {128, 128, 0.78f, 0.8f, false}, {64, 64, 0.f, 0.f, false},
+                                         {128, 64, 0.42f, 0.42f, true}, {256, 128, 1.1f, 1.1f, true}, {192, 128, 0.85f, 0.85f, true}};
 
 // The tile that a grouped product of bfloat16 rows that lie as it needs them takes, an index into g_shapes; -1: the products straight from memory.
 // lists: most_rows is the most entries a group can have, most_entries the most that all groups have together.
@@ -514,7 +520,8 @@ TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_
     return gate && N <= 128 && (long)groups * ((most_rows + 63) / 64) * ((N + 63) / 64) > 2048 ? 1 : 5;
   int pick = 0;
   float best = INFINITY;
-  for (int i = 0; i < 5; ++i) {
+  for (int i = 0; i < 9; ++i) {
+    if (i == 5 || (i > 5 && K <= 9 * 64)) continue;
     if (K < 256 && i != 1 && i != 4) continue;     // few steps: what counts is a tile's beginning and end
     const GroupedShape& q = g_shapes[i];
     const long tn = (N + q.bn - 1) / q.bn;
@@ -563,11 +570,14 @@ TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, lo
         (const bf16*)A, (const bf16*)W, (float*)C, p, groups);                                                            \
   }
       if (pick == 0) TILES(128, 192, 2, 2, 2, 1)
-      else if (pick == 1) TILES(64, 64, 2, 2, 4, 2)
-      else if (pick == 2) TILES(128, 128, 2, 4, 4, 2)
+      else if (pick == 1) TILES(64, 64, 2, 2, 5, 2)
+      else if (pick == 2) TILES(128, 128, 2, 4, 5, 2)
       else if (pick == 3) TILES(256, 256, 2, 4, 2, 1)
       else if (pick == 4) TILES(128, 128, 2, 2, 2, 1)
-      else TILES(64, 64, 2, 2, 2, 1)
+      else if (pick == 5) TILES(64, 64, 2, 2, 2, 1)
+      else if (pick == 6) TILES(128, 64, 4, 2, 6, 2)
+      else if (pick == 7) TILES(256, 128, 4, 2, 3, 1)
+      else TILES(192, 128, 2, 4, 4, 2)
 #undef TILES
     } else if (aligned && most_rows >= 64 * (lists ? groups : 1)) {
       // 64 entries x 128 columns a workgroup, operands straight from memory
