@@ -1,5 +1,5 @@
-"""Products of a model's own layers at the row counts of prompts: every tile of the tiled product, the gate taken on its sums, and
-the choice between it and the library's product."""
+"""Products of a model's own layers: at the row counts of prompts every tile of the tiled product, the gate taken on its sums, and the
+choice between it and the library's product; in 32 bits the norm and the gate inside the product of few rows."""
 from __future__ import annotations
 
 import pytest
@@ -85,3 +85,21 @@ def test_grouped_product_of_many_steps(ops, tile, rows, N, K, gated):
             torch.testing.assert_close(out[mine].double(), g * torch.sigmoid(1.702 * g) * (u + 1.0), rtol=8e-3, atol=2e-3)
         else:
             torch.testing.assert_close(out[mine].double(), want, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (3, 352, 64), (16, 30, 4), (17, 352, 176), (70, 98, 260), (16, 2000, 1024), (33, 20, 1020)])
+def test_norm_and_gate_inside_the_32_bit_product(M, N, K):
+    """The same bits as the norm's, the product's and the gate's own kernels one after the other, on strided rows too; beyond the widths that
+    fuse, the separate kernels."""
+    ops = hip_ops.HipOps("cuda:0", torch.float32)
+    g = torch.Generator().manual_seed(M + N + K)
+    x = (torch.randn(M, K + 8, generator=g) * 3).cuda()[:, 4:K + 4]
+    w, res, gain = torch.randn(N, K, generator=g).cuda(), torch.randn(M, N, generator=g).cuda(), torch.randn(K, generator=g).cuda()
+    rms = (gain, 1e-5)
+    assert ops._plain_fuses(x, w, rms) and not ops._plain_fuses(x[:, 1:], w, rms)
+    normed = ops.rmsnorm(x, *rms)
+    assert torch.equal(ops.linear(x, w, rms=rms), ops.linear(normed, w))
+    assert torch.equal(ops.linear(x, w, rms=rms, residual=res), ops.linear(normed, w, residual=res))
+    assert torch.equal(ops.linear_swiglu(x, w, rms=rms), ops.swiglu(ops.linear(normed, w)))
+    assert torch.equal(ops.linear_swiglu(x, w), ops.swiglu(ops.linear(x.contiguous(), w)))
+    assert not ops.gemm_plain.cdll.tis_gemm_plain_fuses(M, N, 1028)

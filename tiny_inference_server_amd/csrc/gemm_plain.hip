@@ -75,15 +75,22 @@ __global__ __launch_bounds__(GP_THREADS) void gemm_plain_kernel(const TI* __rest
 // 100 rows 1536 x 4096 436 / 74.
 static constexpr int GS_BM = 16, GS_BN = 16, GS_BK = 256, GS_LD = GS_BK + 4;
 
-template <bool VEC, typename TI, typename TO>
+// NORM: A's rows are RMS-normed on the way in, x * sqrt(K) / (||x|| + eps) * gain with the sum of squares added up in the order of the
+// norm's own kernel (256 threads a row, four waves); GATE: C has N / 2 columns, silu(g) u of the columns' pairs (2j, 2j + 1). Both give the
+// bits of the separate kernels. What they save is those kernels' launches, 3 us each where a step is nothing but launches; every column tile
+// sums its 16 rows' squares again, which its first loads hide up to a thousand columns.
+template <bool VEC, typename TI, typename TO, bool NORM = false, bool GATE = false>
 __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI* __restrict__ A, long lda, const TI* __restrict__ W,
                                                                    long ldw, const TO* __restrict__ R, long ldr,
-                                                                   TO* __restrict__ C, long ldc, int M, int N, int K) {
+                                                                   TO* __restrict__ C, long ldc, int M, int N, int K,
+                                                                   const float* __restrict__ gain, float eps) {
+  static_assert(!NORM || (VEC && sizeof(TI) == 4), "normed rows are 32-bit and read 16 bytes at a time");
   constexpr int THREADS = GS_BM * GS_BN, ROWS = GS_BN + GS_BM, PER = ROWS * (GS_BK / 4) / THREADS;   // groups of four a thread copies
   __shared__ __attribute__((aligned(16))) float lds[2][ROWS][GS_LD];                           // W's rows, then A's
   const int t = threadIdx.x, tx = t % GS_BN, ty = t / GS_BN;
   const long m0 = (long)blockIdx.y * GS_BM, n0 = (long)blockIdx.x * GS_BN;
-  float4 held[PER];
+  __shared__ float row_mul[NORM ? GS_BM : 1];
+  float4 held[PER], held_gain[NORM ? PER : 1];
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -95,6 +102,8 @@ __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI*
       held[i] = make_float4(0.f, 0.f, 0.f, 0.f);
       if constexpr (VEC && sizeof(TI) == 4) {
         if (ok && k0 + at * 4 < K) held[i] = *reinterpret_cast<const float4*>(src + k0 + at * 4);
+        if constexpr (NORM)
+          held_gain[i] = !is_w && k0 + at * 4 < K ? *reinterpret_cast<const float4*>(gain + k0 + at * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
       } else {               // elements at, at + 64, ...: neighbouring threads read neighbours
         float* h = reinterpret_cast<float*>(&held[i]);
 #pragma unroll
@@ -110,6 +119,13 @@ __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI*
     for (int i = 0; i < PER; ++i) {
       const int row = (i * THREADS + t) / (GS_BK / 4), at = (i * THREADS + t) % (GS_BK / 4);
       if constexpr (VEC && sizeof(TI) == 4) {
+        if constexpr (NORM) {
+          if (row >= GS_BN) {
+            const float mul = row_mul[row - GS_BN];
+            held[i] = make_float4(held[i].x * mul * held_gain[i].x, held[i].y * mul * held_gain[i].y, held[i].z * mul * held_gain[i].z,
+                                  held[i].w * mul * held_gain[i].w);
+          }
+        }
         *reinterpret_cast<float4*>(&lds[buf][row][at * 4]) = held[i];
       } else {
         const float* h = reinterpret_cast<const float*>(&held[i]);
@@ -124,6 +140,30 @@ __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI*
   if (R && live) res = to_f(R[m * ldr + n]);
   float acc = 0.f;
   fetch(0);
+  if constexpr (NORM) {
+    const int lane = t % TIS_WAVE, wave = t / TIS_WAVE;
+    float ss[4][4];                                      // a wave's four rows, and the four waves that would share each
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const long row = m0 + wave * 4 + r;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        ss[r][v] = 0.f;
+        for (int k = v * TIS_WAVE + lane; k < K; k += 4 * TIS_WAVE) {
+          const float x = row < M ? to_f(A[row * lda + k]) : 0.f;
+          ss[r][v] += x * x;
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float sum = 0.f;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sum += wave_sum(ss[r][v]);
+      if (lane == 0) row_mul[wave * 4 + r] = sqrtf((float)K) / (sqrtf(sum) + eps);
+    }
+    __syncthreads();
+  }
   commit(0);
   __syncthreads();
   int buf = 0;
@@ -146,7 +186,12 @@ __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI*
     if (more) commit(buf ^ 1);
     __syncthreads();
   }
-  if (live) C[m * ldc + n] = from_f<TO>(R ? acc + res : acc);
+  if constexpr (GATE) {
+    const float u = __shfl_xor(acc, 1, TIS_WAVE);        // the odd column beside this one
+    if (live && n % 2 == 0) C[m * ldc + n / 2] = from_f<TO>(acc / (1.f + expf(-acc)) * u);
+  } else if (live) {
+    C[m * ldc + n] = from_f<TO>(R ? acc + res : acc);
+  }
 }
 
 // Whether a product of M rows takes the tiles of 16 x 16; wide: its rows are read 16 bytes at a time. What counts is how many tiles of 64 x 64
@@ -170,7 +215,7 @@ static void launch_plain(const void* A, long lda, const void* W, long ldw, const
   if (tis_gemm_plain_few(vec, M, N, K)) {
     const dim3 grid((N + GS_BN - 1) / GS_BN, (M + GS_BM - 1) / GS_BM);
     const auto kernel = vec ? gemm_plain_few_kernel<true, TI, TO> : gemm_plain_few_kernel<false, TI, TO>;
-    kernel<<<grid, GS_BM * GS_BN, 0, stream>>>((const TI*)A, lda, (const TI*)W, ldw, (const TO*)R, ldr, (TO*)C, ldc, M, N, K);
+    kernel<<<grid, GS_BM * GS_BN, 0, stream>>>((const TI*)A, lda, (const TI*)W, ldw, (const TO*)R, ldr, (TO*)C, ldc, M, N, K, nullptr, 0.f);
     return;
   }
   const dim3 grid((N + GP_BN - 1) / GP_BN, (M + GP_BM - 1) / GP_BM);
@@ -193,4 +238,28 @@ TIS_EXPORT int tis_gemm_plain(int in_dtype, int out_dtype, const void* A, long l
   else
     return tis_fail("gemm: unsupported dtype pair in=%d out=%d", in_dtype, out_dtype);
   return tis_launch_status("gemm_plain");
+}
+
+// The product of 32-bit rows with the norm before it and the gate behind it (see the kernel): whether it takes M rows of K values against N
+// columns. us, norm, product and gate apart / fused, in a captured step: see the test's sizes; beyond 1,024 columns the sums of squares show.
+TIS_EXPORT int tis_gemm_plain_fuses(int M, int N, int K) {
+  return M > 0 && N > 0 && K > 0 && K % 4 == 0 && K <= 1024 && tis_gemm_plain_few(1, M, N, K) && (M + GS_BM - 1) / GS_BM <= 65535;
+}
+
+// gain: null, or the norm's gain [K] (eps is added to the norm); gate: C has N / 2 columns. A, W and gain start on 16 bytes, lda and ldw in steps of 4.
+TIS_EXPORT int tis_gemm_plain_fused(const float* A, long lda, const float* gain, float eps, const float* W, long ldw, const float* R, long ldr,
+                                    float* C, long ldc, int M, int N, int K, int gate, hipStream_t stream) {
+  if (M == 0 || N == 0) return 0;
+  if (!tis_gemm_plain_fuses(M, N, K)) return tis_fail("gemm: no fused product of M=%d N=%d K=%d", M, N, K);
+  if (lda % 4 || ldw % 4 || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)gain) % 16) return tis_fail("gemm: a fused product's rows start on 16 bytes");
+  if (gate && (R || N % 2)) return tis_fail("gemm: a gate goes with pairs of columns and no residual");
+  const dim3 grid((N + GS_BN - 1) / GS_BN, (M + GS_BM - 1) / GS_BM);
+#define FUSED(NORM, GATE) gemm_plain_few_kernel<true, float, float, NORM, GATE><<<grid, GS_BM * GS_BN, 0, stream>>>( \
+    A, lda, W, ldw, R, ldr, C, ldc, M, N, K, gain, eps)
+  if (gain && gate) FUSED(true, true);
+  else if (gain) FUSED(true, false);
+  else if (gate) FUSED(false, true);
+  else FUSED(false, false);
+#undef FUSED
+  return tis_launch_status("gemm_plain_fused");
 }

@@ -77,6 +77,7 @@ _SIGNATURES = {
     }),
     "gemm_plain": ("tis_gemm_plain", {
         "tis_gemm_plain": [_I, _I, _P, _L, _P, _L, _P, _L, _P, _L, _I, _I, _I, _P],
+        "tis_gemm_plain_fused": [_P, _L, _P, _F, _P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _P],
     }),
     "sampling": ("tis_sampling", {
         "tis_sample": [_P, _L, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _P, _P],
@@ -856,6 +857,8 @@ class HipOps:
             if rms[0].numel() != K or not rms[0].is_contiguous():
                 raise KernelError(f"linear: norm gain has {rms[0].numel()} entries for width {K}")
         if self.dtype == torch.float32:
+            if rms is not None and self._plain_fuses(x, w, rms):
+                return self._linear_plain_fused(x, w, rms, residual, self.empty(M, N), 0)
             if rms is not None:
                 x = self.rmsnorm(x, rms[0], rms[1])
             out = self.empty(M, N, dtype=torch.float32)
@@ -885,6 +888,19 @@ class HipOps:
         self.gemm_plain.tis_gemm_plain(1, _DT[out_dtype], _ptr(x), x.stride(0), _ptr(w), K, _ptr(residual),
                                        residual.stride(0) if residual is not None else 0, _ptr(out), out.stride(0), M, N,
                                        K, self._stream())
+        return out
+
+    def _plain_fuses(self, x, w, rms):
+        """Whether the 32-bit product of few rows takes the norm before it and a gate behind it into its own kernel."""
+        return (x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+                and (rms is None or rms[0].data_ptr() % 16 == 0)
+                and bool(self.gemm_plain.cdll.tis_gemm_plain_fuses(x.shape[0], w.shape[0], x.shape[1])))
+
+    def _linear_plain_fused(self, x, w, rms, residual, out, gate):
+        (M, K), N = x.shape, w.shape[0]
+        self.gemm_plain.tis_gemm_plain_fused(_ptr(x), x.stride(0), _ptr(rms[0] if rms else None), float(rms[1]) if rms else 0.0, _ptr(w), K,
+                                             _ptr(residual), residual.stride(0) if residual is not None else 0, _ptr(out), out.stride(0),
+                                             M, N, K, gate, self._stream())
         return out
 
     def _tiles_at_any_width(self, x, M, N, K, residual=None):
@@ -957,6 +973,12 @@ class HipOps:
             if rms is not None:
                 x = self.rmsnorm(x, rms[0], rms[1])
             return self._linear_tiles(x, w, None, self.empty(M, w.shape[0] // 2), w.shape[0], 0, 4)
+        if self.dtype == torch.float32 and w.dim() == 2 and w.shape[0] % 2 == 0 and w.shape[1] == K and w.is_contiguous() \
+                and (rms is None or (rms[0].numel() == K and rms[0].is_contiguous())) and self._plain_fuses(x, w, rms):
+            self._check(w, "linear w")
+            if rms is not None:
+                self._check(rms[0], "rmsnorm gain", torch.float32)
+            return self._linear_plain_fused(x, w, rms, None, self.empty(M, w.shape[0] // 2), 1)
         return self.swiglu(self.linear(x, w, rms=rms))
 
     # activations that a bfloat16 product applies to its 32-bit sums: (few-row kernel's epilogue, tiled kernel's code)
