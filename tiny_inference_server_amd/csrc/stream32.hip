@@ -808,13 +808,16 @@ TIS_EXPORT int tis_softcap(float* z, long ldz, float cap, int rows, int W, hipSt
 // term, and 5 rows of 512 channels were two workgroups). k in rising order for every row, whatever RT. us before / now, rank 64: 5 rows
 // x 1,024 7.0 / 4.3, 64 x 1,024 8.5 / 4.4, 1,531 x 1,024 15.4 / 12.4, 1,531 x 2,048 25.0 / 22.4.
 static constexpr int LR_COLS = 32, LR_BY = S32_THREADS / LR_COLS;
-template <int RT, int LR_K>
+template <int RT, int LR_K, int V>
 __global__ __launch_bounds__(S32_THREADS) void lowrank_act_kernel(const float* __restrict__ low, long ldl, int rank,
                                                                    const float* __restrict__ w2,
                                                                    const float* __restrict__ bias, int kind, float tau,
                                                                    const float* __restrict__ rate, int group,
                                                                    float* __restrict__ out, int rows, int C, int col_blocks) {
   __shared__ __attribute__((aligned(16))) float w[LR_COLS][LR_K + 4], a[LR_BY * RT][LR_K];
+  typedef __attribute__((ext_vector_type(V))) float floats;
+  constexpr int LINE = LR_K / V, WS = LR_COLS * LINE, AS = LR_BY * RT * LINE;      // pieces a line, of w's tile and of a's
+  constexpr int WN = (WS + S32_THREADS - 1) / S32_THREADS, AN = (AS + S32_THREADS - 1) / S32_THREADS;
   // grid (blocks of rows * blocks of channels, a row block's side by side)
   const long r0 = (long)(blockIdx.x / col_blocks) * (LR_BY * RT);
   const int n = (int)min((long)LR_BY * RT, rows - r0);
@@ -825,16 +828,30 @@ __global__ __launch_bounds__(S32_THREADS) void lowrank_act_kernel(const float* _
 #pragma unroll
   for (int i = 0; i < RT; ++i) z[i] = 0.f;
   for (int k0 = 0; k0 < rank; k0 += LR_K) {
-    if (k0) __syncthreads();
+    // all of a chunk's loads at once, from addresses that always hold something (a load under a condition is waited for before the next)
+    floats hw[WN], ha[AN];
 #pragma unroll
-    for (int i = threadIdx.x; i < LR_COLS * LR_K; i += S32_THREADS) {
-      const int row = i / LR_K, k = i % LR_K;
-      w[row][k] = c0 + row < C && k0 + k < rank ? w2[(long)(c0 + row) * rank + k0 + k] : 0.f;
+    for (int i = 0; i < WN; ++i) {
+      const int at = i * S32_THREADS + threadIdx.x, row = c0 + at / LINE, k = k0 + at % LINE * V;
+      hw[i] = *reinterpret_cast<const floats*>(w2 + (long)min(row, C - 1) * rank + min(k, rank - V));
+      if (row >= C || k >= rank) hw[i] = (floats)0.f;
     }
 #pragma unroll
-    for (int i = threadIdx.x; i < LR_BY * RT * LR_K; i += S32_THREADS) {
-      const int row = i / LR_K, k = i % LR_K;
-      a[row][k] = row < n && k0 + k < rank ? low[(r0 + row) * ldl + k0 + k] : 0.f;
+    for (int i = 0; i < AN; ++i) {
+      const int at = i * S32_THREADS + threadIdx.x, row = at / LINE, k = k0 + at % LINE * V;
+      ha[i] = *reinterpret_cast<const floats*>(low + (r0 + min(row, n - 1)) * ldl + min(k, rank - V));
+      if (row >= n || k >= rank) ha[i] = (floats)0.f;
+    }
+    if (k0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < WN; ++i) {
+      const int at = i * S32_THREADS + threadIdx.x;
+      if (WS % S32_THREADS == 0 || at < WS) *reinterpret_cast<floats*>(&w[at / LINE][at % LINE * V]) = hw[i];
+    }
+#pragma unroll
+    for (int i = 0; i < AN; ++i) {
+      const int at = i * S32_THREADS + threadIdx.x;
+      if (AS % S32_THREADS == 0 || at < AS) *reinterpret_cast<floats*>(&a[at / LINE][at % LINE * V]) = ha[i];
     }
     __syncthreads();
     const int kc = min(LR_K, rank - k0);
@@ -869,9 +886,11 @@ static void launch_lowrank(const float* low, long ldl, int rank, const float* w2
   const long small = ((long)rows + LR_BY - 1) / LR_BY * col_blocks;
   const bool few = small <= (rank > 32 ? 2048 : 1024);
   const long blocks = few ? small : ((long)rows + 4 * LR_BY - 1) / (4 * LR_BY) * col_blocks;
-#define LOWRANK(RT, K) \
-  lowrank_act_kernel<RT, K><<<blocks, S32_THREADS, 0, stream>>>(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, col_blocks)
-#define LOWRANK_BY_ROWS(K) { if (few) LOWRANK(1, K); else LOWRANK(4, K); }
+  // lines that start on 16 bytes are read 16 at a time
+  const bool fours = rank % 4 == 0 && ldl % 4 == 0 && ((uintptr_t)low | (uintptr_t)w2) % 16 == 0;
+#define LOWRANK(RT, K, V) \
+  lowrank_act_kernel<RT, K, V><<<blocks, S32_THREADS, 0, stream>>>(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, col_blocks)
+#define LOWRANK_BY_ROWS(K) { if (fours) { if (few) LOWRANK(1, K, 4); else LOWRANK(4, K, 4); } else { if (few) LOWRANK(1, K, 1); else LOWRANK(4, K, 1); } }
   if (rank <= 16) LOWRANK_BY_ROWS(16)
   else if (rank <= 32) LOWRANK_BY_ROWS(32)
   else LOWRANK_BY_ROWS(64)
