@@ -45,6 +45,17 @@ class StepOutput:
     head_valid: Optional[List[List[bool]]]
 
 
+@dataclass
+class _Following:
+    """The step after a replayed one of single tokens, as it will be if the same requests come again in the same order: all that it does
+    not bring itself is worked out while the GPU runs the one before."""
+    graph: object
+    rids: List[Hashable]
+    slots: List[int]
+    starts: List[int]
+    opening: Dict[int, int]          # slot -> positions it must hold, of the requests whose next position opens a page
+
+
 class Engine:
     def __init__(self, model_dir: Optional[str] = None, *, config=None, tensors=None, dtype="bfloat16",
                  page_size: int = 16, max_tokens: Optional[int] = None, n_pages: Optional[int] = None,
@@ -114,6 +125,8 @@ class Engine:
         self.max_graphs = 32
         self.max_decode_graphs = 192
         self._graph_seen: Dict[Tuple[int, int], int] = {}
+        # after a replayed step of single tokens: the step that its captured graph's buffer is filled for already
+        self._following: Optional[_Following] = None
         self._has_windows = any(g.spec.window > 0 for g in self.cache.groups.values())
         self.graph_replays = 0
 
@@ -121,12 +134,14 @@ class Engine:
     def open(self, rid: Hashable) -> None:
         if rid in self.requests:
             raise ValueError(f"request {rid!r} is already live")
+        self._following = None
         slot = self.cache.open_request()
         self._admissions += 1
         self._slot_admission[slot] = self._admissions
         self.requests[rid] = (slot, 0)
 
     def close(self, rid: Hashable) -> None:
+        self._following = None
         slot, _ = self.requests.pop(rid)
         self._slot_admission.pop(slot, None)
         self.cache.close_request(slot)
@@ -137,6 +152,7 @@ class Engine:
     def reserve(self, rid: Hashable, n_tokens: int) -> None:
         """Take now every page that `rid` needs to hold `n_tokens` positions (opening it if it is not live), the way
         the reference's static storage modes do at admission (server.py:163-166). All or nothing: OutOfPages."""
+        self._following = None           # (a request that has pages in hand is planned anew)
         opened = rid not in self.requests
         if opened:
             self.open(rid)
@@ -183,10 +199,55 @@ class Engine:
         """
         if not entries:
             raise ValueError("a step needs at least one entry")
+        following, self._following = self._following, None
+        if following is not None and not heads:
+            tokens = self._tokens_of(following, entries)
+            if tokens is not None:
+                return self._run_following(following, tokens)
         batch_entries = self._single_token_entries(entries)
         if batch_entries is None:
             batch_entries = self._checked_entries(entries)
         return self._run(entries, batch_entries, heads)
+
+    def _tokens_of(self, f: "_Following", entries):
+        """The entries' tokens if they are the step that was prepared, its pages taken; None, with nothing changed, for any other step
+        (and for whatever is wrong with this one: the general path says what)."""
+        if len(entries) != len(f.rids):
+            return None
+        vocab, tokens = self.spec.vocab_size, []
+        for (rid, toks, want), expected in zip(entries, f.rids):
+            if rid != expected or len(toks) != 1 or len(want) != 1 or want[0] != 0:
+                return None
+            t = toks[0]
+            if not isinstance(t, (int, np.integer)) or not (0 <= t < vocab):
+                return None
+            tokens.append(t)
+        if f.opening:
+            if any(len(self.cache.groups[g].tables[slot]) >= width for g, (_, (_, width)) in f.graph.table_at.items() for slot in f.opening):
+                return None              # a block table outgrows the captured width
+            if not self.cache.can_grow(f.opening):
+                return None
+            for slot, n in f.opening.items():
+                self.cache.grow(slot, n)
+        return tokens
+
+    def _run_following(self, f: "_Following", tokens):
+        self.graph_replays += 1
+        logits = f.graph.run_ahead(tokens)[:len(tokens)]
+        for rid, slot, start in zip(f.rids, f.slots, f.starts):
+            self.requests[rid] = (slot, start + 1)
+            if self._has_windows:
+                self.cache.release_behind(slot, start + 1, self.model.max_lag)
+        self._prepare_following(f.graph, f.rids, f.slots, [s + 1 for s in f.starts])
+        return StepOutput(logits, None, None)
+
+    def _prepare_following(self, graph, rids, slots, starts) -> None:
+        """While the GPU runs a replayed step: what the next one is, if its graph serves it too (see _decode_step, whose conditions these are)."""
+        if graph._ahead is None or max(starts) >= self.spec.max_context:
+            return
+        if self.model.plan_mode([(i, s, 1) for i, s in enumerate(starts)]) != graph.mode:      # (the filling lines have no say in it)
+            return
+        self._following = _Following(graph, rids, slots, starts, {slot: s + 1 for slot, s in zip(slots, starts) if s % self.page_size == 0})
 
     def _single_token_entries(self, entries):
         """The step that serving is mostly made of: one token for each of some live requests. Returns its batch
@@ -258,10 +319,10 @@ class Engine:
         return batch_entries
 
     def _run(self, entries, batch_entries, heads):
-        logits = plan = None
+        logits = plan = replayed = None
         if self.use_decode_graphs and not heads:
             if all(len(e.tokens) == 1 and e.start >= self.model.max_lag and list(e.want) == [0] for e in batch_entries):
-                logits = self._decode_step(batch_entries)
+                logits, replayed = self._decode_step(batch_entries)
             elif self.use_graphs:
                 logits, plan = self._repeated_step(batch_entries)
         if logits is None:
@@ -285,6 +346,8 @@ class Engine:
             self.requests[rid] = (e.slot, fed)
             if windows:
                 self.cache.release_behind(e.slot, fed, self.model.max_lag)
+        if replayed is not None:
+            self._prepare_following(replayed, [rid for rid, _, _ in entries], [e.slot for e in batch_entries], [e.start + 1 for e in batch_entries])
         return StepOutput(logits, head_logits, head_valid)
 
     def _sync(self):
@@ -333,7 +396,8 @@ class Engine:
         return graph.run(plan), plan
 
     def _decode_step(self, batch_entries):
-        """A step of single tokens through a captured graph: logits [requests, vocab], valid until the next step."""
+        """A step of single tokens through a captured graph: (logits [requests, vocab], valid until the next step; the graph, if its buffer
+        has been filled for the next step already)."""
         from .graph import DecodeGraph
         pages = max((max(len(g.tables[e.slot]) for e in batch_entries) for g in self.cache.groups.values()), default=1)
         width = -(-pages // self.graph_table_pages) * self.graph_table_pages
@@ -354,7 +418,7 @@ class Engine:
                 if e.start + 1 > self.spec.max_context:
                     raise ValueError(f"request in slot {e.slot} would pass the model's context of {self.spec.max_context}")
             self.graph_replays += 1
-            return graph.run_same_requests(batch_entries)[:n_real]
+            return graph.run_same_requests(batch_entries)[:n_real], graph
         plan = plan_step_batch(batch_entries, self.model.lags, self.model.reads_previous, self.cache,
                                self.spec.max_context, self.model.plan_rows, table_width=width, mode=mode)
         if graph is None:
@@ -367,9 +431,9 @@ class Engine:
                 for st in step.stages:
                     st.max_kv_len = width * self.page_size
                 outs = self.model.forward(step, self.cache)
-                return self.model.logits(outs[0].hidden, step.stages[0].want_index, len(batch_entries))[:n_real]
+                return self.model.logits(outs[0].hidden, step.stages[0].want_index, len(batch_entries))[:n_real], None
             self._make_room(lambda k: k[0] != "step", self.max_decode_graphs)
             graph = self._graphs[key] = DecodeGraph(self, plan, width * self.page_size, occupants,
                                                     capture=self._capture_graphs, mode=mode)
         self.graph_replays += 1
-        return graph.run(plan, occupants)[:n_real]
+        return graph.run(plan, occupants)[:n_real], None

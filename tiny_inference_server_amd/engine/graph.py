@@ -50,6 +50,7 @@ class DecodeGraph:
         self.host = torch.zeros(max(plan.packer.total, 4), dtype=torch.int32, pin_memory=on_gpu)
         self.dev = torch.zeros(max(plan.packer.total, 4), dtype=torch.int32, device=dev)
         self.copied = torch.cuda.Event() if on_gpu else _NoEvent()
+        self.flat = self.host.numpy()
         self.step = materialize(plan, dev, self.host, self.dev)
         for st in self.step.stages:          # later steps of the shape may see more keys than this one
             st.max_kv_len = kv_capacity
@@ -113,7 +114,7 @@ class DecodeGraph:
         step; when it comes, only its tokens, and the lines of requests that have taken a page since, are left to
         write before the copy and the replay."""
         self.copied.synchronize()
-        flat = self.host.numpy()
+        flat = self.flat
         n = len(entries)
         starts = np.fromiter((e.start for e in entries), dtype=np.int64, count=n)
         tokens = np.fromiter((e.tokens[0] for e in entries), dtype=np.int32, count=n)
@@ -123,6 +124,19 @@ class DecodeGraph:
                 self._fill_positions(flat, starts, only=ahead[1])
         else:
             self._fill_positions(flat, starts)
+        return self._run_filled(starts, tokens)
+
+    def run_ahead(self, tokens) -> torch.Tensor:
+        """The step that the buffer was filled for ahead of time, with its requests' tokens (lines that fill the step up keep theirs):
+        run_same_requests for a caller that knows which step this is."""
+        starts, late = self._ahead
+        self._ahead = None
+        if len(late):
+            self._fill_positions(self.flat, starts, only=late)
+        return self._run_filled(starts, tokens)
+
+    def _run_filled(self, starts, tokens) -> torch.Tensor:
+        flat, n = self.flat, len(tokens)
         for st in self.stage_at:
             flat[st["tokens"]:st["tokens"] + n] = tokens
         self.dev.copy_(self.host, non_blocking=True)
@@ -132,7 +146,7 @@ class DecodeGraph:
         self.copied.synchronize()
         nxt = starts + 1
         if self.cache.spare_slot is not None:       # (lines that fill the step up stay where they are)
-            nxt = nxt - np.fromiter((s == self.cache.spare_slot for s in self.slots), dtype=np.int64, count=n)
+            nxt = nxt - np.fromiter((s == self.cache.spare_slot for s in self.slots), dtype=np.int64, count=len(starts))
         self._ahead = (nxt, self._fill_positions(flat, nxt, ahead=True))
         return self.logits
 
