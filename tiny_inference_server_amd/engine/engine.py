@@ -320,7 +320,16 @@ class Engine:
 
     def _run(self, entries, batch_entries, heads):
         logits = plan = replayed = None
-        if self.use_decode_graphs and not heads:
+        head_logits = head_valid = None
+        stages = len(self.model.lags)
+        if self.use_decode_graphs and heads:
+            # (single tokens with every stage's logits are launched as they come)
+            if self.use_graphs and stages > 1 and any(len(e.tokens) > 1 for e in batch_entries):
+                logits, plan = self._repeated_step(batch_entries, heads=True)
+                if logits is not None:       # in memory of their own: who asks for the heads' logits may keep them
+                    logits, head_logits, head_valid = self.model.by_stage(logits.clone(), [pl["valid"] for pl in plan.plans],
+                                                                          sum(len(e.want) for e in batch_entries))
+        elif self.use_decode_graphs:
             if all(len(e.tokens) == 1 and e.start >= self.model.max_lag and list(e.want) == [0] for e in batch_entries):
                 logits, replayed = self._decode_step(batch_entries)
             elif self.use_graphs:
@@ -334,9 +343,8 @@ class Engine:
                                         mode=self.model.plan_mode(first_stage_rows(batch_entries)))
             outs = self.model.forward(step, self.cache)
         n = sum(len(e.want) for e in batch_entries)
-        head_logits = head_valid = None
         if logits is None:
-            if heads and len(outs) > 1:
+            if heads and stages > 1:
                 logits, head_logits, head_valid = self.model.logits_of_stages(outs, n)
             else:
                 logits = self.logits_of(outs, step, n)
@@ -367,7 +375,7 @@ class Engine:
             self._sync()              # no replay of the graph to be dropped is still running
             del self._graphs[keys.pop(0)]
 
-    def _repeated_step(self, batch_entries):
+    def _repeated_step(self, batch_entries, heads=False):
         """Any other step whose shape has come before: the same requests' row counts, the same places wanted, the
         same work for the attention kernels (a batch of equal prompts, a benchmark's prefill). Returns (logits or
         None, the step's plan); from its third occurrence on a shape is replayed from a captured graph."""
@@ -378,7 +386,7 @@ class Engine:
                                self.spec.max_context, self.model.plan_rows, table_width=width,
                                mode=self.model.plan_mode(first_stage_rows(batch_entries)))
         # what the host decides from, beyond the arrays' shapes
-        key = ("step", width, plan.layout(),
+        key = ("step", heads, width, plan.layout(),
                tuple((pl["max_rows"], pl["keep_count"], pl["previous_rows"], tuple(pl["valid"])) for pl in plan.plans))
         graph = self._graphs.get(key)
         if graph is None:
@@ -389,7 +397,7 @@ class Engine:
             if seen < 2:
                 return None, plan
             self._make_room(lambda k: k[0] == "step", self.max_graphs)
-            graph = self._graphs[key] = DecodeGraph(self, plan, width * self.page_size, capture=self._capture_graphs)
+            graph = self._graphs[key] = DecodeGraph(self, plan, width * self.page_size, capture=self._capture_graphs, heads=heads)
         else:
             self._graphs.move_to_end(key)
         self.graph_replays += 1

@@ -40,9 +40,10 @@ class DecodeGraph:
     operations object without a device (a test's stand-in) exercises this file's host logic.
     """
 
-    def __init__(self, engine, plan: StepPlan, kv_capacity: int, occupants=None, capture: bool = True, mode=None):
+    def __init__(self, engine, plan: StepPlan, kv_capacity: int, occupants=None, capture: bool = True, mode=None, heads: bool = False):
         self.layout = plan.layout()
         self.mode = mode
+        self.heads = heads       # every stage's logits, as the model's all_logits gives them
         self.engine = engine
         self.capture = capture
         dev = engine.device
@@ -92,7 +93,7 @@ class DecodeGraph:
     def _launch(self):
         engine, n = self.engine, self.step.n_wanted
         outs = engine.model.forward(self.step, engine.cache)
-        self.logits = engine.logits_of(outs, self.step, n)
+        self.logits = engine.model.all_logits(outs, n) if self.heads else engine.logits_of(outs, self.step, n)
 
     def _replay(self):
         if self.graph is not None:

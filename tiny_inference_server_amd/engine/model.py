@@ -184,26 +184,30 @@ class Model:
         rows that a later stage does not have yet come back as NaN. The first stage's part is what `logits` gives: the
         same gather and the same product on the same rows (up to the order of 32-bit partial sums, which the product
         may choose by the number of rows)."""
-        vocab, S = self.spec.vocab_size, len(outs)
+        return self.by_stage(self.all_logits(outs, n), [o.batch.want_valid for o in outs], n)
+
+    def all_logits(self, outs, n):
+        """The product behind logits_of_stages, [stages * n, vocab]: launches only, whatever stands in rows that a stage does not have."""
+        S = len(outs)
         if n == 0:
-            e = torch.empty(0, vocab, dtype=torch.float32, device=self.ops.device)
-            return e, [e.clone() for _ in outs[1:]], [[] for _ in outs[1:]]
+            return torch.empty(0, self.spec.vocab_size, dtype=torch.float32, device=self.ops.device)
         rows = self.ops.empty(S * n, self.spec.d_model)
-        valid = []
         for j, o in enumerate(outs):
-            v = [True] * n if j == 0 else list(o.batch.want_valid)
             part = rows[j * n:(j + 1) * n]
-            if o.batch.n_rows and any(v):
+            if o.batch.n_rows and (j == 0 or any(o.batch.want_valid)):
                 idx = o.batch.want_index[:n] if j == 0 else torch.clamp(o.batch.want_index[:n], min=0)
                 self._wanted_rows(o.hidden, idx, n, out=part)
             else:
                 part.zero_()
-            valid.append(v)
-        lg = self._project(rows).view(S, n, vocab)
-        later = []
+        return self._project(rows)
+
+    def by_stage(self, logits, valid, n):
+        """What logits_of_stages returns, from all_logits' product and the stages' valid rows (of the first all are)."""
+        S = len(valid)
+        if n == 0:
+            return logits, [logits.clone() for _ in range(S - 1)], [[] for _ in range(S - 1)]
+        lg = logits.view(S, n, self.spec.vocab_size)
         for j in range(1, S):
-            h = lg[j]
             if not all(valid[j]):
-                h[~torch.tensor(valid[j], device=self.ops.device)] = float("nan")
-            later.append(h)
-        return lg[0], later, valid[1:]
+                lg[j][~torch.tensor(valid[j], device=self.ops.device)] = float("nan")
+        return lg[0], [lg[j] for j in range(1, S)], [list(v) for v in valid[1:]]
