@@ -259,27 +259,56 @@ __global__ __launch_bounds__(256) void grouped_mfma_kernel(const bf16* __restric
 #pragma unroll
     for (int j = 0; j < RN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  // U steps of 32 at a time: all their loads are issued before the first product, so that a wave keeps several
-  // steps' worth of requests in flight (the products of one step take far less time than its operands' way here)
-  constexpr int U = 4;
-  for (int k0 = 0; k0 < p.K; k0 += 32 * U) {
-    bf16x8 av[U][RM], wv[U][RN];
+  // A batch is U steps of 32; SETS batches of operands, so that while one is multiplied the next are on their way. A whole batch is read
+  // without a condition: lanes without an entry or a column read the group's first, and nobody looks at what becomes of it. What bounds a few
+  // entries a group is the matrices' way from memory, of which a wave saw 16 trips one after the other. 8 groups, two choices a row, us, one set and
+  // loads under conditions / two sets / three: 8 rows, 5,632 of 2,048 44 / 41 / 40, 2,048 of 2,816 25.0 / 19.6 / 20.1; 5 rows 2,816 of 1,024
+  // 12.4 / 12.8 / 12.9, 1,024 of 1,408 12.7 / 10.1 / 10.0; 1 row 5,632 of 2,048 18.4 / 14.7 / 15.1. (161 MB in 41 us: 4 TB/s.)
+  constexpr int U = 4, SETS = RM + RN <= 2 ? 2 : 1;
+  bf16x8 av[SETS][U][RM], wv[SETS][U][RN];
+  const int whole = p.K / (32 * U);
+  auto load = [&](int set, int b) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = k0 + u * 32;
-      const bool k_ok = k + kg * 8 < p.K;
+      const int k = (b * U + u) * 32;
 #pragma unroll
-      for (int i = 0; i < RM; ++i) av[u][i] = (mine[i] >= 0 && k_ok) ? *reinterpret_cast<const bf16x8*>(arow[i] + k) : zero;
+      for (int i = 0; i < RM; ++i) av[set][u][i] = *reinterpret_cast<const bf16x8*>(arow[i] + k);
 #pragma unroll
-      for (int j = 0; j < RN; ++j) wv[u][j] = (w_ok[j] && k_ok) ? *reinterpret_cast<const bf16x8*>(wrow[j] + k) : zero;
+      for (int j = 0; j < RN; ++j) wv[set][u][j] = *reinterpret_cast<const bf16x8*>(wrow[j] + k);
     }
+  };
+  auto multiply = [&](int set) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int i = 0; i < RM; ++i)
 #pragma unroll
         for (int j = 0; j < RN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u][j], av[u][i], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[set][u][j], av[set][u][i], acc[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int e = 0; e < SETS - 1; ++e)
+    if (e < whole) load(e, e);
+  for (int b0 = 0; b0 < whole; b0 += SETS) {
+#pragma unroll
+    for (int e = 0; e < SETS; ++e) {
+      const int b = b0 + e;
+      if (b >= whole) break;
+      if (b + SETS - 1 < whole) load((e + SETS - 1) % SETS, b + SETS - 1);
+      multiply(e);
+    }
+  }
+  if (whole * 32 * U < p.K) {                    // the last, begun batch: zeros past the end of K
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = (whole * U + u) * 32;
+      const bool k_ok = k + kg * 8 < p.K;
+#pragma unroll
+      for (int i = 0; i < RM; ++i) av[0][u][i] = k_ok ? *reinterpret_cast<const bf16x8*>(arow[i] + k) : zero;
+#pragma unroll
+      for (int j = 0; j < RN; ++j) wv[0][u][j] = k_ok ? *reinterpret_cast<const bf16x8*>(wrow[j] + k) : zero;
+    }
+    multiply(0);
   }
   // the lane holds, of tile (i, j), the columns n0 + 16 j + 4 kg + e of entry i * 16 + c16
 #pragma unroll
