@@ -298,13 +298,25 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
     }
   }
   if (first < 0) return;                         // the grid is as wide as there could be chunks
-  for (int e = t; e < DC * Dp; e += 256) {
-    const int r = e / Dp, d = e % Dp;
-    const long row = first + r;
+  // all of the chunk's loads at once, from addresses that always hold something (a load under a condition is waited for before the next;
+  // 1,531 rows of 8 heads of 128, us: 23 / 20)
+  constexpr int PER = DC * Dp / 256;
+  float hk[PER], hq4[PER], ha[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int e = t + 256 * j, r = e / Dp, d = min(e % Dp, D - 1);
+    const long row = first + min(r, n - 1);
+    hk[j] = u[row * ldu + k_off + hq * D + d];
+    hq4[j] = u[row * ldu + q_off + hq * D + d];
+    ha[j] = decay[row * ldd + h * D + d];
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int e = t + 256 * j, r = e / Dp, d = e % Dp;
     const bool ok = r < n && d < D;
-    k[r][d] = ok ? u[row * ldu + k_off + hq * D + d] : 0.f;
-    q[r][d] = ok ? u[row * ldu + q_off + hq * D + d] : 0.f;
-    a[r][d] = ok ? decay[row * ldd + h * D + d] : 1.f;
+    k[r][d] = ok ? hk[j] : 0.f;
+    q[r][d] = ok ? hq4[j] : 0.f;
+    a[r][d] = ok ? ha[j] : 1.f;
   }
   if (t < DC) beta[t] = t < n ? u[(long)(first + t) * ldu + beta_off + h] : 0.f;
   __syncthreads();
