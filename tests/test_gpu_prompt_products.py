@@ -41,7 +41,7 @@ def test_every_tile(ops, tile):
     assert torch.equal(gated, ops.swiglu(ops._linear_tiles(x, w, None, torch.empty(M, N, dtype=torch.bfloat16, device="cuda"), N, 0, 0)))
 
 
-@pytest.mark.parametrize("M", [129, 300, 1024, 1025])
+@pytest.mark.parametrize("M", [129, 300, 1024, 1025, 2048, 2049])
 def test_products_by_rows(ops, M):
     """Widths of the library's list and another: up to the limit the tiles, beyond it what linear takes. The same sums in the same order
     either way, so the same bits; a residual whose rows the library does not take, too."""

@@ -193,6 +193,10 @@ _TILES_UP_TO = 1024             # a model's own products of more rows than that,
                                 # 11,264 x 2,048 30 / 21, 37 / 27, 48 / 45, 58 / 57. At 1,532 and 2,048 rows the library is the faster:
                                 # 1,536 x 4,096 34 / 35, 35 / 36, 8,192 x 1,536 45 / 48, 53 / 56, 11,264 x 2,048 83 / 78, 96 / 100.
                                 # Both add a row's products up in the same order and give the same bits
+_TILES_NARROW = (2048, 3072, 2048)   # ... and up to (rows, columns, inner columns) of these the tiles go on: 2,304 x 1,536 at 1,280, 1,532, 1,800,
+                                # 2,048 rows 19 / 18, 19 / 19, 24 / 21, 24 / 22.5; 1,536 x 1,536 16 / 13, 17 / 17, 19 / 16, 18.5 / 17.5; 2,048 x 2,048
+                                # 22 / 21, 22 / 21, 24 / 22, 24 / 24; 3,072 x 2,048 25 / 23, 26 / 26, 31 / 28, 30 / 31 (the library's row count is
+                                # rounded up to 256); but 2,048 x 5,632 47 / 50, 45 / 50, and 3,000 rows of 3,072 x 2,048 38 / 49
 
 _WIDTHS_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "library_widths.json")
 
@@ -905,7 +909,9 @@ class HipOps:
 
     def _tiles_at_any_width(self, x, M, N, K, residual=None):
         """Whether a bfloat16 product of these rows runs on the tiled product whatever its widths (see _TILES_UP_TO)."""
-        return (self.dtype == torch.bfloat16 and self.few_rows < M <= _TILES_UP_TO and N % 4 == 0
+        rows, columns, inner = _TILES_NARROW
+        most = rows if N <= columns and K <= inner else _TILES_UP_TO
+        return (self.dtype == torch.bfloat16 and self.few_rows < M <= most and N % 4 == 0
                 and self._route(x, M, N, K, residual=residual) in ("library", "tiles")
                 and (residual is None or (residual.stride(0) % 4 == 0 and residual.data_ptr() % 8 == 0)))
 
