@@ -69,6 +69,8 @@ def test_what_is_wrong_with_a_step_is_said_as_ever():
     with pytest.raises(ValueError, match="twice"):
         eng.step([("a", [1], [0]), ("a", [2], [0])])
     assert eng.fed("a") == eng.fed("b") == 14
+    eng.step([("a", [1], iter([0])), ("b", [2], {0})])      # places wanted as anything that can be walked
+    assert eng.fed("a") == eng.fed("b") == 15
     eng.reserve("a", 40)                     # takes a page the step was not prepared for
     eng.step(one())
     with pytest.raises(OutOfPages):          # four pages in all: b cannot open its second and a third

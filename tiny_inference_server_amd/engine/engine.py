@@ -216,7 +216,7 @@ class Engine:
             return None
         vocab, tokens = self.spec.vocab_size, []
         for (rid, toks, want), expected in zip(entries, f.rids):
-            if rid != expected or len(toks) != 1 or len(want) != 1 or want[0] != 0:
+            if rid != expected or len(toks) != 1 or type(want) not in (list, tuple, range) or len(want) != 1 or want[0] != 0:
                 return None
             t = toks[0]
             if not isinstance(t, (int, np.integer)) or not (0 <= t < vocab):
