@@ -516,13 +516,13 @@ TIS_EXPORT void tis_experts_units(int n) { if (n > 0) g_units = n; }
 //   64 x 64, four waves, two buffers, five a unit      (not by this estimate: for products of few steps)
 //   128 x 64, eight waves, six buffers                 0.42 a round        (these three from ten steps on: what they gain is
 //   256 x 128, eight waves, three buffers              1.1 a round          in the steps, and their buffers take longer to fill)
-//   192 x 128, eight waves, four buffers               0.85 a round
-// us before the last three / with them, 8 groups, two choices a row: 1,531 rows, 5,632 of 2,048 126 / 106, 2,048 of 2,816 70 / 56; 1,000 rows
+//   192 x 128, eight waves, four buffers               0.95 a round
+// us before the last three / with them, 8 groups, two choices a row: 1,531 rows, 5,632 of 2,048 124 / 106, 2,048 of 2,816 70 / 56; 1,000 rows
 // 100 / 88, 60 / 44; 2,048 rows 1,024 of 1,408 37 / 29; 600 rows 2,816 of 1,024 27 / 22, 1,024 of 1,408 18 / 15. A result is the same sum in any tile.
 struct GroupedShape { int bm, bn; float step, least; bool rounds; };
 static const GroupedShape g_shapes[9] = {{128, 192, 1.05f, 1.15f, false}, {64, 64, 0.3f, 0.33f, false}, {128, 128, 0.58f, 0.58f, true},
                                          {256, 256, 1.85f, 1.85f, true}, {128, 128, 0.78f, 0.8f, false}, {64, 64, 0.f, 0.f, false},
-                                         {128, 64, 0.42f, 0.42f, true}, {256, 128, 1.1f, 1.1f, true}, {192, 128, 0.85f, 0.85f, true}};
+                                         {128, 64, 0.42f, 0.42f, true}, {256, 128, 1.1f, 1.1f, true}, {192, 128, 0.95f, 0.95f, true}};
 
 // The tile that a grouped product of bfloat16 rows that lie as it needs them takes, an index into g_shapes; -1: the products straight from memory.
 // lists: most_rows is the most entries a group can have, most_entries the most that all groups have together.
@@ -556,7 +556,16 @@ TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_
     const long tn = (N + q.bn - 1) / q.bn;
     // (with lists, entries / bm row tiles and half a tile more in every group)
     const float r = (lists ? (float)most_entries / q.bm + 0.5f * groups : (float)((long)groups * ((most_rows + q.bm - 1) / q.bm))) * tn / g_units;
-    const float t = fmaxf(q.least, q.step * (q.rounds ? ceilf(r) : r));
+    float t = fmaxf(q.least, q.step * (q.rounds ? ceilf(r) : r));
+    // from ten steps on, with more tiles than units: what a step takes then (us, 8 groups, two choices a row, 128 x 192 / 128 x 128 / 256 x 128 /
+    // 192 x 128: 1,531 rows, 5,632 of 2,048 122 / 124 / 106 / 125; 1,000 rows 110 / 99 / 82 / 88; 600 rows 64 / 70 / 77 / 72; 1,531 rows, 2,048 of 2,816
+    // 79 / 68 / 56 / 83)
+    if (K > 9 * 64 && r > 1.f) {
+      if (i == 0) t = r <= 2.f ? 1.83f : 0.4f + 1.2f * r;
+      else if (i == 2) t = 0.7f * ceilf(r);
+      else if (i == 4) t = fmaxf(1.15f * fminf(r, 2.3f), 0.85f * r);
+      else if (i == 8) t = ceilf(r);
+    }
     if (t < best) best = t, pick = i;
   }
   return pick;

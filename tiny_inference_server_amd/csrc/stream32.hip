@@ -806,7 +806,8 @@ TIS_EXPORT int tis_softcap(float* z, long ldz, float cap, int rows, int W, hipSt
 // A workgroup takes 32 channels and 8 RT rows, a thread one channel of RT of them, and both factors come through LDS in chunks of LR_K of
 // the rank, read in whole runs (a thread that walked its channel's line of w2 by itself touched a line of memory per lane and
 // term, and 5 rows of 512 channels were two workgroups). k in rising order for every row, whatever RT. us before / now, rank 64: 5 rows
-// x 1,024 7.0 / 4.3, 64 x 1,024 8.5 / 4.4, 1,531 x 1,024 15.4 / 12.4, 1,531 x 2,048 25.0 / 22.4.
+// x 1,024 7.0 / 4.3, 64 x 1,024 8.5 / 4.4, 1,531 x 1,024 15.4 / 12.4, 1,531 x 2,048 25.0 / 22.4; with all of a chunk's loads under way
+// together (before, each waited for the one before it), traced inside a pass, before / now: 5 rows 7.0 / 4.0, 1,531 rows, the two widths' mean, 20.1 / 13.1.
 static constexpr int LR_COLS = 32, LR_BY = S32_THREADS / LR_COLS;
 template <int RT, int LR_K, int V>
 __global__ __launch_bounds__(S32_THREADS) void lowrank_act_kernel(const float* __restrict__ low, long ldl, int rank,
