@@ -81,3 +81,24 @@ def test_what_is_wrong_with_a_step_is_said_as_ever():
     eng.step([("b", [3], [0])])
     assert eng.fed("b") == fed + 1
     eng.cache.check()
+
+
+def test_a_prepared_step_is_not_replayed_once_replays_are_switched_off():
+    """use_decode_graphs is read at every step, also at one that was prepared while it was still on."""
+    vocab = H.TINY["A"]["cfg"].vocab_size
+    folder, eng, taken = engine(1)
+    ids = H.random_ids(vocab, 20, 9)
+    eng.step([("a", ids[:10], [])])
+    for p in range(10, 14):
+        eng.step([("a", ids[p:p + 1], [0])])
+    assert eng._following is not None and taken
+    steps, replays = len(taken), eng.graph_replays
+    eng.use_decode_graphs = False
+    out = eng.step([("a", ids[14:15], [0])])
+    assert len(taken) == steps and eng.graph_replays == replays
+    want = H.plain_logits(folder, ids)[0][14]
+    assert (out.logits[0].double() - want).abs().max().item() <= 2e-5 * max(1.0, want.abs().max().item())
+    eng.use_decode_graphs = True
+    for p in range(15, 18):
+        eng.step([("a", ids[p:p + 1], [0])])
+    assert eng.graph_replays > replays and len(taken) > steps

@@ -200,7 +200,7 @@ class Engine:
         if not entries:
             raise ValueError("a step needs at least one entry")
         following, self._following = self._following, None
-        if following is not None and not heads:
+        if following is not None and self.use_decode_graphs and not heads:
             tokens = self._tokens_of(following, entries)
             if tokens is not None:
                 return self._run_following(following, tokens)
