@@ -40,3 +40,26 @@ def test_replayed_heads_are_what_a_launched_step_gives(name, dtype):
         for x, y in step:
             assert torch.equal(torch.isnan(x), torch.isnan(y))
             torch.testing.assert_close(torch.nan_to_num(x), torch.nan_to_num(y), rtol=0, atol=2e-2 if dtype == "bfloat16" else 2e-5)
+
+
+@pytest.mark.parametrize("name,dtype", [pytest.param("A", "float32", marks=pytest.mark.gpu), pytest.param("A", "float32-torch")])
+def test_no_graph_goes_on_holding_logits_of_many_places(name, dtype):
+    """Steps with the heads' logits whose logits pass max_heads_graph_bytes are launched however often their shape comes; one place fewer
+    is captured. Same logits either way."""
+    dtype, _, backend = dtype.partition("-")
+    folder = H.model_folder(name, dtype)
+    vocab = H.TINY[name]["cfg"].vocab_size
+    eng = Engine(folder, dtype=dtype, page_size=16, max_tokens=256, max_requests=1, ops=TorchOps(graphs=True) if backend else None)
+    ids = H.random_ids(vocab, 40, 3)
+    eng.max_heads_graph_bytes = 4 * (1 + eng.model.max_lag) * 39 * vocab
+    kept = []
+    for places in (40, 39):
+        for k in range(4):
+            before = eng.graph_replays
+            out = eng.step([("a", ids, list(range(40 - places, 40)))], heads=True)
+            eng.close("a")
+            kept.append([out.logits[-39:]] + [h[-39:] for h in out.head_logits])
+            assert (eng.graph_replays > before) == (places == 39 and k >= 2)
+    for step in kept[1:]:
+        for x, y in zip(step, kept[0]):
+            torch.testing.assert_close(torch.nan_to_num(x), torch.nan_to_num(y), rtol=0, atol=2e-5)

@@ -124,6 +124,10 @@ class Engine:
         # width, so many of them are kept; other steps (prompt portions) hold a portion's activations each.
         self.max_graphs = 32
         self.max_decode_graphs = 192
+        # A step with every stage's logits (a replay of texts with all their places wanted: 2,048 places of a stage are 393 MB
+        # at 48,000 outputs) is captured only up to this many bytes of them, which its graph would go on holding: beyond, the
+        # launches are a small part of the step, and its logits' memory goes back with them.
+        self.max_heads_graph_bytes = 32 << 20
         self._graph_seen: Dict[Tuple[int, int], int] = {}
         # after a replayed step of single tokens: the step that its captured graph's buffer is filled for already
         self._following: Optional[_Following] = None
@@ -324,7 +328,8 @@ class Engine:
         stages = len(self.model.lags)
         if self.use_decode_graphs and heads:
             # (single tokens with every stage's logits are launched as they come)
-            if self.use_graphs and stages > 1 and any(len(e.tokens) > 1 for e in batch_entries):
+            held = 4 * stages * sum(len(e.want) for e in batch_entries) * self.spec.vocab_size
+            if self.use_graphs and stages > 1 and held <= self.max_heads_graph_bytes and any(len(e.tokens) > 1 for e in batch_entries):
                 logits, plan = self._repeated_step(batch_entries, heads=True)
                 if logits is not None:       # in memory of their own: who asks for the heads' logits may keep them
                     logits, head_logits, head_valid = self.model.by_stage(logits.clone(), [pl["valid"] for pl in plan.plans],
