@@ -103,3 +103,30 @@ def test_norm_and_gate_inside_the_32_bit_product(M, N, K):
     assert torch.equal(ops.linear_swiglu(x, w, rms=rms), ops.swiglu(ops.linear(normed, w)))
     assert torch.equal(ops.linear_swiglu(x, w), ops.swiglu(ops.linear(x.contiguous(), w)))
     assert not ops.gemm_plain.cdll.tis_gemm_plain_fuses(M, N, 1028)
+
+
+@pytest.mark.parametrize("groups,rows,top,N,K", [(64, 40, 2, 96, 1024), (70, 127, 2, 520, 136), (33, 17, 3, 64, 2048), (2, 23, 2, 132, 40), (130, 100, 1, 48, 264)])
+def test_few_entries_in_many_groups(ops, groups, rows, top, N, K):
+    """The product straight from memory with lists of up to several tiles of 16 entries: groups without an entry, of one, and the first of many;
+    the sums against 64 bits, lines that no list names left alone."""
+    from ctypes import c_long
+    lib = ops._lazy("experts")
+    assert lib.cdll.tis_grouped_tile(1, groups, rows, c_long(rows * top), N, K, 0) == -1
+    g = torch.Generator().manual_seed(groups + rows)
+    x, w = rnd((rows, K), 51).cuda(), rnd((groups, N, K), 52, K ** -0.5).cuda()
+    lists, counts = torch.zeros(groups, rows, dtype=torch.int32), [0] * groups
+    group_of = torch.full((rows * top,), -1)
+    for e in range(rows * top):
+        if e == 5:
+            continue                                     # an entry of nobody
+        to = 0 if e % top == 0 and rows > 20 else int(torch.randint(0, groups, (1,), generator=g))
+        if counts[to] < rows:
+            lists[to, counts[to]], group_of[e] = e, to
+            counts[to] += 1
+    out = torch.full((rows * top, N), 7.0, device="cuda")
+    ops._grouped(x, x.stride(0), 0, top, w, out, N, 0, lists.cuda(), torch.tensor(counts, dtype=torch.int32, device="cuda"), rows, rows)
+    for e in range(rows * top):
+        if group_of[e] < 0:
+            assert bool((out[e] == 7.0).all())
+        else:
+            torch.testing.assert_close(out[e].double(), w[group_of[e]].double() @ x[e // top].double(), rtol=1e-4, atol=1e-4)

@@ -228,12 +228,16 @@ __global__ __launch_bounds__(256) void grouped_plain_kernel(const TA* __restrict
 // RM RN products, and what the waves of a workgroup share meets in the caches. Each result is one wave's sum over K in
 // steps of 32. Two shapes are built: 16 entries x 64 columns for groups of a few rows (decoded tokens: the job is to
 // stream the matrices once), 64 x 128 for groups of many that the tiles below do not take.
+// grid (blocks of columns, groups, tiles of entries): every group's first tile, then every group's second, most of which have no entries and
+// end at once. With a group's tiles behind one another the ones that work were every second, fourth .. workgroup, and those go to the same
+// compute units: 64 groups of 512 of 1,024, two choices a row, us, so / as it is: 17 rows 22 / 14, 40 21 / 14.5, 64 43 / 15, 127 47 / 16;
+// 8 groups of 5,632 of 2,048, 17 rows 52 / 43; 16 of 4,096 of 1,536, 24 rows 50 / 43.
 template <typename TO, int WM, int WN, int RM, int RN>
 __global__ __launch_bounds__(256) void grouped_mfma_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                            TO* __restrict__ C, GroupedArgs p) {
   static_assert(WM * WN == 4, "four waves a workgroup");
-  const int g = blockIdx.z, t = threadIdx.x, lane = t % 64, wave = t / 64;
-  const int m0 = blockIdx.y * (16 * RM * WM) + (wave / WN) * (16 * RM);
+  const int g = blockIdx.y, t = threadIdx.x, lane = t % 64, wave = t / 64;
+  const int m0 = blockIdx.z * (16 * RM * WM) + (wave / WN) * (16 * RM);
   const int n0 = blockIdx.x * (16 * RN * WN) + (wave % WN) * (16 * RN);
   const int count = p.lists ? p.counts[g] : p.rows;
   if (m0 >= count || n0 >= p.N) return;
@@ -534,10 +538,8 @@ static const GroupedShape g_shapes[9] = {{128, 192, 1.05f, 1.15f, false}, {64, 6
 // straight from memory / tiles at 1, 2, 4, 6, 8, 12 entries a group, 64 groups of 8 choices a row: 5,632 of 2,048 189 / 193, 221 / 246, 277 / 281, 281 / 267,
 // 322 / 290, 370 / 293; 2,048 of 2,816 106 / 96, 127 / 127, 140 / 135, 152 / 137, 164 / 140, 204 / 140; 2,048 of 704 26 / 35, 36 / 47, 39 / 49, 42 / 49,
 // 44 / 49, 55 / 51. 8 groups of 2, at 4, 6, 8, 12: 5,632 of 2,048 43 / 52, 54 / 52, 54 / 52, 108 / 52; 2,048 of 2,816 25 / 24, 35 / 24, 35 / 24, 31 / 24.
-// (The way straight from memory is not even: its workgroups of tiles that no group fills are spread so that heights of 2, 4, 8 .. tiles leave
-// part of the chip idle. Over 805 sizes of 2 to 128 groups and 1 to 64 entries a group, this rule takes 1.04 times the better way's time, and
-// on 58 of them more than the way straight from memory: most by 1 or 2 us of 8, 64 groups of 2,816 of 1,024 at 4 to 6 entries by an eighth.
-// A line at 48 entries alone takes 1.04 times too, but more than the way straight from memory on 151, up to 1.5 times.)
+// (Those figures are from when a group's tiles lay behind one another in the grid of the way straight from memory, which cost it up to twice the
+// time beyond 16 rows. As it lies now it may be the faster one further up: the line has stayed where nothing became slower.)
 // A product per head of few steps (K below 256) is bound by its results' way to memory and by the beginnings and ends of its tiles: the small tile
 // of which most fit a unit. us, the tiles before the loop / as the estimate picks them / so: 4,096 rows of 64 heads of 128 x 128 46 / 59 / 42,
 // 1,531 rows of 16 of 512 x 128 21 / 20 / 17, 300 of 16 of 512 x 128 7.3 / 8.5 / 6.3, 1,531 of 64 of 64 x 64 9.3 / 13.1 / 10.5. With a gate and heads no
@@ -619,12 +621,13 @@ TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, lo
 #undef TILES
     } else if (aligned && most_rows >= 64 * (lists ? groups : 1)) {
       // 64 entries x 128 columns a workgroup, operands straight from memory
-      dim3 big((N + 127) / 128, (most_rows + 63) / 64, groups);
+      const dim3 big((N + 127) / 128, groups, (most_rows + 63) / 64);
       if (out_dtype == TIS_BF16) grouped_mfma_kernel<bf16, 2, 2, 2, 4><<<big, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);
       else grouped_mfma_kernel<float, 2, 2, 2, 4><<<big, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);
     } else if (aligned) {
-      if (out_dtype == TIS_BF16) grouped_mfma_kernel<bf16, 1, 4, 1, 1><<<grid, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);
-      else grouped_mfma_kernel<float, 1, 4, 1, 1><<<grid, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);
+      const dim3 few(grid.x, groups, tiles_m);
+      if (out_dtype == TIS_BF16) grouped_mfma_kernel<bf16, 1, 4, 1, 1><<<few, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);
+      else grouped_mfma_kernel<float, 1, 4, 1, 1><<<few, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);
     } else {
       if (out_dtype == TIS_BF16) grouped_plain_kernel<bf16, bf16><<<grid, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);
       else grouped_plain_kernel<bf16, float><<<grid, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);
