@@ -555,6 +555,11 @@ TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_
     if (i == 5 || (i > 5 && K <= 9 * 64)) continue;
     if (K < 256 && i != 1 && i != 4) continue;     // few steps: what counts is a tile's beginning and end
     const GroupedShape& q = g_shapes[i];
+    // a tile of 192 or 256 rows only where the groups fill three quarters of one on average: below, a tile a group is nearly all there is, most of it
+    // padding that the estimate's half a tile does not see (us with / without: 64 groups of 8 choices, 1,024 of 1,408, 1,000 rows 123 / 80; 32 of 2, 2,048 of
+    // 704, 2,048 rows 83 / 65; 128 of 8, 2,048 of 768, 1,000 rows 207 / 156; at 800 rows 178 / 147. Without the limit 22 of 255 sizes of 4 to 128 groups take
+    // more than 3 % longer than with the first five tiles alone, with it 11)
+    if (lists && q.bm > 128 && most_entries < (long)groups * q.bm * 3 / 4) continue;
     const long tn = (N + q.bn - 1) / q.bn;
     // (with lists, entries / bm row tiles and half a tile more in every group)
     const float r = (lists ? (float)most_entries / q.bm + 0.5f * groups : (float)((long)groups * ((most_rows + q.bm - 1) / q.bm))) * tn / g_units;
