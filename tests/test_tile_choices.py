@@ -21,3 +21,13 @@ def test_groups_of_few_entries_take_no_high_tiles(groups, top, N, K):
             assert 4 * rows * top >= 3 * groups * GROUPED_ROWS[tile], (rows, tile)
             high += 1
     assert high
+
+
+@pytest.mark.parametrize("groups,top,N,K", [(64, 6, 512, 1024), (128, 8, 768, 2048), (32, 4, 1536, 2048), (17, 2, 4096, 1536)])
+def test_many_groups_of_few_entries_take_the_first_five_tiles(groups, top, N, K):
+    """Beyond sixteen groups, below 200 entries a group: none of the tiles that are for many steps of few groups; at sixteen, and from 200 on, some."""
+    pick = hip_ops.library("experts").cdll.tis_grouped_tile
+    few = {pick(1, groups, rows, c_long(rows * top), N, K, 0) for rows in range(17, 200 * groups // top, 7)}
+    assert few <= {-1, 0, 1, 2, 3, 4}
+    more = {pick(1, g, rows, c_long(rows * top), N, K, 0) for g in (16, groups) for rows in range(-(-200 * g // top), 4000 * g // top, 41)}
+    assert more & {6, 7, 8}

@@ -551,14 +551,18 @@ TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_
     return gate && N <= 128 && (long)groups * ((most_rows + 63) / 64) * ((N + 63) / 64) > 2048 ? 1 : 5;
   int pick = 0;
   float best = INFINITY;
+  // The last three tiles, and what a further round takes below, are for many steps and for groups that the estimate of row tiles fits: sixteen at
+  // most, or of 200 entries on average. us, with the first five alone / with all, at lists that an even and an uneven router makes: 64 groups of 6
+  // choices, 512 of 1,024, 1,200 rows 36 / 52; 128 of 8, 768 of 2,048, 800 rows 132 / 161; 32 of 4, 1,536 of 2,048, 450 rows 64 / 75. Of 918 sizes of 4 to 128
+  // groups 24 now take more than 3 % longer than with those five (before, 87), and all together 0.985 of their time (before, 0.993).
+  const bool all = K > 9 * 64 && (!lists || groups <= 16 || most_entries >= 200L * groups);
   for (int i = 0; i < 9; ++i) {
-    if (i == 5 || (i > 5 && K <= 9 * 64)) continue;
+    if (i == 5 || (i > 5 && !all)) continue;
     if (K < 256 && i != 1 && i != 4) continue;     // few steps: what counts is a tile's beginning and end
     const GroupedShape& q = g_shapes[i];
     // a tile of 192 or 256 rows only where the groups fill three quarters of one on average: below, a tile a group is nearly all there is, most of it
-    // padding that the estimate's half a tile does not see (us with / without: 64 groups of 8 choices, 1,024 of 1,408, 1,000 rows 123 / 80; 32 of 2, 2,048 of
-    // 704, 2,048 rows 83 / 65; 128 of 8, 2,048 of 768, 1,000 rows 207 / 156; at 800 rows 178 / 147. Without the limit 22 of 255 sizes of 4 to 128 groups take
-    // more than 3 % longer than with the first five tiles alone, with it 11)
+    // padding that the estimate's half a tile does not see (us with / without: 64 groups of 8 choices, 1,024 of 1,408, 1,000 rows 123 / 80; 16 of 2, 4,096 of
+    // 1,536, 1,000 rows 128 / 81; 32 of 2, 2,048 of 704, 2,048 rows 83 / 65)
     if (lists && q.bm > 128 && most_entries < (long)groups * q.bm * 3 / 4) continue;
     const long tn = (N + q.bn - 1) / q.bn;
     // (with lists, entries / bm row tiles and half a tile more in every group)
@@ -567,7 +571,7 @@ TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_
     // from ten steps on, with more tiles than units: what a step takes then (us, 8 groups, two choices a row, 128 x 192 / 128 x 128 / 256 x 128 /
     // 192 x 128: 1,531 rows, 5,632 of 2,048 122 / 124 / 106 / 125; 1,000 rows 110 / 99 / 82 / 88; 600 rows 64 / 70 / 77 / 72; 1,531 rows, 2,048 of 2,816
     // 79 / 68 / 56 / 83)
-    if (K > 9 * 64 && r > 1.f) {
+    if (all && r > 1.f) {
       if (i == 0) t = r <= 2.f ? 1.83f : 0.4f + 1.2f * r;
       else if (i == 2) t = 0.7f * ceilf(r);
       else if (i == 4) t = fmaxf(1.15f * fminf(r, 2.3f), 0.85f * r);
