@@ -31,3 +31,11 @@ def test_many_groups_of_few_entries_take_the_first_five_tiles(groups, top, N, K)
     assert few <= {-1, 0, 1, 2, 3, 4}
     more = {pick(1, g, rows, c_long(rows * top), N, K, 0) for g in (16, groups) for rows in range(-(-200 * g // top), 4000 * g // top, 41)}
     assert more & {6, 7, 8}
+
+
+@pytest.mark.parametrize("rows,N,K,tile", [(3000, 2816, 1024, 3), (3492, 15104, 384, 3), (7321, 9088, 704, 3), (1531, 48000, 1536, 0),
+                                           (300, 448, 512, 6)])
+def test_many_results_of_few_steps(rows, N, K, tile):
+    """Products whose results take a good part of their time: the tiles (0: 256 x 256, 3: 128 x 192 two a unit, 6: 64 x 64) that were measured to be the
+    fastest, each by a twentieth to a quarter against the tile that an estimate by the steps alone picks."""
+    assert hip_ops.library("gemm_tiles").cdll.tis_gemm_tiles_pick(rows, N, K) == tile
