@@ -51,6 +51,8 @@ def test_products_by_rows(ops, M):
         want = x.double() @ w.double().t()
         torch.testing.assert_close(ops.linear_by_rows(x, w, residual=res).double(), want + res.double(), rtol=2e-2, atol=2e-2)
         whole = res.contiguous()
+        if M <= 1024:                   # on the tiles either way
+            assert torch.equal(ops.linear_by_rows(x, w, residual=res), ops.linear_by_rows(x, w, residual=whole))
         assert torch.equal(ops.linear_by_rows(x, w, residual=whole), ops.linear(x, w, residual=whole))
         assert torch.equal(ops.linear_by_rows(x, w, rms=(gain, 1e-5)), ops.linear(x, w, rms=(gain, 1e-5)))
         assert torch.equal(ops.linear_swiglu(x, w, rms=(gain, 1e-5)), ops.swiglu(ops.linear(x, w, rms=(gain, 1e-5))))

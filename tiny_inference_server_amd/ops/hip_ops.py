@@ -912,7 +912,7 @@ class HipOps:
         rows, columns, inner = _TILES_NARROW
         most = rows if N <= columns and K <= inner else _TILES_UP_TO
         return (self.dtype == torch.bfloat16 and self.few_rows < M <= most and N % 4 == 0
-                and self._route(x, M, N, K, residual=residual) in ("library", "tiles")
+                and self._route(x, M, N, K) in ("library", "tiles")      # (the tiles read a residual that the library does not)
                 and (residual is None or (residual.stride(0) % 4 == 0 and residual.data_ptr() % 8 == 0)))
 
     def linear_by_rows(self, x, w, residual=None, rms=None, reuse_residual=False):
