@@ -58,6 +58,17 @@ def test_products_by_rows(ops, M):
         assert torch.equal(ops.linear_swiglu(x, w, rms=(gain, 1e-5)), ops.swiglu(ops.linear(x, w, rms=(gain, 1e-5))))
 
 
+@pytest.mark.parametrize("M", [129, 257, 640, 1531, 2048])
+def test_library_and_tiles_give_the_same_bits(ops, M):
+    """At every width of the library's list: which of the two a layer's product takes is not seen in its result."""
+    for i, (N, K) in enumerate(sorted(ops.library_widths)):
+        x, w, res = ops.empty(M, K), rnd((N, K), 60 + i, K ** -0.5).cuda(), rnd((M, N), 80 + i).cuda()
+        x.copy_(rnd((M, K), 70 + i))
+        for residual in (None, res):
+            tiles = ops._linear_tiles(x, w, residual, ops.empty(M, N), N, 0, 0)
+            assert torch.equal(ops._linear_library(x, w, residual), tiles), (N, K)
+
+
 @pytest.mark.parametrize("tile,rows,N,K", [(6, 600, 1020, 1416), (7, 1531, 2044, 1992), (8, 900, 2044, 712), (1, 129, 2052, 648), (2, 600, 2044, 1416)])
 @pytest.mark.parametrize("gated", [False, True])
 def test_grouped_product_of_many_steps(ops, tile, rows, N, K, gated):

@@ -5,6 +5,8 @@
 // used, 0.5 to 1.3.) The reference's engine uses a library product here (x @ W, main_models_new.py:19-20).
 //
 // tile_loop.h holds the loop. A row's sums run over K in the same order whatever M is and whichever tile is taken: its result does not depend on the other rows.
+#include <climits>
+
 #include "tile_loop.h"
 
 TIS_DEFINE_LAST_ERROR(tis_gemm_tiles)
@@ -145,6 +147,12 @@ TIS_EXPORT int tis_gemm_tiles_pick(int M, int N, int K) {
     if (t < best) best = t, pick = i;
   }
   return pick;
+}
+
+// How many workgroups that tile makes of the product.
+TIS_EXPORT int tis_gemm_tiles_count(int M, int N, int K) {
+  const long n = tiles_of(tis_gemm_tiles_pick(M, N, K), M, N);
+  return n < INT_MAX ? (int)n : INT_MAX;
 }
 
 // W: [N, K] contiguous. R: null, or the residual (bfloat16) added to the product; it may be C itself (every element is

@@ -16,6 +16,7 @@ size, slower where there are many rows.
 from __future__ import annotations
 
 import ctypes
+import functools
 import json
 import os
 from ctypes import c_float, c_int, c_long, c_void_p
@@ -185,18 +186,11 @@ def library(name: str) -> _Lib:
 
 
 _FEW_ROWS = 128                 # up to this many rows a product goes to the few-row kernels whatever its widths
-_TILES_UP_TO = 1024             # a model's own products of more rows than that, but no more than these, run on this repository's tiles
-                                # also at the library's widths, where the library has a product of few tiles wait for its matrix.
-                                # us, library / tiles, matrices from memory: 2,304 x 1,536 at 140, 320, 640, 1,024 rows 10 / 8, 17 / 9.6,
-                                # 17 / 13, 18 / 18; 1,536 x 4,096 16 / 15, 21 / 16, 24 / 20, 25 / 25; 2,048 x 5,632 21 / 19, 26 / 27, 34 / 37,
-                                # 41 / 37; with the gate (library and gate kernel / tiles) 8,192 x 1,536 23 / 13, 25 / 18, 31 / 26, 38 / 32;
-                                # 11,264 x 2,048 30 / 21, 37 / 27, 48 / 45, 58 / 57. At 1,532 and 2,048 rows the library is the faster:
-                                # 1,536 x 4,096 34 / 35, 35 / 36, 8,192 x 1,536 45 / 48, 53 / 56, 11,264 x 2,048 83 / 78, 96 / 100.
-                                # Both add a row's products up in the same order and give the same bits
-_TILES_NARROW = (2048, 3072, 2048)   # ... and up to (rows, columns, inner columns) of these the tiles go on: 2,304 x 1,536 at 1,280, 1,532, 1,800,
-                                # 2,048 rows 19 / 18, 19 / 19, 24 / 21, 24 / 22.5; 1,536 x 1,536 16 / 13, 17 / 17, 19 / 16, 18.5 / 17.5; 2,048 x 2,048
-                                # 22 / 21, 22 / 21, 24 / 22, 24 / 24; 3,072 x 2,048 25 / 23, 26 / 26, 31 / 28, 30 / 31 (the library's row count is
-                                # rounded up to 256); but 2,048 x 5,632 47 / 50, 45 / 50, and 3,000 rows of 3,072 x 2,048 38 / 49
+# A model's own products of more rows than that run on this repository's tiles also at the library's widths, up to so many rows, or
+# (rows, columns, inner columns) of narrow matrices, where tiles_pay says so. Both add a row's products up in the same order and give the same
+# bits (at every width of the list).
+_TILES_UP_TO = 1024
+_TILES_NARROW = (2048, 3072, 2048)
 
 _WIDTHS_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "library_widths.json")
 
@@ -229,6 +223,43 @@ def product_route(M: int, N: int, K: int, aligned: bool, out_f32: bool, widths, 
     if (N, K) in widths and not out_f32:
         return "library"
     return "tiles" if N % 4 == 0 else "few_rows"
+
+
+@functools.lru_cache(maxsize=4096)
+def _tiles_pay(M: int, N: int, K: int, gate: bool) -> bool:
+    """tiles_pay with the tile that such a product takes: worked out once for a size."""
+    lib = library("gemm_tiles").cdll
+    return tiles_pay(M, N, K, gate, lib.tis_gemm_tiles_pick(M, N, K) == 5, lib.tis_gemm_tiles_count(M, N, K) / _CHIP_UNITS)
+
+
+def _tiles_up_to(N: int, K: int) -> int:
+    rows, columns, inner = _TILES_NARROW
+    return rows if N <= columns and K <= inner else _TILES_UP_TO
+
+
+def tiles_pay(M: int, N: int, K: int, gate: bool, narrow_tile: bool, share: float) -> bool:
+    """Whether a product of M rows at one of the library's widths runs on the tiles: `share` of them a compute unit, narrow_tile: the 128 x 64 one; gate:
+    with the gate on its sums, which saves the gate's kernel. What speaks for the tiles: rows little beyond the library's last step of rows (it computes
+    them rounded up, see library_rows), and a chip that they fill; the fewer units have one, the longer the idle ones wait with every step of K.
+
+    us, library / tiles, matrices from memory; where the rule takes the tiles: 2,304 x 1,536 at 140, 320, 640, 1,024, 1,537 rows 10 / 8, 16 / 10, 16 / 13,
+    17.6 / 17.5, 20 / 17.5; 1,536 x 4,096 at 257, 513, 640, 832 21 / 16, 24 / 19, 24 / 20.5, 25 / 24; 2,048 x 5,632 at 513, 900, 1,024 33 / 29, 39 / 32,
+    40 / 38; 3,072 x 2,048 at 192, 513, 900, 1,537 21 / 12, 22 / 13.5, 24 / 19, 29 / 26; with the gate 8,192 x 1,536 at 140, 512, 1,024 22 / 13, 26 / 21, 37 / 32,
+    11,264 x 2,048 29 / 22, 37 / 33, 63 / 57. Where it takes the library: 2,048 x 5,632 at 256, 384, 640, 768 21 / 22.6, 26 / 29, 33 / 39, 33 / 39; 1,536 x 4,096 at
+    768, 1,024 24 / 27, 25 / 27; 2,048 x 2,048 at 640, 768 14.6 / 16.1; 3,072 x 2,048 at 512, 2,048 15 / 16, 30 / 32; 1,536 x 1,536 at 1,532 17.8 / 19.1;
+    2,048 x 1,408 at 1,280 17 / 18; 11,264 x 2,048 with the gate at 768 48 / 51. Of 348 products at the twelve widths, 129 to 2,048 rows, none took 4 % longer than
+    with the library on one chip, and 7 of beyond 1,790 rows 4 to 11 % on another; with the flat limits alone 32 did, 640 rows of 2,048 x 5,632 by 18 %. (What it
+    leaves to the library though the tiles are the faster: 900 rows of 1,536 x 3,072 20 / 17, 448 of 3,072 x 2,048 15 / 14, 2,048 of 2,304 x 1,536 23.2 / 21.9.)"""
+    if M > _tiles_up_to(N, K) or N % 4:
+        return False
+    step = 64 if M <= 256 else 256
+    beyond = 1 - (library_rows(M) - M) / step        # of the library's last step of rows
+    if gate:
+        return not (1 < share < 1.5 and beyond > 0.3)
+    if K > 4096 and M <= 512:
+        return False
+    return (beyond <= 0.3 or share >= 0.8 or (K <= 1536 and M <= 1024)
+            or (K <= 3072 and M <= 1024 and not narrow_tile))
 
 
 # wavefronts the attention launch aims for, so that short batches still spread over the chip
@@ -845,9 +876,14 @@ class HipOps:
         reuse_residual: the caller has no further use for `residual`; an operations object may then write the result
         over it. This one never does: every product's result has memory of its own.
         """
+        out_dtype = out_dtype or self.dtype
+        M, N, K = self._linear_operands(x, w, residual, out_dtype, rms)
+        return self._linear(x, w, M, N, K, residual, out_dtype, rms)
+
+    def _linear_operands(self, x, w, residual, out_dtype, rms):
+        """(rows, output, input columns) of a product whose operands fit together."""
         _rows_view(self._check(x, "linear x"), "linear x")
         self._check(w, "linear w")
-        out_dtype = out_dtype or self.dtype
         M, K = x.shape
         if w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
             raise KernelError(f"linear: x {tuple(x.shape)} against w {tuple(w.shape)} (w is [out, in], contiguous)")
@@ -860,6 +896,10 @@ class HipOps:
             self._check(rms[0], "rmsnorm gain", torch.float32)
             if rms[0].numel() != K or not rms[0].is_contiguous():
                 raise KernelError(f"linear: norm gain has {rms[0].numel()} entries for width {K}")
+        return M, N, K
+
+    def _linear(self, x, w, M, N, K, residual, out_dtype, rms, route=None):
+        """The product of operands that _linear_operands has seen, by the given route (None: the one that _route names)."""
         if self.dtype == torch.float32:
             if rms is not None and self._plain_fuses(x, w, rms):
                 return self._linear_plain_fused(x, w, rms, residual, self.empty(M, N), 0)
@@ -870,7 +910,8 @@ class HipOps:
                                            residual.stride(0) if residual is not None else 0, _ptr(out), N, M, N, K,
                                            self._stream())
             return out
-        route = self._route(x, M, N, K, out_dtype, residual)
+        if route is None:
+            route = self._route(x, M, N, K, out_dtype, residual)
         if route == "few_rows":
             out = self.empty(M, N, dtype=out_dtype)
             if out_dtype == torch.float32 and residual is not None:
@@ -907,29 +948,24 @@ class HipOps:
                                              M, N, K, gate, self._stream())
         return out
 
-    def _tiles_at_any_width(self, x, M, N, K, residual=None):
-        """Whether a bfloat16 product of these rows runs on the tiled product whatever its widths (see _TILES_UP_TO)."""
-        rows, columns, inner = _TILES_NARROW
-        most = rows if N <= columns and K <= inner else _TILES_UP_TO
-        return (self.dtype == torch.bfloat16 and self.few_rows < M <= most and N % 4 == 0
-                and self._route(x, M, N, K) in ("library", "tiles")      # (the tiles read a residual that the library does not)
-                and (residual is None or (residual.stride(0) % 4 == 0 and residual.data_ptr() % 8 == 0)))
+    def _layer_route(self, x, M, N, K, residual=None, gate=False):
+        """Which kernel takes a layer's bfloat16 product: as _route, but between the tiles and the library by tiles_pay."""
+        route = self._route(x, M, N, K)
+        if route == "library":
+            if _tiles_pay(M, N, K, gate):
+                route = "tiles"
+            elif residual is not None and (residual.stride(0) % 8 or residual.data_ptr() % 16):
+                route = "tiles" if M <= _tiles_up_to(N, K) and N % 4 == 0 else "few_rows"      # (the library does not read such a residual)
+        if route == "tiles" and residual is not None and (residual.stride(0) % 4 or residual.data_ptr() % 8):
+            route = "few_rows"
+        return route
 
     def linear_by_rows(self, x, w, residual=None, rms=None, reuse_residual=False):
         """What linear gives in the compute type; between this repository's tiles and the library's product the number of rows
         decides, not the widths alone: for the products of a model's own layers."""
-        _rows_view(self._check(x, "linear x"), "linear x")
-        self._check(w, "linear w")
-        (M, K), N = x.shape, w.shape[0]
-        if not (w.dim() == 2 and w.shape[1] == K and w.is_contiguous() and self._tiles_at_any_width(x, M, N, K, residual)):
-            return self.linear(x, w, residual=residual, rms=rms, reuse_residual=reuse_residual)
-        if residual is not None:
-            _rows_view(self._check(residual, "linear residual"), "linear residual")
-            if tuple(residual.shape) != (M, N):
-                raise KernelError(f"linear: residual {tuple(residual.shape)} for result {(M, N)}")
-        if rms is not None:
-            x = self.rmsnorm(x, rms[0], rms[1])
-        return self._linear_tiles(x, w, residual, self.empty(M, N), N, 0, 0)
+        M, N, K = self._linear_operands(x, w, residual, self.dtype, rms)
+        route = self._layer_route(x, M, N, K, residual) if self.dtype == torch.bfloat16 else None
+        return self._linear(x, w, M, N, K, residual, self.dtype, rms, route)
 
     def _linear_tiles(self, x, w, residual, out, N, out_f32, act):
         M, K = x.shape
@@ -961,30 +997,35 @@ class HipOps:
         """silu(g) * u of the rows of f(x) . w^T, w holding gate and up rows interleaved: [M, N/2]."""
         _rows_view(self._check(x, "linear x"), "linear x")
         M, K = x.shape
-        if w.dim() == 2 and w.shape[0] % 2 == 0 and self._few_rows_ok(x, M, w.shape[0], K):
+        pairs = w.dim() == 2 and w.shape[0] % 2 == 0 and w.shape[1] == K and w.is_contiguous()
+        N = w.shape[0] if pairs else 0
+        if self.dtype == torch.bfloat16 and pairs and M:
+            route = self._layer_route(x, M, N, K, gate=True)
             self._check(w, "linear w")
-            if w.shape[1] != K or not w.is_contiguous():
-                raise KernelError(f"linear: x {tuple(x.shape)} against w {tuple(w.shape)} (w is [out, in], contiguous)")
             if rms is not None and (rms[0].numel() != K or rms[0].dtype != torch.float32):
                 raise KernelError(f"linear: norm gain has {rms[0].numel()} entries for width {K}")
-            N = w.shape[0]
-            out = self.empty(M, N // 2)
-            self.gemm_skinny.tis_gemm_skinny(
-                _ptr(x), x.stride(0), _ptr(w), _ptr(rms[0] if rms else None), float(rms[1]) if rms else 0.0,
-                _ptr(None), 0, _ptr(out), out.stride(0), M, N, K, 2, 1, self._stream())
-            return out
-        if w.dim() == 2 and w.shape[1] == K and w.is_contiguous() and self._tiles_at_any_width(x, M, w.shape[0], K):
-            # the gate on the product's 32-bit sums; N in steps of 4, so that gate and up lie in one lane
-            self._check(w, "linear w")
+            if route == "few_rows":
+                out = self.empty(M, N // 2)
+                self.gemm_skinny.tis_gemm_skinny(
+                    _ptr(x), x.stride(0), _ptr(w), _ptr(rms[0] if rms else None), float(rms[1]) if rms else 0.0,
+                    _ptr(None), 0, _ptr(out), out.stride(0), M, N, K, 2, 1, self._stream())
+                return out
+            if route == "tiles" and M <= _tiles_up_to(N, K):
+                # the gate on the product's 32-bit sums; N in steps of 4, so that gate and up lie in one lane
+                if rms is not None:
+                    x = self.rmsnorm(x, rms[0], rms[1])
+                return self._linear_tiles(x, w, None, self.empty(M, N // 2), N, 0, 4)
             if rms is not None:
-                x = self.rmsnorm(x, rms[0], rms[1])
-            return self._linear_tiles(x, w, None, self.empty(M, w.shape[0] // 2), w.shape[0], 0, 4)
-        if self.dtype == torch.float32 and w.dim() == 2 and w.shape[0] % 2 == 0 and w.shape[1] == K and w.is_contiguous() \
-                and (rms is None or (rms[0].numel() == K and rms[0].is_contiguous())) and self._plain_fuses(x, w, rms):
+                self._check(rms[0], "rmsnorm gain", torch.float32)
+                if not rms[0].is_contiguous():
+                    raise KernelError(f"linear: norm gain of {rms[0].numel()} entries is not contiguous")
+            return self.swiglu(self._linear(x, w, M, N, K, None, self.dtype, rms, route))
+        if self.dtype == torch.float32 and pairs and (rms is None or (rms[0].numel() == K and rms[0].is_contiguous())) \
+                and self._plain_fuses(x, w, rms):
             self._check(w, "linear w")
             if rms is not None:
                 self._check(rms[0], "rmsnorm gain", torch.float32)
-            return self._linear_plain_fused(x, w, rms, None, self.empty(M, w.shape[0] // 2), 1)
+            return self._linear_plain_fused(x, w, rms, None, self.empty(M, N // 2), 1)
         return self.swiglu(self.linear(x, w, rms=rms))
 
     # activations that a bfloat16 product applies to its 32-bit sums: (few-row kernel's epilogue, tiled kernel's code)
