@@ -77,8 +77,9 @@ static constexpr int GS_BM = 16, GS_BN = 16, GS_BK = 256, GS_LD = GS_BK + 4;
 
 // NORM: A's rows are RMS-normed on the way in, x * sqrt(K) / (||x|| + eps) * gain with the sum of squares added up in the order of the
 // norm's own kernel (256 threads a row, four waves); GATE: C has N / 2 columns, silu(g) u of the columns' pairs (2j, 2j + 1). Both give the
-// bits of the separate kernels. What they save is those kernels' launches, 3 us each where a step is nothing but launches; every column tile
-// sums its 16 rows' squares again, which its first loads hide up to a thousand columns.
+// bits of the separate kernels. GATE saves a kernel (us, product and gate's kernel / one: 16 x 64 x 352 5.2 / 3.5, 128 x 1,024 x 2,048 26 / 24; faster at all
+// of 370 sizes). NORM saves a launch, but not time on the GPU: every column tile sums its 16 rows' squares again before its first product (see
+// tis_gemm_plain_norms).
 template <bool VEC, typename TI, typename TO, bool NORM = false, bool GATE = false>
 __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI* __restrict__ A, long lda, const TI* __restrict__ W,
                                                                    long ldw, const TO* __restrict__ R, long ldr,
@@ -240,10 +241,17 @@ TIS_EXPORT int tis_gemm_plain(int in_dtype, int out_dtype, const void* A, long l
   return tis_launch_status("gemm_plain");
 }
 
-// The product of 32-bit rows with the norm before it and the gate behind it (see the kernel): whether it takes M rows of K values against N
-// columns. us, norm, product and gate apart / fused, in a captured step: see the test's sizes; beyond 1,024 columns the sums of squares show.
+// The product of 32-bit rows with the gate behind it and the norm before it (see the kernel): whether it takes M rows of K values against N columns.
 TIS_EXPORT int tis_gemm_plain_fuses(int M, int N, int K) {
   return M > 0 && N > 0 && K > 0 && K % 4 == 0 && K <= 1024 && tis_gemm_plain_few(1, M, N, K) && (M + GS_BM - 1) / GS_BM <= 65535;
+}
+
+// Whether such a product is worth taking the norm inside where the host launches it: a launch there is 5 us of the host's time, which a model of this
+// size waits for. Recorded in a graph the norm's own kernel is the faster at every size, us, norm and product / one kernel: 4 rows of 176 x 64 5.3 / 5.6,
+// 128 of 1,024 x 64 6.1 / 7.5, 16 of 2,048 x 128 6.0 / 7.2; beyond 128 inner columns, or 256 tiles, by more than a launch: 16 rows of 2,048 x 512 9.3 / 12.8, 128 of
+// 2,048 x 128 9.4 / 15.3, 512 of 2,048 x 1,024 93 / 216.
+TIS_EXPORT int tis_gemm_plain_norms(int M, int N, int K) {
+  return tis_gemm_plain_fuses(M, N, K) && K <= 128 && (long)((N + GS_BN - 1) / GS_BN) * ((M + GS_BM - 1) / GS_BM) <= 256;
 }
 
 // gain: null, or the norm's gain [K] (eps is added to the norm); gate: C has N / 2 columns. A, W and gain start on 16 bytes, lda and ldw in steps of 4.
@@ -252,14 +260,14 @@ TIS_EXPORT int tis_gemm_plain_fused(const float* A, long lda, const float* gain,
   if (M == 0 || N == 0) return 0;
   if (!tis_gemm_plain_fuses(M, N, K)) return tis_fail("gemm: no fused product of M=%d N=%d K=%d", M, N, K);
   if (lda % 4 || ldw % 4 || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)gain) % 16) return tis_fail("gemm: a fused product's rows start on 16 bytes");
+  if (!gain && !gate) return tis_fail("gemm: a fused product has a norm or a gate");
   if (gate && (R || N % 2)) return tis_fail("gemm: a gate goes with pairs of columns and no residual");
   const dim3 grid((N + GS_BN - 1) / GS_BN, (M + GS_BM - 1) / GS_BM);
 #define FUSED(NORM, GATE) gemm_plain_few_kernel<true, float, float, NORM, GATE><<<grid, GS_BM * GS_BN, 0, stream>>>( \
     A, lda, W, ldw, R, ldr, C, ldc, M, N, K, gain, eps)
   if (gain && gate) FUSED(true, true);
   else if (gain) FUSED(true, false);
-  else if (gate) FUSED(false, true);
-  else FUSED(false, false);
+  else FUSED(false, true);
 #undef FUSED
   return tis_launch_status("gemm_plain_fused");
 }

@@ -901,7 +901,7 @@ class HipOps:
     def _linear(self, x, w, M, N, K, residual, out_dtype, rms, route=None):
         """The product of operands that _linear_operands has seen, by the given route (None: the one that _route names)."""
         if self.dtype == torch.float32:
-            if rms is not None and self._plain_fuses(x, w, rms):
+            if rms is not None and self._plain_norms(M, N, K) and self._plain_fuses(x, w, rms):
                 return self._linear_plain_fused(x, w, rms, residual, self.empty(M, N), 0)
             if rms is not None:
                 x = self.rmsnorm(x, rms[0], rms[1])
@@ -940,6 +940,10 @@ class HipOps:
         return (x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
                 and (rms is None or rms[0].data_ptr() % 16 == 0)
                 and bool(self.gemm_plain.cdll.tis_gemm_plain_fuses(x.shape[0], w.shape[0], x.shape[1])))
+
+    def _plain_norms(self, M, N, K):
+        """Whether that norm is worth having in there: where the host launches each kernel, not where they are recorded (the same bits)."""
+        return bool(self.gemm_plain.cdll.tis_gemm_plain_norms(M, N, K)) and not torch.cuda.is_current_stream_capturing()
 
     def _linear_plain_fused(self, x, w, rms, residual, out, gate):
         (M, K), N = x.shape, w.shape[0]
@@ -1025,6 +1029,8 @@ class HipOps:
             self._check(w, "linear w")
             if rms is not None:
                 self._check(rms[0], "rmsnorm gain", torch.float32)
+                if not self._plain_norms(M, N, K):
+                    x, rms = self.rmsnorm(x, rms[0], rms[1]), None
             return self._linear_plain_fused(x, w, rms, None, self.empty(M, N // 2), 1)
         return self.swiglu(self.linear(x, w, rms=rms))
 
