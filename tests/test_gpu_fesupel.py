@@ -292,6 +292,31 @@ def test_low_rank_projections_of_several_chunks_of_the_rank(rank, n, C):
     close(ops.lowrank_decay(dev, on(w2), on(bias), 7.0), torch.exp(torch.nn.functional.logsigmoid(z) / 7.0), "float32", "decays of a sigmoid")
 
 
+@pytest.mark.parametrize("rank", [4, 16, 20, 32, 64, 68, 132])
+@pytest.mark.parametrize("n,C", [(1, 33), (257, 64), (513, 514), (90, 6000)])
+def test_low_rank_projections_read_16_bytes_at_a_time(rank, n, C):
+    """Rows that begin on 16 bytes, in steps of 16, beside a number that is none: the sums against 64 bits, and the bits of rows that begin
+    in between, which are read one number at a time."""
+    ops = hip_ops("float32")
+    g = torch.Generator().manual_seed(rank * n + C)
+    low, w2 = torch.randn(n, rank, generator=g), torch.randn(C, rank, generator=g) * rank ** -0.5
+    bias, rate = torch.randn(C, generator=g).cuda(), (torch.rand(C, generator=g) * 4).cuda()
+
+    def rows_at(column, columns):
+        wide = torch.full((n, columns), float("nan"))
+        wide[:, column:column + rank] = low
+        return wide.cuda()[:, column:column + rank]
+    aligned, between = rows_at(4, rank + 8), rows_at(1, rank + 3)
+    assert aligned.data_ptr() % 16 == 0 and aligned.stride(0) % 4 == 0 and between.data_ptr() % 16
+    w2 = w2.cuda()
+    got = ops.lowrank_act(aligned, w2, None, "none")
+    bound = (rank + 1) * 2.0 ** -24 * (low.double().abs() @ w2.cpu().double().abs().T)
+    assert ((got.cpu().double() - low.double() @ w2.cpu().double().T).abs() <= bound).all()
+    assert torch.equal(got, ops.lowrank_act(between, w2, None, "none"))
+    assert torch.equal(ops.lowrank_act(aligned, w2, bias, "exp_softplus", rate=rate, group=1), ops.lowrank_act(between, w2, bias, "exp_softplus", rate=rate, group=1))
+    assert torch.equal(ops.lowrank_decay(aligned, w2, bias, 7.0), ops.lowrank_decay(between, w2, bias, 7.0))
+
+
 @pytest.mark.parametrize("n,N,top,groups", [(37, 8, 2, (4, 2)), (5, 12, 3, (3, 1)), (200, 16, 3, (2, 1)), (9, 6, 6, None), (64, 64, 4, (16, 3)),
                                             (33, 10, 1, (10, 1)), (20, 130, 5, (13, 2))])
 def test_choice_in_groups(n, N, top, groups):
