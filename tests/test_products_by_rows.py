@@ -25,11 +25,12 @@ def test_residuals_that_the_library_does_not_read(rows, N, K):
         assert [fn for fn, _ in ops.calls] == [kernel], (residual.stride(), residual.storage_offset())
 
 
-# (rows, columns, inner columns, gate): sizes at which the tiles, and at which the library's product, is the faster by 4 % and more
-ON_TILES = [(140, 2304, 1536, 0), (640, 2304, 1536, 0), (1537, 2304, 1536, 0), (257, 1536, 4096, 0), (640, 1536, 4096, 0), (513, 2048, 5632, 0), (900, 2048, 5632, 0),
-            (192, 3072, 2048, 0), (900, 3072, 2048, 0), (140, 8192, 1536, 1), (1024, 8192, 1536, 1), (512, 11264, 2048, 1), (1000, 11264, 2048, 1), (2048, 2816, 2048, 1)]
-ON_LIBRARY = [(256, 2048, 5632, 0), (384, 2048, 5632, 0), (640, 2048, 5632, 0), (768, 2048, 5632, 0), (768, 1536, 4096, 0), (1024, 1536, 4096, 0), (640, 2048, 2048, 0),
-              (768, 2048, 2048, 0), (768, 2048, 4096, 0), (768, 1536, 3072, 0), (512, 3072, 2048, 0), (2048, 3072, 2048, 0), (1532, 1536, 1536, 0), (1280, 2048, 1408, 0),
+# (rows, columns, inner columns, gate): sizes at which the tiles are the faster, or so small that the host's time decides; at which the library's product is
+# the faster by 4 % and more
+ON_TILES = [(140, 2304, 1536, 0), (640, 2304, 1536, 0), (1537, 2304, 1536, 0), (2048, 2304, 1536, 0), (257, 1536, 4096, 0), (640, 1536, 4096, 0), (513, 2048, 5632, 0),
+            (900, 2048, 5632, 0), (192, 3072, 2048, 0), (900, 3072, 2048, 0), (140, 8192, 1536, 1), (1024, 8192, 1536, 1), (512, 11264, 2048, 1), (1000, 11264, 2048, 1),
+            (2048, 2816, 2048, 1), (384, 2048, 5632, 0), (768, 1536, 4096, 0), (640, 2048, 2048, 0)]
+ON_LIBRARY = [(640, 2048, 5632, 0), (768, 2048, 5632, 0), (2048, 3072, 2048, 0), (1400, 1536, 1536, 0), (1532, 1536, 1536, 0), (1152, 2048, 1408, 0),
               (768, 11264, 2048, 1), (1025, 8192, 1536, 1), (1025, 1536, 4096, 0), (2049, 2304, 1536, 0)]
 
 

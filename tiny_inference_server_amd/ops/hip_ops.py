@@ -229,7 +229,7 @@ def product_route(M: int, N: int, K: int, aligned: bool, out_f32: bool, widths, 
 def _tiles_pay(M: int, N: int, K: int, gate: bool) -> bool:
     """tiles_pay with the tile that such a product takes: worked out once for a size."""
     lib = library("gemm_tiles").cdll
-    return tiles_pay(M, N, K, gate, lib.tis_gemm_tiles_pick(M, N, K) == 5, lib.tis_gemm_tiles_count(M, N, K) / _CHIP_UNITS)
+    return tiles_pay(M, N, K, gate, lib.tis_gemm_tiles_pick(M, N, K), lib.tis_gemm_tiles_count(M, N, K) / _CHIP_UNITS)
 
 
 def _tiles_up_to(N: int, K: int) -> int:
@@ -237,29 +237,38 @@ def _tiles_up_to(N: int, K: int) -> int:
     return rows if N <= columns and K <= inner else _TILES_UP_TO
 
 
-def tiles_pay(M: int, N: int, K: int, gate: bool, narrow_tile: bool, share: float) -> bool:
-    """Whether a product of M rows at one of the library's widths runs on the tiles: `share` of them a compute unit, narrow_tile: the 128 x 64 one; gate:
-    with the gate on its sums, which saves the gate's kernel. What speaks for the tiles: rows little beyond the library's last step of rows (it computes
-    them rounded up, see library_rows), and a chip that they fill; the fewer units have one, the longer the idle ones wait with every step of K.
+_TILE_256x128, _TILE_128x64 = 1, 5      # of the tiled product's tiles
 
-    us, library / tiles, matrices from memory; where the rule takes the tiles: 2,304 x 1,536 at 140, 320, 640, 1,024, 1,537 rows 10 / 8, 16 / 10, 16 / 13,
-    17.6 / 17.5, 20 / 17.5; 1,536 x 4,096 at 257, 513, 640, 832 21 / 16, 24 / 19, 24 / 20.5, 25 / 24; 2,048 x 5,632 at 513, 900, 1,024 33 / 29, 39 / 32,
+# From so many multiply-adds on the library is asked at all up to 1,024 rows: below, a step whose kernels the host launches one by one waits for the host,
+# of whose time a product by the library takes 10 us more than one on the tiles. 0.9B prompts of 130 to 520 rows, us a step, library / library where it is the
+# faster kernel / tiles: 5,390 / 4,200 / 3,780, of 520 to 1,100 5,520 / 4,530 / 4,350; 2.1B 6,960 / 5,800 / 5,020, and 7,850 / 7,470 / 7,420, where the GPU is the
+# slower of the two again.
+_LIBRARY_FROM = 7_000_000_000
+
+
+def tiles_pay(M: int, N: int, K: int, gate: bool, tile: int, share: float) -> bool:
+    """Whether a product of M rows at one of the library's widths runs on the tiles: `tile` is the one it takes, `share` the number of them a compute unit;
+    gate: with the gate on its sums, which saves the gate's kernel. What speaks for the tiles: rows little beyond the library's last step of rows (it
+    computes them rounded up, see library_rows), and a chip that they fill; the fewer units have one, the longer the idle ones wait with every step of K.
+
+    us, library / tiles, matrices from memory; where the rule takes the tiles: 2,304 x 1,536 at 140, 320, 640, 1,024, 1,537, 2,048 rows 10 / 8, 16 / 10, 16 / 13,
+    17.6 / 17.5, 20 / 17.5, 23.2 / 21.9; 1,536 x 4,096 at 257, 513, 640, 832 21 / 16, 24 / 19, 24 / 20.5, 25 / 24; 2,048 x 5,632 at 513, 900, 1,024 33 / 29, 39 / 32,
     40 / 38; 3,072 x 2,048 at 192, 513, 900, 1,537 21 / 12, 22 / 13.5, 24 / 19, 29 / 26; with the gate 8,192 x 1,536 at 140, 512, 1,024 22 / 13, 26 / 21, 37 / 32,
-    11,264 x 2,048 29 / 22, 37 / 33, 63 / 57. Where it takes the library: 2,048 x 5,632 at 256, 384, 640, 768 21 / 22.6, 26 / 29, 33 / 39, 33 / 39; 1,536 x 4,096 at
-    768, 1,024 24 / 27, 25 / 27; 2,048 x 2,048 at 640, 768 14.6 / 16.1; 3,072 x 2,048 at 512, 2,048 15 / 16, 30 / 32; 1,536 x 1,536 at 1,532 17.8 / 19.1;
-    2,048 x 1,408 at 1,280 17 / 18; 11,264 x 2,048 with the gate at 768 48 / 51. Of 348 products at the twelve widths, 129 to 2,048 rows, none took 4 % longer than
-    with the library on one chip, and 7 of beyond 1,790 rows 4 to 11 % on another; with the flat limits alone 32 did, 640 rows of 2,048 x 5,632 by 18 %. (What it
-    leaves to the library though the tiles are the faster: 900 rows of 1,536 x 3,072 20 / 17, 448 of 3,072 x 2,048 15 / 14, 2,048 of 2,304 x 1,536 23.2 / 21.9.)"""
+    11,264 x 2,048 29 / 22, 37 / 33, 63 / 57. Where it takes the library: 2,048 x 5,632 at 640, 768 33 / 39, 33 / 39; 3,072 x 2,048 at 2,048 30 / 32; 1,536 x 1,536 at
+    1,400, 1,532 17.8 / 19.1; 11,264 x 2,048 with the gate at 768 48 / 51. A block's four products are together nowhere slower than by the library alone, at either
+    size, 129 to 2,048 rows, beyond what two chips differ by (2 %); with the row limits alone 2.1B's at 768 rows were by 7 %. Single products that stay on the
+    tiles for the host's sake and are slower there: 1,536 x 4,096 at 768 24 / 27, 2,048 x 2,048 at 640 14.6 / 16.1, 2,048 x 5,632 at 384 26 / 29."""
     if M > _tiles_up_to(N, K) or N % 4:
         return False
     step = 64 if M <= 256 else 256
     beyond = 1 - (library_rows(M) - M) / step        # of the library's last step of rows
+    if M > 1024:
+        return gate or beyond <= 0.3 or share >= (0.8 if tile == _TILE_256x128 else 0.62)
+    if M * N * K < _LIBRARY_FROM:
+        return True
     if gate:
         return not (1 < share < 1.5 and beyond > 0.3)
-    if K > 4096 and M <= 512:
-        return False
-    return (beyond <= 0.3 or share >= 0.8 or (K <= 1536 and M <= 1024)
-            or (K <= 3072 and M <= 1024 and not narrow_tile))
+    return beyond <= 0.3 or share >= 0.8 or K <= 1536 or (K <= 3072 and tile != _TILE_128x64)
 
 
 # wavefronts the attention launch aims for, so that short batches still spread over the chip
@@ -967,9 +976,10 @@ class HipOps:
     def linear_by_rows(self, x, w, residual=None, rms=None, reuse_residual=False):
         """What linear gives in the compute type; between this repository's tiles and the library's product the number of rows
         decides, not the widths alone: for the products of a model's own layers."""
+        if self.dtype != torch.bfloat16 or x.shape[0] <= self.few_rows:
+            return self.linear(x, w, residual, None, rms)
         M, N, K = self._linear_operands(x, w, residual, self.dtype, rms)
-        route = self._layer_route(x, M, N, K, residual) if self.dtype == torch.bfloat16 else None
-        return self._linear(x, w, M, N, K, residual, self.dtype, rms, route)
+        return self._linear(x, w, M, N, K, residual, self.dtype, rms, self._layer_route(x, M, N, K, residual))
 
     def _linear_tiles(self, x, w, residual, out, N, out_f32, act):
         M, K = x.shape
