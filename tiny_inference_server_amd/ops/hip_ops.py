@@ -878,21 +878,17 @@ class HipOps:
         return out
 
     # ---- matrix products -----------------------------------------------------------------------------
-    def linear(self, x, w, residual=None, out_dtype=None, rms=None, reuse_residual=False):
+    def linear(self, x, w, residual=None, out_dtype=None, rms=None, reuse_residual=False, route=None):
         """f(x)[M,K] . w[N,K]^T (+ residual[M,N]); `out_dtype` float32 gives 32-bit results from bfloat16 inputs.
 
         rms = (gain, eps): f is the RMSNorm of the rows, fused into the product where the kernel allows.
         reuse_residual: the caller has no further use for `residual`; an operations object may then write the result
         over it. This one never does: every product's result has memory of its own.
+        route: the kernel of a bfloat16 product, from whoever has worked it out (_layer_route).
         """
-        out_dtype = out_dtype or self.dtype
-        M, N, K = self._linear_operands(x, w, residual, out_dtype, rms)
-        return self._linear(x, w, M, N, K, residual, out_dtype, rms)
-
-    def _linear_operands(self, x, w, residual, out_dtype, rms):
-        """(rows, output, input columns) of a product whose operands fit together."""
         _rows_view(self._check(x, "linear x"), "linear x")
         self._check(w, "linear w")
+        out_dtype = out_dtype or self.dtype
         M, K = x.shape
         if w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
             raise KernelError(f"linear: x {tuple(x.shape)} against w {tuple(w.shape)} (w is [out, in], contiguous)")
@@ -905,10 +901,6 @@ class HipOps:
             self._check(rms[0], "rmsnorm gain", torch.float32)
             if rms[0].numel() != K or not rms[0].is_contiguous():
                 raise KernelError(f"linear: norm gain has {rms[0].numel()} entries for width {K}")
-        return M, N, K
-
-    def _linear(self, x, w, M, N, K, residual, out_dtype, rms, route=None):
-        """The product of operands that _linear_operands has seen, by the given route (None: the one that _route names)."""
         if self.dtype == torch.float32:
             if rms is not None and self._plain_norms(M, N, K) and self._plain_fuses(x, w, rms):
                 return self._linear_plain_fused(x, w, rms, residual, self.empty(M, N), 0)
@@ -976,10 +968,11 @@ class HipOps:
     def linear_by_rows(self, x, w, residual=None, rms=None, reuse_residual=False):
         """What linear gives in the compute type; between this repository's tiles and the library's product the number of rows
         decides, not the widths alone: for the products of a model's own layers."""
-        if self.dtype != torch.bfloat16 or x.shape[0] <= self.few_rows:
-            return self.linear(x, w, residual, None, rms)
-        M, N, K = self._linear_operands(x, w, residual, self.dtype, rms)
-        return self._linear(x, w, M, N, K, residual, self.dtype, rms, self._layer_route(x, M, N, K, residual))
+        route = None
+        if self.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] > self.few_rows and w.dim() == 2 \
+                and (residual is None or residual.dim() == 2):
+            route = self._layer_route(x, x.shape[0], w.shape[0], x.shape[1], residual)
+        return self.linear(x, w, residual, None, rms, reuse_residual, route)
 
     def _linear_tiles(self, x, w, residual, out, N, out_f32, act):
         M, K = x.shape
@@ -1029,11 +1022,7 @@ class HipOps:
                 if rms is not None:
                     x = self.rmsnorm(x, rms[0], rms[1])
                 return self._linear_tiles(x, w, None, self.empty(M, N // 2), N, 0, 4)
-            if rms is not None:
-                self._check(rms[0], "rmsnorm gain", torch.float32)
-                if not rms[0].is_contiguous():
-                    raise KernelError(f"linear: norm gain of {rms[0].numel()} entries is not contiguous")
-            return self.swiglu(self._linear(x, w, M, N, K, None, self.dtype, rms, route))
+            return self.swiglu(self.linear(x, w, rms=rms, route=route))
         if self.dtype == torch.float32 and pairs and (rms is None or (rms[0].numel() == K and rms[0].is_contiguous())) \
                 and self._plain_fuses(x, w, rms):
             self._check(w, "linear w")
