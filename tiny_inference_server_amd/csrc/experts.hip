@@ -513,7 +513,8 @@ TIS_EXPORT void tis_experts_units(int n) { if (n > 0) g_units = n; }
 
 // The tiles of grouped_tiles_kernel, and the microseconds a step of 64 takes with r workgroups a compute unit:
 //   128 x 192, four waves, two buffers, two a unit     1.05 r, at least 1.15
-//   64 x 64, four waves, five buffers, two a unit      0.3 r, at least 0.33
+//   64 x 64, four waves, five buffers, two a unit      0.3 r, at least 0.33   (four below 256 inner columns: gated, 64 heads of 128 x 128 and of
+//                                                      128 x 192, 1,531 rows 50.2 and 51.5, with five 51.2 and 52.8)
 //   128 x 128, eight waves, five buffers               0.58 a round
 //   256 x 256, eight waves, two buffers                1.85 a round
 //   128 x 128, four waves, two buffers, two a unit     0.78 r, at least 0.8
@@ -619,6 +620,7 @@ TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, lo
         (const bf16*)A, (const bf16*)W, (float*)C, p, groups);                                                            \
   }
       if (pick == 0) TILES(128, 192, 2, 2, 2, 1)
+      else if (pick == 1 && K < 256) TILES(64, 64, 2, 2, 4, 2)
       else if (pick == 1) TILES(64, 64, 2, 2, 5, 2)
       else if (pick == 2) TILES(128, 128, 2, 4, 5, 2)
       else if (pick == 3) TILES(256, 256, 2, 4, 2, 1)

@@ -102,11 +102,11 @@ static int g_units = 256;      // compute units of the device: set by whoever kn
 TIS_EXPORT void tis_gemm_tiles_units(int n) { if (n > 0) g_units = n; }
 
 // The tiles, and what a product is estimated to take with each, us: a beginning and end, and the time of a step of 64 by r, the tiles a
-// compute unit. Measured with matrices that come from memory (none that a cache still holds), 200 to 3,000 rows, widths of 256 to 32,000. Over
-// 271 such products the one picked here takes 1.009 times the fastest's time on average.
+// compute unit. Measured with matrices that come from memory (none that a cache still holds), 129 to 8,000 rows, widths of 256 to 48,000. Over
+// 617 such products the one picked here takes 1.006 times the fastest's time on average.
 //
-// What bounds a product of few hundred rows is the way of its matrix from memory: a tile's copies reach three to five steps ahead (what
-// its buffers hold; 5 instead of 4 buffers of 64 x 64, 6 of 64 x 32 and 128 x 64), and there are tiles enough for the chip. us before
+// What bounds a product of few hundred rows is the way of its matrix from memory: a tile's copies reach two to five steps ahead (what
+// its buffers hold; two for the 256 x 256 and the 128 x 192 tile, 5 instead of 4 buffers of 64 x 64, 6 of 64 x 32 and 128 x 64), and there are tiles enough for the chip. us before
 // (tiles of 64 x 64 up to 256 x 256, three steps ahead) / now, and the library's product: 300 rows of 1,536 x 1,536 11.1 / 8.1 (10.6), of
 // 2,304 x 1,536 11.4 / 9.4 (16.6), of 1,536 x 4,096 26 / 15.5 (21.1); 140 rows of 1,536 x 4,096 24.6 / 14.7 (15.6); 700 rows of 2,304 x 1,536
 // 15.2 / 11.3 (16.4); 2,048 rows of 2,304 x 1,536 33 / 22.6 (23.7), of 2,816 x 2,048 41.1 / 31.2 (30.4), of 3,072 x 2,048 41.0 / 32.4 (30.5).
