@@ -121,7 +121,7 @@ def test_norm_and_gate_inside_the_32_bit_product(M, N, K):
 @pytest.mark.parametrize("M,N,K,inside", [(3, 352, 64, True), (16, 4096, 128, True), (33, 1024, 100, True), (17, 2064, 128, False), (5, 352, 132, False), (70, 98, 260, False),
                                           (33, 20, 1020, False)])
 def test_when_the_norm_goes_inside_the_32_bit_product(M, N, K, inside):
-    """Launched by the host: up to 128 inner columns and 256 tiles; recorded in a graph: never. The same bits each way."""
+    """Up to 128 inner columns and 256 tiles, launched and in a graph. The same bits each way."""
     ops = hip_ops.HipOps("cuda:0", torch.float32)
     g = torch.Generator().manual_seed(M + N + K)
     x, w, gain = (torch.randn(M, K, generator=g) * 3).cuda(), torch.randn(N, K, generator=g).cuda(), torch.randn(K, generator=g).cuda()
@@ -141,7 +141,7 @@ def test_when_the_norm_goes_inside_the_32_bit_product(M, N, K, inside):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(out, want))
-    assert len(norms) == 2
+    assert len(norms) == (0 if inside else 2)
 
 
 @pytest.mark.parametrize("groups,rows,top,N,K", [(64, 40, 2, 96, 1024), (70, 127, 2, 520, 136), (33, 17, 3, 64, 2048), (2, 23, 2, 132, 40), (130, 100, 1, 48, 264)])

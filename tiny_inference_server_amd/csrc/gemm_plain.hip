@@ -246,10 +246,11 @@ TIS_EXPORT int tis_gemm_plain_fuses(int M, int N, int K) {
   return M > 0 && N > 0 && K > 0 && K % 4 == 0 && K <= 1024 && tis_gemm_plain_few(1, M, N, K) && (M + GS_BM - 1) / GS_BM <= 65535;
 }
 
-// Whether such a product is worth taking the norm inside where the host launches it: a launch there is 5 us of the host's time, which a model of this
-// size waits for. Recorded in a graph the norm's own kernel is the faster at every size, us, norm and product / one kernel: 4 rows of 176 x 64 5.3 / 5.6,
-// 128 of 1,024 x 64 6.1 / 7.5, 16 of 2,048 x 128 6.0 / 7.2; beyond 128 inner columns, or 256 tiles, by more than a launch: 16 rows of 2,048 x 512 9.3 / 12.8, 128 of
-// 2,048 x 128 9.4 / 15.3, 512 of 2,048 x 1,024 93 / 216.
+// Whether such a product is worth taking the norm inside. On the GPU the norm's own kernel is the faster at every size, us in a graph of such pairs, norm and
+// product / one kernel: 4 rows of 176 x 64 5.3 / 5.6, 128 of 1,024 x 64 6.1 / 7.5, 16 of 2,048 x 128 6.0 / 7.2. But each kernel is the host's time, which
+// steps of models of this size wait for: launched prompts of a 64 wide model, norms inside / apart, 600 / 640 us; replayed, as fast either way.
+// Beyond 128 inner columns, or 256 tiles, it costs more than a launch: 16 rows of 2,048 x 512 9.3 / 12.8, 128 of 2,048 x 128 9.4 / 15.3, 512 of 2,048 x 1,024
+// 93 / 216.
 TIS_EXPORT int tis_gemm_plain_norms(int M, int N, int K) {
   return tis_gemm_plain_fuses(M, N, K) && K <= 128 && (long)((N + GS_BN - 1) / GS_BN) * ((M + GS_BM - 1) / GS_BM) <= 256;
 }

@@ -943,8 +943,8 @@ class HipOps:
                 and bool(self.gemm_plain.cdll.tis_gemm_plain_fuses(x.shape[0], w.shape[0], x.shape[1])))
 
     def _plain_norms(self, M, N, K):
-        """Whether that norm is worth having in there: where the host launches each kernel, not where they are recorded (the same bits)."""
-        return bool(self.gemm_plain.cdll.tis_gemm_plain_norms(M, N, K)) and not torch.cuda.is_current_stream_capturing()
+        """Whether that norm is worth having in there (the same bits)."""
+        return bool(self.gemm_plain.cdll.tis_gemm_plain_norms(M, N, K))
 
     def _linear_plain_fused(self, x, w, rms, residual, out, gate):
         (M, K), N = x.shape, w.shape[0]
