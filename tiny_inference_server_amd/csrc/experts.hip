@@ -100,12 +100,7 @@ __global__ __launch_bounds__(TIS_WAVE) void route_topk_kernel(const float* __res
       const int e = lane + u * TIS_WAVE;
       if (e < n_out && c[u] > best) { best = c[u]; at = e; }       // rising e within a lane: the lower index keeps a tie
     }
-#pragma unroll
-    for (int o = TIS_WAVE / 2; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o, TIS_WAVE);
-      const int oa = __shfl_xor(at, o, TIS_WAVE);
-      if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
-    }
+    wave_argmax(best, at);
     float w = 0.f;
 #pragma unroll
     for (int u = 0; u < PER; ++u) {

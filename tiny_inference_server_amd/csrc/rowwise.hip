@@ -32,7 +32,8 @@ __global__ __launch_bounds__(ROW_THREADS) void rmsnorm_kernel(const T* x, long x
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
 // The same norm for bfloat16 rows whose width is a multiple of 8 and whose rows start on 16 bytes: every thread
-// moves 16 bytes at a time and keeps its values in registers between the two passes.
+// moves 16 bytes at a time and keeps its values in registers between the two passes. The gains are asked for with the values: after the sum
+// they would be a second trip to memory.
 template <int PER_THREAD>
 __global__ __launch_bounds__(ROW_THREADS) void rmsnorm_bf16_vec_kernel(const bf16* __restrict__ x, long x_ld,
                                                                        const float* __restrict__ gain,
@@ -43,12 +44,21 @@ __global__ __launch_bounds__(ROW_THREADS) void rmsnorm_bf16_vec_kernel(const bf1
   const bf16* xr = x + r * x_ld;
   bf16* yr = y + r * y_ld;
   bf16x8 v[PER_THREAD];
+  float4 g[PER_THREAD][2];
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < PER_THREAD; ++i) {
     const int c = (i * ROW_THREADS + threadIdx.x) * 8;
     if (c < D) {
       v[i] = *reinterpret_cast<const bf16x8*>(xr + c);
+      g[i][0] = *reinterpret_cast<const float4*>(gain + c);
+      g[i][1] = *reinterpret_cast<const float4*>(gain + c + 4);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < PER_THREAD; ++i) {
+    const int c = (i * ROW_THREADS + threadIdx.x) * 8;
+    if (c < D) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float f = static_cast<float>(v[i][e]);
@@ -62,11 +72,10 @@ __global__ __launch_bounds__(ROW_THREADS) void rmsnorm_bf16_vec_kernel(const bf1
   for (int i = 0; i < PER_THREAD; ++i) {
     const int c = (i * ROW_THREADS + threadIdx.x) * 8;
     if (c < D) {
-      const float4 g0 = *reinterpret_cast<const float4*>(gain + c), g1 = *reinterpret_cast<const float4*>(gain + c + 4);
-      const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+      const float gs[8] = {g[i][0].x, g[i][0].y, g[i][0].z, g[i][0].w, g[i][1].x, g[i][1].y, g[i][1].z, g[i][1].w};
       bf16x8 w;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) w[e] = static_cast<__bf16>(static_cast<float>(v[i][e]) * mul * g[e]);
+      for (int e = 0; e < 8; ++e) w[e] = static_cast<__bf16>(static_cast<float>(v[i][e]) * mul * gs[e]);
       *reinterpret_cast<bf16x8*>(yr + c) = w;
     }
   }

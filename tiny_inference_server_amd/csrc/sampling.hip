@@ -28,19 +28,17 @@ __device__ __forceinline__ unsigned order_key(float v) {
 
 // (value, index) arg-max over the block; lowest index wins ties. Result valid in every thread.
 __device__ __forceinline__ void block_argmax(float& v, int& ix, float* sv, int* si) {
-#pragma unroll
-  for (int o = TIS_WAVE / 2; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o, TIS_WAVE);
-    const int oi = __shfl_xor(ix, o, TIS_WAVE);
-    if (ov > v || (ov == v && oi < ix)) { v = ov; ix = oi; }
-  }
+  wave_argmax(v, ix);
   const int wave = threadIdx.x / TIS_WAVE, lane = threadIdx.x % TIS_WAVE;
   __syncthreads();
   if (lane == 0) { sv[wave] = v; si[wave] = ix; }
   __syncthreads();
-  v = sv[0]; ix = si[0];
-  for (int i = 1; i < SM_THREADS / TIS_WAVE; ++i)
-    if (sv[i] > v || (sv[i] == v && si[i] < ix)) { v = sv[i]; ix = si[i]; }
+  static_assert(SM_THREADS / TIS_WAVE == 16, "every 16 lanes take the waves' results");
+  v = sv[lane % 16]; ix = si[lane % 16];
+  argmax_step<8>(v, ix);
+  argmax_step<4>(v, ix);
+  argmax_step<2>(v, ix);
+  argmax_step<1>(v, ix);
 }
 
 struct SampleShared {
@@ -518,6 +516,7 @@ TIS_EXPORT int tis_sample(const float* logits, long ld, float* work, int rows, i
   return tis_launch_status("sample");
 }
 
+static constexpr int AM_AHEAD = 6;
 __global__ __launch_bounds__(SM_THREADS) void argmax_kernel(const float* __restrict__ logits, long ld, int V,
                                                             int* __restrict__ out_tokens) {
   __shared__ float sv[16];
@@ -527,17 +526,20 @@ __global__ __launch_bounds__(SM_THREADS) void argmax_kernel(const float* __restr
   int mi = 0x7fffffff;
   const float* row = logits + r * ld;
   if ((((uintptr_t)row) & 15) == 0) {
-    // four values a load, two loads in flight; a thread meets its indices in rising order, so ">" keeps the lowest
+    // four values a load, AM_AHEAD loads in flight (what bounds a row of some ten thousand: one workgroup's trips to memory, two of them at 48,000
+    // values where two loads at a time make six; with the waves' results met by lane moves 7.4 / 5.5 us); a thread meets its indices in rising order, so ">" keeps the lowest
     const int V4 = V & ~3;
-    for (int i = threadIdx.x * 4; i < V4; i += 2 * SM_THREADS * 4) {
-      const int j = i + SM_THREADS * 4;
-      const float4 a = *reinterpret_cast<const float4*>(row + i);
-      const float4 b = j < V4 ? *reinterpret_cast<const float4*>(row + j) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-      const float va[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    for (int i0 = threadIdx.x * 4; i0 < V4; i0 += AM_AHEAD * SM_THREADS * 4) {
+      float4 v[AM_AHEAD];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int at = (e < 4 ? i : j - 4) + e;
-        if (va[e] > mv) { mv = va[e]; mi = at; }
+      for (int u = 0; u < AM_AHEAD; ++u) v[u] = *reinterpret_cast<const float4*>(row + min(i0 + u * SM_THREADS * 4, V4 - 4));
+#pragma unroll
+      for (int u = 0; u < AM_AHEAD; ++u) {
+        const int at = i0 + u * SM_THREADS * 4;
+        const float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (at < V4 && e[k] > mv) { mv = e[k]; mi = at + k; }
       }
     }
     for (int i = V4 + threadIdx.x; i < V; i += SM_THREADS) {
