@@ -10,6 +10,10 @@
 // position p gets slope[h] * (j - p) added (a bias linear in the distance; null: none).
 // Keys are walked in chunks of a fixed size with a running maximum, so the order of every sum depends on
 // the row's own length only, not on what else is in the batch.
+//
+// What bounds it is the chain of trips to memory and through LDS of one small workgroup: the row's position and request, the block table, a
+// key's channels and the values, which are asked for together (rows of up to 50 keys, 8 heads of 8, 32-bit, us: one channel and one value after
+// the other 6.1, AG_AHEAD pieces of 16 bytes of a key and AG_AHEAD values of a thread at a time 5.1). The sums keep their order.
 #include "common.h"
 
 TIS_DEFINE_LAST_ERROR(tis_attention_generic)
@@ -17,8 +21,12 @@ TIS_DEFINE_LAST_ERROR(tis_attention_generic)
 static constexpr int AG_THREADS = 256;
 static constexpr int AG_CHUNK = 1024;
 static constexpr int AG_MAX_HD = 256;
+static constexpr int AG_AHEAD = 4;
 
-template <typename T>
+// WIDE: a key is read 16 bytes at a time
+template <typename T> struct alignas(16) AgPiece { T v[16 / sizeof(T)]; };
+
+template <typename T, bool WIDE>
 __global__ __launch_bounds__(AG_THREADS) void attention_generic_kernel(
     const T* __restrict__ q, long q_ld, const T* __restrict__ plane, const int* __restrict__ block_tables, int bt_ld,
     const int* __restrict__ row_seq, const int* __restrict__ positions, T* __restrict__ out, long out_ld,
@@ -52,12 +60,38 @@ __global__ __launch_bounds__(AG_THREADS) void attention_generic_kernel(
   float m = -INFINITY, l = 0.f, acc = 0.f;
   for (int c0 = first; c0 < kv_end; c0 += AG_CHUNK) {
     const int n = min(AG_CHUNK, kv_end - c0);
+    // a thread's values of the keys g + u groups, u from u0 on (past the chunk's last: that one's)
+    float ahead[AG_AHEAD];
+    auto values = [&](int u0) {
+#pragma unroll
+      for (int u = 0; u < AG_AHEAD; ++u) {
+        const int j = c0 + min(g + (u0 + u) * groups, n - 1);
+        const T* vp = plane + (long)bt[j / page_size] * page_stride + v_off + (j % page_size);
+        ahead[u] = to_f(vp[(long)d * page_size]);  // values lie transposed: [head_dim][slot]
+      }
+    };
+    values(0);                                     // under way while the scores are worked out
     float cmax = -INFINITY;
     for (int i = t; i < n; i += AG_THREADS) {
       const int j = c0 + i;
       const T* kp = plane + (long)bt[j / page_size] * page_stride + k_off + (long)(j % page_size) * HD;
       float s = 0.f;
-      for (int e = 0; e < HD; ++e) s += qs[e] * to_f(kp[e]);
+      if constexpr (WIDE) {
+        constexpr int PIECE = 16 / sizeof(T);
+        for (int e0 = 0; e0 < HD; e0 += AG_AHEAD * PIECE) {
+          AgPiece<T> piece[AG_AHEAD];
+#pragma unroll
+          for (int u = 0; u < AG_AHEAD; ++u) piece[u] = *reinterpret_cast<const AgPiece<T>*>(kp + min(e0 + u * PIECE, HD - PIECE));
+#pragma unroll
+          for (int u = 0; u < AG_AHEAD; ++u) {
+            if (e0 + u * PIECE >= HD) break;
+#pragma unroll
+            for (int e = 0; e < PIECE; ++e) s += qs[e0 + u * PIECE + e] * to_f(piece[u].v[e]);
+          }
+        }
+      } else {
+        for (int e = 0; e < HD; ++e) s += qs[e] * to_f(kp[e]);
+      }
       if (slopes) s += slope * (float)(j - pos);
       sc[i] = s;
       cmax = fmaxf(cmax, s);
@@ -75,11 +109,12 @@ __global__ __launch_bounds__(AG_THREADS) void attention_generic_kernel(
     l = l * rescale + csum;
     acc *= rescale;
     m = m_new;
-    if (pv_thread) {
-      for (int i = g; i < n; i += groups) {
-        const int j = c0 + i;
-        const T* vp = plane + (long)bt[j / page_size] * page_stride + v_off + (j % page_size);
-        acc += sc[i] * to_f(vp[(long)d * page_size]);  // values lie transposed: [head_dim][slot]
+    for (int u0 = 0; g + u0 * groups < n; u0 += AG_AHEAD) {
+      if (u0) values(u0);
+#pragma unroll
+      for (int u = 0; u < AG_AHEAD; ++u) {
+        const int i = g + (u0 + u) * groups;
+        if (pv_thread && i < n) acc += sc[i] * ahead[u];
       }
     }
     __syncthreads();  // sc[] is rewritten by the next chunk
@@ -88,6 +123,7 @@ __global__ __launch_bounds__(AG_THREADS) void attention_generic_kernel(
   __syncthreads();
   if (t < HD) {
     float o = 0.f;
+#pragma unroll 8
     for (int gg = 0; gg < groups; ++gg) o += accm[gg * HD + t];
     out[r * out_ld + (long)h * HD + t] = from_f<T>(o / l);
   }
@@ -106,15 +142,20 @@ TIS_EXPORT int tis_attention_generic(int dtype, const void* q, long q_ld, const 
   if (n_heads > 65535) return tis_fail("attention: %d heads exceed the grid", n_heads);
   dim3 grid(rows, n_heads);
   const int group = n_heads / n_kv_heads;
-  if (dtype == TIS_F32)
-    attention_generic_kernel<float><<<grid, AG_THREADS, 0, stream>>>(
-        (const float*)q, q_ld, (const float*)plane, block_tables, bt_ld, row_seq, positions, (float*)out, out_ld, group,
-        n_kv_heads, head_dim, page_size, window, scale, slopes);
-  else if (dtype == TIS_BF16)
-    attention_generic_kernel<bf16><<<grid, AG_THREADS, 0, stream>>>(
-        (const bf16*)q, q_ld, (const bf16*)plane, block_tables, bt_ld, row_seq, positions, (bf16*)out, out_ld, group,
-        n_kv_heads, head_dim, page_size, window, scale, slopes);
-  else
+  const bool wide = (uintptr_t)plane % 16 == 0 && head_dim * (dtype == TIS_F32 ? 4 : 2) % 16 == 0;     // keys start on 16 bytes
+#define LAUNCH(T, W)                                                                                                          \
+  attention_generic_kernel<T, W><<<grid, AG_THREADS, 0, stream>>>((const T*)q, q_ld, (const T*)plane, block_tables, bt_ld, row_seq,       \
+                                                                  positions, (T*)out, out_ld, group, n_kv_heads, head_dim, page_size,  \
+                                                                  window, scale, slopes)
+  if (dtype == TIS_F32) {
+    if (wide) LAUNCH(float, true);
+    else LAUNCH(float, false);
+  } else if (dtype == TIS_BF16) {
+    if (wide) LAUNCH(bf16, true);
+    else LAUNCH(bf16, false);
+  } else {
     return tis_fail("unknown dtype code %d", dtype);
+  }
+#undef LAUNCH
   return tis_launch_status("attention_generic");
 }

@@ -3,6 +3,8 @@
 // precision mode is used here; inputs may be stored as float or bfloat16 and are widened exactly.
 // Each output element sums its K products in the same order whatever M is, so a row's result does not
 // depend on the other rows of the batch.
+#include <type_traits>
+
 #include "common.h"
 
 TIS_DEFINE_LAST_ERROR(tis_gemm_plain)
@@ -78,7 +80,7 @@ static constexpr int GS_BM = 16, GS_BN = 16, GS_BK = 256, GS_LD = GS_BK + 4;
 // NORM: A's rows are RMS-normed on the way in, x * sqrt(K) / (||x|| + eps) * gain with the sum of squares added up in the order of the
 // norm's own kernel (256 threads a row, four waves); GATE: C has N / 2 columns, silu(g) u of the columns' pairs (2j, 2j + 1). Both give the
 // bits of the separate kernels. GATE saves a kernel (us, product and gate's kernel / one: 16 x 64 x 352 5.2 / 3.5, 128 x 1,024 x 2,048 26 / 24; faster at all
-// of 370 sizes). NORM saves a launch, but not time on the GPU: every column tile sums its 16 rows' squares again before its first product (see
+// of 370 sizes). NORM saves a launch, and little time on the GPU: every column tile sums its 16 rows' squares again before its first product (see
 // tis_gemm_plain_norms).
 template <bool VEC, typename TI, typename TO, bool NORM = false, bool GATE = false>
 __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI* __restrict__ A, long lda, const TI* __restrict__ W,
@@ -143,26 +145,41 @@ __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI*
   fetch(0);
   if constexpr (NORM) {
     const int lane = t % TIS_WAVE, wave = t / TIS_WAVE;
-    float ss[4][4];                                      // a wave's four rows, and the four waves that would share each
+    // NV: of the four waves that would share a row, those that have values (64 a turn); the others' sums are zeros. A wave's four rows are asked
+    // for at once, from addresses that always hold something (3 rows of 64 against 192 or 352 columns, us: 6.6 row after row, 16 sums a wave; 4.6 so).
+    auto squares = [&](auto nv) {
+      constexpr int NV = nv;
+      float ss[4][NV];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const long row = m0 + wave * 4 + r;
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        ss[r][v] = 0.f;
-        for (int k = v * TIS_WAVE + lane; k < K; k += 4 * TIS_WAVE) {
-          const float x = row < M ? to_f(A[row * lda + k]) : 0.f;
-          ss[r][v] += x * x;
-        }
+        for (int v = 0; v < NV; ++v) ss[r][v] = 0.f;
+      for (int k0 = 0; k0 < K; k0 += 4 * TIS_WAVE) {
+        float x[4][NV];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int v = 0; v < NV; ++v)
+            x[r][v] = to_f(A[min(m0 + wave * 4 + r, (long)M - 1) * lda + min(k0 + v * TIS_WAVE + lane, K - 1)]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int v = 0; v < NV; ++v) {
+            const float in = k0 + v * TIS_WAVE + lane < K ? x[r][v] : 0.f;
+            ss[r][v] += in * in;
+          }
       }
-    }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float sum = 0.f;
+      for (int r = 0; r < 4; ++r) {
+        float sum = 0.f;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) sum += wave_sum(ss[r][v]);
-      if (lane == 0) row_mul[wave * 4 + r] = sqrtf((float)K) / (sqrtf(sum) + eps);
-    }
+        for (int v = 0; v < NV; ++v) sum += wave_sum(ss[r][v]);
+        if (lane == 0) row_mul[wave * 4 + r] = sqrtf((float)K) / (sqrtf(sum) + eps);
+      }
+    };
+    if (K <= TIS_WAVE) squares(std::integral_constant<int, 1>{});
+    else if (K <= 2 * TIS_WAVE) squares(std::integral_constant<int, 2>{});
+    else squares(std::integral_constant<int, 4>{});
     __syncthreads();
   }
   commit(0);
