@@ -1,4 +1,5 @@
-"""Small kernels that wait for memory more than they work: attention of the general kernel and the arg-max."""
+"""Small kernels that wait for memory more than they work: attention of the general kernel, the arg-max, and the arrays that a captured step
+takes from the host by itself."""
 from __future__ import annotations
 
 import pytest
@@ -59,3 +60,34 @@ def test_argmax(V):
         rows = torch.zeros(10, -(-V // 4) * 4 + 4 + shift, device="cuda")[:, shift:V + shift]
         rows.copy_(x)
         assert ops.argmax(rows).cpu().tolist()[:9] == x.argmax(-1).tolist()[:9]
+
+
+@pytest.mark.parametrize("ints", [4, 2044, 2048, 2052, 16384, 40004])
+def test_a_captured_step_takes_its_arrays_from_the_host(ints):
+    """Replays take the two sets in turn, with other work between them, two of them launched before either is waited for; the GPU says how many have been taken."""
+    ops = hip_ops.HipOps("cuda:0", torch.bfloat16)
+    n = ops.upload_counters(ints)
+    assert n == min(8, max(1, -(-ints // 2048)))
+    ring = torch.zeros(2, ints, dtype=torch.int32, pin_memory=True)
+    sent, done = torch.zeros(n, dtype=torch.int32, device="cuda"), torch.zeros(n, dtype=torch.int32, pin_memory=True)
+    out, seen = torch.zeros(ints, dtype=torch.int32, device="cuda"), torch.zeros(ints, dtype=torch.int32, device="cuda")
+    ops.upload_ring(ring, out, sent, done)               # (launched, then captured: the counters go on)
+    torch.cuda.synchronize()
+    assert done.tolist() == [1] * n
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.upload_ring(ring, out, sent, done)
+        torch.add(out, 0, out=seen)
+    for k in range(1, 12, 2):
+        want = [torch.arange(ints, dtype=torch.int32) * (k + u) + 7 * u for u in (0, 1)]
+        got = []
+        for u in (0, 1):
+            ring[(k + u) % 2].copy_(want[u])
+            graph.replay()
+            got.append(seen.clone())
+        torch.cuda.synchronize()
+        assert done.tolist() == [k + 2] * n
+        for a, b in zip(got, want):
+            assert torch.equal(a.cpu(), b)
+    with pytest.raises(hip_ops.KernelError):
+        ops.upload_ring(ring[:, :-2], out, sent, done)

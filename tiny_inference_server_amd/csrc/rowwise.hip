@@ -199,6 +199,51 @@ TIS_EXPORT int tis_gather_rows(int dtype, const void* src, long src_ld, const vo
   return tis_launch_status("gather_rows");
 }
 
+// ---- a captured step's arrays -----------------------------------------------------------------------------------------
+//
+// The first kernel of a captured step brings the step's integer arrays from pinned host memory to where the step's other kernels read them:
+// the host only writes memory and launches the graph. `ring` holds two sets; every workgroup counts the replays itself (sent), takes the sets
+// in turn, and says in host memory (done) how many it has read, so that the host knows when it may write a set again without asking the
+// runtime. What bounds it is one trip over the bus. (A copy beside the graph and an event behind it, for the same purpose, were two more
+// calls of the runtime before the graph's launch and two more stops of the queue: 13 us of the host and about as much of the GPU a step.)
+static constexpr int UPLOAD_THREADS = 256, UPLOAD_PER = 4, UPLOAD_BLOCKS = 8;
+
+__global__ __launch_bounds__(UPLOAD_THREADS) void upload_ring_kernel(const uint64_t* ring, int words, uint64_t* __restrict__ dst, uint32_t* sent,
+                                                                     uint32_t* done) {
+  const uint32_t turn = sent[blockIdx.x];
+  const uint64_t* src = ring + (turn & 1 ? words : 0);
+  const int step = gridDim.x * UPLOAD_THREADS;
+  for (int i0 = blockIdx.x * UPLOAD_THREADS + threadIdx.x; i0 < words; i0 += UPLOAD_PER * step) {
+    uint64_t v[UPLOAD_PER];
+#pragma unroll
+    for (int u = 0; u < UPLOAD_PER; ++u)           // (system scope: past the caches, which may hold the set of two replays ago)
+      v[u] = __hip_atomic_load(src + min(i0 + u * step, words - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+    for (int u = 0; u < UPLOAD_PER; ++u)
+      if (i0 + u * step < words) dst[i0 + u * step] = v[u];
+  }
+  __syncthreads();                                 // every thread has what it asked for, and has read `sent`
+  if (threadIdx.x == 0) {
+    sent[blockIdx.x] = turn + 1;
+    __hip_atomic_store(done + blockIdx.x, turn + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// How many workgroups (counters) the arrays take.
+TIS_EXPORT int tis_upload_ring_blocks(int words) {
+  const int n = (words + UPLOAD_THREADS * UPLOAD_PER - 1) / (UPLOAD_THREADS * UPLOAD_PER);
+  return n < 1 ? 1 : n > UPLOAD_BLOCKS ? UPLOAD_BLOCKS : n;
+}
+
+// ring: [2][words] in pinned host memory, words of 8 bytes; dst: [words] on the device; sent: one counter a workgroup, on the device, zero at
+// first; done: the same in pinned host memory.
+TIS_EXPORT int tis_upload_ring(const void* ring, int words, void* dst, void* sent, void* done, hipStream_t stream) {
+  if (words < 1 || (((uintptr_t)ring | (uintptr_t)dst) % 8) || (((uintptr_t)sent | (uintptr_t)done) % 4))
+    return tis_fail("upload_ring: %d words, or arrays that are not aligned", words);
+  upload_ring_kernel<<<tis_upload_ring_blocks(words), UPLOAD_THREADS, 0, stream>>>((const uint64_t*)ring, words, (uint64_t*)dst, (uint32_t*)sent, (uint32_t*)done);
+  return tis_launch_status("upload_ring");
+}
+
 TIS_EXPORT int tis_copy_rows(int dtype, const void* src, long src_ld, const int* src_index, void* dst, long dst_ld,
                              const int* dst_index, int count, int D, hipStream_t stream) {
   if (count == 0) return 0;

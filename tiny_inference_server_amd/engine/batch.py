@@ -88,8 +88,8 @@ class _Packer:
         """What must be equal for two packings to share one device buffer."""
         return tuple(self.offsets)
 
-    def fill(self, host: torch.Tensor) -> None:
-        flat = host.numpy()
+    def fill(self, host) -> None:
+        flat = host if isinstance(host, np.ndarray) else host.numpy()
         for a, (off, _) in zip(self.parts, self.offsets):
             flat[off:off + a.size] = a
 

@@ -3,8 +3,8 @@
 A step in which every request brings exactly one token, far enough into its sequence that every stage has
 one row per request, always launches the same kernels on arrays of the same shapes. Such a step is
 captured once per (number of requests, block-table width) as a HIP graph over a fixed device buffer that
-holds the step's integer arrays; later steps of the same shape copy their arrays into that buffer and
-replay the graph, which removes the launch cost of several hundred small kernels. Any other step is captured
+holds the step's integer arrays; later steps of the same shape write their arrays into pinned memory, from where the
+graph's first kernel takes them, and replay the graph, which removes the launch cost of several hundred small kernels. Any other step is captured
 the same way once its exact shape (row counts, wanted places, attention work) has come three times.
 
 Nothing is cleared inside the graph with a memset, and the first steps of a shape run without a graph (the
@@ -13,6 +13,7 @@ library chooses its algorithms for the shape then), so a capture records kernel 
 from __future__ import annotations
 
 import gc
+import time
 
 import numpy as np
 import torch
@@ -48,11 +49,23 @@ class DecodeGraph:
         self.capture = capture
         dev = engine.device
         on_gpu = torch.device(dev).type == "cuda"
-        self.host = torch.zeros(max(plan.packer.total, 4), dtype=torch.int32, pin_memory=on_gpu)
-        self.dev = torch.zeros(max(plan.packer.total, 4), dtype=torch.int32, device=dev)
-        self.copied = torch.cuda.Event() if on_gpu else _NoEvent()
-        self.flat = self.host.numpy()
-        self.step = materialize(plan, dev, self.host, self.dev)
+        total = max(plan.packer.total, 4)
+        self.uploads = on_gpu and capture and hasattr(engine.ops, "upload_ring")
+        # Two sets of the arrays, written in turn, where the graph itself takes them from the host (upload_ring); else one, which is copied
+        # before every replay.
+        self.ring = torch.zeros(2 if self.uploads else 1, total, dtype=torch.int32, pin_memory=on_gpu)
+        self._sets = list(self.ring.numpy())
+        self._at = 0                 # the set that the next replay takes ...
+        self._held = 0               # ... and the one that holds what the last step left
+        self.dev = torch.zeros(total, dtype=torch.int32, device=dev)
+        self.copied = torch.cuda.Event() if on_gpu and not self.uploads else _NoEvent()
+        self.replays = 0
+        if self.uploads:
+            counters = engine.ops.upload_counters(total)
+            self._sent = torch.zeros(counters, dtype=torch.int32, device=dev)
+            self._done = torch.zeros(counters, dtype=torch.int32, pin_memory=True)
+            self._read = self._done.numpy().view(np.uint32)
+        self.step = materialize(plan, dev, self.ring[0], self.dev)
         for st in self.step.stages:          # later steps of the shape may see more keys than this one
             st.max_kv_len = kv_capacity
         self.graph = None
@@ -71,7 +84,7 @@ class DecodeGraph:
             finally:
                 if collecting:
                     gc.enable()
-        self.copied.record()
+        self.copied.record()         # (with two sets: the copy that `materialize` made was waited for before the capture)
         # what the quick update needs: which requests, in which order, the buffer holds, and where their arrays lie
         self.slots = tuple(e.slot for e in plan.entries)
         self.occupants = tuple(occupants) if occupants is not None else None
@@ -81,6 +94,15 @@ class DecodeGraph:
         self.table_at = {g: (off(i), plan.packer.offsets[i][1]) for g, i in plan.bt_ids.items()}
         self.stage_at = [dict(lag=pl["lag"], tokens=off(pl["tokens"]), positions=off(pl["positions"]),
                               ws={g: off(i) for g, i in pl["ws"].items()}) for pl in plan.plans]
+        # the same for all stages at once: where the requests' positions go [stages, requests], and for each group of pages, of the stages
+        # that write to it, where their slots go and where the requests' block tables begin
+        line = np.arange(len(self.slots))
+        slots = {}
+        for g, (t_off, (_, width)) in self.table_at.items():
+            stages = [j for j, st in enumerate(self.stage_at) if g in st["ws"]]
+            if stages:
+                slots[g] = (stages, np.array([self.stage_at[j]["ws"][g] + line for j in stages]), t_off + line * width)
+        self._places = (np.array([st["positions"] + line for st in self.stage_at]), np.array([[st["lag"]] for st in self.stage_at]), slots)
         self.pages_held = {g: np.array([len(engine.cache.groups[g].tables[s]) for s in self.slots])
                            for g in self.table_at}
         # what the parts planned for each stage (work lists of their kernels): where each array lies, in the order
@@ -92,14 +114,68 @@ class DecodeGraph:
 
     def _launch(self):
         engine, n = self.engine, self.step.n_wanted
+        if self.uploads:
+            engine.ops.upload_ring(self.ring, self.dev, self._sent, self._done)
         outs = engine.model.forward(self.step, engine.cache)
         self.logits = engine.model.all_logits(outs, n) if self.heads else engine.logits_of(outs, self.step, n)
 
+    @property
+    def host(self) -> torch.Tensor:
+        """The arrays as they stand for the next step."""
+        self._carry()
+        return self.ring[self._at]
+
+    def _unread(self) -> int:
+        """How many replays have not yet taken their arrays (which the GPU writes down as it does)."""
+        return max((self.replays - int(n)) & 0xFFFFFFFF for n in self._read) if self.uploads else 0      # (32-bit counters)
+
+    def _free(self) -> np.ndarray:
+        """The set that the next replay takes, once no replay before it still has to read it."""
+        if not self.uploads:
+            self.copied.synchronize()
+        else:
+            waits = 0
+            while self._unread() > 1:
+                waits += 1
+                if waits > 100:
+                    time.sleep(0 if waits < 20000 else 5e-5)
+                if waits % 100000 == 0:           # seconds: either the GPU has that much to do, or it says here what went wrong
+                    torch.cuda.synchronize(self.engine.device)
+                    if self._unread() > 1:
+                        raise RuntimeError("a replayed step never took its arrays")
+        return self._sets[self._at]
+
+    def _carry(self) -> np.ndarray:
+        """The next replay's set, holding what the last step left."""
+        flat = self._free()
+        if self._held != self._at:
+            np.copyto(flat, self._sets[self._held])
+            self._held = self._at
+        return flat
+
     def _replay(self):
+        """The step, on the set that has been filled."""
+        if not self.uploads:
+            self.dev.copy_(self.ring[0], non_blocking=True)
+            self.copied.record()
         if self.graph is not None:
             self.graph.replay()
         else:
             self._launch()
+        self._held = self._at
+        if self.uploads:
+            self.replays += 1
+            self._at ^= 1
+
+    def __del__(self):
+        # A replay that has not started yet reads the sets when it does: they stay until then. (No call of the runtime: a graph may be dropped
+        # while another is being captured.)
+        try:
+            until = time.monotonic() + 10.0
+            while self._unread() and time.monotonic() < until:
+                time.sleep(0)
+        except Exception:            # not made to the end, or the interpreter is going away
+            pass
 
     def holds(self, occupants) -> bool:
         """Whether the buffer's lines are those of exactly these requests, in this order."""
@@ -114,15 +190,14 @@ class DecodeGraph:
         runs it (the caller cannot go on before it has the step's tokens anyway), the buffer is filled for that next
         step; when it comes, only its tokens, and the lines of requests that have taken a page since, are left to
         write before the copy and the replay."""
-        self.copied.synchronize()
-        flat = self.flat
+        flat = self._carry()
         n = len(entries)
         starts = np.fromiter((e.start for e in entries), dtype=np.int64, count=n)
         tokens = np.fromiter((e.tokens[0] for e in entries), dtype=np.int32, count=n)
         ahead, self._ahead = self._ahead, None
         if ahead is not None and len(ahead[0]) == n and np.array_equal(ahead[0], starts):
-            if len(ahead[1]):
-                self._fill_positions(flat, starts, only=ahead[1])
+            if ahead[1]:
+                self._fill_late(flat, starts, ahead[1])
         else:
             self._fill_positions(flat, starts)
         return self._run_filled(starts, tokens)
@@ -132,58 +207,80 @@ class DecodeGraph:
         run_same_requests for a caller that knows which step this is."""
         starts, late = self._ahead
         self._ahead = None
-        if len(late):
-            self._fill_positions(self.flat, starts, only=late)
+        if late:
+            self._fill_late(self._carry(), starts, late)
         return self._run_filled(starts, tokens)
 
     def _run_filled(self, starts, tokens) -> torch.Tensor:
-        flat, n = self.flat, len(tokens)
+        flat, n = self._carry(), len(tokens)
         for st in self.stage_at:
             flat[st["tokens"]:st["tokens"] + n] = tokens
-        self.dev.copy_(self.host, non_blocking=True)
-        self.copied.record()
         self._replay()
-        # the buffer for the step after this one, while this one runs (the copy above has to have left the buffer)
-        self.copied.synchronize()
+        # the arrays of the step after this one, while this one runs
+        flat = self._carry()
         nxt = starts + 1
         if self.cache.spare_slot is not None:       # (lines that fill the step up stay where they are)
             nxt = nxt - np.fromiter((s == self.cache.spare_slot for s in self.slots), dtype=np.int64, count=len(starts))
         self._ahead = (nxt, self._fill_positions(flat, nxt, ahead=True))
         return self.logits
 
-    def _fill_positions(self, flat, starts, only=None, ahead=False):
+    def _table_line(self, flat, g, k, need):
+        """Request k's line of a block table, where it holds fewer than `need` pages; False where the request has not got them either."""
+        held = self.pages_held[g][k]
+        if need <= held:
+            return True
+        t_off, (_, width) = self.table_at[g]
+        t = self.cache.groups[g].tables[self.slots[k]]
+        if len(t) < need:
+            return False
+        if len(t) > width:
+            raise RuntimeError("a block table outgrew the captured width")
+        at = t_off + k * width
+        if self.engine._has_windows:                # (pages that a window has passed are given back: the whole line)
+            flat[at:at + len(t)] = [p if p >= 0 else 0 for p in t]
+        else:
+            flat[at + held:at + len(t)] = t[held:]
+        self.pages_held[g][k] = len(t)
+        return True
+
+    def _fill_late(self, flat, starts, late):
+        """What _fill_positions writes, for the few requests it left out ahead of the step because their positions open pages."""
+        ps = self.page_size
+        for k in late:
+            start = int(starts[k])
+            for g in self.table_at:
+                if not self._table_line(flat, g, k, start // ps + 1):
+                    raise RuntimeError("a request's position lies beyond its pages")
+            for st in self.stage_at:
+                pos = start - st["lag"]
+                flat[st["positions"] + k] = pos
+                for g, w_off in st["ws"].items():
+                    t_off, (_, width) = self.table_at[g]
+                    flat[w_off + k] = flat[t_off + k * width + pos // ps] * ps + pos % ps
+
+    def _fill_positions(self, flat, starts, ahead=False):
         """Positions, write slots, newly taken pages and the parts' work lists for requests that stand at `starts`.
-        only: the indices of the requests whose lines are to be written (the others' are right already).
         ahead: the step has not come yet, so a request whose position opens a page may not have that page; such
         requests are skipped and their indices returned, to be filled when the step comes."""
         n = len(starts)
         ps = self.page_size
-        late = np.zeros(0, dtype=np.int64)
-        for g, (t_off, (rows, width)) in self.table_at.items():
-            tables = self.cache.groups[g].tables
-            need = starts // ps + 1
-            for k in np.nonzero(need > self.pages_held[g])[0]:
-                t = tables[self.slots[k]]
-                if len(t) < need[k]:
+        late = []
+        need = starts // ps + 1
+        for g in self.table_at:
+            for k in np.nonzero(need > self.pages_held[g])[0].tolist():
+                if not self._table_line(flat, g, k, int(need[k])):
                     if not ahead:
                         raise RuntimeError("a request's position lies beyond its pages")
-                    late = np.union1d(late, [k])
-                    continue
-                if len(t) > width:
-                    raise RuntimeError("a block table outgrew the captured width")
-                flat[t_off + k * width:t_off + k * width + len(t)] = [p if p >= 0 else 0 for p in t]
-                self.pages_held[g][k] = len(t)
-        which = np.arange(n) if only is None else np.asarray(only, dtype=np.int64)
-        if ahead and len(late):
-            which = np.setdiff1d(which, late)
-        for st in self.stage_at:
-            pos = starts[which] - st["lag"]
-            flat[st["positions"] + which] = pos
-            for g, w_off in st["ws"].items():
-                t_off, (rows, width) = self.table_at[g]
-                table = flat[t_off:t_off + rows * width].reshape(rows, width)
-                flat[w_off + which] = table[which, pos // ps] * ps + pos % ps
-        if only is None and any(self.extras_at):
+                    if k not in late:
+                        late.append(k)
+        which = [k for k in range(n) if k not in late] if late else slice(None)
+        places, lags, slots = self._places
+        pos = starts[which] - lags               # [stages, requests]
+        flat[places[:, which]] = pos
+        page, at = np.divmod(pos, ps)
+        for g, (stages, into, lines) in slots.items():
+            flat[into[:, which]] = flat[lines[which] + page[stages]] * ps + at[stages]
+        if any(self.extras_at):
             # the parts plan again for the new positions, into the places their arrays have in the buffer
             for at, host_values, st in zip(self.extras_at, self.extras_host, self.stage_at):
                 slots_left = list(at)
@@ -205,11 +302,9 @@ class DecodeGraph:
     def run(self, plan: StepPlan, occupants=None) -> torch.Tensor:
         if plan.layout() != self.layout:
             raise RuntimeError("this step's arrays do not have the captured layout")
-        self.copied.synchronize()            # the previous copy out of the pinned buffer has finished
+        flat = self._free()
         self._ahead = None
-        plan.packer.fill(self.host)
-        self.dev.copy_(self.host, non_blocking=True)
-        self.copied.record()
+        plan.packer.fill(flat)
         self.slots = tuple(e.slot for e in plan.entries)
         self.occupants = tuple(occupants) if occupants is not None else None
         for g in self.table_at:

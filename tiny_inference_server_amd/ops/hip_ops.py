@@ -69,6 +69,7 @@ _SIGNATURES = {
         "tis_gather_rows": [_I, _P, _L, _P, _L, _P, _P, _L, _I, _I, _P],
         "tis_copy_rows": [_I, _P, _L, _P, _P, _L, _P, _I, _I, _P],
         "tis_swiglu": [_I, _P, _L, _P, _L, _I, _I, _P],
+        "tis_upload_ring": [_P, _I, _P, _P, _P, _P],
     }),
     "rope_cache": ("tis_rope_cache", {
         "tis_rope_write_kv": [_I, _P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _L, _P],
@@ -861,6 +862,21 @@ class HipOps:
             raise KernelError(f"copy_rows: widths {src.shape[1]} and {dst.shape[1]}")
         self.rowwise.tis_copy_rows(self.code, _ptr(src), src.stride(0), _ptr(src_index), _ptr(dst), dst.stride(0),
                                    _ptr(dst_index), n, src.shape[1], self._stream())
+
+    def upload_counters(self, ints: int) -> int:
+        """How many counters upload_ring keeps for arrays of so many integers."""
+        return self.rowwise.cdll.tis_upload_ring_blocks(ints // 2)
+
+    def upload_ring(self, ring, out, sent, done):
+        """out = ring[k % 2] for the k-th launch on these counters, captured replays included; then done (pinned) = k + 1."""
+        n = out.numel()
+        counters = self.upload_counters(n)
+        for t, shape, what in ((ring, (2, n), "ring"), (out, (n,), "arrays"), (sent, (counters,), "counters"), (done, (counters,), "counters")):
+            if t.dtype != torch.int32 or tuple(t.shape) != shape or not t.is_contiguous():
+                raise KernelError(f"upload_ring: {what} of {t.dtype} {tuple(t.shape)} for {shape} 32-bit integers")
+        if n % 2 or not ring.is_pinned() or not done.is_pinned() or out.device != self.device or sent.device != self.device:
+            raise KernelError("upload_ring: an even number of integers, from pinned memory to the device")
+        self.rowwise.tis_upload_ring(_ptr(ring), n // 2, _ptr(out), _ptr(sent), _ptr(done), self._stream())
 
     def swiglu(self, gu, out=None):
         """out[:, f] = silu(gu[:, 2f]) * gu[:, 2f + 1]: gate and up columns interleaved."""
