@@ -453,6 +453,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NB <= 2 ? 2 
 // the second, in order.
 static constexpr int TW = 4;               // waves of a tile
 static constexpr int TCOLS = 32;           // columns of a wave
+static_assert(TW * TCOLS <= 255, "a tile's rows have eight bits in a list of pieces");
 static constexpr int TBUF = 3;             // LDS buffers: step s+1's keys, step s's values, and step s+2 being written
 static constexpr int NCH = KD / 8;         // 16-byte pieces of one key
 static constexpr int KCH = 4 * KD, VCH = 4 * VD;     // pieces of a step's keys and of its values: KD / 16, VD / 16 fetches of 64
@@ -491,6 +492,20 @@ __device__ __forceinline__ float pair_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// Which piece of work a workgroup of a flat grid takes, of pieces that go from the longest chain of steps to the shortest. A compute unit holds
+// two workgroups (one where heads are wide), and workgroups go to the units in turn: those that come second on their unit take the pieces from
+// the shortest up, so that the longest has the shortest beside it. Workgroups beyond those start as others end, longest first.
+__device__ __forceinline__ int piece_of(int id, int total, int units) {
+  return WIDER <= 128 && id >= units && id < 2 * units ? units + min(2 * units, total) - 1 - id : id;
+}
+
+// What bounds this kernel on a prompt of a few thousand tokens is the longest chain of steps on one compute unit. pieces: the parts of the
+// tiles that there are, longest first, (first row, rows + 256 * split, position, line of the block table), for a flat grid of pieces x
+// key/value heads; or null: tiles that are not cut, flat_units > 0 and a flat grid of tiles x key/value heads; or null and flat_units 0: the grid's
+// dimensions are tile, key/value head and split, and workgroups whose split a tile does not have return. us with the merge, those three dimensions
+// / flat, the same bits: 2,048 tokens, 12 heads of 128 over 3, 45.3 / 35.7; 1,400 28.7 / 27.1; 4,000 92.0 / 77.4; 1,500 of 16 over 4 38.3 / 31.7; 512 behind
+// 3,000 others, 12 over 3, 43.2 / 42.3; not cut, 1,200 of 32 over 8, 42.5 / 38.0. (Most of it is the order; without the workgroups that return, in the old
+// order, 2,048 tokens take 38.3. With the copies a step further ahead, in four buffers, 33.4 where 34.8, but 2 x 1,024 30.4 where 29.9: not in.)
 // (heads wider than 128 need more than 256 registers a lane: one wave a SIMD)
 template <bool PS16>
 __global__ __launch_bounds__(TW * 64) __attribute__((amdgpu_waves_per_eu(WIDER <= 128 ? 2 : 1))) void attention_tile_kernel(
@@ -498,16 +513,32 @@ __global__ __launch_bounds__(TW * 64) __attribute__((amdgpu_waves_per_eu(WIDER <
     int bt_ld, const int* __restrict__ row_seq, const int* __restrict__ positions, const int2* __restrict__ tiles,
     bf16* __restrict__ out, long out_ld, float* __restrict__ part_o, float2* __restrict__ part_ml, int group_size,
     int n_kv_heads, int n_heads, int page_size_arg, int window, float scale_log2, int n_splits, int max_steps,
-    int split_stride, int* __restrict__ row_splits, int sink, const float* __restrict__ sinks, const float2* __restrict__ turn, Extras extras) {
+    int split_stride, int* __restrict__ row_splits, int sink, const float* __restrict__ sinks, const float2* __restrict__ turn, Extras extras,
+    const int4* __restrict__ pieces, int flat_units) {
   __shared__ __attribute__((aligned(16))) bf16 k_lds[TBUF][KCH * 8];
   __shared__ __attribute__((aligned(16))) bf16 v_lds[TBUF][VCH * 8];
   const int page_size = PS16 ? 16 : page_size_arg;
-  const int tile = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
   // the wave's number is the same on all its lanes: said so, what follows from it is scalar arithmetic and branches
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c32 = lane & 31, h = lane >> 5;
-  const int t_row0 = tiles[tile].x, t_rows = tiles[tile].y;
-  const int* bt = block_tables + (long)row_seq[t_row0] * bt_ld;
-  const int tp_first = positions[t_row0], tp_last = tp_first + t_rows - 1;
+  int kvh, split = 0, t_row0, t_rows, tp_first, line;
+  if (pieces) {                       // (what the workgroup would otherwise load next comes with the list)
+    const int piece = piece_of(blockIdx.x, gridDim.x, flat_units);
+    kvh = piece % n_kv_heads;
+    const int4 e = pieces[piece / n_kv_heads];
+    t_row0 = e.x, t_rows = e.y & 255, split = e.y >> 8, tp_first = e.z, line = e.w;
+  } else {
+    int tile;
+    if (flat_units > 0) {
+      const int piece = piece_of(blockIdx.x, gridDim.x, flat_units);
+      kvh = piece % n_kv_heads, tile = piece / n_kv_heads;
+    } else {
+      tile = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
+    }
+    t_row0 = tiles[tile].x, t_rows = tiles[tile].y;
+    tp_first = positions[t_row0], line = row_seq[t_row0];
+  }
+  const int* bt = block_tables + (long)line * bt_ld;
+  const int tp_last = tp_first + t_rows - 1;
 
   // the wave's rows of the tile; a wave past the tile's last row only helps with the copies
   const int rows_per_wave = TCOLS / group_size;
@@ -1033,7 +1064,8 @@ static int attention_launch(const void* q, long q_ld, const void* plane, const i
                             float* part_ml, int rows, int n_heads, int n_kv_heads, int head_dim, int page_size,
                             int window, float scale, int n_splits, int min_steps, int tile_splits,
                             int tile_max_steps, int* row_splits, hipStream_t stream, int sink = 0, const float* sinks = nullptr,
-                            const float2* turn = nullptr, Extras extras = Extras{}) {
+                            const float2* turn = nullptr, Extras extras = Extras{}, const int* pieces = nullptr, int n_pieces = 0,
+                            int units = 0) {
   if ((n_items == 0 && n_tiles == 0) || rows == 0) return 0;
   if (n_items < 0 || n_tiles < 0 || (n_tiles > 0 && !tiles)) return tis_fail("attention_mfma: bad item counts %d, %d", n_items, n_tiles);
   if (head_dim != KD) return tis_fail("attention_mfma: built for head size %d, called with %d", KD, head_dim);
@@ -1055,6 +1087,9 @@ static int attention_launch(const void* q, long q_ld, const void* plane, const i
   if (n_tiles > 0 && 2L * n_kv_heads * page_size * (KD + VD) >= (1L << 31))
     return tis_fail("attention_mfma: a page of %d key/value heads x %d slots is too large for the tile kernel's 32-bit offsets", n_kv_heads, page_size);
   if (n_tiles == 0) tile_splits = 1;
+  if (pieces && (n_pieces < n_tiles || (uintptr_t)pieces % 16 || units < 1))
+    return tis_fail("attention_mfma: a list of %d pieces of %d tiles, 16-byte aligned, for %d compute units", n_pieces, n_tiles, units);
+  if ((long)std::max(n_pieces, n_tiles) * n_kv_heads >= (1L << 31)) return tis_fail("attention_mfma: too many tiles for one grid");
   if (page_size < 16 || page_size % 16) return tis_fail("attention_mfma: page size %d is no multiple of 16", page_size);
   if (n_splits < 1 || n_splits > 65535 || tile_splits < 1 || tile_splits > 65535 || n_kv_heads > 65535)
     return tis_fail("attention_mfma: bad grid %d x %d (tiles: %d)", n_kv_heads, n_splits, tile_splits);
@@ -1112,12 +1147,16 @@ static int attention_launch(const void* q, long q_ld, const void* plane, const i
     rc = tis_launch_status("attention_mfma");
   }
   if (n_tiles > 0 && rc == 0) {
-    dim3 grid(n_tiles, n_kv_heads, tile_splits);
+    // without a list of pieces: a flat grid where no tile is cut and there are more tiles than compute units (with fewer there is nothing to
+    // arrange, and the grid's own dimensions save the divisions: 500 tokens, 12 heads over 3, 17.2 / 17.7; 2 x 1,024 30.6 / 31.4)
+    const int flat_units = pieces || (tile_splits == 1 && (long)n_tiles * n_kv_heads > units) ? units : 0;
+    const dim3 grid = pieces ? dim3((unsigned)(n_pieces * n_kv_heads)) : flat_units > 0 ? dim3((unsigned)(n_tiles * n_kv_heads))
+                                                                                       : dim3(n_tiles, n_kv_heads, tile_splits);
 #define LAUNCH(PSV)                                                                                                   \
   attention_tile_kernel<PSV><<<grid, TW * 64, 0, tile_stream>>>(                                                      \
       (const bf16*)q, q_ld, (const bf16*)plane, block_tables, bt_ld, row_seq, positions, (const int2*)tiles,     \
       (bf16*)out, out_ld, part_o, (float2*)part_ml, group, n_kv_heads, n_heads, page_size, window, scale_log2,   \
-      tile_splits, tile_max_steps, stride, row_splits, sink, sinks, turn, extras)
+      tile_splits, tile_max_steps, stride, row_splits, sink, sinks, turn, extras, (const int4*)pieces, flat_units)
     if (page_size == 16) LAUNCH(true);
     else LAUNCH(false);
 #undef LAUNCH
@@ -1185,6 +1224,26 @@ TIS_EXPORT int tis_attention_mfma_extras(const void* q, long q_ld, const void* p
                           out, out_ld, part_o, part_ml, rows, n_heads, n_kv_heads, head_dim, page_size, window, scale,
                           n_splits, min_steps, tile_splits, tile_max_steps, row_splits, stream, sink, sinks, (const float2*)turn,
                           extras);
+}
+
+// The same for a caller that knows the device's compute units and has the tiles' pieces: pieces (null: none) holds n_pieces entries of four
+// integers, every part of every tile once, (first row, rows + 256 * split, position of the first row, block-table line), those with the longest
+// chains of steps first; a tile has as many parts as tile_splits and tile_max_steps say. In a library built without extras gate is null, softcap 0.
+TIS_EXPORT int tis_attention_mfma_pieces(const void* q, long q_ld, const void* plane, const int* block_tables, int bt_ld,
+                                         const int* row_seq, const int* positions, const int* items, int n_items, int nb,
+                                         const int* tiles, int n_tiles, void* out, long out_ld, float* part_o,
+                                         float* part_ml, int rows, int n_heads, int n_kv_heads, int head_dim, int page_size,
+                                         int window, float scale, int n_splits, int min_steps, int tile_splits,
+                                         int tile_max_steps, int* row_splits, int sink, const float* sinks,
+                                         const float* turn, const float* gate, long gate_ld, float softcap, const int* pieces,
+                                         int n_pieces, int units, hipStream_t stream) {
+  if (softcap < 0.f) return tis_fail("attention_mfma: a cap of %g", (double)softcap);
+  const float log2e = 1.4426950408889634f;
+  const Extras extras{gate, gate_ld, softcap * log2e, softcap > 0.f ? 2.f * log2e * scale / softcap : 0.f};
+  return attention_launch(q, q_ld, plane, block_tables, bt_ld, row_seq, positions, items, n_items, nb, tiles, n_tiles,
+                          out, out_ld, part_o, part_ml, rows, n_heads, n_kv_heads, head_dim, page_size, window, scale,
+                          n_splits, min_steps, tile_splits, tile_max_steps, row_splits, stream, sink, sinks, (const float2*)turn,
+                          extras, pieces, n_pieces, units);
 }
 
 // ---- the same without a workspace argument: partial results in memory that this library owns for good ----

@@ -104,6 +104,8 @@ _SIGNATURES["attention_mfma"] = ("tis_attention_mfma", {
                            _I, _I, _I, _I, _P, _P],
     "tis_attention_mfma_sink": [_P, _L, _P, _P, _I, _P, _P, _P, _I, _I, _P, _I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F,
                                 _I, _I, _I, _I, _P, _I, _P, _P, _P],
+    "tis_attention_mfma_pieces": [_P, _L, _P, _P, _I, _P, _P, _P, _I, _I, _P, _I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F,
+                                  _I, _I, _I, _I, _P, _I, _P, _P, _P, _L, _F, _P, _I, _I, _P],
     "tis_attention_mfma_extras": [_P, _L, _P, _P, _I, _P, _P, _P, _I, _I, _P, _I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F,
                                   _I, _I, _I, _I, _P, _I, _P, _P, _P, _L, _F, _P],
 })
@@ -662,6 +664,26 @@ def attention_launch_plan(n, n_items, n_tiles, tile_steps, single, max_kv_len, n
                            rs_offset + n if stride > 1 else 0)
 
 
+def tile_pieces(seq_rows, tiles, tile_splits: int, tile_max_steps: int, window: int = 0):
+    """The parts that the tile kernel cuts its tiles into, those with the longest chains of steps first: int32 (first row, rows + 256 * split,
+    position of the first row, block-table line) each. The counts are the kernel's own: a tile of n steps of 32 keys, from a multiple of 32 at or before
+    the first key that any row sees, has min(tile_splits, ceil(n / tile_max_steps)) parts of ceil(n / parts) steps, the last what is left."""
+    rows = np.asarray(seq_rows, dtype=np.int64).reshape(-1, 3)
+    first, count = tiles[:, 0].astype(np.int64), tiles[:, 1].astype(np.int64)
+    live = np.nonzero(rows[:, 2] > 0)[0]                     # (first rows rise; of requests without rows none is a tile's)
+    line = live[np.searchsorted(rows[live, 0], first, side="right") - 1]
+    pos = rows[line, 1] + first - rows[line, 0]
+    seen = np.maximum(0, pos - window + 1) if window > 0 else pos - pos % (-window) if window < 0 else 0
+    steps = (pos + count - (seen & ~31) + 31) // 32
+    parts = np.clip(-(-steps // tile_max_steps), 1, tile_splits)
+    per = -(-steps // parts)
+    who = np.repeat(np.arange(len(tiles)), parts)
+    split = np.arange(len(who)) - np.repeat(np.cumsum(parts) - parts, parts)
+    by = np.argsort(-np.minimum(per[who], steps[who] - split * per[who]), kind="stable")
+    who, split = who[by], split[by]
+    return np.stack((first[who], count[who] + 256 * split, pos[who], line[who]), axis=1).astype(np.int32)
+
+
 _side_streams = {}
 
 
@@ -751,6 +773,13 @@ class HipOps:
                 # (a mixer with a window plans for itself: its lists are the same, its keys are its own)
                 plans[("attention_items", group, cols, n_kv_heads, window)] = (add(np.concatenate((items, tiles))), len(items),
                                                                        nb, len(tiles), steps, 0)
+            if len(tiles) and ("attention_items", group, cols, n_kv_heads, window) in plans:
+                lp = attention_launch_plan(sum(n for _, _, n in seq_rows), len(items) if beside is None else len(entries), len(tiles), steps, False,
+                                           max(p0 + n for _, p0, n in seq_rows), n_heads, n_kv_heads, head_dim,
+                                           planned_splits=0 if beside is None else most, units=self.units)
+                if lp.tile_splits > 1:
+                    pieces = tile_pieces(seq_rows, tiles, lp.tile_splits, lp.tile_max_steps, window)
+                    plans[("attention_tile_pieces", group, cols, n_kv_heads, window)] = (add(pieces), len(pieces), lp.tile_splits, lp.tile_max_steps)
         return plans
 
     # ---- helpers -------------------------------------------------------------------------------------
@@ -1353,15 +1382,19 @@ class HipOps:
                 row_splits = self._workspace[lp.row_splits_offset:]
         if lines.dtype != torch.int32 or not lines.is_contiguous():
             raise KernelError("attention: the work list must be contiguous 32-bit integers")
-        args = (_ptr(q), q.stride(0), _ptr(plane), _ptr(tables), tables.stride(0), _ptr(batch.row_seq), _ptr(batch.positions),
-                _ptr(items), n_items, nb, _ptr(tiles), n_tiles, _ptr(out), out.stride(0), _ptr(part_o), _ptr(part_ml), n, n_heads,
-                n_kv_heads, key_dim, page_size, int(window), float(scale), n_splits, min_steps, tile_splits, tile_max_steps,
-                _ptr(row_splits), 1 if sink else 0, _ptr(sinks), _ptr(turn))
-        if extras:
-            lib.tis_attention_mfma_extras(*args, _ptr(channel_gate), channel_gate.stride(0) if channel_gate is not None else 0,
-                                          float(softcap), self._stream())
-        else:
-            lib.tis_attention_mfma_sink(*args, self._stream())
+        pieces, n_pieces = None, 0
+        if tile_splits > 1:
+            made = batch.extras.get(("attention_tile_pieces", group, cols, n_kv_heads, int(window)))
+            if made is not None and made[2:] == (tile_splits, tile_max_steps):      # (planned for these very cuts)
+                pieces, n_pieces = made[0].reshape(-1), made[1]
+                if pieces.dtype != torch.int32 or not pieces.is_contiguous() or pieces.numel() != 4 * n_pieces:
+                    raise KernelError(f"attention: a list of {pieces.numel()} integers for {n_pieces} pieces of tiles")
+        lib.tis_attention_mfma_pieces(
+            _ptr(q), q.stride(0), _ptr(plane), _ptr(tables), tables.stride(0), _ptr(batch.row_seq), _ptr(batch.positions),
+            _ptr(items), n_items, nb, _ptr(tiles), n_tiles, _ptr(out), out.stride(0), _ptr(part_o), _ptr(part_ml), n, n_heads,
+            n_kv_heads, key_dim, page_size, int(window), float(scale), n_splits, min_steps, tile_splits, tile_max_steps,
+            _ptr(row_splits), 1 if sink else 0, _ptr(sinks), _ptr(turn), _ptr(channel_gate),
+            channel_gate.stride(0) if channel_gate is not None else 0, float(softcap), _ptr(pieces), n_pieces, self.units, self._stream())
 
     def _sink(self, sink, n_heads: int):
         """(whether there is a sink, its scores per head or None for zeros) of a `sink` argument: False or None, True, or a
