@@ -563,6 +563,26 @@ def test_the_delta_rules_walk_in_chunks(Hh, G, D, V, seqs):
     assert not torch.isfinite(broken[at]).any()
 
 
+@pytest.mark.parametrize("D", [64, 130])
+def test_a_walk_in_chunks_gives_a_prefix_its_own_bits(D):
+    """Whatever number of chunks follows, and however many of them the last turn of the loop takes: the rows before get the same bits, whole chunks and
+    begun ones."""
+    Hh, G, V, n = 2, 1, 24, 163
+    ops = hip_ops("float32")
+    g = torch.Generator().manual_seed(D)
+    C = 2 * G * D + Hh * V
+    k, q = (torch.nn.functional.normalize(torch.randn(n, G, D, generator=g), dim=-1) for _ in range(2))
+    u = torch.cat([(q * D ** -0.5).reshape(n, -1), k.reshape(n, -1), torch.randn(n, Hh * V, generator=g), torch.rand(n, Hh, generator=g)], 1).cuda()
+    decay = torch.exp(-torch.rand(n, Hh * D, generator=g)).cuda()
+    start = torch.randn(1, Hh * 2 * D * 16, generator=g).cuda()
+
+    def rows(m):
+        return ops.delta_scan(u[:m], 0, G * D, 2 * G * D, C, decay[:m], start.clone(), fake_batch([(0, 0, m)], [0], None, 8, "cuda"), Hh, G, D, V)
+    whole = rows(n)
+    for m in (48, 49, 63, 64, 65, 80, 95, 96, 112, 128, 129, 144, 160):
+        assert torch.equal(rows(m), whole[:m]), m
+
+
 # Rows walked in chunks against the walk row by row, both against 64 bits: the chunks add the same products up in sums of no more terms and
 # in the rows' order, so neither results nor states lie further off. Either error is the norm of some 100,000 independent roundings of
 # which every one weighs the same, so the two would differ by 1 % if their roundings were as many; 8 % leaves room for T, which

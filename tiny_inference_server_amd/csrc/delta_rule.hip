@@ -12,6 +12,8 @@
 // A request's state line holds S and, from float `conv_at` on, the convolution's last taps - 1
 // inputs [taps - 1][channels], oldest first. Rows of the step are grouped by request: request s owns the rows
 // [cu_rows[s], cu_rows[s + 1]) in order of position and the line seq_slots[s].
+#include <type_traits>
+
 #include "common.h"
 
 TIS_DEFINE_LAST_ERROR(tis_delta_rule)
@@ -254,7 +256,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(
 // with T = (I + beta G)^-1 beta, solved column by column. delta_chunks_kernel makes K~, Q~, K^, A, T and Q of every chunk and head,
 // all chunks at once; delta_chunk_walk_kernel walks them with S in registers, all products on v_mfma_f32_16x16x4_f32 (32-bit
 // multiply-adds). Rows past a request's last have k = q = 0, decay 1 and beta 0 and change nothing. MI355X, 8 heads of 128 x 256,
-// us row by row / in chunks with the step before them: 2,048 rows 546 / 199, 1,531 410 / 155, 512 141 / 59, 128 38 / 24. Off from 64 bits, row
+// us row by row / in chunks with the step before them: 2,048 rows 546 / 153, 1,531 410 / 121, 512 141 / 49, 128 38 / 22. Off from 64 bits, row
 // by row / in chunks, by decays from 0.5, 0.9 and 0.995 on: results 0.99e-7 / 0.98e-7, 1.39e-7 / 1.40e-7, 3.3e-7 / 3.0e-7, states 0.62e-7 / 0.62e-7,
 // 1.16e-7 / 1.19e-7, 3.6e-7 / 3.2e-7. (With rows four apart in a product, the newest among the first, 1.15e-7 and 0.87e-7 at the strongest
 // decays, where the newest are the largest; with one sum over a wave's channels 5 % more, and 162 us where the four take 155.)
@@ -381,8 +383,10 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
 // 4 r + g (see dc_place). The waves' parts of K~ S0 meet in LDS, one barrier a chunk; each then makes W for itself. Q~ S0 is worked out while the parts
 // are on their way, and the fifth wave, which makes W too, adds up the rows' results a chunk later. Three chunks' operands are
 // under way (one ahead, a chunk took what memory takes), or one where a head's channels leave no more registers. Workgroups of one head follow one another by `heads`, so that with 8 heads
-// (or 16, ...) an XCD's L2 serves a head to all of its value channels. What bounds it is a chunk's chain: the products with S, LDS, W, and
-// the products that change S.
+// (or 16, ...) an XCD's L2 serves a head to all of its value channels. What bounds it is a chunk's chain (1.05 us): the products with S, LDS, W, and
+// the products that change S. The loop over the chunks is one straight stretch, whose waits let the later chunks' loads be under way; with loads
+// under conditions and the way out for rows that are not finite inside it, every fourth chunk waited for all of them, and a chunk took 1.38 us
+// (1,531 rows of 8 heads of 128 x 256, with the step before them, 151 / 121 us; of 256 x 128 264 / 208).
 template <int NT>
 __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(const float* __restrict__ u, long ldu, int v_off,
                                                                const float* __restrict__ work, float* __restrict__ state, long lds,
@@ -391,6 +395,7 @@ __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(const float* __re
   constexpr int SETS = NT <= 2 ? 4 : 2;          // chunks whose operands are held or under way
   constexpr int Dp = 64 * NT, OFF_A = 3 * DC * Dp, OFF_T = OFF_A + Dp, OFF_Q = OFF_T + DC * DC;
   __shared__ f32x4 ks_parts[2][4][64], qs_parts[2][4][64];       // turn, wave, lane
+  __shared__ int poisoned[5];
   const int h = blockIdx.x, vb = blockIdx.y, s = blockIdx.z, t = threadIdx.x;
   const int first = cu_rows[s], n_rows = cu_rows[s + 1] - first;
   if (n_rows < DR_CHUNK_FROM) return;
@@ -400,146 +405,183 @@ __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(const float* __re
     int c = s0 + lane < s ? dc_chunks(cu_rows[s0 + lane + 1] - cu_rows[s0 + lane]) : 0;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) c += __shfl_xor(c, o, 64);
-    chunk0 += c;
+    chunk0 += __builtin_amdgcn_readfirstlane(c);
   }
   const int c_v = vb * 16 + n;
   const bool live = c_v < V;
-  const float* base = work + ((long)chunk0 * H + h) * dc_floats(Dp);
-  const long stride = (long)H * dc_floats(Dp);
-  const float* v_column = u + (long)first * ldu + v_off + h * V + min(c_v, V - 1);
   const int chunks = (n_rows + DC - 1) / DC;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 
-  // W of chunk c from the four parts of K~ S0 in LDS. T and Q are triangular, but a product takes their zeros times every row: a row that
-  // is not finite must not reach the rows before it, so such a chunk goes without the matrix product.
-  auto triangle = [&](const float* M, f32x4 m, f32x4 x, f32x4 sum) {      // sum + M x, M lower triangular [16][16], m: the lane's four
+  // Everything of a chunk lies at a scalar address (the same on all lanes) plus each lane's own offset in bytes, which never changes; `ahead` is the
+  // chunk that is asked for next, at the last one it stays (its numbers are then asked for again and not used: loads without conditions).
+  const long stride = (long)H * dc_floats(Dp) * 4, v_stride = (long)DC * ldu * 4;
+  const unsigned char* const base = reinterpret_cast<const unsigned char*>(work + ((long)chunk0 * H + h) * dc_floats(Dp));
+  const unsigned char* const v_base = reinterpret_cast<const unsigned char*>(u + (long)first * ldu + v_off + h * V);
+  const unsigned v_row = (unsigned)ldu * 4, v_col = (unsigned)min(c_v, V - 1) * 4;
+  const unsigned t_off = (n * DC + g * 4) * 4;
+  auto four = [](const unsigned char* at, unsigned lane_off) { return *reinterpret_cast<const f32x4*>(at + lane_off); };
+  int ahead;
+  const unsigned char *p, *pv;
+  auto rewind = [&] { ahead = 0, p = base, pv = v_base; };
+  // (rows past the last: the last one's values, which T's zeros keep out)
+  auto fetch_v = [&] {
+    const int last = n_rows - 1 - ahead * DC;      // of the chunk's rows
+    f32x4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = *reinterpret_cast<const float*>(pv + ((unsigned)min(r * 4 + g, last) * v_row + v_col));
+    return v;
+  };
+  auto advance = [&] {
+    const bool more = ahead + 1 < chunks;
+    ahead += more ? 1 : 0;
+    p += more ? stride : 0;
+    pv += more ? v_stride : 0;
+  };
+
+  // T and Q are triangular, but a product takes their zeros times every row: a row that is not finite must not reach the rows before it.
+  // A walk that meets one therefore notes it (`poison` is no number from then on) and is done again, `careful`, where such chunks go without the
+  // matrix product. (With that way out inside the one loop the compiler waits for all loads under way at its beginning, and the loop is four
+  // times as long.)
+  float poison = 0.f;
+  auto triangle = [&](auto careful, f32x4 m, f32x4 x, f32x4 sum) {   // sum + M x, M [16][16], m: the lane's four, row n, columns 4 g .. 4 g + 3
     const float none = fmaf(x[3], 0.f, fmaf(x[2], 0.f, fmaf(x[1], 0.f, x[0] * 0.f)));
-    if (__all(none == 0.f)) {
+    if constexpr (!careful) poison += none;
+    if (!careful || __all(none == 0.f)) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], x[r], sum, 0, 0, 0);
       return sum;
     }
 #pragma unroll 1
-    for (int i = 0; i < DC; ++i) {
-      const float xi = __shfl(i / 4 == 0 ? x[0] : i / 4 == 1 ? x[1] : i / 4 == 2 ? x[2] : x[3], i % 4 * 16 + n, 64);
+    for (int i = 0; i < DC; ++i) {                 // (dc_place(i) is 4 (i % 4) + i / 4)
+      const int e = i / 4, from = i % 4 * 16;
+      const float xe = e == 0 ? x[0] : e == 1 ? x[1] : e == 2 ? x[2] : x[3], me = e == 0 ? m[0] : e == 1 ? m[1] : e == 2 ? m[2] : m[3];
+      const float xi = __shfl(xe, from + n, 64);
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (i <= r * 4 + g) sum[r] += M[(g * 4 + r) * DC + dc_place(i)] * xi;
+      for (int r = 0; r < 4; ++r) {
+        const float mi = __shfl(me, from + g * 4 + r, 64);
+        if (i <= r * 4 + g) sum[r] += mi * xi;
+      }
     }
     return sum;
   };
-  auto make_w = [&](int c, f32x4 m, f32x4 v) {
-    f32x4 x = v - ((ks_parts[c & 1][0][lane] + ks_parts[c & 1][1][lane]) + (ks_parts[c & 1][2][lane] + ks_parts[c & 1][3][lane]));
+  // W of chunk c from the four parts of K~ S0 in LDS
+  auto make_w = [&](auto careful, int c, f32x4 m, f32x4 v) {
+    const f32x4 k0 = ks_parts[c & 1][0][lane], k1 = ks_parts[c & 1][1][lane], k2 = ks_parts[c & 1][2][lane], k3 = ks_parts[c & 1][3][lane];
+    f32x4 x = v - ((k0 + k1) + (k2 + k3));
 #pragma unroll
     for (int r = 0; r < 4; ++r) x[r] = live ? x[r] : 0.f;
-    return triangle(base + c * stride + OFF_T, m, x, zero);
-  };
-  // (rows past the last: the last one's values, which T's zeros keep out)
-  auto fetch_v = [&](int c) {
-    f32x4 v;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = v_column[(long)min(c * DC + r * 4 + g, n_rows - 1) * ldu];
-    return v;
+    return triangle(careful, m, x, zero);
   };
   // (not __syncthreads, which also waits for what is under way from memory)
   auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
+  // turns(c, set) for every chunk, with the SETS - 1 after it on their way
+  auto walk = [&](auto& sets, auto&& fetch, auto&& turn) {
+    rewind();
+#pragma unroll
+    for (int e = 0; e < SETS - 1; ++e) fetch(sets[e]), advance();
+    int c0 = 0;
+    for (; c0 + SETS <= chunks; c0 += SETS) {
+#pragma unroll
+      for (int e = 0; e < SETS; ++e) {
+        fetch(sets[(e + SETS - 1) % SETS]), advance();
+        __builtin_amdgcn_sched_barrier(0);
+        turn(c0 + e, sets[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < SETS - 1; ++e)
+      if (c0 + e < chunks) turn(c0 + e, sets[e]);
+  };
 
-  if (wave == 4) {                               // the rows' results
+  const int d0 = wave * NT * 16;                 // the wave's first key channel
+  float* S_line = state + (long)seq_slots[s] * lds + ((long)h * gridDim.y + vb) * D * 16;
+  f32x4 S[NT];
+
+  auto results_wave = [&](auto careful) {        // the rows' results
     struct Operands { f32x4 t, q, v; } sets[SETS];
-    auto fetch = [&](Operands& o, int c) {
-      o.t = *reinterpret_cast<const f32x4*>(base + c * stride + OFF_T + n * DC + g * 4);
-      o.q = *reinterpret_cast<const f32x4*>(base + c * stride + OFF_Q + n * DC + g * 4);
-      o.v = fetch_v(c);
-    };
     f32x4 W = zero, q = zero;                    // of the chunk before
     auto results = [&](int c) {
-      const f32x4 o = triangle(base + c * stride + OFF_Q, q, W,
-                               (qs_parts[c & 1][0][lane] + qs_parts[c & 1][1][lane]) + (qs_parts[c & 1][2][lane] + qs_parts[c & 1][3][lane]));
+      const f32x4 a = qs_parts[c & 1][0][lane], b = qs_parts[c & 1][1][lane], d = qs_parts[c & 1][2][lane], e = qs_parts[c & 1][3][lane];
+      const f32x4 o = triangle(careful, q, W, (a + b) + (d + e));
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = c * DC + r * 4 + g;
         if (row < n_rows && live) out[(long)(first + row) * ldo + h * V + c_v] = o[r];
       }
     };
-#pragma unroll
-    for (int c = 0; c < SETS - 1; ++c)
-      if (c < chunks) fetch(sets[c], c);
-    for (int c0 = 0; c0 < chunks; c0 += SETS) {
-#pragma unroll
-      for (int e = 0; e < SETS; ++e) {
-        const int c = c0 + e;
-        if (c >= chunks) break;
-        if (c + SETS - 1 < chunks) fetch(sets[(e + SETS - 1) % SETS], c + SETS - 1);
-        meet();
-        const f32x4 now = make_w(c, sets[e].t, sets[e].v);
-        if (c) results(c - 1);
-        W = now;
-        q = sets[e].q;
-      }
-    }
+    walk(sets, [&](Operands& o) { o.t = four(p + OFF_T * 4, t_off), o.q = four(p + OFF_Q * 4, t_off), o.v = fetch_v(); },
+         [&](int c, const Operands& own) {
+           meet();
+           const f32x4 now = make_w(careful, c, own.t, own.v);
+           if (c) results(c - 1);
+           W = now;
+           q = own.q;
+         });
     meet();
     results(chunks - 1);
-    return;
-  }
-
-  const int d0 = wave * NT * 16;                 // the wave's first key channel
-  float* S_line = state + (long)seq_slots[s] * lds + ((long)h * gridDim.y + vb) * D * 16;
-  f32x4 S[NT];
-#pragma unroll
-  for (int k = 0; k < NT; ++k)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = d0 + k * 16 + g * 4 + r;
-      S[k][r] = d < D ? S_line[d * 16 + n] : 0.f;
-    }
-  struct Operands { f32x4 kt[NT], qt[NT], kh[NT], a[NT], t, v; } sets[SETS];
-  auto fetch = [&](Operands& o, int c) {
-    const float* p = base + c * stride;
-#pragma unroll
-    for (int k = 0; k < NT; ++k) {
-      o.kt[k] = *reinterpret_cast<const f32x4*>(p + n * Dp + d0 + k * 16 + g * 4);
-      o.qt[k] = *reinterpret_cast<const f32x4*>(p + DC * Dp + n * Dp + d0 + k * 16 + g * 4);
-      o.kh[k] = *reinterpret_cast<const f32x4*>(p + 2 * DC * Dp + (d0 + k * 16 + n) * DC + g * 4);
-      o.a[k] = *reinterpret_cast<const f32x4*>(p + OFF_A + d0 + k * 16 + g * 4);
-    }
-    o.t = *reinterpret_cast<const f32x4*>(p + OFF_T + n * DC + g * 4);
-    o.v = fetch_v(c);
   };
-  // the wave's part of a product with S, in four sums, so that none is a longer chain than the walk row by row has
-  auto against = [&](const f32x4 (&rows)[NT]) {
-    f32x4 part[4];
+  auto state_waves = [&](auto careful) {
 #pragma unroll
     for (int k = 0; k < NT; ++k)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) part[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(rows[k][r], S[k][r], k ? part[r] : zero, 0, 0, 0);
-    return (part[0] + part[1]) + (part[2] + part[3]);
+      for (int r = 0; r < 4; ++r) {
+        const int d = d0 + k * 16 + g * 4 + r;
+        S[k][r] = d < D ? S_line[d * 16 + n] : 0.f;
+      }
+    struct Operands { f32x4 kt[NT], qt[NT], kh[NT], a[NT], t, v; } sets[SETS];
+    const unsigned row_off = (n * Dp + d0 + g * 4) * 4, kh_off = ((d0 + n) * DC + g * 4) * 4, a_off = (d0 + g * 4) * 4;
+    // the wave's part of a product with S, in four sums, so that none is a longer chain than the walk row by row has
+    auto against = [&](const f32x4 (&rows)[NT]) {
+      f32x4 part[4];
+#pragma unroll
+      for (int k = 0; k < NT; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(rows[k][r], S[k][r], k ? part[r] : zero, 0, 0, 0);
+      return (part[0] + part[1]) + (part[2] + part[3]);
+    };
+    walk(sets,
+         [&](Operands& o) {
+#pragma unroll
+           for (int k = 0; k < NT; ++k) {
+             o.kt[k] = four(p + k * 64, row_off);
+             o.qt[k] = four(p + DC * Dp * 4 + k * 64, row_off);
+             o.kh[k] = four(p + 2 * DC * Dp * 4 + k * 16 * DC * 4, kh_off);
+             o.a[k] = four(p + OFF_A * 4 + k * 64, a_off);
+           }
+           o.t = four(p + OFF_T * 4, t_off);
+           o.v = fetch_v();
+         },
+         [&](int c, const Operands& now) {
+           ks_parts[c & 1][wave][lane] = against(now.kt);
+           meet();
+           const f32x4 k0 = ks_parts[c & 1][0][lane], k1 = ks_parts[c & 1][1][lane], k2 = ks_parts[c & 1][2][lane], k3 = ks_parts[c & 1][3][lane];
+           __builtin_amdgcn_sched_barrier(0);
+           const f32x4 qs = against(now.qt);
+           __builtin_amdgcn_sched_barrier(0);
+           f32x4 x = now.v - ((k0 + k1) + (k2 + k3));
+#pragma unroll
+           for (int r = 0; r < 4; ++r) x[r] = live ? x[r] : 0.f;
+           const f32x4 W = triangle(careful, now.t, x, zero);
+           qs_parts[c & 1][wave][lane] = qs;
+#pragma unroll
+           for (int k = 0; k < NT; ++k) S[k] *= now.a[k];
+#pragma unroll
+           for (int r = 0; r < 4; ++r)
+#pragma unroll
+             for (int k = 0; k < NT; ++k) S[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kh[k][r], W[r], S[k], 0, 0, 0);
+         });
+    meet();                                      // the fifth wave's last results
   };
-  auto chunk = [&](int c, const Operands& now) {
-    ks_parts[c & 1][wave][lane] = against(now.kt);
-    meet();
-    const f32x4 qs = against(now.qt);
-    const f32x4 W = make_w(c, now.t, now.v);
-    qs_parts[c & 1][wave][lane] = qs;
-#pragma unroll
-    for (int k = 0; k < NT; ++k) S[k] *= now.a[k];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int k = 0; k < NT; ++k) S[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kh[k][r], W[r], S[k], 0, 0, 0);
-  };
-#pragma unroll
-  for (int c = 0; c < SETS - 1; ++c)
-    if (c < chunks) fetch(sets[c], c);
-  for (int c0 = 0; c0 < chunks; c0 += SETS) {
-#pragma unroll
-    for (int e = 0; e < SETS; ++e) {
-      const int c = c0 + e;
-      if (c >= chunks) break;
-      if (c + SETS - 1 < chunks) fetch(sets[(e + SETS - 1) % SETS], c + SETS - 1);
-      chunk(c, sets[e]);
-    }
+
+  if (wave == 4) results_wave(std::false_type{});
+  else state_waves(std::false_type{});
+  poisoned[t >> 6] = __any(!(poison == 0.f)) ? 1 : 0;
+  meet();
+  if (poisoned[0] | poisoned[1] | poisoned[2] | poisoned[3] | poisoned[4]) {      // the same for all waves
+    if (wave == 4) results_wave(std::true_type{});
+    else state_waves(std::true_type{});
   }
-  meet();                                        // the fifth wave's last results
+  if (wave == 4) return;
   // (channels beyond vdim have seen values of zero only and are still zero)
 #pragma unroll
   for (int k = 0; k < NT; ++k)
@@ -586,7 +628,8 @@ TIS_EXPORT int tis_delta_scan(const float* u, long ldu, int q_off, int k_off, in
       ((uintptr_t)state % 16) || ((uintptr_t)work % 16))
     return tis_fail("delta_scan: bad size requests=%d heads=%d qk_heads=%d dim=%d (at most 256) vdim=%d, or state lines that are "
                     "not 16 bytes aligned", n_seqs, H, G, D, V);
-  const bool chunks = work && longest >= DR_CHUNK_FROM && (V + 15) / 16 <= 65535 && dc_most(rows) < (1L << 31);
+  // (ldu: a chunk's rows are read at 32-bit offsets from its first)
+  const bool chunks = work && longest >= DR_CHUNK_FROM && (V + 15) / 16 <= 65535 && dc_most(rows) < (1L << 31) && ldu < (1L << 26);
   const int from = chunks ? DR_CHUNK_FROM : 0x7fffffff;
   if (!(chunks && n_seqs == 1 && longest == rows)) {      // (a single request of that many rows leaves none for the walk row by row)
     const int R = D <= 16 ? 1 : D <= 32 ? 2 : D <= 64 ? 4 : D <= 128 ? 8 : 16;
