@@ -100,6 +100,24 @@ def test_grouped_product_of_many_steps(ops, tile, rows, N, K, gated):
             torch.testing.assert_close(out[mine].double(), want, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("tile,M,N,K", [(8, 1100, 2044, 2312), (8, 1281, 1536, 4096), (8, 2047, 1532, 4040), (9, 1433, 2052, 4104), (9, 1532, 2048, 5632)])
+def test_tiles_of_96(ops, tile, M, N, K):
+    """128 x 96 and 96 x 128, whole tiles and parts of one in both directions and in the steps: against exact sums, as every tile, and with the library's bits
+    where it has the width."""
+    assert ops.gemm_tiles.cdll.tis_gemm_tiles_pick(M, N, K) == tile
+    x, w, res = rnd((M, K), 1).cuda(), rnd((N, K), 2, K ** -0.5).cuda(), rnd((M, N), 3).cuda()
+    want = (x.double() @ w.double().t())
+    torch.testing.assert_close(ops._linear_tiles(x, w, None, torch.empty(M, N, device="cuda"), N, 1, 0).double(), want, rtol=1e-4, atol=1e-4)
+    out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops._linear_tiles(x, w, res, out[:M], N, 0, 0)
+    torch.testing.assert_close(out[:M].double(), want + res.double(), rtol=8e-3, atol=4e-3)
+    assert bool((out[M] == 7.0).all())                  # nothing behind the last row
+    gated = ops._linear_tiles(x, w, None, torch.empty(M, N // 2, dtype=torch.bfloat16, device="cuda"), N, 0, 4)
+    assert torch.equal(gated, ops.swiglu(ops._linear_tiles(x, w, None, torch.empty(M, N, dtype=torch.bfloat16, device="cuda"), N, 0, 0)))
+    if (N, K) in ops.library_widths:
+        assert torch.equal(out[:M], ops.linear(x, w, res, None, None, False, "library"))
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 64, 64), (3, 352, 64), (16, 30, 4), (17, 352, 176), (70, 98, 260), (16, 2000, 1024), (33, 20, 1020)])
 def test_norm_and_gate_inside_the_32_bit_product(M, N, K):
     """The same bits as the norm's, the product's and the gate's own kernels one after the other, on strided rows too; beyond the widths that

@@ -44,6 +44,15 @@ def test_the_faster_of_tiles_and_library(sizes, kernel):
         assert [fn for fn, _ in ops.calls if fn != "tis_swiglu"] == [kernel], (rows, N, K)
 
 
+# (rows, columns, inner columns, gate) beyond 1,024 rows: tiles of 128 x 64, 128 x 96 and 128 x 128 that fill the chip, and what lies beside them
+@pytest.mark.parametrize("sizes,kernel", [
+    ([(1153, 1536, 4096, 0), (1318, 1536, 4096, 0), (2048, 1536, 4096, 0), (1280, 2048, 5632, 0), (1537, 2048, 5632, 0), (2048, 2048, 5632, 0)], "tis_gemm_tiles"),
+    ([(1152, 1536, 4096, 0), (1537, 1536, 4096, 0), (1408, 2048, 5632, 0), (1536, 2048, 5632, 0), (2049, 1536, 4096, 0), (1281, 11264, 2048, 1), (2048, 8192, 1536, 1)],
+     "tis_gemm_library")])
+def test_beyond_a_thousand_rows(sizes, kernel):
+    test_the_faster_of_tiles_and_library(sizes, kernel)
+
+
 def test_what_a_layers_products_refuse():
     """Operands that do not fit together, whichever kernel the sizes go to."""
     ops, x = host_ops(), zeros(300, 1536)

@@ -113,8 +113,14 @@ TIS_EXPORT void tis_gemm_tiles_units(int n) { if (n > 0) g_units = n; }
 // (K in two parts by two sets of waves, for products of less than a tile a unit: 1 to 2.5 us less, but other sums than every other tile's,
 // and than the library's, with which all of these agree to the bit.)
 // Beyond one tile a unit a tile's LDS says how many share one: two of 128 x 192, 64 x 64 and 64 x 32, else one.
+// Tiles of less than 256 x 256 that are alone on their unit are bound by the unit's way from the L2 into LDS, some 60 bytes a nanosecond whatever their size
+// and waves; so for a product of two to three million results, one tile a unit, the smaller the rows of a step the better: 128 x 96 (96 x 128 where only that many
+// fit) in place of 128 x 128, four waves of three 32 x 32 results each. us, 128 x 128 / these, and the library's product: 1,900 rows of 1,536 x 4,096 36.7 / 33.7
+// (35.6), 1,605 34.5 / 31.2 (31.9), 2,048 37.0 / 34.5 (35.8); of 2,048 x 5,632 1,195 44.8 / 40.6 (47.6), 1,482 48.6 / 44.7 (44.0); 1,060 rows of 2,304 x 1,536 17.6 / 16.5
+// (19.9), of 2,048 x 2,048 19.8 / 19.0 (22.9).
 struct TileShape { int bm, bn; };
-static const TileShape g_shapes[8] = {{256, 256}, {256, 128}, {192, 128}, {128, 192}, {128, 128}, {128, 64}, {64, 64}, {64, 32}};
+static constexpr int GT_SHAPES = 10;
+static const TileShape g_shapes[GT_SHAPES] = {{256, 256}, {256, 128}, {192, 128}, {128, 192}, {128, 128}, {128, 64}, {64, 64}, {64, 32}, {128, 96}, {96, 128}};
 static long tiles_of(int i, int M, int N) {
   return (long)((M + g_shapes[i].bm - 1) / g_shapes[i].bm) * ((N + g_shapes[i].bn - 1) / g_shapes[i].bn);
 }
@@ -134,7 +140,10 @@ static float tile_estimate(int i, int M, int N, int K) {
     case 5: return 4.0f + steps * (r <= 0.75f ? 0.32f : r <= 1.f ? 0.37f : 0.03f + 0.36f * ceilf(r));
     case 6: return 3.4f + steps * (r <= 1.f ? 0.25f : r <= 1.25f ? 0.36f : 0.22f * ceilf(r));
     // (up to eight steps the wider tile: 448 x 512, 129 to 600 rows, 4.7 / 4.4)
-    default: return 4.1f + steps * (r <= 1.f ? 0.17f : 0.29f * ceilf(0.5f * r));
+    case 7: return 4.1f + steps * (r <= 1.f ? 0.17f : 0.29f * ceilf(0.5f * r));
+    // (beyond one a unit: none)
+    case 8: return 7.5f + steps * (r <= 0.9f ? 0.36f : r <= 1.f ? 0.42f : 1e3f);
+    default: return 7.8f + steps * (r <= 1.f ? 0.44f : 1e3f);
   }
 }
 
@@ -142,7 +151,7 @@ static float tile_estimate(int i, int M, int N, int K) {
 TIS_EXPORT int tis_gemm_tiles_pick(int M, int N, int K) {
   int pick = 0;
   float best = tile_estimate(0, M, N, K);
-  for (int i = 1; i < 8; ++i) {
+  for (int i = 1; i < GT_SHAPES; ++i) {
     const float t = tile_estimate(i, M, N, K);
     if (t < best) best = t, pick = i;
   }
@@ -199,7 +208,9 @@ TIS_EXPORT int tis_gemm_tiles(const void* X, long x_ld, const void* W, const voi
     case 4: PICK(128, 128, 2, 4, 5, 2) break;
     case 5: PICK(128, 64, 4, 2, 6, 2) break;
     case 6: PICK(64, 64, 2, 2, 5, 2) break;
-    default: PICK(64, 32, 2, 1, 6, 2) break;
+    case 7: PICK(64, 32, 2, 1, 6, 2) break;
+    case 8: PICK(128, 96, 4, 1, 5, 2) break;
+    default: PICK(96, 128, 1, 4, 5, 2) break;
   }
 #undef PICK
 #undef LAUNCH

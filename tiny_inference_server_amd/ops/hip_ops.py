@@ -240,7 +240,7 @@ def _tiles_up_to(N: int, K: int) -> int:
     return rows if N <= columns and K <= inner else _TILES_UP_TO
 
 
-_TILE_256x128, _TILE_128x64 = 1, 5      # of the tiled product's tiles
+_TILE_256x128, _TILE_128x128, _TILE_128x64, _TILES_OF_96 = 1, 4, 5, (8, 9)      # of the tiled product's tiles
 
 # From so many multiply-adds on the library is asked at all up to 1,024 rows: below, a step whose kernels the host launches one by one waits for the host,
 # of whose time a product by the library takes 10 us more than one on the tiles. 0.9B prompts of 130 to 520 rows, us a step, library / library where it is the
@@ -261,12 +261,21 @@ def tiles_pay(M: int, N: int, K: int, gate: bool, tile: int, share: float) -> bo
     1,400, 1,532 17.8 / 19.1; 11,264 x 2,048 with the gate at 768 48 / 51. A block's four products are together nowhere slower than by the library alone, at either
     size, 129 to 2,048 rows, beyond what two chips differ by (2 %); with the row limits alone 2.1B's at 768 rows were by 7 %. Single products that stay on the
     tiles for the host's sake and are slower there: 1,536 x 4,096 at 768 24 / 27, 2,048 x 2,048 at 640 14.6 / 16.1, 2,048 x 5,632 at 384 26 / 29."""
-    if M > _tiles_up_to(N, K) or N % 4:
+    if N % 4:
         return False
+    if M > _tiles_up_to(N, K):
+        # a matrix of many inner columns, where tiles are one a unit and fill the chip (see gemm_tiles.hip). us, library / tiles: 1,536 x 4,096 at 1,190, 1,340, 1,480, 1,926
+        # 29 / 25, 34 / 30, 34 / 31, 35 / 32; 1,536 x 3,072 at 1,411 28 / 23; 2,048 x 5,632 at 1,031, 1,190, 1,580, 1,850 46 / 39, 46 / 40, 53 / 47, 54 / 50. Where the library's
+        # own tiles fill the chip it stays: 1,536 x 4,096 at 1,113, 1,650, 1,792 28 / 32, 32 / 34, 31 / 34, 2,048 x 5,632 at 1,408, 1,532 44 / 48.
+        if gate or M > 2048 or N > _TILES_NARROW[1] or share > 1:
+            return False
+        if tile in _TILES_OF_96:
+            return share >= 0.66 and (share < 0.8 or M <= 1280 or M > 1792)
+        return (tile == _TILE_128x64 and share >= 0.9) or (tile == _TILE_128x128 and share >= 0.66)
     step = 64 if M <= 256 else 256
     beyond = 1 - (library_rows(M) - M) / step        # of the library's last step of rows
     if M > 1024:
-        return gate or beyond <= 0.3 or share >= (0.8 if tile == _TILE_256x128 else 0.62)
+        return gate or beyond <= 0.3 or share >= (0.8 if tile == _TILE_256x128 else 0.83 if tile in _TILES_OF_96 else 0.62)
     if M * N * K < _LIBRARY_FROM:
         return True
     if gate:
