@@ -187,3 +187,32 @@ def test_few_entries_in_many_groups(ops, groups, rows, top, N, K):
             assert bool((out[e] == 7.0).all())
         else:
             torch.testing.assert_close(out[e].double(), w[group_of[e]].double() @ x[e // top].double(), rtol=1e-4, atol=1e-4)
+
+
+# rows, heads, key/value heads, head size, inner columns, page size, the tile that the product takes
+@pytest.mark.parametrize("M,H,G,HD,K,ps,tile", [
+    (2048, 12, 3, 128, 1536, 16, 2), (1101, 12, 3, 128, 1536, 16, 8), (500, 12, 3, 128, 1032, 16, 5), (300, 12, 2, 64, 520, 16, 7), (700, 30, 1, 128, 1032, 32, 4),
+    (2044, 56, 4, 128, 1544, 16, 0), (1020, 44, 2, 128, 1032, 16, 1), (2049, 49, 1, 96, 264, 48, 3), (333, 6, 1, 256, 520, 16, 6), (1433, 12, 2, 128, 4104, 16, 9)])
+def test_queries_keys_and_values_from_the_product(ops, monkeypatch, M, H, G, HD, K, ps, tile):
+    """Turned and cached by the product against the product, then the rotary kernel: the same bits in the queries and in every slot of the cache that a row writes,
+    and nothing in the others; with every tile, heads that begin inside tiles, and keys and values that are not kept."""
+    assert ops.gemm_tiles.cdll.tis_gemm_tiles_pick(M, (H + 2 * G) * HD, K) == tile
+    gen = torch.Generator().manual_seed(M)
+    x, w = rnd((M, K), 1).cuda(), rnd(((H + 2 * G) * HD, K), 2, K ** -0.5).cuda()
+    gain = (1 + 0.1 * torch.randn(K, generator=gen)).cuda()
+    pages = M // ps + 3
+    pos = torch.randint(0, 4000, (M,), generator=gen).to(torch.int32).cuda()
+    slots = torch.arange(5, 5 + M, dtype=torch.int32)             # consecutive, as a portion's are, but for some that change places
+    swap = torch.randperm(M, generator=gen)[:40]
+    slots[swap] = slots[swap.flip(0)]
+    slots = slots.cuda()
+    angle = torch.arange(4000)[:, None] * torch.rand(HD // 2, generator=gen)
+    table = torch.stack((angle.cos(), angle.sin()), -1).contiguous().cuda()
+    monkeypatch.setattr(ops, "_layer_route", lambda *a, **k: "tiles")
+    for write in (True, False):
+        planes = [torch.full((pages, 2, G, ps, HD), 5.0, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+        q = ops.qkv_rope(x, w, (gain, 1e-5), pos, slots, table, planes[0], H, G, HD, ps, write_cache=write)
+        qkv = ops.linear(x, w, None, None, (gain, 1e-5), False, "tiles")
+        want = ops.empty(M, H * HD)
+        ops.rope_write_kv(qkv, pos, slots, table, planes[1], H, G, HD, ps, False, write, paired=True, q_out=want)
+        assert torch.equal(q, want) and torch.equal(*planes) and bool((planes[0] != 5.0).any()) == write

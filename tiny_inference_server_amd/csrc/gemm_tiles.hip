@@ -27,17 +27,12 @@ template <int ACT> __device__ __forceinline__ float gt_gated(float g, float u, f
   return g / (1.f + expf(-g)) * u;
 }
 
-template <int BM, int BN, int WM, int WN, int NSTAGE, int AHEAD, bool RESIDUAL, typename TO, int ACT = 0>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
-    const bf16* __restrict__ X, long x_ld, const bf16* __restrict__ W, const bf16* R, long r_ld, TO* C, long c_ld,
-    int M, int N, int K, float limit) {
-  typedef TileLoop<BM, BN, WM, WN, NSTAGE, AHEAD> Loop;
-  constexpr int LPW = Loop::LPW, TM = Loop::TM, TN = Loop::TN;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[NSTAGE * Loop::STAGE];
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r32 = lane & 31, h = lane >> 5;
-  const int wm = wave / WN, wn = wave % WN;
-  const GtTile tile = gt_tile(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN);
-  const long m0 = (long)tile.m * BM, n0 = (long)tile.n * BN;
+// acc = the tile's sums over K
+template <typename Loop, int BM>
+__device__ __forceinline__ void tile_sums(unsigned char* lds, const bf16* X, long x_ld, const bf16* W, long m0, long n0, int M, int N, int K,
+                                          f32x16 (&acc)[Loop::TM][Loop::TN]) {
+  constexpr int LPW = Loop::LPW;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   // Rows past the matrix's last are the last row again (their results are not stored).
   const unsigned char* first[LPW];
   unsigned lane_off[LPW];
@@ -52,14 +47,28 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
     first[j] = (const unsigned char*)(of_x ? X : W) + g_first * ld * 2;
     lane_off[j] = (unsigned)((g_row - g_first) * ld * 2 + Loop::piece_of(lane, row) * 16);
   }
-  f32x16 acc[TM][TN];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < Loop::TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int j = 0; j < Loop::TN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   Loop::run(lds, first, lane_off, K, acc);
+}
+
+template <int BM, int BN, int WM, int WN, int NSTAGE, int AHEAD, bool RESIDUAL, typename TO, int ACT = 0>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
+    const bf16* __restrict__ X, long x_ld, const bf16* __restrict__ W, const bf16* R, long r_ld, TO* C, long c_ld,
+    int M, int N, int K, float limit) {
+  typedef TileLoop<BM, BN, WM, WN, NSTAGE, AHEAD> Loop;
+  constexpr int TM = Loop::TM, TN = Loop::TN;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[NSTAGE * Loop::STAGE];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r32 = lane & 31, h = lane >> 5;
+  const int wm = wave / WN, wn = wave % WN;
+  const GtTile tile = gt_tile(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN);
+  const long m0 = (long)tile.m * BM, n0 = (long)tile.n * BN;
+  f32x16 acc[TM][TN];
+  tile_sums<Loop, BM>(lds, X, x_ld, W, m0, n0, M, N, K, acc);
 
   // accumulator 4 q + e of block (i, j): row m0 + wm * (BM / WM) + i * 32 + r32, column n0 + wn * (BN / WN) + j * 32 + 8 q + 4 h + e
 #pragma unroll
@@ -98,6 +107,110 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
   }
 }
 
+// The product that makes a prompt's queries, keys and values: W's rows are the heads' channels, the queries' and keys' in pairs (2j, 2j + 1 of a
+// head: channels j and j + head_dim / 2). A lane holds two whole pairs of a row, so they are turned by the row's position where they lie, in 32 bits
+// from the product rounded to bfloat16, as the kernel that reads a stored product takes it (the same bits). Queries go to q_out, keys to the row's slot
+// of the cache's pages, values there transposed. What it saves is that kernel: its launch and the product's way to memory and back (2,048 rows of 18 heads of
+// 128 against 1,536, us: 29.2 / 24.7; 1,532 rows of 24 against 2,048 33.8 / 30.0). The rows' cosines and sines are asked for before the first step, where they find room.
+struct RopeOut {
+  const int* positions;
+  const int* write_slots;     // null: keys and values have no reader
+  const float2* table;        // [positions][head_dim / 2] (cos, sin)
+  bf16* plane;                // [page][keys, values][kv head][page_size * head_dim]
+  int n_heads, n_kv_heads, head_dim, page_size;
+};
+template <int BM, int BN, int WM, int WN, int NSTAGE, int AHEAD>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_rope_kernel(const bf16* __restrict__ X, long x_ld, const bf16* __restrict__ W,
+                                                                       bf16* __restrict__ q_out, long q_ld, int M, int N, int K, RopeOut a) {
+  typedef TileLoop<BM, BN, WM, WN, NSTAGE, AHEAD> Loop;
+  constexpr int TM = Loop::TM, TN = Loop::TN;
+  constexpr bool EARLY = TM * TN <= 4;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[NSTAGE * Loop::STAGE];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r32 = lane & 31, h = lane >> 5;
+  const int wm = wave / WN, wn = wave % WN;
+  const GtTile tile = gt_tile(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN);
+  const long m0 = (long)tile.m * BM, n0 = (long)tile.n * BN;
+  const int HD = a.head_dim, half = HD / 2;
+  int head[TN], d0[TN];                          // of a block of 32 columns (head sizes are multiples of 32): its head, its first channel
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = (int)n0 + wn * (BN / WN) + j * 32;
+    head[j] = __builtin_amdgcn_readfirstlane(n / HD);
+    d0[j] = n - head[j] * HD;
+  }
+  int pos[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) pos[i] = a.positions[min(m0 + wm * (BM / WM) + i * 32 + r32, (long)M - 1)];
+  // (cos, sin) of the lane's two pairs of every eight columns
+  auto factors = [&](int i, int j, float4 (&cs)[4]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) cs[q] = *reinterpret_cast<const float4*>(a.table + (long)pos[i] * half + d0[j] / 2 + q * 4 + h * 2);
+  };
+  float4 held[EARLY ? TM : 1][EARLY ? TN : 1][4];
+  if constexpr (EARLY)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) factors(i, j, held[i][j]);
+  f32x16 acc[TM][TN];
+  tile_sums<Loop, BM>(lds, X, x_ld, W, m0, n0, M, N, K, acc);
+
+  const long page_elems = (long)a.page_size * HD;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const long m = m0 + wm * (BM / WM) + i * 32 + r32;
+    const bool row = m < M;
+    int page = 0, slot = 0;
+    if (a.write_slots) {
+      const int at = a.write_slots[min(m, (long)M - 1)];
+      page = at / a.page_size;
+      slot = at - page * a.page_size;
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if (n0 + wn * (BN / WN) + j * 32 >= N) continue;       // (the same for the wave, as the head is)
+      const int kv = head[j] - a.n_heads, value = kv - a.n_kv_heads;
+      if (kv >= 0 && !a.write_slots) continue;
+      if (value >= 0) {
+        bf16* dst = a.plane + (((long)page * 2 + 1) * a.n_kv_heads + value) * page_elems + slot;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (row) dst[(long)(d0[j] + q * 8 + h * 4 + e) * a.page_size] = static_cast<__bf16>(acc[i][j][q * 4 + e]);
+        continue;
+      }
+      float4 late[4];
+      if constexpr (!EARLY) factors(i, j, late);
+      uint32_t lo[4], hi[4];                     // of the head's halves: the lane's two channels of every four
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+        const float4 cs = EARLY ? held[EARLY ? i : 0][EARLY ? j : 0][q] : late[q];
+        const float c[2] = {cs.x, cs.z}, sn[2] = {cs.y, cs.w};
+        bf16x2 y1, y2;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float x1 = static_cast<float>(static_cast<__bf16>(acc[i][j][q * 4 + 2 * e])), x2 = static_cast<float>(static_cast<__bf16>(acc[i][j][q * 4 + 2 * e + 1]));
+          // (which of the two products is rounded before the sum is spelled out, as the rotary kernel has it: the compiler's choice differs)
+          y1[e] = static_cast<__bf16>(fmaf(x1, c[e], -(x2 * sn[e])));
+          y2[e] = static_cast<__bf16>(fmaf(x1, sn[e], x2 * c[e]));
+        }
+        lo[q] = __builtin_bit_cast(uint32_t, y1);
+        hi[q] = __builtin_bit_cast(uint32_t, y2);
+      }
+      bf16* dst = kv < 0 ? q_out + m * q_ld + (long)head[j] * HD : a.plane + ((long)page * 2 * a.n_kv_heads + kv) * page_elems + (long)slot * HD;
+#pragma unroll
+      for (int q = 0; q < 4; q += 2) {           // the lane beside it (32 on) has the other two of four: each takes four of one piece, 8 bytes
+        const auto l = __builtin_amdgcn_permlane32_swap(lo[q], lo[q + 1], false, false), u = __builtin_amdgcn_permlane32_swap(hi[q], hi[q + 1], false, false);
+        bf16* at = dst + d0[j] / 2 + (q + h) * 4;
+        if (row) *reinterpret_cast<uint2*>(at) = make_uint2(l[0], l[1]);
+        if (row) *reinterpret_cast<uint2*>(at + half) = make_uint2(u[0], u[1]);
+      }
+    }
+  }
+}
+
 static int g_units = 256;      // compute units of the device: set by whoever knows (the default is an MI355X)
 TIS_EXPORT void tis_gemm_tiles_units(int n) { if (n > 0) g_units = n; }
 
@@ -121,6 +234,20 @@ TIS_EXPORT void tis_gemm_tiles_units(int n) { if (n > 0) g_units = n; }
 struct TileShape { int bm, bn; };
 static constexpr int GT_SHAPES = 10;
 static const TileShape g_shapes[GT_SHAPES] = {{256, 256}, {256, 128}, {192, 128}, {128, 192}, {128, 128}, {128, 64}, {64, 64}, {64, 32}, {128, 96}, {96, 128}};
+// DO(BM, BN, WM, WN, NSTAGE, AHEAD) for tile `pick`
+#define GT_EACH_TILE(pick, DO)                   \
+  switch (pick) {                                \
+    case 0: DO(256, 256, 2, 4, 2, 1) break;      \
+    case 1: DO(256, 128, 4, 2, 3, 1) break;      \
+    case 2: DO(192, 128, 2, 4, 4, 2) break;      \
+    case 3: DO(128, 192, 2, 2, 2, 1) break;      \
+    case 4: DO(128, 128, 2, 4, 5, 2) break;      \
+    case 5: DO(128, 64, 4, 2, 6, 2) break;       \
+    case 6: DO(64, 64, 2, 2, 5, 2) break;        \
+    case 7: DO(64, 32, 2, 1, 6, 2) break;        \
+    case 8: DO(128, 96, 4, 1, 5, 2) break;       \
+    default: DO(96, 128, 1, 4, 5, 2) break;      \
+  }
 static long tiles_of(int i, int M, int N) {
   return (long)((M + g_shapes[i].bm - 1) / g_shapes[i].bm) * ((N + g_shapes[i].bn - 1) / g_shapes[i].bn);
 }
@@ -200,19 +327,34 @@ TIS_EXPORT int tis_gemm_tiles(const void* X, long x_ld, const void* W, const voi
     else if (act == 4) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 4);  \
     else LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, bf16, 0);                \
   }
-  switch (pick) {
-    case 0: PICK(256, 256, 2, 4, 2, 1) break;
-    case 1: PICK(256, 128, 4, 2, 3, 1) break;
-    case 2: PICK(192, 128, 2, 4, 4, 2) break;
-    case 3: PICK(128, 192, 2, 2, 2, 1) break;
-    case 4: PICK(128, 128, 2, 4, 5, 2) break;
-    case 5: PICK(128, 64, 4, 2, 6, 2) break;
-    case 6: PICK(64, 64, 2, 2, 5, 2) break;
-    case 7: PICK(64, 32, 2, 1, 6, 2) break;
-    case 8: PICK(128, 96, 4, 1, 5, 2) break;
-    default: PICK(96, 128, 1, 4, 5, 2) break;
-  }
+  GT_EACH_TILE(pick, PICK)
 #undef PICK
 #undef LAUNCH
   return tis_launch_status("gemm_tiles");
+}
+
+// q_out = the queries of X . W^T, turned; keys and values into the cache (see gemm_tiles_rope_kernel). W: [(n_heads + 2 n_kv_heads) head_dim, K], the rows
+// of query and key heads in pairs. write_slots and plane null: keys and values are not kept. Sizes: K, x_ld multiples of 8, head_dim of 32, q_ld of 4; X, W
+// and the table 16-byte aligned, q_out and the plane 8-byte. Launches only: safe under stream capture.
+TIS_EXPORT int tis_gemm_tiles_qkv_rope(const void* X, long x_ld, const void* W, void* q_out, long q_ld, int M, int K, const int* positions,
+                                       const int* write_slots, const float* table, void* plane, int n_heads, int n_kv_heads, int head_dim,
+                                       int page_size, hipStream_t stream) {
+  if (M < 0 || K < 1 || n_heads < 1 || n_kv_heads < 1 || head_dim < 32 || head_dim % 32 || page_size < 1 || (long)(n_heads + 2L * n_kv_heads) * head_dim >= (1L << 31))
+    return tis_fail("gemm_tiles_qkv_rope: bad size M=%d K=%d heads=%d kv_heads=%d head_dim=%d page=%d", M, K, n_heads, n_kv_heads, head_dim, page_size);
+  if (M == 0) return 0;
+  const int N = (n_heads + 2 * n_kv_heads) * head_dim;
+  if (K % 8 || x_ld % 8 || x_ld < K || q_ld % 4 || q_ld < (long)n_heads * head_dim)
+    return tis_fail("gemm_tiles_qkv_rope: K=%d and the row strides %ld, %ld must be multiples of 8, 8 and 4", K, x_ld, q_ld);
+  if (((uintptr_t)X | (uintptr_t)W | (uintptr_t)table) % 16 || ((uintptr_t)q_out | (uintptr_t)plane) % 8 || !positions || !table || !write_slots != !plane)
+    return tis_fail("gemm_tiles_qkv_rope: inputs and table must be 16-byte aligned, queries and cache 8-byte, and slots go with a cache");
+  if ((long)x_ld * 16 >= (1L << 31) || (long)K * 16 >= (1L << 31)) return tis_fail("gemm_tiles: rows of %ld elements are too long for 32-bit offsets", x_ld);
+  const int pick = tis_gemm_tiles_pick(M, N, K);
+  const long tiles = tiles_of(pick, M, N);
+  if (tiles >= (1L << 31)) return tis_fail("gemm_tiles: %ld tiles are more than a grid holds", tiles);
+  const RopeOut a{positions, write_slots, (const float2*)table, (bf16*)plane, n_heads, n_kv_heads, head_dim, page_size};
+#define ROPE(BMV, BNV, WMV, WNV, NSV, AHV)                                                                                   \
+  gemm_tiles_rope_kernel<BMV, BNV, WMV, WNV, NSV, AHV><<<dim3((unsigned)tiles), WMV * WNV * 64, 0, stream>>>((const bf16*)X, x_ld, (const bf16*)W, (bf16*)q_out, q_ld, M, N, K, a);
+  GT_EACH_TILE(pick, ROPE)
+#undef ROPE
+  return tis_launch_status("gemm_tiles_qkv_rope");
 }

@@ -113,8 +113,9 @@ __global__ __launch_bounds__(RC_THREADS) void rope_write_kv_rows_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float x1 = static_cast<float>(x[2 * e]), x2 = static_cast<float>(x[2 * e + 1]);
-        y1[e] = static_cast<__bf16>(x1 * c[e] - x2 * sn[e]);
-        y2[e] = static_cast<__bf16>(x2 * c[e] + x1 * sn[e]);
+        // (which product is rounded before the sum is spelled out: the product that turns its own results does the same)
+        y1[e] = static_cast<__bf16>(fmaf(x1, c[e], -(x2 * sn[e])));
+        y2[e] = static_cast<__bf16>(fmaf(x1, sn[e], x2 * c[e]));
       }
       bf16* dst;
       if (hh < n_heads) {

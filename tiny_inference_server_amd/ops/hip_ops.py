@@ -93,6 +93,7 @@ _SIGNATURES["gemm_skinny"] = ("tis_gemm_skinny", {
 })
 _SIGNATURES["gemm_tiles"] = ("tis_gemm_tiles", {
     "tis_gemm_tiles": [_P, _L, _P, _P, _L, _P, _L, _I, _I, _I, _I, _I, _F, _P],
+    "tis_gemm_tiles_qkv_rope": [_P, _L, _P, _P, _L, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _P],
 })
 _SIGNATURES["gemm_library"] = ("tis_gemm_library", {
     "tis_gemm_library_init": [],
@@ -1191,14 +1192,7 @@ class HipOps:
         if qkv.shape[1] != (n_heads + 2 * n_kv_heads) * head_dim:
             raise KernelError(f"rope_write_kv: row width {qkv.shape[1]} is not (heads {n_heads} + 2 x kv heads "
                               f"{n_kv_heads}) x head size {head_dim}")
-        self._index(positions, "positions", n)
-        if table is not None:
-            self._check(table, "rotary table", torch.float32)
-            if table.dim() != 3 or table.shape[1] != head_dim // 2 or table.shape[2] != 2 or not table.is_contiguous():
-                raise KernelError(f"rope_write_kv: table {tuple(table.shape)} for head size {head_dim}")
-        if write_cache:
-            self._index(write_slots, "write_slots", n)
-            self._check_plane(plane, n_kv_heads, head_dim, page_size)
+        self._check_rotary(n, positions, write_slots, table, plane, n_kv_heads, head_dim, page_size, write_cache)
         self.rope.tis_rope_write_kv(self.code, _ptr(qkv), qkv.stride(0), _ptr(positions),
                                     _ptr(write_slots if write_cache else None), _ptr(table),
                                     _ptr(plane if write_cache else None), n, n_heads, n_kv_heads, head_dim, page_size,
@@ -1236,11 +1230,32 @@ class HipOps:
                 _ptr(plane if write_cache else None), n_heads, n_kv_heads, head_dim, page_size,
                 int(bool(interleaved)), int(bool(write_cache)), self._stream())
             return q
-        qkv = self.linear_by_rows(x, w, rms=rms)
+        route = self._layer_route(x, M, N, K) if self.dtype == torch.bfloat16 and M > self.few_rows else None
+        if route == "tiles" and table is not None and not interleaved and head_dim % 32 == 0 and table.data_ptr() % 16 == 0 \
+                and (not write_cache or plane.data_ptr() % 8 == 0):
+            self._check_rotary(M, positions, write_slots, table, plane, n_kv_heads, head_dim, page_size, write_cache)
+            if rms is not None:
+                x = self.rmsnorm(x, rms[0], rms[1])
+            q = self.empty(M, n_heads * head_dim)
+            self.gemm_tiles.tis_gemm_tiles_qkv_rope(
+                _ptr(x), x.stride(0), _ptr(w), _ptr(q), q.stride(0), M, K, _ptr(positions), _ptr(write_slots if write_cache else None), _ptr(table),
+                _ptr(plane if write_cache else None), n_heads, n_kv_heads, head_dim, page_size, self._stream())
+            return q
+        qkv = self.linear(x, w, None, None, rms, False, route) if route else self.linear_by_rows(x, w, rms=rms)
         q = self.empty(M, n_heads * head_dim)
         self.rope_write_kv(qkv, positions, write_slots, table, plane, n_heads, n_kv_heads, head_dim, page_size,
                            interleaved, write_cache, paired=True, q_out=q)
         return q
+
+    def _check_rotary(self, n, positions, write_slots, table, plane, n_kv_heads, head_dim, page_size, write_cache):
+        self._index(positions, "positions", n)
+        if table is not None:
+            self._check(table, "rotary table", torch.float32)
+            if table.dim() != 3 or table.shape[1] != head_dim // 2 or table.shape[2] != 2 or not table.is_contiguous():
+                raise KernelError(f"rope_write_kv: table {tuple(table.shape)} for head size {head_dim}")
+        if write_cache:
+            self._index(write_slots, "write_slots", n)
+            self._check_plane(plane, n_kv_heads, head_dim, page_size)
 
     def _check_plane(self, plane, n_kv_heads, head_dim, page_size):
         self._check(plane, "cache plane")
