@@ -563,6 +563,41 @@ def test_the_delta_rules_walk_in_chunks(Hh, G, D, V, seqs):
     assert not torch.isfinite(broken[at]).any()
 
 
+@pytest.mark.parametrize("K", [1, 2, 4, 7])
+@pytest.mark.parametrize("seq_rows,slots", [([(0, 40, 1)], [2]), ([(i, 3 * i, 1) for i in range(70)], list(range(70))[::-1]), ([(0, 5, 1), (1, 0, 9), (10, 7, 2)], [1, 0, 2])])
+def test_single_rows_move_their_lines_on_with_the_step_before_the_walk(seq_rows, slots, K):
+    """The bits of the two kernels, in what is prepared and in every line; requests of more rows go to both as before."""
+    ops, g = hip_ops("float32"), torch.Generator().manual_seed(K + len(slots))
+    Hh, G, D, V, off = 4, 2, 70, 24, 3
+    C, n = 2 * G * D + Hh * V, sum(r[2] for r in seq_rows)
+    taps, proj = torch.randn(C, K, generator=g).cuda(), torch.randn(n, off + C + Hh, generator=g).cuda()
+    b, at = fake_batch(seq_rows, slots, None, 8, "cuda"), Hh * 2 * D * 16
+    lines = [torch.randn(max(slots) + 1, at + (K - 1) * C + 4, generator=g).cuda()]
+    lines.append(lines[0].clone())
+    one = ops.delta_prepare_and_keep(proj, off, off + C, taps, lines[0], at, b, Hh, G, D, V)
+    two = ops.delta_prepare(proj, off, off + C, taps, lines[1], at, b, Hh, G, D, V)
+    ops.conv_state_update(proj, off, C, K, lines[1], at, b)
+    assert torch.equal(one, two) and torch.equal(*lines)
+
+
+@pytest.mark.parametrize("n,ranks,widths", [(1, (64, 64), (1024, 2048)), (5, (16, 9), (512, 100)), (257, (64, 64), (1000, 2048)), (300, (64, 40), (1024, 2048)),
+                                            (33, (130, 16), (96, 33)), (300, (33, 64), (1024, 1024))])
+def test_two_low_rank_products_in_one_launch(n, ranks, widths):
+    """Each the bits of its own launch: of one form, and of two (another chunk of the rank, another number of rows a thread, lines read 16 bytes at a time or not)."""
+    ops, g = hip_ops("float32"), torch.Generator().manual_seed(n)
+    low = torch.randn(n, sum(ranks) + 4, generator=g).cuda()
+    w = [torch.randn(c, r, generator=g).cuda() for c, r in zip(widths, ranks)]
+    bias, rate = torch.randn(widths[0], generator=g).cuda(), torch.rand(widths[0], generator=g).cuda()
+    first = dict(low=low[:, :ranks[0]], w2=w[0], bias=bias, kind="exp_softplus", rate=rate, group=1)
+    second = dict(low=low[:, ranks[0]:ranks[0] + ranks[1]], w2=w[1], bias=None, kind="none")
+    for a, b in ((first, second), (second, first)):
+        got = ops.lowrank_act_pair(a, b)
+        assert torch.equal(got[0], ops.lowrank_act(**a)) and torch.equal(got[1], ops.lowrank_act(**b))
+    from tiny_inference_server_amd.ops.hip_ops import KernelError
+    with pytest.raises(KernelError):
+        ops.lowrank_act_pair(first, dict(second, low=second["low"][:n - 1]))
+
+
 @pytest.mark.parametrize("D", [64, 130])
 def test_a_walk_in_chunks_gives_a_prefix_its_own_bits(D):
     """Whatever number of chunks follows, and however many of them the last turn of the loop takes: the rows before get the same bits, whole chunks and

@@ -27,9 +27,12 @@ __device__ __forceinline__ float dr_sigmoid(float z) { return 1.f / (1.f + expf(
 // of this step; inputs before the step's first row come from the state line, which is zero before a request's first row.
 // KT: the number of taps where it is known at compile time (0: K): then all loads of a channel are under way at once, where a loop of unknown length
 // waits for each input before it asks for the next. Same sums in the same order. 1,531 rows of 2 heads of 128, 8 of 256, four taps, us: 26 / 20; 5 rows 6.0 / 4.5.
-template <int KT>
+// KEEP: the row is its request's only one, and the line moves on by it (entry k becomes what entry k + 1 was, the last one this row's input): a
+// channel belongs to one thread, so nobody else reads what it overwrites, and a decoded step saves the kernel that would do this for requests of any number of rows
+// (3 us).
+template <int KT, bool KEEP>
 __device__ __forceinline__ float dr_conv(const float* __restrict__ proj, long ldp, int col, const float* __restrict__ taps,
-                                         int K, int ch, int C, const float* __restrict__ line, long first_row, int i) {
+                                         int K, int ch, int C, float* line, long first_row, int i) {
   float acc = 0.f;
   if constexpr (KT > 0) {
     float x[KT], tap[KT];
@@ -41,11 +44,15 @@ __device__ __forceinline__ float dr_conv(const float* __restrict__ proj, long ld
     }
 #pragma unroll
     for (int j = 0; j < KT; ++j) acc += tap[j] * x[j];
+    if constexpr (KEEP)
+#pragma unroll
+      for (int j = 0; j + 1 < KT; ++j) line[(long)j * C + ch] = x[j + 1];
   } else {                // (a load on either side of the condition: with the address chosen first, 3 to 6 % slower at 2, 3, 5 and 8 taps)
     for (int j = 0; j < K; ++j) {
       const int at = i - (K - 1) + j;
       const float x = at >= 0 ? proj[(first_row + at) * ldp + col] : line[(long)(i + j) * C + ch];
       acc += taps[(long)ch * K + j] * x;
+      if (KEEP && j > 0) line[(long)(j - 1) * C + ch] = x;
     }
   }
   return acc * dr_sigmoid(acc);
@@ -53,10 +60,10 @@ __device__ __forceinline__ float dr_conv(const float* __restrict__ proj, long ld
 
 // grid (rows, units), one wave each. Units: the G query heads (unit vectors times dim^-1/2), the G key heads (unit
 // vectors), blocks of 64 value channels, and one for the heads' beta = sigmoid(.). out: [rows][C + H], C = 2 G D + H V.
-template <int KT>
+template <int KT, bool KEEP>
 __global__ __launch_bounds__(TIS_WAVE) void delta_prepare_kernel(
     const float* __restrict__ proj, long ldp, int conv_off, int beta_off, const float* __restrict__ taps, int K,
-    const float* __restrict__ state, long lds, int conv_at, const int* __restrict__ row_seq, const int* __restrict__ cu_rows,
+    float* state, long lds, int conv_at, const int* __restrict__ row_seq, const int* __restrict__ cu_rows,
     const int* __restrict__ seq_slots, float* __restrict__ out, long ldo, int H, int G, int D, int V) {
   const long r = blockIdx.x;
   const int unit = blockIdx.y, lane = threadIdx.x;
@@ -64,7 +71,7 @@ __global__ __launch_bounds__(TIS_WAVE) void delta_prepare_kernel(
   const int s = row_seq[r];
   const long first_row = cu_rows[s];
   const int i = (int)(r - first_row);
-  const float* line = state + (long)seq_slots[s] * lds + conv_at;
+  float* line = state + (long)seq_slots[s] * lds + conv_at;
   if (unit < 2 * G) {
     float y[DR_PER];
     float ss = 0.f;
@@ -74,7 +81,7 @@ __global__ __launch_bounds__(TIS_WAVE) void delta_prepare_kernel(
       y[u] = 0.f;
       if (e < D) {
         const int ch = unit * D + e;
-        y[u] = dr_conv<KT>(proj, ldp, conv_off + ch, taps, K, ch, C, line, first_row, i);
+        y[u] = dr_conv<KT, KEEP>(proj, ldp, conv_off + ch, taps, K, ch, C, line, first_row, i);
         ss += y[u] * y[u];
       }
     }
@@ -92,7 +99,7 @@ __global__ __launch_bounds__(TIS_WAVE) void delta_prepare_kernel(
     const int e = (unit - 2 * G) * TIS_WAVE + lane;
     if (e < H * V) {
       const int ch = 2 * G * D + e;
-      out[r * ldo + ch] = dr_conv<KT>(proj, ldp, conv_off + ch, taps, K, ch, C, line, first_row, i);
+      out[r * ldo + ch] = dr_conv<KT, KEEP>(proj, ldp, conv_off + ch, taps, K, ch, C, line, first_row, i);
     }
     return;
   }
@@ -592,9 +599,10 @@ __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(const float* __re
     }
 }
 
-TIS_EXPORT int tis_delta_prepare(const float* proj, long ldp, int conv_off, int beta_off, const float* taps, int K,
-                                 const float* state, long lds, int conv_at, const int* row_seq, const int* cu_rows,
-                                 const int* seq_slots, float* out, long ldo, int rows, int H, int G, int D, int V,
+// keep: every request of the step has one row, and its line's convolution inputs move on by it; 0: the lines stay as they are.
+TIS_EXPORT int tis_delta_prepare_keep(const float* proj, long ldp, int conv_off, int beta_off, const float* taps, int K,
+                                 float* state, long lds, int conv_at, const int* row_seq, const int* cu_rows,
+                                 const int* seq_slots, float* out, long ldo, int rows, int H, int G, int D, int V, int keep,
                                  hipStream_t stream) {
   if (rows == 0) return 0;
   if (rows < 0 || H < 1 || G < 1 || H % G || D < 1 || D > DR_PER * TIS_WAVE || V < 1 || K < 1 || K > DR_MAX_TAPS)
@@ -602,10 +610,19 @@ TIS_EXPORT int tis_delta_prepare(const float* proj, long ldp, int conv_off, int 
                     rows, H, G, D, DR_PER * TIS_WAVE, V, K, DR_MAX_TAPS);
   const int units = 2 * G + (H * V + TIS_WAVE - 1) / TIS_WAVE + 1;
   if (units > 65535) return tis_fail("delta_prepare: %d units a row are too many", units);
-  const auto kernel = K == 4 ? delta_prepare_kernel<4> : delta_prepare_kernel<0>;
+  const auto kernel = keep ? (K == 4 ? delta_prepare_kernel<4, true> : delta_prepare_kernel<0, true>)
+                           : (K == 4 ? delta_prepare_kernel<4, false> : delta_prepare_kernel<0, false>);
   kernel<<<dim3(rows, units), TIS_WAVE, 0, stream>>>(proj, ldp, conv_off, beta_off, taps, K, state, lds, conv_at, row_seq, cu_rows, seq_slots,
                                                      out, ldo, H, G, D, V);
   return tis_launch_status("delta_prepare");
+}
+
+TIS_EXPORT int tis_delta_prepare(const float* proj, long ldp, int conv_off, int beta_off, const float* taps, int K,
+                                 const float* state, long lds, int conv_at, const int* row_seq, const int* cu_rows,
+                                 const int* seq_slots, float* out, long ldo, int rows, int H, int G, int D, int V,
+                                 hipStream_t stream) {
+  return tis_delta_prepare_keep(proj, ldp, conv_off, beta_off, taps, K, const_cast<float*>(state), lds, conv_at, row_seq, cu_rows, seq_slots, out, ldo, rows,
+                                H, G, D, V, 0, stream);
 }
 
 // The most chunks that `rows` rows can have, over all requests of DR_CHUNK_FROM rows and more (each begins one that it may not fill).

@@ -809,20 +809,38 @@ TIS_EXPORT int tis_softcap(float* z, long ldz, float cap, int rows, int W, hipSt
 // x 1,024 7.0 / 4.3, 64 x 1,024 8.5 / 4.4, 1,531 x 1,024 15.4 / 12.4, 1,531 x 2,048 25.0 / 22.4; with all of a chunk's loads under way
 // together (before, each waited for the one before it), traced inside a pass, before / now: 5 rows 7.0 / 4.0, 1,531 rows, the two widths' mean, 20.1 / 13.1.
 static constexpr int LR_COLS = 32, LR_BY = S32_THREADS / LR_COLS;
+struct LowRank {
+  const float* low;
+  long ldl;
+  int rank;
+  const float *w2, *bias;
+  int kind;
+  float tau;
+  const float* rate;
+  int group;
+  float* out;
+  int C, col_blocks;
+};
+// x, y: the products of one launch; y's workgroups follow x's, of which there are `of_x` (one product: all)
 template <int RT, int LR_K, int V>
-__global__ __launch_bounds__(S32_THREADS) void lowrank_act_kernel(const float* __restrict__ low, long ldl, int rank,
-                                                                   const float* __restrict__ w2,
-                                                                   const float* __restrict__ bias, int kind, float tau,
-                                                                   const float* __restrict__ rate, int group,
-                                                                   float* __restrict__ out, int rows, int C, int col_blocks) {
+__global__ __launch_bounds__(S32_THREADS) void lowrank_act_kernel(LowRank x, LowRank y, int of_x, int rows) {
+  const bool first = (int)blockIdx.x < of_x;
+  const int block = first ? blockIdx.x : blockIdx.x - of_x;
+  const float *__restrict__ low = first ? x.low : y.low, *__restrict__ w2 = first ? x.w2 : y.w2, *__restrict__ bias = first ? x.bias : y.bias;
+  const float* __restrict__ rate = first ? x.rate : y.rate;
+  float* __restrict__ out = first ? x.out : y.out;
+  const long ldl = first ? x.ldl : y.ldl;
+  const int rank = first ? x.rank : y.rank, kind = first ? x.kind : y.kind, group = first ? x.group : y.group, C = first ? x.C : y.C;
+  const int col_blocks = first ? x.col_blocks : y.col_blocks;
+  const float tau = first ? x.tau : y.tau;
   __shared__ __attribute__((aligned(16))) float w[LR_COLS][LR_K + 4], a[LR_BY * RT][LR_K];
   typedef __attribute__((ext_vector_type(V))) float floats;
   constexpr int LINE = LR_K / V, WS = LR_COLS * LINE, AS = LR_BY * RT * LINE;      // pieces a line, of w's tile and of a's
   constexpr int WN = (WS + S32_THREADS - 1) / S32_THREADS, AN = (AS + S32_THREADS - 1) / S32_THREADS;
   // grid (blocks of rows * blocks of channels, a row block's side by side)
-  const long r0 = (long)(blockIdx.x / col_blocks) * (LR_BY * RT);
+  const long r0 = (long)(block / col_blocks) * (LR_BY * RT);
   const int n = (int)min((long)LR_BY * RT, rows - r0);
-  const int c0 = (blockIdx.x % col_blocks) * LR_COLS, cl = threadIdx.x % LR_COLS, rl = threadIdx.x / LR_COLS, c = c0 + cl;
+  const int c0 = (block % col_blocks) * LR_COLS, cl = threadIdx.x % LR_COLS, rl = threadIdx.x / LR_COLS, c = c0 + cl;
   const float b = bias && c < C ? bias[c] : 0.f;
   const float rt = kind == 1 && c < C ? rate[c / group] : 0.f;
   float z[RT];
@@ -881,22 +899,34 @@ __global__ __launch_bounds__(S32_THREADS) void lowrank_act_kernel(const float* _
 // short rank is, or copying zeros is most of the work. us, eight rows / 32: rank 64, 256 rows x 1,024 6.3 / 8.1, 256 x 2,048 8.5 / 9.0, 257 x 2,048
 // 10.9 / 8.9, 2,048 x 2,048 52 / 31; 2,048 x 32 4.6 / 7.7; rank 16, 256 x 1,024 4.6 / 4.7, 1,000 x 512 7.1 / 5.5, 2,048 x 4,096 71 / 34 (43
 // in chunks of 64; a channel's line of w2 walked by one thread: 31); 1 row x 1,024 3.3 (4.1 in chunks of 64).
-static void launch_lowrank(const float* low, long ldl, int rank, const float* w2, const float* bias, int kind, float tau,
-                           const float* rate, int group, float* out, int rows, int C, hipStream_t stream) {
-  const int col_blocks = (C + LR_COLS - 1) / LR_COLS;
-  const long small = ((long)rows + LR_BY - 1) / LR_BY * col_blocks;
-  const bool few = small <= (rank > 32 ? 2048 : 1024);
-  const long blocks = few ? small : ((long)rows + 4 * LR_BY - 1) / (4 * LR_BY) * col_blocks;
+// Which of the kernel's forms a product takes: rows a thread, chunk of the rank, values a load.
+struct LowRankForm {
+  bool few, fours;
+  int chunk;
+  long blocks;
+  bool operator==(const LowRankForm& o) const { return few == o.few && fours == o.fours && chunk == o.chunk; }
+};
+static LowRankForm lowrank_form(const LowRank& p, int rows) {
+  const long small = ((long)rows + LR_BY - 1) / LR_BY * p.col_blocks;
+  const bool few = small <= (p.rank > 32 ? 2048 : 1024);
   // lines that start on 16 bytes are read 16 at a time
-  const bool fours = rank % 4 == 0 && ldl % 4 == 0 && ((uintptr_t)low | (uintptr_t)w2) % 16 == 0;
-#define LOWRANK(RT, K, V) \
-  lowrank_act_kernel<RT, K, V><<<blocks, S32_THREADS, 0, stream>>>(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, col_blocks)
-#define LOWRANK_BY_ROWS(K) { if (fours) { if (few) LOWRANK(1, K, 4); else LOWRANK(4, K, 4); } else { if (few) LOWRANK(1, K, 1); else LOWRANK(4, K, 1); } }
-  if (rank <= 16) LOWRANK_BY_ROWS(16)
-  else if (rank <= 32) LOWRANK_BY_ROWS(32)
+  return {few, p.rank % 4 == 0 && p.ldl % 4 == 0 && ((uintptr_t)p.low | (uintptr_t)p.w2) % 16 == 0, p.rank <= 16 ? 16 : p.rank <= 32 ? 32 : 64,
+          few ? small : ((long)rows + 4 * LR_BY - 1) / (4 * LR_BY) * p.col_blocks};
+}
+static void launch_lowrank(const LowRank& x, const LowRank* y, int rows, hipStream_t stream) {
+  const LowRankForm f = lowrank_form(x, rows);
+  const long blocks = f.blocks + (y ? lowrank_form(*y, rows).blocks : 0);
+#define LOWRANK(RT, K, V) lowrank_act_kernel<RT, K, V><<<blocks, S32_THREADS, 0, stream>>>(x, y ? *y : x, (int)f.blocks, rows)
+#define LOWRANK_BY_ROWS(K) { if (f.fours) { if (f.few) LOWRANK(1, K, 4); else LOWRANK(4, K, 4); } else { if (f.few) LOWRANK(1, K, 1); else LOWRANK(4, K, 1); } }
+  if (f.chunk == 16) LOWRANK_BY_ROWS(16)
+  else if (f.chunk == 32) LOWRANK_BY_ROWS(32)
   else LOWRANK_BY_ROWS(64)
 #undef LOWRANK_BY_ROWS
 #undef LOWRANK
+}
+static void launch_lowrank(const float* low, long ldl, int rank, const float* w2, const float* bias, int kind, float tau,
+                           const float* rate, int group, float* out, int rows, int C, hipStream_t stream) {
+  launch_lowrank(LowRank{low, ldl, rank, w2, bias, kind, tau, rate, group, out, C, (C + LR_COLS - 1) / LR_COLS}, nullptr, rows, stream);
 }
 
 // out[r] = (1 / n) * sum_i y_i[r] / sqrt(mean(y_i[r]^2) + eps) * gain_i: the mean of one or two RMS-normed rows, 32-bit.
@@ -1003,6 +1033,27 @@ TIS_EXPORT int tis_lowrank_act(const float* low, long ldl, int rank, const float
   if (rank > 1024) return tis_fail("lowrank_act: rank %d (at most 1024)", rank);
   launch_lowrank(low, ldl, rank, w2, bias, kind, tau, rate, group, out, rows, C, stream);
   return tis_launch_status("lowrank_act");
+}
+
+// Two such products of the same rows, at most 2^31 workgroups together, in one launch where both take the same form (a mixer's decays and gates: a launch less, and
+// one tail; 5 rows of 64 against 512 and 1,024, us: 8.2 / 4.2; 1,531 rows against 1,024 and 2,048 27.2 / 22.0), else in two.
+TIS_EXPORT int tis_lowrank_act_pair(const float* low0, long ldl0, int rank0, const float* w0, const float* bias0, int kind0, float tau0, const float* rate0, int group0,
+                                    float* out0, int C0, const float* low1, long ldl1, int rank1, const float* w1, const float* bias1, int kind1, float tau1,
+                                    const float* rate1, int group1, float* out1, int C1, int rows, hipStream_t stream) {
+  if (rows == 0) return 0;
+  const LowRank p[2] = {{low0, ldl0, rank0, w0, bias0, kind0, tau0, rate0, group0, out0, C0, (C0 + LR_COLS - 1) / LR_COLS},
+                        {low1, ldl1, rank1, w1, bias1, kind1, tau1, rate1, group1, out1, C1, (C1 + LR_COLS - 1) / LR_COLS}};
+  for (const LowRank& q : p)
+    if (rows < 0 || q.rank < 1 || q.rank > 1024 || q.C < 1 || q.kind < 0 || q.kind > 2 || (q.kind == 0 && !(q.tau > 0.f)) || (q.kind == 1 && (!q.rate || q.group < 1)))
+      return tis_fail("lowrank_act: bad arguments rows=%d rank=%d channels=%d kind=%d", rows, q.rank, q.C, q.kind);
+  const LowRankForm a = lowrank_form(p[0], rows), b = lowrank_form(p[1], rows);
+  if (a == b && a.blocks + b.blocks < (1L << 31)) {
+    launch_lowrank(p[0], &p[1], rows, stream);
+  } else {
+    launch_lowrank(p[0], nullptr, rows, stream);
+    launch_lowrank(p[1], nullptr, rows, stream);
+  }
+  return tis_launch_status("lowrank_act_pair");
 }
 
 TIS_EXPORT int tis_normed_mean(const float* y0, long ld0, const float* g0, const float* y1, long ld1, const float* g1, float eps,

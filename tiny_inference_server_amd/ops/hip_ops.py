@@ -129,6 +129,7 @@ _SIGNATURES["stream32"] = ("tis_stream32", {
     "tis_gated_act": [_I, _P, _L, _I, _P, _P, _P, _I, _P, _L, _I, _F, _I, _P],
     "tis_softcap": [_P, _L, _F, _I, _I, _P],
     "tis_lowrank_act": [_P, _L, _I, _P, _P, _I, _F, _P, _I, _P, _I, _I, _P],
+    "tis_lowrank_act_pair": [_P, _L, _I, _P, _P, _I, _F, _P, _I, _P, _I, _P, _L, _I, _P, _P, _I, _F, _P, _I, _P, _I, _I, _P],
     "tis_normed_mean": [_P, _L, _P, _P, _L, _P, _F, _P, _I, _I, _P],
     "tis_activate_rows": [_I, _P, _L, _I, _P, _L, _I, _I, _P],
 })
@@ -162,6 +163,7 @@ _SIGNATURES["ssm_parts"] = ("tis_ssm", {
 
 _SIGNATURES["delta_rule"] = ("tis_delta_rule", {
     "tis_delta_prepare": [_P, _L, _I, _I, _P, _I, _P, _L, _I, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _P],
+    "tis_delta_prepare_keep": [_P, _L, _I, _I, _P, _I, _P, _L, _I, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
     "tis_delta_scan": [_P, _L, _I, _I, _I, _I, _P, _L, _P, _L, _P, _P, _I, _I, _I, _P, _P, _L, _I, _I, _I, _I, _P],
 })
 
@@ -1755,6 +1757,19 @@ class HipOps:
         """The second half of a low-rank projection in 32-bit: act(low . w2^T + bias) with low [rows, rank] (a strided view
         is fine), w2 [channels, rank], bias [channels] or None. kind "sigmoid_root": sigmoid(z)^(1/tau); "exp_softplus":
         exp(-rate[c // group] * softplus(z)), a decay with one rate per run of `group` channels; "none": z."""
+        out, args = self._lowrank_args(low, w2, bias, kind, rate, group, tau)
+        self._lazy("stream32").tis_lowrank_act(*args[:-1], low.shape[0], args[-1], self._stream())
+        return out
+
+    def lowrank_act_pair(self, first, second):
+        """lowrank_act(**first) and lowrank_act(**second), two products of the same number of rows, in one launch where their sizes allow."""
+        if first["low"].shape[0] != second["low"].shape[0]:
+            raise KernelError(f"lowrank_act_pair: {first['low'].shape[0]} and {second['low'].shape[0]} rows")
+        (out0, args0), (out1, args1) = self._lowrank_args(**first), self._lowrank_args(**second)
+        self._lazy("stream32").tis_lowrank_act_pair(*args0, *args1, out0.shape[0], self._stream())
+        return out0, out1
+
+    def _lowrank_args(self, low, w2, bias, kind: str, rate=None, group: int = 1, tau: float = 1.0):
         n, rank = low.shape
         _rows_view(self._check(low, "lowrank_act low", torch.float32), "lowrank_act low")
         C = w2.shape[0]
@@ -1768,10 +1783,8 @@ class HipOps:
                 raise KernelError(f"lowrank_act: {C} channels in runs of {group}")
             self._f32(rate, "lowrank_act rates", C // group)
         out = torch.empty(n, C, dtype=torch.float32, device=self.device)
-        self._lazy("stream32").tis_lowrank_act(_ptr(low), low.stride(0), rank, _ptr(w2), _ptr(bias), self._LOWRANK_KINDS[kind],
-                                               float(tau), _ptr(rate if kind == "exp_softplus" else None), int(group),
-                                               _ptr(out), n, C, self._stream())
-        return out
+        return out, (_ptr(low), low.stride(0), rank, _ptr(w2), _ptr(bias), self._LOWRANK_KINDS[kind], float(tau),
+                     _ptr(rate if kind == "exp_softplus" else None), int(group), _ptr(out), C)
 
     def softcap(self, z, cap: float):
         """z <- cap * tanh(z / cap) on 32-bit rows, in place."""
@@ -2385,6 +2398,17 @@ class HipOps:
         before those from the request's state line, from float conv_at on, [taps - 1][channels], oldest first) and silu;
         q and k become unit vectors per head (x / sqrt(sum x^2 + 1e-6)), q times dim^(-1/2). Returns
         u [rows, channels + heads] 32-bit: q, k, v, and beta = sigmoid(proj[:, beta_off + head])."""
+        return self._delta_prepare(proj, conv_off, beta_off, taps, state, conv_at, batch, n_heads, qk_heads, dim, vdim, False)
+
+    def delta_prepare_and_keep(self, proj, conv_off, beta_off, taps, state, conv_at, batch, n_heads, qk_heads, dim, vdim):
+        """delta_prepare, then conv_state_update of its columns: one kernel where every request brings a single row."""
+        single = batch.max_seq_rows <= 1 and taps.shape[1] > 1
+        u = self._delta_prepare(proj, conv_off, beta_off, taps, state, conv_at, batch, n_heads, qk_heads, dim, vdim, single)
+        if not single:
+            self.conv_state_update(proj, conv_off, taps.shape[0], taps.shape[1], state, conv_at, batch)
+        return u
+
+    def _delta_prepare(self, proj, conv_off, beta_off, taps, state, conv_at, batch, n_heads, qk_heads, dim, vdim, keep):
         n = proj.shape[0]
         C, K = taps.shape
         if C != 2 * qk_heads * dim + n_heads * vdim:
@@ -2394,10 +2418,10 @@ class HipOps:
         self._check_lines("delta_prepare", state, conv_at + (K - 1) * C, batch)
         self._index(batch.row_seq, "row_seq", n)
         u = torch.empty(n, C + n_heads, dtype=torch.float32, device=self.device)
-        self._lazy("delta_rule").tis_delta_prepare(
+        self._lazy("delta_rule").tis_delta_prepare_keep(
             _ptr(proj), proj.stride(0), int(conv_off), int(beta_off), _ptr(taps), K, _ptr(state), state.stride(0), int(conv_at),
             _ptr(batch.row_seq), _ptr(batch.cu_rows), _ptr(batch.seq_slots), _ptr(u), u.stride(0), n, n_heads, qk_heads, dim,
-            vdim, self._stream())
+            vdim, 1 if keep else 0, self._stream())
         return u
 
     def delta_scan(self, u, q_off, k_off, v_off, beta_off, decay, state, batch, n_heads, qk_heads, dim, vdim):

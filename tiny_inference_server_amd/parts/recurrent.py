@@ -320,12 +320,16 @@ class GatedDeltaRule:
         ops, b, at = self.ops, ctx.batch, self.at
         H, G, D, V, C = self.H, self.G, self.D, self.V, self.C
         # u: the convolved q (unit, scaled), k (unit), v side by side, then beta
-        u = ops.delta_prepare(proj, at["q"], at["b"], self.taps, ctx.state, self.conv_at, b, H, G, D, V)
-        ops.conv_state_update(proj, at["q"], C, self.K, ctx.state, self.conv_at, b)      # after the rows have read the line
-        decay = ops.lowrank_act(proj[:, at["a1"]:at["a1"] + self.ra], self.w_a2, self.dt_bias, "exp_softplus",
-                                rate=self.rate, group=D)
+        decays = dict(low=proj[:, at["a1"]:at["a1"] + self.ra], w2=self.w_a2, bias=self.dt_bias, kind="exp_softplus", rate=self.rate, group=D)
+        gates = dict(low=proj[:, at["g1"]:at["g1"] + self.rg], w2=self.w_g2, bias=None, kind="none")
+        if hasattr(ops, "delta_prepare_and_keep"):
+            u = ops.delta_prepare_and_keep(proj, at["q"], at["b"], self.taps, ctx.state, self.conv_at, b, H, G, D, V)
+            decay, gate = ops.lowrank_act_pair(decays, gates)
+        else:
+            u = ops.delta_prepare(proj, at["q"], at["b"], self.taps, ctx.state, self.conv_at, b, H, G, D, V)
+            ops.conv_state_update(proj, at["q"], C, self.K, ctx.state, self.conv_at, b)      # after the rows have read the line
+            decay, gate = ops.lowrank_act(**decays), ops.lowrank_act(**gates)
         o = ops.delta_scan(u, 0, G * D, 2 * G * D, C, decay, ctx.state, b, H, G, D, V)
-        gate = ops.lowrank_act(proj[:, at["g1"]:at["g1"] + self.rg], self.w_g2, None, "none")
         return ops.head_norm_gate(o, gate, self.norm_gain, H, V, self.eps, "sigmoid")
 
     def forward_projected(self, proj, ctx):
