@@ -43,6 +43,24 @@ def test_every_part_of_every_tile_once(step, splits, most, window):
         assert lengths == sorted(lengths, reverse=True)
 
 
+@pytest.mark.parametrize("tile_cols", [0, 32])
+@pytest.mark.parametrize("group", [1, 3, 4, 16, 32, 48, 100])
+def test_one_prompt_is_cut_like_a_prompt_among_others(group, tile_cols):
+    """A request alone in its step, against the same beside one without rows, whose lists are made over all requests."""
+    for m in (2, 3, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 1000, 1531, 2048, 6143, 6144, 6145):
+        for f, p0 in ((0, 0), (5, 1), (0, 31), (7, 4001)):
+            if group > 32 and tile_cols:        # (the tile kernel takes no such groups)
+                continue
+            alone, among = (attention_items(rows, group, tile_cols, 3) for rows in ([(f, p0, m)], [(f, p0, m), (f + m, 9, 0)]))
+            assert alone[0] == among[0] and alone[3] == among[3]
+            assert all(np.array_equal(x, y) and x.dtype == y.dtype for x, y in zip(alone[1:3], among[1:3]))
+
+
+def test_a_tile_of_no_request_is_refused():
+    with pytest.raises(hip_ops.KernelError, match="no request's"):
+        tile_pieces([(4, 0, 0), (8, 0, 32)], np.array([[4, 32]], dtype=np.int32), 2, 8)
+
+
 @pytest.mark.parametrize("total", [1, 255, 256, 257, 300, 511, 512, 513, 1000])
 def test_the_grid_takes_every_piece_once(total):
     """What piece_of of the kernel makes of the workgroups, for two a compute unit."""

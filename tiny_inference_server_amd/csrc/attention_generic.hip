@@ -14,6 +14,10 @@
 // What bounds it is the chain of trips to memory and through LDS of one small workgroup: the row's position and request, the block table, a
 // key's channels and the values, which are asked for together (rows of up to 50 keys, 8 heads of 8, 32-bit, us: one channel and one value after
 // the other 6.1, AG_AHEAD pieces of 16 bytes of a key and AG_AHEAD values of a thread at a time 5.1). The sums keep their order.
+#include <algorithm>
+#include <utility>
+#include <vector>
+
 #include "common.h"
 
 TIS_DEFINE_LAST_ERROR(tis_attention_generic)
@@ -158,4 +162,48 @@ TIS_EXPORT int tis_attention_generic(int dtype, const void* q, long q_ld, const 
   }
 #undef LAUNCH
   return tis_launch_status("attention_generic");
+}
+
+// ---- host planning -----------------------------------------------------------------------------------------
+//
+// The parts that the tile kernel of attention_mfma.hip cuts its tiles into, those with the longest chains of steps first (those alike in the order
+// of their tiles): (first row, rows + 256 * split, position of the first row, block-table line) each, into out [capacity][4]. rows: (first row, first
+// position, rows) of each request; tiles: (first row, rows) each. The counts are the kernel's own: a tile of n steps of 32 keys, from a multiple of 32
+// at or before the first key that any row sees, has min(splits, ceil(n / most)) parts of ceil(n / parts) steps, the last what is left. The host's
+// work before a prompt's first launch: 64 tiles cut in five 9 us with the call, 50 as array operations. Returns the parts, or -1.
+TIS_EXPORT int tis_attention_tile_pieces(const long* rows, int n_rows, const int* tiles, int n_tiles, int splits, int most, int window, int* out, int capacity) {
+  if (n_rows < 0 || n_tiles < 0 || splits < 1 || most < 1) return tis_fail("tile_pieces: %d tiles of %d requests, %d parts of %d steps", n_tiles, n_rows, splits, most), -1;
+  try {
+    struct Piece {
+      long steps;
+      int first, rows, pos, line;
+    };
+    std::vector<std::pair<long, int>> live;
+    for (int i = 0; i < n_rows; ++i)
+      if (rows[3 * i + 2] > 0) live.emplace_back(rows[3 * i], i);          // (first rows rise)
+    std::vector<Piece> pieces;
+    pieces.reserve(std::min((long)capacity, (long)n_tiles * splits));
+    for (int t = 0; t < n_tiles; ++t) {
+      const int first = tiles[2 * t], count = tiles[2 * t + 1];
+      auto after = std::upper_bound(live.begin(), live.end(), std::make_pair((long)first, n_rows));
+      if (after == live.begin()) return tis_fail("tile_pieces: the tile at row %d is no request's", first), -1;
+      const int line = (--after)->second;
+      const long pos = rows[3 * line + 1] + first - after->first;
+      const long seen = window > 0 ? std::max(0L, pos - window + 1) : window < 0 ? pos - pos % -(long)window : 0;
+      const long steps = (pos + count - (seen & ~31L) + 31) / 32;
+      const long parts = std::min((long)splits, std::max(1L, (steps + most - 1) / most)), per = (steps + parts - 1) / parts;
+      for (long s = 0; s < parts; ++s) pieces.push_back({std::min(per, steps - s * per), first, count + 256 * (int)s, (int)pos, line});
+    }
+    if (pieces.size() > (size_t)std::max(0, capacity)) return tis_fail("tile_pieces: %zu parts for %d places", pieces.size(), capacity), -1;
+    std::stable_sort(pieces.begin(), pieces.end(), [](const Piece& a, const Piece& b) { return a.steps > b.steps; });
+    for (const Piece& p : pieces) {
+      *out++ = p.first;
+      *out++ = p.rows;
+      *out++ = p.pos;
+      *out++ = p.line;
+    }
+    return (int)pieces.size();
+  } catch (...) {
+    return tis_fail("tile_pieces: no memory"), -1;
+  }
 }

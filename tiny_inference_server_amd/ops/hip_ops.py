@@ -76,6 +76,7 @@ _SIGNATURES = {
     }),
     "attention_generic": ("tis_attention_generic", {
         "tis_attention_generic": [_I, _P, _L, _P, _P, _I, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _F, _P, _P],
+        "tis_attention_tile_pieces": [_P, _I, _P, _I, _I, _I, _I, _P, _I],
     }),
     "gemm_plain": ("tis_gemm_plain", {
         "tis_gemm_plain": [_I, _I, _P, _L, _P, _L, _P, _L, _P, _L, _I, _I, _I, _P],
@@ -353,6 +354,24 @@ def attention_items(seq_rows, group_size: int, tile_cols: int = 0, n_kv_heads: i
     rows at 1,000 beside 8 decoded tokens at 4,095: 54.9 / 64.7, one of 256 rows 40.6 / 30.1, one of 128 35.9 / 23.9.
     """
     none = np.zeros((0, 2), dtype=np.int32)
+    tile_rows = _ATTN_TILE_WAVES * (tile_cols // group_size)
+    if len(seq_rows) == 1 and seq_rows[0][2] > 1:
+        # one prompt: its pieces as they lie, from the last, need neither the masks nor the sort below (64 tiles 9 us, 41 below; it is
+        # what a prompt's first launch waits for)
+        f, q0, m = seq_rows[0]
+        tiled, nb = bool(tile_rows) and m >= max(2, tile_rows // 2), 2
+        if not tiled and group_size <= 64 and -(-m // max(1, 64 // group_size)) >= 384:
+            nb = 4
+        while group_size > 16 * nb:
+            nb *= 2
+        per_item = tile_rows if tiled else max(1, (16 * nb) // group_size)
+        pieces = np.empty((-(-m // per_item), 2), dtype=np.int32)
+        r = np.arange((len(pieces) - 1) * per_item, -1, -per_item)
+        pieces[:, 0], pieces[:, 1], pieces[0, 1] = r + f, per_item, m - (len(pieces) - 1) * per_item
+        if not tiled:
+            return nb, pieces, none, (0, 0)
+        longest = (q0 + m + 31) // 32
+        return nb, none, pieces, (longest + int(((r[1:] + (q0 + per_item + 31)) >> 5).sum()), longest)
     # (arrays over all requests at once: a step may hold hundreds, and this runs for every stage of every step that
     # is not replayed from a graph)
     rows = np.asarray(seq_rows, dtype=np.int64).reshape(-1, 3)
@@ -379,7 +398,6 @@ def attention_items(seq_rows, group_size: int, tile_cols: int = 0, n_kv_heads: i
         steps = (keys + 31) // 32
         return np.stack((firsts[order], counts[order]), axis=1).astype(np.int32), (int(steps.sum()), int(steps.max()))
 
-    tile_rows = _ATTN_TILE_WAVES * (tile_cols // group_size)
     tiled = (n >= max(2, tile_rows // 2)) if tile_rows else np.zeros(len(n), dtype=bool)
     tiles, steps = cut(tiled, tile_rows) if tile_rows else (none, (0, 0))
     if len(tiles) and n_kv_heads and steps[0] * n_kv_heads < _ATTN_TILE_MIN_WORK_MIXED \
@@ -680,20 +698,14 @@ def tile_pieces(seq_rows, tiles, tile_splits: int, tile_max_steps: int, window: 
     """The parts that the tile kernel cuts its tiles into, those with the longest chains of steps first: int32 (first row, rows + 256 * split,
     position of the first row, block-table line) each. The counts are the kernel's own: a tile of n steps of 32 keys, from a multiple of 32 at or before
     the first key that any row sees, has min(tile_splits, ceil(n / tile_max_steps)) parts of ceil(n / parts) steps, the last what is left."""
-    rows = np.asarray(seq_rows, dtype=np.int64).reshape(-1, 3)
-    first, count = tiles[:, 0].astype(np.int64), tiles[:, 1].astype(np.int64)
-    live = np.nonzero(rows[:, 2] > 0)[0]                     # (first rows rise; of requests without rows none is a tile's)
-    line = live[np.searchsorted(rows[live, 0], first, side="right") - 1]
-    pos = rows[line, 1] + first - rows[line, 0]
-    seen = np.maximum(0, pos - window + 1) if window > 0 else pos - pos % (-window) if window < 0 else 0
-    steps = (pos + count - (seen & ~31) + 31) // 32
-    parts = np.clip(-(-steps // tile_max_steps), 1, tile_splits)
-    per = -(-steps // parts)
-    who = np.repeat(np.arange(len(tiles)), parts)
-    split = np.arange(len(who)) - np.repeat(np.cumsum(parts) - parts, parts)
-    by = np.argsort(-np.minimum(per[who], steps[who] - split * per[who]), kind="stable")
-    who, split = who[by], split[by]
-    return np.stack((first[who], count[who] + 256 * split, pos[who], line[who]), axis=1).astype(np.int32)
+    lib = library("attention_generic")
+    rows = np.array(seq_rows, dtype=np.int64)
+    tiles = np.ascontiguousarray(tiles, dtype=np.int32)
+    out = np.empty((len(tiles) * tile_splits, 4), dtype=np.int32)
+    n = lib.cdll.tis_attention_tile_pieces(rows.ctypes.data, len(rows), tiles.ctypes.data, len(tiles), tile_splits, tile_max_steps, window, out.ctypes.data, len(out))
+    if n < 0:
+        raise KernelError(lib._err().decode(errors="replace"))
+    return out[:n]
 
 
 _side_streams = {}
