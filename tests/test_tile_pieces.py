@@ -109,3 +109,36 @@ def test_listed_parts_give_the_same_bits(dim, H, G, window, sink, page, step):
             torch.cuda.synchronize()
             outs.append(out)
         assert torch.equal(*outs) and bool(torch.isfinite(outs[0]).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,H,G,sink", [(128, 8, 2, 0), (64, 8, 8, 1), (48, 5, 1, 0), (256, 8, 2, 0)])
+@pytest.mark.parametrize("cuts", [(2, 60), (4, 40), (5, 30), (9, 16), (80, 1)])
+def test_merged_rows_do_not_depend_on_how_many_there_are(dim, H, G, sink, cuts):
+    """Rows merged by four waves (few rows times heads) and by one (more): the same bits."""
+    ops, page, window = hip_ops.HipOps("cuda:0", torch.bfloat16), 16, 0
+    gen, p0, m = torch.Generator().manual_seed(dim), 2600, 100
+    q1 = torch.randn(m, H * dim, generator=gen).to(torch.bfloat16).cuda()
+    width = -(-(p0 + m) // page)
+    plane = torch.randn(width, 2 * G * page * dim, generator=gen).to(torch.bfloat16).cuda()
+    lib, outs = hip_ops.library(f"attention_mfma@{dim}"), []
+    for copies in (1, 2048 // (m * H) + 1, 8192 // (m * H)):
+        seq_rows = [(i * m, p0, m) for i in range(copies)]
+        n = m * copies
+        assert n * H <= 2048 if copies == 1 else 2048 < n * H <= 8192
+        nb, items, tiles, steps = attention_items(seq_rows, H // G, tile_columns(dim))
+        assert not len(items)
+        q, tables = q1.repeat(copies, 1), torch.arange(width, dtype=torch.int32).repeat(copies, 1).cuda()
+        seq = torch.arange(copies, dtype=torch.int32).repeat_interleave(m).cuda()
+        pos = (torch.arange(m, dtype=torch.int32) + p0).repeat(copies).cuda()
+        on_gpu = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (tiles, tile_pieces(seq_rows, tiles, *cuts, window))]
+        work = torch.empty(n * H * cuts[0] * (dim + 2) + n, device="cuda")
+        ml, rs = work[n * H * cuts[0] * dim:], work[n * H * cuts[0] * (dim + 2):]
+        out = torch.full((n, H * dim), 9.0, dtype=torch.bfloat16, device="cuda")
+        lib.tis_attention_mfma_pieces(
+            _ptr(q), q.stride(0), _ptr(plane), _ptr(tables), width, _ptr(seq), _ptr(pos), None, 0, nb, _ptr(on_gpu[0]), len(tiles), _ptr(out), out.stride(0), _ptr(work),
+            _ptr(ml), n, H, G, dim, page, window, dim ** -0.5, 1, 0, cuts[0], cuts[1], _ptr(rs), sink, None, None, None, 0, 0.0, _ptr(on_gpu[1]), len(on_gpu[1]), ops.units, ops._stream())
+        torch.cuda.synchronize()
+        outs.append(out)
+    for out in outs[1:]:
+        assert torch.equal(out, outs[0].repeat(len(out) // m, 1)) and bool(torch.isfinite(out).all())

@@ -930,6 +930,12 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_kernel(const float* _
 // the previous head's. Up to four splits are asked for all at once, before their weights are known: split after split, each one's
 // load waited for the one before (2,048 rows of 12 heads of 128, up to three splits: 11.3 us; 6.8 so).
 static constexpr int FEW_SPLITS = 4;
+// From so many rows times heads on a wave merges one head of a row. Fewer keep four waves each and their trips to memory short; between this and 8,192
+// the sums are those of that kernel. us of attention and merge, four waves
+// / one: 1,000 tokens of 8 heads over 2 31.9 / 19.3; 512 behind 3,000 others, 12 over 3, 41.3 / 31.0, 190 26.4 / 23.4; 140 behind 4,000, 16 over 4, 28.9 / 26.6.
+static constexpr long MERGE_ROWS_FROM = 2048;
+// APART: with the sums of attention_merge_kernel, to the bit: products rounded by themselves, every MG-th split's added up first.
+template <bool APART>
 __global__ __launch_bounds__(MG * 64) void attention_merge_rows_kernel(const float* __restrict__ part_o,
                                                                        const float2* __restrict__ part_ml,
                                                                        bf16* __restrict__ out, long out_ld,
@@ -962,7 +968,9 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_rows_kernel(const flo
     for (int i = 0; i < FEW_SPLITS; ++i) {
       w[i] = i < n_splits && ml[i].x != -INFINITY ? exp2f(ml[i].x - M) : 0.f;
 #pragma unroll
-      for (int j = 0; j < MD; ++j) acc[j] = w[i] != 0.f ? acc[j] + w[i] * o[i][j] : acc[j];
+      for (int j = 0; j < MD; ++j)
+        if constexpr (APART) acc[j] += w[i] != 0.f ? __builtin_fmaf(w[i], o[i][j], 0.f) : 0.f;
+        else acc[j] = w[i] != 0.f ? acc[j] + w[i] * o[i][j] : acc[j];
       ml[i].y = w[i] != 0.f ? w[i] * ml[i].y : 0.f;
     }
     L = (ml[0].y + ml[2].y) + (ml[1].y + ml[3].y);
@@ -971,6 +979,11 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_rows_kernel(const flo
       if (s0 + lane < n_splits) M = fmaxf(M, part_ml[base + s0 + lane].x);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    float part[MG][MD];
+#pragma unroll
+    for (int g = 0; g < MG; ++g)
+#pragma unroll
+      for (int j = 0; j < MD; ++j) part[g][j] = 0.f;
     for (int s0 = 0; s0 < n_splits; s0 += 64) {
       float w = 0.f;
       if (s0 + lane < n_splits) {
@@ -981,13 +994,36 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_rows_kernel(const flo
         }
       }
       const int cnt = min(64, n_splits - s0);
-      for (int i = 0; i < cnt; ++i) {
+      if constexpr (APART) {
+        for (int i = 0; i < cnt; i += 2 * MG) {
+          float v[2 * MG][MD];
+#pragma unroll
+          for (int u = 0; u < 2 * MG; ++u)
+#pragma unroll
+            for (int j = 0; j < MD; ++j) v[u][j] = part_o[(base + s0 + min(i + u, cnt - 1)) * VD + min(j * 64 + lane, VD - 1)];
+#pragma unroll
+          for (int u = 0; u < 2 * MG; ++u) {
+            const float wi = i + u < cnt ? __shfl(w, i + u, 64) : 0.f;
+#pragma unroll
+            for (int j = 0; j < MD; ++j)
+              if (wi != 0.f) part[u % MG][j] = __builtin_fmaf(wi, v[u][j], part[u % MG][j]);
+          }
+        }
+      } else for (int i = 0; i < cnt; ++i) {
         const float wi = __shfl(w, i, 64);
 #pragma unroll
         for (int j = 0; j < MD; ++j) {
           const int d = j * 64 + lane;
           if (d < VD && wi != 0.f) acc[j] += wi * part_o[(base + s0 + i) * VD + d];
         }
+      }
+    }
+    if constexpr (APART) {
+#pragma unroll
+      for (int j = 0; j < MD; ++j) {
+        acc[j] = part[0][j];
+#pragma unroll
+        for (int g = 1; g < MG; ++g) acc[j] += part[g][j];
       }
     }
 #pragma unroll
@@ -1167,9 +1203,11 @@ static int attention_launch(const void* q, long q_ld, const void* plane, const i
     return tis_fail("attention_mfma: the first stream could not wait for the second");
   if (rc) return rc;
   if (stride > 1) {
-    if ((long)rows * n_heads > 8192) {
+    if ((long)rows * n_heads > MERGE_ROWS_FROM) {
       dim3 mgrid(rows, (n_heads + MG - 1) / MG);
-      attention_merge_rows_kernel<<<mgrid, MG * 64, 0, stream>>>(part_o, (const float2*)part_ml, (bf16*)out, out_ld,
+      if ((long)rows * n_heads <= 8192) attention_merge_rows_kernel<true><<<mgrid, MG * 64, 0, stream>>>(part_o, (const float2*)part_ml, (bf16*)out, out_ld,
+                                                                 n_heads, stride, row_splits, sink, sinks, turn, extras);
+      else attention_merge_rows_kernel<false><<<mgrid, MG * 64, 0, stream>>>(part_o, (const float2*)part_ml, (bf16*)out, out_ld,
                                                                  n_heads, stride, row_splits, sink, sinks, turn, extras);
     } else {
       dim3 mgrid(rows, n_heads);
