@@ -928,7 +928,8 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_kernel(const float* _
 // was not split costs one load. With a workgroup per (row, head) the thousands of rows of a prompt would mean tens of
 // thousands of workgroups; with a wave taking several heads in turn, each head's two round trips to memory follow
 // the previous head's. Up to four splits are asked for all at once, before their weights are known: split after split, each one's
-// load waited for the one before (2,048 rows of 12 heads of 128, up to three splits: 11.3 us; 6.8 so).
+// load waited for the one before (2,048 rows of 12 heads of 128, up to three splits: 11.3 us; 6.8 so). More splits go eight at a time (attention and
+// merge, one by one / so: 1,500 tokens behind 1,000, 8 heads over 2, six splits 35.5 / 32.9 us; 700 behind 3,000, 12 over 3, 42.6 / 37.7).
 static constexpr int FEW_SPLITS = 4;
 // From so many rows times heads on a wave merges one head of a row. Fewer keep four waves each and their trips to memory short; between this and 8,192
 // the sums are those of that kernel. us of attention and merge, four waves
@@ -994,27 +995,20 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_rows_kernel(const flo
         }
       }
       const int cnt = min(64, n_splits - s0);
-      if constexpr (APART) {
-        for (int i = 0; i < cnt; i += 2 * MG) {
-          float v[2 * MG][MD];
+      for (int i = 0; i < cnt; i += 2 * MG) {      // eight splits under way at once (past the last: the last one's again)
+        float v[2 * MG][MD];
 #pragma unroll
-          for (int u = 0; u < 2 * MG; ++u)
+        for (int u = 0; u < 2 * MG; ++u)
 #pragma unroll
-            for (int j = 0; j < MD; ++j) v[u][j] = part_o[(base + s0 + min(i + u, cnt - 1)) * VD + min(j * 64 + lane, VD - 1)];
+          for (int j = 0; j < MD; ++j) v[u][j] = part_o[(base + s0 + min(i + u, cnt - 1)) * VD + min(j * 64 + lane, VD - 1)];
 #pragma unroll
-          for (int u = 0; u < 2 * MG; ++u) {
-            const float wi = i + u < cnt ? __shfl(w, i + u, 64) : 0.f;
+        for (int u = 0; u < 2 * MG; ++u) {
+          const float wi = i + u < cnt ? __shfl(w, i + u, 64) : 0.f;
 #pragma unroll
-            for (int j = 0; j < MD; ++j)
-              if (wi != 0.f) part[u % MG][j] = __builtin_fmaf(wi, v[u][j], part[u % MG][j]);
+          for (int j = 0; j < MD; ++j) {
+            float& sum = APART ? part[u % MG][j] : acc[j];
+            if (wi != 0.f) sum = __builtin_fmaf(wi, v[u][j], sum);
           }
-        }
-      } else for (int i = 0; i < cnt; ++i) {
-        const float wi = __shfl(w, i, 64);
-#pragma unroll
-        for (int j = 0; j < MD; ++j) {
-          const int d = j * 64 + lane;
-          if (d < VD && wi != 0.f) acc[j] += wi * part_o[(base + s0 + i) * VD + d];
         }
       }
     }
