@@ -3,6 +3,7 @@ forms, and the engine (step function, cache manager, scheduler, generate) on the
 plain implementation, in 32-bit."""
 import copy
 import math
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -14,6 +15,7 @@ from torch_ops import TorchOps
 from tiny_inference_server_amd.config import ARCHITECTURES, ConfigError, config_from_dict, load_config
 from tiny_inference_server_amd.engine import Engine
 from tiny_inference_server_amd.engine.generate import generate
+from tiny_inference_server_amd.ops.hip_ops import HipOps
 from tiny_inference_server_amd.parts.attention import slowed_frequencies
 from tiny_inference_server_amd.weights.loader import spec_tensors
 
@@ -358,3 +360,35 @@ def test_the_named_size_runs_with_random_weights(tmp_path):
     eng = Engine(folder, dtype="float32", max_tokens=64, max_requests=2, ops=TorchOps())
     out = eng.step([("a", [5, 9, 1, 300], [3]), ("b", [7], [0])]).logits
     assert out.shape == (2, cfg.vocab) and torch.isfinite(out).all()
+
+
+class PlannedOps(TorchOps):
+    """The stand-in with the device's own attention planning, whose lists it carries through every step and ignores."""
+
+    def plan_attention_mode(self, seq_rows, window=0):
+        return HipOps.plan_attention_mode(SimpleNamespace(dtype=torch.bfloat16), seq_rows, window)
+
+    def plan_attention(self, *args, **kw):
+        return HipOps.plan_attention(SimpleNamespace(dtype=torch.bfloat16, units=256), *args, **kw)
+
+
+@pytest.mark.parametrize("sizes", [((4, 2, 20, 20, 30.0), (4, 2, 20, 20, None)), ((4, 2, 20, 24, None), (4, 2, 20, 24, 6.0), (4, 2, 20, 24, 2.0))])
+@pytest.mark.parametrize("lengths", [(9,), (300, 20, 25, 30, 18, 22, 27, 19, 31, 26, 24, 23)])
+def test_layers_that_differ_in_their_caps_alone_decode_from_captured_steps(sizes, lengths):
+    """Their steps carry lists of one name: a captured step must find a place for everything that is planned for the step after. One request, and
+    requests of such different lengths that their splits are planned."""
+    cfg = TM.config(48, 97, [TM.layer(TM.mixer(H_, G, D, V, 0.4, cap=cap, dims=8), TM.dense(24)) for H_, G, D, V, cap in sizes])
+    c, w = config_from_dict(cfg), {n: t.float() for n, t in TM.random_weights(cfg, 3).items()}
+    replayed, launched = (Engine(config=c, tensors=w, dtype="float32", page_size=16, max_tokens=2048, max_requests=len(lengths), use_graphs=graphs, ops=PlannedOps(graphs=graphs))
+                          for graphs in (True, False))
+    ids = {f"r{i}": H.random_ids(97, n + 8, 40 + i) for i, n in enumerate(lengths)}
+    for eng in (replayed, launched):
+        for rid, t in ids.items():
+            eng.step([(rid, t[:-8], [])])
+    for k in range(8):
+        entries = [(rid, [t[len(t) - 8 + k]], [0]) for rid, t in ids.items()]
+        got, want = replayed.step(entries).logits, launched.step(entries).logits
+        assert (got - want).abs().max().item() <= 1e-5 * max(1.0, want.abs().max().item())
+    assert replayed.graph_replays >= 6
+    if len(lengths) > 1:
+        assert any(g.mode is not None for g in replayed._graphs.values())

@@ -71,21 +71,6 @@ def test_the_grid_takes_every_piece_once(total):
     assert all(b == min(2 * units, total) - 1 - a for a, b in beside)        # the longest has the shortest beside it
 
 
-def test_tiles_with_capped_scores_are_cut_no_later():
-    """Steps that take longer make whole tiles longer and leave the merge as it is: what is cut without a cap is cut alike with one."""
-    earlier = 0
-    for H, G in ((16, 4), (8, 2), (12, 3), (32, 8)):
-        for step in sorted(STEPS) + list(range(200, 3000, 150)):
-            seq_rows = rows_of(STEPS[step] if step in STEPS else [(0, step)])
-            nb, items, tiles, steps = attention_items(seq_rows, H // G, 32)
-            args = (sum(r[2] for r in seq_rows), len(items), len(tiles), steps, False, max(p + n for _, p, n in seq_rows), H, G, 128)
-            plain, capped = attention_launch_plan(*args), attention_launch_plan(*args, capped=True)
-            if plain.tile_splits > 1:
-                assert capped == plain
-            earlier += capped.tile_splits > plain.tile_splits
-    assert earlier
-
-
 @pytest.mark.gpu
 @pytest.mark.parametrize("dim,H,G,window,sink,page", [(128, 12, 3, 0, 0, 16), (128, 16, 4, 700, 0, 16), (64, 8, 8, -512, 0, 16), (256, 8, 2, 0, 1, 32), (48, 32, 1, 0, 0, 48)])
 @pytest.mark.parametrize("step", sorted(STEPS))

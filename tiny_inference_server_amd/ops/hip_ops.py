@@ -315,7 +315,6 @@ _ATTN_TILE_MIN_STEPS = 8        # steps of 32 keys below which a tile's split is
 _ATTN_TILE_SPLIT_SLACK = 1.4    # a split may be this much longer than an even share of all steps
 _ATTN_TILE_STEP_US = (0.72, 1.3)   # what a tile's step of 32 keys takes while a workgroup has a compute unit to itself,
                                 # and once two share one (12 heads of 128 over 3; other geometries differ little)
-_ATTN_TILE_CAPPED = 1.65        # ... and how much longer with capped scores (an exponential and a reciprocal more for each)
 _ATTN_TILE_MERGE_US = (10.0, 4.0, 6e6)   # what cutting tiles into key splits costs beyond the tiles' own time: the
                                 # merge's launch and the per-row counts (less where the items' splits are merged anyway),
                                 # and microseconds per byte of 32-bit partial results. Tiles are cut only where, by
@@ -616,11 +615,11 @@ class AttentionLaunch(NamedTuple):
     need_floats: int
 
 
-def _tiles_us(n, n_tiles, all_steps, longest, cut, cut_steps, n_heads, n_kv_heads, head_dim, merged_anyway, units, longer=1.0):
+def _tiles_us(n, n_tiles, all_steps, longest, cut, cut_steps, n_heads, n_kv_heads, head_dim, merged_anyway, units):
     """Estimated microseconds of a call's tiles left whole, and cut into `cut` key splits of at most `cut_steps` steps:
     the longest chain of steps sets the time (a step takes longer once two workgroups share a compute unit, and no
     less than all steps spread evenly take), and the cut adds the merge."""
-    alone, shared = (us * longer for us in _ATTN_TILE_STEP_US)
+    alone, shared = _ATTN_TILE_STEP_US
 
     def chain_us(steps, workgroups):
         return max(steps * min(shared, alone * max(1.0, workgroups / units)), all_steps * n_kv_heads / (2 * units) * shared)
@@ -648,10 +647,8 @@ def _tiles_cut(n, n_tiles, tile_steps, n_heads, n_kv_heads, head_dim):
 
 
 def attention_launch_plan(n, n_items, n_tiles, tile_steps, single, max_kv_len, n_heads, n_kv_heads, head_dim,
-                          workspace_floats=None, planned_splits=0, units: int = _CHIP_UNITS, capped=False) -> AttentionLaunch:
+                          workspace_floats=None, planned_splits=0, units: int = _CHIP_UNITS) -> AttentionLaunch:
     """Split counts of one attention call over `n` rows, from the planner's items and tiles; pure host arithmetic.
-    capped: scores are capped: a tile's steps take longer, so that its cuts pay earlier (one prompt, 16 heads of 128 over 4, us whole / cut with the
-    merge: 2,048 tokens 78.1 / 57.3, 700 33.5 / 25.7).
     planned_splits > 0: the items are a list planned by decode_items, whose rows have at most that many splits."""
     workspace_floats = _ATTN_WORKSPACE_FLOATS if workspace_floats is None else workspace_floats
     n_splits, min_steps, tile_splits, tile_max_steps = 1, 0, 1, 1 << 20
@@ -684,7 +681,7 @@ def attention_launch_plan(n, n_items, n_tiles, tile_steps, single, max_kv_len, n
         all_steps, longest = tile_steps
         cut, cut_steps = _tiles_cut(n, n_tiles, tile_steps, n_heads, n_kv_heads, head_dim)
         if cut > 1 and _tiles_cut_pays(n, n_tiles, all_steps, longest, cut, cut_steps, n_heads, n_kv_heads, head_dim,
-                                       n_splits > 1, units, *((_ATTN_TILE_CAPPED,) if capped else ())):
+                                       n_splits > 1, units):
             tile_splits, tile_max_steps = cut, cut_steps
     # partial results of split key ranges live in one workspace of fixed size; fewer splits where it
     # would not suffice
@@ -778,7 +775,7 @@ class HipOps:
         request, where the mixer has a window)."""
         return "uneven" if self.dtype == torch.bfloat16 and uneven_lengths(seq_rows, window) else None
 
-    def plan_attention(self, n_heads: int, n_kv_heads: int, head_dim: int, seq_rows, add, mode=None, window: int = 0, capped: bool = False):
+    def plan_attention(self, n_heads: int, n_kv_heads: int, head_dim: int, seq_rows, add, mode=None, window: int = 0):
         """An attention mixer's host planning, called while a step's arrays are packed: the work items of the
         matrix-core kernels for the step's rows. Returns {name: (packed array id, host values...)}."""
         plans = {}
@@ -803,7 +800,7 @@ class HipOps:
             if len(tiles) and ("attention_items", group, cols, n_kv_heads, window) in plans:
                 lp = attention_launch_plan(sum(n for _, _, n in seq_rows), len(items) if beside is None else len(entries), len(tiles), steps, False,
                                            max(p0 + n for _, p0, n in seq_rows), n_heads, n_kv_heads, head_dim,
-                                           planned_splits=0 if beside is None else most, units=self.units, capped=capped)
+                                           planned_splits=0 if beside is None else most, units=self.units)
                 if lp.tile_splits > 1:
                     pieces = tile_pieces(seq_rows, tiles, lp.tile_splits, lp.tile_max_steps, window)
                     plans[("attention_tile_pieces", group, cols, n_kv_heads, window)] = (add(pieces), len(pieces), lp.tile_splits, lp.tile_max_steps)
@@ -1410,7 +1407,7 @@ class HipOps:
                                   f"assumes {cols}")
         single = items is None and n_tiles == 0
         lp = attention_launch_plan(n, n_items, n_tiles, tile_steps, single, batch.max_kv_len, n_heads, n_kv_heads,
-                                   value_dim, planned_splits=planned_splits, units=self.units, capped=softcap > 0)
+                                   value_dim, planned_splits=planned_splits, units=self.units)
         n_splits, min_steps, tile_splits, tile_max_steps = lp.n_splits, lp.min_steps, lp.tile_splits, lp.tile_max_steps
         part_o = part_ml = row_splits = None
         if lp.stride > 1:

@@ -760,15 +760,14 @@ class CappedAttention:
 
     # the matrix-core kernels' work lists (see GqaAttention)
     def plan_key(self):
-        return ("attention", self.H, self.G, max(self.kd, self.vd), 0, self.softcap > 0) if hasattr(self.ops, "plan_attention") else None
+        return ("attention", self.H, self.G, max(self.kd, self.vd), 0) if hasattr(self.ops, "plan_attention") else None
 
     def plan_mode(self, seq_rows):
         mode = getattr(self.ops, "plan_attention_mode", None)
         return mode(seq_rows, 0) if mode is not None else None
 
     def plan_rows(self, seq_rows, add, mode=None):
-        capped = {"capped": True} if self.softcap else {}
-        return self.ops.plan_attention(self.H, self.G, max(self.kd, self.vd), seq_rows, add, mode, 0, **capped)
+        return self.ops.plan_attention(self.H, self.G, max(self.kd, self.vd), seq_rows, add, mode, 0)
 
     def core(self, x, ctx):
         ops, b = self.ops, ctx.batch
