@@ -372,11 +372,12 @@ class PlannedOps(TorchOps):
         return HipOps.plan_attention(SimpleNamespace(dtype=torch.bfloat16, units=256), *args, **kw)
 
 
-@pytest.mark.parametrize("sizes", [((4, 2, 20, 20, 30.0), (4, 2, 20, 20, None)), ((4, 2, 20, 24, None), (4, 2, 20, 24, 6.0), (4, 2, 20, 24, 2.0))])
+@pytest.mark.parametrize("sizes", [((4, 2, 20, 20, 30.0), (4, 2, 20, 20, None)), ((4, 2, 20, 24, None), (4, 2, 20, 24, 6.0), (4, 2, 20, 24, 2.0)),
+                                   ((4, 2, 20, 20, 6.0), (4, 2, 32, 32, 6.0)), ((6, 3, 16, 48, None), (6, 3, 32, 32, None), (6, 3, 48, 16, None))])
 @pytest.mark.parametrize("lengths", [(9,), (300, 20, 25, 30, 18, 22, 27, 19, 31, 26, 24, 23)])
-def test_layers_that_differ_in_their_caps_alone_decode_from_captured_steps(sizes, lengths):
-    """Their steps carry lists of one name: a captured step must find a place for everything that is planned for the step after. One request, and
-    requests of such different lengths that their splits are planned."""
+def test_layers_that_differ_in_caps_or_head_sizes_alone_decode_from_captured_steps(sizes, lengths):
+    """A captured step must find a place for every list that is planned for the step after, whether layers share one or not. One request, and requests of
+    such different lengths that their splits are planned."""
     cfg = TM.config(48, 97, [TM.layer(TM.mixer(H_, G, D, V, 0.4, cap=cap, dims=8), TM.dense(24)) for H_, G, D, V, cap in sizes])
     c, w = config_from_dict(cfg), {n: t.float() for n, t in TM.random_weights(cfg, 3).items()}
     replayed, launched = (Engine(config=c, tensors=w, dtype="float32", page_size=16, max_tokens=2048, max_requests=len(lengths), use_graphs=graphs, ops=PlannedOps(graphs=graphs))

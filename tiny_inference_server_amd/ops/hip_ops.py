@@ -777,33 +777,34 @@ class HipOps:
 
     def plan_attention(self, n_heads: int, n_kv_heads: int, head_dim: int, seq_rows, add, mode=None, window: int = 0):
         """An attention mixer's host planning, called while a step's arrays are packed: the work items of the
-        matrix-core kernels for the step's rows. Returns {name: (packed array id, host values...)}."""
+        matrix-core kernels for the step's rows. Returns {name: (packed array id, host values...)}. A name holds all that the lists depend on:
+        of two mixers that plan under one name, a captured step would keep one list and be given two."""
         plans = {}
         if self.dtype == torch.bfloat16:
             group, cols = n_heads // n_kv_heads, tile_columns(head_dim)
             if (mode == "uneven" and group <= 64 and planned_list_pays(len(seq_rows), n_kv_heads)
                     and all(n == 1 for _, _, n in seq_rows)):
                 entries, most = decode_items(seq_rows, n_heads, n_kv_heads, head_dim, window=window, units=self.units)
-                return {("attention_decode_items", group, cols, n_kv_heads, window): (add(entries), len(entries), most)}
+                return {("attention_decode_items", group, cols, n_kv_heads, window, head_dim): (add(entries), len(entries), most)}
             nb, items, tiles, steps = attention_items(seq_rows, group, cols, n_kv_heads)
             beside = planned_beside_tiles(seq_rows, items, tiles, steps, n_heads, n_kv_heads, head_dim, window, self.units)
             if beside is not None:
                 # one array: the planned entries of four integers, then the tiles' lines of two
                 entries, most = beside
-                plans[("attention_items", group, cols, n_kv_heads, window)] = (
+                plans[("attention_items", group, cols, n_kv_heads, window, head_dim)] = (
                     add(np.concatenate((entries.reshape(-1), tiles.reshape(-1)))), len(entries), 1, len(tiles), steps, most)
             elif nb <= 4 and (len(items) or len(tiles)):
                 # one array: the items' lines, then the tiles'
                 # (a mixer with a window plans for itself: its lists are the same, its keys are its own)
-                plans[("attention_items", group, cols, n_kv_heads, window)] = (add(np.concatenate((items, tiles))), len(items),
-                                                                       nb, len(tiles), steps, 0)
-            if len(tiles) and ("attention_items", group, cols, n_kv_heads, window) in plans:
+                plans[("attention_items", group, cols, n_kv_heads, window, head_dim)] = (add(np.concatenate((items, tiles))), len(items), nb, len(tiles),
+                                                                                         steps, 0)
+            if len(tiles) and ("attention_items", group, cols, n_kv_heads, window, head_dim) in plans:
                 lp = attention_launch_plan(sum(n for _, _, n in seq_rows), len(items) if beside is None else len(entries), len(tiles), steps, False,
                                            max(p0 + n for _, p0, n in seq_rows), n_heads, n_kv_heads, head_dim,
                                            planned_splits=0 if beside is None else most, units=self.units)
                 if lp.tile_splits > 1:
                     pieces = tile_pieces(seq_rows, tiles, lp.tile_splits, lp.tile_max_steps, window)
-                    plans[("attention_tile_pieces", group, cols, n_kv_heads, window)] = (add(pieces), len(pieces), lp.tile_splits, lp.tile_max_steps)
+                    plans[("attention_tile_pieces", group, cols, n_kv_heads, window, head_dim)] = (add(pieces), len(pieces), lp.tile_splits, lp.tile_max_steps)
         return plans
 
     # ---- helpers -------------------------------------------------------------------------------------
@@ -1347,19 +1348,18 @@ class HipOps:
                                    scale, sink, sinks, turn, softcap=0.0, channel_gate=None):
         """The launch that paged_attention and paged_attention_kv share, once they have checked their arguments."""
         n, group = q.shape[0], n_heads // n_kv_heads
-        cols = tile_columns(max(key_dim, value_dim))
-        planned = batch.extras.get(("attention_decode_items", group, cols, n_kv_heads, int(window)))
-        plan = batch.extras.get(("attention_items", group, cols, n_kv_heads, int(window)))
+        size = max(key_dim, value_dim)          # what a mixer's planner goes by
+        cols = tile_columns(size)
+        planned = batch.extras.get(("attention_decode_items", group, cols, n_kv_heads, int(window), size))
+        plan = batch.extras.get(("attention_items", group, cols, n_kv_heads, int(window), size))
         if planned is None and plan is None:
             # a caller that did not plan (a kernel test): plan now, tiles wherever they fit
             if uneven_lengths(batch.seq_rows, int(window)) and planned_list_pays(n, n_kv_heads):
-                entries, most = decode_items(batch.seq_rows, n_heads, n_kv_heads, max(key_dim, value_dim), window=int(window),
-                                             units=self.units)
+                entries, most = decode_items(batch.seq_rows, n_heads, n_kv_heads, size, window=int(window), units=self.units)
                 planned = (torch.from_numpy(entries).reshape(-1).to(self.device), len(entries), most)
             else:
                 nb, host_items, host_tiles, steps = attention_items(batch.seq_rows, group, cols)
-                beside = planned_beside_tiles(batch.seq_rows, host_items, host_tiles, steps, n_heads, n_kv_heads,
-                                              max(key_dim, value_dim), int(window), self.units)
+                beside = planned_beside_tiles(batch.seq_rows, host_items, host_tiles, steps, n_heads, n_kv_heads, size, int(window), self.units)
                 if beside is not None:
                     both = np.concatenate((beside[0].reshape(-1), host_tiles.reshape(-1)))
                     plan = (torch.from_numpy(np.ascontiguousarray(both)).to(self.device), len(beside[0]), 1,
@@ -1422,7 +1422,7 @@ class HipOps:
             raise KernelError("attention: the work list must be contiguous 32-bit integers")
         pieces, n_pieces = None, 0
         if tile_splits > 1:
-            made = batch.extras.get(("attention_tile_pieces", group, cols, n_kv_heads, int(window)))
+            made = batch.extras.get(("attention_tile_pieces", group, cols, n_kv_heads, int(window), size))
             if made is not None and made[2:] == (tile_splits, tile_max_steps):      # (planned for these very cuts)
                 pieces, n_pieces = made[0].reshape(-1), made[1]
                 if pieces.dtype != torch.int32 or not pieces.is_contiguous() or pieces.numel() != 4 * n_pieces:
