@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import gc
 import time
+from collections import deque
 
 import numpy as np
 import torch
@@ -29,6 +30,73 @@ class _NoEvent:
 
     def synchronize(self):
         pass
+
+
+class HostSets:
+    """The sets of a captured step's arrays in host memory: two, written in turn, where the graph itself takes them from there (upload_ring), and
+    `done` is where the GPU writes down how many replays each of its workgroups has taken; else one (done: None), which is copied before every replay.
+    wait: waits for the last copy out of the one set, or for the device, where it has not taken one of two for seconds."""
+    ASK_EVERY = 100000
+
+    def __init__(self, ring: torch.Tensor, done, wait):
+        self.ring, self.done, self.wait = ring, done, wait
+        self._sets = list(ring.numpy())
+        self._read = done.numpy().view(np.uint32) if done is not None else None
+        self.at = 0                  # the set that the next replay takes ...
+        self.held = 0                # ... and the one that holds what the last step left
+        self.replays = 0
+
+    def unread(self) -> int:
+        """How many replays have not yet taken their set."""
+        return max((self.replays - int(n)) & 0xFFFFFFFF for n in self._read) if self._read is not None else 0      # (32-bit counters)
+
+    def free(self) -> np.ndarray:
+        """The set that the next replay takes, once no replay before it still has to read it."""
+        if self._read is None:
+            self.wait()
+        waits = 0
+        while self.unread() > 1:
+            waits += 1
+            if waits > 100:
+                time.sleep(0 if waits < 20000 else 5e-5)
+            if waits % self.ASK_EVERY == 0:       # seconds: either the GPU has that much to do, or it says here what went wrong
+                self.wait()
+                if self.unread() > 1:
+                    raise RuntimeError("a replayed step never took its arrays")
+        return self._sets[self.at]
+
+    def carry(self) -> np.ndarray:
+        """The next replay's set, holding what the last step left."""
+        flat = self.free()
+        if self.held != self.at:
+            np.copyto(flat, self._sets[self.held])
+            self.held = self.at
+        return flat
+
+    def replayed(self) -> None:
+        """The next replay has been launched, on the set that has been filled."""
+        self.held = self.at
+        if self._read is not None:
+            self.replays = (self.replays + 1) & 0xFFFFFFFF
+            self.at ^= 1
+
+
+# Sets of graphs that were dropped while a replay had still to read them: a kernel reads them, of which the memory's allocator knows nothing, so they stay
+# until the counters say that it has. Looked through when a graph is made or dropped; no call of the runtime, because a graph may be dropped while
+# another is being captured.
+_UNREAD = deque()
+
+
+def _release_read(sets=None) -> None:
+    if sets is not None:
+        _UNREAD.append(sets)
+    for _ in range(len(_UNREAD)):
+        try:
+            kept = _UNREAD.popleft()
+        except IndexError:           # (another thread looks through them too)
+            return
+        if kept.unread():
+            _UNREAD.append(kept)
 
 
 class DecodeGraph:
@@ -51,21 +119,17 @@ class DecodeGraph:
         on_gpu = torch.device(dev).type == "cuda"
         total = max(plan.packer.total, 4)
         self.uploads = on_gpu and capture and hasattr(engine.ops, "upload_ring")
-        # Two sets of the arrays, written in turn, where the graph itself takes them from the host (upload_ring); else one, which is copied
-        # before every replay.
-        self.ring = torch.zeros(2 if self.uploads else 1, total, dtype=torch.int32, pin_memory=on_gpu)
-        self._sets = list(self.ring.numpy())
-        self._at = 0                 # the set that the next replay takes ...
-        self._held = 0               # ... and the one that holds what the last step left
+        _release_read()
+        ring = torch.zeros(2 if self.uploads else 1, total, dtype=torch.int32, pin_memory=on_gpu)
         self.dev = torch.zeros(total, dtype=torch.int32, device=dev)
-        self.copied = torch.cuda.Event() if on_gpu and not self.uploads else _NoEvent()
-        self.replays = 0
+        self.copied = torch.cuda.Event() if on_gpu and not self.uploads else _NoEvent()      # (of the one set)
         if self.uploads:
             counters = engine.ops.upload_counters(total)
             self._sent = torch.zeros(counters, dtype=torch.int32, device=dev)
-            self._done = torch.zeros(counters, dtype=torch.int32, pin_memory=True)
-            self._read = self._done.numpy().view(np.uint32)
-        self.step = materialize(plan, dev, self.ring[0], self.dev)
+            self.sets = HostSets(ring, torch.zeros(counters, dtype=torch.int32, pin_memory=True), lambda: torch.cuda.synchronize(dev))
+        else:
+            self.sets = HostSets(ring, None, self.copied.synchronize)
+        self.step = materialize(plan, dev, ring[0], self.dev)
         for st in self.step.stages:          # later steps of the shape may see more keys than this one
             st.max_kv_len = kv_capacity
         self.graph = None
@@ -115,65 +179,31 @@ class DecodeGraph:
     def _launch(self):
         engine, n = self.engine, self.step.n_wanted
         if self.uploads:
-            engine.ops.upload_ring(self.ring, self.dev, self._sent, self._done)
+            engine.ops.upload_ring(self.sets.ring, self.dev, self._sent, self.sets.done)
         outs = engine.model.forward(self.step, engine.cache)
         self.logits = engine.model.all_logits(outs, n) if self.heads else engine.logits_of(outs, self.step, n)
 
     @property
     def host(self) -> torch.Tensor:
         """The arrays as they stand for the next step."""
-        self._carry()
-        return self.ring[self._at]
-
-    def _unread(self) -> int:
-        """How many replays have not yet taken their arrays (which the GPU writes down as it does)."""
-        return max((self.replays - int(n)) & 0xFFFFFFFF for n in self._read) if self.uploads else 0      # (32-bit counters)
-
-    def _free(self) -> np.ndarray:
-        """The set that the next replay takes, once no replay before it still has to read it."""
-        if not self.uploads:
-            self.copied.synchronize()
-        else:
-            waits = 0
-            while self._unread() > 1:
-                waits += 1
-                if waits > 100:
-                    time.sleep(0 if waits < 20000 else 5e-5)
-                if waits % 100000 == 0:           # seconds: either the GPU has that much to do, or it says here what went wrong
-                    torch.cuda.synchronize(self.engine.device)
-                    if self._unread() > 1:
-                        raise RuntimeError("a replayed step never took its arrays")
-        return self._sets[self._at]
-
-    def _carry(self) -> np.ndarray:
-        """The next replay's set, holding what the last step left."""
-        flat = self._free()
-        if self._held != self._at:
-            np.copyto(flat, self._sets[self._held])
-            self._held = self._at
-        return flat
+        self.sets.carry()
+        return self.sets.ring[self.sets.at]
 
     def _replay(self):
         """The step, on the set that has been filled."""
         if not self.uploads:
-            self.dev.copy_(self.ring[0], non_blocking=True)
+            self.dev.copy_(self.sets.ring[0], non_blocking=True)
             self.copied.record()
         if self.graph is not None:
             self.graph.replay()
         else:
             self._launch()
-        self._held = self._at
-        if self.uploads:
-            self.replays += 1
-            self._at ^= 1
+        self.sets.replayed()
 
     def __del__(self):
-        # A replay that has not started yet reads the sets when it does: they stay until then. (No call of the runtime: a graph may be dropped
-        # while another is being captured.)
         try:
-            until = time.monotonic() + 10.0
-            while self._unread() and time.monotonic() < until:
-                time.sleep(0)
+            if self.sets.unread():
+                _release_read(self.sets)
         except Exception:            # not made to the end, or the interpreter is going away
             pass
 
@@ -190,7 +220,7 @@ class DecodeGraph:
         runs it (the caller cannot go on before it has the step's tokens anyway), the buffer is filled for that next
         step; when it comes, only its tokens, and the lines of requests that have taken a page since, are left to
         write before the copy and the replay."""
-        flat = self._carry()
+        flat = self.sets.carry()
         n = len(entries)
         starts = np.fromiter((e.start for e in entries), dtype=np.int64, count=n)
         tokens = np.fromiter((e.tokens[0] for e in entries), dtype=np.int32, count=n)
@@ -208,16 +238,16 @@ class DecodeGraph:
         starts, late = self._ahead
         self._ahead = None
         if late:
-            self._fill_late(self._carry(), starts, late)
+            self._fill_late(self.sets.carry(), starts, late)
         return self._run_filled(starts, tokens)
 
     def _run_filled(self, starts, tokens) -> torch.Tensor:
-        flat, n = self._carry(), len(tokens)
+        flat, n = self.sets.carry(), len(tokens)
         for st in self.stage_at:
             flat[st["tokens"]:st["tokens"] + n] = tokens
         self._replay()
         # the arrays of the step after this one, while this one runs
-        flat = self._carry()
+        flat = self.sets.carry()
         nxt = starts + 1
         if self.cache.spare_slot is not None:       # (lines that fill the step up stay where they are)
             nxt = nxt - np.fromiter((s == self.cache.spare_slot for s in self.slots), dtype=np.int64, count=len(starts))
@@ -302,7 +332,7 @@ class DecodeGraph:
     def run(self, plan: StepPlan, occupants=None) -> torch.Tensor:
         if plan.layout() != self.layout:
             raise RuntimeError("this step's arrays do not have the captured layout")
-        flat = self._free()
+        flat = self.sets.free()
         self._ahead = None
         plan.packer.fill(flat)
         self.slots = tuple(e.slot for e in plan.entries)
