@@ -542,9 +542,9 @@ __global__ __launch_bounds__(SM_THREADS) void argmax_kernel(const float* __restr
           if (at < V4 && e[k] > mv) { mv = e[k]; mi = at + k; }
       }
     }
-    for (int i = V4 + threadIdx.x; i < V; i += SM_THREADS) {
+    for (int i = V4 + threadIdx.x; i < V; i += SM_THREADS) {      // (higher than every index the thread has met; a row of -inf finds none)
       const float v = row[i];
-      if (v > mv || (v == mv && i < mi)) { mv = v; mi = i; }
+      if (v > mv) { mv = v; mi = i; }
     }
   } else {
     for (int i = threadIdx.x; i < V; i += SM_THREADS) {
