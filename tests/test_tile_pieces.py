@@ -62,11 +62,15 @@ def test_a_tile_of_no_request_is_refused():
 
 
 @pytest.mark.parametrize("total", [1, 255, 256, 257, 300, 511, 512, 513, 1000])
-def test_the_grid_takes_every_piece_once(total):
-    """What piece_of of the kernel makes of the workgroups, for two a compute unit."""
-    units = 256
-    took = [units + min(2 * units, total) - 1 - i if units <= i < 2 * units else i for i in range(total)]
+@pytest.mark.parametrize("dim,two", [(128, True), (256, False)])
+def test_the_grid_takes_every_piece_once(total, dim, two):
+    """What the kernel makes of its workgroups: two a compute unit, or one where heads are wide."""
+    units, lib = 256, hip_ops.library(f"attention_mfma@{dim}").cdll
+    took = [lib.tis_attention_mfma_piece_of(i, total, units) for i in range(total)]
     assert sorted(took) == list(range(total))
+    if not two:
+        assert took == list(range(total))
+        return
     beside = [(took[i], took[i + units]) for i in range(min(units, max(0, total - units)))]
     assert all(b == min(2 * units, total) - 1 - a for a, b in beside)        # the longest has the shortest beside it
 

@@ -30,16 +30,20 @@ int tis_attention_mfma_sink(const void* q, long q_ld, const void* plane, const i
                             int min_steps, int tile_splits, int tile_max_steps, int* row_splits, int sink,
                             const float* sinks, const float* turn, hipStream_t stream);
 
-// tis_attention_mfma_sink of a library that was built with extras: gate ([rows] at a stride of gate_ld floats, one number per
-// head and value channel, 16-byte aligned; null where none is built in) multiplies the result by its sigmoid; softcap (0 where
-// none is built in) makes a score softcap * tanh(q.k * scale / softcap).
-int tis_attention_mfma_extras(const void* q, long q_ld, const void* plane, const int* block_tables, int bt_ld,
+// tis_attention_mfma_sink of a library that may be built with extras, and with the tiles' parts as a list. gate ([rows] at a stride of gate_ld floats, one
+// number per head and value channel, 16-byte aligned; null where none is built in) multiplies the result by its sigmoid; softcap (0 where none is built
+// in) makes a score softcap * tanh(q.k * scale / softcap). pieces (null: none): n_pieces entries of four integers, 16-byte aligned, every part of every
+// tile once, those with the longest chains of steps first (see the definition); units: the device's compute units, by which the parts are dealt out.
+int tis_attention_mfma_pieces(const void* q, long q_ld, const void* plane, const int* block_tables, int bt_ld,
                               const int* row_seq, const int* positions, const int* items, int n_items, int nb,
                               const int* tiles, int n_tiles, void* out, long out_ld, float* part_o, float* part_ml, int rows,
                               int n_heads, int n_kv_heads, int head_dim, int page_size, int window, float scale, int n_splits,
                               int min_steps, int tile_splits, int tile_max_steps, int* row_splits, int sink,
                               const float* sinks, const float* turn, const float* gate, long gate_ld, float softcap,
-                              hipStream_t stream);
+                              const int* pieces, int n_pieces, int units, hipStream_t stream);
+
+// Which of `total` pieces (parts times key/value heads) workgroup `id` of the flat grid takes.
+int tis_attention_mfma_piece_of(int id, int total, int units);
 
 // A second stream (default priority, as `stream` must have) on which a call that holds both tiles and items runs its
 // tile kernel, beside the items' kernel on `stream`; the two meet again before the merge, and everything after the

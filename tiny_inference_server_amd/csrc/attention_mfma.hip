@@ -495,9 +495,10 @@ __device__ __forceinline__ float pair_sum(float v) {
 // Which piece of work a workgroup of a flat grid takes, of pieces that go from the longest chain of steps to the shortest. A compute unit holds
 // two workgroups (one where heads are wide), and workgroups go to the units in turn: those that come second on their unit take the pieces from
 // the shortest up, so that the longest has the shortest beside it. Workgroups beyond those start as others end, longest first.
-__device__ __forceinline__ int piece_of(int id, int total, int units) {
-  return WIDER <= 128 && id >= units && id < 2 * units ? units + min(2 * units, total) - 1 - id : id;
+__host__ __device__ __forceinline__ int piece_of(int id, int total, int units) {
+  return WIDER <= 128 && id >= units && id < 2 * units ? units + (2 * units < total ? 2 * units : total) - 1 - id : id;
 }
+TIS_EXPORT int tis_attention_mfma_piece_of(int id, int total, int units) { return piece_of(id, total, units); }
 
 // What bounds this kernel on a prompt of a few thousand tokens is the longest chain of steps on one compute unit. pieces: the parts of the
 // tiles that there are, longest first, (first row, rows + 256 * split, position, line of the block table), for a flat grid of pieces x
@@ -1239,28 +1240,11 @@ TIS_EXPORT int tis_attention_mfma_sink(const void* q, long q_ld, const void* pla
                           n_splits, min_steps, tile_splits, tile_max_steps, row_splits, stream, sink, sinks, (const float2*)turn);
 }
 
-// The same in a library built with extras: gate (rows at a stride of gate_ld floats, 16-byte aligned; null in a library built
-// without gates) and softcap (0 in a library built without caps): scores are softcap * tanh(q.k * scale / softcap).
-TIS_EXPORT int tis_attention_mfma_extras(const void* q, long q_ld, const void* plane, const int* block_tables, int bt_ld,
-                                         const int* row_seq, const int* positions, const int* items, int n_items, int nb,
-                                         const int* tiles, int n_tiles, void* out, long out_ld, float* part_o,
-                                         float* part_ml, int rows, int n_heads, int n_kv_heads, int head_dim, int page_size,
-                                         int window, float scale, int n_splits, int min_steps, int tile_splits,
-                                         int tile_max_steps, int* row_splits, int sink, const float* sinks,
-                                         const float* turn, const float* gate, long gate_ld, float softcap,
-                                         hipStream_t stream) {
-  if (softcap < 0.f) return tis_fail("attention_mfma: a cap of %g", (double)softcap);
-  const float log2e = 1.4426950408889634f;
-  const Extras extras{gate, gate_ld, softcap * log2e, softcap > 0.f ? 2.f * log2e * scale / softcap : 0.f};
-  return attention_launch(q, q_ld, plane, block_tables, bt_ld, row_seq, positions, items, n_items, nb, tiles, n_tiles,
-                          out, out_ld, part_o, part_ml, rows, n_heads, n_kv_heads, head_dim, page_size, window, scale,
-                          n_splits, min_steps, tile_splits, tile_max_steps, row_splits, stream, sink, sinks, (const float2*)turn,
-                          extras);
-}
-
-// The same for a caller that knows the device's compute units and has the tiles' pieces: pieces (null: none) holds n_pieces entries of four
-// integers, every part of every tile once, (first row, rows + 256 * split, position of the first row, block-table line), those with the longest
-// chains of steps first; a tile has as many parts as tile_splits and tile_max_steps say. In a library built without extras gate is null, softcap 0.
+// The same in a library that may be built with extras, for a caller that knows the device's compute units and has the tiles' pieces. gate (rows at a
+// stride of gate_ld floats, 16-byte aligned; null in a library built without gates) and softcap (0 in a library built without caps): scores are
+// softcap * tanh(q.k * scale / softcap). pieces (null: none) holds n_pieces entries of four integers, every part of every tile once, (first row, rows +
+// 256 * split, position of the first row, block-table line), those with the longest chains of steps first; a tile has as many parts as tile_splits and
+// tile_max_steps say.
 TIS_EXPORT int tis_attention_mfma_pieces(const void* q, long q_ld, const void* plane, const int* block_tables, int bt_ld,
                                          const int* row_seq, const int* positions, const int* items, int n_items, int nb,
                                          const int* tiles, int n_tiles, void* out, long out_ld, float* part_o,

@@ -108,8 +108,6 @@ _SIGNATURES["attention_mfma"] = ("tis_attention_mfma", {
                                 _I, _I, _I, _I, _P, _I, _P, _P, _P],
     "tis_attention_mfma_pieces": [_P, _L, _P, _P, _I, _P, _P, _P, _I, _I, _P, _I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F,
                                   _I, _I, _I, _I, _P, _I, _P, _P, _P, _L, _F, _P, _I, _I, _P],
-    "tis_attention_mfma_extras": [_P, _L, _P, _P, _I, _P, _P, _P, _I, _I, _P, _I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F,
-                                  _I, _I, _I, _I, _P, _I, _P, _P, _P, _L, _F, _P],
 })
 
 _SIGNATURES["stream32"] = ("tis_stream32", {
