@@ -617,14 +617,6 @@ TIS_EXPORT int tis_delta_prepare_keep(const float* proj, long ldp, int conv_off,
   return tis_launch_status("delta_prepare");
 }
 
-TIS_EXPORT int tis_delta_prepare(const float* proj, long ldp, int conv_off, int beta_off, const float* taps, int K,
-                                 const float* state, long lds, int conv_at, const int* row_seq, const int* cu_rows,
-                                 const int* seq_slots, float* out, long ldo, int rows, int H, int G, int D, int V,
-                                 hipStream_t stream) {
-  return tis_delta_prepare_keep(proj, ldp, conv_off, beta_off, taps, K, const_cast<float*>(state), lds, conv_at, row_seq, cu_rows, seq_slots, out, ldo, rows,
-                                H, G, D, V, 0, stream);
-}
-
 // The most chunks that `rows` rows can have, over all requests of DR_CHUNK_FROM rows and more (each begins one that it may not fill).
 static long dc_most(long rows) { return rows / DC + rows / DR_CHUNK_FROM + 1; }
 

@@ -161,7 +161,6 @@ _SIGNATURES["ssm_parts"] = ("tis_ssm", {
 })
 
 _SIGNATURES["delta_rule"] = ("tis_delta_rule", {
-    "tis_delta_prepare": [_P, _L, _I, _I, _P, _I, _P, _L, _I, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _P],
     "tis_delta_prepare_keep": [_P, _L, _I, _I, _P, _I, _P, _L, _I, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
     "tis_delta_scan": [_P, _L, _I, _I, _I, _I, _P, _L, _P, _L, _P, _P, _I, _I, _I, _P, _P, _L, _I, _I, _I, _I, _P],
 })
