@@ -329,6 +329,12 @@ _ATTN_WORKSPACE_FLOATS = 16 << 20
 _DELTA_WORK_FLOATS = 128 << 20   # most work space of a delta rule's walk in chunks (8 heads of 128: steps of 26,000 rows)
 
 
+def attention_plan_name(lists: str, n_heads: int, n_kv_heads: int, head_dim: int, window: int = 0):
+    """What a planned list of attention's is called in a stage's extras, by whoever plans it and by the launch that looks for it. A name holds all that the
+    lists depend on: of two mixers that plan under one name, a captured step would keep one list and be given two."""
+    return (lists, n_heads // n_kv_heads, tile_columns(head_dim), n_kv_heads, window, head_dim)
+
+
 def tile_columns(head_dim: int) -> int:
     """Columns (row, query head of a group) of one wave of the tile kernel, as the kernel source sets them."""
     return 32
@@ -774,34 +780,33 @@ class HipOps:
 
     def plan_attention(self, n_heads: int, n_kv_heads: int, head_dim: int, seq_rows, add, mode=None, window: int = 0):
         """An attention mixer's host planning, called while a step's arrays are packed: the work items of the
-        matrix-core kernels for the step's rows. Returns {name: (packed array id, host values...)}. A name holds all that the lists depend on:
-        of two mixers that plan under one name, a captured step would keep one list and be given two."""
+        matrix-core kernels for the step's rows. Returns {name: (packed array id, host values...)}, by attention_plan_name."""
         plans = {}
         if self.dtype == torch.bfloat16:
             group, cols = n_heads // n_kv_heads, tile_columns(head_dim)
             if (mode == "uneven" and group <= 64 and planned_list_pays(len(seq_rows), n_kv_heads)
                     and all(n == 1 for _, _, n in seq_rows)):
                 entries, most = decode_items(seq_rows, n_heads, n_kv_heads, head_dim, window=window, units=self.units)
-                return {("attention_decode_items", group, cols, n_kv_heads, window, head_dim): (add(entries), len(entries), most)}
+                return {attention_plan_name("attention_decode_items", n_heads, n_kv_heads, head_dim, window): (add(entries), len(entries), most)}
             nb, items, tiles, steps = attention_items(seq_rows, group, cols, n_kv_heads)
             beside = planned_beside_tiles(seq_rows, items, tiles, steps, n_heads, n_kv_heads, head_dim, window, self.units)
             if beside is not None:
                 # one array: the planned entries of four integers, then the tiles' lines of two
                 entries, most = beside
-                plans[("attention_items", group, cols, n_kv_heads, window, head_dim)] = (
+                plans[attention_plan_name("attention_items", n_heads, n_kv_heads, head_dim, window)] = (
                     add(np.concatenate((entries.reshape(-1), tiles.reshape(-1)))), len(entries), 1, len(tiles), steps, most)
             elif nb <= 4 and (len(items) or len(tiles)):
                 # one array: the items' lines, then the tiles'
                 # (a mixer with a window plans for itself: its lists are the same, its keys are its own)
-                plans[("attention_items", group, cols, n_kv_heads, window, head_dim)] = (add(np.concatenate((items, tiles))), len(items), nb, len(tiles),
+                plans[attention_plan_name("attention_items", n_heads, n_kv_heads, head_dim, window)] = (add(np.concatenate((items, tiles))), len(items), nb, len(tiles),
                                                                                          steps, 0)
-            if len(tiles) and ("attention_items", group, cols, n_kv_heads, window, head_dim) in plans:
+            if len(tiles) and attention_plan_name("attention_items", n_heads, n_kv_heads, head_dim, window) in plans:
                 lp = attention_launch_plan(sum(n for _, _, n in seq_rows), len(items) if beside is None else len(entries), len(tiles), steps, False,
                                            max(p0 + n for _, p0, n in seq_rows), n_heads, n_kv_heads, head_dim,
                                            planned_splits=0 if beside is None else most, units=self.units)
                 if lp.tile_splits > 1:
                     pieces = tile_pieces(seq_rows, tiles, lp.tile_splits, lp.tile_max_steps, window)
-                    plans[("attention_tile_pieces", group, cols, n_kv_heads, window, head_dim)] = (add(pieces), len(pieces), lp.tile_splits, lp.tile_max_steps)
+                    plans[attention_plan_name("attention_tile_pieces", n_heads, n_kv_heads, head_dim, window)] = (add(pieces), len(pieces), lp.tile_splits, lp.tile_max_steps)
         return plans
 
     # ---- helpers -------------------------------------------------------------------------------------
@@ -1347,8 +1352,8 @@ class HipOps:
         n, group = q.shape[0], n_heads // n_kv_heads
         size = max(key_dim, value_dim)          # what a mixer's planner goes by
         cols = tile_columns(size)
-        planned = batch.extras.get(("attention_decode_items", group, cols, n_kv_heads, int(window), size))
-        plan = batch.extras.get(("attention_items", group, cols, n_kv_heads, int(window), size))
+        planned = batch.extras.get(attention_plan_name("attention_decode_items", n_heads, n_kv_heads, size, int(window)))
+        plan = batch.extras.get(attention_plan_name("attention_items", n_heads, n_kv_heads, size, int(window)))
         if planned is None and plan is None:
             # a caller that did not plan (a kernel test): plan now, tiles wherever they fit
             if uneven_lengths(batch.seq_rows, int(window)) and planned_list_pays(n, n_kv_heads):
@@ -1419,7 +1424,7 @@ class HipOps:
             raise KernelError("attention: the work list must be contiguous 32-bit integers")
         pieces, n_pieces = None, 0
         if tile_splits > 1:
-            made = batch.extras.get(("attention_tile_pieces", group, cols, n_kv_heads, int(window), size))
+            made = batch.extras.get(attention_plan_name("attention_tile_pieces", n_heads, n_kv_heads, size, int(window)))
             if made is not None and made[2:] == (tile_splits, tile_max_steps):      # (planned for these very cuts)
                 pieces, n_pieces = made[0].reshape(-1), made[1]
                 if pieces.dtype != torch.int32 or not pieces.is_contiguous() or pieces.numel() != 4 * n_pieces:

@@ -52,7 +52,7 @@ def parse_segments(text: str):
 
 
 def attention_case(ops, a):
-    from .hip_ops import attention_items, decode_items, planned_list_pays, tile_columns, uneven_lengths
+    from .hip_ops import attention_items, attention_plan_name, decode_items, planned_list_pays, tile_columns, uneven_lengths
     nh, kvh, hd, ps = a.heads, a.kv_heads, a.head_dim, a.page_size
     segs = parse_segments(a.segments)
     pages = [-(-(p0 + n) // ps) for p0, n in segs]
@@ -76,7 +76,7 @@ def attention_case(ops, a):
     if ((uneven_lengths(seq_rows) and planned_list_pays(len(seq_rows), kvh)) or a.planned) and not a.same_splits:
         # decoded tokens of requests that differ widely in length: splits planned request by request, as the engine does
         entries, most = decode_items(seq_rows, nh, kvh, hd)
-        batch.extras[("attention_decode_items", nh // kvh, tile_columns(hd), kvh, 0)] = (
+        batch.extras[attention_plan_name("attention_decode_items", nh, kvh, hd)] = (
             torch.from_numpy(entries).reshape(-1).to(ops.device), len(entries), most)
     else:
         from .hip_ops import planned_beside_tiles
@@ -89,7 +89,7 @@ def attention_case(ops, a):
         else:
             both = torch.from_numpy(np.ascontiguousarray(np.concatenate((items, tiles)))).reshape(-1).to(ops.device)
             plan = (both, len(items), nb, len(tiles), steps, 0)
-        batch.extras[("attention_items", nh // kvh, tile_columns(hd), kvh, 0)] = plan
+        batch.extras[attention_plan_name("attention_items", nh, kvh, hd)] = plan
     us = graph_time(lambda: ops.paged_attention(q, plane, batch, "g", nh, kvh, hd), a.reps)
     kv_bytes = sum(p0 + n for p0, n in segs) * kvh * hd * 2 * 2
     flops = sum(4 * nh * hd * (n * p0 + n * (n + 1) / 2) for p0, n in segs)
