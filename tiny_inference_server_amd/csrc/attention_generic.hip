@@ -12,8 +12,9 @@
 // the row's own length only, not on what else is in the batch.
 //
 // What bounds it is the chain of trips to memory and through LDS of one small workgroup: the row's position and request, the block table, a
-// key's channels and the values, which are asked for together (rows of up to 50 keys, 8 heads of 8, 32-bit, us: one channel and one value after
-// the other 6.1, AG_AHEAD pieces of 16 bytes of a key and AG_AHEAD values of a thread at a time 5.1). The sums keep their order.
+// key's channels and the values, which are asked for together (rows of up to 50 keys, 8 heads of 8, 32-bit, traced in replayed steps,
+// us: one channel and one value after the other 5.7, AG_AHEAD pieces of 16 bytes of a key and AG_AHEAD values of a thread at a time 5.0). The sums keep their
+// order.
 #include <algorithm>
 #include <utility>
 #include <vector>
@@ -166,6 +167,7 @@ TIS_EXPORT int tis_attention_generic(int dtype, const void* q, long q_ld, const 
 
 // ---- host planning -----------------------------------------------------------------------------------------
 //
+// (Here, because every engine loads this library once; the tile kernel's source is built once a head size.)
 // The parts that the tile kernel of attention_mfma.hip cuts its tiles into, those with the longest chains of steps first (those alike in the order
 // of their tiles): (first row, rows + 256 * split, position of the first row, block-table line) each, into out [capacity][4]. rows: (first row, first
 // position, rows) of each request; tiles: (first row, rows) each. The counts are the kernel's own: a tile of n steps of 32 keys, from a multiple of 32

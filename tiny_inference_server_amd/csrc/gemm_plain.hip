@@ -146,7 +146,7 @@ __global__ __launch_bounds__(GS_BM * GS_BN) void gemm_plain_few_kernel(const TI*
   if constexpr (NORM) {
     const int lane = t % TIS_WAVE, wave = t / TIS_WAVE;
     // NV: of the four waves that would share a row, those that have values (64 a turn); the others' sums are zeros. A wave's four rows are asked
-    // for at once, from addresses that always hold something (3 rows of 64 against 192 or 352 columns, us: 6.6 row after row, 16 sums a wave; 4.6 so).
+    // for at once, from addresses that always hold something (3 rows of 64 against 192 or 352 columns, traced in replayed steps, us: 6.6 row after row, 16 sums a wave; 4.5 so).
     auto squares = [&](auto nv) {
       constexpr int NV = nv;
       float ss[4][NV];

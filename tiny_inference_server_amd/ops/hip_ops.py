@@ -267,7 +267,10 @@ def tiles_pay(M: int, N: int, K: int, gate: bool, tile: int, share: float) -> bo
     if M > _tiles_up_to(N, K):
         # a matrix of many inner columns, where tiles are one a unit and fill the chip (see gemm_tiles.hip). us, library / tiles: 1,536 x 4,096 at 1,190, 1,340, 1,480, 1,926
         # 29 / 25, 34 / 30, 34 / 31, 35 / 32; 1,536 x 3,072 at 1,411 28 / 23; 2,048 x 5,632 at 1,031, 1,190, 1,580, 1,850 46 / 39, 46 / 40, 53 / 47, 54 / 50. Where the library's
-        # own tiles fill the chip it stays: 1,536 x 4,096 at 1,113, 1,650, 1,792 28 / 32, 32 / 34, 31 / 34, 2,048 x 5,632 at 1,408, 1,532 44 / 48.
+        # own tiles fill the chip it stays: 1,536 x 4,096 at 1,113, 1,650, 1,792 28 / 32, 32 / 34, 31 / 34, 2,048 x 5,632 at 1,408, 1,532 44 / 48. Tiles of 96 are left out from
+        # 1,281 to 1,792 rows where they are four fifths of the chip and more, because the library's product is the faster one at 1,536 and 1,792 (2,048 x 5,632 43 / 48, 2,048 x 4,096
+        # 32 / 35, 1,536 x 4,096 and x 3,072 at 1,792 31 / 34 and 24.5 / 26.6): measured, not derived from its tiles. Of the listed widths four come here (1,536 and 2,048 columns of
+        # 3,072, 4,096 and 5,632 inner ones); at 26 numbers of rows of each, from 1,025 to 2,048, with a residual, none that goes to the tiles takes more than 1.02 of the library's time.
         if gate or M > 2048 or N > _TILES_NARROW[1] or share > 1:
             return False
         if tile in _TILES_OF_96:
@@ -315,7 +318,10 @@ _ATTN_TILE_STEP_US = (0.72, 1.3)   # what a tile's step of 32 keys takes while a
 _ATTN_TILE_MERGE_US = (10.0, 4.0, 6e6)   # what cutting tiles into key splits costs beyond the tiles' own time: the
                                 # merge's launch and the per-row counts (less where the items' splits are merged anyway),
                                 # and microseconds per byte of 32-bit partial results. Tiles are cut only where, by
-                                # these figures, the shorter chains save more than that. 12 heads of 128 over 3, us,
+                                # these figures, the shorter chains save more than that. They are of a merge by four waves a
+                                # head; a wave a head takes half of it (see MERGE_ROWS_FROM in attention_mfma.hip), so some
+                                # prompts that would be faster cut stay whole: cutting them changes the rounding of their
+                                # results, which is kept. Of that time, 12 heads of 128 over 3, us,
                                 # cut / uncut / one-wave kernel: 4 prompts of 512 tokens 28.8 / 18.8 / 22.8, 8 of 512
                                 # 40.8 / 25.4 / 33.2, 4 of 1,024 50.6 / 39.5 / 57.2, one of 1,024 29.2 / 28.6 / 29.2; but
                                 # one of 1,536 35.3 / 39.9 / 47.7, of 2,048 42.4 / 51.3 / 69.5, 512 tokens behind 3,000
