@@ -67,6 +67,8 @@ class HostSets:
 
     def carry(self) -> np.ndarray:
         """The next replay's set, holding what the last step left."""
+        if self.held == self.at and self._read is not None:
+            return self._sets[self.at]            # (of two sets: free since the call that carried it over, or never launched)
         flat = self.free()
         if self.held != self.at:
             np.copyto(flat, self._sets[self.held])
