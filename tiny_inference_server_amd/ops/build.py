@@ -50,6 +50,7 @@ SOURCES: Dict[str, str] = {
     "attention_mixed": "attention_mixed.hip",
     "hyper_streams": "hyper_streams.hip",
     "convolved_attention": "convolved_attention.hip",
+    "small_block": "small_block.hip",
 }
 HEADERS = ["common.h", "attention_mfma.h", "tile_loop.h"]
 # what a library links beyond the HIP runtime

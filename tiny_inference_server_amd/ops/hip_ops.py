@@ -169,6 +169,9 @@ _SIGNATURES["attention_mixed"] = ("tis_attention_mixed", {
     "tis_attention_mixed_mfma": [_P, _L, _P, _P, _I, _P, _P, _P, _I, _P, _L, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P, _P, _P],
 })
 
+_SIGNATURES["small_block"] = ("tis_small_block", {
+    "tis_small_block": [_P, _L, _P, _L, _P, _F, _P, _P, _P, _F, _P, _P, _P, _I, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P],
+})
 _SIGNATURES["hyper_streams"] = ("tis_hyper_streams", {
     "tis_mix_streams": [_I, _P, _L, _L, _P, _L, _P, _P, _P, _P, _P, _P, _F, _P, _L, _P, _P, _L, _P, _P, _P, _I, _I, _I, _I, _P],
 })
@@ -751,13 +754,14 @@ class HipOps:
         self.code = _DT[dtype]
         # whatever is not built yet is compiled side by side, not one after the other
         _build.build(["rowwise", "rope_cache", "attention_generic", "gemm_plain", "sampling"] +
-                     (["gemm_skinny", "gemm_library", "gemm_tiles"] if dtype == torch.bfloat16 else []))
+                     (["gemm_skinny", "gemm_library", "gemm_tiles"] if dtype == torch.bfloat16 else ["small_block"]))
         self.rowwise = library("rowwise")
         self.rope = library("rope_cache")
         self.attn_generic = library("attention_generic")
         self.gemm_plain = library("gemm_plain")
         self.sampling = library("sampling")
         self.gemm_skinny = library("gemm_skinny") if dtype == torch.bfloat16 else None
+        self.small = library("small_block") if dtype == torch.float32 else None
         self.gemm_library = None
         self.few_rows = _FEW_ROWS
         self.library_widths = library_widths()
@@ -1350,6 +1354,36 @@ class HipOps:
             self.code, _ptr(q), q.stride(0), _ptr(plane), _ptr(tables), tables.stride(0), _ptr(batch.row_seq),
             _ptr(batch.positions), _ptr(out), out.stride(0), n, n_heads, n_kv_heads, head_dim, page_size, int(window),
             float(scale), _ptr(slopes), self._stream())
+        return out
+
+    def small_block(self, x, batch, group, plane, norms, attention, feed_forward):
+        """A pre-norm block (norm, attention, norm, gated feed-forward) in one kernel: what qkv_rope, paged_attention, linear and linear_swiglu give in
+        turn, up to the order of 32-bit sums. norms: (gain, eps) of both; attention: w_qkv, w_o as qkv_rope and linear take them, rotary table, interleaved, heads, kv heads,
+        head size, window, scale; feed_forward: w_gate_up, w_down. None, with nothing done: not a 32-bit block small enough for one compute unit, a step
+        that brings a request several rows, or operands that do not start on 16 bytes."""
+        if self.small is None or batch.max_seq_rows > 1 or not batch.n_rows:
+            return None
+        w_qkv, w_o, table, interleaved, H, G, HD, window, scale = attention
+        w_gu, w_down = feed_forward
+        (gain_a, eps_a), (gain_f, eps_f) = norms
+        M, D = _rows_view(self._check(x, "block x"), "block x").shape
+        F, tables, page_size = w_down.shape[1], batch.block_tables[group], plane.shape[3]
+        shapes = ((w_qkv, ((H + 2 * G) * HD, D)), (w_o, (D, H * HD)), (w_gu, (2 * F, D)), (w_down, (D, F)), (gain_a, (D,)), (gain_f, (D,)))
+        if any(tuple(t.shape) != shape or t.dtype != torch.float32 or not t.is_contiguous() for t, shape in shapes):
+            return None
+        keys = int(batch.max_kv_len) if table is None else min(int(batch.max_kv_len), table.shape[0])      # (no position is beyond the table)
+        if window < 0 or not self.small.cdll.tis_small_block_takes(M, D, F, H, G, HD, keys, page_size) or any(t.data_ptr() % 16 for t in (w_qkv, w_o, w_gu, w_down, plane)):
+            return None
+        self._check_rotary(M, batch.positions, batch.write_slots[group], table, plane, G, HD, page_size, True)
+        self._index(batch.row_seq, "row_seq", M)
+        self._check(tables, "block tables", torch.int32)
+        if tables.dim() != 2 or tables.stride(1) != 1 or batch.max_kv_len > tables.shape[1] * page_size:
+            raise KernelError(f"small_block: a row sees {batch.max_kv_len} keys, block tables {tuple(tables.shape)} of pages of {page_size}")
+        out = self.empty(M, D)
+        self.small.tis_small_block(
+            _ptr(x), x.stride(0), _ptr(out), out.stride(0), _ptr(gain_a), float(eps_a), _ptr(w_qkv), _ptr(w_o), _ptr(gain_f), float(eps_f), _ptr(w_gu),
+            _ptr(w_down), _ptr(table), int(bool(interleaved)), _ptr(batch.positions), _ptr(batch.row_seq), _ptr(batch.write_slots[group]), _ptr(tables),
+            tables.stride(0), _ptr(plane), M, D, F, H, G, HD, page_size, int(window), float(scale), keys, self._stream())
         return out
 
     def _attention_on_matrix_cores(self, q, plane, batch, tables, out, n_heads, n_kv_heads, key_dim, value_dim, page_size, window,

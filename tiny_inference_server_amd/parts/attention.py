@@ -62,6 +62,12 @@ class GqaAttention:
 
     fuses_norm = True
 
+    def whole_block(self, ctx):
+        """What an operations object's kernel for whole small blocks takes of this mixer (HipOps.small_block); None where it is more than that."""
+        if self.slopes is not None or not ctx.writes_cache:
+            return None
+        return (self.w_qkv, self.w_o, *self.position.rotary(), self.n_heads, self.n_kv_heads, self.head_dim, self.window, self.scale)
+
     # work lists for the attention kernels are made on the host, once per step and attention shape
     def plan_key(self):
         if not hasattr(self.ops, "plan_attention"):

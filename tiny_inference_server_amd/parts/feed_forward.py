@@ -35,6 +35,9 @@ class SwiGlu:
 
     fuses_norm = True
 
+    def whole_block(self):
+        return self.w_gate_up, self.w_down
+
     def forward(self, x, residual=None, norm=None, residual_is_spent=False):
         ops = self.ops
         if norm is not None and not hasattr(norm, "as_rms"):
