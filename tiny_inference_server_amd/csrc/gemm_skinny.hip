@@ -60,6 +60,23 @@ struct RopeArgs {
   int n_heads, n_kv_heads, head_dim, page_size, interleaved, write_cache;
 };
 
+// The residual's four columns from n_out on of a row, as they are stored and without a wait: addresses past an end are moved inside instead of branched
+// around, and a value is converted where it is added (a branch a value with its conversion inside was four trips to memory, one after the other, before the finishing
+// wave's first product).
+struct ResidualFour {
+  uint16_t bits[4];
+  __device__ __forceinline__ void ask(const bf16* R_in, long r_ld, int m, int n_out, int M, int N) {
+    const uint16_t* row = reinterpret_cast<const uint16_t*>(R_in) + (long)min(m, M - 1) * r_ld;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bits[i] = row[min(n_out + i, N - 1)];
+  }
+  __device__ __forceinline__ float value(int i) const {
+    unsigned v = bits[i];
+    asm volatile("" : "+v"(v));                    // (or the compiler converts, and waits, where the value is loaded)
+    return __uint_as_float(v << 16);
+  }
+};
+
 // GS_WAVES: waves per workgroup; U: steps of K whose loads a wave issues together before the first product.
 // Eight waves of three or four steps measured best on MI355X for K of 1536 to 4096 (5.6 us for a 25 MB matrix,
 // 23 us for the 147 MB output table: 80 % of the HBM peak); four waves where K is too short to feed eight. Batches
@@ -125,27 +142,20 @@ __global__ __launch_bounds__(GS_WAVES * 64) void gemm_skinny_kernel(
     ss[mb] = 0.f;
   }
 
-  // What the epilogue wants from memory (the residual; the row's position, rotary factors and cache slot) is asked
-  // for here, by the lanes that will use it, so that its round trips run beside the weights' and not after them.
+  // What the epilogue wants from memory (the row's position, rotary factors and cache slot here, the residual behind the first operands) is asked
+  // for by the lanes that will use it, so that its round trips run beside the weights' and not after them.
   // Result lane (g, c16) of wave 0: columns n_out .. n_out + 3 of the rows mb * 16 + c16.
   const bool out_lane = wave == 0 && g < GH && c16 < COLS;
   const int n_out = n0 + g * 4;
-  float res[MB][4];
+  ResidualFour res[MB];
   float2 cs[MB][2];
   int slot[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     const int m = mb * 16 + c16;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) res[mb][i] = 0.f;
     cs[mb][0] = cs[mb][1] = make_float2(1.f, 0.f);
     slot[mb] = 0;
     if (!out_lane || m >= M) continue;
-    if (EPI == EPI_RESIDUAL) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (n_out + i < N) res[mb][i] = static_cast<float>(R_in[(long)m * r_ld + n_out + i]);
-    }
     if (EPI == EPI_ROPE && n_out < N) {
       const int hd = rope.head_dim;
       const int head = n_out / hd, e0 = n_out % hd;
@@ -159,7 +169,9 @@ __global__ __launch_bounds__(GS_WAVES * 64) void gemm_skinny_kernel(
   }
 
   // U steps at a time: all their loads are issued before the first product, so that a wave keeps several
-  // rows' worth of HBM requests in flight
+  // rows' worth of HBM requests in flight; the activations first, which come from L2 (behind the weights they would wait for those), the residual last.
+  // us in a chain of such products from cold memory, operands step by step behind a residual that is waited for / so: 1,536 x 1,536 at 1, 3, 8 rows 4.6 / 4.0, 4.8 / 4.2, 5.2 / 4.5;
+  // 1,536 x 4,096 6.4 / 5.6, 6.8 / 5.9, 6.9 / 6.4; 2,048 x 5,632 8.2 / 7.1, 8.4 / 7.4, 9.1 / 8.3; 1,024 x 2,816 6.1 / 5.0, 6.2 / 5.1, 6.7 / 5.6.
   for (int s0 = wave; s0 < steps; s0 += U * GS_WAVES) {
     bf16x8 a[U][CT];
     bf16x8 b[U][MB];
@@ -169,11 +181,6 @@ __global__ __launch_bounds__(GS_WAVES * 64) void gemm_skinny_kernel(
       const int s = s0 + u * GS_WAVES;
       const int k = s * (32 * R) + chunk * 32 + g * 8;
       const bool k_ok = s < steps && k < K;   // K is a multiple of 8, so a lane's 8 values are all inside or all outside
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        a[u][ct] = (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
-        if (w_ok[ct] && k_ok) a[u][ct] = *reinterpret_cast<const bf16x8*>(wrow[ct] + (long)s * (32 * R));
-      }
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
         b[u][mb] = (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
@@ -185,6 +192,20 @@ __global__ __launch_bounds__(GS_WAVES * 64) void gemm_skinny_kernel(
         gv[u][0] = g0.x; gv[u][1] = g0.y; gv[u][2] = g0.z; gv[u][3] = g0.w;
         gv[u][4] = g1.x; gv[u][5] = g1.y; gv[u][6] = g1.z; gv[u][7] = g1.w;
       }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = s0 + u * GS_WAVES;
+      const bool k_ok = s < steps && s * (32 * R) + chunk * 32 + g * 8 < K;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        a[u][ct] = (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
+        if (w_ok[ct] && k_ok) a[u][ct] = *reinterpret_cast<const bf16x8*>(wrow[ct] + (long)s * (32 * R));
+      }
+    }
+    if (EPI == EPI_RESIDUAL && s0 == 0 && out_lane) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) res[mb].ask(R_in, r_ld, mb * 16 + c16, n_out, M, N);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -303,7 +324,7 @@ __global__ __launch_bounds__(GS_WAVES * 64) void gemm_skinny_kernel(
       for (int i = 0; i < 4; ++i) {
         if (n + i < N) {
           float t = v[i];
-          if (EPI == EPI_RESIDUAL) t += res[mb][i];
+          if (EPI == EPI_RESIDUAL) t += res[mb].value(i);
           C[(long)m * c_ld + n + i] = from_f<TO>(activated<EPI>(t));
         }
       }
@@ -402,23 +423,17 @@ __global__ __launch_bounds__(512) void gemm_staged_kernel(
   // What the epilogue wants from memory, asked for before the main loop by the lanes that will use it. Tile t of the
   // MB x CT tiles is finished by wave t % 8; a result lane (g, c16) holds columns n_out .. n_out + 3 of row m_out.
   constexpr int TILES = MB * CT, TPW = (TILES + WAVES - 1) / WAVES;
-  float res[TPW][4];
+  ResidualFour res[TPW];
   float2 cs[TPW][2];
   int slot[TPW];
 #pragma unroll
   for (int j = 0; j < TPW; ++j) {
     const int t = j * WAVES + wave, mb = t / CT, ct = t % CT;
     const int m = mb * 16 + c16, n_out = n0 + ct * 16 + g * 4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) res[j][i] = 0.f;
     cs[j][0] = cs[j][1] = make_float2(1.f, 0.f);
     slot[j] = 0;
+    if (EPI == EPI_RESIDUAL && t < TILES) res[j].ask(R_in, r_ld, m, n_out, M, N);
     if (t >= TILES || m >= M) continue;
-    if (EPI == EPI_RESIDUAL) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (n_out + i < N) res[j][i] = static_cast<float>(R_in[(long)m * r_ld + n_out + i]);
-    }
     if (EPI == EPI_ROPE && n_out < N) {
       const int hd = rope.head_dim;
       const int head = n_out / hd, e0 = n_out % hd;
@@ -584,7 +599,7 @@ __global__ __launch_bounds__(512) void gemm_staged_kernel(
       for (int i = 0; i < 4; ++i) {
         if (n + i < N) {
           float s = v[i];
-          if (EPI == EPI_RESIDUAL) s += res[j][i];
+          if (EPI == EPI_RESIDUAL) s += res[j].value(i);
           C[(long)m * c_ld + n + i] = from_f<TO>(activated<EPI>(s));
         }
       }
