@@ -6,6 +6,7 @@
 //
 // tile_loop.h holds the loop. A row's sums run over K in the same order whatever M is and whichever tile is taken: its result does not depend on the other rows.
 #include <climits>
+#include <type_traits>
 
 #include "tile_loop.h"
 
@@ -59,7 +60,7 @@ __device__ __forceinline__ void tile_sums(unsigned char* lds, const bf16* X, lon
 template <int BM, int BN, int WM, int WN, int NSTAGE, int AHEAD, bool RESIDUAL, typename TO, int ACT = 0>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
     const bf16* __restrict__ X, long x_ld, const bf16* __restrict__ W, const bf16* R, long r_ld, TO* C, long c_ld,
-    int M, int N, int K, float limit) {
+    int M, int N, int K, float limit, int wide) {
   typedef TileLoop<BM, BN, WM, WN, NSTAGE, AHEAD> Loop;
   constexpr int TM = Loop::TM, TN = Loop::TN;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[NSTAGE * Loop::STAGE];
@@ -67,10 +68,78 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
   const int wm = wave / WN, wn = wave % WN;
   const GtTile tile = gt_tile(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN);
   const long m0 = (long)tile.m * BM, n0 = (long)tile.n * BN;
+  // The residual's four of every eight columns, asked for before the first step where they find room: behind the last one they would be a trip to memory
+  // that nothing hides. (R may be C: a workgroup reads its own results' places before it writes them.)
+  constexpr bool EARLY = RESIDUAL && TM * TN <= 4;
+  bf16x4 res[EARLY ? TM : 1][EARLY ? TN : 1][4];
+  if constexpr (EARLY)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          res[i][j][q] = *(const bf16x4*)(R + min(m0 + wm * (BM / WM) + i * 32 + r32, (long)M - 1) * r_ld + min(n0 + wn * (BN / WN) + j * 32 + q * 8 + h * 4, (long)N - 4));
   f32x16 acc[TM][TN];
   tile_sums<Loop, BM>(lds, X, x_ld, W, m0, n0, M, N, K, acc);
 
-  // accumulator 4 q + e of block (i, j): row m0 + wm * (BM / WM) + i * 32 + r32, column n0 + wn * (BN / WN) + j * 32 + 8 q + 4 h + e
+  // Accumulator 4 q + e of block (i, j): row m0 + wm * (BM / WM) + i * 32 + r32, column n0 + wn * (BN / WN) + j * 32 + 8 q + 4 h + e. A lane's four columns are
+  // 4 (gated), 8 or 16 bytes of a row; stored as they are, an instruction reaches 32 rows with 8 to 32 bytes each. Where the result's rows lie on 16 bytes
+  // they pass through LDS, 32 rows of the wave at a time, and leave 16 bytes a lane, a row's side by side. us, stored as they are with a late residual / so, matrices from
+  // memory: 2,048 rows of 1,536 x 1,536 with a residual 16.6 / 14.7, of 1,536 x 4,096 34.8 / 33.6, of 2,304 x 1,536 21.8 / 19.7; 3,000 of 2,816 x 1,024 28.3 / 24.6; 32-bit
+  // results 1,800 of 32,000 x 2,048 252 / 242, 2,048 of 3,072 x 2,048 32.4 / 30.3; gated 600 of 8,192 x 1,536 23.8 / 22.6. At 30 sizes none slower by more than 0.5 %.
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  using Four = std::conditional_t<(ACT >= 3), bf16x2, std::conditional_t<sizeof(TO) == 4, f32x4, bf16x4>>;
+  auto four = [&](int i, int j, int q, long m, long n) {
+    Four o;
+    if constexpr (ACT >= 3) {
+      o = (bf16x2){static_cast<__bf16>(gt_gated<ACT>(acc[i][j][q * 4], acc[i][j][q * 4 + 1], limit)),
+                   static_cast<__bf16>(gt_gated<ACT>(acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3], limit))};
+    } else {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = gt_activated<ACT>(acc[i][j][q * 4 + e]);
+      if constexpr (RESIDUAL) {
+        bf16x4 r;
+        if constexpr (EARLY) r = res[i][j][q];
+        else r = *(const bf16x4*)(R + min(m, (long)M - 1) * r_ld + min(n, (long)N - 4));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += (float)r[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (sizeof(TO) == 4) o[e] = v[e];       // the 32-bit sums as they are
+        else o[e] = static_cast<__bf16>(v[e]);
+      }
+    }
+    return o;
+  };
+  constexpr int ROW = TN * 8 * sizeof(Four), PITCH = ROW + 16, PIECES = ROW / 16, COLUMNS = 64 / sizeof(Four);      // bytes of a wave's row, 16-byte pieces, W's rows a piece
+  const long out_n0 = n0 + wn * (BN / WN);
+  const int per = ACT >= 3 ? 2 : 1;
+  if (wide) {
+    static_assert(32 * PITCH * WM * WN <= NSTAGE * Loop::STAGE, "the waves' rows in the operands' place");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");      // every wave has its last operands
+    unsigned char* mine = lds + wave * 32 * PITCH;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const long row0 = m0 + wm * (BM / WM) + i * 32;
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *(Four*)(mine + r32 * PITCH + ((j * 4 + q) * 2 + h) * sizeof(Four)) = four(i, j, q, row0 + r32, out_n0 + j * 32 + q * 8 + h * 4);
+      asm volatile("" : : : "memory");
+#pragma unroll
+      for (int k = 0; k < PIECES / 2; ++k) {
+        const int p = k * 64 + lane, row = p / PIECES, at = p % PIECES;
+        const f32x4 v = *(const f32x4*)(mine + row * PITCH + at * 16);
+        if (row0 + row < M && out_n0 + at * COLUMNS < N) *(f32x4*)(C + (row0 + row) * c_ld + (out_n0 + at * COLUMNS) / per) = v;
+      }
+      asm volatile("" : : : "memory");
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const long m = m0 + wm * (BM / WM) + i * 32 + r32;
@@ -79,30 +148,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const long n = n0 + wn * (BN / WN) + j * 32 + q * 8 + h * 4;
-        if (n >= N) continue;                 // (N is a multiple of 4: the four columns are inside or outside together)
-        if constexpr (ACT >= 3) {
-          typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-          *(bf16x2*)(C + m * c_ld + n / 2) = (bf16x2){static_cast<__bf16>(gt_gated<ACT>(acc[i][j][q * 4], acc[i][j][q * 4 + 1], limit)),
-                                                      static_cast<__bf16>(gt_gated<ACT>(acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3], limit))};
-          continue;
-        }
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = gt_activated<ACT>(acc[i][j][q * 4 + e]);
-        if (RESIDUAL) {
-          const bf16x4 r = *(const bf16x4*)(R + m * r_ld + n);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += (float)r[e];
-        }
-        if constexpr (sizeof(TO) == 4) {
-          *(f32x4*)(C + m * c_ld + n) = (f32x4){v[0], v[1], v[2], v[3]};       // the 32-bit sums as they are
-        } else {
-          bf16x4 o;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = static_cast<__bf16>(v[e]);
-          *(bf16x4*)(C + m * c_ld + n) = o;
-        }
+        const long n = out_n0 + j * 32 + q * 8 + h * 4;
+        if (n < N) *(Four*)(C + m * c_ld + n / per) = four(i, j, q, m, n);        // (N is a multiple of 4: the four columns are inside or outside together)
       }
   }
 }
@@ -314,9 +361,12 @@ TIS_EXPORT int tis_gemm_tiles(const void* X, long x_ld, const void* W, const voi
   const int pick = tis_gemm_tiles_pick(M, N, K);
   const long tiles = tiles_of(pick, M, N);
   if (tiles >= (1L << 31)) return tis_fail("gemm_tiles: %ld tiles are more than a grid holds", tiles);
+  // whether the result's rows are whole pieces of 16 bytes
+  const int piece = out_f32 ? 4 : 8;
+  const bool wide = (uintptr_t)C % 16 == 0 && c_ld % piece == 0 && N % (act >= 3 ? 16 : piece) == 0;
 #define LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, RV, TOV, ACTV)                                                               \
   gemm_tiles_kernel<BMV, BNV, WMV, WNV, NSV, AHV, RV, TOV, ACTV><<<dim3((unsigned)tiles), WMV * WNV * 64, 0, stream>>>(   \
-      (const bf16*)X, x_ld, (const bf16*)W, (const bf16*)R, r_ld, (TOV*)C, c_ld, M, N, K, limit)
+      (const bf16*)X, x_ld, (const bf16*)W, (const bf16*)R, r_ld, (TOV*)C, c_ld, M, N, K, limit, wide)
 #define PICK(BMV, BNV, WMV, WNV, NSV, AHV)                                     \
   {                                                                             \
     if (out_f32) LAUNCH(BMV, BNV, WMV, WNV, NSV, AHV, false, float, 0);       \
