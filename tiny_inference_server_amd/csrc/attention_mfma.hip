@@ -235,6 +235,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NB <= 2 ? 2 
       pg[t] = ok ? got : -1;
     }
   };
+  // (of the first two steps: all four under way at once; loaded where each is used they were four trips, see the merge's figures)
+  auto first_page_ids = [&](int (&pa)[2], int (&pn)[2]) {
+    int got[4];
+    bool ok[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int key0 = k_lo + s_begin * 32 + t * 16;
+      ok[t] = s_begin + t / 2 < s_end && key0 < k_hi;
+      got[t] = bt[ok[t] ? (PS16 ? key0 >> 4 : key0 / page_size) : 0];
+    }
+    asm volatile("" : "+s"(got[0]), "+s"(got[1]), "+s"(got[2]), "+s"(got[3]));
+#pragma unroll
+    for (int t = 0; t < 4; ++t) (t < 2 ? pa : pn)[t % 2] = ok[t] ? got[t] : -1;
+  };
   auto load_tiles = [&](int s, const int (&pg)[2], Tiles& T) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -383,8 +397,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NB <= 2 ? 2 
   } else if (s_begin < s_end) {
     Tiles ta, tb;
     int pa[2], pn[2], pq[2];
-    page_ids(s_begin, pa);
-    page_ids(s_begin + 1, pn);
+    first_page_ids(pa, pn);
     load_tiles(s_begin, pa, ta);
     for (int s = s_begin; s < s_end; s += 2) {
       // pn holds the page ids of step s+1; loads past the end are harmless and never consumed
@@ -849,7 +862,10 @@ __global__ __launch_bounds__(TW * 64) __attribute__((amdgpu_waves_per_eu(WIDER <
 
 // out[row, head, :] = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s      (reference paged_attention_kernels.py:121-204)
 // Four groups of 64 lanes take the splits in turn, a lane holding up to four outputs; the groups' sums meet in
-// LDS and are added in a fixed order. All loads of a lane are independent, so they overlap.
+// LDS and are added in a fixed order. What bounds it is a launch and one trip to memory: up to 64 splits' (maximum, sum) pairs, partial outputs and the gate
+// are asked for together, before any is looked at, and the weights are handed round as scalars. us of attention and merge,
+// maxima first and a branch a load / so, with four page ids a trip instead of one: 1 row of 900 keys, 12 heads of 128 over 3, 8.5 / 7.3, 8 of 4,096 15.6 / 14.3, 16 of 2,000
+// 16.5 / 15.1, 64 of 500 16.7 / 15.5, of 4,096 78.3 / 77.6.
 static constexpr int MG = 4;             // split groups per workgroup
 static constexpr int MD = (VD + 63) / 64;  // outputs per lane
 
@@ -861,52 +877,55 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_kernel(const float* _
   __shared__ float so[MG][MD][64];
   const long row = blockIdx.x;
   const int head = blockIdx.y;
-  const int grp = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int n_splits = row_splits ? row_splits[row] : max_splits;   // partial results of this row
   if (n_splits <= 1) return;                                        // its output is final already
   const long base = (row * n_heads + head) * max_splits;
-  // every wave reads the splits' (maximum, sum) pairs with one split per lane, so that the reads go out together
-  // and not one after the other; the weights stay on the lanes and are handed round by index
-  float M = -INFINITY;
-  for (int s0 = 0; s0 < n_splits; s0 += 64)
-    if (s0 + lane < n_splits) M = fmaxf(M, part_ml[base + s0 + lane].x);
+  // a split's (maximum, sum) pair a lane; the group's partial outputs of 64 splits from s0 on
+  auto pairs = [&](int s0) { return part_ml[base + min(s0 + lane, n_splits - 1)]; };
+  float v[64 / MG][MD];
+  auto outputs = [&](int s0) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    for (int q = 0; q < 64 / MG; ++q) {
+#pragma unroll
+      for (int j = 0; j < MD; ++j) v[q][j] = 0.f;
+      const int i = s0 + grp + q * MG;
+      if (i < n_splits)
+#pragma unroll
+        for (int j = 0; j < MD; ++j) v[q][j] = part_o[(base + i) * VD + min(j * 64 + lane, VD - 1)];
+    }
+  };
+  float2 ml = pairs(0);
+  outputs(0);
+  float z[MD];
+  if constexpr (GATED)
+#pragma unroll
+    for (int j = 0; j < MD; ++j) z[j] = extras.gate[row * extras.gate_ld + (long)head * VD + min(j * 64 + lane, VD - 1)];
+  float M = ml.x;
+  for (int s0 = 64; s0 < n_splits; s0 += 64) M = fmaxf(M, pairs(s0).x);
+  M = wave_max(M);
   float acc[MD];
 #pragma unroll
   for (int j = 0; j < MD; ++j) acc[j] = 0.f;
   float L = 0.f;
   for (int s0 = 0; s0 < n_splits; s0 += 64) {
-    const int cnt = min(64, n_splits - s0);
-    // the group's partial outputs of this chunk are asked for before the weights are known: one round trip, not two
-    float v[64 / MG][MD];
-#pragma unroll
-    for (int q = 0; q < 64 / MG; ++q) {
-      const int i = grp + q * MG;
-#pragma unroll
-      for (int j = 0; j < MD; ++j) {
-        const int d = j * 64 + lane;
-        v[q][j] = (i < cnt && d < VD) ? part_o[(base + s0 + i) * VD + d] : 0.f;
-      }
+    if (s0) {
+      ml = pairs(s0);
+      outputs(s0);
     }
     float w = 0.f;
-    if (lane < cnt) {
-      const float2 ml = part_ml[base + s0 + lane];
-      if (ml.x != -INFINITY) {   // else: a split that held no key of this row; its partial output means nothing
-        w = exp2f(ml.x - M);
-        L += w * ml.y;
-      }
+    if (s0 + lane < n_splits && ml.x != -INFINITY) {   // (-inf: a split that held no key of this row; its partial output means nothing)
+      w = exp2f(ml.x - M);
+      L += w * ml.y;
     }
 #pragma unroll
     for (int q = 0; q < 64 / MG; ++q) {
-      const float wi = __shfl(w, min(grp + q * MG, 63), 64);
+      const float wi = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), grp + q * MG));
 #pragma unroll
-      for (int j = 0; j < MD; ++j)
-        if (wi != 0.f) acc[j] += wi * v[q][j];
+      for (int j = 0; j < MD; ++j) acc[j] += wi != 0.f ? __builtin_fmaf(wi, v[q][j], 0.f) : 0.f;       // (the product rounded by itself)
     }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off, 64);
+  L = wave_sum(L);
   if (sink) L += sink_share(sinks, head, M);      // the sink's share of the denominator, once for all splits
 #pragma unroll
   for (int j = 0; j < MD; ++j) so[grp][j][lane] = acc[j];
@@ -920,7 +939,7 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_kernel(const float* _
 #pragma unroll
     for (int gq = 1; gq < MG; ++gq) t += so[gq][j][lane];
     if (turn) t = turn_back_lane(t, lane, turn[row * (VD / 2) + d / 2]);
-    if constexpr (GATED) t *= gate_factor(extras.gate[row * extras.gate_ld + (long)head * VD + d]);
+    if constexpr (GATED) t *= gate_factor(z[j]);
     out[row * out_ld + (long)head * VD + d] = static_cast<__bf16>(t / L);
   }
 }
