@@ -922,7 +922,7 @@ __global__ __launch_bounds__(MG * 64) void attention_merge_kernel(const float* _
     for (int q = 0; q < 64 / MG; ++q) {
       const float wi = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), grp + q * MG));
 #pragma unroll
-      for (int j = 0; j < MD; ++j) acc[j] += wi != 0.f ? __builtin_fmaf(wi, v[q][j], 0.f) : 0.f;       // (the product rounded by itself)
+      for (int j = 0; j < MD; ++j) acc[j] = wi != 0.f ? __builtin_fmaf(wi, v[q][j], acc[j]) : acc[j];
     }
   }
   L = wave_sum(L);
