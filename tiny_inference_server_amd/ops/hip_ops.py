@@ -19,6 +19,7 @@ import ctypes
 import functools
 import json
 import os
+import threading
 from ctypes import c_float, c_int, c_long, c_void_p
 from typing import NamedTuple, Optional
 
@@ -720,6 +721,14 @@ def tile_pieces(seq_rows, tiles, tile_splits: int, tile_max_steps: int, window: 
     return out[:n]
 
 
+# The two mixers of a block run side by side if a request brings at least this many rows, in a captured step and launch by launch. us of a whole pass
+# one after the other / side by side, both in one run. Captured: attention beside a delta rule (4 blocks), one prompt of 16 rows 815 / 833, 64 975 / 950,
+# 256 1242 / 1184, 512 1537 / 1488, 1,024 2090 / 1938, 1,531 2690 / 2430; attention beside a matrix state (6 blocks), 64 rows 750 / 736, 256 880 / 852,
+# 1,024 1628 / 1597. Steps of single rows do not pay for the branches' fork and join: 5 rows 439 / 450, 32 590 / 613, 128 978 / 1034. Launch by
+# launch the host needs some 100 us more a block, which few rows do not cover: 64 rows 1605 / 2090 and 880 / 1100, 1,024 2227 / 2187 and
+# 1712 / 1754, 2,000 3372 / 3187 and 2663 / 2607.
+_BESIDE_FROM, _BESIDE_LAUNCHED_FROM = 64, 1536
+
 _side_streams = {}
 
 
@@ -729,6 +738,19 @@ def _side_stream(device_index: int):
     s = _side_streams.get(device_index)
     if s is None:
         s = _side_streams[device_index] = torch.cuda.Stream(torch.device("cuda", device_index))
+    return s
+
+
+_beside_streams = threading.local()
+
+
+def _beside_stream(device_index: int):
+    """This thread's stream for `HipOps.beside` (default priority): a thread that captures a graph on it shares it with no other, and the
+    allocator keeps that stream's memory from one engine to the next."""
+    of_device = _beside_streams.__dict__
+    s = of_device.get(str(device_index))
+    if s is None:
+        s = of_device[str(device_index)] = torch.cuda.Stream(torch.device("cuda", device_index))
     return s
 
 
@@ -780,6 +802,26 @@ class HipOps:
         # partial results of split key ranges: one buffer of fixed size that never moves (captured graphs hold its address)
         self._workspace = torch.empty(_ATTN_WORKSPACE_FLOATS, dtype=torch.float32, device=self.device) \
             if dtype == torch.bfloat16 else None
+
+    # ---- two branches of a block side by side ----------------------------------------------------------------
+    def beside_pays(self, batch) -> bool:
+        rows = batch.max_seq_rows
+        return rows >= _BESIDE_FROM and self.dtype == torch.bfloat16 and (rows >= _BESIDE_LAUNCHED_FROM or torch.cuda.is_current_stream_capturing())
+
+    def beside(self, first, second):
+        """first() on the current stream and second() on one of this object's own beside it; returns both results, which the current stream may
+        read. What second() launches has to own its memory: no work space of this object."""
+        main = torch.cuda.current_stream(self.device)
+        side = _beside_stream(self._device_index)
+        side.wait_stream(main)
+        try:
+            with torch.cuda.stream(side):
+                other = second()
+            result = first()
+        finally:
+            main.wait_stream(side)      # also where a call failed: what it reads may go back to the allocator after this
+        other.record_stream(main)
+        return result, other
 
     # ---- planning on the host --------------------------------------------------------------------------
     def plan_attention_mode(self, seq_rows, window: int = 0):

@@ -20,7 +20,9 @@ every part      graph_safe = True                      class attribute, only if 
                                                        as graphs); absent or False keeps the model on plain launches;
                                                        "single_rows": the promise holds for steps in which every
                                                        request brings one token (those are still captured)
-mixer           cache_need(params) -> PagedKvNeed | StateNeed | None, or a tuple of one PagedKvNeed and one StateNeed for
+mixer           own_memory = True                      class attribute, optional: what the part launches uses no work space that other
+                                                       parts' launches use (it may run on another stream beside them)
+                cache_need(params) -> PagedKvNeed | StateNeed | None, or a tuple of one PagedKvNeed and one StateNeed for
                                                        a mixer that keeps both      classmethod
                 forward(x, ctx, residual=None) -> y    x: normed rows; ctx: CallContext; adds `residual` if given
 feed-forward    forward(x, residual=None) -> y
@@ -149,6 +151,18 @@ def layer_product(ops):
     """The product x . w^T (+ residual) of a layer's own matrices: by rows, where the operations object tells such products
     apart (it has kernels of its own for them), else its plain product."""
     return getattr(ops, "linear_by_rows", None) or ops.linear
+
+
+def side_by_side(ops, batch, calls):
+    """The results of the calls [(mixer, call)] of a block's mixers, which read the same rows. One of two runs beside the other where the operations
+    object can (`beside`), says that it pays for this step, and that mixer promises own_memory."""
+    if len(calls) == 2 and hasattr(ops, "beside") and ops.beside_pays(batch):
+        own = [getattr(m, "own_memory", False) for m, _ in calls]
+        if own[1]:
+            return list(ops.beside(calls[0][1], calls[1][1]))
+        if own[0]:
+            return list(ops.beside(calls[1][1], calls[0][1]))[::-1]
+    return [call() for _, call in calls]
 
 
 def normed_linear(ops, x, w, norm, **kw):

@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import torch
 
-from .base import ARRANGEMENTS, NORMS, TOKEN_INPUTS, Arrangement, to_compute, to_gain
+from .base import ARRANGEMENTS, NORMS, TOKEN_INPUTS, Arrangement, side_by_side, to_compute, to_gain
 from .stream32 import Stream32
 
 
@@ -187,9 +187,10 @@ class SandwichStream32(PreNormStream32):
         post = (self.post_a.gain, self.post_a.eps)
         if self.w_in is not None:
             proj = self.ops.linear(h, self.w_in, out_dtype=torch.float32)
-            results = [m.forward_projected(proj[:, c0:c1], ctx.of(n)) for (n, m, _), (c0, c1) in zip(self.mixers, self.cols)]
+            calls = [(m, lambda m=m, n=n, c=c: m.forward_projected(proj[:, c[0]:c[1]], ctx.of(n))) for (n, m, _), c in zip(self.mixers, self.cols)]
         else:
-            results = [m.forward32(h, ctx.of(n)) for n, m, _ in self.mixers]
+            calls = [(m, lambda m=m, n=n: m.forward32(h, ctx.of(n))) for n, m, _ in self.mixers]
+        results = side_by_side(self.ops, ctx.of(self.mixers[0][0]).batch, calls)
         if len(results) == 1:
             return results[0], post
         eps = {j.eps for _, _, j in self.mixers}

@@ -17,6 +17,7 @@ def state_floats(kind: str, n_heads: int, dim: int, vdim: int) -> int:
 class _MatrixStateMixer:
     """What the two mixers below share: stacked input matrices, the output matrix, the ways in."""
     graph_safe = True
+    own_memory = True
 
     def _stack(self, spec, tensors, keys):
         """The input matrices under `keys`, stacked as stored; returns their first columns in the product."""
@@ -272,6 +273,7 @@ class GatedDeltaRule:
     (heads*dim,), g1 (gate_rank, width), g2 (heads*vdim, gate_rank), norm (vdim,), o (width, heads*vdim).
     """
     graph_safe = True
+    own_memory = True
 
     @classmethod
     def _sizes(cls, params):

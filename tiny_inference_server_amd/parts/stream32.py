@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import torch
 
-from .base import ARRANGEMENTS, FEED_FORWARDS, GATES, NORMS, STAGE_INPUTS, Arrangement, to_compute, to_gain
+from .base import ARRANGEMENTS, FEED_FORWARDS, GATES, NORMS, STAGE_INPUTS, Arrangement, side_by_side, to_compute, to_gain
 
 
 class Stream32:
@@ -177,7 +177,9 @@ class PostNormGated(Arrangement):
     def forward(self, x, ctx):
         ops = self.ops
         proj = ops.linear(x.rows, self.w_in, out_dtype=torch.float32)
-        branches = [(m.forward_projected(proj[:, c0:c1], ctx.of(name)), scale) for name, m, (c0, c1), scale in self.mixers]
+        calls = [(m, lambda m=m, n=n, c=c: m.forward_projected(proj[:, c[0]:c[1]], ctx.of(n))) for n, m, c, _ in self.mixers]
+        results = side_by_side(ops, ctx.of(self.mixers[0][0]).batch, calls)
+        branches = [(y, scale) for y, (_, _, _, scale) in zip(results, self.mixers)]
         gate = proj[:, self.gate_cols[0]:self.gate_cols[1]] if self.gate_cols else None
         full, rows = ops.gated_postnorm(x.full, branches, gate, self.gate_a.bias if gate is not None else None,
                                         self.alpha, self.norm_a.gain, self.norm_a.eps)
