@@ -221,28 +221,35 @@ __global__ __launch_bounds__(256) void grouped_plain_kernel(const TA* __restrict
 // wave owns RM x RN tiles of 16 x 16. A matrix row and an input row are the two operands of v_mfma_f32_16x16x32_bf16
 // straight from memory, 16 bytes a lane (rows 16-byte aligned, K a multiple of 8); a wave's RM + RN loads of a step feed
 // RM RN products, and what the waves of a workgroup share meets in the caches. Each result is one wave's sum over K in
-// steps of 32. Two shapes are built: 16 entries x 64 columns for groups of a few rows (decoded tokens: the job is to
-// stream the matrices once), 64 x 128 for groups of many that the tiles below do not take.
+// steps of 32, or the sum of KS waves' such sums, of every KS-th batch each. Three shapes are built: 16 entries x 64 columns, or x 16 with the sum over K
+// split (split_k), for groups of a few rows (decoded tokens: the job is to stream the matrices once), 64 x 128 for groups of many that the tiles
+// below do not take.
 // grid (blocks of columns, groups, tiles of entries): every group's first tile, then every group's second, most of which have no entries and
 // end at once. With a group's tiles behind one another the ones that work were every second, fourth .. workgroup, and those go to the same
 // compute units: 64 groups of 512 of 1,024, two choices a row, us, so / as it is: 17 rows 22 / 14, 40 21 / 14.5, 64 43 / 15, 127 47 / 16;
 // 8 groups of 5,632 of 2,048, 17 rows 52 / 43; 16 of 4,096 of 1,536, 24 rows 50 / 43.
-template <typename TO, int WM, int WN, int RM, int RN>
+template <typename TO, int WM, int WN, int RM, int RN, int KS>
 __global__ __launch_bounds__(256) void grouped_mfma_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                            TO* __restrict__ C, GroupedArgs p) {
-  static_assert(WM * WN == 4, "four waves a workgroup");
+  static_assert(WM * WN * KS == 4 && (KS == 1 || WM * RM * RN == 1), "four waves a workgroup");
   const int g = blockIdx.y, t = threadIdx.x, lane = t % 64, wave = t / 64;
-  const int m0 = blockIdx.z * (16 * RM * WM) + (wave / WN) * (16 * RM);
+  const int part = KS > 1 ? wave / WN : 0;
+  const int m0 = blockIdx.z * (16 * RM * WM) + (KS > 1 ? 0 : (wave / WN) * (16 * RM));
   const int n0 = blockIdx.x * (16 * RN * WN) + (wave % WN) * (16 * RN);
-  const int count = p.lists ? p.counts[g] : p.rows;
-  if (m0 >= count || n0 >= p.N) return;
   const int c16 = lane & 15, kg = lane >> 4;
+  // the group's count and the entries asked for together (an entry past the count is the line's last, which nobody looks at)
   int mine[RM];
-  const bf16* arow[RM];
 #pragma unroll
   for (int i = 0; i < RM; ++i) {
     const int m = m0 + i * 16 + c16;
-    mine[i] = m < count ? (p.lists ? p.lists[(long)g * p.line + m] : m) : -1;
+    mine[i] = p.lists ? p.lists[(long)g * p.line + (m < p.line ? m : p.line - 1)] : m;
+  }
+  const int count = p.lists ? p.counts[g] : p.rows;
+  if (m0 >= count || (KS == 1 && n0 >= p.N)) return;
+  const bf16* arow[RM];
+#pragma unroll
+  for (int i = 0; i < RM; ++i) {
+    if (m0 + i * 16 + c16 >= count) mine[i] = -1;
     arow[i] = A + (long)(mine[i] < 0 ? 0 : mine[i] / p.a_div) * p.lda + (long)g * p.a_group + kg * 8;
   }
   bool w_ok[RN];
@@ -265,11 +272,11 @@ __global__ __launch_bounds__(256) void grouped_mfma_kernel(const bf16* __restric
   // 12.4 / 12.8 / 12.9, 1,024 of 1,408 12.7 / 10.1 / 10.0; 1 row 5,632 of 2,048 18.4 / 14.7 / 15.1. (161 MB in 41 us: 4 TB/s.)
   constexpr int U = 4, SETS = RM + RN <= 2 ? 2 : 1;
   bf16x8 av[SETS][U][RM], wv[SETS][U][RN];
-  const int whole = p.K / (32 * U);
+  const int batches = p.K / (32 * U), whole = KS > 1 ? (batches - part + KS - 1) / KS : batches;      // (in all, and this wave's: every KS-th)
   auto load = [&](int set, int b) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = (b * U + u) * 32;
+      const int k = ((KS > 1 ? b * KS + part : b) * U + u) * 32;
 #pragma unroll
       for (int i = 0; i < RM; ++i) av[set][u][i] = *reinterpret_cast<const bf16x8*>(arow[i] + k);
 #pragma unroll
@@ -297,10 +304,10 @@ __global__ __launch_bounds__(256) void grouped_mfma_kernel(const bf16* __restric
       multiply(e);
     }
   }
-  if (whole * 32 * U < p.K) {                    // the last, begun batch: zeros past the end of K
+  if (batches * 32 * U < p.K && (KS == 1 || batches % KS == part)) {                    // the last, begun batch: zeros past the end of K
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = (whole * U + u) * 32;
+      const int k = (batches * U + u) * 32;
       const bool k_ok = k + kg * 8 < p.K;
 #pragma unroll
       for (int i = 0; i < RM; ++i) av[0][u][i] = k_ok ? *reinterpret_cast<const bf16x8*>(arow[i] + k) : zero;
@@ -308,6 +315,14 @@ __global__ __launch_bounds__(256) void grouped_mfma_kernel(const bf16* __restric
       for (int j = 0; j < RN; ++j) wv[0][u][j] = k_ok ? *reinterpret_cast<const bf16x8*>(wrow[j] + k) : zero;
     }
     multiply(0);
+  }
+  if constexpr (KS > 1) {                        // the waves' parts of a column block added in order
+    __shared__ f32x4 parts[KS - 1][WN][64];
+    if (part > 0) parts[part - 1][wave % WN][lane] = acc[0][0];
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int s = 0; s < KS - 1; ++s) acc[0][0] += parts[s][wave % WN][lane];
   }
   // the lane holds, of tile (i, j), the columns n0 + 16 j + 4 kg + e of entry i * 16 + c16
 #pragma unroll
@@ -580,6 +595,15 @@ TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_
 
 // in_dtype / out_dtype: 0 float, 1 bfloat16 (a bfloat16 input may give a 32-bit output). most_rows: the most entries a
 // group can have (the grid's height); most_entries: the most that all groups' lists can have together.
+// Whether a column block's sum over K is split over a workgroup's four waves (16 columns a workgroup) or every wave sums its own 16 (64 a
+// workgroup): split if each wave but one gets a batch at least, and either K is long or the blocks in all are few, so that the chip has more loads
+// under way and compute units differ less in what they get. us, whole / split, 8 groups, two choices a row: 1 row 2,816 of 1,024 7.6 / 6.1,
+// 1,024 of 1,408 9.1 / 4.9, 5,632 of 2,048 21.5 / 14.9, 2,048 of 2,816 16.1 / 7.9; 5 rows 12.4 / 8.6, 9.9 / 7.3, 37.8 / 35.4, 17.5 / 18.2; 8 rows 13.6 / 10.4,
+// 10.1 / 7.3, 38.7 / 38.5, 19.0 / 18.8, 7,168 of 4,096 105 / 78, 1,024 of 384 4.5 / 4.0; 64 groups of 512 of 1,024, 4 rows 11.8 / 7.4, 40 rows
+// 13.6 / 13.9. Whole where that is better: 64 rows, 64 groups of 1,024 of 256 8.6 / 12.0, of 512 14.4 / 16.9, of 640 17.7 / 18.9; 128 groups of
+// 1,536 of 1,024 79 / 86. (Mean error against 64 bits, K = 1,408, 2e-7 / 1e-7.)
+static bool split_k(long blocks, int K) { return K >= 384 && (K >= 1536 || blocks <= 3L * g_units); }
+
 TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, long lda, long a_group, int a_div, const void* W,
                                   void* C, long ldc, long c_group, const int* lists, const int* counts, int line,
                                   int groups, int most_rows, long most_entries, int N, int K, int act, const float* gate, long ldg,
@@ -628,12 +652,18 @@ TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, lo
     } else if (aligned && most_rows >= 64 * (lists ? groups : 1)) {
       // 64 entries x 128 columns a workgroup, operands straight from memory
       const dim3 big((N + 127) / 128, groups, (most_rows + 63) / 64);
-      if (out_dtype == TIS_BF16) grouped_mfma_kernel<bf16, 2, 2, 2, 4><<<big, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);
-      else grouped_mfma_kernel<float, 2, 2, 2, 4><<<big, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);
+      if (out_dtype == TIS_BF16) grouped_mfma_kernel<bf16, 2, 2, 2, 4, 1><<<big, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);
+      else grouped_mfma_kernel<float, 2, 2, 2, 4, 1><<<big, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);
     } else if (aligned) {
-      const dim3 few(grid.x, groups, tiles_m);
-      if (out_dtype == TIS_BF16) grouped_mfma_kernel<bf16, 1, 4, 1, 1><<<few, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);
-      else grouped_mfma_kernel<float, 1, 4, 1, 1><<<few, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);
+#define FEW(WN, KS)                                                                                                       \
+  {                                                                                                                       \
+    const dim3 few((N + 16 * WN - 1) / (16 * WN), groups, tiles_m);                                                       \
+    if (out_dtype == TIS_BF16) grouped_mfma_kernel<bf16, 1, WN, 1, 1, KS><<<few, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);  \
+    else grouped_mfma_kernel<float, 1, WN, 1, 1, KS><<<few, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);            \
+  }
+      if (split_k((lists ? (most_entries < groups ? most_entries : groups) : (long)groups * tiles_m) * ((N + 63) / 64), K)) FEW(1, 4)
+      else FEW(4, 1)
+#undef FEW
     } else {
       if (out_dtype == TIS_BF16) grouped_plain_kernel<bf16, bf16><<<grid, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);
       else grouped_plain_kernel<bf16, float><<<grid, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);
