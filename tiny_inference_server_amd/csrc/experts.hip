@@ -237,19 +237,17 @@ __global__ __launch_bounds__(256) void grouped_mfma_kernel(const bf16* __restric
   const int m0 = blockIdx.z * (16 * RM * WM) + (KS > 1 ? 0 : (wave / WN) * (16 * RM));
   const int n0 = blockIdx.x * (16 * RN * WN) + (wave % WN) * (16 * RN);
   const int c16 = lane & 15, kg = lane >> 4;
-  // the group's count and the entries asked for together (an entry past the count is the line's last, which nobody looks at)
-  int mine[RM];
-#pragma unroll
-  for (int i = 0; i < RM; ++i) {
-    const int m = m0 + i * 16 + c16;
-    mine[i] = p.lists ? p.lists[(long)g * p.line + (m < p.line ? m : p.line - 1)] : m;
-  }
+  // The count by itself: a workgroup without entries ends on it, and with many groups those are most of the grid. us, the entries asked for beside the count / behind it: 128
+  // groups, 8 choices a row, 1 row 5,632 of 2,048 47.7 / 38.2, 3 rows 2,048 of 1,536 34.6 / 28.3, 5 rows 2,048 of 1,024 37.0 / 31.4; 8 groups of 2, 8 rows 2,048 of 2,816
+  // 17.6 / 17.8.
   const int count = p.lists ? p.counts[g] : p.rows;
   if (m0 >= count || (KS == 1 && n0 >= p.N)) return;
+  int mine[RM];
   const bf16* arow[RM];
 #pragma unroll
   for (int i = 0; i < RM; ++i) {
-    if (m0 + i * 16 + c16 >= count) mine[i] = -1;
+    const int m = m0 + i * 16 + c16;
+    mine[i] = m < count ? (p.lists ? p.lists[(long)g * p.line + m] : m) : -1;
     arow[i] = A + (long)(mine[i] < 0 ? 0 : mine[i] / p.a_div) * p.lda + (long)g * p.a_group + kg * 8;
   }
   bool w_ok[RN];
