@@ -39,3 +39,17 @@ def test_many_results_of_few_steps(rows, N, K, tile):
     """Products whose results take a good part of their time: the tiles (0: 256 x 256, 3: 128 x 192 two a unit, 6: 64 x 64) that were measured to be the
     fastest, each by a twentieth to a quarter against the tile that an estimate by the steps alone picks."""
     assert hip_ops.library("gemm_tiles").cdll.tis_gemm_tiles_pick(rows, N, K) == tile
+
+
+@pytest.mark.parametrize("groups,top,rows,N,K,split", [
+    # slower with the sum over K split, by 4 to 24 %
+    (128, 8, 1, 5632, 384, False), (128, 8, 1, 5632, 512, False), (16, 4, 16, 2048, 384, False), (16, 4, 16, 2048, 512, False), (16, 4, 16, 2048, 704, False),
+    (32, 4, 16, 1024, 512, False), (64, 8, 40, 512, 704, False), (8, 2, 16, 5632, 704, False), (64, 8, 5, 2048, 384, False),
+    # faster, by 4 to 100 %
+    (8, 2, 1, 2048, 2816, True), (8, 2, 8, 5632, 2048, True), (16, 4, 16, 5632, 2048, True), (64, 8, 16, 2048, 2048, True), (128, 8, 8, 2048, 1536, True),
+    (64, 8, 5, 1024, 1024, True), (8, 2, 5, 2816, 1024, True), (8, 2, 5, 1024, 1408, True), (64, 8, 5, 512, 384, True), (16, 4, 16, 1024, 704, True), (8, 2, 1, 2048, 384, True)])
+def test_sums_over_k_are_split_where_that_was_faster(groups, top, rows, N, K, split):
+    """A sum over K goes to a workgroup's four waves from 1,536 terms on, and below while the blocks of columns are few."""
+    lib = hip_ops.library("experts").cdll
+    assert lib.tis_grouped_tile(1, groups, rows, c_long(rows * top), N, K, 0) < 0
+    assert bool(lib.tis_grouped_split(1, groups, rows, c_long(rows * top), N, K)) == split

@@ -15,8 +15,8 @@
 // g * c_group: with a_div = top the input rows are the step's rows and the outputs lie by assignment (an expert's first
 // product), with a_div = 1 both lie by assignment (its second); without lists every group takes all rows, and a_group /
 // c_group move from one group's columns to the next (a product per head on a head's own columns). Sums are 32-bit in
-// an order that depends on K and on the kernel: the products straight from memory add steps of 32, the tiles steps of 16. Within one of them a
-// row's result does not depend on what else is in the step; which of them a step takes hangs on its entries (tis_grouped_tile), and a
+// an order that depends on K and on the kernel: the products straight from memory add steps of 32, in one chain or in four (tis_grouped_split), the tiles steps of 16.
+// Within one of them a row's result does not depend on what else is in the step; which of them a step takes hangs on its entries (tis_grouped_tile), and a
 // row's last bits may differ from one to the other.
 #include "tile_loop.h"
 
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256) void grouped_plain_kernel(const TA* __restrict
 // straight from memory, 16 bytes a lane (rows 16-byte aligned, K a multiple of 8); a wave's RM + RN loads of a step feed
 // RM RN products, and what the waves of a workgroup share meets in the caches. Each result is one wave's sum over K in
 // steps of 32, or the sum of KS waves' such sums, of every KS-th batch each. Three shapes are built: 16 entries x 64 columns, or x 16 with the sum over K
-// split (split_k), for groups of a few rows (decoded tokens: the job is to stream the matrices once), 64 x 128 for groups of many that the tiles
+// split (tis_grouped_split), for groups of a few rows (decoded tokens: the job is to stream the matrices once), 64 x 128 for groups of many that the tiles
 // below do not take.
 // grid (blocks of columns, groups, tiles of entries): every group's first tile, then every group's second, most of which have no entries and
 // end at once. With a group's tiles behind one another the ones that work were every second, fourth .. workgroup, and those go to the same
@@ -591,17 +591,21 @@ TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_
   return pick;
 }
 
+// Whether, where no tile takes a product of a few rows a group, a column block's sum over K is split over a workgroup's four waves (16 columns a workgroup) or every wave sums
+// its own 16 (64 a workgroup). Split, the chip has more loads under way and compute units differ less in what they get; but there are four times the workgroups, each with a
+// beginning and an end, groups without entries among them. So: K long enough that each wave but one gets a batch; from 1,536 on always, below only while the blocks of 64
+// columns in all are few. us, matrices from memory, whole / split: 8 groups, two choices a row, 2,048 of 2,816, 1 row 15.5 / 9.2, 3 rows 19.2 / 14.0, 8 20.2 / 17.8, 16 21.0 / 20.3;
+// 5,632 of 2,048, 3 rows 31.6 / 23.9, 16 42.2 / 38.8, 1 row 13.9 / 15.3 alone but a decode step with it 325 / 306; 16 of 4, 16 rows 5,632 of 2,048 74.6 / 67.1; 64 of 8, 16 rows 2,048 of
+// 2,048 91.8 / 85.0; 128 of 8, 8 rows 2,048 of 1,536 60.4 / 56.3, 16 rows 2,048 of 4,096 254 / 227. Where the line lies, 256 blocks (16 of 4, 16 rows) / 512 (the same, twice the columns): K = 384
+// 5.7 / 5.7 and 8.0 / 8.7, 512 6.6 / 6.4 and 9.5 / 10.4, 704 8.1 / 7.4 and 12.2 / 13.2, 1,024 9.6 / 9.2 and 15.6 / 16.1; 640 blocks of 1,024 (64 of 8, 5 rows) 22.1 / 16.1, of 512 12.6 / 11.2; 1,280
+// of 384 13.9 / 16.1. (Mean error against 64 bits, K = 1,408, 2e-7 / 1e-7.)
+TIS_EXPORT int tis_grouped_split(int lists, int groups, int most_rows, long most_entries, int N, int K) {
+  const long blocks = (lists ? (most_entries < groups ? most_entries : groups) : (long)groups * ((most_rows + 15) / 16)) * ((N + 63) / 64);
+  return K >= 384 && (K >= 1536 || 2 * blocks <= (K >= 1024 ? 6L : 3L) * g_units);
+}
+
 // in_dtype / out_dtype: 0 float, 1 bfloat16 (a bfloat16 input may give a 32-bit output). most_rows: the most entries a
 // group can have (the grid's height); most_entries: the most that all groups' lists can have together.
-// Whether a column block's sum over K is split over a workgroup's four waves (16 columns a workgroup) or every wave sums its own 16 (64 a
-// workgroup): split if each wave but one gets a batch at least, and either K is long or the blocks in all are few, so that the chip has more loads
-// under way and compute units differ less in what they get. us, whole / split, 8 groups, two choices a row: 1 row 2,816 of 1,024 7.6 / 6.1,
-// 1,024 of 1,408 9.1 / 4.9, 5,632 of 2,048 21.5 / 14.9, 2,048 of 2,816 16.1 / 7.9; 5 rows 12.4 / 8.6, 9.9 / 7.3, 37.8 / 35.4, 17.5 / 18.2; 8 rows 13.6 / 10.4,
-// 10.1 / 7.3, 38.7 / 38.5, 19.0 / 18.8, 7,168 of 4,096 105 / 78, 1,024 of 384 4.5 / 4.0; 64 groups of 512 of 1,024, 4 rows 11.8 / 7.4, 40 rows
-// 13.6 / 13.9. Whole where that is better: 64 rows, 64 groups of 1,024 of 256 8.6 / 12.0, of 512 14.4 / 16.9, of 640 17.7 / 18.9; 128 groups of
-// 1,536 of 1,024 79 / 86. (Mean error against 64 bits, K = 1,408, 2e-7 / 1e-7.)
-static bool split_k(long blocks, int K) { return K >= 384 && (K >= 1536 || blocks <= 3L * g_units); }
-
 TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, long lda, long a_group, int a_div, const void* W,
                                   void* C, long ldc, long c_group, const int* lists, const int* counts, int line,
                                   int groups, int most_rows, long most_entries, int N, int K, int act, const float* gate, long ldg,
@@ -659,7 +663,7 @@ TIS_EXPORT int tis_grouped_linear(int in_dtype, int out_dtype, const void* A, lo
     if (out_dtype == TIS_BF16) grouped_mfma_kernel<bf16, 1, WN, 1, 1, KS><<<few, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (bf16*)C, p);  \
     else grouped_mfma_kernel<float, 1, WN, 1, 1, KS><<<few, 256, 0, stream>>>((const bf16*)A, (const bf16*)W, (float*)C, p);            \
   }
-      if (split_k((lists ? (most_entries < groups ? most_entries : groups) : (long)groups * tiles_m) * ((N + 63) / 64), K)) FEW(1, 4)
+      if (tis_grouped_split(lists ? 1 : 0, groups, most_rows, most_entries, N, K)) FEW(1, 4)
       else FEW(4, 1)
 #undef FEW
     } else {
