@@ -22,10 +22,14 @@ every part      graph_safe = True                      class attribute, only if 
                                                        request brings one token (those are still captured)
 mixer           own_memory = True                      class attribute, optional: what the part launches uses no work space that other
                                                        parts' launches use (it may run on another stream beside them)
+                whole_block(ctx) -> operands | None    optional: what the operations object's kernel for a whole block takes of a part
+                                                       whose forward does nothing else (HipOps.small_block); None: not this call
+                own_memory and whole_block speak for the class that states them and for none derived from it
                 cache_need(params) -> PagedKvNeed | StateNeed | None, or a tuple of one PagedKvNeed and one StateNeed for
                                                        a mixer that keeps both      classmethod
                 forward(x, ctx, residual=None) -> y    x: normed rows; ctx: CallContext; adds `residual` if given
 feed-forward    forward(x, residual=None) -> y
+                whole_block() -> operands              optional, as for mixers
                 a mixer or feed-forward with the class attribute fuses_norm = True takes forward(..., norm=part)
                 instead: x arrives un-normed and the part applies `norm` itself, fused into its first product
                 where it can
@@ -153,11 +157,16 @@ def layer_product(ops):
     return getattr(ops, "linear_by_rows", None) or ops.linear
 
 
+def states(part, name: str) -> bool:
+    """Whether the part's own class states `name`, and no class above it: a derived class may do more than what it inherited was said of."""
+    return bool(type(part).__dict__.get(name))
+
+
 def side_by_side(ops, batch, calls):
     """The results of the calls [(mixer, call)] of a block's mixers, which read the same rows. One of two runs beside the other where the operations
     object can (`beside`), says that it pays for this step, and that mixer promises own_memory."""
     if len(calls) == 2 and hasattr(ops, "beside") and ops.beside_pays(batch):
-        own = [getattr(m, "own_memory", False) for m, _ in calls]
+        own = [states(m, "own_memory") for m, _ in calls]
         if own[1]:
             return list(ops.beside(calls[0][1], calls[1][1]))
         if own[0]:

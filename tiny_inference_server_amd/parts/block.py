@@ -1,7 +1,7 @@
 """Arrangements: how a block wires its norms, its mixer and its feed-forward."""
 from __future__ import annotations
 
-from .base import ARRANGEMENTS, Arrangement
+from .base import ARRANGEMENTS, Arrangement, states
 
 
 @ARRANGEMENTS.register("prenorm_residual")
@@ -14,7 +14,7 @@ class PreNormResidual(Arrangement):
         self.mixer_norm, self.mixer = self.parts["mixer_norm"], self.parts["mixer"]
         self.ffn_norm, self.ffn = self.parts["feed_forward_norm"], self.parts["feed_forward"]
         # a block of parts that say what they are made of may be one kernel, where the operations object has it and takes the step
-        self.one_kernel = ops.small_block if (getattr(ops, "small", None) is not None and hasattr(self.mixer, "whole_block") and hasattr(self.ffn, "whole_block")
+        self.one_kernel = ops.small_block if (getattr(ops, "small", None) is not None and states(self.mixer, "whole_block") and states(self.ffn, "whole_block")
                                               and hasattr(self.mixer_norm, "as_rms") and hasattr(self.ffn_norm, "as_rms")) else None
 
     def forward(self, x, ctx):

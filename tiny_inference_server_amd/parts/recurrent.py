@@ -15,9 +15,8 @@ def state_floats(kind: str, n_heads: int, dim: int, vdim: int) -> int:
 
 
 class _MatrixStateMixer:
-    """What the two mixers below share: stacked input matrices, the output matrix, the ways in."""
+    """What the mixers below share: stacked input matrices, the output matrix, the ways in."""
     graph_safe = True
-    own_memory = True
 
     def _stack(self, spec, tensors, keys):
         """The input matrices under `keys`, stacked as stored; returns their first columns in the product."""
@@ -51,6 +50,7 @@ class GatedLinearAttention(_MatrixStateMixer):
     params: width, n_heads, dim, vdim, tau, rank, eps. tensors, stored [out, in]: q, k (heads*dim, width), v, g
     (heads*vdim, width), o (width, heads*vdim), norm (vdim,), a1 (rank, width), a2 (heads*dim, rank), a2_bias.
     """
+    own_memory = True
 
     @classmethod
     def tensor_shapes(cls, params):
@@ -93,6 +93,7 @@ class MatrixMemory(_MatrixStateMixer):
     params: width, n_heads, dim, vdim, gate_cap, eps. tensors, stored [out, in]: q, k (heads*dim, width), v, g
     (heads*vdim, width), o (width, heads*vdim), norm (heads*vdim,), i, f (heads, width), i_bias, f_bias (heads,).
     """
+    own_memory = True
 
     @classmethod
     def tensor_shapes(cls, params):
@@ -132,6 +133,7 @@ class LightningAttention(_MatrixStateMixer):
     params: width, n_heads, dim, vdim, decay (one number per head), eps. tensors, stored [out, in]: q, k
     (heads*dim, width), v, g (heads*vdim, width), o (width, heads*vdim), norm (heads*vdim,).
     """
+    own_memory = True
 
     @classmethod
     def tensor_shapes(cls, params):
