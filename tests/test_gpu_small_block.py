@@ -84,3 +84,21 @@ def test_what_it_leaves_alone():
     p = hip_ops._ptr(torch.zeros(64, device="cuda"))
     with pytest.raises(hip_ops.KernelError):
         ops.small.tis_small_block(p, 64, p, 64, p, 0.0, p, p, p, 0.0, p, p, hip_ops._ptr(None), 0, p, p, p, p, 1, p, 1, 128, 176, 8, 2, 8, 16, 0, 1.0, 16, ops._stream())
+
+
+def test_a_small_call_leaves_a_larger_one_its_lds():
+    """The kernel's limit of dynamic LDS is the process's: a call that needs little must not lower it under one that another thread is about to launch."""
+    ops = hip_ops.HipOps("cuda:0", torch.float32)
+    D, H, G, HD, F, ps, keys = 64, 8, 2, 8, 176, 16, 16
+    batch = SimpleNamespace(positions=torch.tensor([keys - 1], dtype=torch.int32).cuda(), row_seq=torch.zeros(1, dtype=torch.int32).cuda(),
+                            write_slots={"g": torch.tensor([keys - 1], dtype=torch.int32).cuda()}, block_tables={"g": torch.zeros(1, 1, dtype=torch.int32).cuda()},
+                            max_kv_len=keys, max_seq_rows=1, n_rows=1, extras={}, seq_rows=[])
+
+    def ones(*shape):
+        return torch.ones(*shape, device="cuda")
+
+    norm = (ones(D), 1e-5)
+    y = ops.small_block(ones(1, D), batch, "g", ones(1, 2, G, ps, HD), (norm, norm),
+                        (ones((H + 2 * G) * HD, D), ones(D, H * HD), None, False, H, G, HD, 0, 1.0), (ones(2 * F, D), ones(D, F)))
+    torch.cuda.synchronize()
+    assert y is not None and ops.small.cdll.tis_small_block_lds() == 160 * 1024

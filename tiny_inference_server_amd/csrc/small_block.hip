@@ -15,6 +15,8 @@
 // bits of the separate kernels: 22.7.)
 //
 // Sums are 32-bit: a product's sixteen partial sums of up to 12 terms added up in pairs, where the separate kernels have one chain.
+#include <mutex>
+
 #include "common.h"
 
 TIS_DEFINE_LAST_ERROR(tis_small_block)
@@ -246,6 +248,27 @@ TIS_EXPORT int tis_small_block_takes(int rows, int D, int F, int H, int G, int H
   return sb_layout(H, G, HD, page_size, (int)cap).end * 4L <= SB_LDS;
 }
 
+// The dynamic LDS that the kernel may be launched with on this device, -1 where the runtime does not say.
+TIS_EXPORT int tis_small_block_lds() {
+  hipFuncAttributes got;
+  return hipFuncGetAttributes(&got, (const void*)small_block_kernel) == hipSuccess ? got.maxDynamicSharedSizeBytes : -1;
+}
+
+// The kernel may be launched with all of a compute unit's LDS, said once a device: said for each call's own size it would be lowered by a smaller call, under a
+// larger one that another thread is about to launch.
+static hipError_t sb_allow_lds() {
+  static std::mutex lock;
+  static unsigned long long allowed = 0;         // a bit a device
+  int device = 0;
+  if (hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
+  const unsigned long long bit = device < 64 ? 1ull << device : 0;
+  std::lock_guard<std::mutex> held(lock);
+  if (allowed & bit) return hipSuccess;
+  const hipError_t e = hipFuncSetAttribute((const void*)small_block_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SB_LDS);
+  if (e == hipSuccess) allowed |= bit;
+  return e;
+}
+
 // x, out: [rows, D] 32-bit, row strides x_ld, out_ld; the matrices as the separate kernels take them (rows of query and key heads in rotary pairs, gate
 // and up rows in turn), on 16 bytes; keys: the most a row sees of its request's (its position is below). Launches only: safe under stream capture.
 TIS_EXPORT int tis_small_block(const float* x, long x_ld, float* out, long out_ld, const float* gain_a, float eps_a, const float* w_qkv, const float* w_o,
@@ -263,8 +286,7 @@ TIS_EXPORT int tis_small_block(const float* x, long x_ld, float* out, long out_l
   const SmallBlock a{x, x_ld, out, out_ld, gain_a, gain_f, eps_a, eps_f, w_qkv, w_o, w_gu, w_down, (const float2*)table, positions, row_seq, write_slots,
                      block_tables, plane, bt_ld, D, F, H, G, HD, page_size, window, interleaved, cap, scale};
   const size_t bytes = sb_layout(H, G, HD, page_size, cap).end * sizeof(float);
-  if (hipError_t e = hipFuncSetAttribute((const void*)small_block_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes); e != hipSuccess)
-    return tis_fail("small_block: %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
+  if (hipError_t e = sb_allow_lds(); e != hipSuccess) return tis_fail("small_block: %ld bytes of LDS: %s", SB_LDS, hipGetErrorString(e));
   small_block_kernel<<<rows, SB_THREADS, bytes, stream>>>(a);
   return tis_launch_status("small_block");
 }
