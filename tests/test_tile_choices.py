@@ -53,3 +53,15 @@ def test_sums_over_k_are_split_where_that_was_faster(groups, top, rows, N, K, sp
     lib = hip_ops.library("experts").cdll
     assert lib.tis_grouped_tile(1, groups, rows, c_long(rows * top), N, K, 0) < 0
     assert bool(lib.tis_grouped_split(1, groups, rows, c_long(rows * top), N, K)) == split
+
+
+@pytest.mark.parametrize("rows,D,F,H,G,HD,keys,takes", [
+    # slower in one kernel, by 5 to 45 %
+    (1, 64, 192, 2, 1, 32, 512, False), (64, 64, 192, 2, 1, 32, 512, False), (1, 64, 176, 2, 1, 24, 384, False), (1, 64, 128, 1, 1, 40, 192, False), (260, 32, 96, 4, 4, 8, 384, False),
+    (320, 60, 176, 5, 1, 12, 384, False), (260, 64, 176, 2, 1, 24, 192, False), (512, 64, 192, 2, 1, 32, 512, False), (260, 64, 128, 1, 1, 40, 64, False), (260, 32, 88, 2, 1, 16, 256, False),
+    (300, 64, 192, 4, 2, 16, 512, False),
+    # faster, or as fast
+    (1, 64, 176, 8, 2, 8, 512, True), (256, 64, 176, 8, 4, 8, 512, True), (512, 64, 176, 8, 2, 8, 512, True), (1, 64, 192, 2, 1, 32, 256, True), (256, 64, 192, 4, 2, 16, 512, True),
+    (1, 64, 128, 1, 1, 40, 128, True), (260, 32, 96, 4, 4, 8, 256, True), (320, 64, 192, 16, 4, 4, 512, True), (512, 60, 176, 5, 1, 12, 192, True)])
+def test_small_blocks_where_one_kernel_was_faster(rows, D, F, H, G, HD, keys, takes):
+    assert bool(hip_ops.library("small_block").cdll.tis_small_block_takes(rows, D, F, H, G, HD, keys, 16)) == takes

@@ -10,9 +10,14 @@
 // SB_DOWN pieces, which sets the sizes that the kernel takes); the row's keys and values go to LDS beside them. A head's attention is one wave's and every
 // wave norms the row for itself, so that four barriers are left.
 // us a block in a graph, separate kernels / this one, 64 wide, 8 heads of 8 over 2, 176 hidden: rows that see 40 keys, 3 of them 21.5 / 10.0, 64 24.6 / 10.5, 512
-// 35.8 / 21.1; 250 keys, 3 rows 22.6 / 15.6, 512 41.3 / 31.2. At 900 keys, which one wave walks here and a workgroup there, 28.3 / 31.2:
-// more than SB_KEYS keys are left to the separate kernels, and more than SB_ROWS_MOST rows, two a compute unit. (Matrices through LDS and sums in one chain over K, the
-// bits of the separate kernels: 22.7.)
+// 36.1 / 20.9; 250 keys, 3 rows 22.6 / 15.6, 512 43.0 / 32.2; 512 keys, 1 row 24.7 / 21.6, 256 39.9 / 23.7, 300 46.5 / 44.1, 512 57.6 / 45.8. (Matrices through LDS and sums in one chain
+// over K, the bits of the separate kernels: 22.7 for 3 rows of 40.)
+// Which steps it takes. A head's attention is one wave's, 64 / HD keys at a time, and beyond 256 rows a compute unit has two workgroups one after the other; the separate kernels
+// walk keys on many waves. So up to 256 rows, 128 keys for each of a wave's groups (separate / this one, 1 row: heads of 32, 256 keys 29.0 / 25.7, 384 33.4 / 33.8, 512 37.0 / 41.9; of 24, 256 26.8 / 24.2,
+// 384 30.1 / 31.8; of 40, 128 25.5 / 22.9, 192 27.4 / 30.0; of 16, 512 28.4 / 27.3); beyond, 8 for each group and head, as many heads are what the separate kernels
+// take long for (260 rows: 4 heads of 8 over 4, 256 keys 1.00 of their time, 384 1.11; 5 of 12, 192 keys 0.94, 256 1.08; 2 of 16, 128 keys 0.92, 256 1.10; 2 of 32, 64 keys 0.89, 128 1.02; 8 of 8 over 2, 512 keys
+// 0.97, over 4 1.02; 16 of 4, 512 keys 0.95). The keys are the most that a row may see: in a captured step, and in the launch before it, what its block tables hold (64 pages at least) or the rotary table, whichever is
+// shorter, not what the requests are long. So a model of more positions than SB_KEYS, or one without a rotary table, has its decoded steps run by the separate kernels.
 //
 // Sums are 32-bit: a product's sixteen partial sums of up to 12 terms added up in pairs, where the separate kernels have one chain.
 #include <mutex>
@@ -25,7 +30,7 @@ static constexpr int SB_THREADS = 1024, SB_WAVES = SB_THREADS / TIS_WAVE, SB_LAN
 static constexpr int SB_QKV = 2, SB_O = 1, SB_GU = 6, SB_DOWN = 3, SB_KV = 2;        // pieces of each matrix that a thread holds, and of the cache
 static constexpr int SB_WIDTH = SB_LANES * 4;                                       // most of D and of all heads' channels together
 static constexpr int SB_HIDDEN = SB_DOWN * SB_LANES * 4;                            // most of F
-static constexpr int SB_KEYS = 512, SB_ROWS_MOST = 512;
+static constexpr int SB_KEYS = 512, SB_ROWS_MOST = 512, SB_ROWS_ROUND = 256;          // (a workgroup a compute unit)
 static constexpr long SB_LDS = 160 * 1024;
 static_assert(SB_WIDTH == TIS_WAVE && SB_WIDTH == SB_ROWS && 2 * SB_HIDDEN == SB_GU * SB_ROWS, "a row of the stream is a wave's, an output a turn's");
 
@@ -238,11 +243,13 @@ __global__ __launch_bounds__(SB_THREADS) void small_block_kernel(SmallBlock a) {
 }
 
 // Whether this kernel takes a block of these sizes, whose rows see up to `keys` keys: its matrices in the threads' registers, its keys and values in LDS, and
-// no more rows and keys than it is the faster one for.
+// no more rows and keys than it is the faster one for (see the figures above).
 TIS_EXPORT int tis_small_block_takes(int rows, int D, int F, int H, int G, int HD, int keys, int page_size) {
   if (rows < 1 || rows > SB_ROWS_MOST || D < 4 || D > SB_WIDTH || D % 4 || F < 4 || F % 4 || F > SB_HIDDEN || H < 1 || G < 1 || H % G || HD < 4 || HD % 4 ||
       H > SB_WIDTH || HD > SB_WIDTH || H * HD > SB_WIDTH || (H + 2 * G) * HD > SB_QKV * SB_ROWS || keys < 1 || keys > SB_KEYS || page_size < 1 || page_size > SB_KEYS)
     return 0;
+  const int groups = TIS_WAVE / HD;              // keys that a wave's value sums take at a time
+  if (keys > (rows <= SB_ROWS_ROUND ? 128 : 8 * H) * groups) return 0;
   const long cap = ((long)keys + page_size - 1) / page_size * page_size;
   if (cap * (2L * G * HD + H) * 4 > SB_LDS) return 0;
   return sb_layout(H, G, HD, page_size, (int)cap).end * 4L <= SB_LDS;
