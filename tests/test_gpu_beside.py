@@ -50,3 +50,34 @@ def test_the_same_bits(family, name, launched, monkeypatch):
         results.append(seen)
     assert all(torch.isfinite(y).all() for y in results[0])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+def test_a_captured_pass_does_not_keep_every_blocks_result():
+    """Eight blocks in a row in a capture, whose side results of 64 MB each are dropped block by block: their memory is taken again within the capture, so that
+    the graph's pool holds two at most and not eight; and every replay, with eager work in between, gives what the blocks give by themselves."""
+    from tiny_inference_server_amd.ops.hip_ops import HipOps
+    ops = HipOps("cuda:0", torch.bfloat16)
+    n, blocks = 16 << 20, 8
+    x = torch.randn(n, device="cuda")
+
+    def passes():
+        total = torch.zeros(1024, device="cuda")
+        for i in range(blocks):
+            here, there = ops.beside(lambda: x[:1024] * (i + 1.0), lambda: x + float(i))
+            total = total + here + there[i * 1024:(i + 1) * 1024]
+            del here, there
+        return total
+
+    want = passes().clone()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_reserved()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = passes()
+    assert torch.cuda.memory_reserved() - before < 3 * 4 * n
+    for _ in range(4):
+        graph.replay()
+        passes()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
