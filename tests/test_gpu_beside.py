@@ -81,3 +81,27 @@ def test_a_captured_pass_does_not_keep_every_blocks_result():
         passes()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+def test_the_side_stream_is_the_threads_own():
+    """None of the streams that the framework hands out in turn, nor another running thread's; a thread that has ended leaves its stream to the next."""
+    import threading
+
+    from tiny_inference_server_amd.ops.hip_ops import _beside_stream
+    others = {torch.cuda.Stream().cuda_stream for _ in range(40)}
+    mine, seen, gone = _beside_stream(0), [], []
+
+    def ask():
+        seen.append(_beside_stream(0))
+        y = torch.zeros(4, device="cuda")
+        torch.cuda.synchronize()
+        with torch.cuda.stream(seen[-1]):
+            gone.append(float((y + 1).sum()))
+
+    for _ in range(2):
+        t = threading.Thread(target=ask)
+        t.start()
+        t.join()
+    assert _beside_stream(0).cuda_stream == mine.cuda_stream not in others
+    assert seen[0].cuda_stream == seen[1].cuda_stream not in others | {mine.cuda_stream}
+    assert seen[0].priority == 0 and gone == [4.0, 4.0]

@@ -246,6 +246,12 @@ TIS_EXPORT int tis_upload_ring(const void* ring, int words, void* dst, void* sen
   return tis_launch_status("upload_ring");
 }
 
+// A new stream of the default priority on the current device.
+TIS_EXPORT int tis_stream_create(hipStream_t* stream) {
+  const hipError_t e = hipStreamCreateWithFlags(stream, hipStreamNonBlocking);
+  return e == hipSuccess ? 0 : tis_fail("stream_create: %s", hipGetErrorString(e));
+}
+
 TIS_EXPORT int tis_copy_rows(int dtype, const void* src, long src_ld, const int* src_index, void* dst, long dst_ld,
                              const int* dst_index, int count, int D, hipStream_t stream) {
   if (count == 0) return 0;

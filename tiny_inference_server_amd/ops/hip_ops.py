@@ -71,6 +71,7 @@ _SIGNATURES = {
         "tis_copy_rows": [_I, _P, _L, _P, _P, _L, _P, _I, _I, _P],
         "tis_swiglu": [_I, _P, _L, _P, _L, _I, _I, _P],
         "tis_upload_ring": [_P, _I, _P, _P, _P, _P],
+        "tis_stream_create": [_P],
     }),
     "rope_cache": ("tis_rope_cache", {
         "tis_rope_write_kv": [_I, _P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _L, _P],
@@ -741,17 +742,37 @@ def _side_stream(device_index: int):
     return s
 
 
+class _OwnStream:
+    """A stream (default priority) that belongs to nobody else in the process while this object lives. torch.cuda.Stream hands out the same 32 in turn, so one of those may be
+    another thread's too, who captures on it. Given up, it is kept for the next who asks: the allocator goes by its handle and keeps its memory."""
+    _spare = {}         # device index -> streams
+
+    def __init__(self, device_index: int):
+        spare = self._spare.setdefault(device_index, [])
+        try:
+            stream = spare.pop()
+        except IndexError:
+            handle = c_void_p()
+            with torch.cuda.device(device_index):
+                library("rowwise").tis_stream_create(ctypes.byref(handle))
+            stream = torch.cuda.ExternalStream(handle.value, torch.device("cuda", device_index))
+        self.stream, self._back = stream, spare
+
+    def __del__(self):
+        if hasattr(self, "_back"):
+            self._back.append(self.stream)
+
+
 _beside_streams = threading.local()
 
 
 def _beside_stream(device_index: int):
-    """This thread's stream for `HipOps.beside` (default priority): a thread that captures a graph on it shares it with no other, and the
-    allocator keeps that stream's memory from one engine to the next."""
+    """This thread's stream for `HipOps.beside`: a thread that captures a graph on it shares it with no other as long as it runs."""
     of_device = _beside_streams.__dict__
-    s = of_device.get(str(device_index))
-    if s is None:
-        s = of_device[str(device_index)] = torch.cuda.Stream(torch.device("cuda", device_index))
-    return s
+    held = of_device.get(str(device_index))
+    if held is None:
+        held = of_device[str(device_index)] = _OwnStream(device_index)
+    return held.stream
 
 
 def _rows_view(t: torch.Tensor, what: str):
