@@ -913,9 +913,9 @@ def test_products_of_drawn_shapes(ops_for, first):
 
 @pytest.mark.parametrize("M", [1, 8, 16, 20, 40, 70])
 def test_skinny_product_with_two_column_tiles_a_workgroup(ops_for, M):
-    """Very wide matrices give a workgroup of the staged kernel two column tiles. Forced here at a small width that
-    ends inside the second tile, for the plain, the 32-bit and the normed and gated product, with one and with two
-    blocks of 16 rows, and with two stages of LDS instead of four."""
+    """Wide matrices give a workgroup of the staged kernel two column tiles. Forced here at a small width that leaves the last
+    workgroup's second tile empty, for the plain, the 32-bit and the normed and gated product, with one and with two
+    blocks of 16 rows, and with as few stages of LDS as are built (three, or two) instead of four."""
     ops, ref = ops_for(torch.bfloat16), TorchOps(dtype=torch.bfloat16)
     N, K = 138, 800
     x, w = rnd((M, K), torch.bfloat16, 91, 2.0), rnd((N, K), torch.bfloat16, 92, K ** -0.5)
@@ -927,17 +927,88 @@ def test_skinny_product_with_two_column_tiles_a_workgroup(ops_for, M):
         ops.gemm_skinny.cdll.tis_gemm_skinny_wide_tiles(1)
         wide = [ops.linear(x.cuda(), w.cuda()).cpu(), ops.linear(x.cuda(), w.cuda(), out_dtype=torch.float32).cpu(),
                 ops.linear_swiglu(x.cuda(), w.cuda(), rms=(gain.cuda(), 1e-5)).cpu()]
-        ops.gemm_skinny.cdll.tis_gemm_skinny_staged_stages(2)
+        ops.gemm_skinny.cdll.tis_gemm_skinny_staged_stages(3 if M <= 16 else 2)
         wide2 = [ops.linear(x.cuda(), w.cuda()).cpu(), ops.linear(x.cuda(), w.cuda(), out_dtype=torch.float32).cpu(),
                  ops.linear_swiglu(x.cuda(), w.cuda(), rms=(gain.cuda(), 1e-5)).cpu()]
     finally:
-        ops.gemm_skinny.cdll.tis_gemm_skinny_wide_tiles(256)
+        ops.gemm_skinny.cdll.tis_gemm_skinny_wide_tiles(2 ** 31 - 1)
         ops.gemm_skinny.cdll.tis_gemm_skinny_staged_stages(0)
         ops.gemm_skinny.cdll.tis_gemm_skinny_staged_always(0)
     for a, b, c in zip(narrow, wide, wide2):
         assert torch.equal(a, b)          # the same sums in the same order, only spread over workgroups differently
         assert torch.equal(a, c)
     torch.testing.assert_close(wide[1].double(), x.double() @ w.double().t(), rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 20, 40, 70])
+@pytest.mark.parametrize("N", [138, 144, 150, 155])
+def test_two_column_tiles_with_a_residual(ops_for, M, N):
+    """As above, with a residual, its rows side by side and apart: widths that end inside the first tile, with it, and inside the second, also off a lane's four
+    columns. The same bits as with one column tile a workgroup."""
+    from tiny_inference_server_amd.ops.hip_ops import KernelError
+    ops, ref = ops_for(torch.bfloat16), TorchOps(dtype=torch.bfloat16)
+    K, lib = 328, ops.gemm_skinny.cdll
+    x, w, res = rnd((M, K), torch.bfloat16, 94, 2.0), rnd((N, K), torch.bfloat16, 95, K ** -0.5), rnd((M, N), torch.bfloat16, 96)
+
+    def both():
+        apart = torch.full((M, N + 5), float("nan"), dtype=torch.bfloat16, device="cuda")
+        apart[:, :N] = res.cuda()
+        return [ops.linear(x.cuda(), w.cuda(), residual=r).cpu() for r in (res.cuda(), apart[:, :N])]
+
+    lib.tis_gemm_skinny_staged_always(1)
+    try:
+        results = both()
+        lib.tis_gemm_skinny_staged_stages(2)
+        with pytest.raises(KernelError, match="2 stages"):       # (with one column tile four are built)
+            both()
+        lib.tis_gemm_skinny_wide_tiles(1)
+        for stages in (0, 3 if M <= 16 else 2):
+            lib.tis_gemm_skinny_staged_stages(stages)
+            results += both()
+    finally:
+        lib.tis_gemm_skinny_wide_tiles(2 ** 31 - 1)
+        lib.tis_gemm_skinny_staged_stages(0)
+        lib.tis_gemm_skinny_staged_always(0)
+    assert all(torch.equal(r, results[0]) for r in results)
+    torch.testing.assert_close(results[0].float(), ref.linear(x, w, residual=res).float(), rtol=3e-2, atol=3e-2)
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 20, 40, 70])
+@pytest.mark.parametrize("n_heads,n_kv,hd,interleaved", [(1, 1, 12, False), (2, 1, 20, True), (3, 1, 12, False), (5, 1, 28, False)])
+def test_two_column_tiles_with_rotary_and_cache_write(ops_for, M, n_heads, n_kv, hd, interleaved):
+    """36, 80, 60 and 196 columns: the last workgroup's second tile empty, cut and whole, heads that begin inside a tile. The same bits as with one column tile."""
+    ops, ref = ops_for(torch.bfloat16), TorchOps(dtype=torch.bfloat16)
+    K, page_size, lib = 328, 16, ops.gemm_skinny.cdll
+    n_pages, N = -(-M // page_size) + 3, (n_heads + 2 * n_kv) * hd
+    ang = torch.rand(300, hd // 2, generator=torch.Generator().manual_seed(97)) * 6.28
+    table = torch.stack((torch.cos(ang), torch.sin(ang)), -1).contiguous()
+    x, w, gain = rnd((M, K), torch.bfloat16, 98), rnd((N, K), torch.bfloat16, 99, K ** -0.5), 1 + 0.1 * rnd((K,), torch.float32, 100)
+    positions = torch.tensor(random.Random(101).choices(range(300), k=M), dtype=torch.int32)
+    slots = torch.tensor(random.Random(102).sample(range(n_pages * page_size), M), dtype=torch.int32)
+    plane0 = rnd((n_pages, 2, n_kv, page_size, hd), torch.bfloat16, 103)
+
+    def on(o, device):
+        plane = plane0.clone().to(device)
+        q = o.qkv_rope(x.to(device), w.to(device), (gain.to(device), 1e-5), positions.to(device), slots.to(device), table.to(device), plane, n_heads, n_kv, hd,
+                       page_size, interleaved)
+        return q.cpu(), plane.cpu()
+
+    lib.tis_gemm_skinny_staged_always(1)
+    try:
+        results = [on(ops, "cuda")]
+        lib.tis_gemm_skinny_wide_tiles(1)
+        for stages in (0, 3 if M <= 16 else 2):
+            lib.tis_gemm_skinny_staged_stages(stages)
+            results.append(on(ops, "cuda"))
+    finally:
+        lib.tis_gemm_skinny_wide_tiles(2 ** 31 - 1)
+        lib.tis_gemm_skinny_staged_stages(0)
+        lib.tis_gemm_skinny_staged_always(0)
+    want = on(ref, "cpu")
+    for r in results:
+        assert torch.equal(r[0], results[0][0]) and torch.equal(r[1], results[0][1])
+    torch.testing.assert_close(results[0][0].float(), want[0].float(), rtol=3e-2, atol=3e-2)
+    torch.testing.assert_close(results[0][1].float(), want[1].float(), rtol=3e-2, atol=3e-2)
 
 
 @pytest.mark.parametrize("V", [777, 48000])

@@ -28,6 +28,8 @@
 //   ROPE      the q/k/v projection: rotary encoding of q and k by the row's position, q written out, k and v
 //             written into the row's cache slot (main_models_new.py:75-80, block_table.py:6-28); see RopeArgs
 // Output bfloat16 or float (the output table writes 32-bit logits).
+#include <climits>
+
 #include "common.h"
 
 TIS_DEFINE_LAST_ERROR(tis_gemm_skinny)
@@ -608,10 +610,10 @@ __global__ __launch_bounds__(512) void gemm_staged_kernel(
 }
 
 // (these can be set from outside: the kernel tests make small matrices take the wide path, and measurements compare
-// panel heights)
-static int g_wide_tiles = 256;   // from this many 32-column workgroups on a workgroup takes two column tiles, however few units are idle
+// stages)
+static int g_wide_tiles = INT_MAX;   // tests: two column tiles a workgroup also from this many 32-column workgroups on
 TIS_EXPORT void tis_gemm_skinny_wide_tiles(int n_workgroups) { g_wide_tiles = n_workgroups; }
-static int g_staged_stages = 0;    // measurements and tests: stages of LDS with two column tiles, 2 (the fewest that are built) or 4 (0: as chosen below)
+static int g_staged_stages = 0;    // measurements and tests: stages of LDS (0: as chosen below); a launch for which that many are not built fails
 static int g_staged_always = 0;    // measurements and tests: the staged kernel also where the first one would be chosen
 TIS_EXPORT void tis_gemm_skinny_staged_always(int on) { g_staged_always = on; }
 static int g_units = 256;          // compute units of the device: set by whoever knows (the default is an MI355X)
@@ -632,12 +634,11 @@ static int launch_staged(const void* X, long x_ld, const void* W, const float* g
   // serve twice as many weights, and up to twice the units' number of column tiles run at once with a unit's whole LDS. us, one tile / two, K = 2,048: 1 row of
   // 4,096 columns (256 tiles) 6.3 / 6.8, of 4,352 8.6 / 7.0, of 5,120 8.9 / 7.3, 5,632 9.1 / 7.6, 8,160 10.0 / 9.4; 32 rows of 4,096 7.3 / 8.4, of 5,120 10.4 / 8.9; 64 rows (two
   // panels) of 2,560 9.1 / 7.9, of 4,096 9.8 / 8.4, of 7,168 17.1 / 12.3; 128 of 4,096 16.7 / 11.3; at K = 1,024 the line lies at the same place.
-  const int ct = (long)((N + 31) / 32) * panels >= g_wide_tiles || (long)((N + 15) / 16) * panels > g_units ? 2 : 1;
+  const int ct = (long)((N + 15) / 16) * panels > g_units || (long)((N + 31) / 32) * panels >= g_wide_tiles ? 2 : 1;
   const dim3 grid((N + 16 * ct - 1) / (16 * ct), panels);
   // Stages of LDS: four (three chunks in flight) while every workgroup has a compute unit to itself; beyond, three, so that two share one, or with two blocks of rows two
   // (us, two stages / three: 1 row of 48,000 x 1,536 28.7 / 27.7, of 32,000 x 2,048 32.2 / 30.3, 8 rows 33.3 / 30.2, of 48,000 x 1,536 30.6 / 30.9; 32 rows of 48,000 37.8 / 42.4).
-  int ns = (long)grid.x * grid.y <= g_units ? 4 : mb == 1 ? 3 : 2;
-  if (g_staged_stages && ct == 2) ns = g_staged_stages == 2 && mb == 1 ? 3 : g_staged_stages;
+  const int ns = g_staged_stages ? g_staged_stages : (long)grid.x * grid.y <= g_units ? 4 : mb == 1 ? 3 : 2;
 #define STAGED(MBV, CTV, NS)                                                                                      \
   if (mb == MBV && ct == CTV && ns == NS) {                                                                       \
     gemm_staged_kernel<MBV, CTV, NORM, EPI, TO, NS><<<grid, 512, 0, stream>>>(                                    \
@@ -646,7 +647,7 @@ static int launch_staged(const void* X, long x_ld, const void* W, const float* g
   }
   STAGED(1, 1, 4) STAGED(2, 1, 4) STAGED(1, 2, 4) STAGED(1, 2, 3) STAGED(2, 2, 4) STAGED(2, 2, 2)
 #undef STAGED
-  return tis_fail("gemm_skinny: no staged kernel for %d column tiles and %d stages", ct, ns);
+  return tis_fail("gemm_skinny: no staged kernel of %d stages for %d row blocks and %d column tiles", ns, mb, ct);
 }
 
 template <bool NORM, int EPI, typename TO>
