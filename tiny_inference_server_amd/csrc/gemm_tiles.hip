@@ -69,7 +69,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(
   const GtTile tile = gt_tile(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN);
   const long m0 = (long)tile.m * BM, n0 = (long)tile.n * BN;
   // The residual's four of every eight columns, asked for before the first step where they find room: behind the last one they would be a trip to memory
-  // that nothing hides. (R may be C: a workgroup reads its own results' places before it writes them.)
+  // that nothing hides. (R may be C: a wave reads its own results' places before it writes them; what lanes past an end read nobody looks at.)
   constexpr bool EARLY = RESIDUAL && TM * TN <= 4;
   bf16x4 res[EARLY ? TM : 1][EARLY ? TN : 1][4];
   if constexpr (EARLY)
@@ -263,21 +263,23 @@ TIS_EXPORT void tis_gemm_tiles_units(int n) { if (n > 0) g_units = n; }
 
 // The tiles, and what a product is estimated to take with each, us: a beginning and end, and the time of a step of 64 by r, the tiles a
 // compute unit. Measured with matrices that come from memory (none that a cache still holds), 129 to 8,000 rows, widths of 256 to 48,000. Over
-// 617 such products the one picked here takes 1.006 times the fastest's time on average.
+// 617 such products the one picked here took 1.006 times the fastest's time on average while results left as they lay. The estimates are as they were then: as results leave
+// now (see gemm_tiles_kernel) it takes 1.02 times over 132 products, 90 of them drawn, and 25 of the 132 take more than 3 % longer than with the fastest
+// (159 rows of 32,928 x 1,792 49 / 43, 1,172 of 3,016 x 832 13.5 / 11.6).
 //
 // What bounds a product of few hundred rows is the way of its matrix from memory: a tile's copies reach two to five steps ahead (what
 // its buffers hold; two for the 256 x 256 and the 128 x 192 tile, 5 instead of 4 buffers of 64 x 64, 6 of 64 x 32 and 128 x 64), and there are tiles enough for the chip. us before
-// (tiles of 64 x 64 up to 256 x 256, three steps ahead) / now, and the library's product: 300 rows of 1,536 x 1,536 11.1 / 8.1 (10.6), of
-// 2,304 x 1,536 11.4 / 9.4 (16.6), of 1,536 x 4,096 26 / 15.5 (21.1); 140 rows of 1,536 x 4,096 24.6 / 14.7 (15.6); 700 rows of 2,304 x 1,536
-// 15.2 / 11.3 (16.4); 2,048 rows of 2,304 x 1,536 33 / 22.6 (23.7), of 2,816 x 2,048 41.1 / 31.2 (30.4), of 3,072 x 2,048 41.0 / 32.4 (30.5).
+// (tiles of 64 x 64 up to 256 x 256, three steps ahead) / now, and the library's product: 300 rows of 1,536 x 1,536 11.1 / 7.7 (10.6), of
+// 2,304 x 1,536 11.4 / 9.3 (16.6), of 1,536 x 4,096 26 / 15.3 (21.1); 140 rows of 1,536 x 4,096 24.6 / 14.9 (15.6); 700 rows of 2,304 x 1,536
+// 15.2 / 11.0 (16.4); 2,048 rows of 2,304 x 1,536 33 / 21.1 (23.7), of 2,816 x 2,048 41.1 / 28.7 (30.4), of 3,072 x 2,048 41.0 / 31.2 (30.5).
 // (K in two parts by two sets of waves, for products of less than a tile a unit: 1 to 2.5 us less, but other sums than every other tile's,
 // and than the library's, with which all of these agree to the bit.)
 // Beyond one tile a unit a tile's LDS says how many share one: two of 128 x 192, 64 x 64 and 64 x 32, else one.
 // Tiles of less than 256 x 256 that are alone on their unit are bound by the unit's way from the L2 into LDS, some 60 bytes a nanosecond whatever their size
 // and waves; so for a product of two to three million results, one tile a unit, the smaller the rows of a step the better: 128 x 96 (96 x 128 where only that many
-// fit) in place of 128 x 128, four waves of three 32 x 32 results each. us, 128 x 128 / these, and the library's product: 1,900 rows of 1,536 x 4,096 36.7 / 33.7
-// (35.6), 1,605 34.5 / 31.2 (31.9), 2,048 37.0 / 34.5 (35.8); of 2,048 x 5,632 1,195 44.8 / 40.6 (47.6), 1,482 48.6 / 44.7 (44.0); 1,060 rows of 2,304 x 1,536 17.6 / 16.5
-// (19.9), of 2,048 x 2,048 19.8 / 19.0 (22.9).
+// fit) in place of 128 x 128, four waves of three 32 x 32 results each. us, 128 x 128 / these, and the library's product: 1,900 rows of 1,536 x 4,096 38.4 / 34.1
+// (35.6), 1,605 34.2 / 31.1 (31.9), 2,048 38.5 / 34.7 (35.8); of 2,048 x 5,632 1,195 46.5 / 40.0 (47.6), 1,482 50.5 / 45.8 (44.0); 1,060 rows of 2,304 x 1,536 15.1 / 14.6
+// (19.9), of 2,048 x 2,048 18.4 / 17.2 (22.9).
 struct TileShape { int bm, bn; };
 static constexpr int GT_SHAPES = 10;
 static const TileShape g_shapes[GT_SHAPES] = {{256, 256}, {256, 128}, {192, 128}, {128, 192}, {128, 128}, {128, 64}, {64, 64}, {64, 32}, {128, 96}, {96, 128}};
@@ -301,9 +303,9 @@ static long tiles_of(int i, int M, int N) {
 static float tile_estimate(int i, int M, int N, int K) {
   const float r = (float)tiles_of(i, M, N) / g_units, steps = (float)((K + GT_BK - 1) / GT_BK), part = r - floorf(r);
   // The results' own way to memory, a million of them: tiles that are alone on their unit store while no product runs there. (The time that all
-  // tiles have in common is left out.) It decides where outputs are many and steps few, us with / without: 3,000 rows of 2,816 x 1,024 29 / 36, 7,321 of
-  // 9,088 x 704 122 / 143, 1,531 of 48,000 x 1,536 244 / 290, 3,492 of 15,104 x 384 71 / 83. Of 617 products of 129 to 8,000 rows, 256 to 48,000 columns, 17
-  // instead of 34 now take more than 3 % longer than with the first four tiles there were (256 x 256, 128 x 192, 128 x 128, 64 x 64), all together 0.933 of it.
+  // tiles have in common is left out.) It decides where outputs are many and steps few, us with / without: 3,000 rows of 2,816 x 1,024 26.0 / 30.6, 7,321 of
+  // 9,088 x 704 109 / 118, 1,531 of 48,000 x 1,536 241 / 267, 3,492 of 15,104 x 384 59 / 64. Of the 132 products above 25 instead of 33 take more than 3 % longer than with
+  // the fastest tile. (While results left as they lay, 617 products together took 0.933 of what they did with the first four tiles there were, 256 x 256, 128 x 192, 128 x 128, 64 x 64.)
   const float out = 1e-6f * (float)M * (float)N;
   switch (i) {
     case 0: return 5.0f + steps * (1.85f * floorf(r) + (part > 0.f ? fmaxf(1.5f, 1.5f + 1.2f * (part - 0.6f)) : 0.f));
@@ -338,8 +340,8 @@ TIS_EXPORT int tis_gemm_tiles_count(int M, int N, int K) {
   return n < INT_MAX ? (int)n : INT_MAX;
 }
 
-// W: [N, K] contiguous. R: null, or the residual (bfloat16) added to the product; it may be C itself (every element is
-// read and then written by the same lane). out_f32: C holds 32-bit floats, the sums as they are (the output table's
+// W: [N, K] contiguous. R: null, or the residual (bfloat16) added to the product; it may be C itself: an element is read by the wave that writes it, and a wave
+// has read 32 rows of its own before it writes the first of them (through LDS another lane may write what one has read). out_f32: C holds 32-bit floats, the sums as they are (the output table's
 // logits), and takes no residual. act: 1 the tanh form of gelu, 2 the square of relu, 3 clamped_swish of pairs of columns at
 // `limit`, 4 silu(g) u of pairs of columns of the rounded product
 // (3 and 4: C has N / 2 columns), the others applied to the 32-bit sums; a bfloat16 result without a residual.

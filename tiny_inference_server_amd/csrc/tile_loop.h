@@ -8,7 +8,7 @@
 // bytes are eight such indices at each of two offsets in the 256 bytes that the banks span, so no two of them meet
 // (XORed by the row's number itself, rows r and r + 8 did: half of the LDS's busy cycles were bank conflicts). The
 // copying lane picks the piece that belongs in its slot. The result tile is computed transposed (W's rows are the first operand), so that a
-// lane ends up with four consecutive columns of one row: 8-byte stores, and the residual read the same way.
+// lane ends up with four consecutive columns of one row; how they leave is the kernels' business.
 // A row's sums run over K in the same order whatever M is: its result does not depend on the other rows.
 //
 // What bounds it: the clock under load (8,192 cubed runs at 1.42 PFLOP/s here: 1.5 us for a step of a 256 x 256 tile on every

@@ -266,7 +266,9 @@ def tiles_pay(M: int, N: int, K: int, gate: bool, tile: int, share: float) -> bo
     11,264 x 2,048 29 / 22, 37 / 33, 63 / 57. Where it takes the library: 2,048 x 5,632 at 640, 768 33 / 39, 33 / 39; 3,072 x 2,048 at 2,048 30 / 32; 1,536 x 1,536 at
     1,400, 1,532 17.8 / 19.1; 11,264 x 2,048 with the gate at 768 48 / 51. A block's four products are together nowhere slower than by the library alone, at either
     size, 129 to 2,048 rows, beyond what two chips differ by (2 %); with the row limits alone 2.1B's at 768 rows were by 7 %. Single products that stay on the
-    tiles for the host's sake and are slower there: 1,536 x 4,096 at 768 24 / 27, 2,048 x 2,048 at 640 14.6 / 16.1, 2,048 x 5,632 at 384 26 / 29."""
+    tiles for the host's sake and are slower there: 1,536 x 4,096 at 768 24 / 27, 2,048 x 2,048 at 640 14.6 / 16.1, 2,048 x 5,632 at 384 26 / 29.
+    (The tiles' times and the lines are of results that left as they lay in registers. Through LDS, as they leave now, most of these are within 5 % of the figures; shorter are
+    2,304 x 1,536 at 1,024 rows 15.2, 1,536 x 1,536 at 1,400 and 1,532 13.3 and 13.9, 2,048 x 5,632 at 768 37.7: no product that stays on the tiles has become the slower for it.)"""
     if N % 4:
         return False
     if M > _tiles_up_to(N, K):
