@@ -1,6 +1,8 @@
 """The grouped product of a few rows a group with its sum over K split over a workgroup's waves."""
 from __future__ import annotations
 
+from ctypes import c_long
+
 import pytest
 import torch
 
@@ -46,3 +48,25 @@ def test_against_64_bits(N, K, rows, groups, top):
         bound = (size[:, 0::2] * 1.2 * (1 + limit) + size[:, 1::2] * limit) * (K / 4) * 2.0 ** -24 + gated.abs() * 2.0 ** -20 + 2.0 ** -24
         got = out.double().cpu()
         assert ((got - gated).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("N,K", [(1, 384), (16, 392), (17, 520), (65, 1032), (48, 1544)])
+@pytest.mark.parametrize("rows,heads", [(1, 2), (16, 3), (17, 4), (40, 2)])
+def test_a_product_per_head_against_64_bits(N, K, rows, heads):
+    """Groups of all rows, their columns apart in inputs and results, with and without a gate: edges of blocks of 16 rows and columns, sums that end inside a batch. The bound
+    is that of the lists above; the gate's sigmoid (at most 1, slope 1/4) adds a few roundings of the result."""
+    ops = hip_ops.HipOps("cuda:0", torch.bfloat16)
+    assert ops._lazy("experts").cdll.tis_grouped_split(0, heads, rows, c_long(rows), N, K)
+    g = torch.Generator().manual_seed(N + rows)
+    x, w = torch.randn(rows, heads * K, generator=g).bfloat16(), (torch.randn(heads, N, K, generator=g) * K ** -0.5).bfloat16()
+    gate = torch.randn(rows, heads * N + 3, generator=g)
+    per_head = x.double().view(rows, heads, K)
+    want = torch.einsum("rhk,hnk->rhn", per_head, w.double())
+    size = torch.einsum("rhk,hnk->rhn", per_head.abs(), w.double().abs())
+    for gated in (False, True):
+        out = torch.full((rows, 2 + heads * (N + 3)), 7.0, device="cuda")
+        ops.heads_linear(x.cuda(), w.cuda(), out, N + 3, 2, gate=gate.cuda()[:, 3:] if gated else None)
+        got = out[:, 2:].reshape(rows, heads, N + 3).double().cpu()
+        assert (got[..., N:] == 7.0).all() and (out[:, :2] == 7.0).all()
+        factor = torch.sigmoid(gate[:, 3:].double()).view(rows, heads, N) if gated else 1.0
+        assert ((got[..., :N] - want * factor).abs() <= size * (K / 4) * 2.0 ** -24 + want.abs() * 2.0 ** -20).all()

@@ -55,6 +55,16 @@ def test_sums_over_k_are_split_where_that_was_faster(groups, top, rows, N, K, sp
     assert bool(lib.tis_grouped_split(1, groups, rows, c_long(rows * top), N, K)) == split
 
 
+@pytest.mark.parametrize("heads,rows,N,K,split", [
+    # a product per head; slower with the sum over K split, by 5 to 25 %
+    (64, 32, 128, 1024, False), (128, 16, 128, 512, False), (32, 63, 128, 1536, False), (64, 63, 64, 512, False), (128, 16, 512, 1536, False), (128, 32, 128, 1024, False),
+    (80, 16, 192, 1024, False), (112, 32, 128, 512, False),
+    # faster
+    (16, 16, 128, 512, True), (64, 5, 128, 512, True), (32, 1, 128, 1536, True), (64, 16, 192, 512, True), (64, 32, 64, 512, True), (64, 32, 192, 512, True), (128, 1, 192, 512, True)])
+def test_products_per_head_are_split_where_that_takes_fewer_rounds(heads, rows, N, K, split):
+    assert bool(hip_ops.library("experts").cdll.tis_grouped_split(0, heads, rows, c_long(rows), N, K)) == split
+
+
 @pytest.mark.parametrize("rows,D,F,H,G,HD,keys,takes", [
     # slower in one kernel, by 5 to 45 %
     (1, 64, 192, 2, 1, 32, 512, False), (64, 64, 192, 2, 1, 32, 512, False), (1, 64, 176, 2, 1, 24, 384, False), (1, 64, 128, 1, 1, 40, 192, False), (260, 32, 96, 4, 4, 8, 384, False),

@@ -598,9 +598,16 @@ TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_
 // 5,632 of 2,048, 3 rows 31.6 / 23.9, 16 42.2 / 38.8, 1 row 13.9 / 15.3 alone but a decode step with it 325 / 306; 16 of 4, 16 rows 5,632 of 2,048 74.6 / 67.1; 64 of 8, 16 rows 2,048 of
 // 2,048 91.8 / 85.0; 128 of 8, 8 rows 2,048 of 1,536 60.4 / 56.3, 16 rows 2,048 of 4,096 254 / 227. Where the line lies, 256 blocks (16 of 4, 16 rows) / 512 (the same, twice the columns): K = 384
 // 5.7 / 5.7 and 8.0 / 8.7, 512 6.6 / 6.4 and 9.5 / 10.4, 704 8.1 / 7.4 and 12.2 / 13.2, 1,024 9.6 / 9.2 and 15.6 / 16.1; 640 blocks of 1,024 (64 of 8, 5 rows) 22.1 / 16.1, of 512 12.6 / 11.2; 1,280
-// of 384 13.9 / 16.1. (Mean error against 64 bits, K = 1,408, 2e-7 / 1e-7.)
+// of 384 13.9 / 16.1. Without lists every group has all rows and the blocks are as many as
+// they are counted: split where quarters of blocks take at most 0.85 of the rounds over the units that whole ones take. 128 heads of 128 of 1,024, 16 rows (256 blocks, a round either way) 10.5 / 12.9, 32
+// (two) 17.8 / 22.2; 64, 16 rows (half a round for one) 10.0 / 7.1; 64 of 192 of 512, 32 rows (384: one and a half for two) 10.5 / 9.0; at 510 sizes of 4 to 128 heads never slower than whole, and 1.005 of
+// the faster one's time. (Mean error against 64 bits, K = 1,408, 2e-7 / 1e-7.)
 TIS_EXPORT int tis_grouped_split(int lists, int groups, int most_rows, long most_entries, int N, int K) {
   const long blocks = (lists ? (most_entries < groups ? most_entries : groups) : (long)groups * ((most_rows + 15) / 16)) * ((N + 63) / 64);
+  if (!lists) {
+    const long whole = (blocks + g_units - 1) / g_units, quarters = (4 * blocks + g_units - 1) / g_units;
+    return K >= 384 && 5 * quarters <= 17 * whole;
+  }
   return K >= 384 && (K >= 1536 || 2 * blocks <= (K >= 1024 ? 6L : 3L) * g_units);
 }
 
