@@ -630,22 +630,44 @@ static int launch_staged(const void* X, long x_ld, const void* W, const float* g
   const int panels = (M + mb * 16 - 1) / (mb * 16);
   if (panels > 65535) return tis_fail("gemm_skinny: %d rows are more panels than a grid holds", M);
   if (NORM && ((uintptr_t)gain % 16)) return tis_fail("gemm_skinny: the norm's gains must be 16-byte aligned");
-  // Two column tiles a workgroup once one each would be more workgroups than there are units: the panel's activations, which a workgroup copies in full, then
-  // serve twice as many weights, and up to twice the units' number of column tiles run at once with a unit's whole LDS. us, one tile / two, K = 2,048: 1 row of
-  // 4,096 columns (256 tiles) 6.3 / 6.8, of 4,352 8.6 / 7.0, of 5,120 8.9 / 7.3, 5,632 9.1 / 7.6, 8,160 10.0 / 9.4; 32 rows of 4,096 7.3 / 8.4, of 5,120 10.4 / 8.9; 64 rows (two
-  // panels) of 2,560 9.1 / 7.9, of 4,096 9.8 / 8.4, of 7,168 17.1 / 12.3; 128 of 4,096 16.7 / 11.3; at K = 1,024 the line lies at the same place.
-  const int ct = (long)((N + 15) / 16) * panels > g_units || (long)((N + 31) / 32) * panels >= g_wide_tiles ? 2 : 1;
+  // Column tiles a workgroup (two serve twice as many weights with the panel's activations, which a workgroup copies in full) and stages of LDS (four, three chunks in
+  // flight, are for a workgroup that has its compute unit to itself; with two, several share one). us, matrices from memory, one tile and two stages / two tiles and as many stages as the
+  // rule gives them, K = 2,048 unless said, plain or gated:
+  // - one tile each for every unit at most: one, four stages (two tiles would leave half of the units idle: 12 rows of 4,096 6.7 / 7.7).
+  // - two each would: two, four stages (12 rows of 4,608 9.2 / 7.9, of 7,168 10.0 / 9.2, of 8,192 10.4 / 10.1; 64 rows, two panels, of 2,304 9.3 / 8.1, of 4,096 10.3 / 8.9), from
+  //   1,024 inner columns on for one block of rows and 512 for two (1 row of 4,112 x 512 3.61 / 3.76, of 4,112 x 256 2.95 / 3.22; 32 rows x 256 3.5 / 3.9).
+  // - beyond, one block of rows: one while a unit has three at most, because the few workgroups of two tiles that come after the first round are alone with their unit's way from memory (12 rows
+  //   of 8,320 11.2 / 11.6, x 4,096 17.8 / 19.5; of 12,288 x 4,096 20.6 / 23.5); then two (of 16,384 x 1,536 12.5 / 11.7, of 48,000 x 1,536 31.3 / 28.7), with
+  //   three stages where chunks and workgroups are many (32-bit results, 1 row of 48,000 x 1,536, two stages / three 27.4 / 26.5, 12 rows of 32,000 x 1,536 22.2 / 20.2). With a residual or the rotary epilogue, which
+  //   weigh less on a lane, always one (12 rows of 16,384 x 4,096 26.9 / 30.0, of 8,320 x 4,096 16.2 / 19.7).
+  // - beyond, two blocks: two (64 rows of 7,168 18.4 / 12.8, 128 of 4,096 17.7 / 11.8); with a residual one where two would leave up to 16 workgroups for a round of their own (64 rows of
+  //   8,320 19.9 / 22.6, 128 of 4,112 x 4,096 32.2 / 40.6).
+  // Of 1,359 such products (256 to 5,632 inner columns) ten take more than 2 % longer than with one tile where there is a residual and two from as many workgroups as units on where there is none, two more
+  // than 5 % (with a residual, 64 rows of 4,112 x 4,096 21.8 / 23.9, 128 of 16,384 x 4,096 102 / 112); all together 0.917 of it.
+  constexpr bool light = EPI == EPI_RESIDUAL || EPI == EPI_ROPE;
+  const long one = (long)((N + 15) / 16) * panels, two = (long)((N + 31) / 32) * panels;
+  int ct, ns = 2;
+  if (one <= g_units) ct = 1, ns = 4;
+  else if (two <= g_units) {
+    ct = K >= (mb == 1 ? 1024 : 512) ? 2 : 1;
+    if (ct == 2) ns = 4;
+  } else if (mb == 1) {
+    ct = light || one <= 3L * g_units ? 1 : 2;
+    if (ct == 2 && K >= 1536 && two >= 3L * g_units) ns = 3;
+  } else {
+    const long last = two % (2L * g_units);
+    ct = light && last > 0 && last <= 16 ? 1 : 2;
+  }
+  if (two >= g_wide_tiles) ct = 2, ns = two <= g_units ? 4 : 2;
+  if (g_staged_stages) ns = g_staged_stages;
   const dim3 grid((N + 16 * ct - 1) / (16 * ct), panels);
-  // Stages of LDS: four (three chunks in flight) while every workgroup has a compute unit to itself; beyond, three, so that two share one, or with two blocks of rows two
-  // (us, two stages / three: 1 row of 48,000 x 1,536 28.7 / 27.7, of 32,000 x 2,048 32.2 / 30.3, 8 rows 33.3 / 30.2, of 48,000 x 1,536 30.6 / 30.9; 32 rows of 48,000 37.8 / 42.4).
-  const int ns = g_staged_stages ? g_staged_stages : (long)grid.x * grid.y <= g_units ? 4 : mb == 1 ? 3 : 2;
 #define STAGED(MBV, CTV, NS)                                                                                      \
   if (mb == MBV && ct == CTV && ns == NS) {                                                                       \
     gemm_staged_kernel<MBV, CTV, NORM, EPI, TO, NS><<<grid, 512, 0, stream>>>(                                    \
         (const bf16*)X, x_ld, (const bf16*)W, gain, eps, (const bf16*)R, r_ld, (TO*)C, c_ld, M, N, K, rope);      \
     return 0;                                                                                                     \
   }
-  STAGED(1, 1, 4) STAGED(2, 1, 4) STAGED(1, 2, 4) STAGED(1, 2, 3) STAGED(2, 2, 4) STAGED(2, 2, 2)
+  STAGED(1, 1, 4) STAGED(1, 1, 2) STAGED(2, 1, 4) STAGED(2, 1, 2) STAGED(1, 2, 4) STAGED(1, 2, 3) STAGED(1, 2, 2) STAGED(2, 2, 4) STAGED(2, 2, 2)
 #undef STAGED
   return tis_fail("gemm_skinny: no staged kernel of %d stages for %d row blocks and %d column tiles", ns, mb, ct);
 }

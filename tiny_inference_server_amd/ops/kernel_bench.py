@@ -146,8 +146,7 @@ def main(argv=None) -> int:
     pr.add_argument("--in", dest="inner", type=int, default=1536)
     pr.add_argument("--kind", choices=["plain", "residual", "norm", "norm+gate", "logits"], default="plain")
     pr.add_argument("--copies", type=int, default=1, help="weight matrices that the launches take in turn")
-    pr.add_argument("--staged", default="", help="LDS stages of the staged few-row kernel: 4, or where a workgroup takes two column tiles 3 for up to 16 rows and 2 beyond "
-                         "(default: its own choice; others are refused)")
+    pr.add_argument("--staged", default="", help="LDS stages of the staged few-row kernel, 2 or 4 (default: its own choice; others are refused where they are not built)")
     pr.add_argument("--staged-always", action="store_true", help="that kernel also for up to 8 rows of narrow matrices")
     pr.add_argument("--few-rows", type=int, default=0, help="the row count up to which the few-row kernel is used (0: as built)")
     for p in (at, pr):
