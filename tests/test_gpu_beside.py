@@ -19,6 +19,7 @@ def test_the_same_bits(family, name, launched, monkeypatch):
     from tiny_inference_server_amd.config import config_from_dict
     from tiny_inference_server_amd.engine import Engine
     from tiny_inference_server_amd.ops.hip_ops import _BESIDE_FROM, HipOps
+    monkeypatch.setattr("tiny_inference_server_amd.ops.hip_ops._BESIDE_WIDTH", 1)        # (as many rows as a wide model, however narrow this one is)
     if launched:
         monkeypatch.setattr("tiny_inference_server_amd.ops.hip_ops._BESIDE_LAUNCHED_FROM", _BESIDE_FROM)
     if family == "fesupel":
@@ -34,7 +35,7 @@ def test_the_same_bits(family, name, launched, monkeypatch):
     monkeypatch.setattr(HipOps, "beside", lambda self, *a: (counts.append(1), inner(self, *a))[1])
     for beside in (True, False):
         if not beside:
-            monkeypatch.setattr(HipOps, "beside_pays", lambda self, batch: False)
+            monkeypatch.setattr(HipOps, "beside_pays", lambda self, batch, width: False)
         eng = Engine(config=config_from_dict(cfg), tensors=w, dtype="bfloat16", max_requests=4, page_size=16, max_tokens=2048)
         g = torch.Generator().manual_seed(3)
         seen, ran = [], [{} for _ in range(5)]

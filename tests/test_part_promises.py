@@ -3,6 +3,7 @@ with a stand-in for the operations that only a GPU has."""
 from __future__ import annotations
 
 import dataclasses
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -10,6 +11,7 @@ import torch
 from tiny_inference_server_amd.architectures.gqa_mtp import build_spec
 from tiny_inference_server_amd.config import ARCHITECTURES, Architecture, GqaMtpConfig
 from tiny_inference_server_amd.engine import Engine
+from tiny_inference_server_amd.ops.hip_ops import HipOps
 from tiny_inference_server_amd.parts import FEED_FORWARDS, MIXERS
 from tiny_inference_server_amd.parts.attention import GqaAttention
 from tiny_inference_server_amd.parts.base import side_by_side
@@ -95,8 +97,8 @@ class _Streams:
     def __init__(self, pays=True):
         self.pays, self.log = pays, []
 
-    def beside_pays(self, batch):
-        return self.pays
+    def beside_pays(self, batch, width):
+        return self.pays and width == 7
 
     def beside(self, first, second):
         self.log.append(("beside", second()))
@@ -122,12 +124,22 @@ class _FromOwn(_Own):
 def test_which_mixer_goes_beside_the_other(left, right, beside, pays):
     """The one that owns its memory, whichever side it is on; results come in the order of the calls."""
     ops = _Streams(pays)
-    assert side_by_side(ops, None, [(left(), lambda: "left"), (right(), lambda: "right")]) == ["left", "right"]
+    assert side_by_side(ops, None, 7, [(left(), lambda: "left"), (right(), lambda: "right")]) == ["left", "right"]
     if pays and beside:
         assert ops.log == [("beside", beside), ("here", "left" if beside == "right" else "right")]
     else:
         assert ops.log == []
-    assert side_by_side(ops, None, [(_Own(), lambda: 1)]) == [1] and side_by_side(object(), None, [(_Own(), lambda: 1), (_Own(), lambda: 2)]) == [1, 2]
+    assert side_by_side(ops, None, 7, [(_Own(), lambda: 1)]) == [1] and side_by_side(object(), None, 7, [(_Own(), lambda: 1), (_Own(), lambda: 2)]) == [1, 2]
+
+
+@pytest.mark.parametrize("width,captured,launched", [(512, 1024, 6144), (1024, 256, 3072), (1408, 136, 2235), (2048, 64, 1536), (4096, 64, 1536)])
+def test_rows_from_which_mixers_run_side_by_side(width, captured, launched, monkeypatch):
+    """More of them the narrower the model is, as it has less to do in the same launches."""
+    ops = SimpleNamespace(dtype=torch.bfloat16)
+    for capturing, first in ((True, captured), (False, launched)):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+        assert [HipOps.beside_pays(ops, SimpleNamespace(max_seq_rows=n), width) for n in (1, first - 1, first, first + 5000)] == [False, False, True, True]
+    assert not HipOps.beside_pays(SimpleNamespace(dtype=torch.float32), SimpleNamespace(max_seq_rows=9999), width)
 
 
 def test_mixers_that_own_their_memory():

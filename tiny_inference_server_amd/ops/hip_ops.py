@@ -724,13 +724,17 @@ def tile_pieces(seq_rows, tiles, tile_splits: int, tile_max_steps: int, window: 
     return out[:n]
 
 
-# The two mixers of a block run side by side if a request brings at least this many rows, in a captured step and launch by launch. us of a whole pass
+# The two mixers of a block run side by side if a request brings at least this many rows, in a captured step and launch by launch, where the model is this wide or wider. us of a whole pass
 # one after the other / side by side, both in one run. Captured: attention beside a delta rule (4 blocks), one prompt of 16 rows 815 / 833, 64 975 / 950,
 # 256 1242 / 1184, 512 1537 / 1488, 1,024 2090 / 1938, 1,531 2690 / 2430; attention beside a matrix state (6 blocks), 64 rows 750 / 736, 256 880 / 852,
 # 1,024 1628 / 1597. Steps of single rows do not pay for the branches' fork and join: 5 rows 439 / 450, 32 590 / 613, 128 978 / 1034. Launch by
 # launch the host needs some 100 us more a block, which few rows do not cover: 64 rows 1605 / 2090 and 880 / 1100, 1,024 2227 / 2187 and
 # 1712 / 1754, 2,000 3372 / 3187 and 2663 / 2607.
-_BESIDE_FROM, _BESIDE_LAUNCHED_FROM = 64, 1536
+# A narrower model's mixers have less to do, by the square of the width where products make most of it, while fork and join and the host's share stay what they are; so the rows
+# rise with the square of what is missing in width in a captured step, and launch by launch with the width. 1,024 wide, the two designs, captured, 66 rows 669 / 670 and 547 / 560, 130 746 / 759
+# and 549 / 565, 300 832 / 830 and 610 / 604; launched, 1,540 rows 1854 / 2066 and 1192 / 1337, 1,900 2033 / 2094 and 1275 / 1373, 2,600 2790 / 2366 and 1560 / 1520, 3,200 3132 / 2724 and
+# 1818 / 1774; 512 wide, launched, 2,000 rows 1718 / 2121 and 1062 / 1257, 4,000 2607 / 2547 and 1395 / 1386, 7,000 4026 / 3821 and 1960 / 1941.
+_BESIDE_FROM, _BESIDE_LAUNCHED_FROM, _BESIDE_WIDTH = 64, 1536, 2048
 
 _side_streams = {}
 
@@ -827,9 +831,10 @@ class HipOps:
             if dtype == torch.bfloat16 else None
 
     # ---- two branches of a block side by side ----------------------------------------------------------------
-    def beside_pays(self, batch) -> bool:
-        rows = batch.max_seq_rows
-        return rows >= _BESIDE_FROM and self.dtype == torch.bfloat16 and (rows >= _BESIDE_LAUNCHED_FROM or torch.cuda.is_current_stream_capturing())
+    def beside_pays(self, batch, width: int) -> bool:
+        rows, narrow = batch.max_seq_rows, max(1.0, _BESIDE_WIDTH / width)
+        return (rows >= _BESIDE_FROM * narrow * narrow and self.dtype == torch.bfloat16
+                and (rows >= _BESIDE_LAUNCHED_FROM * narrow or torch.cuda.is_current_stream_capturing()))
 
     def beside(self, first, second):
         """first() on the current stream and second() on one of this thread's own beside it; returns both results, which the current stream may

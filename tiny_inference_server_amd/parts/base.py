@@ -162,10 +162,10 @@ def states(part, name: str) -> bool:
     return bool(type(part).__dict__.get(name))
 
 
-def side_by_side(ops, batch, calls):
-    """The results of the calls [(mixer, call)] of a block's mixers, which read the same rows. One of two runs beside the other where the operations
-    object can (`beside`), says that it pays for this step, and that mixer promises own_memory."""
-    if len(calls) == 2 and hasattr(ops, "beside") and ops.beside_pays(batch):
+def side_by_side(ops, batch, width, calls):
+    """The results of the calls [(mixer, call)] of a block's mixers, which read the same rows of `width` columns. One of two runs beside the other where the
+    operations object can (`beside`), says that it pays for this step, and that mixer promises own_memory."""
+    if len(calls) == 2 and hasattr(ops, "beside") and ops.beside_pays(batch, width):
         own = [states(m, "own_memory") for m, _ in calls]
         if own[1]:
             return list(ops.beside(calls[0][1], calls[1][1]))

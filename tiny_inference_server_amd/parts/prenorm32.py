@@ -190,7 +190,7 @@ class SandwichStream32(PreNormStream32):
             calls = [(m, lambda m=m, n=n, c=c: m.forward_projected(proj[:, c[0]:c[1]], ctx.of(n))) for (n, m, _), c in zip(self.mixers, self.cols)]
         else:
             calls = [(m, lambda m=m, n=n: m.forward32(h, ctx.of(n))) for n, m, _ in self.mixers]
-        results = side_by_side(self.ops, ctx.of(self.mixers[0][0]).batch, calls)
+        results = side_by_side(self.ops, ctx.of(self.mixers[0][0]).batch, h.shape[1], calls)
         if len(results) == 1:
             return results[0], post
         eps = {j.eps for _, _, j in self.mixers}

@@ -178,7 +178,7 @@ class PostNormGated(Arrangement):
         ops = self.ops
         proj = ops.linear(x.rows, self.w_in, out_dtype=torch.float32)
         calls = [(m, lambda m=m, n=n, c=c: m.forward_projected(proj[:, c[0]:c[1]], ctx.of(n))) for n, m, c, _ in self.mixers]
-        results = side_by_side(ops, ctx.of(self.mixers[0][0]).batch, calls)
+        results = side_by_side(ops, ctx.of(self.mixers[0][0]).batch, x.rows.shape[1], calls)
         branches = [(y, scale) for y, (_, _, _, scale) in zip(results, self.mixers)]
         gate = proj[:, self.gate_cols[0]:self.gate_cols[1]] if self.gate_cols else None
         full, rows = ops.gated_postnorm(x.full, branches, gate, self.gate_a.bias if gate is not None else None,
