@@ -601,7 +601,8 @@ TIS_EXPORT int tis_grouped_tile(int lists, int groups, int most_rows, long most_
 // of 384 13.9 / 16.1. Without lists every group has all rows and the blocks are as many as
 // they are counted: split where quarters of blocks take at most 0.85 of the rounds over the units that whole ones take. 128 heads of 128 of 1,024, 16 rows (256 blocks, a round either way) 10.5 / 12.9, 32
 // (two) 17.8 / 22.2; 64, 16 rows (half a round for one) 10.0 / 7.1; 64 of 192 of 512, 32 rows (384: one and a half for two) 10.5 / 9.0; at 510 sizes of 4 to 128 heads never slower than whole, and 1.005 of
-// the faster one's time. (Mean error against 64 bits, K = 1,408, 2e-7 / 1e-7.)
+// the faster one's time. Four shorter chains are also the more exact ones: relative error against 64 bits, whole / split, K = 384 1.1e-7 / 0.7e-7, 1,024 1.8e-7 /
+// 1.0e-7, 2,048 2.7e-7 / 1.3e-7, 5,632 4.7e-7 / 2.2e-7.
 TIS_EXPORT int tis_grouped_split(int lists, int groups, int most_rows, long most_entries, int N, int K) {
   const long blocks = (lists ? (most_entries < groups ? most_entries : groups) : (long)groups * ((most_rows + 15) / 16)) * ((N + 63) / 64);
   if (!lists) {
