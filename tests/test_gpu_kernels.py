@@ -961,7 +961,7 @@ def test_two_column_tiles_with_a_residual(ops_for, M, N):
         lib.tis_gemm_skinny_staged_stages(2)
         results += both()
         lib.tis_gemm_skinny_wide_tiles(1)
-        for stages in (0, 2):
+        for stages in (0, 2, 3) if M <= 16 else (0, 2):
             lib.tis_gemm_skinny_staged_stages(stages)
             results += both()
         lib.tis_gemm_skinny_staged_stages(5)
@@ -999,7 +999,7 @@ def test_two_column_tiles_with_rotary_and_cache_write(ops_for, M, n_heads, n_kv,
     try:
         results = [on(ops, "cuda")]
         lib.tis_gemm_skinny_wide_tiles(1)
-        for stages in (0, 2):
+        for stages in (0, 2, 3) if M <= 16 else (0, 2):
             lib.tis_gemm_skinny_staged_stages(stages)
             results.append(on(ops, "cuda"))
     finally:
